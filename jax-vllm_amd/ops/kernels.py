@@ -658,9 +658,72 @@ def paged_attention_generic(out, q, q_row_stride, k_pages, v_pages, block_tables
     )
 
 
+ATTN_F32_HEAD_DIMS = (32, 64, 96, 128, 256)
+
+
+def attn_f32_possible(dtype, head_dim: int, page_size: int) -> bool:
+    """Whether the 32-bit attention on the matrix cores takes these sizes (else: ``paged_attention_generic``)."""
+    return dtype == torch.float32 and head_dim in ATTN_F32_HEAD_DIMS and page_size % 4 == 0
+
+
+def attn_f32_rows() -> int:
+    """(query, head-in-group) rows of a work item."""
+    return library.core().jv_attn_f32_rows()
+
+
+def attn_f32_splits(n_work: int, nkv: int, keys: int, device) -> int:
+    """Blocks that share out a work item's keys: one while the items give every compute unit a block, else as many as do,
+    each with a whole turn of its waves' keys (16 q heads over 4 kv heads of 128, launches included: a token each of 16
+    requests of 1,000 keys 19.8 us with 4 blocks an item, 36.6 with one, 27.8 with 9; one such token 17.5 with 16, 32.9 with
+    one; 100 tokens behind 1,000 27.7 with two, 38.4 with one)."""
+    turns = -(-keys // library.core().jv_attn_f32_tile_keys())
+    return max(1, min(compute_units(device) // max(1, n_work * nkv), turns))
+
+
+def attn_f32_part_floats(n_work: int, nkv: int, splits: int, head_dim: int) -> int:
+    lib = library.core()
+    lib.jv_attn_f32_part_floats.restype = c_longlong
+    return lib.jv_attn_f32_part_floats(c_int(n_work), c_int(nkv), c_int(splits), c_int(head_dim))
+
+
+def attn_f32(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_seqlens, context_lens, work, n_work,
+             nq, nkv, head_dim, scale, window=0, splits=1, parts=None, sinks=None, cap: float = 0.0, keep: int = 0) -> None:
+    """Causal attention of every token over its request's pages in true 32-bit on the matrix cores.  ``work`` is int32
+    [n_work, 2]: (request index, first row of ``attn_f32_rows`` (query, head-in-group) rows); every row of every request
+    must be in exactly one item.  With ``splits`` > 1 that many blocks share out an item's keys and ``parts`` (float32,
+    ``attn_f32_part_floats`` entries) holds their sums.  The other arguments: as for ``paged_attention_generic``."""
+    _dev(out, q, k_pages, v_pages, block_tables, cu_seqlens, context_lens, work, sinks)
+    if sinks is not None:
+        _f32(sinks, "sinks", nq)
+    n = out.shape[0]
+    page_size = k_pages.shape[2]
+    _need(q.dtype == torch.float32 and attn_f32_possible(out.dtype, head_dim, page_size), "32-bit attention: see attn_f32_possible")
+    _need(out.shape == (n, nq * head_dim), "out must be [tokens, nq * D]")
+    _need(q.numel() >= (n - 1) * q_row_stride + nq * head_dim if n else True, "q is too small for its stride")
+    _need(nkv > 0 and nq % nkv == 0, "q heads must be a multiple of kv heads")
+    _check_pages(k_pages, v_pages, q.dtype, nkv, page_size, head_dim)
+    _need(block_tables.dim() == 2, "block_tables must be [requests, pages]")
+    for t, name in ((block_tables, "block_tables"), (cu_seqlens, "cu_seqlens"), (context_lens, "context_lens"), (work, "work")):
+        _i32(t, name)
+    _need(cu_seqlens.numel() == context_lens.numel() + 1 == block_tables.shape[0] + 1,
+          "cu_seqlens, context_lens and block_tables disagree on the number of requests")
+    _need(work.numel() >= 2 * n_work, "work list shorter than n_work")
+    if splits > 1:
+        _need(parts is not None and parts.is_cuda and parts.dtype == torch.float32
+              and parts.numel() >= attn_f32_part_floats(n_work, nkv, splits, head_dim), "parts too small for the splits")
+    _check(
+        library.core().jv_attn_f32(_ptr(out), _ptr(q), c_longlong(q_row_stride), _ptr(k_pages), _ptr(v_pages), _ptr(block_tables),
+                                   c_int(block_tables.shape[1]), _ptr(cu_seqlens), _ptr(context_lens), _ptr(work),
+                                   c_int(n_work), c_int(splits), _ptr(parts if splits > 1 else None), c_int(page_size),
+                                   c_int(nq), c_int(nkv), c_int(head_dim), c_float(scale), c_int(window or 0), _ptr(sinks),
+                                   c_float(cap), c_int(keep if window else 0), _stream()),
+        "attn_f32",
+    )
+
+
 # --------------------------------------------------------------------------- matrix products
 def gemm_f32(a: torch.Tensor, w: torch.Tensor, out=None) -> torch.Tensor:
-    """out = a @ w.T in true 32-bit (float FMA).  a [M, K], w [N, K], both row-major."""
+    """out = a @ w.T in true 32-bit (float products and sums).  a [M, K], w [N, K], both row-major."""
     _dev(a, w)
     _f32(a, "a")
     _f32(w, "w")
@@ -890,7 +953,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
            partial_max_width: int | None = PARTIAL_SUM_MAX_WIDTH):
     """x @ w.T for w stored [out, in].
 
-    float32: the library's own float-FMA kernel (no reduced-precision matrix mode).
+    float32: the library's own kernel in true 32-bit (no reduced-precision matrix mode).
     bfloat16, at most 16 rows (and some shapes up to 64): a weight-streaming MFMA kernel of this
     library (``streaming_plan``).
     bfloat16 otherwise: a plain library matrix product (hipBLASLt through torch), float accumulation.

@@ -6,8 +6,9 @@ requests would leave the chip idle), all others to the prefill kernel in groups 
 head-in-group) rows; a work item names two groups of one request, heaviest items first: two
 neighbours where the kernel gives each group waves of its own (they see the same keys), else,
 while all blocks are on the chip at once, a group that sees many keys with one that sees few, so
-that all blocks carry the same load.  Everything else
-(float32, other head sizes) runs the generic float-math kernel.  The plan depends on the
+that all blocks carry the same load.  float32 with a head size and page size the 32-bit
+matrix-core kernel is built for runs that one, in work items of 16 rows.  Everything else
+(other head sizes and page sizes) runs the generic float-math kernel.  The plan depends on the
 step's lengths, the heads-per-group ratio and which keys the layer's queries see, so it is built
 once per step and shared by all layers alike.
 """
@@ -150,6 +151,32 @@ def plan_mfma(ctx, nq: int, nkv: int, head_dim: int, window: int, device, keep: 
                     dev[3 * n_pre:] if decode and not decode_only else None, len(decode), splits, scratch)
 
 
+@dataclass
+class F32Plan:
+    work: torch.Tensor               # int32 [n, 2]
+    n_work: int
+    splits: int
+    parts: Optional[torch.Tensor]
+
+
+def f32_work_items(q_lens, context_lens, g: int, rows: int):
+    """Work items (request, first row) of the 32-bit kernel, those that see the most keys first."""
+    items = [(-(cl + -(-min(ql * g, m0 + rows) // g)), r, m0)
+             for r, (ql, cl) in enumerate(zip(q_lens, context_lens)) for m0 in range(0, ql * g, rows)]
+    return [(r, m0) for _, r, m0 in sorted(items)]
+
+
+def plan_f32(ctx, nq: int, nkv: int, head_dim: int, window: int, device, keep: int) -> F32Plan:
+    items = f32_work_items(ctx.q_lens_host, ctx.context_lens_host, nq // nkv, K.attn_f32_rows())
+    most = max(c + q for c, q in zip(ctx.context_lens_host, ctx.q_lens_host))
+    splits = K.attn_f32_splits(len(items), nkv, keys_seen(most, window, keep), device)
+    parts = None
+    if splits > 1:
+        parts = torch.empty(K.attn_f32_part_floats(len(items), nkv, splits, head_dim), dtype=torch.float32, device=device)
+    flat = torch.tensor([x for item in items for x in item], dtype=torch.int32)
+    return F32Plan(flat.pin_memory().to(device, non_blocking=True), len(items), splits, parts)
+
+
 def run(att, out, qkv, ctx, mem) -> None:
     # q heads of a row sit at the front of the fused q/k/v projection, unless the mixer says where else
     q_row_stride = getattr(att, "q_row_stride", None) or (att.nq + 2 * att.nkv) * att.d
@@ -157,6 +184,15 @@ def run(att, out, qkv, ctx, mem) -> None:
     sinks = getattr(att, "sinks", None)      # float [nq] or None: one more term exp(sink) in every softmax denominator
     cap = getattr(att, "softcap", None) or 0.0                       # scores under a soft cap
     keep = (getattr(att, "keep_first", 0) or 0) if window else 0     # first keys seen whatever the window
+    if K.attn_f32_possible(qkv.dtype, att.d, ctx.page_size):
+        key = ("attn_f32_plan", att.nq, att.nkv, att.d, window, keep)
+        plan = ctx.plans.get(key)
+        if plan is None:
+            plan = ctx.plans[key] = plan_f32(ctx, att.nq, att.nkv, att.d, window, qkv.device, keep)
+        K.attn_f32(out, qkv, q_row_stride, mem.pages["k"], mem.pages["v"], ctx.block_tables[mem.group], ctx.cu_seqlens,
+                   ctx.context_lens, plan.work, plan.n_work, att.nq, att.nkv, att.d, att.scale, window, plan.splits,
+                   plan.parts, sinks=sinks, cap=cap, keep=keep)
+        return
     if not K.mfma_attention_supported(qkv.dtype, att.d, ctx.page_size):
         K.paged_attention_generic(
             out, qkv, q_row_stride, mem.pages["k"], mem.pages["v"], ctx.block_tables[mem.group], ctx.token_req,

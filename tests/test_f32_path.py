@@ -1,9 +1,9 @@
-"""The 32-bit path's products on the matrix cores: against float64 at the edges of tiles and parts, and bit by bit across
-batches."""
+"""The 32-bit path's products and attention on the matrix cores: against float64, at the edges of tiles and parts, and the
+products bit by bit across batches."""
 import pytest
 import torch
 
-from .test_kernels_gpu import K, randn
+from .test_kernels_gpu import K, build_paged, randn
 
 
 # ------------------------------------------------------------------ matrix products
@@ -19,3 +19,109 @@ def test_gemm_f32_tiles_and_parts(m, n, k):
     # whatever tile the batch takes, a row's bits are the same
     for rows in (slice(0, 1), slice(m // 2, m // 2 + 1), slice(0, (m + 1) // 2)):
         assert torch.equal(K().gemm_f32(a[rows].contiguous(), w), out[rows])
+
+
+# ------------------------------------------------------------------ attention
+def reference(q, k, v, pos, scale, window, chunk, keep, cap, sinks):
+    g = q.shape[1] // k.shape[1]
+    kk, vv = (torch.repeat_interleave(x.double(), g, dim=1) for x in (k, v))
+    s = torch.einsum("qhd,khd->hqk", q.double(), kk) * scale
+    if cap:
+        s = cap * torch.tanh(s / cap)
+    i, j = pos[:, None], torch.arange(k.shape[0])[None, :]
+    seen = j <= i
+    if window:
+        seen &= (i - j < window) | (j < keep)
+    if chunk:
+        seen &= (i // chunk == j // chunk) | (j < keep)
+    s = s.masked_fill(~seen[None], float("-inf"))
+    if sinks is not None:
+        s = torch.cat([s, sinks.double()[:, None, None].expand(-1, s.shape[1], 1)], -1)
+    p = torch.softmax(s, -1)[..., :k.shape[0]]
+    return torch.einsum("hqk,khd->qhd", p, vv)
+
+
+# nq, nkv, d, page size, [(cached, new)], window, chunk, keep, cap, sinks
+CASES = [
+    (4, 2, 32, 4, [(0, 1), (0, 5), (14, 3), (15, 1), (16, 1)], None, None, 0, 0.0, False),
+    (8, 2, 64, 8, [(0, 33), (31, 2), (200, 1)], None, None, 0, 0.0, True),
+    (6, 2, 96, 16, [(300, 1), (0, 17), (7, 50)], 24, None, 5, 0.0, True),
+    (16, 4, 128, 16, [(205, 1), (0, 70), (1000, 9)], None, None, 0, 50.0, False),
+    (16, 4, 128, 16, [(205, 1), (409, 1), (614, 1)], 64, None, 16, 30.0, True),
+    (8, 2, 128, 32, [(0, 130), (90, 40)], None, 48, 0, 0.0, True),
+    (8, 2, 128, 16, [(0, 130), (90, 40)], None, 48, 20, 0.0, False),
+    (16, 1, 256, 16, [(10, 3), (255, 1), (0, 40)], 100, None, 0, 0.0, True),
+    (40, 2, 64, 16, [(37, 1), (0, 9)], None, None, 0, 0.0, False),                  # more than 16 rows for one token
+]
+
+
+def paged(case, seed=3):
+    nq, nkv, d, page, reqs = case[:5]
+    g = torch.Generator().manual_seed(seed)
+    ks, vs = ([torch.randn(c + n, nkv, d, generator=g) for c, n in reqs] for _ in range(2))
+    qs = [torch.randn(n, nq, d, generator=g) for _, n in reqs]
+    return ks, vs, qs, build_paged(ks, vs, page)
+
+
+def run_kernel(case, qs, k_pages, v_pages, tables, sinks, splits=1):
+    from jax_vllm_amd.parts.attention_backend import f32_work_items
+
+    nq, nkv, d, _, reqs, window, chunk, keep, cap, _ = case
+    lens, ctx = [n for _, n in reqs], [c for c, _ in reqs]
+    items = f32_work_items(lens, ctx, nq // nkv, K().attn_f32_rows())
+    total, stride = sum(lens), (nq + 2 * nkv) * d
+    buf = torch.zeros(total, stride)
+    buf[:, :nq * d] = torch.cat(qs).reshape(total, nq * d)
+    cu = torch.tensor([0] + lens).cumsum(0).int()
+    out = torch.full((total, nq * d), float("nan")).cuda()
+    K().attn_f32(out, buf.cuda(), stride, k_pages.cuda(), v_pages.cuda(), tables.cuda(), cu.cuda(), torch.tensor(ctx).int().cuda(),
+                 torch.tensor(items).int().cuda(), len(items), nq, nkv, d, d ** -0.5, K().key_window(window, chunk), splits,
+                 torch.full((K().attn_f32_part_floats(len(items), nkv, splits, d),), float("nan")).cuda(), sinks=None if sinks is None else sinks.cuda(), cap=cap, keep=keep)
+    return out.cpu().view(total, nq, d)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("splits", [1, 2, 9])          # 9: blocks without a key among them
+@pytest.mark.parametrize("case", CASES, ids=[f"h{c[0]}g{c[1]}d{c[2]}p{c[3]}w{c[5]}c{c[6]}k{c[7]}" for c in CASES])
+def test_attention_f32(case, splits):
+    nq, nkv, d, _, reqs, window, chunk, keep, cap, with_sinks = case
+    ks, vs, qs, (k_pages, v_pages, tables) = paged(case)
+    sinks = torch.linspace(-1.0, 2.0, nq) if with_sinks else None
+    out = run_kernel(case, qs, k_pages, v_pages, tables, sinks, splits)
+    want = torch.cat([reference(q, k, v, torch.arange(c, c + n), d ** -0.5, window, chunk, keep, cap, sinks)
+                      for q, k, v, (c, n) in zip(qs, ks, vs, reqs)])
+    # sums over d and over the keys in float, the scores' error enters the exponent: a few 2^-24 sqrt(d) of scores up to ~5
+    torch.testing.assert_close(out.double(), want, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,page", [(32, 4), (128, 16)])
+def test_a_value_that_is_not_finite_stays_with_those_who_see_it(d, page):
+    """A key in the middle of a tile holds infinity or NaN: rows before it (and rows whose window has passed it) are as if it
+    were not there, and stale slots behind the last key are nobody's."""
+    case = (4, 2, d, page, [(0, 40), (3, 21)], 12, None, 0, 0.0, False)
+    ks, vs, qs, (k_pages, v_pages, tables) = paged(case)
+    clean = run_kernel(case, qs, k_pages, v_pages, tables, None)
+    bad = 21                                                            # of the first request
+    k_pages, v_pages = k_pages.clone(), v_pages.clone()
+    slot = int(tables[0, bad // page])
+    v_pages[slot, :, :, bad % page] = float("nan")
+    k_pages[slot, :, bad % page] = float("inf")
+    last = int(tables[1, 23 // page])
+    v_pages[last, :, :, 23 % page + 1:] = float("inf")                  # behind the second request's last key
+    out = run_kernel(case, qs, k_pages, v_pages, tables, None)
+    sees = torch.zeros(out.shape[0], dtype=torch.bool)
+    sees[bad:bad + 12] = True
+    assert torch.isnan(out[sees]).all()
+    torch.testing.assert_close(out[~sees], clean[~sees], rtol=1e-6, atol=1e-6)      # one key walked by hand instead of by product
+
+
+def test_f32_work_items_hold_every_row_once():
+    from jax_vllm_amd.parts.attention_backend import f32_work_items
+
+    lens, ctx, g = [1, 40, 3, 16], [900, 0, 12, 64], 3
+    for rows in (16, 32):
+        items = f32_work_items(lens, ctx, g, rows)
+        covered = sorted((r, m) for r, m0 in items for m in range(m0, min(m0 + rows, lens[r] * g)))
+        assert covered == [(r, m) for r, n in enumerate(lens) for m in range(n * g)]
+        assert items[0][0] == 0                                          # the request with the most keys first
