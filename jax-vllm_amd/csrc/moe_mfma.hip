@@ -1,12 +1,18 @@
 // The two grouped products of routed experts on the matrix cores (bfloat16, float accumulation); the
-// grouping they read (tiles of 64 or 128 rows of one expert each) is made by moe.hip.
+// grouping they read (tiles of 64 or 128 rows of one expert each) is made by moe.hip.  And the router's logits.
 //
-// A block of 4 waves takes one tile of (token, choice) rows against 64 rows of the expert's weight and
-// walks the inner size in chunks of 64: the rows of x (gathered by token) and of W go through LDS, the
-// next chunk's global loads are asked for (unconditionally, clamped) before the current chunk is
-// multiplied.  v_mfma_f32_16x16x32_bf16 with A = 16 rows of W (wave w owns rows 16 w .. 16 w + 15 of the
-// tile), B = 16 rows of x: the accumulator of row tile mt holds y^T[n = 4 lc + e][m = 16 mt + li].
-// Each output row is a sum over the inner size in a fixed order, whatever else is in the step.
+// A block takes one tile of (token, choice) rows against TW rows of the expert's weight and walks the inner size in
+// chunks of 64: the rows of x (gathered by token) and of W go straight from memory into LDS, chunks ahead of their use;
+// v_mfma_f32_32x32x16_bf16 with A = 32 rows of x, B = 32 rows of W, a wave 64 (or 32) rows of x against 64 of W.
+// Each output is a sum over the inner size in ascending steps of 16, whatever else is in the step.
+//
+// Bound by what a compute unit draws from its L2, 40..45 bytes a nanosecond as in every product of this kind here: a tile of
+// 128 rows needs 1.5 bytes of operands where 256 x 256 would need 1, but an expert of a prompt has few rows, and half the
+// tiles are not full.  2,048 tokens, gate/up + down, microseconds (before: one buffer through registers, 64 rows of W):
+//   32 experts x 512, 4 chosen, width 2,048:    85 + 50   (96 + 76)
+//   64 experts x 1,024, 8 chosen, width 4,096: 478 + 296  (570 + 439)
+// Not better: 128 rows of W and two blocks a unit 83 + 50, 495 + 300; a wave for 64 x 128 (one a SIMD: nothing overlaps its own
+// reads) 134 + 71, 626 + 358; a register copy of row tiles to skip empty ones 87 + 56.
 //   MM_GATED:  z[pos] = act(w g) * (w u), g = Wg[e] x[token], u = Wu[e] x[token]    (bf16)
 //   MM_PLAIN:  z[pos] = act(w u), u = Wu[e] x[token]: experts without a gate        (bf16)
 //   MM_DOWN:   y[kk][token] = (Wd[e] z[pos]) * w_out                                (float)
@@ -14,148 +20,161 @@
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 enum { MM_DOWN = 0, MM_GATED = 1, MM_PLAIN = 2 };
 
-#define MM_T 64            // rows of a tile, rows of W of a block, columns of a chunk
-#define MM_S 80            // LDS row length: 40 dwords, 8 mod 16: 16-byte reads of 16 rows are conflict-free
+#define MM_K 64            // columns of a chunk: a row of it is 128 bytes, 8 pieces of 16
 
-// MT: row tiles of 16 a block takes (a tile of the grouping has 16 MT rows).  Without a grouping
-// (tile_expert null) the product is a plain one: rows in order, one weight matrix, float output [rows, N].
-template <int MODE, int MT>
-__global__ void __launch_bounds__(256)
+// What a lane reads for columns behind the inner size, of x and of W alike.
+static __device__ __attribute__((aligned(16))) const unsigned mm_zeros[4] = {0, 0, 0, 0};
+
+// TM: rows of a tile of the grouping, 64 or 128; TW: rows of W of a block (gated: half of them of each matrix).  Without a grouping (tile_expert null) the product is a plain one: rows
+// in order, one weight matrix, float output [rows, N].
+template <int MODE, int TM, int TW, int BUFS>
+__global__ void __launch_bounds__(2 * TW, TW == 128 ? 2 : 1)
 moe_mfma_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, const bf16_t* __restrict__ W0,
                 const bf16_t* __restrict__ W1, const int* __restrict__ meta, const int* __restrict__ offsets,
                 const int* __restrict__ tile_expert, const int* __restrict__ tile_row0, const int* __restrict__ order,
                 const float* __restrict__ weights, int top, int n_tokens, int K, int N, JvAct act, int use_weight) {
-  constexpr int TM = 16 * MT;
+  constexpr int MT = TM / 64;               // 32-row tiles of x of a wave
   constexpr bool GATED = MODE == MM_GATED, BY_TOKEN = MODE != MM_DOWN;
+  constexpr int WAVES = TW / 32;                    // 2 along the rows of x, the others 64 rows of W each
+  constexpr int NB = GATED ? TW / 2 : TW;           // output columns of a block
+  constexpr int XI = TM / 8 / WAVES, WI = TW / 8 / WAVES;      // instructions a wave brings of a chunk, each 8 rows of 128 bytes
+  constexpr int BUF = (TM + TW) * MM_K;             // elements of a buffer: rows of x, then rows of W
+  static_assert(XI % 2 == 0 && WI % 2 == 0, "see col");
   // Blocks b, b + 8, b + 16, ... run on one XCD (with an L2 of its own): each of the 8 takes one run of the (tile, rows of W)
   // pairs, rows of W fastest, so the rows of x of a tile and the weights of an expert are read into one L2 and used there.
-  const int per_tile = (N + MM_T - 1) / MM_T;
-  const int live = (tile_expert ? meta[0] : (n_tokens + TM - 1) / TM) * per_tile, chunk = (live + 7) / 8;
+  const int per_tile = (N + NB - 1) / NB;
+  const int live = meta[0] * per_tile, chunk = (live + 7) / 8;
   const int pair = ((int)blockIdx.x & 7) * chunk + ((int)blockIdx.x >> 3);
   if (((int)blockIdx.x >> 3) >= chunk || pair >= live) return;
   const int tile = pair / per_tile;
-  __shared__ __attribute__((aligned(16))) bf16_t xs[TM * MM_S];
-  __shared__ __attribute__((aligned(16))) bf16_t w0s[MM_T * MM_S];
-  __shared__ __attribute__((aligned(16))) bf16_t w1s[GATED ? MM_T * MM_S : 8];
-  __shared__ int ent[TM];
-  const int e = tile_expert ? tile_expert[tile] : 0, row0 = tile_expert ? tile_row0[tile] : tile * TM;
-  const int rows = min(TM, (tile_expert ? offsets[e + 1] : n_tokens) - row0);
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, lc = lane >> 4;
-  const int n0 = (pair - tile * per_tile) * MM_T;
-  if (tid < TM) ent[tid] = tile_expert ? order[row0 + min(tid, rows - 1)] : row0 + min(tid, rows - 1);   // rows beyond the tile repeat its last row
+  __shared__ __attribute__((aligned(1024))) bf16_t bufs[BUFS * BUF];
+  __shared__ int from[TM];                  // a row's row of x
+  __shared__ long long to[TM];              // where its results go
+  __shared__ float wts[TM];
+  const int e = tile_expert[tile], row0 = tile_row0[tile];
+  const int rows = min(TM, offsets[e + 1] - row0);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n0 = (pair - tile * per_tile) * NB;
+  if (tid < TM) {                           // rows beyond the tile repeat its last row
+    const int s = order[row0 + min(tid, rows - 1)];
+    const int token = s / top;
+    from[tid] = BY_TOKEN ? token : row0 + min(tid, rows - 1);
+    to[tid] = (MODE == MM_DOWN ? (long long)(s - token * top) * n_tokens + token : (long long)(row0 + tid)) * N;
+    wts[tid] = use_weight ? weights[s] : 1.f;
+  }
   __syncthreads();
-  // staging: thread t brings pieces t and t + 256 of each operand: piece p = row p / 8, columns (p % 8) * 8 .. + 7
-  const int pr = tid >> 3, pc = (tid & 7) * 8;
-  constexpr int XQ = TM / 32;        // pieces of x a thread brings
-  const bf16_t* xrow[XQ];
-  const bf16_t* w0row[2];
-  const bf16_t* w1row[2];
+
+  // Loads straight into LDS: an instruction brings 8 rows, lane l row l / 8, and fills 1 KB in the order of the lanes.  Piece
+  // c of row r lies at slot c ^ ((r / 2) % 8) of its row, so that 16 lanes reading one piece of 16 rows meet 16 slots.
+  const int lr = lane >> 3;
+  const bf16_t* src[XI + WI];
+  int col[2];                               // a lane's columns in a chunk, for rows 16 i + lr and 16 i + 8 + lr
 #pragma unroll
-  for (int q = 0; q < XQ; ++q) {
-    const int r = pr + 32 * q;
-    const long long src = BY_TOKEN ? (long long)(ent[r] / top) : (long long)(row0 + min(r, rows - 1));
-    xrow[q] = a_rows + src * K;
+  for (int h = 0; h < 2; ++h) col[h] = (((lane & 7) ^ ((lr + 8 * h) >> 1)) & 7) * 8;
+#pragma unroll
+  for (int i = 0; i < XI; ++i) {
+    const int r = (wave * XI + i) * 8 + lr;
+    src[i] = a_rows + (long long)from[r] * K;
   }
 #pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const long long wr = (long long)e * N + min(n0 + pr + 32 * q, N - 1);
-    w0row[q] = W0 + wr * K;
-    w1row[q] = GATED ? W1 + wr * K : W0;
+  for (int i = 0; i < WI; ++i) {
+    const int r = (wave * WI + i) * 8 + lr;
+    // gated: rows 64 w .. + 31 of the block's W are gate rows 32 w .. + 31, the 32 behind them the same rows of up
+    const int n = GATED ? n0 + (r >> 6) * 32 + (r & 31) : n0 + r;
+    const bf16_t* w = GATED && (r & 32) ? W1 : W0;
+    src[XI + i] = w + ((long long)e * N + min(n, N - 1)) * K;
   }
-  bf16x8 rx[XQ], rw0[2], rw1[2];
-  auto fetch = [&](int k0) {
-    const int k = min(k0 + pc, K - 8);
+  auto fetch = [&](int k0, int buf) {
 #pragma unroll
-    for (int q = 0; q < XQ; ++q) rx[q] = *(const bf16x8*)(xrow[q] + k);
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      rw0[q] = *(const bf16x8*)(w0row[q] + k);
-      if (GATED) rw1[q] = *(const bf16x8*)(w1row[q] + k);
+    for (int i = 0; i < XI + WI; ++i) {
+      const int first = i < XI ? (wave * XI + i) * 8 : TM + (wave * WI + i - XI) * 8;      // the instruction's first row in the buffer
+      const int k = k0 + col[i & 1];                  // XI and WI are even: odd instructions bring the upper 8 of 16 rows
+      const bf16_t* piece = k < K ? src[i] + k : (const bf16_t*)mm_zeros;
+      const unsigned at = (unsigned)(unsigned long long)(const __attribute__((address_space(3))) void*)(bufs + buf * BUF + first * MM_K);
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(piece), "s"(at) : "memory", "m0");
     }
   };
-  const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  f32x4 acc0[MT], acc1[GATED ? MT : 1];
+
+  f32x16 acc[2][MT];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    acc0[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (GATED) acc1[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += MM_T) {
-    const bool inside = k0 + pc < K;          // a chunk's columns beyond the inner size are zeros of x
-    __syncthreads();                          // the chunk before is multiplied
+  for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int q = 0; q < XQ; ++q) *(bf16x8*)(xs + (pr + 32 * q) * MM_S + pc) = inside ? rx[q] : zero;
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int at = (pr + 32 * q) * MM_S + pc;
-      *(bf16x8*)(w0s + at) = rw0[q];
-      if (GATED) *(bf16x8*)(w1s + at) = rw1[q];
+      for (int i = 0; i < 16; ++i) acc[a][mt][i] = 0.f;
+  // wave (wm, wn): rows of x (TM / 2) wm .., rows of W 64 wn ..
+  const int wm = wave & 1, wn = wave >> 1, l32 = lane & 31, half = lane >> 5, swz = (l32 >> 1) & 7;
+  const int chunks = (K + MM_K - 1) / MM_K;
+  for (int c = 0; c < BUFS - 1 && c < chunks; ++c) fetch(c * MM_K, c);
+  for (int c = 0, buf = 0; c < chunks; ++c, buf = buf + 1 == BUFS ? 0 : buf + 1) {
+    // this wave's part of chunk c is there (loads arrive in order; those of the next BUFS - 2 chunks may be on their way)
+    if (BUFS > 2 && c + BUFS - 2 < chunks) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((BUFS - 2) * (XI + WI)) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();                                      // and everybody's, and the buffer before is no longer read
+    if (c + BUFS - 1 < chunks) fetch((c + BUFS - 1) * MM_K, buf == 0 ? BUFS - 1 : buf - 1);
+    const bf16_t* xb = bufs + buf * BUF + (wm * (TM / 2) + l32) * MM_K;
+    const bf16_t* wb = bufs + buf * BUF + (TM + wn * 64 + l32) * MM_K;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const int at = ((ks * 2 + half) ^ swz) * 8;
+      bf16x8 xf[MT], wf[2];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) xf[mt] = *(const bf16x8*)(xb + mt * 32 * MM_K + at);
+#pragma unroll
+      for (int a = 0; a < 2; ++a) wf[a] = *(const bf16x8*)(wb + a * 32 * MM_K + at);
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[a][mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[mt], wf[a], acc[a][mt], 0, 0, 0);
     }
-    __syncthreads();
-    fetch(k0 + MM_T);                         // beyond the end: the last pieces again, never used
-    __builtin_amdgcn_sched_barrier(0);
+  }
+  // a lane holds column l32 of both tiles of W, rows 8 q + 4 half + i of each tile of x
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      const int col = ks * 32 + lc * 8;
-      const bf16x8 a0 = *(const bf16x8*)(w0s + (wave * 16 + li) * MM_S + col);
-      bf16x8 a1 = zero;
-      if (GATED) a1 = *(const bf16x8*)(w1s + (wave * 16 + li) * MM_S + col);
+  for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const bf16x8 b = *(const bf16x8*)(xs + (mt * 16 + li) * MM_S + col);
-        acc0[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b, acc0[mt], 0, 0, 0);
-        if (GATED) acc1[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b, acc1[mt], 0, 0, 0);
+    for (int i = 0; i < 16; ++i) {
+      const int m = wm * (TM / 2) + mt * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
+      if (m >= rows) continue;
+      const float w = wts[m];
+      if (GATED) {
+        const int n = n0 + wn * 32 + l32;
+        if (n < N) ((bf16_t*)out)[to[m] + n] = from_f32<bf16_t>(jv_gated(act, acc[0][mt][i] * w, acc[1][mt][i] * w));
+      } else {
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          const int n = n0 + wn * 64 + a * 32 + l32;
+          if (n >= N) continue;
+          if (MODE == MM_PLAIN) ((bf16_t*)out)[to[m] + n] = from_f32<bf16_t>(jv_act(act.id, acc[a][mt][i] * w));
+          else ((float*)out)[to[m] + n] = acc[a][mt][i] * w;
+        }
       }
     }
-  }
-  const int nb = n0 + wave * 16 + lc * 4;
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int m = mt * 16 + li;
-    if (m >= rows) continue;
-    const int s = ent[m];
-    const float w = use_weight ? weights[s] : 1.f;
-    if (GATED) {
-      bf16_t* z = (bf16_t*)out + (long long)(row0 + m) * N;
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        if (nb + c < N) z[nb + c] = from_f32<bf16_t>(jv_gated(act, acc0[mt][c] * w, acc1[mt][c] * w));
-    } else if (MODE == MM_PLAIN) {
-      bf16_t* z = (bf16_t*)out + (long long)(row0 + m) * N;
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        if (nb + c < N) z[nb + c] = from_f32<bf16_t>(jv_act(act.id, acc0[mt][c] * w));
-    } else {
-      const int token = s / top, kk = s - token * top;
-      float* y = (float*)out + ((long long)kk * n_tokens + token) * N;
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        if (nb + c < N) y[nb + c] = acc0[mt][c] * w;
-    }
-  }
 }
 
-template <int MODE>
-static int launch_moe_mfma(int tile_rows, int max_tiles, hipStream_t stream, void* out, const bf16_t* a, const bf16_t* W0,
-                           const bf16_t* W1, const int* meta, const int* offsets, const int* tile_expert,
-                           const int* tile_row0, const int* order, const float* weights, int top, int n_tokens, int K,
-                           int N, JvAct act, int use_weight) {
-  const long long pairs = (long long)max_tiles * ((N + MM_T - 1) / MM_T);
+template <int MODE, int TM, int TW, int BUFS>
+static int launch_moe_tiles(int max_tiles, hipStream_t stream, void* out, const bf16_t* a, const bf16_t* W0,
+                            const bf16_t* W1, const int* meta, const int* offsets, const int* tile_expert,
+                            const int* tile_row0, const int* order, const float* weights, int top, int n_tokens, int K,
+                            int N, JvAct act, int use_weight) {
+  const int nb = MODE == MM_GATED ? TW / 2 : TW;
+  const long long pairs = (long long)max_tiles * ((N + nb - 1) / nb);
   if (pairs > 0x7ffffff0ll) return (int)hipErrorInvalidValue;
-  const dim3 grid((unsigned)(pairs + 7));
-  if (tile_rows == 128)
-    hipLaunchKernelGGL((moe_mfma_kernel<MODE, 8>), grid, dim3(256), 0, stream, out, a, W0, W1, meta, offsets, tile_expert,
-                       tile_row0, order, weights, top, n_tokens, K, N, act, use_weight);
-  else if (tile_rows == 64)
-    hipLaunchKernelGGL((moe_mfma_kernel<MODE, 4>), grid, dim3(256), 0, stream, out, a, W0, W1, meta, offsets, tile_expert,
-                       tile_row0, order, weights, top, n_tokens, K, N, act, use_weight);
-  else
-    return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL((moe_mfma_kernel<MODE, TM, TW, BUFS>), dim3((unsigned)(pairs + 7)), dim3(2 * TW), 0, stream, out, a, W0, W1,
+                     meta, offsets, tile_expert, tile_row0, order, weights, top, n_tokens, K, N, act, use_weight);
   return JV_LAUNCH_CHECK();
+}
+
+// 128 rows against 256 of W by 8 waves with two chunks on their way, 64 rows (where an expert gets so few that the stream of its
+// weights is what is waited for) against 128 by 4 waves, three blocks a compute unit.
+template <int MODE, typename... Args>
+static int launch_moe_mfma(int tile_rows, Args... args) {
+  if (tile_rows == 128) return launch_moe_tiles<MODE, 128, 256, 3>(args...);
+  if (tile_rows == 64) return launch_moe_tiles<MODE, 64, 128, 2>(args...);
+  return (int)hipErrorInvalidValue;
 }
 
 // gate/up: x [tokens, hidden], Wg, Wu [experts, ff, hidden] -> z [entries, ff] bf16 by position; tile_rows (64 or
@@ -165,7 +184,7 @@ extern "C" int jv_moe_gate_up_mfma_bf16(void* z, const void* x, const void* Wg, 
                                         const int* order, const float* weights, int max_tiles, int top, int hidden,
                                         int ff, int act, float act_limit, float act_slope, int scale_input, int tile_rows, void* stream) {
   if (max_tiles <= 0 || ff <= 0) return 0;
-  if (!(Wg ? jv_act_known(act) : jv_plain_act_known(act)) || hidden < 8 || hidden % 8 || (ff + MM_T - 1) / MM_T > 65535) return (int)hipErrorInvalidValue;
+  if (!(Wg ? jv_act_known(act) : jv_plain_act_known(act)) || hidden < 8 || hidden % 8) return (int)hipErrorInvalidValue;
   if (!Wg)
     return launch_moe_mfma<MM_PLAIN>(tile_rows, max_tiles, (hipStream_t)stream, z,
                                      (const bf16_t*)x, (const bf16_t*)Wu, nullptr, meta, offsets, tile_expert, tile_row0,
@@ -181,17 +200,73 @@ extern "C" int jv_moe_down_mfma_bf16(float* y, const void* z, const void* Wd, co
                                      const float* weights, int max_tiles, int top, int n_tokens, int hidden, int ff,
                                      int scale_output, int tile_rows, void* stream) {
   if (max_tiles <= 0 || hidden <= 0) return 0;
-  if (ff < 8 || ff % 8 || (hidden + MM_T - 1) / MM_T > 65535) return (int)hipErrorInvalidValue;
+  if (ff < 8 || ff % 8) return (int)hipErrorInvalidValue;
   return launch_moe_mfma<MM_DOWN>(tile_rows, max_tiles, (hipStream_t)stream, y,
                                 (const bf16_t*)z, (const bf16_t*)Wd, nullptr, meta, offsets, tile_expert, tile_row0, order,
                                 weights, top, n_tokens, ff, hidden, JvAct{}, scale_output);
 }
 
-// y [M, N] float = x [M, K] W[N, K]^T for bfloat16 x and W: the same kernel without a grouping (router logits
-// of many tokens).  K a multiple of 8.
+// y [M, N] float = x [M, K] W[N, K]^T for bfloat16 x and W: the router's logits of a prompt's rows, few columns over a long
+// inner size.  A block takes 16 rows of x against 16 NT rows of W; its 8 waves take an eighth of the inner size each, in
+// steps of 32 columns straight from memory into operands, and meet in LDS: the parts are added in ascending order, so a row's
+// logits do not depend on the batch.  Bound by its one round trip to memory: 2,048 rows x 32 x 2,048 7.9 us (25 as one
+// column of the tiles above, 16 blocks of 32 chunks in a row).
+template <int NT>
+__global__ void __launch_bounds__(512)
+gemm_rows_kernel(float* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, int M, int N, int K) {
+  __shared__ f32x4 red[NT][8][64];
+  const int part = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lq = lane >> 4;
+  const int m0 = blockIdx.x * 16, n0 = blockIdx.y * (16 * NT);
+  const int len = (K + 255) / 256 * 32, k_begin = part * len, k_end = min(K, k_begin + len);
+  const bf16_t* xrow = x + (long long)min(m0 + li, M - 1) * K;
+  const bf16_t* wrow[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) wrow[t] = W + (long long)min(n0 + t * 16 + li, N - 1) * K;
+  f32x4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  constexpr int U = NT > 2 ? 2 : 4;               // steps whose loads are asked for together
+  for (int k0 = k_begin; k0 < k_end; k0 += 32 * U) {
+    bf16x8 xf[U], wf[U][NT];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + u * 32 + lq * 8, at = min(k, K - 8);
+      xf[u] = *(const bf16x8*)(xrow + at);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) wf[u][t] = *(const bf16x8*)(wrow[t] + at);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool inside = k0 + u * 32 + lq * 8 < k_end;
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(inside ? wf[u][t] : zero, inside ? xf[u] : zero, acc[t], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) red[t][part][lane] = acc[t];
+  __syncthreads();
+  if (part < NT) {
+    f32x4 sum = red[part][0][lane];
+#pragma unroll
+    for (int p = 1; p < 8; ++p) sum += red[part][p][lane];
+    const int m = m0 + li, n = n0 + part * 16 + lq * 4;      // a lane holds 4 columns of a row
+    if (m < M)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (n + c < N) y[(long long)m * N + n + c] = sum[c];
+  }
+}
+
 extern "C" int jv_gemm_rows_f32out_bf16(float* y, const void* x, const void* W, int M, int N, int K, void* stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (K < 8 || K % 8 || (N + MM_T - 1) / MM_T > 65535) return (int)hipErrorInvalidValue;
-  return launch_moe_mfma<MM_DOWN>(128, (M + 127) / 128, (hipStream_t)stream, y, (const bf16_t*)x,
-                                (const bf16_t*)W, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 1, M, K, N, JvAct{}, 0);
+  const int nt = N <= 16 ? 1 : N <= 32 ? 2 : 4;
+  const dim3 grid((M + 15) / 16, (N + 16 * nt - 1) / (16 * nt));
+  if (K < 8 || K % 8 || grid.y > 65535) return (int)hipErrorInvalidValue;
+  const bf16_t *xb = (const bf16_t*)x, *wb = (const bf16_t*)W;
+  if (nt == 1) hipLaunchKernelGGL(gemm_rows_kernel<1>, grid, dim3(512), 0, (hipStream_t)stream, y, xb, wb, M, N, K);
+  else if (nt == 2) hipLaunchKernelGGL(gemm_rows_kernel<2>, grid, dim3(512), 0, (hipStream_t)stream, y, xb, wb, M, N, K);
+  else hipLaunchKernelGGL(gemm_rows_kernel<4>, grid, dim3(512), 0, (hipStream_t)stream, y, xb, wb, M, N, K);
+  return JV_LAUNCH_CHECK();
 }
