@@ -8,6 +8,7 @@ functions: a missing library raises ``KernelLibraryError``.
 from __future__ import annotations
 
 import ctypes
+import functools
 from ctypes import c_float, c_int, c_longlong, c_void_p
 
 import torch
@@ -956,16 +957,89 @@ def streaming_plan(m: int, n: int, k: int, gate_pairs: bool = False, partial_ok:
     return (0, 0, 0), 1
 
 
+STREAM_MAX_ROWS = 128
+STREAM_MODES = {"parts": 0, "rows": 1, "pairs": 2}
+
+
+@functools.lru_cache(maxsize=4096)
+def ring_plan(m: int, n: int, k: int, mode: str, cus: int = 256):
+    """How ``linear`` runs a bfloat16 product of 17 to 128 rows through ``gemm_stream``: (rows of x, rows of w, parts of the
+    inner size) of a block, or None where another way is better.  ``mode``: "parts" (the reader adds float partial
+    products), "rows", "pairs" (rows of w alternate gate and up rows).
+
+    The form with the least time by this count (all of one product's forms give it within rounding): every round of one
+    block a compute unit takes 3 us and then, a chunk of 64 columns, the longest of 0.31 us, what its units draw from
+    the L2s at 9.6 TB/s and what they draw of w from memory at 5.3 TB/s, as measured over 32 to 128 rows.
+
+    A matrix below 1 MB is no stream, and stays with the library.  Others are better, measured (microseconds here / there):
+
+    * blocks that stay with x in registers, for narrow matrices they cover: up to 32 rows and 5,120 wide (4,096 x 4,096 at
+      24 rows 10.8 / 10.0), up to 64 rows and 1,024 wide (x 4,096: 7.9 / 7.3);
+    * the library, about 11.5 us + w at 5.1 TB/s and 2 us for the activation (the count here is up to 15 % high beside
+      that), where blocks with the whole inner size cannot fill the chip (2,080 x 2,048 at 96 rows 12.9 / 11.4) or a large
+      matrix leaves a fifth of a round empty (51,200 x 5,120 at 64 rows 118 / 111)."""
+    if not SKINNY_AUTO_ROWS < m <= STREAM_MAX_ROWS or k % 64 or n % 4 or n * k < 500_000:
+        return None
+    tm = 32 if m <= 32 else 64 if m <= 64 else 128
+    if mode == "parts" and n <= (5120 if m <= 32 else 1024 if m <= 64 else 0):
+        nl = _stay_pieces(k, 4)
+        if nl is not None and (nl <= 5 or (m <= 32 and nl <= 8)):
+            return None
+    best = None
+    for tw in (32, 64, 96, 128):
+        for parts in ((4, 3, 2) if mode == "parts" else (1,)):
+            if parts > k // 64:
+                continue
+            blocks, chunks, cost = -(-n // tw) * parts, -(-(k // 64) // parts), 3.0
+            for units, rounds in ((cus, blocks // cus), (blocks % cus, 1 if blocks % cus else 0)):
+                cost += rounds * chunks * max(0.31, (tm + tw) * 128 / 40e3, units * tw * 128 / 5.3e6)
+            if best is None or cost < best[0]:
+                best = (cost, blocks, (tm, tw, parts))
+    if best is None:
+        return None
+    cost, blocks, form = best
+    if mode != "parts":
+        mb = n * k * 2e-6
+        if cost > 1.15 * (11.5 + 0.195 * mb + (2.0 if mode == "pairs" else 0.0)):
+            return None
+        if mb > 400 and blocks < 0.8 * -(-blocks // cus) * cus:
+            return None
+    return form
+
+
+def gemm_stream(x: torch.Tensor, w: torch.Tensor, form, mode: str = "rows", gate_pairs: "str | tuple | None" = None,
+                out_dtype=torch.bfloat16) -> torch.Tensor:
+    """x @ w.T for 17 to 128 rows of bfloat16 x (any up to 128 are taken) against bfloat16 w [N, K], K a multiple of 64: chunks
+    of both through a ring in LDS.  ``form``: (rows of x, rows of w, parts of the inner size) of a block, see
+    ``ring_plan``; ``mode``: "parts": float32 [parts, M, N], to be added in order; "rows": bfloat16 [M, N] (or float32, with
+    one part); "pairs" with ``gate_pairs``: bfloat16 [M, N / 2]."""
+    _dev(x, w)
+    _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "gemm_stream takes bfloat16")
+    m, k = x.shape
+    n = w.shape[0]
+    tm, tw, parts = form
+    _need(w.shape[1] == k and m <= tm, "inner sizes differ, or more rows than the form takes")
+    _need(mode in STREAM_MODES and (parts == 1 or mode == "parts") and (mode == "pairs") == bool(gate_pairs), "only partial products have parts")
+    as_float = mode == "parts" or out_dtype == torch.float32
+    _need(not (as_float and gate_pairs), "the activation's result is bfloat16")
+    shape = (parts, m, n) if mode == "parts" else (m, n // 2) if gate_pairs else (m, n)
+    y = torch.empty(shape, dtype=torch.float32 if as_float else torch.bfloat16, device=x.device)
+    _check(library.core().jv_gemm_stream_bf16(
+        _ptr(y), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), c_longlong(k), c_int(STREAM_MODES["parts" if as_float else mode]),
+        *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), c_int(tm), c_int(tw), c_int(parts), _stream()), "gemm_stream")
+    return y
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = False, gate_pairs: "str | tuple | None" = None,
            partial_max_width: int | None = PARTIAL_SUM_MAX_WIDTH):
     """x @ w.T for w stored [out, in].
 
     float32: the library's own kernel in true 32-bit (no reduced-precision matrix mode).
     bfloat16, at most 16 rows (and some shapes up to 64): a weight-streaming MFMA kernel of this
-    library (``streaming_plan``).
+    library (``streaming_plan``); 17 to 128 rows: chunks of x and w through a ring in LDS (``ring_plan``).
     bfloat16 otherwise: a plain library matrix product (hipBLASLt through torch), float accumulation.
     With ``partial_ok`` the caller takes a float32 stack [parts, M, N] of partial products as well
-    (to be added in order, as ``add_rmsnorm`` does); it is returned for narrow matrices at up to 64 rows
+    (to be added in order, as ``add_rmsnorm`` does); it is returned for narrow matrices at up to 128 rows
     (``partial_max_width``: the widest row whose parts the caller's reader adds; None: any).
     With ``gate_pairs`` (one of ``GATE_ACTIVATIONS``) the rows of w alternate gate and up rows and the
     result is act(x.w[2j]) * (x.w[2j+1]) of width N/2 (an epilogue of the streaming kernels, a kernel
@@ -978,6 +1052,15 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
         y = gemm_f32(x, w)
     else:
         _need(x.dtype == w.dtype, "x and w must have one type")
+        m, (n, k) = x.shape[0], w.shape
+        if SKINNY_AUTO_ROWS < m <= STREAM_MAX_ROWS and scale is None and w.dtype == torch.bfloat16:
+            parts_ok = partial_ok and not gate_pairs and out_dtype in (None, torch.bfloat16) and (
+                partial_max_width is None or n <= partial_max_width)
+            mode = "pairs" if gate_pairs else "parts" if parts_ok and k >= 128 else "rows"
+            form = ring_plan(m, n, k, mode, compute_units(x.device))
+            if form is not None and out_dtype in (None, torch.bfloat16, torch.float32) and x.is_contiguous() and w.is_contiguous() \
+                    and not (x.data_ptr() | w.data_ptr()) & 15 and not (gate_pairs and out_dtype == torch.float32):
+                return gemm_stream(x, w, form, mode, gate_pairs, out_dtype or torch.bfloat16)
         plan = streaming_plan(x.shape[0], w.shape[0], w.shape[1], bool(gate_pairs),
                               partial_ok and out_dtype in (None, torch.bfloat16), x.device, partial_max_width)
         _need(scale is None or (plan is not None and plan[0][0] == -2),
