@@ -1030,6 +1030,50 @@ def gemm_stream(x: torch.Tensor, w: torch.Tensor, form, mode: str = "rows", gate
     return y
 
 
+SHARES_MAX_ROWS = 1024
+_SHARES_TILES = {(128, 128): 0.6, (256, 128): 0.9, (256, 256): 1.6}      # rows of x, rows of w: microseconds a chunk of 64 columns
+
+
+def shares_plan(m: int, n: int, k: int, cus: int = 256):
+    """How ``linear`` runs a bfloat16 product of 129 to 1,024 rows whose reader adds partial products through
+    ``gemm_shares``: (rows of x, rows of w of a tile, parts of the inner size), or None where the library is better.
+
+    By a count of both, in microseconds, that meets what 160 to 1,024 rows against 2,048 x 2,048 up to 4,096 x 12,288 take
+    within a tenth.  Here: 5, then every round of one tile a compute unit the chunks of a part (a round that leaves units
+    idle is faster, by up to a fifth), then the partial products, written at 6 TB/s and read at 5.  The library:
+    3 + k (0.0036 + 1.32e-9 m n).  300 rows against 4,096 x 12,288: 48 / 70, against 4,096 x 4,096 20 / 26; 1,525 rows
+    140 and 9 for the parts / 147."""
+    if not STREAM_MAX_ROWS < m <= SHARES_MAX_ROWS or k % 64 or n % 4 or n * k < 500_000:
+        return None
+    best = None
+    for (tm, tw), chunk in _SHARES_TILES.items():
+        for parts in (2, 3, 4):
+            if parts > k // 64:
+                continue
+            blocks = -(-m // tm) * -(-n // tw) * parts
+            full, rest = divmod(blocks, cus)
+            rounds = full + (max(0.8, rest / cus) if rest else 0.0)
+            cost = 5.0 + rounds * -(-(k // 64) // parts) * chunk + m * n * (parts * 4 / 6e6 + (parts * 4 - 2) / 5e6)
+            if best is None or cost < best[0]:
+                best = (cost, (tm, tw, parts))
+    return best[1] if best is not None and best[0] < 3.0 + k * (0.0036 + 1.32e-9 * m * n) else None
+
+
+def gemm_shares(x: torch.Tensor, w: torch.Tensor, form) -> torch.Tensor:
+    """x @ w.T for bfloat16 x [M, K] and w [N, K], K a multiple of 64, as float32 partial products [parts, M, N] to be added in
+    order.  ``form``: (rows of x, rows of w of a tile, parts), see ``shares_plan``."""
+    _dev(x, w)
+    _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "gemm_shares takes bfloat16")
+    m, k = x.shape
+    n = w.shape[0]
+    tm, tw, parts = form
+    _need(w.shape[1] == k, "inner sizes differ")
+    y = torch.empty((parts, m, n), dtype=torch.float32, device=x.device)
+    _check(library.core().jv_gemm_shares_bf16(_ptr(y), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), c_int(tm), c_int(tw),
+                                              c_int(parts), _stream()), "gemm_shares")
+    return y
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = False, gate_pairs: "str | tuple | None" = None,
            partial_max_width: int | None = PARTIAL_SUM_MAX_WIDTH):
     """x @ w.T for w stored [out, in].
@@ -1039,7 +1083,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
     library (``streaming_plan``); 17 to 128 rows: chunks of x and w through a ring in LDS (``ring_plan``).
     bfloat16 otherwise: a plain library matrix product (hipBLASLt through torch), float accumulation.
     With ``partial_ok`` the caller takes a float32 stack [parts, M, N] of partial products as well
-    (to be added in order, as ``add_rmsnorm`` does); it is returned for narrow matrices at up to 128 rows
+    (to be added in order, as ``add_rmsnorm`` does); it is returned for narrow matrices at up to 128 rows, and up to 1,024
+    where the inner size is long (``shares_plan``)
     (``partial_max_width``: the widest row whose parts the caller's reader adds; None: any).
     With ``gate_pairs`` (one of ``GATE_ACTIVATIONS``) the rows of w alternate gate and up rows and the
     result is act(x.w[2j]) * (x.w[2j+1]) of width N/2 (an epilogue of the streaming kernels, a kernel
@@ -1061,6 +1106,11 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
             if form is not None and out_dtype in (None, torch.bfloat16, torch.float32) and x.is_contiguous() and w.is_contiguous() \
                     and not (x.data_ptr() | w.data_ptr()) & 15 and not (gate_pairs and out_dtype == torch.float32):
                 return gemm_stream(x, w, form, mode, gate_pairs, out_dtype or torch.bfloat16)
+        elif m > STREAM_MAX_ROWS and partial_ok and not gate_pairs and scale is None and w.dtype == torch.bfloat16 \
+                and out_dtype in (None, torch.bfloat16) and partial_max_width is not None and n <= partial_max_width:
+            form = shares_plan(m, n, k, compute_units(x.device))
+            if form is not None and x.is_contiguous() and w.is_contiguous() and not (x.data_ptr() | w.data_ptr()) & 15:
+                return gemm_shares(x, w, form)
         plan = streaming_plan(x.shape[0], w.shape[0], w.shape[1], bool(gate_pairs),
                               partial_ok and out_dtype in (None, torch.bfloat16), x.device, partial_max_width)
         _need(scale is None or (plan is not None and plan[0][0] == -2),
