@@ -20,8 +20,8 @@
 // row m = query_index * G + head_in_group, G = q heads per kv head; any G works.
 //   prefill kernel: 128 rows per block (4 waves x 2 row tiles of 16; 64 rows for heads above 128), K/V tiles of 64 keys staged
 //                   in LDS and shared by the 4 waves; causal limit and window per row.  Head sizes that are
-//                   multiples of 32 up to 128 have a kernel of their own instead (32x32x16 products, one tile
-//                   of 32 rows per wave, tiles straight from global memory into LDS): see JV_PREFILL32.
+//                   multiples of 32 up to 128 have a kernel of their own instead, 256 besides (32x32x16 products,
+//                   one tile of 32 rows per wave, tiles straight from global memory into LDS): see JV_PREFILL32.
 //   decode kernel:  one query per request; each of the 4 waves streams its own 32-key tiles
 //                   straight from global memory into MFMA operands (no LDS), the waves'
 //                   partial (max, sum, acc) are merged in LDS; with num_splits > 1 several
@@ -33,8 +33,11 @@
 #error "compile with -DJV_HEAD_DIM=<head size>"
 #endif
 static_assert(JV_HEAD_DIM % 16 == 0 && JV_HEAD_DIM >= 16 && JV_HEAD_DIM <= 256, "head size");
-#if JV_HEAD_DIM % 32 == 0 && JV_HEAD_DIM <= 128
-#define JV_PREFILL32 1   // the prefill kernel with 32-row tiles is built, the one with 16-row tiles is not
+#if JV_HEAD_DIM % 32 == 0 && (JV_HEAD_DIM <= 128 || JV_HEAD_DIM == 256)
+#define JV_PREFILL32 1   // the prefill kernel with 32-row tiles is built
+#endif
+#if !defined(JV_PREFILL32) || JV_HEAD_DIM == 256
+#define JV_PREFILL16 1   // the one with 16-row tiles is built
 #endif
 
 constexpr int D = JV_HEAD_DIM;
@@ -126,7 +129,7 @@ constexpr int NO_GAP = 0x7fffffff;
 #else
 #define PREFILL_OCCUPANCY
 #endif
-#ifndef JV_PREFILL32
+#ifdef JV_PREFILL16
 // PAGES: 1 = the page size is 8, 16, 32 or 64 (pages tile the 64 keys: a thread's slot in its
 // page is the same in every tile), 2 = a larger power of two, 0 = any other multiple of 8.
 // MORE: capped scores and kept first keys (AttnArgs) are looked at.
@@ -525,10 +528,13 @@ __global__ void __launch_bounds__(256) PREFILL_OCCUPANCY attn_prefill_kernel(Att
   }
 }
 
-#endif  // !JV_PREFILL32
+#endif  // JV_PREFILL16
 
 // ------------------------------------------------------------------------------------ prefill, 32-row tiles
-// Head sizes that are multiples of 32 up to 128 take this kernel.  It reads the same work items
+// Head sizes that are multiples of 32 up to 128 take this kernel, and 256 where the prompts fill the chip or see many keys
+// (one wave a SIMD then; half the LDS reads a row of the 16-row tiles: 16 heads over one kv head, 2,048 tokens with a window of
+// 1,024: 73 against 107 us, 8 kv heads and 8,192 tokens 772 against 1,414, 512 tokens after 4,000 183 against 200; where it
+// starts up in vain: 300 tokens 26 against 20).  It reads the same work items
 // (two groups of 64 rows) but gives every wave ONE tile of 32 rows (waves 0, 1: first group,
 // waves 2, 3: second group) and multiplies with v_mfma_f32_32x32x16_bf16: a 16-byte fragment of K
 // or V^T read from LDS then feeds a product of 32 cycles, twice as much as with 16x16x32 tiles
@@ -566,7 +572,7 @@ constexpr bool KB_ADDS = (32 * CPK / 16) % 16 == 0;   // the second key block's 
 __device__ __forceinline__ int swizzle(int q) { return q ^ ((q >> 4) & 15); }   // chunk index -> chunk position
 
 template <int PAGES, bool MORE>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) attn_prefill32_kernel(AttnArgs p) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1, D <= 128 ? 2 : 1))) attn_prefill32_kernel(AttnArgs p) {
   __shared__ __attribute__((aligned(16))) bf16_t Ks[2][BN * D];
   __shared__ __attribute__((aligned(16))) bf16_t Vs[2][D * BN];
   // FAST: pages of 16 keys and a head size that is a power of two.  Every load instruction of a wave
@@ -1154,7 +1160,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 
 // the host's plan: rows per group, and groups a work item may name
 extern "C" int jv_attn_prefill_group_rows() { return GROUP_ROWS; }
+#ifdef JV_PREFILL32
+extern "C" int jv_attn_prefill_groups_per_item() { return 2; }
+#else
 extern "C" int jv_attn_prefill_groups_per_item() { return RT; }
+#endif
 // 1: each group of a work item has waves of its own (pair groups that see the same keys); 0: every wave
 // takes rows of both groups (pair a light group with a heavy one)
 #ifdef JV_PREFILL32
@@ -1481,11 +1491,12 @@ extern "C" int jv_attn_head_dim() { return D; }
 extern "C" int jv_attn_decode_table_entries() { return DEC_TBL_MAX; }
 extern "C" int jv_attn_decode_tile_keys() { return BND; }
 
+// one_group: the items name one group each; where both kernels are built, the one with 16-row tiles takes them.
 extern "C" int jv_attn_prefill(void* out, const void* q, long long q_row_stride, const void* k_pages,
                                const void* v_pages, const int* block_tables, int table_stride,
                                const int* cu_seqlens, const int* context_lens, const int* work,
                                int n_work, int page_size, int nq, int nkv, float scale, int window,
-                               const float* sinks, float cap, int keep, void* stream) {
+                               const float* sinks, float cap, int keep, int one_group, void* stream) {
   if (n_work <= 0) return 0;
   AttnArgs a{};
   a.sinks = sinks;
@@ -1501,20 +1512,21 @@ extern "C" int jv_attn_prefill(void* out, const void* q, long long q_row_stride,
   if ((long long)nkv * page_size * D >= (1ll << 31)) return (int)hipErrorInvalidValue;   // offsets inside a page are 32-bit
   if ((long long)n_work * nkv >= (1ll << 31)) return (int)hipErrorInvalidValue;
   const int mode = (a.page_shift >= 3 && a.page_shift <= 6) ? 1 : (a.page_shift > 6 ? 2 : 0);
-#ifdef JV_PREFILL32
   constexpr bool pow2 = (D & (D - 1)) == 0;
   auto pick = [&](auto m) -> void (*)(AttnArgs) {
     constexpr bool M = decltype(m)::value;
+#ifdef JV_PREFILL16
+#ifdef JV_PREFILL32
+    if (one_group)
+#endif
+      return mode == 1 ? attn_prefill_kernel<1, M> : (mode == 2 ? attn_prefill_kernel<2, M> : attn_prefill_kernel<0, M>);
+#endif
+#ifdef JV_PREFILL32
     return (page_size == 16 && pow2) ? attn_prefill32_kernel<pow2 ? 16 : 1, M>
            : mode == 1 ? attn_prefill32_kernel<1, M>
            : mode == 2 ? attn_prefill32_kernel<2, M> : attn_prefill32_kernel<0, M>;
-  };
-#else
-  auto pick = [&](auto m) -> void (*)(AttnArgs) {
-    constexpr bool M = decltype(m)::value;
-    return mode == 1 ? attn_prefill_kernel<1, M> : (mode == 2 ? attn_prefill_kernel<2, M> : attn_prefill_kernel<0, M>);
-  };
 #endif
+  };
   void (*kernel)(AttnArgs) = more ? pick(std::true_type{}) : pick(std::false_type{});
   hipLaunchKernelGGL(kernel, dim3(n_work * nkv), dim3(256), 0, (hipStream_t)stream, a);
   return JV_LAUNCH_CHECK();

@@ -1168,15 +1168,15 @@ MFMA_ATTENTION_MAX_HEAD_DIM = 256
 def attn_prefill_geometry(head_dim: int) -> tuple[int, int]:
     """(rows of a group, groups a work item of the prefill kernel may name).  A row is a (query,
     head-in-group) pair."""
-    return 64, (2 if head_dim <= 128 else 1)
+    return 64, (2 if head_dim <= 128 or head_dim == 256 else 1)
 
 
 def attn_prefill_waves_split(head_dim: int) -> bool:
-    """Whether each group of a work item has waves of its own (head sizes 32, 64, 96, 128: two waves
+    """Whether each group of a work item has waves of its own (head sizes 32, 64, 96, 128, 256: two waves
     of 32 rows per group), so that a block is busy only while both groups see keys: neighbouring
     groups belong together.  Otherwise each of the 4 waves takes 16 rows of every group, and pairing
     a light group with a heavy one evens out the blocks."""
-    return head_dim % 32 == 0 and head_dim <= 128
+    return head_dim % 32 == 0 and (head_dim <= 128 or head_dim == 256)
 
 
 _checked_attention_libraries = set()
@@ -1234,13 +1234,13 @@ def _sinks_ok(sinks, nq: int) -> None:
 
 
 def attn_prefill_mfma(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_seqlens, context_lens, work, n_work,
-                      nq, nkv, head_dim, scale, window=0, sinks=None, cap: float = 0.0, keep: int = 0) -> None:
+                      nq, nkv, head_dim, scale, window=0, sinks=None, cap: float = 0.0, keep: int = 0, one_group: bool = False) -> None:
     """Causal attention of prompt portions.  ``work`` is int32 [n_work, 3]: (request index, first row
     of a group, first row of a second group of the same request or -1), see ``attn_prefill_geometry``;
     every row of every request must be in exactly one group.  ``window``: see ``key_window``.  Pairing a group that sees many keys with
     one that sees few gives all blocks the same amount of work.  ``sinks`` (float32 [nq]): exp(sinks[h]) joins every
     row's softmax denominator (a term without key and value, not scaled).  ``cap``, ``keep``: as for
-    ``paged_attention_generic``."""
+    ``paged_attention_generic``.  ``one_group``: no item names a second group (head size 256 then has 16 rows a wave instead of 32)."""
     _sinks_ok(sinks, nq)
     page_size = _attn_common(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_seqlens, context_lens, work,
                              nq, nkv, head_dim)
@@ -1250,7 +1250,7 @@ def attn_prefill_mfma(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_s
         lib.jv_attn_prefill(_ptr(out), _ptr(q), c_longlong(q_row_stride), _ptr(k_pages), _ptr(v_pages),
                             _ptr(block_tables), c_int(block_tables.shape[1]), _ptr(cu_seqlens), _ptr(context_lens),
                             _ptr(work), c_int(n_work), c_int(page_size), c_int(nq), c_int(nkv), c_float(scale),
-                            c_int(window or 0), _ptr(sinks), c_float(cap), c_int(keep if window else 0), _stream()),
+                            c_int(window or 0), _ptr(sinks), c_float(cap), c_int(keep if window else 0), c_int(one_group), _stream()),
         "attn_prefill_mfma",
     )
 

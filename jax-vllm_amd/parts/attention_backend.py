@@ -35,6 +35,7 @@ class MfmaPlan:
     n_decode: int
     num_splits: int
     scratch: Optional[torch.Tensor]
+    one_group: bool = False                # prefill items of one group, 16 rows a wave, where the kernel has both forms
 
 
 def keys_seen(kv_len: int, window: int, keep: int = 0) -> int:
@@ -122,16 +123,30 @@ def prefill_item_shape(rows: int, nkv: int, group_rows: int, kernel_groups: int,
     return kernel_groups, blocks <= RESIDENT_BLOCKS * compute_units
 
 
+def few_rows_of_256(rows: int, keys: int, group_rows: int, compute_units: int) -> bool:
+    """Whether a step's prompt portions at head size 256 take items of one group (16 rows a wave) instead of two (32): while
+    those give no more than a quarter of the compute units a second block, and nobody sees 2,048 keys.  An item of two groups takes about 13 us and 2.6
+    for every 64 keys, one of one group 6 and 2.85, or twice that beside another (measured: 300 tokens of 16 heads over one
+    20 / 26 us, 1,200 in two prompts 38 / 43, 1,024 tokens over 8 kv heads
+    49 / 50, 2,048 over 2 95 / 90, 2,048 over one with a window of 1,024 107 / 73, 512 after 4,000 200 / 183)."""
+    return 4 * -(-rows // group_rows) <= 5 * compute_units and keys < 2048
+
+
 def plan_mfma(ctx, nq: int, nkv: int, head_dim: int, window: int, device, keep: int = 0) -> MfmaPlan:
     g = nq // nkv
     group_rows, kernel_groups = K.attn_prefill_geometry(head_dim)
     rows = sum(ql * g for ql in ctx.q_lens_host if ql > 1)
     groups_per_item, balance = prefill_item_shape(rows, nkv, group_rows, kernel_groups, K.compute_units(device),
                                                   K.attn_prefill_waves_split(head_dim))
+    cus = K.compute_units(device)
+    one_group = head_dim == 256 and few_rows_of_256(
+        rows * nkv, max([keys_seen(cl + ql, window, keep) for ql, cl in zip(ctx.q_lens_host, ctx.context_lens_host) if ql > 1],
+                        default=0), group_rows, cus)
+    if one_group:
+        groups_per_item, balance = 1, False
     prefill = prefill_work_items(ctx.q_lens_host, ctx.context_lens_host, g, window, group_rows, groups_per_item,
                                  balance=balance, keep=keep)
-    cus = K.compute_units(device)
-    if cus < len(prefill) * nkv <= RESIDENT_BLOCKS * cus:
+    if cus < len(prefill) * nkv <= RESIDENT_BLOCKS * cus and head_dim != 256:      # 256: one block a unit, or fewer blocks
         prefill = pair_up_resident_items(prefill, cus // nkv)
     decode = [r for r, ql in enumerate(ctx.q_lens_host) if ql == 1]
     max_kv_decode = max([ctx.context_lens_host[r] + 1 for r in decode], default=1)
@@ -148,7 +163,7 @@ def plan_mfma(ctx, nq: int, nkv: int, head_dim: int, window: int, device, keep: 
         scratch = torch.empty(K.attn_decode_scratch_floats(len(decode), nq, splits, head_dim),
                               dtype=torch.float32, device=device)
     return MfmaPlan(dev[: 3 * n_pre] if n_pre else None, n_pre,
-                    dev[3 * n_pre:] if decode and not decode_only else None, len(decode), splits, scratch)
+                    dev[3 * n_pre:] if decode and not decode_only else None, len(decode), splits, scratch, one_group)
 
 
 @dataclass
@@ -207,7 +222,7 @@ def run(att, out, qkv, ctx, mem) -> None:
     if plan.n_prefill:
         K.attn_prefill_mfma(out, qkv, q_row_stride, mem.pages["k"], mem.pages["v"], tables, ctx.cu_seqlens,
                             ctx.context_lens, plan.prefill_work, plan.n_prefill, att.nq, att.nkv, att.d, att.scale,
-                            window, sinks=sinks, cap=cap, keep=keep)
+                            window, sinks=sinks, cap=cap, keep=keep, one_group=plan.one_group)
     if plan.n_decode:
         K.attn_decode_mfma(out, qkv, q_row_stride, mem.pages["k"], mem.pages["v"], tables, ctx.cu_seqlens,
                            ctx.context_lens, plan.decode_work, plan.n_decode, att.nq, att.nkv, att.d, att.scale,

@@ -1,0 +1,38 @@
+"""Prefill attention at head size 256 in its two forms (16 and 32 rows a wave): the rule between them, and both against float64."""
+import math
+
+import pytest
+import torch
+
+from jax_vllm_amd.parts.attention_backend import few_rows_of_256
+
+from .test_kernels_gpu import K, _mfma_inputs, _mfma_reference, _prefill_work
+
+
+def test_the_rule():
+    assert few_rows_of_256(300 * 16, 300, 64, 256) and few_rows_of_256(320 * 64, 2047, 64, 256)
+    assert not few_rows_of_256(320 * 64 + 1, 300, 64, 256) and not few_rows_of_256(64, 2048, 64, 256)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("plan", ["single", "planner", "far", "one_group"])
+@pytest.mark.parametrize("case", [
+    # nq, nkv, page_size, (context, tokens), window
+    (4, 2, 16, [(0, 1), (0, 64), (5, 131)], None),
+    (16, 1, 16, [(0, 70), (300, 9)], 100),
+    (6, 2, 8, [(0, 65), (63, 33)], None),           # 3 heads a group, pages of 8
+    (4, 1, 64, [(130, 100)], 64),
+    (4, 4, 24, [(0, 77), (40, 64)], None),          # pages that are no power of two
+    (2, 1, 128, [(200, 130)], None),                # pages larger than a key tile
+    (8, 1, 16, [(1900, 40)], 1024),
+])
+def test_both_forms(case, plan):
+    nq, nkv, page_size, reqs, window = case
+    d, one = 256, plan == "one_group"
+    qs, ks, vs, dev = _mfma_inputs(nq, nkv, d, page_size, reqs)
+    work, n_work = _prefill_work(reqs, nq // nkv, d, window, "single" if one else plan)
+    out = torch.full((dev["n"], nq * d), float("nan"), dtype=torch.bfloat16).cuda()
+    K().attn_prefill_mfma(out, dev["q"], dev["stride"], dev["k_pages"], dev["v_pages"], dev["tables"], dev["cu"], dev["ctx"],
+                          work, n_work, nq, nkv, d, 1.0 / math.sqrt(d), window or 0, one_group=one)
+    ref = _mfma_reference(qs, ks, vs, reqs, 1.0 / math.sqrt(d), window, nq, d)
+    torch.testing.assert_close(out.double().cpu(), ref, rtol=2e-2, atol=2e-2)       # probabilities and results in 8 bits of fraction
