@@ -1093,11 +1093,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 1
     if (j0 + BN > kv_end) fix_tail(j0, 0);
     __syncthreads();
     if (wave_live) tile_qk(sa, Ks[0]);
+    // The first turn asks for K(2) where K(0) is, so every wave must have read K(0): the later turns' reads end at their barrier,
+    // these have none (and a wave without rows would ask at once).  The same decision in every thread.
+    if (j2 < kv_end) __syncthreads();
     // one turn: tile t (scores in sc, K and V in buffers b), tile t + 1 (scores into sn, K in buffer b ^ 1)
     auto turn = [&](f32x16 (&sc)[2], f32x16 (&sn)[2], int b) {
       const bool has2 = j2 < kv_end;
       fetch_v(b ^ 1, pga);                            // V(t+1) where V(t-1) was
-      if (has2) fetch_k(b, pgb);                      // K(t+2) where K(t) was: its scores were made in the last turn
+      if (has2) fetch_k(b, pgb);                      // K(t+2) where K(t) was: its scores were made before the last barrier
       const int j3 = has2 ? next_tile(j2) : j2;
 #pragma unroll
       for (int i = 0; i < PCS; ++i) pga[i] = pgb[i];

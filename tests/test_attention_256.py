@@ -36,3 +36,24 @@ def test_both_forms(case, plan):
                           work, n_work, nq, nkv, d, 1.0 / math.sqrt(d), window or 0, one_group=one)
     ref = _mfma_reference(qs, ks, vs, reqs, 1.0 / math.sqrt(d), window, nq, d)
     torch.testing.assert_close(out.double().cpu(), ref, rtol=2e-2, atol=2e-2)       # probabilities and results in 8 bits of fraction
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [32, 64, 128, 256])
+@pytest.mark.parametrize("tokens", [16, 40])                # items whose second pair of waves, and second wave, have no rows
+def test_the_first_keys_of_a_walk_of_three_tiles_and_more(d, tokens):
+    """Pages of 16: the third tile's keys are loaded where the first tile's were, which every wave must have read by then,
+    also beside waves that have no rows and do not read.  Warm keys arrive soonest, so each launch is repeated."""
+    nq, nkv, page_size = 4, 2, 16
+    reqs = [(112, tokens), (300, tokens), (0, 200)]         # three tiles exactly, several, and growing walks
+    qs, ks, vs, dev = _mfma_inputs(nq, nkv, d, page_size, reqs)
+    work, n_work = _prefill_work(reqs, nq // nkv, d, None, "single")
+    ref = _mfma_reference(qs, ks, vs, reqs, 1.0 / math.sqrt(d), None, nq, d)
+    first = None
+    for _ in range(5):
+        out = torch.full((dev["n"], nq * d), float("nan"), dtype=torch.bfloat16).cuda()
+        K().attn_prefill_mfma(out, dev["q"], dev["stride"], dev["k_pages"], dev["v_pages"], dev["tables"], dev["cu"], dev["ctx"],
+                              work, n_work, nq, nkv, d, 1.0 / math.sqrt(d))
+        torch.testing.assert_close(out.double().cpu(), ref, rtol=2e-2, atol=2e-2)   # probabilities and results in 8 bits of fraction
+        first = out if first is None else first
+        assert torch.equal(out, first)
