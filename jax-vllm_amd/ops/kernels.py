@@ -679,27 +679,33 @@ def attn_f32_rows() -> int:
     return library.core().jv_attn_f32_rows()
 
 
-def attn_f32_splits(n_work: int, nkv: int, keys: int, device) -> int:
-    """Blocks that share out a work item's keys: one while the items give every compute unit a block, else as many as do,
-    each with a whole turn of its waves' keys (16 q heads over 4 kv heads of 128, launches included: a token each of 16
-    requests of 1,000 keys 19.8 us with 4 blocks an item, 36.6 with one, 27.8 with 9; one such token 17.5 with 16, 32.9 with
-    one; 100 tokens behind 1,000 27.7 with two, 38.4 with one)."""
-    turns = -(-keys // library.core().jv_attn_f32_tile_keys())
-    return max(1, min(compute_units(device) // max(1, n_work * nkv), turns))
+def attn_f32_range_keys() -> int:
+    """Keys of a range: a row's sums over a range are added to those of the ranges before it (``attn_f32``)."""
+    return library.core().jv_attn_f32_range_keys()
 
 
-def attn_f32_part_floats(n_work: int, nkv: int, splits: int, head_dim: int) -> int:
+def attn_f32_splits(n_work: int, nkv: int, ranges: int, device) -> int:
+    """Blocks that share out a work item's ranges: one while the items give every compute unit a block, else as many as do
+    (16 q heads over 4 kv heads of 128, launches included: a token each of 16 requests of 1,000 keys 18.9 us with 4 blocks an
+    item, 35 with one; one such token 15.1 and 32; 32 requests 30 with two and 36 with one; 48 requests 47 with two and 37 with
+    one; 100 tokens behind 1,000 32 with two, 31 with 5, 37 with one).  No number depends on it."""
+    return max(1, min(compute_units(device) // max(1, n_work * nkv), ranges))
+
+
+def attn_f32_part_floats(n_work: int, nkv: int, ranges: int, head_dim: int) -> int:
     lib = library.core()
     lib.jv_attn_f32_part_floats.restype = c_longlong
-    return lib.jv_attn_f32_part_floats(c_int(n_work), c_int(nkv), c_int(splits), c_int(head_dim))
+    return lib.jv_attn_f32_part_floats(c_int(n_work), c_int(nkv), c_int(ranges), c_int(head_dim))
 
 
 def attn_f32(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_seqlens, context_lens, work, n_work,
              nq, nkv, head_dim, scale, window=0, splits=1, parts=None, sinks=None, cap: float = 0.0, keep: int = 0) -> None:
     """Causal attention of every token over its request's pages in true 32-bit on the matrix cores.  ``work`` is int32
     [n_work, 2]: (request index, first row of ``attn_f32_rows`` (query, head-in-group) rows); every row of every request
-    must be in exactly one item.  With ``splits`` > 1 that many blocks share out an item's keys and ``parts`` (float32,
-    ``attn_f32_part_floats`` entries) holds their sums.  The other arguments: as for ``paged_attention_generic``."""
+    must be in exactly one item.  With ``splits`` > 1 that many blocks share out an item's ranges of ``attn_f32_range_keys`` keys
+    and ``parts`` (float32, ``attn_f32_part_floats`` entries for at least ``splits`` ranges) holds the ranges' sums; an item
+    of more ranges than ``parts`` has room for is one block's all the same.  A row's bits depend neither on that nor on the
+    other rows.  The other arguments: as for ``paged_attention_generic``."""
     _dev(out, q, k_pages, v_pages, block_tables, cu_seqlens, context_lens, work, sinks)
     if sinks is not None:
         _f32(sinks, "sinks", nq)
@@ -716,14 +722,17 @@ def attn_f32(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_seqlens, c
     _need(cu_seqlens.numel() == context_lens.numel() + 1 == block_tables.shape[0] + 1,
           "cu_seqlens, context_lens and block_tables disagree on the number of requests")
     _need(work.numel() >= 2 * n_work, "work list shorter than n_work")
-    if splits > 1:
-        _need(parts is not None and parts.is_cuda and parts.dtype == torch.float32
-              and parts.numel() >= attn_f32_part_floats(n_work, nkv, splits, head_dim), "parts too small for the splits")
+    room = 0
+    if splits > 1 and n_work > 0:
+        a_range = attn_f32_part_floats(n_work, nkv, 2, head_dim) // 2
+        _need(parts is not None and parts.is_cuda and parts.is_contiguous() and parts.dtype == torch.float32
+              and parts.numel() >= splits * a_range and parts.data_ptr() % 16 == 0, "parts too small for the splits")
+        room = min(parts.numel() // a_range, 2**31 - 1)
     _check(
         library.core().jv_attn_f32(_ptr(out), _ptr(q), c_longlong(q_row_stride), _ptr(k_pages), _ptr(v_pages), _ptr(block_tables),
                                    c_int(block_tables.shape[1]), _ptr(cu_seqlens), _ptr(context_lens), _ptr(work),
-                                   c_int(n_work), c_int(splits), _ptr(parts if splits > 1 else None), c_int(page_size),
-                                   c_int(nq), c_int(nkv), c_int(head_dim), c_float(scale), c_int(window or 0), _ptr(sinks),
+                                   c_int(n_work), c_int(splits), _ptr(parts if splits > 1 else None), c_int(room),
+                                   c_int(page_size), c_int(nq), c_int(nkv), c_int(head_dim), c_float(scale), c_int(window or 0), _ptr(sinks),
                                    c_float(cap), c_int(keep if window else 0), _stream()),
         "attn_f32",
     )

@@ -181,13 +181,26 @@ def f32_work_items(q_lens, context_lens, g: int, rows: int):
     return [(r, m0) for _, r, m0 in sorted(items)]
 
 
+def f32_ranges(kv_len: int, window: int, keep: int, rows: int, range_keys: int) -> int:
+    """The most ranges of keys that a work item of the 32-bit kernel touches: its ``rows`` rows are queries next to one another,
+    the last at ``kv_len`` - 1 at most.  (An interval of n keys touches up to (n + size - 2) / size + 1 ranges.)"""
+    whole = -(-kv_len // range_keys)
+    if not window:
+        return whole
+    return min(whole, -(-keep // range_keys) + (abs(window) + rows - 1 + range_keys - 2) // range_keys + 1)
+
+
 def plan_f32(ctx, nq: int, nkv: int, head_dim: int, window: int, device, keep: int) -> F32Plan:
-    items = f32_work_items(ctx.q_lens_host, ctx.context_lens_host, nq // nkv, K.attn_f32_rows())
+    rows = K.attn_f32_rows()
+    items = f32_work_items(ctx.q_lens_host, ctx.context_lens_host, nq // nkv, rows)
     most = max(c + q for c, q in zip(ctx.context_lens_host, ctx.q_lens_host))
-    splits = K.attn_f32_splits(len(items), nkv, keys_seen(most, window, keep), device)
+    size = K.attn_f32_range_keys()
+    # keys that fit a range: nothing to share out, though they may touch two
+    ranges = f32_ranges(most, window, keep, rows, size) if keys_seen(most, window, keep) > size else 1
+    splits = K.attn_f32_splits(len(items), nkv, ranges, device)
     parts = None
     if splits > 1:
-        parts = torch.empty(K.attn_f32_part_floats(len(items), nkv, splits, head_dim), dtype=torch.float32, device=device)
+        parts = torch.empty(K.attn_f32_part_floats(len(items), nkv, ranges, head_dim), dtype=torch.float32, device=device)
     flat = torch.tensor([x for item in items for x in item], dtype=torch.int32)
     return F32Plan(flat.pin_memory().to(device, non_blocking=True), len(items), splits, parts)
 

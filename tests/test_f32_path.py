@@ -125,3 +125,75 @@ def test_f32_work_items_hold_every_row_once():
         covered = sorted((r, m) for r, m0 in items for m in range(m0, min(m0 + rows, lens[r] * g)))
         assert covered == [(r, m) for r, n in enumerate(lens) for m in range(n * g)]
         assert items[0][0] == 0                                          # the request with the most keys first
+
+
+def run_step(case_sizes, reqs, pages, tables, queries, window=None, chunk=None, keep=0, cap=None, sinks=None):
+    """A step of these requests [(cached, new)] through the backend, with its own plan: the kernel's choice of blocks included."""
+    from types import SimpleNamespace
+
+    from jax_vllm_amd.parts import attention_backend
+    from jax_vllm_amd.parts.spec import LayerMemory, StepContext
+
+    nq, nkv, d, page = case_sizes
+    lens, ctx = [n for _, n in reqs], [c for c, _ in reqs]
+
+    def i32(values):
+        return torch.tensor(values, dtype=torch.int32).cuda()
+
+    step = StepContext(num_tokens=sum(lens), num_requests=len(reqs), positions=i32([c + i for c, n in reqs for i in range(n)]),
+                       token_req=i32([r for r, n in enumerate(lens) for _ in range(n)]),
+                       cu_seqlens=i32([0] + torch.tensor(lens).cumsum(0).tolist()), context_lens=i32(ctx), slot_ids=i32([0] * len(reqs)),
+                       block_tables=[tables.cuda()], slot_mappings=[None], page_size=page, q_lens_host=lens, context_lens_host=ctx,
+                       slot_ids_host=[0] * len(reqs), max_q_len=max(lens), max_kv_len=max(c + n for c, n in reqs))
+    att = SimpleNamespace(nq=nq, nkv=nkv, d=d, window=window, chunk=chunk, q_row_stride=nq * d, sinks=sinks, softcap=cap, keep_first=keep,
+                          scale=d ** -0.5)
+    out = torch.full((sum(lens), nq * d), float("nan")).cuda()
+    attention_backend.run(att, out, torch.cat(queries).reshape(sum(lens), nq * d).cuda(), step,
+                          LayerMemory(pages={"k": pages[0].cuda(), "v": pages[1].cuda()}, group=0))
+    return out.cpu()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [(16, 4, 128, 16), (8, 1, 256, 16), (12, 4, 32, 4), (4, 2, 64, 24)])
+@pytest.mark.parametrize("mask", [{}, {"window": 300}, {"window": 40, "keep": 20}, {"window": 500, "keep": 700}, {"chunk": 384}, {"cap": 30.0}])
+def test_a_token_s_bits_depend_on_what_it_sees_alone(sizes, mask):
+    """The same tokens over the same keys: alone, beside other requests (few and many: an item's ranges with blocks of their own or
+    in one), and cut into portions."""
+    nq, nkv, d, page = sizes
+    g = torch.Generator().manual_seed(d)
+    total = 1100
+    lengths = [total, 5, 2500] + [700] * 40
+    ks, vs = ([torch.randn(n, nkv, d, generator=g) for n in lengths] for _ in range(2))
+    q = [torch.randn(n, nq, d, generator=g) for n in lengths]
+    *pages, tables = build_paged(ks, vs, page)
+
+    def step(who):                                # [(request, cached, new)]
+        return run_step(sizes, [(c, n) for _, c, n in who], pages, tables[[r for r, _, _ in who]], [q[r][c:c + n] for r, c, n in who], **mask)
+
+    alone = step([(0, total - 1, 1)])
+    assert torch.isfinite(alone).all()
+    for others in ([(1, 4, 1)], [(r, lengths[r] - 1, 1) for r in range(1, 17)], [(r, 600, 1) for r in range(3, 43)], [(2, 0, 2500)]):
+        assert torch.equal(step([(0, total - 1, 1)] + others)[:1], alone)
+        assert torch.equal(step(others + [(0, total - 1, 1)])[-1:], alone)
+    whole = step([(0, 0, total)])
+    assert torch.equal(whole[-1:], alone)
+    at = 0
+    for n in (1, 250, 18, 400, 431):              # the ends of tiles and ranges inside and between portions
+        assert torch.equal(step([(0, at, n)]), whole[at:at + n])
+        at += n
+    assert at == total
+
+
+def test_the_ranges_that_a_work_item_may_touch():
+    from jax_vllm_amd.parts.attention_backend import f32_ranges
+
+    for rows in (1, 16):
+        for kv_len in (1, 16, 255, 256, 257, 300, 1000, 5000):
+            for window, keep in ((0, 0), (1, 0), (40, 20), (257, 0), (241, 300), (3000, 16), (-384, 0), (-7, 33)):
+                bound = f32_ranges(kv_len, window, keep, rows, 256)
+                for last in {kv_len - 1, max(0, kv_len - 130), max(0, kv_len - 256)}:
+                    first = max(0, last - rows + 1)
+                    begin = max(0, first - window + 1) if window > 0 else first - first % -window if window else 0
+                    begin = begin // 16 * 16                                       # whole tiles
+                    touched = {j // 256 for j in list(range(min(keep, begin))) + list(range(begin, last + 1))}
+                    assert len(touched) <= bound, (kv_len, window, keep, rows, last)
