@@ -970,48 +970,62 @@ STREAM_MAX_ROWS = 128
 STREAM_MODES = {"parts": 0, "rows": 1, "pairs": 2}
 
 
+def _ring_time(m: int, n: int, k: int, tm: int, tw: int, parts: int, cus: int) -> float:
+    """Microseconds of a product in this form, mostly within a tenth (800 sizes of 17 to 128 rows, 1 to 1,500 MB): 3.2, then for
+    every round of blocks (one a compute unit; two of 32 + 32 rows, each a third slower beside the other) the chunks of 64 columns
+    of a part; a chunk is bound by its block (a fifth slower where the inner size is no power of two) or, at 5.4 TB/s, by what the
+    blocks draw of w, and where both are alike takes a little longer than either."""
+    blocks, chunks, cost = -(-n // tw) * parts, -(-(k // 64) // parts), 3.2
+    own = max(0.27, 0.19 + 8.3e-4 * tw + 1.15e-5 * (tw - 32) * tm + 9e-4 * m) * (1.2 if k & (k - 1) else 1.0)
+    slots = cus * (2 if tm + tw <= 64 else 1)
+    for units, rounds in ((slots, blocks // slots), (blocks % slots, 1)):
+        if units and rounds:
+            cost += rounds * chunks * ((own * (1.35 if units > cus else 1.0)) ** 4 + (units * tw * 128 / 5.4e6) ** 4) ** 0.25
+    return cost
+
+
+def _library_time(m: int, n: int, k: int, pairs: bool) -> float:
+    """Microseconds that the library takes for 17 to 128 rows, rather too few (it is irregular: up to a half more at some sizes): a
+    floor by the inner size, then the stream of w; more rows cost it more.  Of 800 sizes the choice by these two counts is slower
+    than the library by more than 3 % at 7, at most 9 % (32,000 x 1,024 at 128 rows)."""
+    mb = n * k * 2e-6
+    floor = 10.5 + 0.08 * mb if k >= 2048 else 0.0 if k >= 1024 and m <= 24 and n <= 2048 else 9.0
+    stream = min(5.0 + 0.2 * mb, 10.0 + 0.18 * mb) + max(0.0, 0.03 * (mb - 524.0))
+    rows = 1.0 if m <= 32 else 1.08 if m <= 64 else (1.25 if mb < 130.0 else 1.14) if k >= 3072 else (1.1 if mb < 130.0 else 1.05)
+    return max(floor, stream * rows) + (2.0 if pairs else 0.0)
+
+
 @functools.lru_cache(maxsize=4096)
 def ring_plan(m: int, n: int, k: int, mode: str, cus: int = 256):
     """How ``linear`` runs a bfloat16 product of 17 to 128 rows through ``gemm_stream``: (rows of x, rows of w, parts of the
     inner size) of a block, or None where another way is better.  ``mode``: "parts" (the reader adds float partial
     products), "rows", "pairs" (rows of w alternate gate and up rows).
 
-    The form with the least time by this count (all of one product's forms give it within rounding): every round of one
-    block a compute unit takes 3 us and then, a chunk of 64 columns, the longest of 0.31 us, what its units draw from
-    the L2s at 9.6 TB/s and what they draw of w from memory at 5.3 TB/s, as measured over 32 to 128 rows.
-
-    A matrix below 1 MB is no stream, and stays with the library.  Others are better, measured (microseconds here / there):
+    The form with the least time by ``_ring_time`` (all of one product's forms give it within rounding).  Others are better,
+    measured (microseconds here / there):
 
     * blocks that stay with x in registers, for narrow matrices they cover: up to 32 rows and 5,120 wide (4,096 x 4,096 at
-      24 rows 10.8 / 10.0), up to 64 rows and 1,024 wide (x 4,096: 7.9 / 7.3);
-    * the library, about 11.5 us + w at 5.1 TB/s and 2 us for the activation (the count here is up to 15 % high beside
-      that), where blocks with the whole inner size cannot fill the chip (2,080 x 2,048 at 96 rows 12.9 / 11.4) or a large
-      matrix leaves a fifth of a round empty (51,200 x 5,120 at 64 rows 118 / 111)."""
+      24 rows 10.6 / 10.2), up to 40 rows and 2,560 wide (x 4,096: 9.3 / 9.1), up to 64 rows and 1,024 wide (x 4,096: 8.1 / 7.3);
+    * the library, which may share out the inner size, where blocks with the whole inner size wait for their chunks and not for
+      the memory (4,096 x 3,072 at 32 rows 16.4 / 10.9, 6,144 x 4,096 20.6 / 15.5, 8,192 x 5,120 26.5 / 19.9; but 16,384 x 4,096 with its
+      activation 28.6 / 33.9, 32,000 x 2,048 27.7 / 32.6), by ``_library_time``; and where a large matrix leaves a fifth of a round
+      empty (51,200 x 5,120 at 72 rows 119 / 111).
+
+    A matrix of less than 500,000 elements (1 MB) stays with the library although the ring would be quicker (512 x 512 at 32 rows
+    4.8 / 6.4, 1,024 x 448 5.5 / 7.8): the models that small are those whose bfloat16 outputs are compared token by token, and
+    the two round differently."""
     if not SKINNY_AUTO_ROWS < m <= STREAM_MAX_ROWS or k % 64 or n % 4 or n * k < 500_000:
         return None
     tm = 32 if m <= 32 else 64 if m <= 64 else 128
-    if mode == "parts" and n <= (5120 if m <= 32 else 1024 if m <= 64 else 0):
+    if mode == "parts" and n <= (5120 if m <= 32 else 2560 if m <= 40 else 1024 if m <= 64 else 0):
         nl = _stay_pieces(k, 4)
         if nl is not None and (nl <= 5 or (m <= 32 and nl <= 8)):
             return None
-    best = None
-    for tw in (32, 64, 96, 128):
-        for parts in ((4, 3, 2) if mode == "parts" else (1,)):
-            if parts > k // 64:
-                continue
-            blocks, chunks, cost = -(-n // tw) * parts, -(-(k // 64) // parts), 3.0
-            for units, rounds in ((cus, blocks // cus), (blocks % cus, 1 if blocks % cus else 0)):
-                cost += rounds * chunks * max(0.31, (tm + tw) * 128 / 40e3, units * tw * 128 / 5.3e6)
-            if best is None or cost < best[0]:
-                best = (cost, blocks, (tm, tw, parts))
-    if best is None:
-        return None
-    cost, blocks, form = best
-    if mode != "parts":
-        mb = n * k * 2e-6
-        if cost > 1.15 * (11.5 + 0.195 * mb + (2.0 if mode == "pairs" else 0.0)):
-            return None
-        if mb > 400 and blocks < 0.8 * -(-blocks // cus) * cus:
+    cost, form = min(((_ring_time(m, n, k, tm, tw, parts, cus), (tm, tw, parts)) for tw in (32, 64, 96, 128)
+                      for parts in ((4, 3, 2) if mode == "parts" else (1,)) if parts <= k // 64), default=(0.0, None))
+    if form is not None and mode != "parts":
+        blocks = -(-n // form[1])
+        if cost > _library_time(m, n, k, mode == "pairs") or (n * k > 200_000_000 and blocks < 0.8 * -(-blocks // cus) * cus):
             return None
     return form
 

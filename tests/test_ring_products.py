@@ -25,6 +25,20 @@ def test_plans_are_ones_the_kernel_takes():
     assert K.ring_plan(64, 51200, 5120, "pairs") is None                   # the library
 
 
+def test_whole_inner_sizes_go_where_they_are_faster():
+    """Blocks that take the whole inner size wait for their chunks, not for the memory, while w is small beside its inner size:
+    there the library, which may share it out, was measured faster; and forms that leave compute units without a block lose."""
+    for m, n, k in ((32, 4096, 3072), (24, 6144, 4096), (32, 8192, 5120), (17, 8192, 4096), (24, 10240, 4096), (24, 2080, 2048), (48, 6144, 4096),
+                    (112, 3072, 1536), (24, 5120, 5120), (64, 2048, 4096)):
+        assert K.ring_plan(m, n, k, "rows") is None, (m, n, k)
+    for m, n, k, mode, tw in ((32, 16384, 4096, "pairs", 64), (24, 11296, 2048, "rows", 64), (64, 32000, 2048, "rows", 128), (72, 10240, 4096, "rows", 64),
+                              (64, 151936, 4096, "rows", 128), (72, 8192, 1024, "rows", 32), (24, 24576, 4096, "pairs", 96)):
+        form = K.ring_plan(m, n, k, mode)
+        assert form is not None and form[1] == tw, (m, n, k, form)
+    assert K.ring_plan(32, 8192, 4096, "parts") == (32, 128, 4) and K.ring_plan(32, 8192, 2048, "parts") == (32, 128, 4)
+    assert K.ring_plan(40, 2560, 4096, "parts") is None                    # blocks that stay
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("tm,tw", FORMS)
 def test_products_at_the_edges(tm, tw):
