@@ -1065,8 +1065,10 @@ def shares_plan(m: int, n: int, k: int, cus: int = 256):
     within a tenth.  Here: 5, then every round of one tile a compute unit the chunks of a part (a round that leaves units
     idle is faster, by up to a fifth), then the partial products, written at 6 TB/s and read at 5.  The library:
     3 + k (0.0036 + 1.32e-9 m n).  300 rows against 4,096 x 12,288: 48 / 70, against 4,096 x 4,096 20 / 26; 1,525 rows
-    140 and 9 for the parts / 147."""
-    if not STREAM_MAX_ROWS < m <= SHARES_MAX_ROWS or k % 64 or n % 4 or n * k < 500_000:
+    140 and 9 for the parts / 147.  Results of up to 262,144 numbers are the library's, which takes less there than the count says
+    (with the norm that reads them, 256 rows against 1,024 x 3,072: 16.5 / 13.4, 200 against 768 x 3,072 14.6 / 13.3; 257 against
+    1,024 x 3,072 14.9 / 18.5).  Of 336 sizes 9 are then slower than the library by more than 2 %, at most 10 %; the mean is 0.86."""
+    if not STREAM_MAX_ROWS < m <= SHARES_MAX_ROWS or k % 64 or n % 4 or n * k < 500_000 or m * n <= 262_144:
         return None
     best = None
     for (tm, tw), chunk in _SHARES_TILES.items():

@@ -23,6 +23,13 @@ def test_plans_are_ones_the_kernel_takes():
     assert K.shares_plan(2048, 4096, 4096) is None and K.shares_plan(300, 2048, 512) is None       # the library
 
 
+def test_small_results_stay_with_the_library():
+    """Measured faster there: 256 rows against 1,024 x 3,072 13.4 us with the norm that reads the result, 16.5 through partial sums."""
+    for m, n, k in ((256, 1024, 3072), (200, 1024, 4096), (300, 768, 3072), (129, 768, 3072)):
+        assert K.shares_plan(m, n, k) is None
+    assert K.shares_plan(257, 1024, 3072) is not None and K.shares_plan(160, 2048, 4096) is not None
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("tm,tw", TILES)
 def test_products_at_the_edges(tm, tw):
