@@ -2076,6 +2076,19 @@ def _router_logits_plan(x, w_router, one_launch: bool):
 ROUTER_FUSED_MAX_ROWS = 64      # 17..64 rows: logits and choice in one launch
 
 
+def rows_by_tiles(m: int, n: int, k: int, cus: int = 256) -> bool:
+    """Whether ``gemm_rows_f32out`` runs as tiles of 128 x 128 (``gemm_shares``, the inner size in one piece) instead of blocks of 16
+    rows that share the inner size out to their waves: those are one round trip to memory while each compute unit has one of
+    them, and read w once for every 16 rows beyond.  Microseconds (blocks of 16 rows / tiles): 2,048 rows x 256 x 2,048 22 / 16,
+    8,192 x 512 x 2,048 147 / 27, 8,192 x 256 x 7,168 248 / 48, 2,048 x 128 x 4,096 22 / 27, 8,192 x 32 x 2,048 14.6 / 15.5."""
+    if k % 64 or n % 4 or k < 64 or k > 1 << 20:
+        return False
+    nt = 1 if n <= 16 else 2 if n <= 32 else 4
+    rounds = -(-(-(-m // 16) * -(-n // (16 * nt))) // cus)
+    tiles = -(-(-(-m // 128) * -(-n // 128)) // cus)
+    return 2.5 + rounds * k * {1: 0.0017, 2: 0.0028, 4: 0.0047}[nt] > 5.5 + tiles * k * 0.0051
+
+
 def gemm_rows_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """float32 x @ w.T for bfloat16 x [M, K] and w [N, K] on the matrix cores (K a multiple of 8): products
     whose result must not be rounded to the activation type (router logits)."""
@@ -2084,6 +2097,8 @@ def gemm_rows_f32out(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     m, k = x.shape
     n = w.shape[0]
     _need(w.shape[1] == k and k % 8 == 0 and k >= 8, "inner sizes must agree and be a multiple of 8")
+    if m > 0 and n > 0 and rows_by_tiles(m, n, k, compute_units(x.device)) and not (x.data_ptr() | w.data_ptr()) & 15:
+        return gemm_shares(x, w, (128, 128, 1))[0]
     out = torch.empty((m, n), dtype=torch.float32, device=x.device)
     _check(library.core().jv_gemm_rows_f32out_bf16(_ptr(out), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), _stream()),
            "gemm_rows_f32out")

@@ -18,6 +18,19 @@ def test_router_logits(m, n, k):
     assert torch.equal(K().gemm_rows_f32out(x[m // 2:].contiguous().cuda(), w.cuda()), y[m // 2:])      # whatever the batch
 
 
+@pytest.mark.parametrize("m,n,k,tiles", [(4096, 64, 1024, False), (4097, 64, 1024, True), (2050, 132, 2048, True), (1100, 516, 448, True),
+                                         (8192, 32, 256, False), (1100, 513, 448, False), (1100, 516, 456, False)])
+def test_router_logits_of_many_rows(m, n, k, tiles):
+    """Beyond a round of blocks of 16 rows: tiles of 128 x 128, where the sizes allow them."""
+    assert K().rows_by_tiles(m, n, k) == tiles
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x, w = torch.randn(m, k, generator=g, device="cuda").bfloat16(), torch.randn(n, k, generator=g, device="cuda").bfloat16()
+    y = K().gemm_rows_f32out(x, w)
+    assert y.shape == (m, n) and y.dtype == torch.float32 and y.is_contiguous()
+    bound = 2.0 ** -24 * k * (x.double().abs() @ w.double().abs().T)       # exact products, sums of k terms in float
+    assert ((y.double() - x.double() @ w.double().T).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("tile_rows", [64, 128])
 @pytest.mark.parametrize("hidden,ff", [(8, 8), (56, 72), (64, 264), (136, 128), (200, 520)])
 @pytest.mark.parametrize("gated", [True, False])
