@@ -184,7 +184,8 @@ extern "C" int jv_moe_gate_up_mfma_bf16(void* z, const void* x, const void* Wg, 
                                         const int* order, const float* weights, int max_tiles, int top, int hidden,
                                         int ff, int act, float act_limit, float act_slope, int scale_input, int tile_rows, void* stream) {
   if (max_tiles <= 0 || ff <= 0) return 0;
-  if (!(Wg ? jv_act_known(act) : jv_plain_act_known(act)) || hidden < 8 || hidden % 8) return (int)hipErrorInvalidValue;
+  if (!(Wg ? jv_act_known(act) : jv_plain_act_known(act)) || hidden < 8 || hidden % 8 || (((uintptr_t)x | (uintptr_t)Wg | (uintptr_t)Wu) & 15))
+    return (int)hipErrorInvalidValue;
   if (!Wg)
     return launch_moe_mfma<MM_PLAIN>(tile_rows, max_tiles, (hipStream_t)stream, z,
                                      (const bf16_t*)x, (const bf16_t*)Wu, nullptr, meta, offsets, tile_expert, tile_row0,
@@ -200,7 +201,7 @@ extern "C" int jv_moe_down_mfma_bf16(float* y, const void* z, const void* Wd, co
                                      const float* weights, int max_tiles, int top, int n_tokens, int hidden, int ff,
                                      int scale_output, int tile_rows, void* stream) {
   if (max_tiles <= 0 || hidden <= 0) return 0;
-  if (ff < 8 || ff % 8) return (int)hipErrorInvalidValue;
+  if (ff < 8 || ff % 8 || (((uintptr_t)z | (uintptr_t)Wd) & 15)) return (int)hipErrorInvalidValue;
   return launch_moe_mfma<MM_DOWN>(tile_rows, max_tiles, (hipStream_t)stream, y,
                                 (const bf16_t*)z, (const bf16_t*)Wd, nullptr, meta, offsets, tile_expert, tile_row0, order,
                                 weights, top, n_tokens, ff, hidden, JvAct{}, scale_output);

@@ -2273,6 +2273,8 @@ def moe_experts(x, plan: MoePlan, w_gate, w_up, w_down, activation: str, out: to
             c_int(0 if weight_on_input else 1), _stream()), "moe_down")
         return
     if mfma:
+        # straight into LDS: 16-byte pieces of rows, which begin on such a boundary (a view that does not is copied)
+        x, w_gate, w_up, w_down = (t if t is None or t.data_ptr() % 16 == 0 else t.clone() for t in (x, w_gate, w_up, w_down))
         _check(lib.jv_moe_gate_up_mfma_bf16(
             _ptr(z), _ptr(x), _ptr(w_gate), _ptr(w_up), _ptr(p.meta), _ptr(p.offsets), _ptr(p.tile_expert),
             _ptr(p.tile_row0), _ptr(p.order), _ptr(p.weights), c_int(p.max_tiles), c_int(p.top), c_int(hidden), c_int(ff),

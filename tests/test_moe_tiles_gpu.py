@@ -59,3 +59,23 @@ def test_expert_tiles(tile_rows, hidden, ff, gated):
         # z may be rounded the other way where the float sum and this one straddle: half a unit of bfloat16 in one term
         scale = z.abs() @ wd[e].double().abs().T + 1e-3
         assert ((out[0].cpu()[at].double() - want).abs() <= 2.0 ** -8 * scale).all()
+
+
+@pytest.mark.parametrize("which", [0, 1, 2, 3])
+def test_an_operand_off_its_boundary(which):
+    """Rows go into LDS in pieces of 16 bytes: an operand that begins 2 bytes off gives what its copy gives."""
+    n, experts, hidden, ff = 150, 3, 72, 136
+    g = torch.Generator().manual_seed(5)
+    shapes = [(n, hidden), (experts, ff, hidden), (experts, ff, hidden), (experts, hidden, ff)]
+    tensors = [(torch.randn(s, generator=g) * s[-1] ** -0.5).bfloat16().cuda() for s in shapes]
+    off = list(tensors)
+    flat = torch.empty(tensors[which].numel() + 1, dtype=torch.bfloat16, device="cuda")
+    off[which] = flat[1:].view(shapes[which]).copy_(tensors[which])
+    assert off[which].data_ptr() % 16 == 2 and off[which].is_contiguous()
+    plan = K().moe_route(torch.randn(n, experts, generator=g).cuda(), 2, tile_rows=64)
+    results = []
+    for x, wg, wu, wd in (tensors, off):
+        out = torch.full((2, n, hidden), float("nan"), device="cuda")
+        K().moe_experts(x, plan, wg, wu, wd, "silu", out)
+        results.append(out)
+    assert torch.isfinite(results[0]).all() and torch.equal(*results)
