@@ -29,8 +29,7 @@ enum { MM_DOWN = 0, MM_GATED = 1, MM_PLAIN = 2 };
 // What a lane reads for columns behind the inner size, of x and of W alike.
 static __device__ __attribute__((aligned(16))) const unsigned mm_zeros[4] = {0, 0, 0, 0};
 
-// TM: rows of a tile of the grouping, 64 or 128; TW: rows of W of a block (gated: half of them of each matrix).  Without a grouping (tile_expert null) the product is a plain one: rows
-// in order, one weight matrix, float output [rows, N].
+// TM: rows of a tile of the grouping, 64 or 128; TW: rows of W of a block (gated: half of them of each matrix).
 template <int MODE, int TM, int TW, int BUFS>
 __global__ void __launch_bounds__(2 * TW, TW == 128 ? 2 : 1)
 moe_mfma_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, const bf16_t* __restrict__ W0,
@@ -168,29 +167,33 @@ static int launch_moe_tiles(int max_tiles, hipStream_t stream, void* out, const 
   return JV_LAUNCH_CHECK();
 }
 
-// 128 rows against 256 of W by 8 waves with two chunks on their way, 64 rows (where an expert gets so few that the stream of its
-// weights is what is waited for) against 128 by 4 waves, three blocks a compute unit.
+// 128 rows against 256 of W by 8 waves with two chunks on their way; 64 rows against 128 by 4 waves, three blocks a compute unit with
+// one chunk on its way each, or (`deep`) two blocks with two: where an expert gets so few rows that nearly all are one tile, the
+// stream of the weights is what is waited for.  gate/up + down, cold weights, microseconds (deep / not): 64 experts x 1,024, width
+// 4,096, 25 rows each 302 / 334, 8 x 4,096 at 40 rows 167 / 184, 16 x 2,048, width 1,024, at 25 56 / 64, 32 x 512, width 2,048, at
+// 40 52 / 57; at 50 rows, with second tiles, 66 / 62.
 template <int MODE, typename... Args>
-static int launch_moe_mfma(int tile_rows, Args... args) {
+static int launch_moe_mfma(int tile_rows, int deep, Args... args) {
   if (tile_rows == 128) return launch_moe_tiles<MODE, 128, 256, 3>(args...);
+  if (tile_rows == 64 && deep) return launch_moe_tiles<MODE, 64, 128, 3>(args...);
   if (tile_rows == 64) return launch_moe_tiles<MODE, 64, 128, 2>(args...);
   return (int)hipErrorInvalidValue;
 }
 
 // gate/up: x [tokens, hidden], Wg, Wu [experts, ff, hidden] -> z [entries, ff] bf16 by position; tile_rows (64 or
-// 128) is what the grouping was made with.  Wg null: experts without a gate, act one that stands alone.
+// 128) is what the grouping was made with; deep: see launch_moe_mfma.  Wg null: experts without a gate, act one that stands alone.
 extern "C" int jv_moe_gate_up_mfma_bf16(void* z, const void* x, const void* Wg, const void* Wu, const int* meta,
                                         const int* offsets, const int* tile_expert, const int* tile_row0,
                                         const int* order, const float* weights, int max_tiles, int top, int hidden,
-                                        int ff, int act, float act_limit, float act_slope, int scale_input, int tile_rows, void* stream) {
+                                        int ff, int act, float act_limit, float act_slope, int scale_input, int tile_rows, int deep, void* stream) {
   if (max_tiles <= 0 || ff <= 0) return 0;
   if (!(Wg ? jv_act_known(act) : jv_plain_act_known(act)) || hidden < 8 || hidden % 8 || (((uintptr_t)x | (uintptr_t)Wg | (uintptr_t)Wu) & 15))
     return (int)hipErrorInvalidValue;
   if (!Wg)
-    return launch_moe_mfma<MM_PLAIN>(tile_rows, max_tiles, (hipStream_t)stream, z,
+    return launch_moe_mfma<MM_PLAIN>(tile_rows, deep, max_tiles, (hipStream_t)stream, z,
                                      (const bf16_t*)x, (const bf16_t*)Wu, nullptr, meta, offsets, tile_expert, tile_row0,
                                      order, weights, top, 0, hidden, ff, JvAct{act, act_limit, act_slope}, scale_input);
-  return launch_moe_mfma<MM_GATED>(tile_rows, max_tiles, (hipStream_t)stream, z, (const bf16_t*)x,
+  return launch_moe_mfma<MM_GATED>(tile_rows, deep, max_tiles, (hipStream_t)stream, z, (const bf16_t*)x,
                                (const bf16_t*)Wg, (const bf16_t*)Wu, meta, offsets, tile_expert, tile_row0, order,
                                weights, top, 0, hidden, ff, JvAct{act, act_limit, act_slope}, scale_input);
 }
@@ -199,10 +202,10 @@ extern "C" int jv_moe_gate_up_mfma_bf16(void* z, const void* x, const void* Wg, 
 extern "C" int jv_moe_down_mfma_bf16(float* y, const void* z, const void* Wd, const int* meta, const int* offsets,
                                      const int* tile_expert, const int* tile_row0, const int* order,
                                      const float* weights, int max_tiles, int top, int n_tokens, int hidden, int ff,
-                                     int scale_output, int tile_rows, void* stream) {
+                                     int scale_output, int tile_rows, int deep, void* stream) {
   if (max_tiles <= 0 || hidden <= 0) return 0;
   if (ff < 8 || ff % 8 || (((uintptr_t)z | (uintptr_t)Wd) & 15)) return (int)hipErrorInvalidValue;
-  return launch_moe_mfma<MM_DOWN>(tile_rows, max_tiles, (hipStream_t)stream, y,
+  return launch_moe_mfma<MM_DOWN>(tile_rows, deep, max_tiles, (hipStream_t)stream, y,
                                 (const bf16_t*)z, (const bf16_t*)Wd, nullptr, meta, offsets, tile_expert, tile_row0, order,
                                 weights, top, n_tokens, ff, hidden, JvAct{}, scale_output);
 }

@@ -2038,12 +2038,13 @@ MOE_SKINNY_MAX_MEAN = 6         # up to so many rows an expert (on average over 
 
 def moe_tile_rows_for(dtype, hidden: int, ff: int, entries: int, experts: int) -> int:
     """Rows of a tile for a step: 16 (the kernels that stream the experts' weights) where an expert gets a few rows at
-    most, 128 where the matrix-core kernels run and an expert gets about a hundred rows or more (a row of W then feeds
-    twice the products), else 64."""
+    most, 128 where the matrix-core kernels run and an expert gets more than 64 rows on average (a second tile of 64 would be
+    nearly empty: 8 experts x 4,096 of width 4,096 at 75 rows each 198 us with 128, 270 with 64; 64 x 1,024 at 68 rows 361 / 430,
+    128 x 768 of width 2,048 at 68 rows 296 / 313; at 60 rows 32 x 512 66 / 61), else 64."""
     if moe_matrix_cores_possible(dtype, hidden, ff):
         if entries <= MOE_SKINNY_MAX_MEAN * experts:
             return MOE_SKINNY_ROWS
-        if entries >= 96 * experts:
+        if entries > 64 * experts:
             return 128
     return moe_tile_rows()
 
@@ -2275,14 +2276,15 @@ def moe_experts(x, plan: MoePlan, w_gate, w_up, w_down, activation: str, out: to
     if mfma:
         # straight into LDS: 16-byte pieces of rows, which begin on such a boundary (a view that does not is copied)
         x, w_gate, w_up, w_down = (t if t is None or t.data_ptr() % 16 == 0 else t.clone() for t in (x, w_gate, w_up, w_down))
+        deep = n * p.top <= 40 * experts        # few rows an expert: the weights' stream is what is waited for
         _check(lib.jv_moe_gate_up_mfma_bf16(
             _ptr(z), _ptr(x), _ptr(w_gate), _ptr(w_up), _ptr(p.meta), _ptr(p.offsets), _ptr(p.tile_expert),
             _ptr(p.tile_row0), _ptr(p.order), _ptr(p.weights), c_int(p.max_tiles), c_int(p.top), c_int(hidden), c_int(ff),
-            *act, c_int(1 if weight_on_input else 0), c_int(p.tile_rows), _stream()), "moe_gate_up")
+            *act, c_int(1 if weight_on_input else 0), c_int(p.tile_rows), c_int(deep), _stream()), "moe_gate_up")
         _check(lib.jv_moe_down_mfma_bf16(
             _ptr(out), _ptr(z), _ptr(w_down), _ptr(p.meta), _ptr(p.offsets), _ptr(p.tile_expert), _ptr(p.tile_row0),
             _ptr(p.order), _ptr(p.weights), c_int(p.max_tiles), c_int(p.top), c_int(n), c_int(hidden), c_int(ff),
-            c_int(0 if weight_on_input else 1), c_int(p.tile_rows), _stream()), "moe_down")
+            c_int(0 if weight_on_input else 1), c_int(p.tile_rows), c_int(deep), _stream()), "moe_down")
         return
     _check(getattr(lib, f"jv_moe_gate_up_{suf}")(
         _ptr(z), _ptr(x), _ptr(w_gate), _ptr(w_up), _ptr(p.meta), _ptr(p.offsets), _ptr(p.tile_expert),

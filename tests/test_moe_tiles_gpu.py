@@ -31,12 +31,21 @@ def test_router_logits_of_many_rows(m, n, k, tiles):
     assert ((y.double() - x.double() @ w.double().T).abs() <= bound).all()
 
 
-@pytest.mark.parametrize("tile_rows", [64, 128])
+FEW = [40, 0, 1, 65, 17]           # 25 an expert: the form with two chunks on their way
+
+
+def test_more_than_64_rows_an_expert_take_tiles_of_128():
+    args = torch.bfloat16, 4096, 4096
+    assert [K().moe_tile_rows_for(*args, n, 8) for n in (48, 49, 512, 513, 600)] == [16, 64, 64, 128, 128]
+    assert K().moe_tile_rows_for(torch.float32, 4096, 4096, 600, 8) == 64
+
+
+@pytest.mark.parametrize("tile_rows,few", [(64, False), (128, False), (64, True)])
 @pytest.mark.parametrize("hidden,ff", [(8, 8), (56, 72), (64, 264), (136, 128), (200, 520)])
 @pytest.mark.parametrize("gated", [True, False])
-def test_expert_tiles(tile_rows, hidden, ff, gated):
+def test_expert_tiles(tile_rows, few, hidden, ff, gated):
     """Experts with no row, one row, a tile exactly, one more, and several tiles; one to nine chunks of the inner size."""
-    rows = [tile_rows, 0, 1, tile_rows + 1, 2 * tile_rows + 33]
+    rows = FEW if few else [tile_rows, 0, 1, tile_rows + 1, 2 * tile_rows + 33]
     n, experts = sum(rows), len(rows)
     g = torch.Generator().manual_seed(hidden + ff)
     x = torch.randn(n, hidden, generator=g).bfloat16()
