@@ -123,13 +123,17 @@ def prefill_item_shape(rows: int, nkv: int, group_rows: int, kernel_groups: int,
     return kernel_groups, blocks <= RESIDENT_BLOCKS * compute_units
 
 
-def few_rows_of_256(rows: int, keys: int, group_rows: int, compute_units: int) -> bool:
+def few_rows_of_256(rows: int, keys: int, group_rows: int, compute_units: int, page_size: int = 16) -> bool:
     """Whether a step's prompt portions at head size 256 take items of one group (16 rows a wave) instead of two (32): while
-    those give no more than a quarter of the compute units a second block, and nobody sees 2,048 keys.  An item of two groups takes about 13 us and 2.6
-    for every 64 keys, one of one group 6 and 2.85, or twice that beside another (measured: 300 tokens of 16 heads over one
-    20 / 26 us, 1,200 in two prompts 38 / 43, 1,024 tokens over 8 kv heads
-    49 / 50, 2,048 over 2 95 / 90, 2,048 over one with a window of 1,024 107 / 73, 512 after 4,000 200 / 183)."""
-    return 4 * -(-rows // group_rows) <= 5 * compute_units and keys < 2048
+    those give no more than a quarter of the compute units a second block, unless pages of 16 and 2,048 keys make up for the start
+    (only there does the larger form overlap its own work); with pages of 16 also where nobody sees more than 256 keys, for an item
+    of two groups is slow to start.  Microseconds, two groups / one, 1,064 steps measured: 300 tokens of 16 heads over one 26 / 20, 2,048
+    over 2 90 / 95, 2,048 over one with a window of 1,024 73 / 107, of 256 44 / 43, of 128 39 / 34, 4,000 over 8 kv heads with 128
+    51 / 35; 512 after 4,000 181 / 194, with pages of 32 203 / 192, of 24 259 / 209; 2,048 over 8 kv heads with pages of 32 98 / 93."""
+    few = 4 * -(-rows // group_rows) <= 5 * compute_units
+    if page_size != 16:
+        return few
+    return keys <= 256 or (few and keys < 2048)
 
 
 def plan_mfma(ctx, nq: int, nkv: int, head_dim: int, window: int, device, keep: int = 0) -> MfmaPlan:
@@ -141,12 +145,14 @@ def plan_mfma(ctx, nq: int, nkv: int, head_dim: int, window: int, device, keep: 
     cus = K.compute_units(device)
     one_group = head_dim == 256 and few_rows_of_256(
         rows * nkv, max([keys_seen(cl + ql, window, keep) for ql, cl in zip(ctx.q_lens_host, ctx.context_lens_host) if ql > 1],
-                        default=0), group_rows, cus)
+                        default=0), group_rows, cus, ctx.page_size)
     if one_group:
         groups_per_item, balance = 1, False
     prefill = prefill_work_items(ctx.q_lens_host, ctx.context_lens_host, g, window, group_rows, groups_per_item,
                                  balance=balance, keep=keep)
-    if cus < len(prefill) * nkv <= RESIDENT_BLOCKS * cus and head_dim != 256:      # 256: one block a unit, or fewer blocks
+    # head size 256: items of two groups have a unit each, and items of one group were not helped (168 steps of 257 to 512 items, all
+    # page sizes: 0.97 to 1.24 of the time, 1.04 on average)
+    if cus < len(prefill) * nkv <= RESIDENT_BLOCKS * cus and head_dim != 256:
         prefill = pair_up_resident_items(prefill, cus // nkv)
     decode = [r for r, ql in enumerate(ctx.q_lens_host) if ql == 1]
     max_kv_decode = max([ctx.context_lens_host[r] + 1 for r in decode], default=1)

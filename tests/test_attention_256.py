@@ -14,6 +14,14 @@ def test_the_rule():
     assert not few_rows_of_256(320 * 64 + 1, 300, 64, 256) and not few_rows_of_256(64, 2048, 64, 256)
 
 
+def test_the_rule_looks_at_pages_and_short_windows():
+    assert few_rows_of_256(64 * 5000, 128, 64, 256) and few_rows_of_256(64 * 5000, 256, 64, 256)      # short walks
+    assert not few_rows_of_256(64 * 5000, 257, 64, 256)
+    for page_size in (8, 24, 32, 64):                     # no work of its own to overlap: rows alone count
+        assert few_rows_of_256(64 * 320, 100000, 64, 256, page_size)
+        assert not few_rows_of_256(64 * 320 + 1, 128, 64, 256, page_size)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("plan", ["single", "planner", "far", "one_group"])
 @pytest.mark.parametrize("case", [
