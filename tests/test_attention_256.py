@@ -6,7 +6,8 @@ import torch
 
 from jax_vllm_amd.parts.attention_backend import few_rows_of_256
 
-from .test_kernels_gpu import K, _mfma_inputs, _mfma_reference, _prefill_work
+from .test_f32_path import reference, run_step
+from .test_kernels_gpu import K, _mfma_inputs, _mfma_reference, _prefill_work, build_paged
 
 
 def test_the_rule():
@@ -65,3 +66,55 @@ def test_the_first_keys_of_a_walk_of_three_tiles_and_more(d, tokens):
         torch.testing.assert_close(out.double().cpu(), ref, rtol=2e-2, atol=2e-2)   # probabilities and results in 8 bits of fraction
         first = out if first is None else first
         assert torch.equal(out, first)
+
+
+MASKS = [{"window": 100}, {"window": 100, "keep": 20}, {"window": 70, "keep": 200}, {"chunk": 96}, {"chunk": 64, "keep": 33}, {}]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("page_size", [16, 24, 64])
+@pytest.mark.parametrize("one_group", [True, False])
+@pytest.mark.parametrize("mask", MASKS, ids=str)
+def test_both_forms_with_sinks_caps_kept_keys_and_blocks(mask, one_group, page_size):
+    nq, nkv, d, scale = 6, 2, 256, 0.09
+    reqs = [(0, 70), (230, 90), (5, 131)]
+    qs, ks, vs, dev = _mfma_inputs(nq, nkv, d, page_size, reqs)
+    sinks = torch.linspace(-1.0, 2.0, nq)
+    window, chunk, keep = mask.get("window"), mask.get("chunk"), mask.get("keep", 0)
+    for cap, with_sinks in ((0.0, True), (3.0, False), (3.0, True)):
+        work, n_work = _prefill_work(reqs, nq // nkv, d, window, "single" if one_group else "neighbours")
+        out = torch.full((dev["n"], nq * d), float("nan"), dtype=torch.bfloat16).cuda()
+        K().attn_prefill_mfma(out, dev["q"], dev["stride"], dev["k_pages"], dev["v_pages"], dev["tables"], dev["cu"], dev["ctx"], work, n_work,
+                              nq, nkv, d, scale, K().key_window(window, chunk), sinks=sinks.cuda() if with_sinks else None, cap=cap, keep=keep,
+                              one_group=one_group)
+        want = torch.cat([reference(q, k, v, torch.arange(c, c + n), scale, window, chunk, keep, cap, sinks if with_sinks else None)
+                          for q, k, v, (c, n) in zip(qs, ks, vs, reqs)]).reshape(-1, nq * d)
+        torch.testing.assert_close(out.double().cpu(), want, rtol=2e-2, atol=2e-2)      # probabilities and results in 8 bits of fraction
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("reqs,page_size,mask,one_group", [
+    ([(0, 70), (300, 9), (40, 1)], 16, {"window": 100, "keep": 20}, True),              # few rows
+    ([(0, 1400), (40, 1)], 16, {"window": 300, "keep": 20}, False),                     # more than 320 groups
+    ([(0, 1400)], 16, {"chunk": 256}, True),                                            # short walks
+    ([(2100, 30)], 16, {}, False),                                                      # many keys
+    ([(2100, 30)], 32, {}, True),                                                       # but pages of 32
+    ([(0, 1400)], 32, {"chunk": 256, "keep": 5}, False),
+])
+def test_the_plan_and_its_kernel(reqs, page_size, mask, one_group):
+    """The backend's plan at head size 256 on each side of the rule: its items and the form it names belong together (an item of
+    two groups in the form of one would leave half its rows out)."""
+    nq, nkv, d = 16, 1, 256
+    g = torch.Generator().manual_seed(7)
+    bf = torch.bfloat16
+    ks, vs = ([torch.randn(c + n, nkv, d, generator=g).to(bf).float() for c, n in reqs] for _ in range(2))
+    qs = [torch.randn(n, nq, d, generator=g).to(bf).float() for _, n in reqs]
+    *pages, tables = build_paged(ks, vs, page_size)
+    sinks, plans = torch.linspace(-1.0, 2.0, nq), []
+    out = run_step((nq, nkv, d, page_size), reqs, pages, tables, qs, **mask, cap=4.0, sinks=sinks.cuda(), dtype=bf, plans=plans)
+    plan, = plans
+    assert plan.one_group == one_group
+    assert bool((plan.prefill_work.view(-1, 3)[:, 2] >= 0).any()) == (not one_group)
+    want = torch.cat([reference(q, k, v, torch.arange(c, c + n), d ** -0.5, mask.get("window"), mask.get("chunk"), mask.get("keep", 0), 4.0, sinks)
+                      for q, k, v, (c, n) in zip(qs, ks, vs, reqs)]).reshape(-1, nq * d)
+    torch.testing.assert_close(out.double(), want, rtol=2e-2, atol=2e-2)

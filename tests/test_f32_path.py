@@ -127,8 +127,9 @@ def test_f32_work_items_hold_every_row_once():
         assert items[0][0] == 0                                          # the request with the most keys first
 
 
-def run_step(case_sizes, reqs, pages, tables, queries, window=None, chunk=None, keep=0, cap=None, sinks=None):
-    """A step of these requests [(cached, new)] through the backend, with its own plan: the kernel's choice of blocks included."""
+def run_step(case_sizes, reqs, pages, tables, queries, window=None, chunk=None, keep=0, cap=None, sinks=None, dtype=torch.float32, plans=None):
+    """A step of these requests [(cached, new)] through the backend, with its own plan: the kernel's choice of blocks included.
+    ``plans``: a list that receives the step's plan."""
     from types import SimpleNamespace
 
     from jax_vllm_amd.parts import attention_backend
@@ -147,9 +148,11 @@ def run_step(case_sizes, reqs, pages, tables, queries, window=None, chunk=None, 
                        slot_ids_host=[0] * len(reqs), max_q_len=max(lens), max_kv_len=max(c + n for c, n in reqs))
     att = SimpleNamespace(nq=nq, nkv=nkv, d=d, window=window, chunk=chunk, q_row_stride=nq * d, sinks=sinks, softcap=cap, keep_first=keep,
                           scale=d ** -0.5)
-    out = torch.full((sum(lens), nq * d), float("nan")).cuda()
-    attention_backend.run(att, out, torch.cat(queries).reshape(sum(lens), nq * d).cuda(), step,
-                          LayerMemory(pages={"k": pages[0].cuda(), "v": pages[1].cuda()}, group=0))
+    out = torch.full((sum(lens), nq * d), float("nan"), dtype=dtype).cuda()
+    attention_backend.run(att, out, torch.cat(queries).reshape(sum(lens), nq * d).to(dtype).cuda(), step,
+                          LayerMemory(pages={"k": pages[0].to(dtype).cuda(), "v": pages[1].to(dtype).cuda()}, group=0))
+    if plans is not None:
+        plans.extend(step.plans.values())
     return out.cpu()
 
 
