@@ -30,15 +30,13 @@ def _suffix(dtype: torch.dtype) -> str:
 
 
 # An eager step is launched call by call, and a short prompt's kernels are shorter than what a careless wrapper costs (37 tokens
-# through 36 layers: 330 launches, 4.6 ms of kernels): these four run several times per launch.
-_raw_stream, _device_index = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
-
-
+# through 36 layers: 330 launches, 4.6 ms of kernels): these run several times per launch.
 def _stream() -> c_void_p:
-    """torch's current stream, without the Python object around it (with the checks below 2.7 of the 17 us that a launch took)."""
+    """torch's current stream, without the Python object around it (with the checks below 2.7 of the 17 us that a launch took).
+    Asked of torch at the call: a torch without a GPU build, which can plan but not launch, has no such names."""
     if not torch.cuda.is_initialized():
         torch.cuda.init()
-    return c_void_p(_raw_stream(_device_index()))
+    return c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
 
 
 def _ptr(t) -> c_void_p:

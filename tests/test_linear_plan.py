@@ -75,3 +75,19 @@ def test_plans_at_the_sizes_they_were_measured_at():
     assert plan(8, 10240, 5120, partial_ok=True) == ((0, 0, 0), 1)              # wider than the norm adds parts of ...
     assert plan(8, 10240, 5120, partial_ok=True, partial_max_width=None) == ((-2, 256, 5), 4)   # ... but the rotation kernel does
     assert plan(8, 4096, 4100) is None                                          # inner size no multiple of 8
+
+
+def test_the_plans_need_no_gpu_build_of_torch():
+    """The module imports, and plans are made, where torch has none of the names that a launch asks it for."""
+    import subprocess
+    import sys
+
+    code = ("import torch\n"
+            "for name in [n for n in dir(torch._C) if n.startswith('_cuda_')]:\n"
+            "    delattr(torch._C, name)\n"
+            "from jax_vllm_amd.ops import kernels as K\n"
+            "from jax_vllm_amd.parts.attention_backend import prefill_work_items\n"
+            "assert K.streaming_plan(8, 4096, 4096, partial_ok=True) and K.ring_plan(64, 24576, 4096, 'pairs')\n"
+            "assert prefill_work_items([70], [0], 4, 0, 64, 2)\n")
+    run = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    assert run.returncode == 0, run.stderr
