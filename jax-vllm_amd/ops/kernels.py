@@ -1121,7 +1121,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
     else:
         _need(x.dtype == w.dtype, "x and w must have one type")
         m, (n, k) = x.shape[0], w.shape
-        if SKINNY_AUTO_ROWS < m <= STREAM_MAX_ROWS and scale is None and w.dtype == torch.bfloat16:
+        # (chunks of 64 columns; tensors of other inner sizes are never asked for their device's compute units)
+        if k % 64 == 0 and SKINNY_AUTO_ROWS < m <= STREAM_MAX_ROWS and scale is None and w.dtype == torch.bfloat16:
             parts_ok = partial_ok and not gate_pairs and out_dtype in (None, torch.bfloat16) and (
                 partial_max_width is None or n <= partial_max_width)
             mode = "pairs" if gate_pairs else "parts" if parts_ok and k >= 128 else "rows"
@@ -1129,7 +1130,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
             if form is not None and out_dtype in (None, torch.bfloat16, torch.float32) and x.is_contiguous() and w.is_contiguous() \
                     and not (x.data_ptr() | w.data_ptr()) & 15 and not (gate_pairs and out_dtype == torch.float32):
                 return gemm_stream(x, w, form, mode, gate_pairs, out_dtype or torch.bfloat16)
-        elif m > STREAM_MAX_ROWS and partial_ok and not gate_pairs and scale is None and w.dtype == torch.bfloat16 \
+        elif k % 64 == 0 and m > STREAM_MAX_ROWS and partial_ok and not gate_pairs and scale is None and w.dtype == torch.bfloat16 \
                 and out_dtype in (None, torch.bfloat16) and partial_max_width is not None and n <= partial_max_width:
             form = shares_plan(m, n, k, compute_units(x.device))
             if form is not None and x.is_contiguous() and w.is_contiguous() and not (x.data_ptr() | w.data_ptr()) & 15:

@@ -7,6 +7,8 @@ import pytest
 
 from jax_vllm_amd.ops import kernels as K
 
+from .conftest import ROOT
+
 ROWS = [1, 2, 3, 8, 9, 16, 17, 32, 33, 64, 65, 200]
 WIDTHS = [16, 64, 520, 1024, 2048, 2560, 4096, 5120, 6144, 7168, 8192, 8200, 10240, 24576, 34816, 51200, 151936]
 INNER = [8, 256, 264, 512, 1000, 1024, 1536, 2048, 2560, 3072, 4096, 5120, 6152, 8192, 9728, 12288, 17408, 25600]
@@ -89,5 +91,16 @@ def test_the_plans_need_no_gpu_build_of_torch():
             "from jax_vllm_amd.parts.attention_backend import prefill_work_items\n"
             "assert K.streaming_plan(8, 4096, 4096, partial_ok=True) and K.ring_plan(64, 24576, 4096, 'pairs')\n"
             "assert prefill_work_items([70], [0], 4, 0, 64, 2)\n")
-    run = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
+    run = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300, cwd=ROOT)
     assert run.returncode == 0, run.stderr
+
+
+@pytest.mark.parametrize("m", [8, 20, 64, 200])
+def test_inner_sizes_of_no_kernel_are_taken_on_the_host_too(m):
+    """An inner size that is no multiple of 8 goes to the library on whatever device it lies."""
+    import torch
+
+    x, w = torch.randn(m, 12).bfloat16(), torch.randn(16, 12).bfloat16()
+    for partial_ok in (False, True):
+        y = K.linear(x, w, partial_ok=partial_ok)
+        assert torch.equal(y, torch.mm(x, w.t()))
