@@ -200,3 +200,44 @@ def test_the_ranges_that_a_work_item_may_touch():
                     begin = begin // 16 * 16                                       # whole tiles
                     touched = {j // 256 for j in list(range(min(keep, begin))) + list(range(begin, last + 1))}
                     assert len(touched) <= bound, (kv_len, window, keep, rows, last)
+
+
+@pytest.mark.gpu
+def test_a_request_s_logits_do_not_depend_on_its_company():
+    """A dense model in 32 bits through the engine: a prompt's portions and decoded tokens, alone and beside others, to the bit
+    (steps of 256 tokens and more prepare heads by another kernel, so both walks cut alike)."""
+    import numpy as np
+
+    from jax_vllm_amd import LLM
+    from jax_vllm_amd.engine.entries import StepEntry
+
+    cfg = dict(architectures=["Qwen3ForCausalLM"], hidden_size=256, num_attention_heads=8, num_key_value_heads=2, head_dim=64,
+               intermediate_size=384, vocab_size=512, num_hidden_layers=3, rope_theta=1e6, rms_norm_eps=1e-6, tie_word_embeddings=False,
+               max_position_embeddings=4096)
+    rng = np.random.default_rng(3)
+    mine = rng.integers(0, 512, size=640).tolist()
+    others = [rng.integers(0, 512, size=n).tolist() for n in (3, 900, 40, 333, 17, 600, 64, 5, 128, 450)]
+
+    def walk(cuts, company):
+        """My logits at every cut's end, with the others' prompts in the first step and their tokens in the rest."""
+        llm = LLM(cfg, random_seed=5, dtype="fp32", block_size=16, num_blocks=1 + 11 * 64, max_num_seqs=11, max_model_len=1024,
+                  max_num_batched_tokens=4096, enable_prefix_cache=False)
+        core, out, at = llm.core, [], 0
+        names = ["me"] + [f"o{i}" for i in range(len(others))] if company else ["me"]
+        for name in names:
+            core.start_request(name)
+        for step, n in enumerate(cuts):
+            entries = [StepEntry("me", mine[at:at + n], [n - 1])]
+            if company:
+                entries += [StepEntry(f"o{i}", t if step == 0 else [t[step % len(t)]], [0]) for i, t in enumerate(others)]
+            if step % 2:
+                entries = entries[::-1]                    # I am the last request of every other step
+            logits = core.run(entries).cpu()
+            out.append(logits[-1] if step % 2 else logits[0])
+            at += n
+        return torch.stack(out)
+
+    cuts = [300, 1, 1, 20, 1, 310] + [1] * 7
+    assert sum(cuts) == 640
+    alone = walk(cuts, False)
+    assert torch.isfinite(alone).all() and torch.equal(walk(cuts, True), alone)
