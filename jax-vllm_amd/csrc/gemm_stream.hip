@@ -9,8 +9,9 @@
 //
 // Blocks begin at different chunks and walk round (by their number on their XCD, which takes every eighth block): in
 // lockstep all units would ask for the same 128-byte columns of rows that lie a power of two apart, which few channels
-// hold (24,576 x 4,096 at 64 rows: 50.6 us in lockstep, 40.2 so).  Which chunk comes first depends on the columns
-// of y alone, so a row's result does not depend on the other rows.
+// hold (24,576 x 4,096 at 64 rows: 50.6 us in lockstep, 40.2 so).  In one form (rows of x, rows of W, shares) which
+// chunk comes first depends on the columns of y alone, so a row's result does not depend on the other rows; the form is
+// chosen by their number.
 //
 // Measured at 64 rows, microseconds (before; a plain read of W): 24,576 x 4,096 with its activation 40.2 (52.3; 33.6),
 // 4,096 x 12,288 25.5 (32.8; 16.8), 4,096 x 4,096 11.6 (13.4; 5.6), 6,144 x 4,096 14.0 (17.6; 8.4); at 128 rows 46.9 (57.1),

@@ -904,18 +904,16 @@ def streaming_plan(m: int, n: int, k: int, gate_pairs: bool = False, partial_ok:
       blocks wherever a piece count fits the inner size (4,096 x 12,288 at 8 rows: 20.7 us against 24.9
       with x resident in LDS; 5,120 x 17,408: 35.9 against 40.8; 5,120 x 8,192: 17.9 against 20.0), x
       resident in LDS otherwise (5,120 x 25,600, which would need more than 4 groups);
-    * the same at 17..64 rows when every block gets at least 3,072 columns: blocks of 64 rows of w,
-      one per compute unit (the feed-forward's second product: 4,096 x 12,288 at 64 rows 30 us
-      against the library's 37; 5,120 x 17,408 65 against 131; 5,120 x 25,600 91 against 157);
-    * 17..64 rows against narrow matrices with a short inner size (the attention's products): staying
-      blocks, one per compute unit, with two to four row tiles of x in registers (up to 8 pieces a
-      wave for two, 5 for more), the inner size shared out to 4 groups (4,096 x 4,096: 10.3 us at
-      32 rows, 13.2 at 64, against the library's 13.0 and 15.0; 5,120 x 5,120 at 48 rows: 16.5
-      against 26.6);
-    * 17..32 rows against wide matrices with an inner size of 12 or 16 pieces a wave (gate and up, the output
-      embedding): staying blocks with two row tiles of x in registers and W in four slots (24,576 x 4,096
-      with the activation at 24 rows 41.9 us, at 32 rows 43.7, against 47.5 and 47.2 by the library and the
-      activation kernel; 151,936 x 4,096 at 24 rows 248 against 270);
+    * 17..64 rows, where ``linear`` asks ``ring_plan`` first and comes here for what that leaves:
+      - narrow matrices with a short inner size (the attention's products): staying blocks, one per compute unit, with two to
+        four row tiles of x in registers (up to 8 pieces a wave for two, 5 for more), the inner size shared out to 4 groups
+        (4,096 x 4,096 at 24 rows 10.2 us against the ring's 10.6 and the library's 13.0);
+      - narrow matrices that the ring does not take (an inner size that is no multiple of 64, rows of x that are a view, operands
+        off 16 bytes), when every block gets at least 3,072 columns: blocks of 64 rows of w, one per compute unit (``TILE64``;
+        4,096 x 12,288 at 64 rows 30 us against the library's 37; the ring takes 24.6);
+      - up to 32 rows against wide matrices with an inner size of 12 or 16 pieces a wave: staying blocks with two row tiles of x
+        in registers and W in four slots (24,576 x 4,096 with the activation at 24 rows 44.7 us against 47.5 by the library and
+        the activation kernel; the ring takes 41.8);
     * one or two rows against very wide matrices (the output embedding): x resident in LDS (chosen
       inside the kernel library; 1.24 GB in 202 us against 205);
     * 9..16 rows of a large matrix that fits none of these: the library (its wider tiles amortise
@@ -1066,7 +1064,7 @@ def shares_plan(m: int, n: int, k: int, cus: int = 256):
     140 and 9 for the parts / 147.  Results of up to 262,144 numbers are the library's, which takes less there than the count says
     (with the norm that reads them, 256 rows against 1,024 x 3,072: 16.5 / 13.4, 200 against 768 x 3,072 14.6 / 13.3; 257 against
     1,024 x 3,072 14.9 / 18.5).  Of 336 sizes 9 are then slower than the library by more than 2 %, at most 10 %; the mean is 0.86."""
-    if not STREAM_MAX_ROWS < m <= SHARES_MAX_ROWS or k % 64 or n % 4 or n * k < 500_000 or m * n <= 262_144:
+    if not STREAM_MAX_ROWS < m <= SHARES_MAX_ROWS or k % 64 or n % 4 or n * k < 500_000 or m * n <= 262_144:      # 500,000: as in ring_plan
         return None
     best = None
     for (tm, tw), chunk in _SHARES_TILES.items():
@@ -1102,8 +1100,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
     """x @ w.T for w stored [out, in].
 
     float32: the library's own kernel in true 32-bit (no reduced-precision matrix mode).
-    bfloat16, at most 16 rows (and some shapes up to 64): a weight-streaming MFMA kernel of this
-    library (``streaming_plan``); 17 to 128 rows: chunks of x and w through a ring in LDS (``ring_plan``).
+    bfloat16, at most 16 rows: a weight-streaming MFMA kernel of this library (``streaming_plan``); 17 to 128 rows: chunks
+    of x and w through a ring in LDS (``ring_plan``), or what ``streaming_plan`` has for what that leaves.
     bfloat16 otherwise: a plain library matrix product (hipBLASLt through torch), float accumulation.
     With ``partial_ok`` the caller takes a float32 stack [parts, M, N] of partial products as well
     (to be added in order, as ``add_rmsnorm`` does); it is returned for narrow matrices at up to 128 rows, and up to 1,024
