@@ -30,13 +30,16 @@ def _suffix(dtype: torch.dtype) -> str:
 
 
 # An eager step is launched call by call, and a short prompt's kernels are shorter than what a careless wrapper costs (37 tokens
-# through 36 layers: 330 launches, 4.6 ms of kernels): these run several times per launch.
+# through 36 layers: 330 launches, 4.6 ms of kernels): these four run several times per launch.  A torch without a GPU build, which can
+# plan but not launch, has neither name.
+_raw_stream, _device_index = (getattr(torch._C, name, None) for name in ("_cuda_getCurrentRawStream", "_cuda_getDevice"))
+
+
 def _stream() -> c_void_p:
-    """torch's current stream, without the Python object around it (with the checks below 2.7 of the 17 us that a launch took).
-    Asked of torch at the call: a torch without a GPU build, which can plan but not launch, has no such names."""
+    """torch's current stream, without the Python object around it (with the checks below 2.7 of the 17 us that a launch took)."""
     if not torch.cuda.is_initialized():
         torch.cuda.init()
-    return c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
+    return c_void_p(_raw_stream(_device_index()))
 
 
 def _ptr(t) -> c_void_p:
