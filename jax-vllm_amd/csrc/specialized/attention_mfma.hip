@@ -531,10 +531,10 @@ __global__ void __launch_bounds__(256) PREFILL_OCCUPANCY attn_prefill_kernel(Att
 #endif  // JV_PREFILL16
 
 // ------------------------------------------------------------------------------------ prefill, 32-row tiles
-// Head sizes that are multiples of 32 up to 128 take this kernel, and 256 where the prompts fill the chip or see many keys
-// (one wave a SIMD then; half the LDS reads a row of the 16-row tiles: 16 heads over one kv head, 2,048 tokens with a window of
+// Head sizes that are multiples of 32 up to 128 take this kernel, and 256 where the prompts fill the chip and, with pages of 16, see
+// more than 256 keys, or with pages of 16 see 2,048 (one wave a SIMD then; half the LDS reads a row of the 16-row tiles: 16 heads over one kv head, 2,048 tokens with a window of
 // 1,024: 73 against 107 us, 8 kv heads and 8,192 tokens 772 against 1,414, 512 tokens after 4,000 183 against 200; where it
-// starts up in vain: 300 tokens 26 against 20).  It reads the same work items
+// starts up in vain: 300 tokens 26 against 20, a window of 128 39 against 34).  It reads the same work items
 // (two groups of 64 rows) but gives every wave ONE tile of 32 rows (waves 0, 1: first group,
 // waves 2, 3: second group) and multiplies with v_mfma_f32_32x32x16_bf16: a 16-byte fragment of K
 // or V^T read from LDS then feeds a product of 32 cycles, twice as much as with 16x16x32 tiles
