@@ -1,173 +1,439 @@
-// C[M,N] = A[M,K] * W[N,K]^T in true 32-bit: float inputs, float products and sums on the matrix cores
-// (v_mfma_f32_16x16x4_f32), no reduced-precision matrix mode.
+// C[M,N] = A[M,K] * W[N,K]^T in 32 bits: float inputs, float sums, on the bf16 matrix unit without losing a bit of the inputs.
 //
-// Order of the sums: the inner size is cut into 8 parts of equal length (a multiple of 16); a part is summed in
-// ascending steps of 16 columns (inside a step columns j, j + 4, j + 8, j + 12 enter together), the parts' sums are added
-// in ascending order.  That order depends on K alone, so a row's result depends neither on the other rows of the
-// batch nor on the tile that computes it, and eight short chains err less than one long one.
+// A float is the sum of three bf16 numbers (8 bits each: the nearest bf16, the nearest to what that leaves, the rest).  Of the
+// nine products of two such sums the six largest are taken; the others are below 2^-26 of the whole.  The bf16 unit makes 13
+// times the products of the 32-bit one, so six of its instructions take half the time of one of the 32-bit unit's.
 //
-// A block's 8 waves take one part of the inner size each, all for the same tile of (16 NT) rows of W by (16 MT) rows of
-// A; operands go from global memory straight into the matrix unit's registers (a lane's 16 bytes are 4 columns of one row:
-// four products), one stage of U steps ahead of their use; the parts meet in LDS once, at the end.  Nothing waits for
-// another wave inside the loop, and a decode step's narrow products still have 8 waves a row tile pulling at W.
-// A 16 x 16 x 4 product keeps its unit busy for 32 cycles, so at 4 x 4 tiles a wave needs 8 KB per 2,048 cycles and the
-// kernel is bound by the matrix unit; at few rows it is bound by the stream of W.
+// Order of the sums: steps of 32 columns; a step's six products are summed from the smallest on by themselves, from zero; the
+// inner size is cut into two halves of whole steps, a half's steps are added in ascending order, then the halves.  That
+// order depends on K alone, so a row's result depends neither on the other rows of the batch nor on the kernel that computes
+// it.  Error against 64 bits over normal, positive and wide (e^3N) inputs, K 32 to 4,096: 0.4 to 0.8 of that of one 32-bit
+// matrix product after another (relative 2-norm at 1,003 x 2,048 x 2,048 1.3e-7, before 2.9e-7).
+//
+// A sum that is not finite may come from the split (a value above the largest bf16, infinity less itself): it is made again
+// from the numbers themselves.  Numbers below 2^-110 lose their last terms to the range of bf16.
+//
+// Microseconds, before with the 32-bit instruction: 5 rows against 2,048 x 2,048 10.9 -> 8.8, 6,144 x 2,048 16.4 -> 13.3 (50 MB:
+// the stream of W); 16 rows 13.5 -> 9.1, 18.5 -> 13.4; 300 x 6,144 x 2,048 121 -> 75; 1,003 x 6,144 x 2,048 226 -> 150 with the 5 that the terms
+// of A take; 2,048 x 24,576 x 4,096 3,430 -> 2,222 = 186 TFLOP/s of 32-bit products, 1.1 PFLOP/s of the matrix unit's.
 #include "common.h"
 
-typedef float g32_f4 __attribute__((ext_vector_type(4)));
-typedef float g32_f4u __attribute__((ext_vector_type(4), aligned(4)));      // 16 bytes from any address of a float
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));      // 16 bytes from any address of a float
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-#define G32_PARTS 8
-#define G32_ROUND_TILES 8      // 16 x 16 tiles that meet in LDS at once: 64 KB
+#define G32_STEP 32            // columns of a step and of v_mfma_f32_16x16x32_bf16
 
-template <int NT, int MT, int U>
-__global__ void __launch_bounds__(64 * G32_PARTS)
-gemm_f32_kernel(float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ W,
-                int M, int N, int K, long long lda, long long ldw, long long ldc) {
-  constexpr int TILES = NT * MT;
-  constexpr int ROUND = TILES < G32_ROUND_TILES ? TILES : G32_ROUND_TILES;
-  __shared__ g32_f4 red[ROUND][G32_PARTS][64];
-  const int tid = threadIdx.x, part = tid >> 6, lane = tid & 63, li = lane & 15, lq = lane >> 4;
-  const int n0 = blockIdx.x * (16 * NT), m0 = blockIdx.y * (16 * MT);
-  const int len = ((K + G32_PARTS - 1) / G32_PARTS + 15) / 16 * 16;
-  const int k_begin = part * len;
-  const int k_end = k_begin + len < K ? k_begin + len : K;
-
-  // rows behind the last one read the last one's numbers; their results are not stored
-  const float* wrow[NT];
-  const float* arow[MT];
+// Pair i of a lane's 8 numbers: its part of the three terms.
+__device__ __forceinline__ void split_pair(float a, float b, int i, u32x4 (&t)[3]) {
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int n = n0 + t * 16 + li;
-    wrow[t] = W + (long long)(n < N ? n : N - 1) * ldw + lq * 4;
+  for (int e = 0; e < 3; ++e) {
+    t[e][i] = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){a, b}, bf16x2));
+    if (e < 2) {
+      a -= __uint_as_float(t[e][i] << 16);
+      b -= __uint_as_float(t[e][i] & 0xffff0000u);
+    }
   }
+}
+__device__ __forceinline__ void split8(const f32x4 (&v)[2], u32x4 (&t)[3]) {
 #pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    const int m = m0 + t * 16 + li;
-    arow[t] = A + (long long)(m < M ? m : M - 1) * lda + lq * 4;
+  for (int i = 0; i < 4; ++i) split_pair(v[i / 2][i % 2 * 2], v[i / 2][i % 2 * 2 + 1], i, t);
+}
+// The products of a step, (term of w, term of x), from the smallest on.
+#define G32_PRODUCTS 6
+__device__ constexpr int G32_W[G32_PRODUCTS] = {0, 1, 2, 0, 1, 0}, G32_X[G32_PRODUCTS] = {2, 1, 0, 1, 0, 0};
+__device__ __forceinline__ f32x4 mfma(const u32x4& w, const u32x4& x, const f32x4& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, x), c, 0, 0, 0);
+}
+__device__ __forceinline__ float settle(float sum, const float* a, const float* w, int K) {
+  if (!(__builtin_fabsf(sum) <= 3.402823466e38f)) {
+    sum = 0.f;
+    int k = 0;
+    for (; k + 8 <= K && sum == sum; k += 8) {      // a NaN stays one
+      float p[8], q[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) p[e] = a[k + e], q[e] = w[k + e];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sum = fmaf(p[e], q[e], sum);
+    }
+    for (; k < K && sum == sum; ++k) sum = fmaf(a[k], w[k], sum);
   }
-  // a lane's 4 columns k + 4 lq .. + 3 of a step that may reach beyond K: zeros there, in both operands
-  auto load4_tail = [&](const float* row, int k) -> g32_f4 {
-    g32_f4 v = {0.f, 0.f, 0.f, 0.f};
+  return sum;
+}
+// 16 bytes a lane from base + off straight into LDS, 1 KB in the order of the lanes from `at` on.
+__device__ __forceinline__ void lds_load(unsigned off, const void* base, unsigned at) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(at) : "memory", "m0");
+}
+__device__ __forceinline__ unsigned lds_address(const void* p) {
+  return (unsigned)(unsigned long long)(const __attribute__((address_space(3))) void*)p;
+}
+
+// ---------------------------------------------------------------------------- few rows
+// A block takes TW rows of W by XR rows of A; its 8 waves share out the steps (waves 0 to 3 every fourth of the first half, 4 to
+// 7 of the second), each through a ring of its own in LDS, straight from memory, S steps on their way, no wave waiting for
+// another but once in R steps of each, when the steps' sums meet in LDS and are added in their order.
+// DMA false: operands through registers, a round ahead, for rows that do not begin on 16 bytes.
+template <int TW, int XR, int S, int R, bool DMA>
+__global__ void __launch_bounds__(512)
+gemm_f32_few_kernel(float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K) {
+  constexpr int ROWS = TW + XR, L = ROWS / 8, BUF = ROWS * G32_STEP, NT = TW / 16, MT = XR / 16, TILES = NT * MT;
+  static_assert(TW % 16 == 0 && XR % 16 == 0 && TILES <= 4 && L * (S - 1) <= 63, "a wave adds a tile; what s_waitcnt counts to");
+  __shared__ __attribute__((aligned(1024))) float bufs[DMA ? 8 * S * BUF : 4];
+  __shared__ f32x4 met[2][2][4 * R][TILES][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wave >> 2, turn = wave & 3;
+  const int li = lane & 15, lq = lane >> 4, n0 = blockIdx.x * TW, m0 = blockIdx.y * XR;
+  const int total = (K + G32_STEP - 1) / G32_STEP, first = half ? (total + 1) / 2 : 0, steps = half ? total / 2 : (total + 1) / 2;
+  // piece c of row r lies at slot c ^ (r % 8); a row's last step may have fewer pieces than 8: the last one again for those
+  const int piece = ((lane & 7) ^ (lane >> 3)) * 16, beyond = max(piece + 16 - (K * 4 - (total - 1) * G32_STEP * 4), 0);
+  unsigned off[L];
+  const float* row[NT + MT];
+  if constexpr (DMA) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (k + lq * 4 + e < K) v[e] = row[k + e];
-    return v;
+    for (int j = 0; j < L; ++j) {
+      const int r = (j < TW / 8 ? j : j - TW / 8) * 8 + (lane >> 3);
+      const int at = j < TW / 8 ? min(n0 + r, N - 1) - n0 : min(m0 + r, M - 1) - m0;      // rows behind the last one repeat it
+      off[j] = (unsigned)at * (unsigned)(K * 4) + piece;
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) row[t] = W + (long long)min(n0 + t * 16 + li, N - 1) * K;
+#pragma unroll
+    for (int t = 0; t < MT; ++t) row[NT + t] = A + (long long)min(m0 + t * 16 + li, M - 1) * K;
+  }
+  const float* ws = W + (long long)n0 * K;
+  const float* xs = A + (long long)m0 * K;
+  float* ring = bufs + (DMA ? wave * S * BUF : 0);
+  const unsigned lds0 = lds_address(ring);
+  auto dma = [&](int i, int slot) {      // the wave's step i; behind the last one the last step of all again
+    const int s = min(first + turn + 4 * i, total - 1), less = s == total - 1 ? beyond : 0;
+#pragma unroll
+    for (int j = 0; j < L; ++j) lds_load(off[j] - less, (j < TW / 8 ? ws : xs) + s * G32_STEP, lds0 + slot * (BUF * 4) + j * 1024);
   };
+  const int wrow = li * G32_STEP, xrow = (TW + li) * G32_STEP;
+  const int p0 = ((2 * lq) ^ (li & 7)) * 4, p1 = ((2 * lq + 1) ^ (li & 7)) * 4;
+  // without the ring: a round's numbers, those beyond K zeros
+  f32x4 ahead[DMA ? 1 : R][NT + MT][2];
+  auto load_round = [&](int s0) {
+#pragma unroll
+    for (int r = 0; r < (DMA ? 0 : R); ++r) {
+      const int k0 = (first + turn + s0 + 4 * r) * G32_STEP + lq * 8;
+#pragma unroll
+      for (int t = 0; t < NT + MT; ++t) {
+        if (k0 + 8 <= K) {
+          ahead[r][t][0] = *(const f32x4u*)(row[t] + k0), ahead[r][t][1] = *(const f32x4u*)(row[t] + k0 + 4);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) ahead[r][t][e / 4][e % 4] = k0 + e < K ? row[t][k0 + e] : 0.f;
+        }
+      }
+    }
+  };
+  if constexpr (DMA)
+    for (int v = 0; v < S; ++v) dma(v, v);
+  else load_round(0);
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  int slot = 0;
+  const int longest = (total + 1) / 2;
+  for (int s0 = 0, round = 0; s0 < longest; s0 += 4 * R, round ^= 1) {
+    f32x4 now[DMA ? 1 : R][NT + MT][2];
+    if constexpr (!DMA) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int t = 0; t < NT + MT; ++t) now[r][t][0] = ahead[r][t][0], now[r][t][1] = ahead[r][t][1];
+      load_round(s0 + 4 * R);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      f32x4 raw[NT + MT][2];
+      if constexpr (DMA) {
+        const int i = s0 / 4 + r;
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * L) : "memory");
+        const float* b = ring + slot * BUF;
+#pragma unroll
+        for (int t = 0; t < NT + MT; ++t) {
+          const float* at = b + (t < NT ? wrow + t * 16 * G32_STEP : xrow + (t - NT) * 16 * G32_STEP);
+          raw[t][0] = *(const f32x4*)(at + p0), raw[t][1] = *(const f32x4*)(at + p1);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // read before the slot is filled again
+        dma(i + S, slot);
+        slot = slot + 1 == S ? 0 : slot + 1;
+        const int k0 = (first + turn + 4 * i) * G32_STEP;
+        if (k0 + G32_STEP > K) {      // zeros of A beyond K: what W repeats there does not count
+#pragma unroll
+          for (int t = NT; t < NT + MT; ++t)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+              if (k0 + lq * 8 + h * 4 >= K) raw[t][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      } else {
+#pragma unroll
+        for (int t = 0; t < NT + MT; ++t) raw[t][0] = now[r][t][0], raw[t][1] = now[r][t][1];
+      }
+      u32x4 wt[NT][3], xt[3];
+#pragma unroll
+      for (int a = 0; a < NT; ++a) split8(raw[a], wt[a]);
+#pragma unroll
+      for (int b = 0; b < MT; ++b) {
+        split8(raw[NT + b], xt);
+        f32x4 t[NT];
+#pragma unroll
+        for (int e = 0; e < G32_PRODUCTS; ++e)
+#pragma unroll
+          for (int a = 0; a < NT; ++a) t[a] = mfma(wt[a][G32_W[e]], xt[G32_X[e]], e ? t[a] : zero);
+#pragma unroll
+        for (int a = 0; a < NT; ++a) met[round][half][4 * r + turn][a * MT + b][lane] = t[a];
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();      // (the buffer of the round before the last was read before the last round's barrier)
+    asm volatile("" ::: "memory");
+    if (turn < TILES) {
+#pragma unroll
+      for (int s = 0; s < 4 * R; ++s)
+        if (s0 + s < steps) sum += met[round][half][s][turn][lane];
+    }
+  }
+  if constexpr (DMA) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // nothing on its way to this LDS when the block ends
+  __syncthreads();
+  if (half && turn < TILES) met[0][1][0][turn][lane] = sum;
+  __syncthreads();
+  if (half || turn >= TILES) return;
+  sum += met[0][1][0][turn][lane];
+  const int m = m0 + turn % MT * 16 + li, n = n0 + turn / MT * 16 + lq * 4;      // a lane holds C[m][n .. n + 3]
+  if (m >= M) return;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (n + e < N) C[(long long)m * N + n + e] = settle(sum[e], A + (long long)m * K, W + (long long)(n + e) * K, K);
+}
 
-  g32_f4 acc[NT][MT];
+// ---------------------------------------------------------------------------- many rows
+// The rows of A as their three terms, [M][steps][term][32]: made once for all the blocks that multiply a row.
+__global__ void __launch_bounds__(256)
+split_rows_kernel(unsigned* __restrict__ y, const float* __restrict__ A, int K, int steps) {
+  const int k = (blockIdx.y * 256 + threadIdx.x) * 8;
+  if (k >= steps * G32_STEP) return;
+  const float* a = A + (long long)blockIdx.x * K + k;
+  f32x4 v[2];
+  if (k + 8 <= K && ((uintptr_t)a & 15) == 0) {
+    v[0] = *(const f32x4*)a, v[1] = *(const f32x4*)(a + 4);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e / 4][e % 4] = k + e < K ? a[e] : 0.f;
+  }
+  u32x4 t[3];
+  split8(v, t);
+  u32x4* out = (u32x4*)y + ((long long)blockIdx.x * steps + k / G32_STEP) * 12 + k % G32_STEP / 8;
+#pragma unroll
+  for (int e = 0; e < 3; ++e) out[e * 4] = t[e];
+}
+
+// Tiles of TM rows of A (as terms) by TW rows of W (as floats); two groups of 2 x 2 waves take a half of the steps each, through
+// rings of S steps in LDS.  Bound by what a SIMD issues: a product of 16 cycles takes 8 of them, a vector instruction 2 to 4
+// (measured), so a wave splits the next 16 rows of W (44 instructions) while it multiplies these with all its rows of A.
+template <int TM, int TW>
+__global__ void __launch_bounds__(512, 2)
+gemm_f32_tile_kernel(float* __restrict__ C, const unsigned* __restrict__ X, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K, int KA) {
+  constexpr int MT = TM / 32, NT = TW / 32, XL = TM * 3 / 64, WL = TW / 32, L = XL + WL;      // L: loads of a wave for a step
+  constexpr int XBYTES = TM * 192, BYTES = XBYTES + TW * 128, FIT = 160 * 1024 / (2 * BYTES), S = FIT < 4 ? FIT : 4;
+  static_assert(S >= 2 && XL * 64 == TM * 3 && (S - 1) * L <= 63, "");
+  __shared__ __attribute__((aligned(1024))) char bufs[2 * S * BYTES];
+  const int lane = threadIdx.x & 63, all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), group = all >> 2, wave = all & 3;
+  // Blocks b, b + 8, ... run on one XCD: each takes one run of the tiles, rows of A fastest
+  const int mtiles = (M + TM - 1) / TM, live = mtiles * ((N + TW - 1) / TW), per = (live + 7) / 8;
+  const int u = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || u >= live) return;
+  const int m0 = u % mtiles * TM, n0 = u / mtiles * TW;
+  const int total = (K + G32_STEP - 1) / G32_STEP, turns = (total + 1) / 2, first = group * turns, steps = group ? total - turns : turns;
+  // (a row's last step may have fewer pieces of W than 8: the last one again for those, against zeros of A)
+  const int piece = ((lane & 7) ^ (lane >> 3)) * 16, beyond = max(piece + 16 - (K * 4 - (total - 1) * 128), 0);
+  unsigned off[L];
+#pragma unroll
+  for (int j = 0; j < XL; ++j) {      // an instruction brings 16 rows of 64 bytes of one term; piece c of row r lies at slot c ^ (r / 2 % 4)
+    const int q = wave * XL + j, e = q / (TM / 16), r = q % (TM / 16) * 16 + (lane >> 2);
+    off[j] = (unsigned)(min(m0 + r, M - 1) - m0) * (unsigned)(total * 192) + e * 64 + (((lane & 3) ^ (r >> 1)) & 3) * 16;
+  }
+#pragma unroll
+  for (int j = 0; j < WL; ++j) {      // 8 rows of 128 bytes; piece c of row r lies at slot c ^ (r % 8)
+    const int r = (wave * WL + j) * 8 + (lane >> 3);
+    off[XL + j] = (unsigned)(min(n0 + r, N - 1) - n0) * (unsigned)(K * 4) + piece;
+  }
+  const char* xs = (const char*)X + (long long)m0 * total * 192;
+  const char* ws = (const char*)(W + (long long)n0 * K);
+  const char* ring = bufs + group * (S * BYTES);
+  const unsigned lds0 = lds_address(ring);
+  auto dma = [&](int c, int slot) {
+    const int at = min(first + c, total - 1), less = at == total - 1 ? beyond : 0;
+#pragma unroll
+    for (int j = 0; j < L; ++j)
+      lds_load(j < XL ? off[j] : off[j] - less, j < XL ? xs + at * 192 : ws + at * 128,
+               lds0 + slot * BYTES + (j < XL ? (wave * XL + j) * 1024 : XBYTES + (wave * WL + j - XL) * 1024));
+  };
+  const int wm = wave >> 1, wn = wave & 1, li = lane & 15, lq = lane >> 4;
+  const int xat = (wm * MT * 16 + li) * 64 + ((lq ^ (li >> 1)) & 3) * 16;
+  const int wrow = XBYTES + (wn * NT * 16 + li) * 128;
+  const int p0 = wrow + ((2 * lq) ^ (li & 7)) * 16, p1 = wrow + ((2 * lq + 1) ^ (li & 7)) * 16;
+  f32x4 tot[NT][MT];
 #pragma unroll
   for (int a = 0; a < NT; ++a)
 #pragma unroll
-    for (int b = 0; b < MT; ++b) acc[a][b] = g32_f4{0.f, 0.f, 0.f, 0.f};
-  auto products = [&](const g32_f4* w, const g32_f4* x) {
+    for (int b = 0; b < MT; ++b) tot[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 xt[3][MT], wt[2][3];
+  auto read_x = [&](int e, int slot) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int a = 0; a < NT; ++a)
-#pragma unroll
-        for (int b = 0; b < MT; ++b)
-          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[a][j], x[b][j], acc[a][b], 0, 0, 0);
+    for (int b = 0; b < MT; ++b) xt[e][b] = *(const u32x4*)(ring + slot * BYTES + e * (TM * 64) + xat + b * 1024);
   };
-
-  const int full = k_end > k_begin ? (k_end - k_begin) / 16 : 0;
-  const int stages = full / U;
-  if (stages > 0) {
-    g32_f4 wc[U][NT], xc[U][MT], wn[U][NT], xn[U][MT];
-    auto load_stage = [&](int s, g32_f4 (*w)[NT], g32_f4 (*x)[MT]) {
-      const int k = k_begin + s * (16 * U);
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  for (int v = 0; v < S; ++v) dma(v, v);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * L) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  {
+    const f32x4 v[2] = {*(const f32x4*)(ring + p0), *(const f32x4*)(ring + p1)};
+    split8(v, wt[0]);
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
+    for (int e = 0; e < 3; ++e) read_x(e, 0);
+  }
+  // W's rows a of step c against all rows of A; the rows that come next are read at `at` and split meanwhile
+  auto stage = [&](auto last, auto set, int a, int at, int next, bool real) {
+    constexpr bool LAST = decltype(last)::value;
+    constexpr int SET = decltype(set)::value, SLOTS = G32_PRODUCTS * MT;
+    const f32x4 v[2] = {*(const f32x4*)(ring + at + p0), *(const f32x4*)(ring + at + p1)};
+    f32x4 t[MT];
+    int pairs = 0;
 #pragma unroll
-        for (int t = 0; t < NT; ++t) w[u][t] = *(const g32_f4u*)(wrow[t] + k + u * 16);
+    for (int e = 0; e < G32_PRODUCTS; ++e) {
 #pragma unroll
-        for (int t = 0; t < MT; ++t) x[u][t] = *(const g32_f4u*)(arow[t] + k + u * 16);
+      for (int b = 0; b < MT; ++b) {
+        t[b] = mfma(wt[SET][G32_W[e]], xt[G32_X[e]][b], e ? t[b] : zero);
+        const int i = e * MT + b + 1 - MT;      // the first MT products cover the reads' way
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+          if (i > 0 && p == pairs && p * (SLOTS - MT) < i * 4) {
+            split_pair(v[p / 2][p % 2 * 2], v[p / 2][p % 2 * 2 + 1], p, wt[SET ^ 1]);
+            // the split stays between these products
+            asm volatile("" : "+v"(wt[SET ^ 1][0][p]), "+v"(wt[SET ^ 1][1][p]), "+v"(wt[SET ^ 1][2][p]));
+            ++pairs;
+          }
+        __builtin_amdgcn_sched_barrier(0);
       }
-    };
-    load_stage(0, wc, xc);
-    for (int s = 0; s < stages; ++s) {
-      load_stage(s + 1 < stages ? s + 1 : s, wn, xn);      // never skipped: a conditional prefetch would be waited for at once
-      __builtin_amdgcn_sched_barrier(0);                   // and not moved down to its use
+      if (LAST && e == 0) read_x(2, next);      // a term's last product is made: the next step's
+      if (LAST && e == 3) read_x(1, next);
+      if (LAST && e == 5) read_x(0, next);
+    }
+    if (real) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) products(wc[u], xc[u]);
+      for (int b = 0; b < MT; ++b) tot[a][b] += t[b];
+    }
+  };
+  using std::integral_constant;
+  int slot = 0;
+  auto step = [&](auto parity, int c) {
+    constexpr int P = decltype(parity)::value;
+    const int next = slot + 1 == S ? 0 : slot + 1;
+    const bool real = c < steps;
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-#pragma unroll
-        for (int t = 0; t < NT; ++t) wc[u][t] = wn[u][t];
-#pragma unroll
-        for (int t = 0; t < MT; ++t) xc[u][t] = xn[u][t];
-      }
+    for (int a = 0; a + 1 < NT; ++a) {
+      if ((P + a) & 1) stage(integral_constant<bool, false>{}, integral_constant<int, 1>{}, a, slot * BYTES + (a + 1) * 2048, next, real);
+      else stage(integral_constant<bool, false>{}, integral_constant<int, 0>{}, a, slot * BYTES + (a + 1) * 2048, next, real);
+    }
+    // step c is in registers everywhere, step c + 1 is there
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * L) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    dma(c + S, slot);
+    stage(integral_constant<bool, true>{}, integral_constant<int, (P + NT - 1) & 1>{}, NT - 1, next * BYTES, next, real);
+    slot = next;
+  };
+  if constexpr (NT % 2 == 0) {
+    for (int c = 0; c < turns; ++c) step(integral_constant<int, 0>{}, c);
+  } else {
+    for (int c = 0; c < turns; c += 2) {
+      step(integral_constant<int, 0>{}, c);
+      if (c + 1 < turns) step(integral_constant<int, 1>{}, c + 1);
     }
   }
-  for (int k = k_begin + stages * (16 * U); k < k_end; k += 16) {
-    g32_f4 w[NT], x[MT];
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  f32x4* meet = (f32x4*)bufs;
+  static_assert(TM * TW * 4 <= 2 * S * BYTES, "");
+  if (group) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) w[t] = load4_tail(wrow[t], k);
+    for (int a = 0; a < NT; ++a)
 #pragma unroll
-    for (int t = 0; t < MT; ++t) x[t] = load4_tail(arow[t], k);
-    products(w, x);
+      for (int b = 0; b < MT; ++b) meet[((a * MT + b) * 4 + wave) * 64 + lane] = tot[a][b];
   }
-
-  // the parts meet, a round of 16 x 16 tiles at a time; a lane holds C[m0 + 16 b + li][n0 + 16 a + 4 lq .. + 3]
+  __syncthreads();
+  if (group) return;
+  const bool pieces = !(N & 3) && !((uintptr_t)C & 15);
 #pragma unroll
-  for (int r0 = 0; r0 < TILES; r0 += ROUND) {
-    if (r0 > 0) __syncthreads();
+  for (int b = 0; b < MT; ++b) {
+    const int m = m0 + (wm * MT + b) * 16 + li;
+    if (m >= M) continue;
 #pragma unroll
-    for (int t = 0; t < ROUND; ++t) red[t][part][lane] = acc[(r0 + t) / MT][(r0 + t) % MT];
-    __syncthreads();
-    for (int t = part; t < ROUND; t += G32_PARTS) {
-      g32_f4 sum = red[t][0][lane];
+    for (int a = 0; a < NT; ++a) {
+      const int n = n0 + (wn * NT + a) * 16 + lq * 4;
+      f32x4 v = tot[a][b] + meet[((a * MT + b) * 4 + wave) * 64 + lane];
+      bool ok = pieces && n + 4 <= N;
 #pragma unroll
-      for (int p = 1; p < G32_PARTS; ++p) sum += red[t][p][lane];
-      const int m = m0 + (r0 + t) % MT * 16 + li, n = n0 + (r0 + t) / MT * 16 + lq * 4;
-      if (m < M) {
-        float* c = C + (long long)m * ldc + n;
-        if (n + 4 <= N && (ldc & 3) == 0 && ((uintptr_t)C & 15) == 0) {
-          *(g32_f4*)c = sum;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n + e < N) c[e] = sum[e];
-        }
-      }
+      for (int e = 0; e < 4; ++e) ok = ok && __builtin_fabsf(v[e]) <= 3.402823466e38f;
+      if (ok) *(f32x4*)(C + (long long)m * N + n) = v;
+      else
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) C[(long long)m * N + n + e] = settle(v[e], A + (long long)m * KA, W + (long long)(n + e) * K, KA);
     }
   }
 }
 
-extern "C" int jv_gemm_f32(float* C, const float* A, const float* W, int M, int N, int K,
-                           long long lda, long long ldw, long long ldc, void* stream) {
-  if (M <= 0 || N <= 0) return 0;
-  if (K < 0) return (int)hipErrorInvalidValue;
-  // The tile: all give the same bits, so it is chosen by time alone.  `us` is what a round of 256 blocks (one a compute
-  // unit) was measured to take at K = 2,048; time grows with the rounds, and with K for all alike.  So few rows take
-  // small tiles until W fills the chip (5 rows: N = 3,072 11.1 us with 1 x 1 and 13.7 with 2 x 1; N = 32,000 73 and 58), many
-  // rows the tile whose last round is fullest (1,003 rows: N = 3,072 122 us with 4 x 4 and 148 with 4 x 8; N = 2,048 84 and
-  // 79 = 107 TFLOP/s; 2,048 rows, N = 24,576, K = 4,096: 4 x 8 3.39 ms = 122 TFLOP/s, 4 x 4 4.06).
-  struct Tile { int nt, mt; float us; };
-  static const Tile tiles[] = {{1, 1, 13.f}, {2, 1, 16.3f}, {1, 2, 16.2f}, {2, 2, 22.3f}, {1, 4, 23.f}, {2, 4, 30.f}, {4, 4, 42.f}, {4, 8, 75.f}};
-  int best = 0;
-  double least = 0;
-  for (int i = 0; i < (int)(sizeof(tiles) / sizeof(tiles[0])); ++i) {
-    const long long blocks = ((long long)N + 16 * tiles[i].nt - 1) / (16 * tiles[i].nt) * (((long long)M + 16 * tiles[i].mt - 1) / (16 * tiles[i].mt));
-    const double t = (double)((blocks + 255) / 256) * tiles[i].us;
-    if (((long long)M + 16 * tiles[i].mt - 1) / (16 * tiles[i].mt) > 65535) continue;
-    if (least == 0 || t < least) best = i, least = t;
-  }
-  if (least == 0) return (int)hipErrorInvalidValue;
-#define G32_LAUNCH(NT, MT, U)                                                                             \
-  hipLaunchKernelGGL((gemm_f32_kernel<NT, MT, U>),                                                        \
-                     dim3(((long long)N + 16 * NT - 1) / (16 * NT), ((long long)M + 16 * MT - 1) / (16 * MT)), \
-                     dim3(64 * G32_PARTS), 0, (hipStream_t)stream, C, A, W, M, N, K, lda, ldw, ldc)
-  switch (best) {
-    case 0: G32_LAUNCH(1, 1, 8); break;
-    case 1: G32_LAUNCH(2, 1, 4); break;
-    case 2: G32_LAUNCH(1, 2, 4); break;
-    case 3: G32_LAUNCH(2, 2, 4); break;
-    case 4: G32_LAUNCH(1, 4, 2); break;
-    case 5: G32_LAUNCH(2, 4, 2); break;
-    case 6: G32_LAUNCH(4, 4, 1); break;
-    default: G32_LAUNCH(4, 8, 1); break;
-  }
-#undef G32_LAUNCH
+// How C is made (jv_gemm_f32): 0, 1: few rows, 16 x 16 or 32 x 32, through registers; 2 to 4: few rows through the ring, 16 x 16, 32 x 16, 32 x 32
+// (rows of W x rows of A); from 5 on tiles, 128 x 128, 128 x 96, 128 x 64, 64 x 96, 64 x 64, 64 x 32 (rows of A x rows of W).
+template <int TW, int XR, int S, int R, bool DMA>
+static int few_launch(float* C, const float* A, const float* W, int M, int N, int K, hipStream_t s) {
+  if ((M + XR - 1) / XR > 65535) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL((gemm_f32_few_kernel<TW, XR, S, R, DMA>), dim3((N + TW - 1) / TW, (M + XR - 1) / XR), dim3(512), 0, s, C, A, W, M, N, K);
   return JV_LAUNCH_CHECK();
+}
+template <int TM, int TW>
+static int tile_launch(float* C, const void* X, const float* A, const float* W, int M, int N, int K, int KA, hipStream_t s) {
+  const long long live = ((long long)M + TM - 1) / TM * (((long long)N + TW - 1) / TW);
+  if (live > 1 << 24) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL((gemm_f32_tile_kernel<TM, TW>), dim3((unsigned)((live + 7) / 8 * 8)), dim3(512), 0, s, C, (const unsigned*)X, A, W, M, N, K, KA);
+  return JV_LAUNCH_CHECK();
+}
+// Rows of A [M][KA] as terms, [M][steps][3][32] bf16 with zeros behind KA; steps = ceil(KA / 32).
+extern "C" int jv_split_rows_f32(void* X, const float* A, int M, int KA, void* stream) {
+  if (M <= 0 || KA <= 0) return 0;
+  if ((uintptr_t)X & 15) return (int)hipErrorInvalidValue;
+  const int steps = (KA + G32_STEP - 1) / G32_STEP;
+  if ((steps * G32_STEP + 2047) / 2048 > 65535) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(split_rows_kernel, dim3(M, (steps * G32_STEP + 2047) / 2048), dim3(256), 0, (hipStream_t)stream, (unsigned*)X, A, KA, steps);
+  return JV_LAUNCH_CHECK();
+}
+// A [M][KA], W [N][K], C [M][N].  K = KA but for tiles, where W may have columns behind KA (finite; as many steps of 32 as KA has).
+// X: the rows of A by jv_split_rows_f32, for tiles.
+extern "C" int jv_gemm_f32(float* C, const float* A, const float* W, const void* X, int M, int N, int K, int KA, int form, void* stream) {
+  if (M <= 0 || N <= 0) return 0;
+  const bool pieces = !(K & 3) && !((uintptr_t)W & 15) && K > 0;
+  if (K < 0 || KA > K || (KA + 31) / 32 != (K + 31) / 32) return (int)hipErrorInvalidValue;
+  if (form >= 5 ? !pieces || !X || ((uintptr_t)X & 15) || K > 1 << 22 : KA != K || (form >= 2 && (!pieces || ((uintptr_t)A & 15) || K > 1 << 24)))
+    return (int)hipErrorInvalidValue;
+  const hipStream_t s = (hipStream_t)stream;
+  switch (form) {
+    case 0: return few_launch<16, 16, 1, 2, false>(C, A, W, M, N, K, s);
+    case 1: return few_launch<32, 32, 1, 1, false>(C, A, W, M, N, K, s);
+    case 2: return few_launch<16, 16, 2, 2, true>(C, A, W, M, N, K, s);
+    case 3: return few_launch<32, 16, 1, 1, true>(C, A, W, M, N, K, s);
+    case 4: return few_launch<32, 32, 1, 1, true>(C, A, W, M, N, K, s);
+    case 5: return tile_launch<128, 128>(C, X, A, W, M, N, K, KA, s);
+    case 6: return tile_launch<128, 96>(C, X, A, W, M, N, K, KA, s);
+    case 7: return tile_launch<128, 64>(C, X, A, W, M, N, K, KA, s);
+    case 8: return tile_launch<64, 96>(C, X, A, W, M, N, K, KA, s);
+    case 9: return tile_launch<64, 64>(C, X, A, W, M, N, K, KA, s);
+    case 10: return tile_launch<64, 32>(C, X, A, W, M, N, K, KA, s);
+  }
+  return (int)hipErrorInvalidValue;
 }

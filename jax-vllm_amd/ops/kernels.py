@@ -740,8 +740,49 @@ def attn_f32(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_seqlens, c
 
 
 # --------------------------------------------------------------------------- matrix products
+F32_STEP = 32         # columns of a step of the 32-bit product
+# tiles of the 32-bit product: form, rows of a, rows of w, microseconds of a round per 1,024 columns on one unit and on all
+_F32_TILES = ((5, 128, 128, 34.0, 45.0), (6, 128, 96, 26.0, 35.0), (7, 128, 64, 19.2, 28.0), (8, 64, 96, 17.7, 22.0), (9, 64, 64, 13.1, 17.0),
+              (10, 64, 32, 7.5, 12.5))
+
+
+@functools.lru_cache(maxsize=4096)
+def f32_plan(m: int, n: int, k: int, pieces: bool = True, a_pieces: bool = True) -> int:
+    """Form of the 32-bit product (``jv_gemm_f32``).  All give the same bits, so it is the one that takes the least time by a count of
+    rounds over 256 units that meets what was measured (1 to 2,048 rows, n 256 to 32,000, k 512 to 12,288) mostly within a sixth; for example
+    k = 2,048: 5 x 2,048 8.8 us (form 2), 16 x 32,000 53 (3), 37 x 3,072 15.5 (4), 250 x 6,144 50 (8), 1,003 x 6,144 145 (6), 2,048 x 2,048 101 (5).
+    ``pieces``: rows of w begin on 16 bytes (else they are copied for tiles, and few rows go through registers); ``a_pieces``: rows of a too."""
+    q, mb = k / 1024, n * k * 4e-6
+
+    def blocks(tm, tw):
+        return -(-m // tm) * -(-n // tw)
+
+    def rounds(tm, tw, fixed, one, full, slots=256):      # a unit alone works faster than all of them
+        b = blocks(tm, tw)
+        return -(-b // slots) * (fixed + (one + (full - one) * min(1.0, b / slots)) * q)
+
+    times, through_ring = {}, pieces and a_pieces and 0 < k <= 1 << 24
+    if m <= 65535 * 16:                                           # the grid's rows
+        if through_ring:
+            times[2] = max(3 + rounds(16, 16, 1.3, 2.3, 3.2), 5 + mb / 4.2)
+            times[3] = max(3 + rounds(16, 32, 2, 3.3, 7.5, 512), 3 + mb / 5.1)      # two of these to a unit
+        else:
+            times[0] = 4 + rounds(16, 16, 2, 8, 10, 512)
+    if m <= 65535 * 32:
+        if through_ring:
+            times[4] = max(3 + rounds(32, 32, 1, 5.3, 6.2), 3 + mb / 4.9)
+        else:
+            times[1] = 4 + rounds(32, 32, 2, 16, 18, 512)
+    if m > 32 and 0 < k <= 1 << 22:
+        for form, tm, tw, one, full in _F32_TILES:
+            if blocks(tm, tw) <= 1 << 24:
+                times[form] = 10 + (0 if pieces else 10 + mb / 2) + m * k * 2e-6 + rounds(tm, tw, 1, one, full)
+    _need(bool(times), f"no 32-bit product for {m} x {n} x {k}")
+    return min(times, key=times.get)
+
+
 def gemm_f32(a: torch.Tensor, w: torch.Tensor, out=None) -> torch.Tensor:
-    """out = a @ w.T in true 32-bit (float products and sums).  a [M, K], w [N, K], both row-major."""
+    """out = a @ w.T in 32-bit: float inputs of which no bit is dropped, float sums.  a [M, K], w [N, K], both row-major."""
     _dev(a, w)
     _f32(a, "a")
     _f32(w, "w")
@@ -752,9 +793,21 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, out=None) -> torch.Tensor:
         out = torch.empty((m, n), dtype=torch.float32, device=a.device)
     _dev(out)
     _need(out.shape == (m, n) and out.dtype == torch.float32, "out must be float32 [M, N]")
-    fn = library.core().jv_gemm_f32
-    _check(fn(_ptr(out), _ptr(a), _ptr(w), c_int(m), c_int(n), c_int(k), c_longlong(k), c_longlong(k),
-              c_longlong(n), _stream()), "gemm_f32")
+    if not m or not n:
+        return out
+    pieces = not k & 3 and not w.data_ptr() & 15
+    form, lib, terms, kw = f32_plan(m, n, k, pieces, not a.data_ptr() & 15), library.core(), None, k
+    if form >= 5:      # the rows of a as sums of three bfloat16 numbers, [M, steps, 3, 32]
+        steps = -(-k // F32_STEP)
+        terms = torch.empty((m, steps, 3, F32_STEP), dtype=torch.bfloat16, device=a.device)
+        _check(lib.jv_split_rows_f32(_ptr(terms), _ptr(a), c_int(m), c_int(k), _stream()), "split_rows_f32")
+        if not pieces:
+            kw = -(-k // 4) * 4
+            copy = torch.empty((n, kw), dtype=torch.float32, device=w.device)
+            copy[:, :k], copy[:, k:] = w, 0.0
+            w = copy
+    _check(lib.jv_gemm_f32(_ptr(out), _ptr(a), _ptr(w), _ptr(terms), c_int(m), c_int(n), c_int(kw), c_int(k), c_int(form), _stream()),
+           "gemm_f32")
     return out
 
 
@@ -1102,7 +1155,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
            partial_max_width: int | None = PARTIAL_SUM_MAX_WIDTH):
     """x @ w.T for w stored [out, in].
 
-    float32: the library's own kernel in true 32-bit (no reduced-precision matrix mode).
+    float32: the library's own kernel, from which no bit of the inputs is dropped (``gemm_f32``).
     bfloat16, at most 16 rows: a weight-streaming MFMA kernel of this library (``streaming_plan``); 17 to 128 rows: chunks
     of x and w through a ring in LDS (``ring_plan``), or what ``streaming_plan`` has for what that leaves.
     bfloat16 otherwise: a plain library matrix product (hipBLASLt through torch), float accumulation.
