@@ -256,6 +256,80 @@ head_linear_mfma_kernel(bf16_t* __restrict__ y, long long ldy, int ys, const bf1
   }
 }
 
+// More rows than a block of those takes: a wave has 16 rows and 64 outputs, so an operand of x serves four products, and the
+// results go through LDS into whole lines of y (2 bytes at a time the stores took longer than the rest).  The sums keep the order
+// of the kernel above.  16 heads, 64 into 224 and 224 into 64, microseconds (before): 2,048 rows 16.6 (25.7) and 10.0 (21.4), 600 rows 7.4
+// (10.5) and 5.9 (8.6); 250 rows 4.1 (5.4) and 5.8 (4.5), where the second stays with the kernel above.
+#define HL_N 64
+__global__ void __launch_bounds__(256)
+head_linear_lines_kernel(bf16_t* __restrict__ y, long long ldy, int ys, const bf16_t* __restrict__ x, long long ldx,
+                         int xs, const bf16_t* __restrict__ W, int M, int N, int K, const bf16_t* __restrict__ g,
+                         long long ldg, int gn, bool y_pieces, bool g_pieces) {
+  __shared__ __attribute__((aligned(16))) float lines[4][16][HL_N + 4];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lc = lane >> 4;
+  const int h = blockIdx.z, n0 = blockIdx.x * HL_N, m0 = (blockIdx.y * 4 + wave) * 16;
+  if (m0 >= M) return;      // (no barrier below: a wave's lines are its own)
+  const bf16_t* wr[HL_N / 16];
+#pragma unroll
+  for (int t = 0; t < HL_N / 16; ++t) wr[t] = W + ((long long)h * N + min(n0 + t * 16 + li, N - 1)) * K;
+  const bf16_t* xr = x + (long long)min(m0 + li, M - 1) * ldx + (long long)h * xs;
+  const hl_bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  hl_f32x4 acc[HL_N / 16] = {};
+  hl_bf16x8 b = *(const hl_bf16x8*)(xr + min(lc * 8, K - 8)), w[HL_N / 16];
+#pragma unroll
+  for (int t = 0; t < HL_N / 16; ++t) w[t] = *(const hl_bf16x8*)(wr[t] + min(lc * 8, K - 8));
+  for (int k0 = 0; k0 < K; k0 += 32) {
+    const int next = min(k0 + 32 + lc * 8, K - 8);      // asked for without a condition, also behind the last step
+    const hl_bf16x8 bn = *(const hl_bf16x8*)(xr + next);
+    hl_bf16x8 wn[HL_N / 16];
+#pragma unroll
+    for (int t = 0; t < HL_N / 16; ++t) wn[t] = *(const hl_bf16x8*)(wr[t] + next);
+    const hl_bf16x8 bk = k0 + lc * 8 < K ? b : zero;
+#pragma unroll
+    for (int t = 0; t < HL_N / 16; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t], bk, acc[t], 0, 0, 0);
+    b = bn;
+#pragma unroll
+    for (int t = 0; t < HL_N / 16; ++t) w[t] = wn[t];
+  }
+#pragma unroll
+  for (int t = 0; t < HL_N / 16; ++t) *(hl_f32x4*)&lines[wave][li][t * 16 + lc * 4] = acc[t];
+  const int c = (lane & 7) * 8, n = n0 + c;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = i * 8 + (lane >> 3), m = m0 + r;
+    if (m >= M || n >= N) continue;
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; e += 4) *(hl_f32x4*)(v + e) = *(const hl_f32x4*)&lines[wave][r][c + e];
+    if (g) {
+      const bf16_t* gr = g + (long long)m * ldg + (long long)h * gn;
+      hl_bf16x8 gv;
+      if (gn == 1) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) gv[e] = gr[0];
+      } else if (g_pieces && n + 8 <= N) {
+        gv = *(const hl_bf16x8*)(gr + n);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) gv[e] = gr[min(n + e, N - 1)];
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] *= 1.f / (1.f + expf(-(float)gv[e]));
+    }
+    bf16_t* out = y + (long long)m * ldy + (long long)h * ys + n;
+    if (y_pieces && n + 8 <= N) {
+      hl_bf16x8 o;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = (bf16_t)v[e];
+      *(hl_bf16x8*)out = o;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (n + e < N) out[e] = (bf16_t)v[e];
+    }
+  }
+}
+
 extern "C" int jv_head_linear_mfma_bf16(void* y, long long ldy, int ys, const void* x, long long ldx, int xs,
                                         const void* W, int M, int N, int K, int heads, const void* g, long long ldg,
                                         int gn, void* stream) {
@@ -263,6 +337,13 @@ extern "C" int jv_head_linear_mfma_bf16(void* y, long long ldy, int ys, const vo
   if (g && gn != N && gn != 1) return (int)hipErrorInvalidValue;
   const unsigned gy = (M + 63) / 64;
   if (gy > 65535u || heads > 65535 || K < 8 || K % 8 || ldx % 8 || xs % 8) return (int)hipErrorInvalidValue;
+  if (M >= 80 && (long long)M * N * heads >= 480000) {      // fewer rows or outputs: more, shorter waves end sooner
+    const bool y_pieces = ldy % 8 == 0 && ys % 8 == 0 && (uintptr_t)y % 16 == 0;
+    const bool g_pieces = g && ldg % 8 == 0 && gn % 8 == 0 && (uintptr_t)g % 16 == 0;
+    hipLaunchKernelGGL(head_linear_lines_kernel, dim3((N + HL_N - 1) / HL_N, gy, heads), dim3(256), 0, (hipStream_t)stream, (bf16_t*)y,
+                       ldy, ys, (const bf16_t*)x, ldx, xs, (const bf16_t*)W, M, N, K, (const bf16_t*)g, ldg, gn, y_pieces, g_pieces);
+    return JV_LAUNCH_CHECK();
+  }
   hipLaunchKernelGGL(head_linear_mfma_kernel, dim3((N + 15) / 16, gy, heads), dim3(256), 0, (hipStream_t)stream,
                      (bf16_t*)y, ldy, ys, (const bf16_t*)x, ldx, xs, (const bf16_t*)W, M, N, K, (const bf16_t*)g, ldg, gn);
   return JV_LAUNCH_CHECK();

@@ -80,114 +80,116 @@ lightning_steps_kernel(float* __restrict__ out, const T* __restrict__ proj, long
 
 // ---------------------------------------------------------------- by chunks
 // Three launches, so that the chunks of a long prompt run side by side and only the cheap part is serial:
-//   local:  per (chunk, head)   a[i][j] = decay^(i-j) q_i . k_j (j <= i);  out_i = sum_j a[i][j] v_j;
-//                               U = sum_j decay^(n-1-j) k_j v_j^T                       -> scratch[chunk]
+//   chunk:  per (chunk, head)   U = sum_j decay^(n-1-j) k_j v_j^T                       -> scratch[chunk]
 //   scan:   per (request, head) for its chunks in order: scratch[chunk] <- S (the state BEFORE the chunk),
 //                               S <- decay^n S + U;  at the end state <- S
-//   apply:  per (chunk, head)   out_i += decay^(i+1) S_before^T q_i
-#define LC 32        // tokens of a chunk
+//   out:    per (chunk, head)   a[i][j] = decay^(i-j) q_i . k_j (j <= i);  out_i = decay^(i+1) S_before^T q_i + sum_j a[i][j] v_j
+// The products are 32-bit on the matrix unit (v_mfma_f32_32x32x2_f32, lane l holds row or column l % 32 and inner index l / 32 of
+// an operand); chunks of 64 tokens halve what the states of 32 cost in memory traffic, and two blocks of 80 KB share a unit, so that
+// one's loads and activations (25 instructions each, as many cycles as the products) run beside the other's products.
+// 2,048 tokens of 16 heads of 128 x 128, a layer, microseconds: chunk 35, scan 16,
+// out 49 (chunks of 32 in float FMA: 96, 70 and 49 for the state's part alone).
+#define LC 64        // tokens of a chunk
 #define LV 128       // columns (elements of v) a block takes
-#define LQ_PAD 4     // row padding of q and k in LDS: rows stay 16-byte aligned
+#define LD 128       // the largest key size
+
+typedef float lt_f16 __attribute__((ext_vector_type(16)));
+typedef __bf16 lt_b4 __attribute__((ext_vector_type(4)));
+
+// Four elements of a row, as floats; `pieces`: rows begin on 4 elements.
+__device__ __forceinline__ float4 lt_load4(const bf16_t* p, bool pieces, int left) {
+  if (pieces && left >= 4) {
+    const lt_b4 v = *(const lt_b4*)p;
+    return {(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+  }
+  return {left > 0 ? (float)p[0] : 0.f, left > 1 ? (float)p[1] : 0.f, left > 2 ? (float)p[2] : 0.f, left > 3 ? (float)p[3] : 0.f};
+}
+__device__ __forceinline__ float4 lt_load4(const float* p, bool pieces, int left) {
+  if (pieces && left >= 4) return *(const float4*)p;
+  return {left > 0 ? p[0] : 0.f, left > 1 ? p[1] : 0.f, left > 2 ? p[2] : 0.f, left > 3 ? p[3] : 0.f};
+}
+__device__ __forceinline__ float4 lt_silu4(float4 z) { return {lt_silu(z.x), lt_silu(z.y), lt_silu(z.z), lt_silu(z.w)}; }
+__device__ __forceinline__ lt_f16 lt_mfma(float a, float b, lt_f16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
+// Thread t brings elements 4 (t % 32) .. + 3 of tokens t / 32 + 8 i, i < LC / 8: raw numbers, zeros behind the chunk or the row.
+template <typename T>
+__device__ __forceinline__ void lt_load_rows(float4 (&v)[LC / 8], const T* rows, long long ld, int n, int width, bool pieces) {
+  const int c = (threadIdx.x & 31) * 4, j0 = threadIdx.x >> 5;
+#pragma unroll
+  for (int i = 0; i < LC / 8; ++i) {
+    const int j = j0 + 8 * i;
+    v[i] = j < n && c < width ? lt_load4(rows + j * ld + c, pieces, width - c) : float4{0.f, 0.f, 0.f, 0.f};
+  }
+}
 
 // grid (chunks, heads, column slices of LV); work: chunk -> (request, first token)
 template <typename T>
 __global__ void __launch_bounds__(256)
-lightning_local_kernel(float* __restrict__ out, float* __restrict__ scratch, const T* __restrict__ proj, long long ld,
-                       int q_off, int k_off, int v_off, const int* __restrict__ work,
-                       const int* __restrict__ cu_seqlens, const float* __restrict__ decay, int heads, int dim, int vdim) {
-  extern __shared__ __attribute__((aligned(16))) float lds[];
+lightning_chunk_kernel(float* __restrict__ scratch, const T* __restrict__ proj, long long ld, int k_off, int v_off,
+                       const int* __restrict__ work, const int* __restrict__ cu_seqlens, const float* __restrict__ decay, int heads,
+                       int dim, int vdim, bool k_pieces, bool v_pieces) {
+  __shared__ __attribute__((aligned(16))) float ks[LC * LD], vs[LC * LV], pw[LC];
   const int ch = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * LV;
   const int r = work[2 * ch], b0 = work[2 * ch + 1];
-  const int n = min(LC, cu_seqlens[r + 1] - b0);
-  const int dq = dim + LQ_PAD;
-  float* qs = lds;                       // [LC][dq]
-  float* ks = qs + LC * dq;              // [LC][dq]
-  float* vs = ks + LC * dq;              // [LC][LV]
-  float* as = vs + LC * LV;              // [LC][LC + 1]
-  float* pw = as + LC * (LC + 1);        // [LC + 1]
-  const int tid = threadIdx.x;
-  const float lam = decay[h];
-  const int ncols = min(LV, vdim - c0);
-  if (tid <= LC) pw[tid] = powf(lam, (float)tid);
-  for (int i = tid; i < LC * dq; i += 256) {
-    const int j = i / dq, d = i - j * dq;
-    float qv = 0.f, kv = 0.f;
-    if (j < n && d < dim) {
-      const T* row = proj + (long long)(b0 + j) * ld;
-      qv = lt_silu(to_f32(row[q_off + h * dim + d]));
-      kv = lt_silu(to_f32(row[k_off + h * dim + d]));
-    }
-    qs[i] = qv;
-    ks[i] = kv;
-  }
-  for (int i = tid; i < LC * LV; i += 256) {
-    const int j = i / LV, c = i % LV;
-    vs[i] = (j < n && c < ncols) ? lt_silu(to_f32(proj[(long long)(b0 + j) * ld + v_off + h * vdim + c0 + c])) : 0.f;
-  }
-  __syncthreads();
-  // a: thread (i, 4 consecutive j)
+  const int n = min(LC, cu_seqlens[r + 1] - b0), ncols = min(LV, vdim - c0);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, half = lane >> 5;
   {
-    const int i = tid >> 3, j0 = (tid & 7) * 4;
-    float dot[4] = {0.f, 0.f, 0.f, 0.f};
-    if (j0 <= i) {
-      for (int d = 0; d < dim; ++d) {
-        const float qv = qs[i * dq + d];
+    float4 k[LC / 8], v[LC / 8];
+    lt_load_rows(k, proj + (long long)b0 * ld + k_off + h * dim, ld, n, dim, k_pieces);
+    lt_load_rows(v, proj + (long long)b0 * ld + v_off + h * vdim + c0, ld, n, ncols, v_pieces);
+    if (threadIdx.x < LC) pw[threadIdx.x] = powf(decay[h], (float)threadIdx.x);
+    __syncthreads();
+    const int c = (threadIdx.x & 31) * 4, j0 = threadIdx.x >> 5;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) dot[u] = fmaf(qv, ks[(j0 + u) * dq + d], dot[u]);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) as[i * (LC + 1) + j0 + u] = (j0 + u <= i) ? dot[u] * pw[i - j0 - u] : 0.f;
-  }
-  __syncthreads();
-  // k_j <- decay^(n-1-j) k_j (rows beyond the chunk are zero already); out = a v
-  for (int i = tid; i < LC * dq; i += 256) {
-    const int j = i / dq;
-    if (j < n) ks[i] *= pw[n - 1 - j];
-  }
-  for (int e = tid; e < LC * (LV / 4); e += 256) {
-    const int i = e / (LV / 4), c = (e % (LV / 4)) * 4;
-    if (i < n && c < ncols) {
-      float4 o = {0.f, 0.f, 0.f, 0.f};
-      for (int j = 0; j <= i; ++j) {
-        const float a = as[i * (LC + 1) + j];
-        const float4 v = *(const float4*)(vs + j * LV + c);
-        o.x = fmaf(a, v.x, o.x); o.y = fmaf(a, v.y, o.y); o.z = fmaf(a, v.z, o.z); o.w = fmaf(a, v.w, o.w);
-      }
-      float* dst = out + (long long)(b0 + i) * heads * vdim + h * vdim + c0 + c;
-      dst[0] = o.x;
-      if (c + 1 < ncols) dst[1] = o.y;
-      if (c + 2 < ncols) dst[2] = o.z;
-      if (c + 3 < ncols) dst[3] = o.w;
+    for (int i = 0; i < LC / 8; ++i) {
+      const int j = j0 + 8 * i;
+      const float w = j < n ? pw[n - 1 - j] : 0.f;
+      const float4 kk = lt_silu4(k[i]);
+      *(float4*)(ks + j * LD + c) = float4{w * kk.x, w * kk.y, w * kk.z, w * kk.w};
+      *(float4*)(vs + j * LV + c) = lt_silu4(v[i]);
     }
   }
   __syncthreads();
-  // U[d][c]: tiles of 4 x 4 per thread
+  // wave w: rows 32 w .. of U against all columns
+  if (wave * 32 >= dim) return;
+  lt_f16 acc[LV / 32] = {};
+  const int tiles = (ncols + 31) / 32;
+  const float *kr = ks + half * LD + wave * 32 + l32, *vr = vs + half * LV + l32;
+  float a[2][4], b[2][4][LV / 32];
+  auto read = [&](int set, int j) {      // tokens behind the chunk are zeros
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int row = min(j + 2 * u, LC - 2);
+      a[set][u] = kr[row * LD];
+#pragma unroll
+      for (int t = 0; t < LV / 32; ++t) b[set][u][t] = vr[row * LV + t * 32];
+    }
+  };
+  auto products = [&](int set) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int t = 0; t < LV / 32; ++t)
+        if (t < tiles) acc[t] = lt_mfma(a[set][u], b[set][u][t], acc[t]);
+  };
+  read(0, 0);
+  for (int j = 0; j < n; j += 16) {
+    read(1, j + 8);
+    products(0);
+    read(0, j + 16);
+    products(1);
+  }
   float* U = scratch + (((long long)ch * heads + h) * dim) * vdim + c0;
-  const int dt = (dim + 3) / 4;
-  for (int e = tid; e < dt * (LV / 4); e += 256) {
-    const int d0 = (e / (LV / 4)) * 4, c = (e % (LV / 4)) * 4;
-    if (c >= ncols) continue;
-    float u[4][4] = {};
-    for (int j = 0; j < n; ++j) {
-      const float4 kv = *(const float4*)(ks + j * dq + d0);
-      const float4 v = *(const float4*)(vs + j * LV + c);
-      const float kk[4] = {kv.x, kv.y, kv.z, kv.w}, vv[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-      for (int a = 0; a < 4; ++a)
+  for (int t = 0; t < LV / 32; ++t)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) u[a][b] = fmaf(kk[a], vv[b], u[a][b]);
+    for (int i = 0; i < 16; ++i) {
+      const int d = wave * 32 + i / 4 * 8 + half * 4 + i % 4, c = t * 32 + l32;
+      if (d < dim && c < ncols) U[(long long)d * vdim + c] = acc[t][i];
     }
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-      if (d0 + a < dim)
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-          if (c + b < ncols) U[(long long)(d0 + a) * vdim + c + b] = u[a][b];
-  }
 }
 
-// grid (requests, heads, slices of the dim x vdim elements); req_chunks [requests + 1]: first chunk of each request
+// grid (requests, heads, slices of the dim x vdim elements); req_chunks [requests + 1]: first chunk of each request.
+// Bound by memory: a thread asks for eight chunks' numbers before it stores the first.
 __global__ void __launch_bounds__(256)
 lightning_scan_kernel(float* __restrict__ scratch, float* __restrict__ state, const int* __restrict__ slot_ids,
                       const int* __restrict__ req_chunks, const int* __restrict__ work,
@@ -197,78 +199,172 @@ lightning_scan_kernel(float* __restrict__ scratch, float* __restrict__ state, co
   if (last <= first) return;
   const int e = blockIdx.z * 256 + threadIdx.x;
   if (e >= dim * vdim) return;
-  const float lam = decay[h];
+  const float lam = decay[h], whole = powf(lam, (float)LC), rest = powf(lam, (float)(cu_seqlens[r + 1] - work[2 * (last - 1) + 1]));
   float* S = state + ((long long)slot_ids[r] * heads + h) * dim * vdim + e;
+  const long long step = (long long)heads * dim * vdim;
+  float* U = scratch + (long long)first * step + (long long)h * dim * vdim + e;
   float s = *S;
-  const int end = cu_seqlens[r + 1];
-  float next = scratch[((long long)first * heads + h) * dim * vdim + e];
-  for (int ch = first; ch < last; ++ch) {
-    float* U = scratch + ((long long)ch * heads + h) * dim * vdim + e;
-    const float u = next;
-    if (ch + 1 < last) next = U[(long long)heads * dim * vdim];     // asked for before this chunk's store
-    *U = s;
-    const int n = min(LC, end - work[2 * ch + 1]);
-    s = fmaf(powf(lam, (float)n), s, u);
+  for (int ch = first; ch < last; ch += 8, U += 8 * step) {
+    float u[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) u[i] = U[min(i, last - 1 - ch) * step];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (ch + i < last) {
+        U[i * step] = s;
+        s = fmaf(ch + i + 1 < last ? whole : rest, s, u[i]);
+      }
   }
   *S = s;
 }
 
-// grid as the local kernel
+// grid as the chunk kernel
 template <typename T>
-__global__ void __launch_bounds__(256)
-lightning_apply_kernel(float* __restrict__ out, const float* __restrict__ scratch, const T* __restrict__ proj,
-                       long long ld, int q_off, const int* __restrict__ work, const int* __restrict__ cu_seqlens,
-                       const float* __restrict__ decay, int heads, int dim, int vdim) {
-  extern __shared__ __attribute__((aligned(16))) float lds[];
+__global__ void __launch_bounds__(256, 2)
+lightning_out_kernel(float* __restrict__ out, const float* __restrict__ scratch, const T* __restrict__ proj, long long ld, int q_off,
+                     int k_off, int v_off, const int* __restrict__ work, const int* __restrict__ cu_seqlens,
+                     const float* __restrict__ decay, int heads, int dim, int vdim, bool k_pieces, bool v_pieces) {
+  // q and k: element d of row j at d ^ (j % 32), so that 32 rows' element d lies in 32 banks; v takes k's place
+  __shared__ __attribute__((aligned(16))) float qs[LC * LD], kv[LC * LD], as[3][32 * 33], pw[LC + 1];
+  static_assert(LV == LD, "v takes k's place");
   const int ch = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * LV;
   const int r = work[2 * ch], b0 = work[2 * ch + 1];
-  const int n = min(LC, cu_seqlens[r + 1] - b0);
-  const int dq = dim + 1;
-  float* qs = lds;                       // [LC][dq]
-  float* ps = qs + LC * dq;              // [32][LV]: a slab of 32 rows of the state
-  const int tid = threadIdx.x;
-  const int ncols = min(LV, vdim - c0);
-  for (int i = tid; i < LC * dim; i += 256) {
-    const int j = i / dim, d = i - j * dim;
-    qs[j * dq + d] = j < n ? lt_silu(to_f32(proj[(long long)(b0 + j) * ld + q_off + h * dim + d])) : 0.f;
-  }
-  const float* P = scratch + (((long long)ch * heads + h) * dim) * vdim + c0;
-  const int i0 = (tid >> 5) * 4, c = (tid & 31) * 4;       // thread: rows i0..i0+3, columns c..c+3
-  float o[4][4] = {};
-  for (int d0 = 0; d0 < dim; d0 += 32) {
-    __syncthreads();
-    for (int e = tid; e < 32 * LV; e += 256) {
-      const int d = d0 + e / LV, cc = e % LV;
-      ps[e] = (d < dim && cc < ncols) ? P[(long long)d * vdim + cc] : 0.f;
-    }
-    __syncthreads();
-    const int dn = min(32, dim - d0);
-    for (int d = 0; d < dn; ++d) {
-      const float4 p = *(const float4*)(ps + d * LV + c);
-      const float pp[4] = {p.x, p.y, p.z, p.w};
+  const int n = min(LC, cu_seqlens[r + 1] - b0), ncols = min(LV, vdim - c0);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, half = lane >> 5;
+  const int c = (tid & 31) * 4, j0 = tid >> 5;
+  const T* rows = proj + (long long)b0 * ld;
+  if (tid <= LC) pw[tid] = powf(decay[h], (float)tid);
+  float4 v[LC / 8];
+  {
+    float4 q[LC / 8], k[LC / 8];
+    lt_load_rows(q, rows + q_off + h * dim, ld, n, dim, k_pieces);
+    lt_load_rows(k, rows + k_off + h * dim, ld, n, dim, k_pieces);
+    lt_load_rows(v, rows + v_off + h * vdim + c0, ld, n, ncols, v_pieces);
 #pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        const float qv = qs[(i0 + a) * dq + d0 + d];
+    for (int i = 0; i < LC / 8; ++i) {
+      const int j = j0 + 8 * i;
+      const float4 a = lt_silu4(q[i]), b = lt_silu4(k[i]);
 #pragma unroll
-        for (int b = 0; b < 4; ++b) o[a][b] = fmaf(qv, pp[b], o[a][b]);
+      for (int e = 0; e < 4; ++e) {
+        const int at = j * LD + ((c + e) ^ (j & 31));
+        qs[at] = (&a.x)[e], kv[at] = (&b.x)[e];
       }
     }
   }
-  const float lam = decay[h];
+  __syncthreads();
+  // scores: waves 0 to 2 the tiles (0, 0), (1, 0), (1, 1) of 32 x 32 tokens
+  const int ti = wave == 0 ? 0 : 1, tj = wave == 2 ? 1 : 0;
+  if (wave < 3 && ti * 32 < n) {
+    lt_f16 acc = {};
+    const float *qr = qs + (ti * 32 + l32) * LD, *kr = kv + (tj * 32 + l32) * LD;
+    float a[2][8], b[2][8];      // operands of 8 products are read while the 8 before them are made
+    auto read = [&](int set, int d) {
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    const int i = i0 + a;
-    if (i >= n) continue;
-    const float w = powf(lam, (float)(i + 1));
-    float* dst = out + (long long)(b0 + i) * heads * vdim + h * vdim + c0 + c;
+      for (int u = 0; u < 8; ++u) {
+        const int at = min(d + 2 * u + half, LD - 1) ^ l32;      // behind the key size: zeros
+        a[set][u] = qr[at], b[set][u] = kr[at];
+      }
+    };
+    read(0, 0);
+    for (int d = 0; d < dim; d += 32) {
+      read(1, d + 16);
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
-      if (c + b < ncols) dst[b] += w * o[a][b];
+      for (int u = 0; u < 8; ++u) acc = lt_mfma(a[0][u], b[0][u], acc);
+      read(0, d + 32);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc = lt_mfma(a[1][u], b[1][u], acc);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {      // a lane holds column l32
+      const int row = i / 4 * 8 + half * 4 + i % 4, back = ti * 32 + row - tj * 32 - l32;
+      as[wave][row * 33 + l32] = back >= 0 ? acc[i] * pw[back] : 0.f;
+    }
   }
+  __syncthreads();
+  bool odd = false;      // a value that is not finite: tokens before it must not meet it, not even times zero
+#pragma unroll
+  for (int i = 0; i < LC / 8; ++i) {
+    const float4 x = lt_silu4(v[i]);
+    odd = odd || !(fabsf(x.x) + fabsf(x.y) + fabsf(x.z) + fabsf(x.w) < INFINITY);
+    *(float4*)(kv + (j0 + 8 * i) * LV + c) = x;
+  }
+  // wave w: columns 32 w .. of all rows; first the state's part
+  const float* P = scratch + (((long long)ch * heads + h) * dim) * vdim + c0;
+  const int col = wave * 32 + l32;
+  const bool live = wave * 32 < ncols, two = n > 32;
+  lt_f16 o[2] = {};
+  if (live) {
+    const float* p = P + min(col, ncols - 1);
+    constexpr int G = 8;      // steps of two rows of the state that are asked for at once
+    float now[G], next[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) now[g] = p[(long long)min(2 * g + half, dim - 1) * vdim];
+    for (int d = 0; d < dim; d += 2 * G) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) next[g] = p[(long long)min(d + 2 * (G + g) + half, dim - 1) * vdim];
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        if (d + 2 * g < dim) {
+          const int at = (d + 2 * g + half) ^ l32;
+          o[0] = lt_mfma(qs[l32 * LD + at], now[g], o[0]);
+          if (two) o[1] = lt_mfma(qs[(32 + l32) * LD + at], now[g], o[1]);
+        }
+#pragma unroll
+      for (int g = 0; g < G; ++g) now[g] = next[g];
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[b][i] *= pw[b * 32 + i / 4 * 8 + half * 4 + i % 4 + 1];
+  odd = __syncthreads_or(odd);
+  if (!live) return;
+  if (odd) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int row = i / 4 * 8 + half * 4 + i % 4;
+        for (int j = 0; j <= b * 32 + row; ++j) o[b][i] = fmaf(as[b + (j >> 5)][row * 33 + (j & 31)], kv[j * LV + col], o[b][i]);
+      }
+  }
+#pragma unroll 4
+  for (int j = 0; j < 32 && !odd; j += 2) {
+    const float a = kv[(j + half) * LV + col], b = kv[(32 + j + half) * LV + col];
+    o[0] = lt_mfma(as[0][l32 * 33 + j + half], a, o[0]);
+    if (two) {
+      o[1] = lt_mfma(as[1][l32 * 33 + j + half], a, o[1]);
+      o[1] = lt_mfma(as[2][l32 * 33 + j + half], b, o[1]);
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int row = b * 32 + i / 4 * 8 + half * 4 + i % 4;
+      if (row < n && col < ncols) out[((long long)(b0 + row) * heads + h) * vdim + c0 + col] = o[b][i];
+    }
 }
 
 extern "C" int jv_lightning_chunk_tokens() { return LC; }
-extern "C" int jv_lightning_max_dim(int chunks) { return chunks ? 128 : LT_ROWS * 256; }
+extern "C" int jv_lightning_max_dim(int chunks) { return chunks ? LD : LT_ROWS * 256; }
+
+template <typename T>
+static int lightning_by_chunks(float* out, const T* proj, long long ld, int q_off, int k_off, int v_off, float* state, const int* slot_ids,
+                               const int* cu_seqlens, const float* decay, int n_requests, int heads, int dim, int vdim, int chunks,
+                               const int* work, const int* req_chunks, float* scratch, hipStream_t s) {
+  if (dim > LD || dim % 4 || !work || !req_chunks || !scratch) return (int)hipErrorInvalidValue;
+  const int slices = (vdim + LV - 1) / LV;
+  const bool rows = ld % 4 == 0 && (uintptr_t)proj % (4 * sizeof(T)) == 0;      // begin on four elements
+  const bool k_pieces = rows && q_off % 4 == 0 && k_off % 4 == 0, v_pieces = rows && v_off % 4 == 0 && vdim % 4 == 0;
+  hipLaunchKernelGGL(lightning_chunk_kernel<T>, dim3(chunks, heads, slices), dim3(256), 0, s, scratch, proj, ld, k_off, v_off, work,
+                     cu_seqlens, decay, heads, dim, vdim, k_pieces, v_pieces);
+  hipLaunchKernelGGL(lightning_scan_kernel, dim3(n_requests, heads, (dim * vdim + 255) / 256), dim3(256), 0, s, scratch, state, slot_ids,
+                     req_chunks, work, cu_seqlens, decay, heads, dim, vdim);
+  hipLaunchKernelGGL(lightning_out_kernel<T>, dim3(chunks, heads, slices), dim3(256), 0, s, out, scratch, proj, ld, q_off, k_off, v_off,
+                     work, cu_seqlens, decay, heads, dim, vdim, k_pieces, v_pieces);
+  return JV_LAUNCH_CHECK();
+}
 
 // chunks = 0: token by token.  chunks = number of chunks (> 0): by chunks, with work [chunks][2] = (request,
 // first token) in the order of requests and tokens, req_chunks [requests + 1], and scratch of
@@ -283,19 +379,8 @@ extern "C" int jv_lightning_max_dim(int chunks) { return chunks ? 128 : LT_ROWS 
     if (dim <= 0 || vdim <= 0 || heads > 65535) return (int)hipErrorInvalidValue;                              \
     hipStream_t s = (hipStream_t)stream;                                                                       \
     if (chunks > 0) {                                                                                          \
-      if (dim > 128 || !work || !req_chunks || !scratch) return (int)hipErrorInvalidValue;                     \
-      const int slices = (vdim + LV - 1) / LV;                                                                 \
-      const size_t lds_local = (2 * LC * (dim + LQ_PAD) + LC * LV + LC * (LC + 1) + LC + 1) * sizeof(float);   \
-      const size_t lds_apply = (LC * (dim + 1) + 32 * LV) * sizeof(float);                                     \
-      hipLaunchKernelGGL(lightning_local_kernel<T>, dim3(chunks, heads, slices), dim3(256), lds_local, s, out, \
-                         scratch, (const T*)proj, ld, q_off, k_off, v_off, work, cu_seqlens, decay, heads,     \
-                         dim, vdim);                                                                           \
-      hipLaunchKernelGGL(lightning_scan_kernel, dim3(n_requests, heads, (dim * vdim + 255) / 256), dim3(256),  \
-                         0, s, scratch, state, slot_ids, req_chunks, work, cu_seqlens, decay, heads, dim,      \
-                         vdim);                                                                                \
-      hipLaunchKernelGGL(lightning_apply_kernel<T>, dim3(chunks, heads, slices), dim3(256), lds_apply, s, out, \
-                         scratch, (const T*)proj, ld, q_off, work, cu_seqlens, decay, heads, dim, vdim);       \
-      return JV_LAUNCH_CHECK();                                                                                \
+      return lightning_by_chunks<T>(out, (const T*)proj, ld, q_off, k_off, v_off, state, slot_ids, cu_seqlens, \
+                                    decay, n_requests, heads, dim, vdim, chunks, work, req_chunks, scratch, s);  \
     }                                                                                                          \
     int cols = 64;                       /* the widest slice that keeps a thread's rows in registers */        \
     while (cols > 1 && (cols / 2 >= vdim || (long long)dim * cols > 256LL * LT_ROWS)) cols /= 2;               \
