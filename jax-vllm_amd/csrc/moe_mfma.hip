@@ -1,5 +1,5 @@
 // The two grouped products of routed experts on the matrix cores (bfloat16, float accumulation); the
-// grouping they read (tiles of 64 or 128 rows of one expert each) is made by moe.hip.  And the router's logits.
+// grouping they read (tiles of 64, 128 or 192 rows of one expert each) is made by moe.hip.  And the router's logits.
 //
 // A block takes one tile of (token, choice) rows against TW rows of the expert's weight and walks the inner size in
 // chunks of 64: the rows of x (gathered by token) and of W go straight from memory into LDS, chunks ahead of their use;
@@ -29,7 +29,7 @@ enum { MM_DOWN = 0, MM_GATED = 1, MM_PLAIN = 2 };
 // What a lane reads for columns behind the inner size, of x and of W alike.
 static __device__ __attribute__((aligned(16))) const unsigned mm_zeros[4] = {0, 0, 0, 0};
 
-// TM: rows of a tile of the grouping, 64 or 128; TW: rows of W of a block (gated: half of them of each matrix).
+// TM: rows of a tile of the grouping, 64, 128 or 192; TW: rows of W of a block (gated: half of them of each matrix).
 template <int MODE, int TM, int TW, int BUFS>
 __global__ void __launch_bounds__(2 * TW, TW == 128 ? 2 : 1)
 moe_mfma_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, const bf16_t* __restrict__ W0,
@@ -42,7 +42,6 @@ moe_mfma_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, const
   constexpr int NB = GATED ? TW / 2 : TW;           // output columns of a block
   constexpr int XI = TM / 8 / WAVES, WI = TW / 8 / WAVES;      // instructions a wave brings of a chunk, each 8 rows of 128 bytes
   constexpr int BUF = (TM + TW) * MM_K;             // elements of a buffer: rows of x, then rows of W
-  static_assert(XI % 2 == 0 && WI % 2 == 0, "see col");
   // Blocks b, b + 8, b + 16, ... run on one XCD (with an L2 of its own): each of the 8 takes one run of the (tile, rows of W)
   // pairs, rows of W fastest, so the rows of x of a tile and the weights of an expert are read into one L2 and used there.
   const int per_tile = (N + NB - 1) / NB;
@@ -91,7 +90,7 @@ moe_mfma_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, const
 #pragma unroll
     for (int i = 0; i < XI + WI; ++i) {
       const int first = i < XI ? (wave * XI + i) * 8 : TM + (wave * WI + i - XI) * 8;      // the instruction's first row in the buffer
-      const int k = k0 + col[i & 1];                  // XI and WI are even: odd instructions bring the upper 8 of 16 rows
+      const int k = k0 + col[(first >> 3) & 1];       // odd groups of 8 rows are the upper half of 16
       const bf16_t* piece = k < K ? src[i] + k : (const bf16_t*)mm_zeros;
       const unsigned at = (unsigned)(unsigned long long)(const __attribute__((address_space(3))) void*)(bufs + buf * BUF + first * MM_K);
       asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(piece), "s"(at) : "memory", "m0");
@@ -167,21 +166,23 @@ static int launch_moe_tiles(int max_tiles, hipStream_t stream, void* out, const 
   return JV_LAUNCH_CHECK();
 }
 
-// 128 rows against 256 of W by 8 waves with two chunks on their way; 64 rows against 128 by 4 waves, three blocks a compute unit with
+// 128 rows against 256 of W by 8 waves with two chunks on their way; 192 rows with one, for groupings that fill the units with fewer
+// tiles (32 experts x 512, width 2,048, 256 rows each: 256 tiles instead of 320, gate/up 57 us, before 85); 64 rows against 128 by 4 waves, three blocks a compute unit with
 // one chunk on its way each, or (`deep`) two blocks with two: where an expert gets so few rows that nearly all are one tile, the
 // stream of the weights is what is waited for.  gate/up + down, cold weights, microseconds (deep / not): 64 experts x 1,024, width
 // 4,096, 25 rows each 302 / 334, 8 x 4,096 at 40 rows 167 / 184, 16 x 2,048, width 1,024, at 25 56 / 64, 32 x 512, width 2,048, at
 // 40 52 / 57; at 50 rows, with second tiles, 66 / 62.
 template <int MODE, typename... Args>
 static int launch_moe_mfma(int tile_rows, int deep, Args... args) {
+  if (tile_rows == 192) return launch_moe_tiles<MODE, 192, 256, 2>(args...);
   if (tile_rows == 128) return launch_moe_tiles<MODE, 128, 256, 3>(args...);
   if (tile_rows == 64 && deep) return launch_moe_tiles<MODE, 64, 128, 3>(args...);
   if (tile_rows == 64) return launch_moe_tiles<MODE, 64, 128, 2>(args...);
   return (int)hipErrorInvalidValue;
 }
 
-// gate/up: x [tokens, hidden], Wg, Wu [experts, ff, hidden] -> z [entries, ff] bf16 by position; tile_rows (64 or
-// 128) is what the grouping was made with; deep: see launch_moe_mfma.  Wg null: experts without a gate, act one that stands alone.
+// gate/up: x [tokens, hidden], Wg, Wu [experts, ff, hidden] -> z [entries, ff] bf16 by position; tile_rows (64,
+// 128 or 192) is what the grouping was made with; deep: see launch_moe_mfma.  Wg null: experts without a gate, act one that stands alone.
 extern "C" int jv_moe_gate_up_mfma_bf16(void* z, const void* x, const void* Wg, const void* Wu, const int* meta,
                                         const int* offsets, const int* tile_expert, const int* tile_row0,
                                         const int* order, const float* weights, int max_tiles, int top, int hidden,

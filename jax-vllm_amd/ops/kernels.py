@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import math
 from ctypes import c_float, c_int, c_longlong, c_void_p
 
 import torch
@@ -2081,7 +2082,7 @@ def group_gated_norm(o: torch.Tensor, gate: torch.Tensor, weight, group: int, ep
 
 # --------------------------------------------------------------------------- routed experts
 def moe_tile_rows() -> int:
-    """Rows of a tile of the float-FMA expert kernels (the matrix-core ones also take tiles of 128)."""
+    """Rows of a tile of the float-FMA expert kernels (the matrix-core ones also take tiles of 128 and 192)."""
     return library.core().jv_moe_tile_rows()
 
 
@@ -2089,16 +2090,35 @@ MOE_SKINNY_ROWS = 16            # rows of a tile of the weight-streaming expert 
 MOE_SKINNY_MAX_MEAN = 6         # up to so many rows an expert (on average over all experts) they are preferred
 
 
+@functools.lru_cache(maxsize=4096)
+def moe_tile_rounds(tile_rows: int, hidden: int, ff: int, entries: int, experts: int, cus: int = 256) -> int:
+    """Chunks of 64 columns that a compute unit walks in both expert products of a prompt, one after another, by tiles of ``tile_rows``
+    rows against 256 of the weights: whole rounds over the units (a twentieth more is none), for an expert's rows spread about their mean as a router spreads
+    them (1.4 times the square root: 32 experts of 256 rows get up to 303)."""
+    mean = entries / experts
+    spread = 1.4 * mean ** 0.5 * 2 ** 0.5
+    tiles, k = 0.0, 0
+    while k * tile_rows < mean + 4 * spread:                                  # an expert has more than k whole tiles
+        tiles += 0.5 * math.erfc((k * tile_rows - mean) / spread)
+        k += 1
+    tiles = max(1.0, tiles) * experts
+    gate_up, down = (max(1, math.ceil(tiles * blocks / cus - 0.05)) for blocks in (-(-ff // 128), -(-hidden // 256)))
+    return gate_up * -(-hidden // 64) + down * -(-ff // 64)
+
+
 def moe_tile_rows_for(dtype, hidden: int, ff: int, entries: int, experts: int) -> int:
     """Rows of a tile for a step: 16 (the kernels that stream the experts' weights) where an expert gets a few rows at
     most, 128 where the matrix-core kernels run and an expert gets more than 64 rows on average (a second tile of 64 would be
     nearly empty: 8 experts x 4,096 of width 4,096 at 75 rows each 198 us with 128, 270 with 64; 64 x 1,024 at 68 rows 361 / 430,
-    128 x 768 of width 2,048 at 68 rows 296 / 313; at 60 rows 32 x 512 66 / 61), else 64."""
+    128 x 768 of width 2,048 at 68 rows 296 / 313; at 60 rows 32 x 512 66 / 61), else 64.  192 instead of 128 where that spares so many
+    rounds over the compute units (``moe_tile_rounds``) that their longer chunks, 1.45 times the time, are made up for: 2,048 tokens, 4 of 32
+    experts x 512, width 2,048 111 us (138 with 128), 1,500 tokens 111 (86); 4,096 tokens, 8 of 64 x 1,024 571 (633), 2,048 382 (371)."""
     if moe_matrix_cores_possible(dtype, hidden, ff):
         if entries <= MOE_SKINNY_MAX_MEAN * experts:
             return MOE_SKINNY_ROWS
         if entries > 64 * experts:
-            return 128
+            larger, smaller = (moe_tile_rounds(rows, hidden, ff, entries, experts) for rows in (192, 128))
+            return 192 if 1.45 * larger < smaller else 128
     return moe_tile_rows()
 
 
@@ -2241,7 +2261,7 @@ def moe_route(logits: "torch.Tensor | None", top: int, x=None, w_router=None, lo
     all_experts, per = experts + always, top + always
     entries = n * per
     tile_rows = tile_rows or moe_tile_rows()
-    _need(tile_rows in (16, 64, 128), "tiles have 16, 64 or 128 rows")
+    _need(tile_rows in (16, 64, 128, 192), "tiles have 16, 64, 128 or 192 rows")
     max_tiles = min(entries, -(-entries // tile_rows) + all_experts)
     ints = torch.empty(entries * 3 + 1 + all_experts + 1 + 2 * max_tiles, dtype=torch.int32, device=dev)
     ids, rank, order = ints[:entries], ints[entries:2 * entries], ints[2 * entries:3 * entries]
