@@ -1,0 +1,145 @@
+// y[M,N] = x[M,K] W[N,K]^T for up to 16 rows of x and matrices too small for blocks that stay (gemm_skinny.hip): bf16 in, float
+// sums, bf16 or float out, or the activation of pairs of rows of W as an epilogue.
+//
+// Bound by the stream of W and what stands before it: a matrix of 25 MB is read in 4.6 us, and every round trip to memory that a
+// block waits for in a row costs one more.  So a block takes TW rows of W against all rows of x and its 8 waves an eighth of the
+// inner size each; a wave asks for its part of x (into registers, where it stays) and for the first S chunks of its part of W
+// (straight into a ring of its own in LDS) in one go, and no wave waits for another before the parts meet at the end.  Two blocks
+// of 80 KB share a unit, and TW is such that all blocks are on the chip at once: the units then need not carry equal loads, for
+// what they share is the memory.  The parts are added in ascending order, so a row's result does not depend on the others.
+//
+// Microseconds in a graph, cold weights, at 1, 8 and 16 rows (before, x staged chunk by chunk in LDS for all waves of a block):
+// 6,144 x 2,048 with its activation 8.7, 9.1, 9.0 (9.8, 11.2, 11.8), 11,296 x 2,048 12.0, 12.5, 14.0 (17.3, 15.3, 17.3),
+// 2,048 x 2,048 4.0, 4.7, 5.4 (5.5, 6.2, 7.1), 1,536 x 768 2.9, 3.2, 3.4 (4.6, 5.0, 6.2), 3,072 x 4,096 7.9, 8.6, 10.1 (9.4, 10.4, 13.2).
+// Blocks that stay are better from about 16,384 rows of W on (24,576 x 2,048 at 16 rows 22.5, here 26.3).
+#include "common.h"
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+enum { FEW_BF16 = 0, FEW_F32 = 1, FEW_PAIRS = 2 };
+
+#define FEW_K 64           // columns of a chunk: a row of it is 128 bytes, 8 pieces of 16
+#define FEW_WAVES 8
+
+// CW: the most chunks of a wave.
+template <int MODE, int TW, int CW>
+__global__ void __launch_bounds__(64 * FEW_WAVES)
+gemm_few_kernel(void* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, int M, int N, int K, long long ldx, JvAct act) {
+  constexpr int NT = TW / 16, L = TW / 8, CHUNK = TW * FEW_K, S = 64 * 1024 / (FEW_WAVES * CHUNK * 2) < CW ? 64 * 1024 / (FEW_WAVES * CHUNK * 2) : CW;
+  static_assert(NT * 1024 <= S * CHUNK * 2, "the parts meet in the ring's place");
+  __shared__ __attribute__((aligned(1024))) bf16_t bufs[FEW_WAVES][S * CHUNK];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, lq = lane >> 4;
+  const int n0 = blockIdx.x * TW, all = K / FEW_K;
+  const int first = all * wave / FEW_WAVES, chunks = all * (wave + 1) / FEW_WAVES - first;
+  // an instruction brings 8 rows, lane l row l / 8, and fills 1 KB in the order of the lanes; piece c of row r lies at slot
+  // c ^ (r % 8) of its row.  Rows beyond the last repeat it.
+  const bf16_t* src[L];
+#pragma unroll
+  for (int j = 0; j < L; ++j)
+    src[j] = W + (long long)min(n0 + j * 8 + (lane >> 3), N - 1) * K + first * FEW_K + ((lane & 7) ^ (lane >> 3)) * 8;
+  const unsigned lds0 = (unsigned)(unsigned long long)(const __attribute__((address_space(3))) void*)bufs[wave];
+  auto fetch = [&](int c, int slot) {
+#pragma unroll
+    for (int j = 0; j < L; ++j)
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src[j] + c * FEW_K), "s"(lds0 + slot * (CHUNK * 2) + j * 1024) : "memory", "m0");
+  };
+#pragma unroll
+  for (int c = 0; c < S; ++c)
+    if (c < chunks) fetch(c, c);
+  // rows of x beyond the last are zeros: their lanes load nothing
+  bf16x8 xf[CW][2];
+  const bf16_t* xr = x + (long long)min(li, M - 1) * ldx + first * FEW_K + lq * 8;
+#pragma unroll
+  for (int c = 0; c < CW; ++c)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      xf[c][h] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (li < M && c < chunks) xf[c][h] = *(const bf16x8*)(xr + c * FEW_K + h * 32);
+    }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int c = 0; c < CW; ++c)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) asm volatile("" : "+v"(xf[c][h]));      // x is there: nothing below waits for it, and with it for W
+  f32x4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < CW; ++c) {
+    if (c >= chunks) break;
+    if (c >= S) {      // chunk c was asked for with chunk c - S; S - 1 of those behind it may be on their way
+      if (c + S - 1 < chunks) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * L) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    const bf16_t* b = bufs[wave] + c % S * CHUNK + li * FEW_K;
+    bf16x8 wf[NT][2];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) wf[t][h] = *(const bf16x8*)(b + t * 16 * FEW_K + (((h * 4 + lq) ^ li) & 7) * 8);
+    if (c + S < chunks) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // read before the slot is filled again
+      fetch(c + S, c % S);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[t][h], xf[c][h], acc[t], 0, 0, 0);
+  }
+  __syncthreads();
+  f32x4* red = (f32x4*)bufs;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) red[(t * FEW_WAVES + wave) * 64 + lane] = acc[t];
+  __syncthreads();
+  if (wave >= NT) return;
+  f32x4 sum = red[wave * FEW_WAVES * 64 + lane];
+#pragma unroll
+  for (int p = 1; p < FEW_WAVES; ++p) sum += red[(wave * FEW_WAVES + p) * 64 + lane];
+  const int m = li, n = n0 + wave * 16 + lq * 4;      // a lane holds y[m][n .. n + 3]; N is a multiple of 4
+  if (m >= M || n >= N) return;
+  if (MODE == FEW_F32) {
+    *(f32x4*)((float*)y + (long long)m * N + n) = sum;
+  } else if (MODE == FEW_BF16) {
+    bf16x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = from_f32<bf16_t>(sum[e]);
+    *(bf16x4*)((bf16_t*)y + (long long)m * N + n) = v;
+  } else {
+    bf16x2 v;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) v[e] = from_f32<bf16_t>(jv_gated(act, sum[2 * e], sum[2 * e + 1]));
+    *(bf16x2*)((bf16_t*)y + (long long)m * (N / 2) + n / 2) = v;
+  }
+}
+
+template <int MODE, int TW>
+static int few_launch(void* y, const void* x, const void* W, int M, int N, int K, long long ldx, JvAct act, hipStream_t s) {
+  const int cw = (K / FEW_K + FEW_WAVES - 1) / FEW_WAVES;
+#define FEW(CW)                                                                                                                        \
+  if (cw <= CW) {                                                                                                                      \
+    hipLaunchKernelGGL((gemm_few_kernel<MODE, TW, CW>), dim3((N + TW - 1) / TW), dim3(64 * FEW_WAVES), 0, s, y, (const bf16_t*)x,     \
+                       (const bf16_t*)W, M, N, K, ldx, act);                                                                           \
+    return JV_LAUNCH_CHECK();                                                                                                          \
+  }
+  FEW(2) FEW(4) FEW(8)
+#undef FEW
+  return (int)hipErrorInvalidValue;
+}
+extern "C" int jv_gemm_few_max_inner() { return 8 * FEW_WAVES * FEW_K; }
+// mode: FEW_*; tw (16, 32): rows of W of a block.
+extern "C" int jv_gemm_few_bf16(void* y, const void* x, const void* W, int M, int N, int K, long long ldx, int mode, int gate_act,
+                                float act_limit, float act_slope, int tw, void* stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (M > 16 || K < FEW_K || K % FEW_K || N % 4 || ldx % 8 || (((uintptr_t)x | (uintptr_t)W | (uintptr_t)y) & 15))
+    return (int)hipErrorInvalidValue;
+  if (mode == FEW_PAIRS && !jv_act_known(gate_act)) return (int)hipErrorInvalidValue;
+  const JvAct act{gate_act, act_limit, act_slope};
+  const hipStream_t s = (hipStream_t)stream;
+  if (mode == FEW_BF16) return tw == 16 ? few_launch<FEW_BF16, 16>(y, x, W, M, N, K, ldx, act, s) : few_launch<FEW_BF16, 32>(y, x, W, M, N, K, ldx, act, s);
+  if (mode == FEW_F32) return tw == 16 ? few_launch<FEW_F32, 16>(y, x, W, M, N, K, ldx, act, s) : few_launch<FEW_F32, 32>(y, x, W, M, N, K, ldx, act, s);
+  if (mode == FEW_PAIRS) return tw == 16 ? few_launch<FEW_PAIRS, 16>(y, x, W, M, N, K, ldx, act, s) : few_launch<FEW_PAIRS, 32>(y, x, W, M, N, K, ldx, act, s);
+  return (int)hipErrorInvalidValue;
+}

@@ -941,6 +941,7 @@ def _stay_pieces(k: int, parts: int):
     return None
 
 
+STAGED = (0, 0, 0), 1               # x staged chunk by chunk in LDS, whole inner size a block
 TILE64 = (-3, 0, 0)                 # block shape that stands for ``gemm_tile64`` in a plan
 TILE64_MIN_SHARE = 3072             # columns a block of gemm_tile64 needs to pay for its start
 LIBRARY_MAX_INNER = 12288           # beyond this inner size the library's choice for few rows collapses
@@ -977,6 +978,7 @@ def streaming_plan(m: int, n: int, k: int, gate_pairs: bool = False, partial_ok:
       x), unless the inner size is beyond 12,288, where the library needs 113 us for the 178 MB
       that x resident in LDS streams in 45;
     * otherwise x staged chunk by chunk in LDS.
+    Of the last two, ``linear`` gives what ``few_tile`` takes (inner sizes up to 4,096) to ``gemm_few``.
     """
     if k % 8:
         return None
@@ -1016,7 +1018,7 @@ def streaming_plan(m: int, n: int, k: int, gate_pairs: bool = False, partial_ok:
             return (-2, (2 if tiles >= 16 * cus else 1) * cus, nl), 1
     if m > 8 and n * k >= SKINNY_LARGE_MATRIX:
         return None
-    return (0, 0, 0), 1
+    return STAGED
 
 
 STREAM_MAX_ROWS = 128
@@ -1106,6 +1108,36 @@ def gemm_stream(x: torch.Tensor, w: torch.Tensor, form, mode: str = "rows", gate
     return y
 
 
+FEW_MODES = {"rows": 0, "float": 1, "pairs": 2}
+FEW_MAX_INNER = 4096      # eight waves of eight chunks of 64 columns, x in registers
+
+
+def few_tile(m: int, n: int, k: int, cus: int = 256) -> "int | None":
+    """Rows of w of a block of ``gemm_few`` (16 or 32) where it can take the product, else None: 32 where 16 would give a unit more than
+    one block and most units only one (4,608 x 3,072 9.3 us against 10.5, 6,144 x 2,048 at 8 rows 9.1 / 9.4, at one row 8.7 / 8.4; 4,096 x
+    2,048 6.8 / 5.9, 8,192 x 2,048 10.0 / 9.1, 11,296 x 2,048 12.6 / 12.0)."""
+    if not 0 < m <= SKINNY_AUTO_ROWS or k % 64 or not 64 <= k <= FEW_MAX_INNER or n % 4:
+        return None
+    return 32 if cus < -(-n // 16) <= 1.5 * cus else 16
+
+
+def gemm_few(x: torch.Tensor, w: torch.Tensor, tile: int, gate_pairs: "str | tuple | None" = None, out_dtype=torch.bfloat16) -> torch.Tensor:
+    """x @ w.T for up to 16 rows of bfloat16 x against bfloat16 w [N, K], K a multiple of 64 up to 4,096, ``tile`` (16 or 32) rows of w a
+    block: see ``csrc/gemm_few.hip``.  bfloat16 or float32 [M, N], or with ``gate_pairs`` the activation, bfloat16 [M, N / 2]."""
+    _dev(x, w)
+    _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "gemm_few takes bfloat16")
+    m, k = x.shape
+    n = w.shape[0]
+    _need(w.shape[1] == k and m <= SKINNY_AUTO_ROWS and tile in (16, 32), "inner sizes differ, or more than 16 rows")
+    _need(out_dtype in (torch.bfloat16, torch.float32) and not (gate_pairs and out_dtype == torch.float32), "the activation's result is bfloat16")
+    y = torch.empty((m, n // 2 if gate_pairs else n), dtype=out_dtype, device=x.device)
+    mode = "pairs" if gate_pairs else "float" if out_dtype == torch.float32 else "rows"
+    _check(library.core().jv_gemm_few_bf16(
+        _ptr(y), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), c_longlong(k), c_int(FEW_MODES[mode]),
+        *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), c_int(tile), _stream()), "gemm_few")
+    return y
+
+
 SHARES_MAX_ROWS = 1024
 _SHARES_TILES = {(128, 128): 0.6, (256, 128): 0.9, (256, 256): 1.6}      # rows of x, rows of w: microseconds a chunk of 64 columns
 
@@ -1157,7 +1189,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
     """x @ w.T for w stored [out, in].
 
     float32: the library's own kernel, from which no bit of the inputs is dropped (``gemm_f32``).
-    bfloat16, at most 16 rows: a weight-streaming MFMA kernel of this library (``streaming_plan``); 17 to 128 rows: chunks
+    bfloat16, at most 16 rows: a weight-streaming MFMA kernel of this library (``streaming_plan``, ``few_tile``); 17 to 128 rows: chunks
     of x and w through a ring in LDS (``ring_plan``), or what ``streaming_plan`` has for what that leaves.
     bfloat16 otherwise: a plain library matrix product (hipBLASLt through torch), float accumulation.
     With ``partial_ok`` the caller takes a float32 stack [parts, M, N] of partial products as well
@@ -1192,6 +1224,11 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
                 return gemm_shares(x, w, form)
         plan = streaming_plan(x.shape[0], w.shape[0], w.shape[1], bool(gate_pairs),
                               partial_ok and out_dtype in (None, torch.bfloat16), x.device, partial_max_width)
+        if plan in (None, STAGED) and m <= SKINNY_AUTO_ROWS and not k % 64 and w.dtype == torch.bfloat16 and out_dtype in (None, torch.bfloat16, torch.float32):
+            tile = few_tile(m, n, k, compute_units(x.device))
+            if tile is not None and x.is_contiguous() and w.is_contiguous() and not (x.data_ptr() | w.data_ptr()) & 15 \
+                    and not (gate_pairs and out_dtype == torch.float32):
+                return gemm_few(x, w, tile, gate_pairs, out_dtype or torch.bfloat16)
         _need(scale is None or (plan is not None and plan[0][0] == -2),
               "un-normalised rows need a product by the blocks that stay (ask linear_takes_unscaled_rows first)")
         if plan is not None:

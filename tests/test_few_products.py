@@ -1,0 +1,53 @@
+"""Products of up to 16 rows with the inner size shared out to a block's waves: every output form at odd numbers of rows, chunks and
+rows of W, against float64, and where they are taken."""
+import pytest
+import torch
+
+from .test_kernels_gpu import K, randn
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 5, 15, 16])
+@pytest.mark.parametrize("n,k", [(4, 64), (20, 448), (36, 512), (100, 576), (1028, 1088), (64, 2048), (48, 2112), (4100, 4096)])
+@pytest.mark.parametrize("tile", [16, 32])
+def test_few_rows(m, n, k, tile):
+    x, w = randn(m, k, seed=m).bfloat16(), randn(n, k, seed=n + k).bfloat16()
+    want = x.double() @ w.double().T
+    y = K().gemm_few(x, w, tile, out_dtype=torch.float32)
+    # exact products, eight chains of k / 8 terms and eight sums in float
+    bound = 2.0 ** -24 * (k / 8 + 8) * (x.double().abs() @ w.double().abs().T)
+    assert ((y.double() - want).abs() <= bound).all()
+    assert torch.equal(K().gemm_few(x, w, tile), y.bfloat16())
+    assert torch.equal(K().gemm_few(x[m // 2:].contiguous(), w, tile, out_dtype=torch.float32), y[m // 2:])      # whatever the batch
+    gated = K().gemm_few(x, w, tile, "silu")
+    g, u = y[:, 0::2], y[:, 1::2]
+    torch.testing.assert_close(gated, (g / (1 + torch.exp(-g)) * u).bfloat16(), rtol=2.0 ** -7, atol=1e-6)      # a rounding of bfloat16
+
+
+@pytest.mark.gpu
+def test_rows_that_are_not_finite_stay_alone():
+    x, w = randn(9, 512, seed=1).bfloat16(), randn(64, 512, seed=2).bfloat16()
+    clean = K().gemm_few(x, w, 16)
+    x[4, 100], w[33, 7] = float("nan"), float("inf")
+    y = K().gemm_few(x, w, 16)
+    rows, cols = torch.arange(9) != 4, torch.arange(64) != 33
+    assert torch.equal(y[rows][:, cols], clean[rows][:, cols]) and not y[4].isfinite().any() and not y[:, 33].isfinite().any()
+
+
+@pytest.mark.gpu
+def test_operands_the_form_does_not_take_go_the_old_way():
+    x, w = randn(6, 2048, seed=1).bfloat16(), randn(2048, 2048, seed=2).bfloat16()
+    want = K().linear(x, w)
+    flat = torch.empty(6 * 2048 + 1, dtype=torch.bfloat16, device="cuda")
+    off = flat[1:].view(6, 2048).copy_(x)
+    torch.testing.assert_close(K().linear(off.clone(), w), want)
+    assert K().few_tile(6, 2048, 2040) is None and K().few_tile(6, 2048, 4160) is None and K().few_tile(17, 2048, 2048) is None
+    torch.testing.assert_close(K().linear(x[:, :2040].contiguous(), w[:, :2040].contiguous()).double(),
+                               x[:, :2040].double() @ w[:, :2040].double().T, rtol=2.0 ** -7, atol=0.05)
+
+
+def test_rows_of_w_of_a_block():
+    from jax_vllm_amd.ops.kernels import STAGED, few_tile, streaming_plan
+
+    assert [few_tile(8, n, 2048) for n in (32, 4096, 4112, 6144, 6160, 11296)] == [16, 16, 32, 32, 16, 16]
+    assert streaming_plan(8, 6144, 2048, True) == STAGED and streaming_plan(12, 12288, 4096) is None
