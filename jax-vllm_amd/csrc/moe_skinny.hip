@@ -112,11 +112,141 @@ moe_skinny_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, con
   }
 }
 
+// The same where an expert's rows begin on 16 bytes and the inner size is a multiple of 64 up to 4,096: WK of a block's 8 waves share
+// out the inner size of 16 rows of W, the others take further 16 rows.  A wave asks for its rows of x (into registers, where they
+// stay) and for its first chunks of W (whole lines, straight into a ring of its own in LDS) in one go and waits for no other wave
+// before the parts meet; two blocks of 64 KB share a unit, so one's chain of addresses runs beside the other's stream.
+// Both products of a layer in a graph, cold weights, microseconds (the kernel above): 32 experts x 768, 4 chosen, width 2,048: 4
+// tokens 28.2 (29.9), 16 56.3 (59.9), 48 62.7 (69.9); 32 x 512 of width 1,536: 1 token 10.7 (14.2), 8 31.1 (35.0); 64 x 1,024, 8 chosen, width
+// 4,096: 16 tokens 252 (261), 48 288 (318), 5.5 TB/s.  Not better: one wave a row tile at inner sizes up to 512, 4 at 2,048.
+#define MF_K 64            // columns of a chunk: a row of it is 128 bytes, 8 pieces of 16
+#define MF_WAVES 8
+
+// CW: the most chunks of a wave.
+template <int MODE, int WK, int CW>
+__global__ void __launch_bounds__(64 * MF_WAVES)
+moe_few_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, const bf16_t* __restrict__ W0,
+               const bf16_t* __restrict__ W1, const int* __restrict__ meta, const int* __restrict__ offsets,
+               const int* __restrict__ tile_expert, const int* __restrict__ tile_row0, const int* __restrict__ order,
+               const float* __restrict__ weights, int top, int n_tokens, int K, int N, JvAct act, int use_weight) {
+  constexpr bool GATED = MODE == MS_GATED, BY_TOKEN = MODE != MS_DOWN;
+  constexpr int NT = MF_WAVES / WK, NB = 16 * NT, MATS = GATED ? 2 : 1, L = 2 * MATS, CHUNK = 16 * MATS * MF_K;
+  constexpr int FIT = 64 * 1024 / (MF_WAVES * CHUNK * 2), S = FIT < CW ? FIT : CW;
+  __shared__ __attribute__((aligned(1024))) bf16_t bufs[MF_WAVES][S * CHUNK];
+  const int per_tile = (N + NB - 1) / NB, tile = blockIdx.x / per_tile;      // (neighbouring blocks: see the kernel above)
+  const int tiles = meta[0], e = tile_expert[tile], row0 = tile_row0[tile];
+  if (tile >= tiles) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, lq = lane >> 4;
+  const int part = wave % WK, n0 = (blockIdx.x - tile * per_tile) * NB + wave / WK * 16;
+  const int all = K / MF_K, first = all * part / WK, chunks = n0 < N ? all * (part + 1) / WK - first : 0;
+  const bf16_t* src[L];      // an instruction brings 8 rows; piece c of row r lies at slot c ^ (r % 8); rows beyond the last repeat it
+#pragma unroll
+  for (int j = 0; j < L; ++j)
+    src[j] = (j < 2 ? W0 : W1) + ((long long)e * N + min(n0 + (j & 1) * 8 + (lane >> 3), N - 1)) * K + first * MF_K + ((lane & 7) ^ (lane >> 3)) * 8;
+  const unsigned lds0 = (unsigned)(unsigned long long)(const __attribute__((address_space(3))) void*)bufs[wave];
+  auto fetch = [&](int c, int slot) {
+#pragma unroll
+    for (int j = 0; j < L; ++j)
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src[j] + c * MF_K), "s"(lds0 + slot * (CHUNK * 2) + j * 1024) : "memory", "m0");
+  };
+#pragma unroll
+  for (int c = 0; c < S; ++c)
+    if (c < chunks) fetch(c, c);
+  const int rows = min(MS_ROWS, offsets[e + 1] - row0), mine = row0 + min(li, rows - 1), s = order[mine], token = s / top;
+  const float weight = use_weight ? weights[s] : 1.f;
+  const bf16_t* xr = a_rows + (long long)(BY_TOKEN ? token : mine) * K + first * MF_K + lq * 8;
+  ms_bf16x8 xf[CW][2];      // rows beyond the tile's are zeros: their lanes load nothing
+#pragma unroll
+  for (int c = 0; c < CW; ++c)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      xf[c][h] = ms_bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (li < rows && c < chunks) xf[c][h] = *(const ms_bf16x8*)(xr + c * MF_K + h * 32);
+    }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int c = 0; c < CW; ++c)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) asm volatile("" : "+v"(xf[c][h]));      // x is there: nothing below waits for it, and with it for W
+  ms_f32x4 acc[MATS] = {};
+#pragma unroll
+  for (int c = 0; c < CW; ++c) {
+    if (c >= chunks) break;
+    if (c >= S) {      // chunk c was asked for with chunk c - S; S - 1 of those behind it may be on their way
+      if (c + S - 1 < chunks) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * L) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    const bf16_t* b = bufs[wave] + c % S * CHUNK + li * MF_K;
+    ms_bf16x8 wf[MATS][2];
+#pragma unroll
+    for (int t = 0; t < MATS; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) wf[t][h] = *(const ms_bf16x8*)(b + t * 16 * MF_K + (((h * 4 + lq) ^ li) & 7) * 8);
+    if (c + S < chunks) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // read before the slot is filled again
+      fetch(c + S, c % S);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int t = 0; t < MATS; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[t][h], xf[c][h], acc[t], 0, 0, 0);
+  }
+  ms_f32x4* red = (ms_f32x4*)bufs;
+  static_assert(MATS * 1024 <= S * CHUNK * 2, "the parts meet in the ring's place");
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < MATS; ++t) red[(t * MF_WAVES + wave) * 64 + lane] = acc[t];
+  __syncthreads();
+  if (part) return;
+  ms_f32x4 sum[MATS];
+#pragma unroll
+  for (int t = 0; t < MATS; ++t) {
+    sum[t] = red[(t * MF_WAVES + wave) * 64 + lane];
+#pragma unroll
+    for (int p = 1; p < WK; ++p) sum[t] += red[(t * MF_WAVES + wave + p) * 64 + lane];
+  }
+  const int n = n0 + lq * 4;      // a lane holds outputs n .. n + 3 of row li; N is a multiple of 4
+  if (li >= rows || n >= N) return;
+  if (MODE == MS_DOWN) {
+    float* y = (float*)out + ((long long)(s - token * top) * n_tokens + token) * N + n;
+    *(ms_f32x4*)y = ms_f32x4{sum[0][0] * weight, sum[0][1] * weight, sum[0][2] * weight, sum[0][3] * weight};
+  } else {
+    typedef __bf16 ms_bf16x4 __attribute__((ext_vector_type(4)));
+    ms_bf16x4 v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      v[i] = from_f32<bf16_t>(GATED ? jv_gated(act, sum[0][i] * weight, sum[MATS - 1][i] * weight) : jv_act(act.id, sum[0][i] * weight));
+    *(ms_bf16x4*)((bf16_t*)out + (long long)(row0 + li) * N + n) = v;
+  }
+}
+
+template <int MODE, int WK, int CW, typename... Args>
+static int launch_moe_few(int max_tiles, int N, hipStream_t stream, Args... args) {
+  const int nb = 16 * MF_WAVES / WK;
+  const long long blocks = (long long)max_tiles * ((N + nb - 1) / nb);
+  if (blocks > 0x7fffffffll) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL((moe_few_kernel<MODE, WK, CW>), dim3((unsigned)blocks), dim3(64 * MF_WAVES), 0, stream, args...);
+  return JV_LAUNCH_CHECK();
+}
+
 template <int MODE>
 static int launch_moe_skinny(void* out, const void* a, const void* W0, const void* W1, const int* meta, const int* offsets,
                              const int* tile_expert, const int* tile_row0, const int* order, const float* weights,
                              int max_tiles, int top, int n_tokens, int K, int N, JvAct act, int use_weight, void* stream) {
   if (K < 8 || K % 8) return (int)hipErrorInvalidValue;
+  if (K % MF_K == 0 && K <= 8 * MF_WAVES * MF_K && N % 4 == 0 && (((uintptr_t)out | (uintptr_t)a | (uintptr_t)W0 | (uintptr_t)W1) & 15) == 0) {
+    auto go = [&](auto wk, auto cw) {
+      return launch_moe_few<MODE, decltype(wk)::value, decltype(cw)::value>(
+          max_tiles, N, (hipStream_t)stream, out, (const bf16_t*)a, (const bf16_t*)W0, (const bf16_t*)W1, meta, offsets, tile_expert,
+          tile_row0, order, weights, top, n_tokens, K, N, act, use_weight);
+    };
+    using std::integral_constant;
+    if (K <= 512) return go(integral_constant<int, 2>{}, integral_constant<int, 4>{});
+    if (K <= 1024 && MODE == MS_GATED) return go(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+    if (K <= 1024) return go(integral_constant<int, 2>{}, integral_constant<int, 8>{});
+    if (K <= 2048) return go(integral_constant<int, 8>{}, integral_constant<int, 4>{});
+    return go(integral_constant<int, 8>{}, integral_constant<int, 8>{});
+  }
   const int wk = K >= 2048 ? 4 : 2;
   auto kernel = wk == 4 ? moe_skinny_kernel<MODE, 4> : moe_skinny_kernel<MODE, 2>;
   const int nb = 64 / wk;

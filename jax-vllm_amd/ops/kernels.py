@@ -2258,7 +2258,10 @@ def moe_route(logits: "torch.Tensor | None", top: int, x=None, w_router=None, lo
         if how == "rows":
             logits = gemm_rows_f32out(x, w_router)
         elif how is not None:
-            logits = gemm_tile64(x, w_router, torch.float32, ksplit=how)
+            few = x.is_contiguous() and w_router.is_contiguous() and not (x.data_ptr() | w_router.data_ptr()) & 15
+            tile = few_tile(x.shape[0], *w_router.shape) if few and w_router.dtype == x.dtype else None
+            # (8 rows x 32 x 2,048: 4.1 us and one sum a number for the choice, against 4.9 and eight)
+            logits = gemm_tile64(x, w_router, torch.float32, ksplit=how) if tile is None else gemm_few(x, w_router, tile, out_dtype=torch.float32)
         if logits is not None and logits_out is not None:
             whole = logits.sum(0) if logits.dim() == 3 else logits
             logits_out.copy_(whole if bias is None else whole + bias)
