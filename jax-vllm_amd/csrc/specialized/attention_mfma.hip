@@ -1188,7 +1188,11 @@ __global__ void __launch_bounds__(256) PREFILL_OCCUPANCY attn_decode_kernel(Attn
   const int G = p.nq / p.nkv, P = p.page_size;
   const PageSplit ps{P, p.page_shift};
   const int mt_per_head = (G + 15) / 16;
-  const int w = blockIdx.x;
+  // Heads fastest: neighbouring blocks go to different dies, so every die gets the same heads' share of all requests, however
+  // uneven these are (requests fastest put all of a request's heads on one die).  With V in
+  // pieces of 16 bytes instead of 8, microseconds (before): 64 requests of 512 to 1,536 keys 57.6 (58.5), one of 1,030 keys in 8 splits
+  // with its merge 9.9 (10.4), 16 of 400 to 1,200 over 4 kv heads in 4 splits 12.6 (13.3), head size 256, 8 over one 15.5 (16.6).
+  const int heads = p.nkv * mt_per_head, w = blockIdx.x / heads, at = blockIdx.x - w * heads;
   // Without a work list the requests are 0, 1, ... and request r's token is row r (a step of
   // decoded tokens only): nothing has to be looked up before the loads below can start.  The
   // kernel's time at small batches is its chain of dependent memory round trips (~1.5 us each
@@ -1196,8 +1200,8 @@ __global__ void __launch_bounds__(256) PREFILL_OCCUPANCY attn_decode_kernel(Attn
   // once, beside the load of its context length, instead of being read key range by key range
   // after it.
   const int r = p.work ? p.work[w] : w;
-  const int g = blockIdx.y / mt_per_head, mt = blockIdx.y - g * mt_per_head;
-  const int split = blockIdx.z;
+  const int g = at / mt_per_head, mt = at - g * mt_per_head;
+  const int split = blockIdx.y;
   const int* gtable = p.block_tables + (long long)r * p.table_stride;
   // A table row beyond DEC_TBL_MAX entries does not fit: the block then copies only the entries of its own
   // split's keys, once it knows them (one more round trip, at contexts where that does not matter; the
@@ -1272,16 +1276,17 @@ __global__ void __launch_bounds__(256) PREFILL_OCCUPANCY attn_decode_kernel(Attn
   // One tile's operands, global -> registers.  Nothing here looks at a loaded value, so a tile's
   // loads are in flight while the tile before it is multiplied.  Keys at or past kv_len read the
   // null page: their scores are masked by position, their V entries are zeroed before use.
-  //   K operand: lane (key li of sub-tile kt, chunk lc) <- 8 consecutive d of that key
-  //   V^T operand: lane (d = dt*16 + li, chunk lc) <- keys kt*16 + lc*4 .. +4 of that d
+  //   K operand: lane (row li of product kt, chunk lc) <- 8 consecutive d of key 8 (li / 4) + 4 kt + li % 4, so that
+  //   a lane's scores of both products are those of keys 8 lc .. + 7, and
+  //   V^T operand: lane (d = dt*16 + li, chunk lc) <- keys lc*8 .. +8 of that d, 16 bytes (a page holds a multiple of 8)
   // `real` false (the prefetch behind the wave's last tile): everything is read from the null page.  The
   // prefetch is never skipped: after a conditional one the compiler must assume that nothing younger is
   // in flight, and its waits for this tile's operands would wait for the prefetched tile as well.
-  auto load_tile = [&](int t, bool real, bf16x8 (&kf)[2][NKS], bf16x4 (&vf)[2][NDT]) {
+  auto load_tile = [&](int t, bool real, bf16x8 (&kf)[2][NKS], bf16x8 (&vf)[NDT]) {
     const int j0 = first_key_of(t);
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt) {
-      const int j = j0 + kt * 16 + li;
+      const int j = j0 + (li >> 2) * 8 + kt * 4 + (li & 3);
       const bool ok = real && j < kv_len;
       const long long looked = page_at(ok ? ps.index(j) : some_entry);
       const long long page = ok ? looked : 0;
@@ -1292,18 +1297,17 @@ __global__ void __launch_bounds__(256) PREFILL_OCCUPANCY attn_decode_kernel(Attn
         kf[kt][ks] = *(const bf16x8*)(krow + (DK != D && d0 >= D ? 0 : d0));
       }
     }
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-      const int j = j0 + kt * 16 + lc * 4;
+    {
+      const int j = j0 + lc * 8;
       const bool ok = real && j < kv_len;
       const long long looked = page_at(ok ? ps.index(j) : some_entry);
       const long long page = ok ? looked : 0;
       const bf16_t* vbase = p.v_pages + (page * p.nkv + g) * (long long)D * P + (ok ? ps.slot(j) : 0);
 #pragma unroll
-      for (int dt = 0; dt < NDT; ++dt) vf[kt][dt] = *(const bf16x4*)(vbase + (long long)(dt * 16 + li) * P);
+      for (int dt = 0; dt < NDT; ++dt) vf[dt] = *(const bf16x8*)(vbase + (long long)(dt * 16 + li) * P);
     }
   };
-  auto multiply = [&](int t, bf16x8 (&kf)[2][NKS], bf16x4 (&vf)[2][NDT]) {
+  auto multiply = [&](int t, bf16x8 (&kf)[2][NKS], bf16x8 (&vf)[NDT]) {
     const int j0 = first_key_of(t);
     if (DK != D) {                       // columns that pad the head size to the contraction step
 #pragma unroll
@@ -1314,12 +1318,10 @@ __global__ void __launch_bounds__(256) PREFILL_OCCUPANCY attn_decode_kernel(Attn
     }
     if (j0 + BND > kv_len) {             // the last tile (the same in every lane): zero times a stale NaN is not zero
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
+      for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-        for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (j0 + kt * 16 + lc * 4 + e >= kv_len) vf[kt][dt][e] = (bf16_t)0.f;
+        for (int e = 0; e < 8; ++e)
+          if (j0 + lc * 8 + e >= kv_len) vf[dt][e] = (bf16_t)0.f;
     }
     f32x4 s[2];
 #pragma unroll
@@ -1333,7 +1335,7 @@ __global__ void __launch_bounds__(256) PREFILL_OCCUPANCY attn_decode_kernel(Attn
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int j = j0 + kt * 16 + lc * 4 + e;
+        const int j = j0 + lc * 8 + kt * 4 + e;
         const bool ok = row_ok && j <= pos && (j >= kv_begin || (MORE && j < p.keep));
         const float raw = MORE && p.cap > 0.f ? capped_score(s[kt][e], p.cap_in, p.cap) : s[kt][e];
         const float v = ok ? raw * p.scale_log2 : -INFINITY;
@@ -1358,16 +1360,12 @@ __global__ void __launch_bounds__(256) PREFILL_OCCUPANCY attn_decode_kernel(Attn
     l_lane = l_lane * alpha + psum;
     m_run = m_new;
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) {
-      const bf16x4 a0 = vf[0][dt], a1 = vf[1][dt];
-      const bf16x8 a = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-      acc[dt] = mfma16(a, b, acc[dt] * alpha);
-    }
+    for (int dt = 0; dt < NDT; ++dt) acc[dt] = mfma16(vf[dt], b, acc[dt] * alpha);
   };
   // two register sets take turns: while one tile is multiplied the wave's next one is on its way
   {
     bf16x8 kf_a[2][NKS], kf_b[2][NKS];
-    bf16x4 vf_a[2][NDT], vf_b[2][NDT];
+    bf16x8 vf_a[NDT], vf_b[NDT];
     int t = t_lo + wave;
     load_tile(t, t < t_hi, kf_a, vf_a);
     while (t < t_hi) {
@@ -1565,7 +1563,8 @@ extern "C" int jv_attn_decode(void* out, const void* q, long long q_row_stride, 
     a.part_ml = scratch + (long long)n_work * nq * a.num_splits * D;
   }
   const int G = nq / nkv, mt_per_head = (G + 15) / 16;
-  if ((long long)nkv * mt_per_head > 65535 || a.num_splits > 65535) return (int)hipErrorInvalidValue;
+  if ((long long)nkv * mt_per_head > 65535 || a.num_splits > 65535 || (long long)n_work * nkv * mt_per_head > 0x7fffffffll)
+    return (int)hipErrorInvalidValue;
   // a table row that does not fit in LDS whole: every split's own entries must (keys of a split span at most
   // ceil(tiles / splits) tiles of BND keys, hence that many keys over the page size, plus the pages it cuts)
   if (table_stride > DEC_TBL_MAX) {
@@ -1582,7 +1581,7 @@ extern "C" int jv_attn_decode(void* out, const void* q, long long q_row_stride, 
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
     if (e != hipSuccess) return (int)e;
   }
-  hipLaunchKernelGGL(kernel, dim3(n_work, nkv * mt_per_head, a.num_splits), dim3(256),
+  hipLaunchKernelGGL(kernel, dim3((unsigned)n_work * (nkv * mt_per_head), a.num_splits), dim3(256),
                      shmem, (hipStream_t)stream, a);
   int e = JV_LAUNCH_CHECK();
   if (e) return e;

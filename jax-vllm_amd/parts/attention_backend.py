@@ -22,7 +22,7 @@ import torch
 from ..ops import kernels as K
 
 TARGET_BLOCKS = 256          # blocks of the decode kernel that fill the chip: one per compute unit (measured: 8 requests of
-                             # 1,060 keys over 8 kv heads take 14.2 us with 4 splits, 16.0 with 8; 16 requests 20.3 with 2)
+                             # 1,060 keys over 8 kv heads take 13.7 us with 4 splits, 15.5 with 8)
 MIN_KEYS_PER_SPLIT = 128     # one 32-key tile for each of a block's 4 waves
 RESIDENT_BLOCKS = 2          # blocks of the prefill kernel that a compute unit holds at once
 
@@ -45,8 +45,11 @@ def keys_seen(kv_len: int, window: int, keep: int = 0) -> int:
 
 
 def decode_splits(n_decode: int, blocks_per_request: int, max_kv_len: int) -> int:
+    """Blocks that share out a request's keys: as many as give no unit a second block (one more costs a further merge and leaves
+    units with twice the load of others: 12 requests of 500 to 1,500 keys over 8 kv heads 18.9 us with 2, 22.2 with 3; 24 of 450 to 1,350
+    24.7 with 1, 29.6 with 2; 9 of 500 to 1,500 15.4 with 3, 19.3 with 4)."""
     base = max(1, n_decode * blocks_per_request)
-    by_fill = -(-TARGET_BLOCKS // base)
+    by_fill = max(1, TARGET_BLOCKS // base)
     by_len = max(1, max_kv_len // MIN_KEYS_PER_SPLIT)
     return max(1, min(by_fill, by_len))
 
