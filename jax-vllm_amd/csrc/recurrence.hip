@@ -13,13 +13,9 @@
 // enters it is float.  The state of a request lives in a row of `state` [slots + 1][heads][dim][vdim]
 // between steps.  Columns of S never mix, so a block takes one (request, head, slice of columns) and a
 // thread keeps up to RC_ROWS rows of one column in registers.
-#include "common.h"
+#include "recurrence_math.h"
 
 #define RC_ROWS 32
-#define RC_MAX_LAGS 7        // a convolution has at most 8 taps
-
-__device__ __forceinline__ float rc_silu(float z) { return z / (1.f + expf(-z)); }
-__device__ __forceinline__ float rc_softplus(float z) { return z > 20.f ? z : log1pf(expf(z)); }
 
 // ---------------------------------------------------------------- short causal convolution with state
 // out[t][c] = act( bias[c] + sum_j w[c][j] * in[t - (taps - 1) + j][c] ), in = proj[:, c_off + c] of the

@@ -17,7 +17,7 @@
 // r, k, v and the decay's rate are products in the activation type; everything from there on is float.  The state of a
 // request lives in a row of `state` [slots + 1][heads][dim][vdim] between steps.  Columns of S never mix, so a block
 // takes one (request, head, slice of columns) and a thread keeps up to WKV_ROWS rows of one column in registers.
-#include "common.h"
+#include "recurrence_math.h"
 
 #define WKV_ROWS 32
 
@@ -345,14 +345,6 @@ wkv_apply_kernel(float* __restrict__ out, const float* __restrict__ scratch, con
 }
 
 // ---------------------------------------------------------------- decays from a projection of small rank
-// log(1 + e^-a) for a >= 0: u = 1 + e rounded, and log(u) e / (u - 1) takes that rounding back (Kahan's log1p), so the
-// hardware's logarithm and exponential give the result to a few units in the last place.
-__device__ __forceinline__ float softplus_of_negative(float a) {
-  const float e = __builtin_amdgcn_exp2f(-a * 1.4426950408889634f);
-  const float u = 1.f + e, d = u - 1.f;
-  return d > 0.f ? __builtin_amdgcn_logf(u) * 0.6931471805599453f * (e * __builtin_amdgcn_rcpf(d)) : e;
-}
-
 // out[t][c] = log(sigmoid(z)) / tau,  z = sum_r W[c][r] low[t][r] + b[c]; W [channels][rank] and low (rows of stride ldl) in
 // the activation type, sums and logarithm float.  grid (channel blocks of 256, blocks of LD_TOKENS tokens).
 #define LD_TOKENS 8

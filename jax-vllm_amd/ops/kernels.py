@@ -2089,6 +2089,76 @@ def step_chunk_plan(ctx, dim: int, delta: bool = False):
     return plan
 
 
+def recurrence_token_possible(dim: int, vdim: int, state: torch.Tensor) -> bool:
+    """Whether ``delta_token`` and ``gated_linear_token`` take heads of these sizes with this state: a block holds the whole of a
+    head's state in registers, in pieces of 16 bytes of a row."""
+    return dim <= library.core().jv_recurrence_token_max_dim() and 4 <= vdim <= library.core().jv_recurrence_token_max_dim() \
+        and vdim % 4 == 0 and state.data_ptr() % 16 == 0
+
+
+def _token_operands(proj, cols, norm_weight, state, slot_ids, cu_seqlens, heads: int, dim: int, vdim: int):
+    """What both kernels of one token check: ``cols`` are (first column, columns) read from rows of ``proj``."""
+    _dev(proj, norm_weight, state, slot_ids, cu_seqlens)
+    n, ld = proj.shape
+    _need(all(0 <= c and c + width <= ld for c, width in cols), "proj rows are too short")
+    _f32(norm_weight, "norm weight", vdim)
+    _f32(state, "state")
+    _need(state.dim() == 4 and tuple(state.shape[1:]) == (heads, dim, vdim), "state must be [slots, heads, dim, vdim]")
+    _i32(slot_ids, "slot_ids")
+    _i32(cu_seqlens, "cu_seqlens", slot_ids.numel() + 1)
+    _need(n <= slot_ids.numel(), "a request has one token at most")
+    return torch.empty((n, heads * vdim), dtype=proj.dtype, device=proj.device)
+
+
+def delta_token(proj, at: int, conv_weight, conv_state, dt_bias, a_log, unit_eps: float, q_scale: float, norm_weight, eps: float,
+                out_scale: float, state, slot_ids, cu_seqlens, heads: int, dim: int, vdim: int) -> torch.Tensor:
+    """A decode step (one token a request at most) of the gated delta rule behind its input product, in one launch: ``short_conv``,
+    ``recurrence_gates``, ``head_unit_norm``, ``recurrence_steps`` and ``group_gated_norm`` over the columns [q | k | v | gate | decay |
+    write strength] of ``proj`` from ``at``, a q/k head per head.  Returns [n, heads * vdim] of ``proj``'s type."""
+    channels = heads * (2 * dim + vdim)
+    gate_at = at + channels
+    out = _token_operands(proj, ((at, channels + heads * (vdim + 2)),), norm_weight, state, slot_ids, cu_seqlens, heads, dim, vdim)
+    _dev(conv_weight, conv_state, dt_bias, a_log)
+    _need(conv_weight.dim() == 2 and conv_weight.shape[0] == channels, "weight must be [channels, taps]")
+    taps = conv_weight.shape[1]
+    _f32(conv_weight, "weight")
+    _need(1 <= taps <= short_conv_max_taps(), f"a convolution of {taps} taps: the kernel takes up to {short_conv_max_taps()}")
+    _f32(conv_state, "conv state")
+    _need(conv_state.dim() == 3 and tuple(conv_state.shape[1:]) == (taps - 1, channels), "state must be [slots, taps - 1, channels]")
+    _f32(dt_bias, "dt_bias", heads)
+    _f32(a_log, "a_log", heads)
+    fn = getattr(library.core(), f"jv_delta_token_{_suffix(proj.dtype)}")
+    _check(fn(_ptr(out), _ptr(proj), c_longlong(proj.shape[1]), c_int(at), c_int(gate_at), c_int(gate_at + heads * vdim),
+              c_int(gate_at + heads * vdim + heads), c_int(taps), _ptr(conv_weight), _ptr(conv_state), _ptr(dt_bias), _ptr(a_log),
+              c_float(unit_eps), c_float(q_scale), _ptr(norm_weight), c_float(eps), c_float(out_scale), _ptr(state), _ptr(slot_ids),
+              _ptr(cu_seqlens), c_int(slot_ids.numel()), c_int(heads), c_int(dim), c_int(vdim), _stream()), "delta_token")
+    return out
+
+
+def gated_linear_token_possible(dim: int, vdim: int, rank: int, state: torch.Tensor) -> bool:
+    """Longer products for the decays are better spread over more blocks (``low_rank_decay``)."""
+    return rank <= library.core().jv_recurrence_token_max_rank() and recurrence_token_possible(dim, vdim, state)
+
+
+def gated_linear_token(proj, at: int, decay_up, decay_bias, tau: float, q_scale: float, norm_weight, eps: float, state, slot_ids,
+                       cu_seqlens, heads: int, dim: int, vdim: int) -> torch.Tensor:
+    """A decode step (one token a request at most) of gated linear attention behind its input product, in one launch:
+    ``low_rank_decay``, ``wkv_steps`` read after the update and ``group_gated_norm`` over the columns [q | k | v | gate | the decay's
+    inner size] of ``proj`` from ``at``.  Returns [n, heads * vdim] of ``proj``'s type."""
+    gate_at = at + heads * (2 * dim + vdim)
+    rank = decay_up.shape[1]
+    out = _token_operands(proj, ((at, heads * (2 * dim + 2 * vdim) + rank),), norm_weight, state, slot_ids, cu_seqlens, heads, dim, vdim)
+    _dev(decay_up, decay_bias)
+    _need(decay_up.dtype == proj.dtype and decay_up.shape[0] == heads * dim, "decay_up must be [heads * dim, rank] of proj's type")
+    _f32(decay_bias, "bias", heads * dim)
+    fn = getattr(library.core(), f"jv_gated_linear_token_{_suffix(proj.dtype)}")
+    _check(fn(_ptr(out), _ptr(proj), c_longlong(proj.shape[1]), c_int(at), c_int(gate_at), c_int(gate_at + heads * vdim), c_int(rank),
+              _ptr(decay_up), _ptr(decay_bias), c_float(tau), c_float(q_scale), _ptr(norm_weight), c_float(eps), _ptr(state),
+              _ptr(slot_ids), _ptr(cu_seqlens), c_int(slot_ids.numel()), c_int(heads), c_int(dim), c_int(vdim), _stream()),
+           "gated_linear_token")
+    return out
+
+
 NORM_GATES = {"silu": 1, "sigmoid": 2}
 
 

@@ -198,6 +198,10 @@ class GatedDeltaMixer:
     def forward_projected(self, proj, at: int, ctx: StepContext, mem: LayerMemory):
         """The mixer behind its input product, whose columns begin at ``at``."""
         H, d, dv, qk, inner = self.heads, self.dim, self.vdim, self.qk, self.inner
+        if ctx.decode_only and self.qk_heads == H and K.recurrence_token_possible(d, dv, mem.states["S"]):
+            y = K.delta_token(proj, at, self.conv_w, mem.states["conv"], self.dt_bias, self.a_log, self.unit_eps, d ** -0.5,
+                              self.norm_weight, self.eps, self.out_scale, mem.states["S"], ctx.slot_ids, ctx.cu_seqlens, H, d, dv)
+            return K.linear(y, self.w_o, partial_ok=True)
         qkv = K.short_conv(proj, at, self.channels, self.conv_w, None, mem.states["conv"], ctx.slot_ids, ctx.cu_seqlens,
                            ctx.max_q_len)
         gate_at = at + self.channels
@@ -350,6 +354,10 @@ class GatedLinearAttention:
         k_at, v_at = at + H * d, at + 2 * H * d
         gate_at = v_at + H * dv
         low_at = gate_at + H * dv
+        if ctx.decode_only and K.gated_linear_token_possible(d, dv, self.rank, mem.states["S"]):
+            y = K.gated_linear_token(proj, at, self.w_decay_up, self.b_decay, self.tau, d ** -0.5, self.norm_weight, self.eps,
+                                     mem.states["S"], ctx.slot_ids, ctx.cu_seqlens, H, d, dv)
+            return K.linear(y, self.w_o, partial_ok=True)
         log_decay = K.low_rank_decay(proj[:, low_at:low_at + self.rank], self.w_decay_up, self.b_decay, self.tau)
         o = K.wkv_steps(proj[:, at:k_at], proj[:, k_at:v_at], proj[:, v_at:gate_at], log_decay, None, None, mem.states["S"],
                         ctx.slot_ids, ctx.cu_seqlens, H, d, dv, chunk_plan=K.wkv_chunk_plan(ctx, d), after=True,
