@@ -42,6 +42,9 @@ moe_mfma_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, const
   constexpr int NB = GATED ? TW / 2 : TW;           // output columns of a block
   constexpr int XI = TM / 8 / WAVES, WI = TW / 8 / WAVES;      // instructions a wave brings of a chunk, each 8 rows of 128 bytes
   constexpr int BUF = (TM + TW) * MM_K;             // elements of a buffer: rows of x, then rows of W
+  constexpr bool RING = BUFS == 0;                  // units of half the rows of x and of W of a chunk in a ring of five
+  constexpr int HALF = BUF / 2, SLOTS = 5;
+  static_assert(!RING || (WAVES == 8 && MT == 3 && WI == 4), "how a wave's loads fall on the two units of a chunk");
   // Blocks b, b + 8, b + 16, ... run on one XCD (with an L2 of its own): each of the 8 takes one run of the (tile, rows of W)
   // pairs, rows of W fastest, so the rows of x of a tile and the weights of an expert are read into one L2 and used there.
   const int per_tile = (N + NB - 1) / NB;
@@ -49,7 +52,7 @@ moe_mfma_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, const
   const int pair = ((int)blockIdx.x & 7) * chunk + ((int)blockIdx.x >> 3);
   if (((int)blockIdx.x >> 3) >= chunk || pair >= live) return;
   const int tile = pair / per_tile;
-  __shared__ __attribute__((aligned(1024))) bf16_t bufs[BUFS * BUF];
+  __shared__ __attribute__((aligned(1024))) bf16_t bufs[RING ? SLOTS * HALF : BUFS * BUF];
   __shared__ int from[TM];                  // a row's row of x
   __shared__ long long to[TM];              // where its results go
   __shared__ float wts[TM];
@@ -73,14 +76,19 @@ moe_mfma_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, const
   int col[2];                               // a lane's columns in a chunk, for rows 16 i + lr and 16 i + 8 + lr
 #pragma unroll
   for (int h = 0; h < 2; ++h) col[h] = (((lane & 7) ^ ((lr + 8 * h) >> 1)) & 7) * 8;
+  // In a ring, unit h of a chunk has rows h TM / 2 .. of x and h TW / 2 .. of W.  A wave brings 8 rows of x and 16 of W of each, and the 8
+  // that are left over of x: of unit 0 by waves 0 to 3, of unit 1 by 4 to 7.  src: x of units 0, 1, left over; W two of unit 0, two of 1.
+  auto first_row = [&](int i) {             // of instruction i of this wave, in x or in W
+    if (!RING) return (i < XI ? wave * XI + i : wave * WI + i - XI) * 8;
+    if (i < 2) return i * (TM / 2) + wave * 8;
+    if (i == 2) return (wave >> 2) * (TM / 2) + 64 + (wave & 3) * 8;
+    return ((i - XI) >> 1) * (TW / 2) + (wave * 2 + ((i - XI) & 1)) * 8;
+  };
 #pragma unroll
-  for (int i = 0; i < XI; ++i) {
-    const int r = (wave * XI + i) * 8 + lr;
-    src[i] = a_rows + (long long)from[r] * K;
-  }
+  for (int i = 0; i < XI; ++i) src[i] = a_rows + (long long)from[first_row(i) + lr] * K;
 #pragma unroll
   for (int i = 0; i < WI; ++i) {
-    const int r = (wave * WI + i) * 8 + lr;
+    const int r = first_row(XI + i) + lr;
     // gated: rows 64 w .. + 31 of the block's W are gate rows 32 w .. + 31, the 32 behind them the same rows of up
     const int n = GATED ? n0 + (r >> 6) * 32 + (r & 31) : n0 + r;
     const bf16_t* w = GATED && (r & 32) ? W1 : W0;
@@ -107,6 +115,66 @@ moe_mfma_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, const
   // wave (wm, wn): rows of x (TM / 2) wm .., rows of W 64 wn ..
   const int wm = wave & 1, wn = wave >> 1, l32 = lane & 31, half = lane >> 5, swz = (l32 >> 1) & 7;
   const int chunks = (K + MM_K - 1) / MM_K;
+  if constexpr (RING) {
+    auto load = [&](int i, int c, int slot) {       // instruction i, columns of chunk c, into the slot of its unit
+      const int row = first_row(i), h = i < 2 ? i : i == 2 ? wave >> 2 : (i - XI) >> 1;
+      const int in_unit = i < XI ? row - h * (TM / 2) : TM / 2 + row - h * (TW / 2), k = c * MM_K + col[(in_unit >> 3) & 1];
+      const bf16_t* piece = k < K ? src[i] + k : (const bf16_t*)mm_zeros;
+      const unsigned at = (unsigned)(unsigned long long)(const __attribute__((address_space(3))) void*)(bufs + slot * HALF + in_unit * MM_K);
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(piece), "s"(at) : "memory", "m0");
+    };
+    // load j of a wave's 4 (or 3: no left-over rows) of unit h
+    auto unit = [&](int j, int h, int c, int slot) {
+      if (j < 2) load(XI + 2 * h + j, c, slot);
+      else if (j == 2) load(h, c, slot);
+      else if ((wave >> 2) == h) load(2, c, slot);
+    };
+    auto wrap = [](int v) { return v >= SLOTS ? v - SLOTS : v; };
+    bf16x8 xf[2][MT], wf[2][2];
+    auto read = [&](int i, int set, int ks, int s0) {      // s0: slot of the chunk's first unit
+      const int at = ((ks * 2 + half) ^ swz) * 8;
+      if (i < 2) wf[set][i] = *(const bf16x8*)(bufs + wrap(s0 + (wn >> 1)) * HALF + (TM / 2 + (wn & 1) * 64 + i * 32 + l32) * MM_K + at);
+      else xf[set][i - 2] = *(const bf16x8*)(bufs + wrap(s0 + wm) * HALF + ((i - 2) * 32 + l32) * MM_K + at);
+    };
+    // Chunk c: its products, the reads of the next 16 columns between them, and the loads of units 2 c + 4 and 2 c + 5 into the slots
+    // that chunks c - 1 and c left.  more: 2: those units exist; 1: chunk c + 1 exists; 0: the last.
+    auto chunk = [&](auto more, int c, int s0) {
+      constexpr int MORE = decltype(more)::value;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const int set = ks & 1;
+        if (ks == 3 && MORE > 0) {      // chunk c is in registers everywhere, c + 1 is there; unit 2 c + 4 may be on its way
+          if (MORE == 1) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+          else if (wave < 4) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+          else asm volatile("s_waitcnt vmcnt(3) lgkmcnt(0)" ::: "memory");
+          __builtin_amdgcn_s_barrier();
+          asm volatile("" ::: "memory");
+        }
+#pragma unroll
+        for (int i = 0; i < 2 * MT; ++i) {
+          if (i < MT + 2 && (ks < 3 || MORE > 0)) read(i, set ^ 1, (ks + 1) & 3, ks < 3 ? s0 : wrap(s0 + 2));
+          if (MORE > 1 && ks < 3 && (ks * 6 + i) % 4 == 1 && (ks * 6 + i) / 4 < 4) unit((ks * 6 + i) / 4, 0, c + 2, wrap(s0 + 4));
+          if (MORE > 1 && ks == 3 && i < 4) unit(i, 1, c + 2, s0);
+          acc[i / MT][i % MT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[set][i % MT], wf[set][i / MT], acc[i / MT][i % MT], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    };
+    for (int c = 0; c < 2 && c < chunks; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) unit(j, h, c, 2 * c + h);
+    if (chunks > 1) asm volatile("s_waitcnt vmcnt(7)" ::: "memory");      // of both units of a chunk a wave has 7
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < MT + 2; ++i) read(i, 0, 0, 0);
+    int c = 0, s0 = 0;
+    for (; c + 2 < chunks; ++c, s0 = wrap(s0 + 2)) chunk(std::integral_constant<int, 2>{}, c, s0);
+    if (c + 1 < chunks) { chunk(std::integral_constant<int, 1>{}, c, s0); ++c, s0 = wrap(s0 + 2); }
+    chunk(std::integral_constant<int, 0>{}, c, s0);
+  } else {
   for (int c = 0; c < BUFS - 1 && c < chunks; ++c) fetch(c * MM_K, c);
   for (int c = 0, buf = 0; c < chunks; ++c, buf = buf + 1 == BUFS ? 0 : buf + 1) {
     // this wave's part of chunk c is there (loads arrive in order; those of the next BUFS - 2 chunks may be on their way)
@@ -129,6 +197,7 @@ moe_mfma_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, const
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[a][mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[mt], wf[a], acc[a][mt], 0, 0, 0);
     }
+  }
   }
   // a lane holds column l32 of both tiles of W, rows 8 q + 4 half + i of each tile of x
 #pragma unroll
@@ -166,15 +235,18 @@ static int launch_moe_tiles(int max_tiles, hipStream_t stream, void* out, const 
   return JV_LAUNCH_CHECK();
 }
 
-// 128 rows against 256 of W by 8 waves with two chunks on their way; 192 rows with one, for groupings that fill the units with fewer
-// tiles (32 experts x 512, width 2,048, 256 rows each: 256 tiles instead of 320, gate/up 57 us, before 85); 64 rows against 128 by 4 waves, three blocks a compute unit with
+// 128 rows against 256 of W by 8 waves with two chunks on their way; 192 rows, for groupings that fill the units with fewer tiles (32
+// experts x 512, width 2,048, 256 rows each: 256 tiles instead of 320, gate/up 61 us, before 85), through a ring of five half chunks
+// (three whole ones do not fit), whose loads are spread over the products: both products of 4,096 tokens, 8 of 64 x 1,024, width 4,096
+// 1,038 us (1,136 with two whole buffers), width 2,048 547 (597), 2 of 8 x 4,096 605 (654), 4 of 32 x 512 at 2,500 tokens 108 (113);
+// 64 rows against 128 by 4 waves, three blocks a compute unit with
 // one chunk on its way each, or (`deep`) two blocks with two: where an expert gets so few rows that nearly all are one tile, the
 // stream of the weights is what is waited for.  gate/up + down, cold weights, microseconds (deep / not): 64 experts x 1,024, width
 // 4,096, 25 rows each 302 / 334, 8 x 4,096 at 40 rows 167 / 184, 16 x 2,048, width 1,024, at 25 56 / 64, 32 x 512, width 2,048, at
 // 40 52 / 57; at 50 rows, with second tiles, 66 / 62.
 template <int MODE, typename... Args>
 static int launch_moe_mfma(int tile_rows, int deep, Args... args) {
-  if (tile_rows == 192) return launch_moe_tiles<MODE, 192, 256, 2>(args...);
+  if (tile_rows == 192) return launch_moe_tiles<MODE, 192, 256, 0>(args...);
   if (tile_rows == 128) return launch_moe_tiles<MODE, 128, 256, 3>(args...);
   if (tile_rows == 64 && deep) return launch_moe_tiles<MODE, 64, 128, 3>(args...);
   if (tile_rows == 64) return launch_moe_tiles<MODE, 64, 128, 2>(args...);

@@ -2304,14 +2304,15 @@ def moe_tile_rows_for(dtype, hidden: int, ff: int, entries: int, experts: int) -
     most, 128 where the matrix-core kernels run and an expert gets more than 64 rows on average (a second tile of 64 would be
     nearly empty: 8 experts x 4,096 of width 4,096 at 75 rows each 198 us with 128, 270 with 64; 64 x 1,024 at 68 rows 361 / 430,
     128 x 768 of width 2,048 at 68 rows 296 / 313; at 60 rows 32 x 512 66 / 61), else 64.  192 instead of 128 where that spares so many
-    rounds over the compute units (``moe_tile_rounds``) that their longer chunks, 1.45 times the time, are made up for: 2,048 tokens, 4 of 32
-    experts x 512, width 2,048 111 us (138 with 128), 1,500 tokens 111 (86); 4,096 tokens, 8 of 64 x 1,024 571 (633), 2,048 382 (371)."""
+    rounds over the compute units (``moe_tile_rounds``) that their longer chunks, 1.2 times the time, are made up for: 2,048 tokens, 4 of 32
+    experts x 512, width 2,048 (0.55 of the rounds) 108 us (138 with 128), 1,500 tokens (1.0) 107 (94); 4,096 tokens, 8 of 64 x 1,024 (0.67) 547
+    (657), 2,048 (0.80) 366 (377); 2,048 tokens, 4 of 32 x 768 (0.88) 164 (157)."""
     if moe_matrix_cores_possible(dtype, hidden, ff):
         if entries <= MOE_SKINNY_MAX_MEAN * experts:
             return MOE_SKINNY_ROWS
         if entries > 64 * experts:
             larger, smaller = (moe_tile_rounds(rows, hidden, ff, entries, experts) for rows in (192, 128))
-            return 192 if 1.45 * larger < smaller else 128
+            return 192 if 1.2 * larger < smaller else 128
     return moe_tile_rows()
 
 

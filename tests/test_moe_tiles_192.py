@@ -35,5 +35,6 @@ def test_where_tiles_of_192_are_chosen():
         return moe_tile_rows_for(torch.bfloat16, hidden, ff, tokens * top, experts)
 
     assert [rows(n, 32, 4, 2048, 512) for n in (2048, 1500, 1024, 512)] == [192, 128, 128, 64]
-    assert [rows(n, 64, 8, 2048, 1024) for n in (4096, 2048)] == [192, 128]
+    assert [rows(n, 64, 8, 2048, 1024) for n in (4096, 2048)] == [192, 192]
+    assert [rows(n, 32, 4, 2048, 768) for n in (4096, 2048)] == [192, 128]
     assert moe_tile_rows_for(torch.float32, 2048, 512, 8192, 32) == 64
