@@ -1,4 +1,4 @@
-// y[parts][M,N] = x[M,K] W[N,K]^T for 129 to 1,024 rows against a narrow W with a long inner size (the down and output products
+// y[parts][M,N] = x[M,K] W[N,K]^T for 129 to 1,792 rows against a narrow W with a long inner size (the down and output products
 // of prompts), bf16 in, float sums: `ksplit` blocks share out the inner size of a tile, as float partial products that the
 // reader adds in order, because the tiles of y alone do not fill the chip.
 //
@@ -11,7 +11,8 @@
 // that hands a chunk over stands before the products of the last 16 columns, whose operands are in registers.
 //
 // Against 4,096 x 12,288, microseconds (the library's bf16 product): 160 rows 36.9 (77.7), 300 rows 48.3 (69.6), 512 rows 54.2
-// (81.6), 1,024 rows 94.1 (116); against 4,096 x 4,096: 17.0 (27.5), 20.5 (26.0), 25.8 (30.0), 39.2 (42.7).
+// (81.6), 1,024 rows 94.1 (116); against 4,096 x 4,096: 17.0 (27.5), 20.5 (26.0), 25.8 (30.0), 39.2 (42.7).  With the norm that adds the parts, against 4,096 x 12,288: 1,525 rows by tiles of 192 x 256 (96 x 128 a wave,
+// one a SIMD) 140 (162); 5,120 x 17,408 185 at 1,152 rows (310).
 #include "common.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -157,7 +158,7 @@ static int sh_launch(float* y, const void* x, const void* W, int M, int N, int K
                      (const bf16_t*)x, (const bf16_t*)W, M, N, K, ksplit);
   return JV_LAUNCH_CHECK();
 }
-// tm, tw: rows of x and of W of a tile, (128, 128), (256, 128) or (256, 256); y float [ksplit][M][N].
+// tm, tw: rows of x and of W of a tile, (128, 128), (256, 128), (192, 256) or (256, 256); y float [ksplit][M][N].
 extern "C" int jv_gemm_shares_bf16(float* y, const void* x, const void* W, int M, int N, int K, int tm, int tw, int ksplit, void* stream) {
   if (M <= 0 || N <= 0) return 0;
   if (K < SH_K || K % SH_K || K > 1 << 20 || N % 4 || ksplit < 1 || ksplit > K / SH_K || (((uintptr_t)x | (uintptr_t)W | (uintptr_t)y) & 15))
@@ -165,6 +166,7 @@ extern "C" int jv_gemm_shares_bf16(float* y, const void* x, const void* W, int M
   const hipStream_t s = (hipStream_t)stream;
   if (tm == 128 && tw == 128) return sh_launch<128, 128, 2, 2>(y, x, W, M, N, K, ksplit, s);
   if (tm == 256 && tw == 128) return sh_launch<256, 128, 2, 2>(y, x, W, M, N, K, ksplit, s);
+  if (tm == 192 && tw == 256) return sh_launch<192, 256, 2, 2>(y, x, W, M, N, K, ksplit, s);
   if (tm == 256 && tw == 256) return sh_launch<256, 256, 2, 4>(y, x, W, M, N, K, ksplit, s);
   return (int)hipErrorInvalidValue;
 }

@@ -1169,9 +1169,25 @@ def shares_plan(m: int, n: int, k: int, cus: int = 256):
     return best[1] if best is not None and best[0] < 3.0 + k * (0.0036 + 1.32e-9 * m * n) else None
 
 
+def tall_shares_plan(m: int, n: int, k: int, cus: int = 256):
+    """The same for 1,025 to 1,792 rows against a long inner size: halves of it by tiles of 192 x 256, or of 256 x 256 where those would
+    be more blocks than compute units, if they are one round that leaves at most a quarter of the units idle.  The library, whose tiles leave
+    a round mostly empty there, and this, microseconds with the norm that reads the result, 126 sizes measured: against 4,096 x 12,288 at
+    1,025, 1,152, 1,525 rows 147, 129, 162 / 135, 125, 140, at 1,600 and 1,792 308, 182 / 168, 171 (1,900: 183 / 188); 5,120 x 17,408 at 1,025 and
+    1,536 284, 371 / 178, 239; 5,120 x 8,192 at 1,025 104 / 96, by tiles of 256 x 256 at 1,344 117 / 124; 4,096 x 4,096 at 1,525 61 / 64."""
+    if not SHARES_MAX_ROWS < m <= 1792 or k % 64 or n % 4 or k < 8192:
+        return None
+    for tm, tw in ((192, 256), (256, 256)):
+        if tm == 192 or k >= 12288:
+            blocks = -(-m // tm) * -(-n // tw) * 2
+            if 0.75 * cus <= blocks <= cus:
+                return tm, tw, 2
+    return None
+
+
 def gemm_shares(x: torch.Tensor, w: torch.Tensor, form) -> torch.Tensor:
     """x @ w.T for bfloat16 x [M, K] and w [N, K], K a multiple of 64, as float32 partial products [parts, M, N] to be added in
-    order.  ``form``: (rows of x, rows of w of a tile, parts), see ``shares_plan``."""
+    order.  ``form``: (rows of x, rows of w of a tile, parts), see ``shares_plan`` and ``tall_shares_plan``."""
     _dev(x, w)
     _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "gemm_shares takes bfloat16")
     m, k = x.shape
@@ -1194,7 +1210,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
     bfloat16 otherwise: a plain library matrix product (hipBLASLt through torch), float accumulation.
     With ``partial_ok`` the caller takes a float32 stack [parts, M, N] of partial products as well
     (to be added in order, as ``add_rmsnorm`` does); it is returned for narrow matrices at up to 128 rows, and up to 1,024
-    where the inner size is long (``shares_plan``)
+    where the inner size is long (``shares_plan``), 1,792 where it is 8,192 or more (``tall_shares_plan``)
     (``partial_max_width``: the widest row whose parts the caller's reader adds; None: any).
     With ``gate_pairs`` (one of ``GATE_ACTIVATIONS``) the rows of w alternate gate and up rows and the
     result is act(x.w[2j]) * (x.w[2j+1]) of width N/2 (an epilogue of the streaming kernels, a kernel
@@ -1219,7 +1235,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
                 return gemm_stream(x, w, form, mode, gate_pairs, out_dtype or torch.bfloat16)
         elif k % 64 == 0 and m > STREAM_MAX_ROWS and partial_ok and not gate_pairs and scale is None and w.dtype == torch.bfloat16 \
                 and out_dtype in (None, torch.bfloat16) and partial_max_width is not None and n <= partial_max_width:
-            form = shares_plan(m, n, k, compute_units(x.device))
+            cus = compute_units(x.device)
+            form = shares_plan(m, n, k, cus) or tall_shares_plan(m, n, k, cus)
             if form is not None and x.is_contiguous() and w.is_contiguous() and not (x.data_ptr() | w.data_ptr()) & 15:
                 return gemm_shares(x, w, form)
         plan = streaming_plan(x.shape[0], w.shape[0], w.shape[1], bool(gate_pairs),
