@@ -1241,7 +1241,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
                 return gemm_shares(x, w, form)
         plan = streaming_plan(x.shape[0], w.shape[0], w.shape[1], bool(gate_pairs),
                               partial_ok and out_dtype in (None, torch.bfloat16), x.device, partial_max_width)
-        if plan in (None, STAGED) and m <= SKINNY_AUTO_ROWS and not k % 64 and w.dtype == torch.bfloat16 and out_dtype in (None, torch.bfloat16, torch.float32):
+        if plan in (None, STAGED) and m <= SKINNY_AUTO_ROWS and not k % 64 and scale is None and w.dtype == torch.bfloat16 \
+                and out_dtype in (None, torch.bfloat16, torch.float32):
             tile = few_tile(m, n, k, compute_units(x.device))
             if tile is not None and x.is_contiguous() and w.is_contiguous() and not (x.data_ptr() | w.data_ptr()) & 15 \
                     and not (gate_pairs and out_dtype == torch.float32):

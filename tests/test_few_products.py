@@ -51,3 +51,21 @@ def test_rows_of_w_of_a_block():
 
     assert [few_tile(8, n, 2048) for n in (32, 4096, 4112, 6144, 6160, 11296)] == [16, 16, 32, 32, 16, 16]
     assert streaming_plan(8, 6144, 2048, True) == STAGED and streaming_plan(12, 12288, 4096) is None
+
+
+@pytest.mark.parametrize("m,n,k,partial_ok", [(4, 2048, 2048, False), (1, 151936, 4096, False), (12, 12288, 4096, False), (3, 96, 512, True), (16, 32, 512, False)])
+def test_rows_without_their_scale_are_refused(monkeypatch, m, n, k, partial_ok):
+    """Only blocks that stay multiply a row by its norm's scale: every other plan says so instead of leaving the scale out."""
+    from jax_vllm_amd.ops import kernels
+
+    def launched(*_, **__):
+        raise AssertionError("a product of rows whose scale is still to be applied")
+
+    monkeypatch.setattr(kernels, "compute_units", lambda device: 256)
+    for name in ("gemm_few", "gemm_skinny", "gemm_stream", "gemm_tile64", "gemm_shares"):
+        monkeypatch.setattr(kernels, name, launched)
+    x, w = torch.zeros(m, k, dtype=torch.bfloat16), torch.empty(n, k, dtype=torch.bfloat16)      # (never read)
+    rows = kernels.UnscaledRows(x, torch.ones(m, kernels.UNSCALED_MAX_SHARES), k, 1e-6)
+    assert not kernels.linear_takes_unscaled_rows(m, w, partial_ok=partial_ok)
+    with pytest.raises(kernels.KernelArgumentError, match="un-normalised rows"):
+        kernels.linear(rows, w, partial_ok=partial_ok)
