@@ -236,7 +236,7 @@ def run(att, out, qkv, ctx, mem) -> None:
             ctx.positions, att.nq, att.nkv, att.d, att.scale, window, sinks=sinks, cap=cap, keep=keep,
         )
         return
-    key = ("mfma_attention_plan", att.nq, att.nkv, att.d, window, keep, ctx.page_size)     # (prompts written out have pages of their own)
+    key = ("mfma_attention_plan", att.nq, att.nkv, att.d, window, keep)
     plan = ctx.plans.get(key)
     if plan is None:
         plan = ctx.plans[key] = plan_mfma(ctx, att.nq, att.nkv, att.d, window, qkv.device, keep)
