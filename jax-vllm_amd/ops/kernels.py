@@ -1694,92 +1694,6 @@ def latent_query_rope(q, qe, heads: int, dim: int, rot: int, rot_dims: int, rank
               c_int(rank), _ptr(cos_sin if rot_dims else None), c_int(1 if interleaved else 0), _stream()), "latent_query_rope")
 
 
-# Tokens of a step from which prompts of latent attention write out their heads' keys and values: from there on the
-# pairs spared outweigh two more launches.  8 layers of 16 heads of 64 + 32 over a vector of 224 + 32, window 1,024, latent / written out,
-# microseconds: 256 tokens 2,640 / 2,674, 384 2,732 / 2,741, 512 2,801 / 2,773, 5 prompts of 512 2,862 / 2,844, 1,024 2,931 / 2,851, 4 of
-# 1,024 3,018 / 2,916, 2,048 3,400 / 3,021, 5 of 2,048 3,247 / 3,035.
-LATENT_EXPAND_MIN_TOKENS = 512
-
-
-def latent_expand_possible(dtype, dim: int, rot: int, vdim: int, rank: int) -> bool:
-    """Whether prompts can go through heads of ``dim + rot`` written out (``latent_expand``) and the prefill kernel is one of those
-    whose waves split the keys' tiles (the sizes at which it was measured against the latent's own space), and that saves half of a
-    pair's products at least."""
-    lib = library.core()
-    d = dim + rot
-    return (dtype == torch.bfloat16 and attn_prefill_waves_split(d) and d <= 128 and 2 * d <= rank + rot <= lib.jv_latent_expand_max_vector()
-            and 16 <= dim and dim % 16 == 0 and 16 <= vdim <= d and vdim % 16 == 0 and rot % 8 == 0 and rank % 32 == 0)
-
-
-def latent_expand_tokens() -> int:
-    """Tokens of a page of what ``latent_expand`` writes."""
-    return library.core().jv_latent_expand_tokens()
-
-
-def latent_expand_plan(q_lens, device):
-    """(pages int32 [pages, 2] = (first row of the step, tokens), their number, block tables int32 [requests, width]) of prompts that begin
-    their requests: every request's tokens cut into pages, numbered in order."""
-    size = latent_expand_tokens()
-    pages, first, at = [], [0], 0
-    for n in q_lens:
-        pages += [(at + b, min(size, n - b)) for b in range(0, n, size)]
-        first.append(len(pages))
-        at += n
-    width = max(b - a for a, b in zip(first, first[1:]))
-    flat = [x for p in pages for x in p]
-    for a, b in zip(first, first[1:]):
-        flat += [*range(a, b)] + [0] * (width - (b - a))
-    dev = torch.tensor(flat, dtype=torch.int32).pin_memory().to(device, non_blocking=True)
-    return dev[:2 * len(pages)], len(pages), dev[2 * len(pages):].view(len(q_lens), width)
-
-
-def latent_expand(e_pages, slot_mapping, plan, k_up, v_up, heads: int, dim: int, rot: int, vdim: int, rank: int):
-    """(key pages [pages, heads, 64, dim + rot], value pages [pages, heads, dim + rot, 64]) of a step's prompts from
-    their cached vectors in ``e_pages`` [.., 1, page_size, rank + rot]: keys [k_up e | rotated part], values v_up e and zeros.
-    ``plan``: ``latent_expand_plan``; ``k_up`` [heads * dim, rank], ``v_up`` [heads, vdim, rank]."""
-    pages, n_pages, _ = plan
-    _dev(e_pages, slot_mapping, pages, k_up, v_up)
-    _need(e_pages.dtype == k_up.dtype == v_up.dtype == torch.bfloat16, "latent_expand takes bfloat16")
-    _need(e_pages.dim() == 4 and e_pages.shape[1] == 1 and e_pages.shape[3] == rank + rot, "pages must be [pages, 1, page_size, rank + rot]")
-    _need(k_up.numel() == heads * dim * rank and v_up.numel() == heads * vdim * rank, "k_up and v_up must be one matrix per head")
-    _i32(slot_mapping, "slot_mapping")
-    _i32(pages, "pages", 2 * n_pages)
-    size, d = latent_expand_tokens(), dim + rot
-    k = torch.empty((n_pages, heads, size, d), dtype=torch.bfloat16, device=e_pages.device)
-    v = torch.empty((n_pages, heads, d, size), dtype=torch.bfloat16, device=e_pages.device)
-    _check(library.core().jv_latent_expand_bf16(_ptr(k), _ptr(v), _ptr(e_pages), _ptr(slot_mapping), _ptr(pages), c_int(n_pages), _ptr(k_up),
-                                                _ptr(v_up), c_int(heads), c_int(dim), c_int(rot), c_int(vdim), c_int(rank), _stream()),
-           "latent_expand")
-    return k, v
-
-
-def latent_turn_queries(q, heads: int, dim: int, rot: int, rot_dims: int, cos_sin, interleaved: bool = False) -> None:
-    """q[t, h, dim : dim + rot_dims] turn in place, for bfloat16 rows that begin with heads * (dim + rot) columns."""
-    _dev(q, cos_sin)
-    _need(q.dtype == torch.bfloat16 and q.dim() == 2 and q.shape[1] >= heads * (dim + rot), "q rows must begin with heads * (dim + rot) columns")
-    _f32(cos_sin, "cos_sin", q.shape[0] * rot_dims)
-    _check(library.core().jv_latent_turn_queries_bf16(_ptr(q), c_longlong(q.shape[1]), c_int(q.shape[0]), c_int(heads), c_int(dim), c_int(rot),
-                                                      c_int(rot_dims), _ptr(cos_sin), c_int(1 if interleaved else 0), _stream()),
-           "latent_turn_queries")
-
-
-def latent_cut_heads(att, heads: int, vdim: int, d: int, gate=None) -> torch.Tensor:
-    """[n, heads * vdim]: the first ``vdim`` of every head's ``d`` columns of ``att``, times sigmoid(gate): ``gate`` a [n, heads * vdim]
-    or [n, heads] view with unit column stride, or None."""
-    _dev(att)
-    n = att.shape[0]
-    _need(att.dtype == torch.bfloat16 and att.shape == (n, heads * d), "att must be bfloat16 [n, heads * d]")
-    if gate is not None:
-        _need(gate.is_cuda and gate.dtype == att.dtype and gate.shape in ((n, heads * vdim), (n, heads)) and gate.stride(1) == 1,
-              "gate must be a [n, heads * vdim] or [n, heads] view with unit column stride")
-    o = torch.empty((n, heads * vdim), dtype=att.dtype, device=att.device)
-    gn = 0 if gate is None else gate.shape[1] // heads
-    _check(library.core().jv_latent_cut_heads_bf16(_ptr(o), _ptr(att), c_longlong(n), c_int(heads), c_int(vdim), c_int(d), _ptr(gate),
-                                                   c_longlong(0 if gate is None else gate.stride(0)), c_int(gn), _stream()),
-           "latent_cut_heads")
-    return o
-
-
 def head_linear(y, y_head_stride: int, x, x_head_stride: int, w, gate=None, matrix_cores: "bool | None" = None) -> None:
     """One matrix per head: y[t, h * ys : h * ys + N] = w[h] @ x[t, h * xs : h * xs + K], w [heads, N, K];
     with ``gate`` (a [n, heads * N] view with unit column stride) the result is multiplied by sigmoid(gate); a gate

@@ -13,9 +13,8 @@ Since q_plain . (W_uk[h] c) = (W_uk[h]^T q_plain) . c and sum_j p_j W_uv[h] c_j 
 the cached vector e = [c | k_rot] serves as key AND value of one shared kv head of size rank + rot: the
 paged attention kernels of grouped-query attention run unchanged (one kv head, ``heads`` q heads), on a
 query [W_uk[h]^T q_plain | q_rot], and W_uv[h] is applied to the first ``rank`` elements of their result.
-The same arithmetic serves prompts and decoded tokens, so logits do not depend on how a prompt is cut; except that in bfloat16 the
-heads' keys and values are written out (rounded to bfloat16) for prompts that begin their requests, where a (query, key) pair
-then costs a head dim + rot products in place of rank + rot.  The cache keeps e in the two layouts those kernels read (``parts.spec.kv_cache_spec``).
+The same arithmetic serves prompts and decoded tokens, so logits do not depend on how a prompt is cut.
+The cache keeps e in the two layouts those kernels read (``parts.spec.kv_cache_spec``).
 
 Options: ``q_rank`` 0: the queries are projected directly, q = W_q h (no query latent, no query norm);
 the rotation may pair (i, i + dims/2) or (2i, 2i + 1), as its position part says; ``sinks``: a learned number
@@ -27,7 +26,6 @@ back furthest needs).
 """
 from __future__ import annotations
 
-from types import SimpleNamespace
 from typing import Optional
 
 import torch
@@ -116,7 +114,6 @@ class LatentAttention:
         self.kv_norm = tensors["kv_norm.weight"] if self.own_cache else None
         self.w_q_up = tensors["q_up.weight"] if self.q_rank else None
         self.sinks = tensors["sinks"].contiguous() if self.has_sinks else None
-        self.w_k_up = tensors["k_up.weight"].contiguous()      # [H * dim, rank], for prompts
         self.w_k_up_t = tensors["k_up.weight"].view(H, self.dim, self.rank).transpose(1, 2).contiguous()   # [H, rank, dim]
         self.w_v_up = tensors["v_up.weight"].view(H, self.vdim, self.rank).contiguous()
         self.w_o = tensors["o_proj.weight"]
@@ -138,9 +135,6 @@ class LatentAttention:
         elif self.q_rank:
             cq = K.latent_prepare(proj, self.q_rank, 0, 0, 0, self.q_norm, None, self.eps, None, None, None, None, ctx.page_size)
         q = K.linear(cq, self.w_q_up) if self.q_rank else proj       # proj's rows begin with the queries
-        gate = proj[:, self.gate_at:self.gate_at + self.gate_width] if self.output_gate else None
-        if self._written_out(x, ctx):
-            return K.linear(self._prompts(q, gate, cos_sin, ctx, mem), self.w_o, partial_ok=True)
         qe = torch.empty((n, H * E), dtype=x.dtype, device=x.device)
         K.head_linear(qe, E, q, self.dim + self.rot, self.w_k_up_t)             # W_uk[h]^T q_plain
         if self.rot:
@@ -150,33 +144,9 @@ class LatentAttention:
 
         attention_backend.run(self, att, qe, ctx, mem)
         o = torch.empty((n, H * self.vdim), dtype=x.dtype, device=x.device)
+        gate = proj[:, self.gate_at:self.gate_at + self.gate_width] if self.output_gate else None
         K.head_linear(o, self.vdim, att, E, self.w_v_up, gate=gate)
         return K.linear(o, self.w_o, partial_ok=True)
-
-    def _written_out(self, x, ctx: StepContext) -> bool:
-        """Whether the step's heads get keys and values of their own: its tokens are all that its requests see, and enough of them."""
-        return (not ctx.captured and self.own_cache and x.shape[0] >= K.LATENT_EXPAND_MIN_TOKENS and not any(ctx.context_lens_host)
-                and K.latent_expand_possible(self.dtype, self.dim, self.rot, self.vdim, self.rank))
-
-    def _prompts(self, q, gate, cos_sin, ctx: StepContext, mem: LayerMemory) -> torch.Tensor:
-        """Attention of prompts over keys and values of every head, written out for this call."""
-        from . import attention_backend
-
-        H, d = self.heads, self.dim + self.rot
-        plan = ctx.plans.get("latent_expand")
-        if plan is None:
-            plan = ctx.plans["latent_expand"] = K.latent_expand_plan(ctx.q_lens_host, q.device)
-        k, v = K.latent_expand(mem.pages["k"], ctx.slot_mappings[mem.group], plan, self.w_k_up, self.w_v_up, H, self.dim, self.rot,
-                               self.vdim, self.rank)
-        if self.rot_dims:
-            K.latent_turn_queries(q, H, self.dim, self.rot, self.rot_dims, cos_sin, self.interleaved)
-        att = torch.empty((q.shape[0], H * d), dtype=q.dtype, device=q.device)
-        heads = SimpleNamespace(nq=H, nkv=H, d=d, q_row_stride=q.shape[1], scale=self.scale, window=self.window, sinks=self.sinks)
-        step = SimpleNamespace(block_tables=[plan[2]], cu_seqlens=ctx.cu_seqlens, context_lens=ctx.context_lens,
-                               page_size=K.latent_expand_tokens(),
-                               q_lens_host=ctx.q_lens_host, context_lens_host=ctx.context_lens_host, plans=ctx.plans)
-        attention_backend.run(heads, att, q, step, SimpleNamespace(pages={"k": k, "v": v}, group=0))
-        return K.latent_cut_heads(att, H, self.vdim, d, gate)
 
 
 register_part("mixer", "latent_attention", LatentAttention)
