@@ -1,4 +1,4 @@
-// C[M,N] = A[M,K] * W[N,K]^T in 32 bits: float inputs, float sums, on the bf16 matrix unit without losing a bit of the inputs.
+// C[M,N] = A[M,K] * W[N,K]^T in 32 bits: float inputs that are kept whole, float sums, on the bf16 matrix unit.
 //
 // A float is the sum of three bf16 numbers (8 bits each: the nearest bf16, the nearest to what that leaves, the rest).  Of the
 // nine products of two such sums the six largest are taken; the others are below 2^-26 of the whole.  The bf16 unit makes 13
@@ -10,12 +10,15 @@
 // it.  Error against 64 bits over normal, positive and wide (e^3N) inputs, K 32 to 4,096: 0.4 to 0.8 of that of one 32-bit
 // matrix product after another (relative 2-norm at 1,003 x 2,048 x 2,048 1.3e-7, before 2.9e-7).
 //
-// A sum that is not finite may come from the split (a value above the largest bf16, infinity less itself): it is made again
-// from the numbers themselves.  Numbers below 2^-110 lose their last terms to the range of bf16.
+// The third term of a small number would be below bf16's range (from 2^-110 on, down to 8 bits at 2^-126), so both operands are
+// multiplied by 2^24 first, which changes no bit of a float, and the sums by 2^-48: the terms of every float, the smallest
+// one among them, are then whole.  A sum that is not finite may come from the split (2^80 of the true sum, a value near the
+// largest float, infinity less itself): it is made again from the numbers themselves.
 //
-// Microseconds, before with the 32-bit instruction: 5 rows against 2,048 x 2,048 10.9 -> 8.8, 6,144 x 2,048 16.4 -> 13.3 (50 MB:
-// the stream of W); 16 rows 13.5 -> 9.1, 18.5 -> 13.4; 300 x 6,144 x 2,048 121 -> 75; 1,003 x 6,144 x 2,048 226 -> 150 with the 5 that the terms
-// of A take; 2,048 x 24,576 x 4,096 3,430 -> 2,222 = 186 TFLOP/s of 32-bit products, 1.1 PFLOP/s of the matrix unit's.
+// Microseconds, before with the 32-bit instruction: 5 rows against 2,048 x 2,048 10.9 -> 9.2, 6,144 x 2,048 16.4 -> 13.8 (50 MB:
+// the stream of W); 16 rows 13.5 -> 9.3, 18.5 -> 13.9; 300 x 6,144 x 2,048 121 -> 78; 1,003 x 6,144 x 2,048 226 -> 154 with the 5 that the terms
+// of A take; 2,048 x 24,576 x 4,096 3,430 -> 2,250 = 183 TFLOP/s of 32-bit products, 1.1 PFLOP/s of the matrix unit's.  The scaling is 1 to 5 %
+// of these (in turn, without / with: 5 x 2,048 x 2,048 9.1 / 9.5, 250 x 6,144 x 2,048 56.5 / 59.6, 1,003 x 6,144 x 2,048 165 / 169).
 #include "common.h"
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -27,8 +30,12 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 #define G32_STEP 32            // columns of a step and of v_mfma_f32_16x16x32_bf16
 
-// Pair i of a lane's 8 numbers: its part of the three terms.
+#define G32_SCALE 0x1p24f
+#define G32_UNSCALE 0x1p-48f
+
+// Pair i of a lane's 8 numbers: its part of the three terms of 2^24 times these.
 __device__ __forceinline__ void split_pair(float a, float b, int i, u32x4 (&t)[3]) {
+  a *= G32_SCALE, b *= G32_SCALE;
 #pragma unroll
   for (int e = 0; e < 3; ++e) {
     t[e][i] = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){a, b}, bf16x2));
@@ -48,8 +55,11 @@ __device__ constexpr int G32_W[G32_PRODUCTS] = {0, 1, 2, 0, 1, 0}, G32_X[G32_PRO
 __device__ __forceinline__ f32x4 mfma(const u32x4& w, const u32x4& x, const f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, x), c, 0, 0, 0);
 }
+// The result of a sum of scaled products, or of the numbers themselves where that left the range of float.
 __device__ __forceinline__ float settle(float sum, const float* a, const float* w, int K) {
-  if (!(__builtin_fabsf(sum) <= 3.402823466e38f)) {
+  const bool held = __builtin_fabsf(sum) <= 3.402823466e38f;
+  sum *= G32_UNSCALE;
+  if (!held) {
     sum = 0.f;
     int k = 0;
     for (; k + 8 <= K && sum == sum; k += 8) {      // a NaN stays one
@@ -234,7 +244,7 @@ split_rows_kernel(unsigned* __restrict__ y, const float* __restrict__ A, int K, 
 
 // Tiles of TM rows of A (as terms) by TW rows of W (as floats); two groups of 2 x 2 waves take a half of the steps each, through
 // rings of S steps in LDS.  Bound by what a SIMD issues: a product of 16 cycles takes 8 of them, a vector instruction 2 to 4
-// (measured), so a wave splits the next 16 rows of W (44 instructions) while it multiplies these with all its rows of A.
+// (measured), so a wave splits the next 16 rows of W (52 instructions) while it multiplies these with all its rows of A.
 template <int TM, int TW>
 __global__ void __launch_bounds__(512, 2)
 gemm_f32_tile_kernel(float* __restrict__ C, const unsigned* __restrict__ X, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K, int KA) {
@@ -381,7 +391,7 @@ gemm_f32_tile_kernel(float* __restrict__ C, const unsigned* __restrict__ X, cons
       bool ok = pieces && n + 4 <= N;
 #pragma unroll
       for (int e = 0; e < 4; ++e) ok = ok && __builtin_fabsf(v[e]) <= 3.402823466e38f;
-      if (ok) *(f32x4*)(C + (long long)m * N + n) = v;
+      if (ok) *(f32x4*)(C + (long long)m * N + n) = v * G32_UNSCALE;
       else
         for (int e = 0; e < 4; ++e)
           if (n + e < N) C[(long long)m * N + n + e] = settle(v[e], A + (long long)m * KA, W + (long long)(n + e) * K, KA);

@@ -70,6 +70,27 @@ def test_values_that_the_split_does_not_hold(k):
         assert ((out - want).abs()[fine] <= (2.0 ** -24 * k * (a.double().abs() @ w.double().abs().T))[fine]).all()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("ea,ew", [(-112, 0), (0, -118), (-126, 90), (80, -140), (-140, 20), (-60, -75), (100, -140), (30, 49)])
+def test_numbers_at_the_ends_of_the_range_keep_their_bits(ea, ew):
+    """Operands around 2^ea and 2^ew, subnormal ones among them, beside ones 2^20 larger and zeros: as exact as ordinary numbers, and a
+    result below the smallest normal float within half a unit of its last place."""
+    k = 160
+    a, w = (randn(40, k, seed=1).double() * 2.0 ** ea).float(), (randn(70, k, seed=2).double() * 2.0 ** ew).float()
+    a[:, ::7] *= 2.0 ** 20
+    a[:, ::5], w[:, 1::9], a[11] = 0.0, 0.0, 0.0
+    want = a.double() @ w.double().T
+    outs = [product(form, a, w) for form in FORMS]
+    assert (want.abs() > 2.0 ** -149).sum() > 1000      # something is left of them
+    if ea > 80 or ea + ew > 50:      # beyond what the scaled split holds: one chain of k terms
+        near = 2.0 ** -24 * k * (a.double().abs() @ w.double().abs().T)
+    else:
+        near = bound(a, w)
+    assert ((outs[0].double() - want).abs() <= near + 2.0 ** -149).all()
+    for form, out in zip(FORMS, outs):
+        assert torch.equal(out, outs[0]), form
+
+
 def test_every_size_has_a_form():
     from jax_vllm_amd.ops.kernels import KernelArgumentError, f32_plan
 
