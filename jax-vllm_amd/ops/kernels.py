@@ -972,8 +972,9 @@ def streaming_plan(m: int, n: int, k: int, gate_pairs: bool = False, partial_ok:
       - up to 32 rows against wide matrices with an inner size of 12 or 16 pieces a wave: staying blocks with two row tiles of x
         in registers and W in four slots (24,576 x 4,096 with the activation at 24 rows 44.7 us against 47.5 by the library and
         the activation kernel; the ring takes 41.8);
-    * one or two rows against very wide matrices (the output embedding): x resident in LDS (chosen
-      inside the kernel library; 1.24 GB in 202 us against 205);
+    * one or two rows against very wide matrices (the output embedding), where ``few_tile`` leaves them (one row, inner
+      sizes of 3,584 to 4,096; any that are no multiple of 64): x resident in LDS (chosen inside the kernel library; 1.24 GB
+      in 200 us against 205);
     * 9..16 rows of a large matrix that fits none of these: the library (its wider tiles amortise
       x), unless the inner size is beyond 12,288, where the library needs 113 us for the 178 MB
       that x resident in LDS streams in 45;
@@ -1115,8 +1116,13 @@ FEW_MAX_INNER = 4096      # eight waves of eight chunks of 64 columns, x in regi
 def few_tile(m: int, n: int, k: int, cus: int = 256) -> "int | None":
     """Rows of w of a block of ``gemm_few`` (16 or 32) where it can take the product, else None: 32 where 16 would give a unit more than
     one block and most units only one (4,608 x 3,072 9.3 us against 10.5, 6,144 x 2,048 at 8 rows 9.1 / 9.4, at one row 8.7 / 8.4; 4,096 x
-    2,048 6.8 / 5.9, 8,192 x 2,048 10.0 / 9.1, 11,296 x 2,048 12.6 / 12.0)."""
+    2,048 6.8 / 5.9, 8,192 x 2,048 10.0 / 9.1, 11,296 x 2,048 12.6 / 12.0).
+    One row against the output embedding stays with x resident in LDS where its 4,096 columns are nearly filled: us here / resident, 151,936
+    rows of W: k = 4,096 204.6 / 200.4, 3,840 191.4 / 190.4, 3,584 180.3 / 178.5, 3,328 167.5 / 174.4, 2,048 104 / 154; two rows 205.4 / 205.0,
+    193.5 / 203.8, 183.2 / 193.4; 65,536 x 4,096 91.2 / 88.0, two rows 92.3 / 93.9; 16,000 x 4,096 25.3 / 25.0."""
     if not 0 < m <= SKINNY_AUTO_ROWS or k % 64 or not 64 <= k <= FEW_MAX_INNER or n % 4:
+        return None
+    if m == 1 and n >= 65536 and k >= 3584:
         return None
     return 32 if cus < -(-n // 16) <= 1.5 * cus else 16
 

@@ -69,3 +69,11 @@ def test_rows_without_their_scale_are_refused(monkeypatch, m, n, k, partial_ok):
     assert not kernels.linear_takes_unscaled_rows(m, w, partial_ok=partial_ok)
     with pytest.raises(kernels.KernelArgumentError, match="un-normalised rows"):
         kernels.linear(rows, w, partial_ok=partial_ok)
+
+
+def test_one_row_against_the_output_embedding_stays_with_x_resident():
+    from jax_vllm_amd.ops.kernels import STAGED, few_tile, streaming_plan
+
+    assert streaming_plan(1, 151936, 4096) == streaming_plan(2, 151936, 4096) == STAGED      # the kernel library's choice: x resident
+    assert [few_tile(m, n, k) for m, n, k in ((1, 151936, 4096), (1, 65536, 3584), (2, 151936, 4096), (1, 151936, 3328), (1, 151936, 2048), (1, 16000, 4096))] \
+        == [None, None, 16, 16, 16, 16]
