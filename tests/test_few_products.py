@@ -77,3 +77,10 @@ def test_one_row_against_the_output_embedding_stays_with_x_resident():
     assert streaming_plan(1, 151936, 4096) == streaming_plan(2, 151936, 4096) == STAGED      # the kernel library's choice: x resident
     assert [few_tile(m, n, k) for m, n, k in ((1, 151936, 4096), (1, 65536, 3584), (2, 151936, 4096), (1, 151936, 3328), (1, 151936, 2048), (1, 16000, 4096))] \
         == [None, None, 16, 16, 16, 16]
+
+
+def test_rows_of_w_of_a_block_where_the_library_was():
+    from jax_vllm_amd.ops.kernels import few_tile, streaming_plan
+
+    sizes = ((16, 15360, 4096), (9, 12304, 1536), (16, 12288, 4096), (8, 15360, 4096), (16, 15360, 1024))
+    assert streaming_plan(16, 15360, 4096) is None and [few_tile(*s) for s in sizes] == [32, 32, 16, 16, 16]
