@@ -5,13 +5,16 @@
 // block waits for in a row costs one more.  So a block takes TW rows of W against all rows of x and its 8 waves an eighth of the
 // inner size each; a wave asks for its part of x (into registers, where it stays) and for the first S chunks of its part of W
 // (straight into a ring of its own in LDS) in one go, and no wave waits for another before the parts meet at the end.  Two blocks
-// of 80 KB share a unit, and TW is such that all blocks are on the chip at once: the units then need not carry equal loads, for
-// what they share is the memory.  The parts are added in ascending order, so a row's result does not depend on the others.
+// with rings of up to 64 KB share a unit; up to 512 blocks are on the chip at once, and their units need not carry equal loads, for
+// what they share is the memory.  TW follows from where more are a further round (few_tile, with the figures).  The parts are added
+// in ascending order, so a row's result does not depend on the others.
 //
 // Microseconds in a graph, cold weights, at 1, 8 and 16 rows (before, x staged chunk by chunk in LDS for all waves of a block):
 // 6,144 x 2,048 with its activation 8.7, 9.1, 9.0 (9.8, 11.2, 11.8), 11,296 x 2,048 12.0, 12.5, 14.0 (17.3, 15.3, 17.3),
 // 2,048 x 2,048 4.0, 4.7, 5.4 (5.5, 6.2, 7.1), 1,536 x 768 2.9, 3.2, 3.4 (4.6, 5.0, 6.2), 3,072 x 4,096 7.9, 8.6, 10.1 (9.4, 10.4, 13.2).
-// Blocks that stay are better from about 16,384 rows of W on (24,576 x 2,048 at 16 rows 22.5, here 26.3).
+// Blocks that stay are better from about 16,384 rows of W on (24,576 x 2,048 at 16 rows 22.5, here 26.3); one and two rows against the
+// output embedding, which those do not take, run here in many rounds (151,936 x 2,048 104 us, x resident in LDS 154; 151,936 x 4,096 at two
+// rows 205.4, resident 205.0, staying 208).
 #include "common.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -128,7 +131,6 @@ static int few_launch(void* y, const void* x, const void* W, int M, int N, int K
 #undef FEW
   return (int)hipErrorInvalidValue;
 }
-extern "C" int jv_gemm_few_max_inner() { return 8 * FEW_WAVES * FEW_K; }
 // mode: FEW_*; tw (16, 32): rows of W of a block.
 extern "C" int jv_gemm_few_bf16(void* y, const void* x, const void* W, int M, int N, int K, long long ldx, int mode, int gate_act,
                                 float act_limit, float act_slope, int tw, void* stream) {
