@@ -35,12 +35,23 @@ def test_rows_that_are_not_finite_stay_alone():
 
 
 @pytest.mark.gpu
-def test_operands_the_form_does_not_take_go_the_old_way():
+def test_operands_the_form_does_not_take_go_the_old_way(monkeypatch):
     x, w = randn(6, 2048, seed=1).bfloat16(), randn(2048, 2048, seed=2).bfloat16()
-    want = K().linear(x, w)
-    flat = torch.empty(6 * 2048 + 1, dtype=torch.bfloat16, device="cuda")
-    off = flat[1:].view(6, 2048).copy_(x)
-    torch.testing.assert_close(K().linear(off.clone(), w), want)
+    off = [torch.empty(t.numel() + 4, dtype=torch.bfloat16, device="cuda")[4:].view(t.shape).copy_(t) for t in (x, w)]
+    assert all(t.data_ptr() % 16 == 8 and t.is_contiguous() for t in off)      # 8 bytes off
+
+    def taken(*_, **__):
+        raise AssertionError("operands that the form does not take")
+
+    want = x.double() @ w.double().T
+    with monkeypatch.context() as patch:
+        patch.setattr(K(), "gemm_few", taken)
+        for operands in ((off[0], w), (x, off[1])):
+            y = K().linear(*operands)
+            # a rounding to bfloat16 of a float sum of 2,048 products
+            assert ((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -24 * 2048 * (x.double().abs() @ w.double().abs().T)).all()
+        with pytest.raises(AssertionError, match="does not take"):
+            K().linear(x, w)      # (aligned: it would be)
     assert K().few_tile(6, 2048, 2040) is None and K().few_tile(6, 2048, 4160) is None and K().few_tile(17, 2048, 2048) is None
     torch.testing.assert_close(K().linear(x[:, :2040].contiguous(), w[:, :2040].contiguous()).double(),
                                x[:, :2040].double() @ w[:, :2040].double().T, rtol=2.0 ** -7, atol=0.05)
