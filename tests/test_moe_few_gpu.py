@@ -8,7 +8,7 @@ from .test_kernels_gpu import K
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("hidden,ff", [(64, 64), (448, 576), (704, 1024), (1088, 320), (2112, 132), (4096, 192), (40, 72), (4160, 64)])
+@pytest.mark.parametrize("hidden,ff", [(64, 64), (448, 576), (704, 1024), (1088, 320), (2112, 136), (4096, 192), (40, 72), (4160, 64)])
 @pytest.mark.parametrize("gated,on_input", [(True, True), (True, False), (False, False)])
 def test_few_rows_an_expert(hidden, ff, gated, on_input):
     rows = [1, 0, 16, 17, 3]
@@ -20,8 +20,6 @@ def test_few_rows_an_expert(hidden, ff, gated, on_input):
     expert = torch.cat([torch.full((r,), e) for e, r in enumerate(rows)])[torch.randperm(n, generator=g)]
     logits = torch.full((n, experts), -4.0)
     logits[torch.arange(n), expert] = 1.0
-    if hidden % 8 or ff % 8:
-        pytest.skip("no form for these sizes")
     plan = K().moe_route(logits.cuda(), 1, tile_rows=16)
     out = torch.full((1, n, hidden), float("nan"), device="cuda")
     K().moe_experts(x.cuda(), plan, wg.cuda() if gated else None, wu.cuda(), wd.cuda(), "silu", out, weight_on_input=on_input)
