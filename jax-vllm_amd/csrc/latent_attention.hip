@@ -259,7 +259,9 @@ head_linear_mfma_kernel(bf16_t* __restrict__ y, long long ldy, int ys, const bf1
 // More rows than a block of those takes: a wave has 16 rows and 64 outputs, so an operand of x serves four products, and the
 // results go through LDS into whole lines of y (2 bytes at a time the stores took longer than the rest).  The sums keep the order
 // of the kernel above.  16 heads, 64 into 224 and 224 into 64, microseconds (before): 2,048 rows 16.6 (25.7) and 10.0 (21.4), 600 rows 7.4
-// (10.5) and 5.9 (8.6); 250 rows 4.1 (5.4) and 5.8 (4.5), where the second stays with the kernel above.
+// (10.5) and 5.9 (8.6); 250 rows 4.1 (5.4) and 5.8 (4.5), where the second stays with the kernel above.  From 480,000 results on it
+// was faster at 16 sizes (2 to 64 heads, 32 to 512 outputs, inner sizes 32 to 512, 80 to 2,048 rows: 0.33 to 0.97 of the time) but for 130
+// rows of 8 heads, 128 into 512, 5.0 (4.7) and 300 of 64 heads, 128 into 32, 7.6 (7.5); at 260,000 it still takes up to 1.3 times as long.
 #define HL_N 64
 __global__ void __launch_bounds__(256)
 head_linear_lines_kernel(bf16_t* __restrict__ y, long long ldy, int ys, const bf16_t* __restrict__ x, long long ldx,

@@ -416,6 +416,41 @@ def test_one_matrix_per_head(dtype, n, heads, N, K):
         assert float(got[..., N:].abs().max()) == 0.0           # nothing is written between the heads
 
 
+@pytest.mark.parametrize("n,heads,N,K", [(601, 5, 200, 72), (1003, 16, 36, 136), (80, 40, 152, 24), (130, 64, 64, 224)])
+@pytest.mark.parametrize("gate,gate_off", [(None, 0), ("element", 8), ("element", 5), ("head", 3)])
+@pytest.mark.parametrize("extra", [3, 4, 8])
+def test_one_matrix_per_head_in_whole_lines(n, heads, N, K, gate, gate_off, extra):
+    """The per-head product of many rows, whose results leave through LDS: outputs that are no multiple of 64, inner sizes that are no
+    multiple of 32, last rows that do not fill a wave, results and gates off 16 bytes; the same sums as from few rows."""
+    from jax_vllm_amd.ops import kernels as K_
+
+    assert n >= 80 and n * N * heads >= 480000      # the form of many rows; up to 79 the other one
+    g = torch.Generator().manual_seed(n + N)
+    xs, ys = K + 8, N + extra
+    x = torch.randn(n, heads * xs, generator=g).bfloat16().cuda()
+    w = (torch.randn(heads, N, K, generator=g) * K ** -0.5).bfloat16().cuda()
+    width = {"element": heads * N, "head": heads, None: 0}[gate]
+    wide = torch.randn(n, width + 16, generator=g).bfloat16().cuda()
+    gv = wide[:, gate_off:gate_off + width] if gate else None
+
+    def run(a, b):
+        y = torch.zeros(b - a, heads * ys, dtype=torch.bfloat16, device="cuda")
+        K_.head_linear(y, ys, x[a:b], xs, w, gate=gv[a:b] if gate else None)
+        return y
+
+    y = run(0, n)
+    got = y.double().view(n, heads, ys)
+    assert float(got[..., N:].abs().max()) == 0.0           # nothing is written between the heads
+    exact = torch.stack([x.double().view(n, heads, xs)[:, h, :K] @ w[h].double().T for h in range(heads)], 1)
+    size = torch.stack([x.double().view(n, heads, xs)[:, h, :K].abs() @ w[h].double().abs().T for h in range(heads)], 1)
+    if gate:
+        exact = exact * torch.sigmoid(gv.double()).view(n, heads, -1)
+    # a rounding to bfloat16 of a float sum of K products (times a float sigmoid)
+    assert ((got[..., :N] - exact).abs() <= 2.0 ** -8 * exact.abs() + (K + 8) * 2.0 ** -24 * size).all()
+    if not gate:
+        assert torch.equal(y, torch.cat([run(a, min(a + 79, n)) for a in range(0, n, 79)]))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_odd_width_and_a_cached_vector_above_256(tmp_path, dtype):
     """A width that is no multiple of 4 (no kernel may take its 16-byte path), a cached vector of 288 elements
