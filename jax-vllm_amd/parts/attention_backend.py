@@ -47,7 +47,10 @@ def keys_seen(kv_len: int, window: int, keep: int = 0) -> int:
 def decode_splits(n_decode: int, blocks_per_request: int, max_kv_len: int) -> int:
     """Blocks that share out a request's keys: as many as give no unit a second block (one more costs a further merge and leaves
     units with twice the load of others: 12 requests of 500 to 1,500 keys over 8 kv heads 18.9 us with 2, 22.2 with 3; 24 of 450 to 1,350
-    24.7 with 1, 29.6 with 2; 9 of 500 to 1,500 15.4 with 3, 19.3 with 4)."""
+    24.7 with 1, 29.6 with 2; 9 of 500 to 1,500 15.4 with 3, 19.3 with 4).  So also at long contexts, where a merge weighs little (8 kv
+    heads, even keys, 1 / 2 splits: 17 requests of 256 keys 10.0 / 14.2, 2,600 40.8 / 50.5, 7,800 111 / 131; 20 of 3,850 61.0 / 71.4; 24 68.0 / 76.0;
+    28 78.6 / 81.4; 31 86.8 / 88.8; spread over half to one and a half of that the same but for less).  Open: 3 splits at 17 to 20
+    requests of 1,600 spread keys or more (17 of 3,850 60.9, with one 68.3)."""
     base = max(1, n_decode * blocks_per_request)
     by_fill = max(1, TARGET_BLOCKS // base)
     by_len = max(1, max_kv_len // MIN_KEYS_PER_SPLIT)

@@ -73,6 +73,13 @@ def test_decode_splits_fill_the_chip_but_keep_a_tile_per_wave():
     assert decode_splits(64, 8, 8192) == 1                   # enough blocks already
 
 
+def test_decode_splits_give_no_unit_a_second_block():
+    """Measured between 256 and 7,800 keys: with 17 to 31 requests of 8 kv heads one split, however long they are."""
+    for n in (17, 20, 24, 31):
+        assert decode_splits(n, 8, 300) == decode_splits(n, 8, 8192) == 1
+    assert [decode_splits(n, 8, 8192) for n in (5, 6, 7, 9, 11, 16)] == [6, 5, 4, 3, 2, 2]
+
+
 def test_item_shape_follows_the_fill_of_the_chip():
     """Few rows: items of one group, so that more blocks than compute units exist at all; more:
     two groups, light paired with heavy; many: two neighbouring groups."""
