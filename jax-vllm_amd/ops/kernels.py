@@ -751,7 +751,8 @@ _F32_TILES = ((5, 128, 128, 34.0, 45.0), (6, 128, 96, 26.0, 35.0), (7, 128, 64, 
 def f32_plan(m: int, n: int, k: int, pieces: bool = True, a_pieces: bool = True) -> int:
     """Form of the 32-bit product (``jv_gemm_f32``).  All give the same bits, so it is the one that takes the least time by a count of
     rounds over 256 units that meets what was measured (1 to 2,048 rows, n 256 to 32,000, k 512 to 12,288) mostly within a sixth; for example
-    k = 2,048: 5 x 2,048 9.2 us (form 2), 16 x 32,000 53 (3), 37 x 3,072 16 (4), 250 x 6,144 53 (8), 1,003 x 6,144 149 (6), 2,048 x 2,048 103 (5).
+    k = 2,048: 5 x 2,048 8.8 us (form 2), 16 x 32,000 53 (3), 37 x 3,072 15.5 (4), 250 x 6,144 50 (8), 1,003 x 6,144 145 (6), 2,048 x 2,048 101 (5);
+    in graphs with cold weights and operands scaled 9.6, 57, 17.6, 60, 172, 114.
     ``pieces``: rows of w begin on 16 bytes (else they are copied for tiles, and few rows go through registers); ``a_pieces``: rows of a too."""
     q, mb = k / 1024, n * k * 4e-6
 
