@@ -415,7 +415,7 @@ static int tile_launch(float* C, const void* X, const float* A, const float* W, 
   hipLaunchKernelGGL((gemm_f32_tile_kernel<TM, TW>), dim3((unsigned)((live + 7) / 8 * 8)), dim3(512), 0, s, C, (const unsigned*)X, A, W, M, N, K, KA);
   return JV_LAUNCH_CHECK();
 }
-// Rows of A [M][KA] as terms, [M][steps][3][32] bf16 with zeros behind KA; steps = ceil(KA / 32).
+// Rows of A [M][KA] as terms (of 2^24 times A), [M][steps][3][32] bf16 with zeros behind KA; steps = ceil(KA / 32).
 extern "C" int jv_split_rows_f32(void* X, const float* A, int M, int KA, void* stream) {
   if (M <= 0 || KA <= 0) return 0;
   if ((uintptr_t)X & 15) return (int)hipErrorInvalidValue;

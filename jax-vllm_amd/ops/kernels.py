@@ -799,7 +799,7 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, out=None) -> torch.Tensor:
         return out
     pieces = not k & 3 and not w.data_ptr() & 15
     form, lib, terms, kw = f32_plan(m, n, k, pieces, not a.data_ptr() & 15), library.core(), None, k
-    if form >= 5:      # the rows of a as sums of three bfloat16 numbers, [M, steps, 3, 32]
+    if form >= 5:      # the rows of a, scaled, as sums of three bfloat16 numbers, [M, steps, 3, 32]
         steps = -(-k // F32_STEP)
         terms = torch.empty((m, steps, 3, F32_STEP), dtype=torch.bfloat16, device=a.device)
         _check(lib.jv_split_rows_f32(_ptr(terms), _ptr(a), c_int(m), c_int(k), _stream()), "split_rows_f32")
