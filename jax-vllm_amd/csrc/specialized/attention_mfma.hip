@@ -104,6 +104,17 @@ struct AttnArgs {
   int num_splits;
   float* part_acc;            // [n_work, nq, num_splits, D]
   float* part_ml;             // [n_work, nq, num_splits, 2] (max, sum)
+  // decode from the q/k/v product (DEC_PARTS, DEC_ROWS) only: its columns are the q heads, the k heads, the v heads
+  const float* parts;         // DEC_PARTS: [n_parts][tokens][(nq + 2 nkv) * D], n_parts <= 4, part_stride floats apart
+  long long part_stride;
+  int n_parts, rotary_dim;
+  const float* q_weight;      // per-head norms, or null
+  const float* k_weight;
+  float norm_eps;
+  const float* cos_sin;       // [tokens, rotary_dim], or null
+  const int* slot_mapping;    // [tokens] page * page_size + slot of the token's key, or negative: not stored
+  bf16_t* k_pages_out;
+  bf16_t* v_pages_out;
 };
 
 // ------------------------------------------------------------------------------------ prefill
@@ -1180,9 +1191,29 @@ extern "C" int jv_attn_prefill_waves_split() { return 0; }
 constexpr int BND = 32;  // keys per wave iteration
 constexpr int DEC_TBL_MAX = 4096;  // page-table entries of a request that a decode block keeps in LDS
 
-template <bool MORE>
-__global__ void __launch_bounds__(256) PREFILL_OCCUPANCY attn_decode_kernel(AttnArgs p) {
-  extern __shared__ float smem[];  // per wave: m[16], l[16], acc[16][D]
+// Where a decode block's queries come from.  A step of single tokens at head size 128 goes from the q/k/v product to its attention
+// in one launch: norm, rotation and page writes are a launch and a chain of round trips of their own (2.3 to 5 us a layer) that the blocks'
+// wait for the page table and the keys hides.  Both launches and now, microseconds with the merge (8 kv heads of 4 q heads, the same
+// splits): one request of 1,024 keys 11.5 and 10.2, 8 of 1,030 16.9 and 14.8, 8 of 7,900 59.6 and 57.7, 64 of 512 to 1,536 64.2 and 61.8, 64 of 200
+// 19.1 and 16.3.  The new key does not go through its page: its score is a dot product of its own and it joins the waves' sums.
+enum {
+  DEC_READY = 0,    // q rows in bf16, normed and rotated; the step's keys and values are in their pages
+  DEC_PARTS = 1,    // the q/k/v product as float partial products: the block adds, norms and rotates its heads itself, and one block
+                    // of every (request, kv head) writes the new key and value to their pages
+  DEC_ROWS = 2      // the same from bf16 rows
+};
+#if JV_HEAD_DIM == 128
+#define JV_DECODE_FUSED 1    // a wave holds elements l, l + 64 of a head: both numbers of a rotation's pair in one lane
+#endif
+constexpr int DEC_WAVES = 4;                // (8, each side with its best number of splits: 0.97 to 1.32 of the time over 54 steps, 1.02 on average)
+constexpr int DEC_STRIDE = D + 4;          // floats of a row of a wave's sums in LDS (16 rows' pieces on different banks)
+constexpr int QN_STRIDE = D + 8;           // bf16 elements of a prepared head in LDS
+constexpr int DEC_NEW_BYTES = 16 * QN_STRIDE * 2 + D * 2 + D * 4 + 16 * 4;      // prepared q heads, the new key, value and scores
+
+template <bool MORE, int INPUT>
+__global__ void __launch_bounds__(64 * DEC_WAVES) PREFILL_OCCUPANCY attn_decode_kernel(AttnArgs p) {
+  extern __shared__ __attribute__((aligned(16))) float smem[];  // per wave: m[16], l[16], acc[rows][DEC_STRIDE]
+  constexpr int WAVES = DEC_WAVES, THREADS = 64 * WAVES;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int li = lane & 15, lc = lane >> 4;
   const int G = p.nq / p.nkv, P = p.page_size;
@@ -1202,25 +1233,133 @@ __global__ void __launch_bounds__(256) PREFILL_OCCUPANCY attn_decode_kernel(Attn
   const int r = p.work ? p.work[w] : w;
   const int g = at / mt_per_head, mt = at - g * mt_per_head;
   const int split = blockIdx.y;
+  const int rows = G - mt * 16 < 16 ? G - mt * 16 : 16;
   const int* gtable = p.block_tables + (long long)r * p.table_stride;
   // A table row beyond DEC_TBL_MAX entries does not fit: the block then copies only the entries of its own
   // split's keys, once it knows them (one more round trip, at contexts where that does not matter; the
   // entry point makes sure that a split's entries fit).  Pages are always looked up in LDS: a lookup in
   // global memory beside it would be a load inside a branch, at whose end the compiler waits for every
   // load in flight, tile after tile.
-  int* tbl = (int*)(smem + 4 * (32 + 16 * D));
+  const int stride_w = 32 + (G < 16 ? G : 16) * DEC_STRIDE;        // floats of a wave's share of smem
+  int* tbl = (int*)(smem + WAVES * stride_w);
   const bool whole_row = p.table_stride <= DEC_TBL_MAX;
   if (whole_row)
-    for (int i = tid; i < p.table_stride; i += 256) tbl[i] = gtable[i];
+    for (int i = tid; i < p.table_stride; i += THREADS) tbl[i] = gtable[i];
   const int tok = p.cu_seqlens ? p.cu_seqlens[r] : r;
-  const int pos = p.context_lens[r];      // the query's position; keys 0..pos are stored
-  const int kv_len = pos + 1;
+  const int pos = p.context_lens[r];      // the query's position
+  // keys 0 .. kv_len - 1 are read from the pages; a key that this launch makes itself joins the sums at the end
+  const int kv_len = INPUT == DEC_READY ? pos + 1 : pos;
   const int kv_begin = first_key(pos, p.window);
+  const bool takes_new = INPUT != DEC_READY && split == p.num_splits - 1;     // this block adds the new key
+
+  // ---- heads of the q/k/v product on their way: wave v prepares rows v, v + WAVES, ... of (the block's q heads, the k head, the v
+  // head); the first PRE of them are asked for here, before the page table is looked at
+  constexpr int E = D < 64 ? 1 : D / 64, PRE = 2;      // (D is 128 where heads are prepared)
+  bf16_t* const q_new = (bf16_t*)(tbl + ((p.table_stride < DEC_TBL_MAX ? p.table_stride : DEC_TBL_MAX) + 3) / 4 * 4);
+  bf16_t* const k_new = q_new + 16 * QN_STRIDE;
+  float* const v_new = (float*)(k_new + D);
+  float* const s_new = v_new + D;
+  const int n_prep = rows + (takes_new ? 2 : 0);
+  struct Head { float v[4][E], w[E]; };
+  Head pre[INPUT == DEC_READY ? 1 : PRE];
+  float cs[E], sn[E];
+  int slot_raw = -1;
+  const int half = p.rotary_dim / 2, HE = half / 64;       // pair (e, e + HE) for e < HE
+  // no load inside a branch: what is not there is read from the block table and not used
+  auto ask = [&](int i, Head& h) {
+    const int ii = i < n_prep ? i : 0;
+    const int head = ii < rows ? g * G + mt * 16 + ii : ii == rows ? p.nq + g : p.nq + p.nkv + g;
+    const long long col = (long long)head * D + lane;
+    if (INPUT == DEC_PARTS) {
+      const float* px = p.parts + (long long)tok * (p.nq + 2 * p.nkv) * D + col;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < E; ++e) h.v[q][e] = px[(q < p.n_parts ? q : 0) * p.part_stride + e * 64];
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; ++e) h.v[0][e] = to_f32(p.q[(long long)tok * p.q_row_stride + col + e * 64]);
+    }
+    const float* w0 = ii < rows ? p.q_weight : p.k_weight;
+    const float* wp = w0 ? w0 + lane : (const float*)p.q;
+#pragma unroll
+    for (int e = 0; e < E; ++e) h.w[e] = wp[w0 ? e * 64 : 0];
+  };
+  auto prepare = [&](int i, Head& h) {
+    float v[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      v[e] = h.v[0][e];
+      if (INPUT == DEC_PARTS) {
+#pragma unroll
+        for (int q = 1; q < 4; ++q)
+          if (q < p.n_parts) v[e] += h.v[q][e];
+      }
+    }
+    const int slot = __builtin_amdgcn_readfirstlane(slot_raw);
+    const bool store = slot >= 0 && mt == 0;
+    const long long page = store ? ps.index(slot) : 0;
+    const int off = store ? ps.slot(slot) : 0;
+    if (i > rows) {                          // the value: to its (transposed) page
+      bf16_t* dst = p.v_pages_out + (page * p.nkv + g) * (long long)D * P + off;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const bf16_t x = from_f32<bf16_t>(v[e]);
+        v_new[e * 64 + lane] = to_f32(x);
+        if (store) dst[(long long)(e * 64 + lane) * P] = x;
+      }
+      return;
+    }
+    if (i < rows ? p.q_weight != nullptr : p.k_weight != nullptr) {
+      float ss = 0.f;
+#pragma unroll
+      for (int e = 0; e < E; ++e) ss += v[e] * v[e];
+      ss = wave_sum(ss);
+      const float inv = rsqrtf(ss / (float)D + p.norm_eps);
+#pragma unroll
+      for (int e = 0; e < E; ++e) v[e] = v[e] * inv * h.w[e];
+    }
+    if (p.cos_sin) {
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        if (e < HE) {
+#pragma unroll
+          for (int f = e + 1; f < E; ++f)
+            if (f == e + HE) {
+              const float a = v[e], b = v[f];
+              v[e] = a * cs[e] - b * sn[e];
+              v[f] = b * cs[e] + a * sn[e];
+            }
+        }
+    }
+    bf16_t* dst = p.k_pages_out + ((page * p.nkv + g) * P + off) * (long long)D;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const bf16_t x = from_f32<bf16_t>(v[e]);
+      (i < rows ? q_new + i * QN_STRIDE : k_new)[e * 64 + lane] = x;
+      if (i == rows && store) dst[e * 64 + lane] = x;
+    }
+  };
+  if constexpr (INPUT != DEC_READY) {
+    // through the vector unit: a scalar load would be waited for before the loads below are even asked for
+    int lane_zero;
+    asm volatile("v_mov_b32 %0, 0" : "=v"(lane_zero));
+    slot_raw = p.slot_mapping[tok + lane_zero];
+    const float* cp = p.cos_sin ? p.cos_sin + (long long)tok * p.rotary_dim + lane : (const float*)p.q;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int ee = e < HE ? e : 0;
+      cs[e] = cp[p.cos_sin ? ee * 64 : 0];
+      sn[e] = cp[p.cos_sin ? half + ee * 64 : 0];
+    }
+#pragma unroll
+    for (int i = 0; i < PRE; ++i) ask(wave + i * WAVES, pre[i]);
+  }
 
   const int hg = mt * 16 + li;
   const bool row_ok = hg < G;
   bf16x8 qf[NKS];
-  {
+  if constexpr (INPUT == DEC_READY) {
     const bf16_t* qrow = p.q + (long long)tok * p.q_row_stride + (long long)(g * G + (row_ok ? hg : 0)) * D;
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
@@ -1230,7 +1369,7 @@ __global__ void __launch_bounds__(256) PREFILL_OCCUPANCY attn_decode_kernel(Attn
       qf[ks] = v;
     }
   }
-  // tiles of this split, shared out to the 4 waves round-robin
+  // tiles of this split, shared out to the waves round-robin
   // (with kept first keys the tiles in front of the window that hold them are shared out too: tile numbers are then
   // counted without the gap, t_first - n_keep .. , and the first n_keep of them stand for tiles 0, 1, ...)
   const int t_first = kv_begin / BND;
@@ -1256,7 +1395,7 @@ __global__ void __launch_bounds__(256) PREFILL_OCCUPANCY attn_decode_kernel(Attn
   if (!whole_row && t_lo < t_hi) {
     if (MORE && n_keep > 0) {
       kept_entries = ps.index(n_keep * BND - 1) + 1;
-      for (int i = tid; i < kept_entries; i += 256) tbl[i] = gtable[i];
+      for (int i = tid; i < kept_entries; i += THREADS) tbl[i] = gtable[i];
     }
     // (a split of kept keys alone has no entries of its own)
     const int j_lo = (MORE && t_lo < t_first ? t_first : t_lo) * BND;
@@ -1264,7 +1403,7 @@ __global__ void __launch_bounds__(256) PREFILL_OCCUPANCY attn_decode_kernel(Attn
     tbl_first = ps.index(j_lo);
     int n = j_last >= j_lo ? ps.index(j_last) - tbl_first + 1 : 0;
     if (n > DEC_TBL_MAX - kept_entries) n = DEC_TBL_MAX - kept_entries;       // never, by the entry point's check
-    for (int i = tid; i < n; i += 256) tbl[kept_entries + i] = gtable[tbl_first + i];
+    for (int i = tid; i < n; i += THREADS) tbl[kept_entries + i] = gtable[tbl_first + i];
   }
   __syncthreads();   // the table entries are in LDS
   auto page_at = [&](int idx) -> long long {
@@ -1336,7 +1475,7 @@ __global__ void __launch_bounds__(256) PREFILL_OCCUPANCY attn_decode_kernel(Attn
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int j = j0 + lc * 8 + kt * 4 + e;
-        const bool ok = row_ok && j <= pos && (j >= kv_begin || (MORE && j < p.keep));
+        const bool ok = row_ok && j < kv_len && (j >= kv_begin || (MORE && j < p.keep));
         const float raw = MORE && p.cap > 0.f ? capped_score(s[kt][e], p.cap_in, p.cap) : s[kt][e];
         const float v = ok ? raw * p.scale_log2 : -INFINITY;
         s[kt][e] = v;
@@ -1368,49 +1507,82 @@ __global__ void __launch_bounds__(256) PREFILL_OCCUPANCY attn_decode_kernel(Attn
     bf16x8 vf_a[NDT], vf_b[NDT];
     int t = t_lo + wave;
     load_tile(t, t < t_hi, kf_a, vf_a);
+    if constexpr (INPUT != DEC_READY) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < PRE; ++i)
+        if (wave + i * WAVES < n_prep) prepare(wave + i * WAVES, pre[i]);
+      for (int i = wave + PRE * WAVES; i < n_prep; i += WAVES) {
+        ask(i, pre[0]);
+        prepare(i, pre[0]);
+      }
+      __syncthreads();                     // the block's heads are in LDS
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks)
+        qf[ks] = row_ok ? *(const bf16x8*)(q_new + (row_ok ? li : 0) * QN_STRIDE + ks * 32 + lc * 8) : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (takes_new) {                     // the new key's score of every row: 16 lanes a row, 8 elements each
+        const bf16_t *a = q_new + (tid >> 4) * QN_STRIDE, *b = k_new;
+        float s = 0.f;
+        if ((tid >> 4) < rows) {
+#pragma unroll
+          for (int c = 0; c < D / 128; ++c) {
+            const bf16x8 x = *(const bf16x8*)(a + c * 128 + li * 8), y = *(const bf16x8*)(b + c * 128 + li * 8);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s += (float)x[e] * (float)y[e];
+          }
+        }
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+        if (li == 0 && (tid >> 4) < rows) s_new[tid >> 4] = s * p.scale_log2;
+      }
+    }
     while (t < t_hi) {
       __builtin_amdgcn_sched_barrier(0);
-      load_tile(t + 4, t + 4 < t_hi, kf_b, vf_b);
+      load_tile(t + WAVES, t + WAVES < t_hi, kf_b, vf_b);
       __builtin_amdgcn_sched_barrier(0);
       multiply(t, kf_a, vf_a);
-      t += 4;
+      t += WAVES;
       if (t >= t_hi) break;
       __builtin_amdgcn_sched_barrier(0);
-      load_tile(t + 4, t + 4 < t_hi, kf_a, vf_a);
+      load_tile(t + WAVES, t + WAVES < t_hi, kf_a, vf_a);
       __builtin_amdgcn_sched_barrier(0);
       multiply(t, kf_b, vf_b);
-      t += 4;
+      t += WAVES;
     }
   }
 
-  // ---- merge the 4 waves through LDS
+  // ---- merge the waves through LDS
   float l = l_lane + __shfl_xor(l_lane, 16, 64);
   l += __shfl_xor(l, 32, 64);
-  float* sm = smem + wave * (32 + 16 * D);
+  float* sm = smem + wave * stride_w;
   if (lc == 0) {
     sm[li] = m_run;
     sm[16 + li] = l;
   }
+  if (row_ok) {
 #pragma unroll
-  for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) sm[32 + li * D + dt * 16 + lc * 4 + e] = acc[dt][e];
+    for (int dt = 0; dt < NDT; ++dt) *(f32x4*)(sm + 32 + li * DEC_STRIDE + dt * 16 + lc * 4) = acc[dt];
+  }
   __syncthreads();
-  const int rows = G - mt * 16 < 16 ? G - mt * 16 : 16;
-  for (int idx = tid; idx < rows * D; idx += 256) {
+  for (int idx = tid; idx < rows * D; idx += THREADS) {
     const int rr = idx / D, d = idx - rr * D;
-    float mx = -INFINITY;
+    float mx = takes_new ? s_new[rr] : -INFINITY;
 #pragma unroll
-    for (int ww = 0; ww < 4; ++ww) mx = fmaxf(mx, smem[ww * (32 + 16 * D) + rr]);
+    for (int ww = 0; ww < WAVES; ++ww) mx = fmaxf(mx, smem[ww * stride_w + rr]);
     float num = 0.f, den = 0.f;
     if (mx != -INFINITY) {
 #pragma unroll
-      for (int ww = 0; ww < 4; ++ww) {
-        const float* s2 = smem + ww * (32 + 16 * D);
+      for (int ww = 0; ww < WAVES; ++ww) {
+        const float* s2 = smem + ww * stride_w;
         const float f = fast_exp2(s2[rr] - mx);
-        num += s2[32 + rr * D + d] * f;
+        num += s2[32 + rr * DEC_STRIDE + d] * f;
         den += s2[16 + rr] * f;
       }
+    }
+    if (takes_new) {                       // a key whose weight has not been rounded (a NaN of its score passes through)
+      const float f = fast_exp2(s_new[rr] - mx);
+      num += v_new[d] * f;
+      den += f;
     }
     const int head = g * G + mt * 16 + rr;
     if (p.num_splits == 1) {
@@ -1538,23 +1710,10 @@ extern "C" long long jv_attn_decode_scratch_floats(int n_work, int nq, int num_s
   return num_splits > 1 ? (long long)n_work * nq * num_splits * (D + 2) : 0;
 }
 
-extern "C" int jv_attn_decode(void* out, const void* q, long long q_row_stride, const void* k_pages,
-                              const void* v_pages, const int* block_tables, int table_stride,
-                              const int* cu_seqlens, const int* context_lens, const int* work,
-                              int n_work, int page_size, int nq, int nkv, float scale, int window,
-                              int num_splits, float* scratch, const float* sinks, float cap, int keep,
-                              void* stream) {
-  if (n_work <= 0) return 0;
-  AttnArgs a{};
-  a.sinks = sinks;
-  a.cap = cap; a.keep = keep;
-  a.out = (bf16_t*)out; a.q = (const bf16_t*)q; a.q_row_stride = q_row_stride;
-  a.k_pages = (const bf16_t*)k_pages; a.v_pages = (const bf16_t*)v_pages;
-  a.block_tables = block_tables; a.table_stride = table_stride;
-  a.cu_seqlens = cu_seqlens; a.context_lens = context_lens; a.work = work;
-  a.page_size = page_size; a.nq = nq; a.nkv = nkv;
-  a.scale_log2 = scale * 1.4426950408889634f; a.window = window;
-  a.num_splits = num_splits < 1 ? 1 : num_splits;
+static int launch_decode(AttnArgs& a, int n_work, float scale, float* scratch, int input, hipStream_t stream) {
+  const int page_size = a.page_size, table_stride = a.table_stride, nq = a.nq, nkv = a.nkv;
+  a.scale_log2 = scale * 1.4426950408889634f;
+  if (a.num_splits < 1) a.num_splits = 1;
   if (int e = check_common(a)) return e;
   const bool more = set_more(a, scale);
   if (a.num_splits > 1) {
@@ -1573,22 +1732,77 @@ extern "C" int jv_attn_decode(void* out, const void* q, long long q_row_stride, 
     const long long kept = (a.keep + BND - 1) / BND * BND / page_size + 1;
     if (per_split * BND / page_size + 2 + (a.keep > 0 ? kept : 0) > DEC_TBL_MAX) return (int)hipErrorInvalidValue;
   }
-  const size_t shmem = 4 * (32 + 16 * D) * sizeof(float) +
-                       (size_t)(table_stride <= DEC_TBL_MAX ? table_stride : DEC_TBL_MAX) * sizeof(int);
-  void (*kernel)(AttnArgs) = more ? attn_decode_kernel<true> : attn_decode_kernel<false>;
+  const int entries = ((table_stride <= DEC_TBL_MAX ? table_stride : DEC_TBL_MAX) + 3) / 4 * 4;
+  const size_t shmem = (size_t)DEC_WAVES * (32 + (G < 16 ? G : 16) * DEC_STRIDE) * sizeof(float) + (size_t)entries * sizeof(int) +
+                       (input == DEC_READY ? 0 : DEC_NEW_BYTES);
+  void (*kernel)(AttnArgs) = nullptr;
+  if (input == DEC_READY) kernel = more ? attn_decode_kernel<true, DEC_READY> : attn_decode_kernel<false, DEC_READY>;
+#ifdef JV_DECODE_FUSED
+  else if (!more) kernel = input == DEC_PARTS ? attn_decode_kernel<false, DEC_PARTS> : attn_decode_kernel<false, DEC_ROWS>;
+#endif
+  if (!kernel || shmem > 160 * 1024) return (int)hipErrorInvalidValue;
   if (shmem > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute((const void*)kernel,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
     if (e != hipSuccess) return (int)e;
   }
-  hipLaunchKernelGGL(kernel, dim3((unsigned)n_work * (nkv * mt_per_head), a.num_splits), dim3(256),
-                     shmem, (hipStream_t)stream, a);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)n_work * (nkv * mt_per_head), a.num_splits), dim3(64 * DEC_WAVES), shmem, stream, a);
   int e = JV_LAUNCH_CHECK();
   if (e) return e;
   if (a.num_splits > 1) {
-    hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(n_work, nq), dim3((D + 63) / 64 * 64), 0,
-                       (hipStream_t)stream, a);
+    hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(n_work, nq), dim3((D + 63) / 64 * 64), 0, stream, a);
     e = JV_LAUNCH_CHECK();
   }
   return e;
 }
+
+extern "C" int jv_attn_decode(void* out, const void* q, long long q_row_stride, const void* k_pages,
+                              const void* v_pages, const int* block_tables, int table_stride,
+                              const int* cu_seqlens, const int* context_lens, const int* work,
+                              int n_work, int page_size, int nq, int nkv, float scale, int window,
+                              int num_splits, float* scratch, const float* sinks, float cap, int keep,
+                              void* stream) {
+  if (n_work <= 0) return 0;
+  AttnArgs a{};
+  a.sinks = sinks;
+  a.cap = cap; a.keep = keep;
+  a.out = (bf16_t*)out; a.q = (const bf16_t*)q; a.q_row_stride = q_row_stride;
+  a.k_pages = (const bf16_t*)k_pages; a.v_pages = (const bf16_t*)v_pages;
+  a.block_tables = block_tables; a.table_stride = table_stride;
+  a.cu_seqlens = cu_seqlens; a.context_lens = context_lens; a.work = work;
+  a.page_size = page_size; a.nq = nq; a.nkv = nkv;
+  a.window = window;
+  a.num_splits = num_splits;
+  return launch_decode(a, n_work, scale, scratch, DEC_READY, (hipStream_t)stream);
+}
+
+#ifdef JV_DECODE_FUSED
+// The same from the q/k/v product of a step of single tokens, request r's in row r: per-head norm (with weights), rotation (with a
+// table; half-split pairs, rotary_dim a multiple of 128), the new keys and values into their pages, attention, in one launch.
+// `parts` (n_parts 1..4) or, with null, bf16 rows `qkv`.
+extern "C" int jv_attn_decode_token(void* out, const void* qkv, const float* parts, int n_parts, long long part_stride,
+                                    const float* q_weight, const float* k_weight, float eps, const float* cos_sin, int rotary_dim,
+                                    const int* slot_mapping, void* k_pages, void* v_pages, const int* block_tables, int table_stride,
+                                    const int* context_lens, int n_work, int page_size, int nq, int nkv, float scale, int window,
+                                    int num_splits, float* scratch, const float* sinks, void* stream) {
+  if (n_work <= 0) return 0;
+  if ((parts && (n_parts < 1 || n_parts > 4)) || (!parts && !qkv) || !slot_mapping || (cos_sin && (rotary_dim % 128 || rotary_dim > D || rotary_dim <= 0)))
+    return (int)hipErrorInvalidValue;
+  AttnArgs a{};
+  a.sinks = sinks;
+  a.out = (bf16_t*)out;
+  a.q = parts ? (const bf16_t*)parts : (const bf16_t*)qkv;
+  a.q_row_stride = (long long)(nq + 2 * nkv) * D;
+  a.k_pages = (const bf16_t*)k_pages; a.v_pages = (const bf16_t*)v_pages;
+  a.k_pages_out = (bf16_t*)k_pages; a.v_pages_out = (bf16_t*)v_pages;
+  a.block_tables = block_tables; a.table_stride = table_stride;
+  a.context_lens = context_lens;
+  a.page_size = page_size; a.nq = nq; a.nkv = nkv;
+  a.window = window;
+  a.num_splits = num_splits;
+  a.parts = parts; a.part_stride = part_stride; a.n_parts = n_parts;
+  a.rotary_dim = cos_sin ? rotary_dim : 0;
+  a.q_weight = q_weight; a.k_weight = k_weight; a.norm_eps = eps; a.cos_sin = cos_sin; a.slot_mapping = slot_mapping;
+  return launch_decode(a, n_work, scale, scratch, parts ? DEC_PARTS : DEC_ROWS, (hipStream_t)stream);
+}
+#endif

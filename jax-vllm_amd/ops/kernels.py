@@ -1456,6 +1456,58 @@ def attn_decode_mfma(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_se
     )
 
 
+def attn_decode_token_possible(dtype, head_dim: int, page_size: int, interleaved: bool, rotary_dim: int, rotated: bool) -> bool:
+    """Whether ``attn_decode_token`` takes a step of single tokens of these heads."""
+    return (mfma_attention_supported(dtype, head_dim, page_size) and head_dim == 128
+            and rope_takes_parts(dtype, head_dim, interleaved, rotary_dim, rotated))
+
+
+def attn_decode_token(out, qkv, slot_mapping, q_weight, k_weight, eps, cos_sin, rotary_dim, k_pages, v_pages, block_tables,
+                      context_lens, nq, nkv, head_dim, scale, window=0, num_splits=1, scratch=None, sinks=None) -> None:
+    """``qk_norm_rope_write`` and ``attn_decode_mfma`` of a step of single tokens (request r's in row r) in one launch: ``qkv`` is
+    the q/k/v product, bfloat16 rows or float32 parts [1..4, tokens, (nq + 2 nkv) * D]; new keys and values go to their pages
+    where ``slot_mapping`` is not negative."""
+    _dev(out, qkv, slot_mapping, q_weight, k_weight, cos_sin, k_pages, v_pages, block_tables, context_lens)
+    _sinks_ok(sinks, nq)
+    page_size = k_pages.shape[2]
+    width = (nq + 2 * nkv) * head_dim
+    n = out.shape[0]
+    parts = qkv if qkv.dim() == 3 else None
+    _need(attn_decode_token_possible(out.dtype, head_dim, page_size, False, rotary_dim, cos_sin is not None),
+          "one launch takes bfloat16, head size 128, half-split pairs, a full rotation or none")
+    _need(out.shape == (n, nq * head_dim) and out.is_contiguous(), "out must be [tokens, nq * D]")
+    _need(qkv.shape[-2:] == (n, width) and qkv.stride(-1) == 1 and qkv.stride(-2) == width,
+          "qkv must be [tokens, (nq + 2 nkv) * D], or parts of that")
+    _need(qkv.dtype == torch.bfloat16 if parts is None else qkv.dtype == torch.float32 and 1 <= qkv.shape[0] <= 4,
+          "qkv is bfloat16, or up to 4 float32 parts")
+    for weight, name in ((q_weight, "q_weight"), (k_weight, "k_weight")):
+        if weight is not None:
+            _f32(weight, name, head_dim)
+    if cos_sin is not None:
+        _f32(cos_sin, "cos_sin", n * rotary_dim)
+    _i32(slot_mapping, "slot_mapping", n)
+    _check_pages(k_pages, v_pages, out.dtype, nkv, page_size, head_dim)
+    _i32(block_tables, "block_tables")
+    _i32(context_lens, "context_lens", n)
+    _need(block_tables.dim() == 2 and block_tables.shape[0] == n, "a block table row for every request")
+    least = attn_decode_min_splits(block_tables.shape[1], page_size)
+    _need(num_splits >= least, f"block tables of {block_tables.shape[1]} pages need at least {least} splits")
+    if num_splits > 1:
+        _need(scratch is not None and scratch.is_cuda and scratch.dtype == torch.float32
+              and scratch.numel() >= attn_decode_scratch_floats(n, nq, num_splits, head_dim),
+              "scratch too small for the splits")
+    lib = _attention_library(head_dim)
+    _check(
+        lib.jv_attn_decode_token(
+            _ptr(out), _ptr(qkv if parts is None else None), _ptr(parts), c_int(0 if parts is None else parts.shape[0]),
+            c_longlong(0 if parts is None else parts.stride(0)), _ptr(q_weight), _ptr(k_weight), c_float(eps), _ptr(cos_sin),
+            c_int(rotary_dim if cos_sin is not None else 0), _ptr(slot_mapping), _ptr(k_pages), _ptr(v_pages), _ptr(block_tables),
+            c_int(block_tables.shape[1]), _ptr(context_lens), c_int(n), c_int(page_size), c_int(nq), c_int(nkv), c_float(scale),
+            c_int(window or 0), c_int(num_splits), _ptr(scratch if num_splits > 1 else None), _ptr(sinks), _stream()),
+        "attn_decode_token",
+    )
+
+
 # --------------------------------------------------------------------------- what the chip delivers (for the measurement program)
 def calibrate_read(buffer: torch.Tensor, sink: torch.Tensor, blocks: int = 2048) -> None:
     """Launch the kernel that only reads ``buffer`` (its byte size must split into 16-byte pieces

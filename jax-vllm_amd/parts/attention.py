@@ -248,6 +248,12 @@ class GroupedQueryAttention:
             return self._forward_filtered(qkv, ctx, mem, cos_sin, rotary_dim)
         if self.b_qkv is not None:
             K.add_bias(qkv, self.b_qkv)
+        from . import attention_backend
+
+        out = torch.empty((n, self.nq * self.d), dtype=x.dtype, device=x.device)
+        if attention_backend.token_possible(self, ctx, mem, interleaved, rotary_dim):
+            attention_backend.run_token(self, out, qkv, cos_sin, rotary_dim, ctx, mem)
+            return self._project(out)
         parts = None
         if qkv.dim() == 3:
             parts, qkv = qkv, torch.empty(qkv.shape[1:], dtype=x.dtype, device=x.device)
@@ -258,15 +264,14 @@ class GroupedQueryAttention:
             mem.pages["k"] if writes else None, mem.pages["v"] if writes else None, ctx.page_size,
             self.nq, self.nkv, self.d, parts=parts,
         )
-        out = torch.empty((n, self.nq * self.d), dtype=x.dtype, device=x.device)
-        from . import attention_backend
-
         attention_backend.run(self, out, qkv, ctx, mem)
+        return self._project(out)
+
+    def _project(self, out):
         y = K.linear(out, self.w_o, partial_ok=True)      # the next norm adds the partial products
         if self.b_o is not None:
             K.add_bias(y, self.b_o)
         return y
-
 
     def _forward_filtered(self, qkv, ctx: StepContext, mem: LayerMemory, cos_sin, rotary_dim: int):
         if not mem.writes:

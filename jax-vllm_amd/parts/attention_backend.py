@@ -23,7 +23,7 @@ from ..ops import kernels as K
 
 TARGET_BLOCKS = 256          # blocks of the decode kernel that fill the chip: one per compute unit (measured: 8 requests of
                              # 1,060 keys over 8 kv heads take 13.7 us with 4 splits, 15.5 with 8)
-MIN_KEYS_PER_SPLIT = 128     # one 32-key tile for each of a block's 4 waves
+DECODE_TILE = K.ATTN_DECODE_TILE_KEYS      # keys of a tile of the decode kernel; a block has 4 waves with a tile each
 RESIDENT_BLOCKS = 2          # blocks of the prefill kernel that a compute unit holds at once
 
 
@@ -52,9 +52,20 @@ def decode_splits(n_decode: int, blocks_per_request: int, max_kv_len: int) -> in
     28 78.6 / 81.4; 31 86.8 / 88.8; spread over half to one and a half of that the same but for less).  Open: 3 splits at 17 to 20
     requests of 1,600 spread keys or more (17 of 3,850 60.9, with one 68.3)."""
     base = max(1, n_decode * blocks_per_request)
-    by_fill = max(1, TARGET_BLOCKS // base)
-    by_len = max(1, max_kv_len // MIN_KEYS_PER_SPLIT)
-    return max(1, min(by_fill, by_len))
+    tiles = -(-max_kv_len // DECODE_TILE)
+    splits = min(max(1, TARGET_BLOCKS // base), splits_by_length(tiles))
+    # two blocks spare less than the merge costs while few waves have a third tile (8 kv heads, one request of 300 keys 9.8 alone, 11.3 by
+    # two, 9.3 by eight; 16 requests 11.5, 13.4; 16 of 1,100 26.7, 23.8)
+    return 1 if splits == 2 and tiles < 24 else splits
+
+
+def splits_by_length(tiles: int) -> int:
+    """How many blocks a request's tiles of keys are worth.  One unit brings in about 48 GB/s whatever a block's waves ask for (1.35 us
+    for a tile a wave), so tiles are shared out thinly; the merge takes partial results in batches of 8.  Head size 128, one request
+    over 8 kv heads, microseconds with its merge: 150 keys 8.4 by one block, 8.9 by four; 300 keys 9.8 by one, 9.25 by eight; 520 keys
+    12.1, by four 10.2, by eight 9.3; 1,024 keys 15.2, 10.2 by eight, 10.7 by sixteen; 2,500 keys 13.7 by eight, 12.2 by sixteen, 12.9 by nineteen;
+    7,900 keys 17.3 by sixteen, 16.6 by 24, 17.2 by 32; one over 4 kv heads 15.0 by 32, 17.7 by 61."""
+    return 1 if tiles < 8 else 8 if tiles <= 48 else max(16, tiles // 8)
 
 
 KEY_TILE = 64                # keys of one tile of the prefill kernel
@@ -217,6 +228,29 @@ def plan_f32(ctx, nq: int, nkv: int, head_dim: int, window: int, device, keep: i
     return F32Plan(flat.pin_memory().to(device, non_blocking=True), len(items), splits, parts)
 
 
+def token_possible(att, ctx, mem, interleaved: bool, rotary_dim: int) -> bool:
+    """Whether a step of single tokens goes from the q/k/v product to its attention in one launch (``run_token``)."""
+    return (ctx.decode_only and mem.writes and not getattr(att, "softcap", None) and not getattr(att, "keep_first", 0)
+            and K.attn_decode_token_possible(att.dtype, att.d, ctx.page_size, interleaved, rotary_dim, att.rotation is not None))
+
+
+def _mfma_plan(att, ctx, window: int, keep: int, device) -> MfmaPlan:
+    key = ("mfma_attention_plan", att.nq, att.nkv, att.d, window, keep)
+    plan = ctx.plans.get(key)
+    if plan is None:
+        plan = ctx.plans[key] = plan_mfma(ctx, att.nq, att.nkv, att.d, window, device, keep)
+    return plan
+
+
+def run_token(att, out, qkv, cos_sin, rotary_dim: int, ctx, mem) -> None:
+    """Head norms, rotation, page writes and attention of a step of single tokens; ``qkv``: the q/k/v product or its parts."""
+    window = K.key_window(att.window, att.chunk)
+    plan = _mfma_plan(att, ctx, window, 0, out.device)
+    K.attn_decode_token(out, qkv, ctx.slot_mappings[mem.group], att.q_norm, att.k_norm, att.qk_norm_eps or 0.0, cos_sin, rotary_dim,
+                        mem.pages["k"], mem.pages["v"], ctx.block_tables[mem.group], ctx.context_lens, att.nq, att.nkv, att.d,
+                        att.scale, window, plan.num_splits, plan.scratch, sinks=att.sinks)
+
+
 def run(att, out, qkv, ctx, mem) -> None:
     # q heads of a row sit at the front of the fused q/k/v projection, unless the mixer says where else
     q_row_stride = getattr(att, "q_row_stride", None) or (att.nq + 2 * att.nkv) * att.d
@@ -239,10 +273,7 @@ def run(att, out, qkv, ctx, mem) -> None:
             ctx.positions, att.nq, att.nkv, att.d, att.scale, window, sinks=sinks, cap=cap, keep=keep,
         )
         return
-    key = ("mfma_attention_plan", att.nq, att.nkv, att.d, window, keep)
-    plan = ctx.plans.get(key)
-    if plan is None:
-        plan = ctx.plans[key] = plan_mfma(ctx, att.nq, att.nkv, att.d, window, qkv.device, keep)
+    plan = _mfma_plan(att, ctx, window, keep, qkv.device)
     tables = ctx.block_tables[mem.group]
     if plan.n_prefill:
         K.attn_prefill_mfma(out, qkv, q_row_stride, mem.pages["k"], mem.pages["v"], tables, ctx.cu_seqlens,
