@@ -27,7 +27,9 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));      // 16 bytes from any address of a float
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 #define G32_STEP 32            // columns of a step and of v_mfma_f32_16x16x32_bf16
 
@@ -74,6 +76,35 @@ __device__ __forceinline__ float settle(float sum, const float* a, const float* 
   }
   return sum;
 }
+// Numbers n .. n + 3 of row m of C, settled; with an activation the rows of W alternate gate and up rows and C is [M, N / 2].
+__device__ __forceinline__ void leave(float* C, int m, int n, int N, const float (&v)[4], JvAct act) {
+  if (act.id) {
+#pragma unroll
+    for (int e = 0; e < 4; e += 2)
+      if (n + e < N) C[(long long)m * (N / 2) + (n + e) / 2] = jv_gated(act, v[e], v[e + 1]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < N) C[(long long)m * N + n + e] = v[e];
+  }
+}
+// The same from sums of scaled products.  `pieces`: N a multiple of 4, C begins on 16 bytes.
+__device__ __forceinline__ void leave_sums(float* C, int m, int n, int M, int N, const f32x4& v, bool pieces, JvAct act, const float* A, const float* W, int K, int KA) {
+  bool ok = pieces && n + 4 <= N;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) ok = ok && __builtin_fabsf(v[e]) <= 3.402823466e38f;
+  if (ok && act.id) {
+    const f32x4 r = v * G32_UNSCALE;
+    *(f32x2*)(C + (long long)m * (N / 2) + n / 2) = f32x2{jv_gated(act, r[0], r[1]), jv_gated(act, r[2], r[3])};
+  } else if (ok) {
+    *(f32x4*)(C + (long long)m * N + n) = v * G32_UNSCALE;
+  } else {
+    float r[4];
+    for (int e = 0; e < 4; ++e)
+      if (n + e < N) r[e] = settle(v[e], A + (long long)m * KA, W + (long long)(n + e) * K, KA);
+    leave(C, m, n, N, r, act);
+  }
+}
 // 16 bytes a lane from base + off straight into LDS, 1 KB in the order of the lanes from `at` on.
 __device__ __forceinline__ void lds_load(unsigned off, const void* base, unsigned at) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(at) : "memory", "m0");
@@ -89,7 +120,7 @@ __device__ __forceinline__ unsigned lds_address(const void* p) {
 // DMA false: operands through registers, a round ahead, for rows that do not begin on 16 bytes.
 template <int TW, int XR, int S, int R, bool DMA>
 __global__ void __launch_bounds__(512)
-gemm_f32_few_kernel(float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K) {
+gemm_f32_few_kernel(float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K, JvAct act) {
   constexpr int ROWS = TW + XR, L = ROWS / 8, BUF = ROWS * G32_STEP, NT = TW / 16, MT = XR / 16, TILES = NT * MT;
   static_assert(TW % 16 == 0 && XR % 16 == 0 && TILES <= 4 && L * (S - 1) <= 63, "a wave adds a tile; what s_waitcnt counts to");
   __shared__ __attribute__((aligned(1024))) float bufs[DMA ? 8 * S * BUF : 4];
@@ -217,9 +248,11 @@ gemm_f32_few_kernel(float* __restrict__ C, const float* __restrict__ A, const fl
   sum += met[0][1][0][turn][lane];
   const int m = m0 + turn % MT * 16 + li, n = n0 + turn / MT * 16 + lq * 4;      // a lane holds C[m][n .. n + 3]
   if (m >= M) return;
+  float r[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e)
-    if (n + e < N) C[(long long)m * N + n + e] = settle(sum[e], A + (long long)m * K, W + (long long)(n + e) * K, K);
+    if (n + e < N) r[e] = settle(sum[e], A + (long long)m * K, W + (long long)(n + e) * K, K);
+  leave(C, m, n, N, r, act);
 }
 
 // ---------------------------------------------------------------------------- many rows
@@ -243,12 +276,12 @@ split_rows_kernel(unsigned* __restrict__ y, const float* __restrict__ A, int K, 
   for (int e = 0; e < 3; ++e) out[e * 4] = t[e];
 }
 
-// Tiles of TM rows of A (as terms) by TW rows of W (as floats); two groups of 2 x 2 waves take a half of the steps each, through
+// Tiles of TM (64) rows of A (as terms) by TW rows of W (as floats); two groups of 2 x 2 waves take a half of the steps each, through
 // rings of S steps in LDS.  Bound by what a SIMD issues: a product of 16 cycles takes 8 of them, a vector instruction 2 to 4
 // (measured), so a wave splits the next 16 rows of W (52 instructions) while it multiplies these with all its rows of A.
 template <int TM, int TW>
 __global__ void __launch_bounds__(512, 2)
-gemm_f32_tile_kernel(float* __restrict__ C, const unsigned* __restrict__ X, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K, int KA) {
+gemm_f32_tile_kernel(float* __restrict__ C, const unsigned* __restrict__ X, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K, int KA, JvAct act) {
   constexpr int MT = TM / 32, NT = TW / 32, XL = TM * 3 / 64, WL = TW / 32, L = XL + WL;      // L: loads of a wave for a step
   constexpr int XBYTES = TM * 192, BYTES = XBYTES + TW * 128, FIT = 160 * 1024 / (2 * BYTES), S = FIT < 4 ? FIT : 4;
   static_assert(S >= 2 && XL * 64 == TM * 3 && (S - 1) * L <= 63, "");
@@ -388,31 +421,218 @@ gemm_f32_tile_kernel(float* __restrict__ C, const unsigned* __restrict__ X, cons
 #pragma unroll
     for (int a = 0; a < NT; ++a) {
       const int n = n0 + (wn * NT + a) * 16 + lq * 4;
-      f32x4 v = tot[a][b] + meet[((a * MT + b) * 4 + wave) * 64 + lane];
-      bool ok = pieces && n + 4 <= N;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) ok = ok && __builtin_fabsf(v[e]) <= 3.402823466e38f;
-      if (ok) *(f32x4*)(C + (long long)m * N + n) = v * G32_UNSCALE;
-      else
-        for (int e = 0; e < 4; ++e)
-          if (n + e < N) C[(long long)m * N + n + e] = settle(v[e], A + (long long)m * KA, W + (long long)(n + e) * K, KA);
+      leave_sums(C, m, n, M, N, tot[a][b] + meet[((a * MT + b) * 4 + wave) * 64 + lane], pieces, act, A, W, K, KA);
     }
   }
 }
 
+// The same for 128 rows of A by TW rows of W, with v_mfma_f32_32x32x16_bf16: two of them give the bits of one 16x16x32 (its 32 products
+// are added in four groups of 8, in order; measured over 80,000 sums of four kinds of numbers) for the issue of half as many.  Two
+// groups of 4 waves take a half of the steps each, a wave 32 rows of A against all TW of W.  A wave's rows of A are its own: their
+// terms come straight into registers, one or two steps ahead, in pieces of 1 KB in the order of the lanes (split_fragments_kernel; 16 bytes from
+// each of 64 rows an instruction cost a fifth more).  W is split once a group: a thread takes 4 numbers a row two or three steps
+// ahead, splits them beside the products of a step and leaves the terms in a ring of 3 steps in LDS.
+// Against tiles of 128 rows by the 16x16x32 instruction, in which every wave split its W and which were bound by what a SIMD issues,
+// microseconds with the split of A, before -> now: 1,003 x 6,144 x 2,048 160 -> 149, x 2,048 61 -> 56, 384 x 4,096 x 4,096 111 -> 88, 2,048 x 24,576 x
+// 4,096 2,385 -> 2,070 (1.2 PFLOP/s of the matrix unit's, where its power ends it); over 199 sizes 0.94 of the time with what f32_plan takes.
+template <int TW>
+__global__ void __launch_bounds__(512, 2)
+gemm_f32_rows_kernel(float* __restrict__ C, const unsigned* __restrict__ X, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K, int KA, JvAct act) {
+  constexpr int TM = 128, NT = TW / 32, TERMS = 3 * TW * 64, RING = 3;
+  static_assert(2 * RING * TERMS <= 160 * 1024 && TM * TW * 4 <= 2 * RING * TERMS, "");
+  __shared__ __attribute__((aligned(1024))) char bufs[2 * RING * TERMS];
+  const int lane = threadIdx.x & 63, all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), group = all >> 2, wave = all & 3;
+  const int mtiles = (M + TM - 1) / TM, live = mtiles * ((N + TW - 1) / TW), per = (live + 7) / 8;
+  const int u = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || u >= live) return;
+  const int m0 = u % mtiles * TM, n0 = u / mtiles * TW;
+  const int total = (K + G32_STEP - 1) / G32_STEP, turns = (total + 1) / 2, first = group * turns, steps = group ? total - turns : turns;
+  const int li = lane & 31, lh = lane >> 5;
+  const char* xrow = (const char*)X + (long long)min(m0 / 32 + wave, (M - 1) / 32) * total * 6144 + lane * 16;
+  const int gt = threadIdx.x & 255, wr = gt >> 3, wp = gt & 7;
+  const float* wrow[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) wrow[j] = W + (long long)min(n0 + j * 32 + wr, N - 1) * K;
+  char* const ring = bufs + group * (RING * TERMS);
+  // where this thread's pieces go: piece c (16 bytes) of row r of a term lies at slot c ^ (r / 2 % 4)
+  const int put = wr * 64 + (((wp >> 1) ^ (wr >> 1)) & 3) * 16 + (wp & 1) * 8;
+  const int get0 = li * 64 + ((lh ^ (li >> 1)) & 3) * 16, get1 = li * 64 + (((2 + lh) ^ (li >> 1)) & 3) * 16;
+  constexpr int XS = TW > 96 ? 2 : 3, WS = TW > 64 ? 2 : 3;      // sets of registers for rows of A and of W on their way
+  f32x4 raw[WS][NT];
+  u32x4 xt[XS][3][2], wt[2][3][2];
+  f32x16 tot[NT], t[2];
+  auto load_w = [&](int c, f32x4 (&r)[NT]) {
+    const int at = min(min(first + c, total - 1) * G32_STEP + wp * 4, K - 4);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) r[j] = *(const f32x4*)(wrow[j] + at);
+  };
+  auto load_x = [&](int c, u32x4 (&x)[3][2]) {
+    const char* at = xrow + (long long)min(first + c, total - 1) * 6144;
+#pragma unroll
+    for (int e = 2; e >= 0; --e)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) x[e][b] = *(const u32x4*)(at + (e * 2 + b) * 1024);
+  };
+  auto put_w = [&](const f32x4& r, int j, char* slot) {
+    u32x4 q[3];
+    split_pair(r[0], r[1], 0, q);
+    split_pair(r[2], r[3], 1, q);
+#pragma unroll
+    for (int e = 0; e < 3; ++e) *(u32x2*)(slot + e * (TW * 64) + j * 2048 + put) = u32x2{q[e][0], q[e][1]};
+  };
+  auto get_w = [&](int a, const char* slot, u32x4 (&w)[3][2]) {
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+      w[e][0] = *(const u32x4*)(slot + e * (TW * 64) + a * 2048 + get0);
+      w[e][1] = *(const u32x4*)(slot + e * (TW * 64) + a * 2048 + get1);
+    }
+  };
+  auto meet_all = [&] {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+#pragma unroll
+  for (int a = 0; a < NT; ++a)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) tot[a][e] = 0.f;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) t[0][e] = t[1][e] = 0.f;
+  {
+    f32x4 w0[NT], w1[NT];
+    load_w(0, w0);
+    load_w(1, w1);
+#pragma unroll
+    for (int i = 0; i + 1 < XS; ++i) load_x(i, xt[i]);
+#pragma unroll
+    for (int i = 0; i < WS; ++i) load_w(2 + i, raw[i]);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) put_w(w0[j], j, ring);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) put_w(w1[j], j, ring + TERMS);
+  }
+  meet_all();
+  get_w(0, ring, wt[0]);
+  int slot = 0;
+  // Step c: its W lies in `slot`, that of c + 1 in the next; W of c + 2, in registers, is split into the one after, a piece of 4 numbers
+  // beside the products of 32 rows.  A tile's products of a step join its total beside the next tile's.
+  auto step = [&](auto phase, int c) {
+    constexpr int PH = decltype(phase)::value;
+    const int s1 = slot + 1 == RING ? 0 : slot + 1, s2 = s1 + 1 == RING ? 0 : s1 + 1;
+    load_x(c + XS - 1, xt[(PH + XS - 1) % XS]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (c < steps) {
+#pragma unroll
+      for (int a = 0; a < NT; ++a) {
+        const int cur = (PH * NT + a) & 1, before = (a + NT - 1) % NT;
+        auto& w = wt[cur];
+        if (a + 1 < NT) get_w(a + 1, ring + slot * TERMS, wt[cur ^ 1]);
+        else get_w(0, ring + s1 * TERMS, wt[cur ^ 1]);
+        __builtin_amdgcn_sched_barrier(0);
+        f32x16 q;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) q[e] = 0.f;
+#pragma unroll
+        for (int e = 0; e < G32_PRODUCTS; ++e)
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+            q = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w[G32_W[e]][b]), __builtin_bit_cast(bf16x8, xt[PH % XS][G32_X[e]][b]), q, 0, 0, 0);
+        put_w(raw[PH % WS][a], a, ring + s2 * TERMS);
+        tot[before] += t[cur ^ 1];
+        t[cur] = q;
+#pragma unroll
+        for (int i = 0; i < 12; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);      // a product, then four or five others
+          __builtin_amdgcn_sched_group_barrier(0x2, 5, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      load_w(c + 2 + WS, raw[PH % WS]);
+    }
+    meet_all();
+    slot = s1;
+  };
+  using std::integral_constant;
+  for (int c = 0; c < turns; c += 6) {
+    step(integral_constant<int, 0>{}, c);
+    if (c + 1 < turns) step(integral_constant<int, 1>{}, c + 1);
+    if (c + 2 < turns) step(integral_constant<int, 2>{}, c + 2);
+    if (c + 3 < turns) step(integral_constant<int, 3>{}, c + 3);
+    if (c + 4 < turns) step(integral_constant<int, 4>{}, c + 4);
+    if (c + 5 < turns) step(integral_constant<int, 5>{}, c + 5);
+  }
+  if constexpr (NT % 2 == 0) tot[NT - 1] += t[1];
+  else tot[NT - 1] += steps & 1 ? t[0] : t[1];
+  __syncthreads();
+  f32x4* meet = (f32x4*)bufs;
+  if (group) {
+#pragma unroll
+    for (int a = 0; a < NT; ++a)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) meet[((a * 4 + q) * 4 + wave) * 64 + lane] = f32x4{tot[a][q * 4], tot[a][q * 4 + 1], tot[a][q * 4 + 2], tot[a][q * 4 + 3]};
+  }
+  __syncthreads();
+  if (group) return;
+  const bool pieces = !(N & 3) && !((uintptr_t)C & 15);
+  const int m = m0 + wave * 32 + li;
+  if (m >= M) return;
+#pragma unroll
+  for (int a = 0; a < NT; ++a)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int n = n0 + a * 32 + q * 8 + lh * 4;
+      const f32x4 v = f32x4{tot[a][q * 4], tot[a][q * 4 + 1], tot[a][q * 4 + 2], tot[a][q * 4 + 3]} + meet[((a * 4 + q) * 4 + wave) * 64 + lane];
+      leave_sums(C, m, n, M, N, v, pieces, act, A, W, K, KA);
+    }
+}
+
 // How C is made (jv_gemm_f32): 0, 1: few rows, 16 x 16 or 32 x 32, through registers; 2 to 4: few rows through the ring, 16 x 16, 32 x 16, 32 x 32
-// (rows of W x rows of A); from 5 on tiles, 128 x 128, 128 x 96, 128 x 64, 64 x 96, 64 x 64, 64 x 32 (rows of A x rows of W).
+// (rows of W x rows of A); 5 to 7 tiles of 128 rows of A by 128, 96, 64 of W, 8 to 10 of 64 rows by 96, 64, 32.
 template <int TW, int XR, int S, int R, bool DMA>
-static int few_launch(float* C, const float* A, const float* W, int M, int N, int K, hipStream_t s) {
+static int few_launch(float* C, const float* A, const float* W, int M, int N, int K, JvAct act, hipStream_t s) {
   if ((M + XR - 1) / XR > 65535) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL((gemm_f32_few_kernel<TW, XR, S, R, DMA>), dim3((N + TW - 1) / TW, (M + XR - 1) / XR), dim3(512), 0, s, C, A, W, M, N, K);
+  hipLaunchKernelGGL((gemm_f32_few_kernel<TW, XR, S, R, DMA>), dim3((N + TW - 1) / TW, (M + XR - 1) / XR), dim3(512), 0, s, C, A, W, M, N, K, act);
   return JV_LAUNCH_CHECK();
 }
 template <int TM, int TW>
-static int tile_launch(float* C, const void* X, const float* A, const float* W, int M, int N, int K, int KA, hipStream_t s) {
+static int tile_launch(float* C, const void* X, const float* A, const float* W, int M, int N, int K, int KA, JvAct act, hipStream_t s) {
   const long long live = ((long long)M + TM - 1) / TM * (((long long)N + TW - 1) / TW);
   if (live > 1 << 24) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL((gemm_f32_tile_kernel<TM, TW>), dim3((unsigned)((live + 7) / 8 * 8)), dim3(512), 0, s, C, (const unsigned*)X, A, W, M, N, K, KA);
+  hipLaunchKernelGGL((gemm_f32_tile_kernel<TM, TW>), dim3((unsigned)((live + 7) / 8 * 8)), dim3(512), 0, s, C, (const unsigned*)X, A, W, M, N, K, KA, act);
+  return JV_LAUNCH_CHECK();
+}
+// The same in the order in which gemm_f32_rows_kernel multiplies: [M / 32][steps][term][16 columns][8 columns][32 rows][8].
+__global__ void __launch_bounds__(256)
+split_fragments_kernel(unsigned* __restrict__ y, const float* __restrict__ A, int M, int K, int steps) {
+  const int row = threadIdx.x >> 3, m = blockIdx.x * 32 + row, k = (blockIdx.y * 8 + (threadIdx.x & 7)) * 8;
+  if (m >= M || k >= steps * G32_STEP) return;
+  const float* a = A + (long long)m * K + k;
+  f32x4 v[2];
+  if (k + 8 <= K && ((uintptr_t)a & 15) == 0) {
+    v[0] = *(const f32x4*)a, v[1] = *(const f32x4*)(a + 4);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e / 4][e % 4] = k + e < K ? a[e] : 0.f;
+  }
+  u32x4 t[3];
+  split8(v, t);
+  u32x4* out = (u32x4*)y + ((long long)blockIdx.x * steps + k / G32_STEP) * 384 + k % G32_STEP / 16 * 64 + k % 16 / 8 * 32 + row;
+#pragma unroll
+  for (int e = 0; e < 3; ++e) out[e * 128] = t[e];
+}
+extern "C" int jv_split_fragments_f32(void* X, const float* A, int M, int KA, void* stream) {
+  if (M <= 0 || KA <= 0) return 0;
+  if ((uintptr_t)X & 15) return (int)hipErrorInvalidValue;
+  const int steps = (KA + G32_STEP - 1) / G32_STEP;
+  if ((steps + 1) / 2 > 65535) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(split_fragments_kernel, dim3((M + 31) / 32, (steps + 1) / 2), dim3(256), 0, (hipStream_t)stream, (unsigned*)X, A, M, KA, steps);
+  return JV_LAUNCH_CHECK();
+}
+template <int TW>
+static int rows_launch(float* C, const void* X, const float* A, const float* W, int M, int N, int K, int KA, JvAct act, hipStream_t s) {
+  const long long live = ((long long)M + 127) / 128 * (((long long)N + TW - 1) / TW);
+  if (live > 1 << 24) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL((gemm_f32_rows_kernel<TW>), dim3((unsigned)((live + 7) / 8 * 8)), dim3(512), 0, s, C, (const unsigned*)X, A, W, M, N, K, KA, act);
   return JV_LAUNCH_CHECK();
 }
 // Rows of A [M][KA] as terms (of 2^24 times A), [M][steps][3][32] bf16 with zeros behind KA; steps = ceil(KA / 32).
@@ -425,26 +645,30 @@ extern "C" int jv_split_rows_f32(void* X, const float* A, int M, int KA, void* s
   return JV_LAUNCH_CHECK();
 }
 // A [M][KA], W [N][K], C [M][N].  K = KA but for tiles, where W may have columns behind KA (finite; as many steps of 32 as KA has).
-// X: the rows of A by jv_split_rows_f32, for tiles.
-extern "C" int jv_gemm_f32(float* C, const float* A, const float* W, const void* X, int M, int N, int K, int KA, int form, void* stream) {
+// X, for tiles: the rows of A by jv_split_fragments_f32 (forms 5 to 7) or jv_split_rows_f32 (from 8 on).
+// gate_act (JV_ACT_*, not 0): the rows of W alternate gate and up rows and C is [M][N / 2], act(gate) * up.
+extern "C" int jv_gemm_f32(float* C, const float* A, const float* W, const void* X, int M, int N, int K, int KA, int form, int gate_act, float act_limit,
+                           float act_slope, void* stream) {
   if (M <= 0 || N <= 0) return 0;
   const bool pieces = !(K & 3) && !((uintptr_t)W & 15) && K > 0;
   if (K < 0 || KA > K || (KA + 31) / 32 != (K + 31) / 32) return (int)hipErrorInvalidValue;
+  if (gate_act && (!jv_act_known(gate_act) || N % 2)) return (int)hipErrorInvalidValue;
   if (form >= 5 ? !pieces || !X || ((uintptr_t)X & 15) || K > 1 << 22 : KA != K || (form >= 2 && (!pieces || ((uintptr_t)A & 15) || K > 1 << 24)))
     return (int)hipErrorInvalidValue;
+  const JvAct act{gate_act, act_limit, act_slope};
   const hipStream_t s = (hipStream_t)stream;
   switch (form) {
-    case 0: return few_launch<16, 16, 1, 2, false>(C, A, W, M, N, K, s);
-    case 1: return few_launch<32, 32, 1, 1, false>(C, A, W, M, N, K, s);
-    case 2: return few_launch<16, 16, 2, 2, true>(C, A, W, M, N, K, s);
-    case 3: return few_launch<32, 16, 1, 1, true>(C, A, W, M, N, K, s);
-    case 4: return few_launch<32, 32, 1, 1, true>(C, A, W, M, N, K, s);
-    case 5: return tile_launch<128, 128>(C, X, A, W, M, N, K, KA, s);
-    case 6: return tile_launch<128, 96>(C, X, A, W, M, N, K, KA, s);
-    case 7: return tile_launch<128, 64>(C, X, A, W, M, N, K, KA, s);
-    case 8: return tile_launch<64, 96>(C, X, A, W, M, N, K, KA, s);
-    case 9: return tile_launch<64, 64>(C, X, A, W, M, N, K, KA, s);
-    case 10: return tile_launch<64, 32>(C, X, A, W, M, N, K, KA, s);
+    case 0: return few_launch<16, 16, 1, 2, false>(C, A, W, M, N, K, act, s);
+    case 1: return few_launch<32, 32, 1, 1, false>(C, A, W, M, N, K, act, s);
+    case 2: return few_launch<16, 16, 2, 2, true>(C, A, W, M, N, K, act, s);
+    case 3: return few_launch<32, 16, 1, 1, true>(C, A, W, M, N, K, act, s);
+    case 4: return few_launch<32, 32, 1, 1, true>(C, A, W, M, N, K, act, s);
+    case 5: return rows_launch<128>(C, X, A, W, M, N, K, KA, act, s);
+    case 6: return rows_launch<96>(C, X, A, W, M, N, K, KA, act, s);
+    case 7: return rows_launch<64>(C, X, A, W, M, N, K, KA, act, s);
+    case 8: return tile_launch<64, 96>(C, X, A, W, M, N, K, KA, act, s);
+    case 9: return tile_launch<64, 64>(C, X, A, W, M, N, K, KA, act, s);
+    case 10: return tile_launch<64, 32>(C, X, A, W, M, N, K, KA, act, s);
   }
   return (int)hipErrorInvalidValue;
 }

@@ -743,16 +743,17 @@ def attn_f32(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_seqlens, c
 # --------------------------------------------------------------------------- matrix products
 F32_STEP = 32         # columns of a step of the 32-bit product
 # tiles of the 32-bit product: form, rows of a, rows of w, microseconds of a round per 1,024 columns on one unit and on all
-_F32_TILES = ((5, 128, 128, 34.0, 45.0), (6, 128, 96, 26.0, 35.0), (7, 128, 64, 19.2, 28.0), (8, 64, 96, 17.7, 22.0), (9, 64, 64, 13.1, 17.0),
-              (10, 64, 32, 7.5, 12.5))
+_F32_TILES = ((5, 128, 128, 23.5, 38.3), (6, 128, 96, 19.6, 30.8), (7, 128, 64, 11.6, 23.2), (8, 64, 96, 16.7, 22.2), (9, 64, 64, 11.2, 16.3),
+              (10, 64, 32, 4.0, 10.0))
+_F32_FRAGMENTS = 8    # forms below take the terms of a in the order of the matrix unit's operands
 
 
 @functools.lru_cache(maxsize=4096)
 def f32_plan(m: int, n: int, k: int, pieces: bool = True, a_pieces: bool = True) -> int:
     """Form of the 32-bit product (``jv_gemm_f32``).  All give the same bits, so it is the one that takes the least time by a count of
-    rounds over 256 units that meets what was measured (1 to 2,048 rows, n 256 to 32,000, k 512 to 12,288) mostly within a sixth; for example
-    k = 2,048: 5 x 2,048 8.8 us (form 2), 16 x 32,000 53 (3), 37 x 3,072 15.5 (4), 250 x 6,144 50 (8), 1,003 x 6,144 145 (6), 2,048 x 2,048 101 (5);
-    in graphs with cold weights and operands scaled 9.6, 57, 17.6, 60, 172, 114.
+    rounds over 256 units, fitted to 199 sizes (17 to 2,048 rows, n 1,024 to 32,000, k 512 to 12,288, in graphs with cold weights): within 2 %
+    of the best form at all of them but 33 to 64 rows of 8,192 x 1,024 (20 %); for example k = 2,048: 5 x 2,048 9.6 us (form 2), 16 x 32,000 57 (3),
+    37 x 3,072 17.1 (4), 100 x 6,144 39.6 (9; 4 takes 48), 250 x 6,144 48 (7), 1,003 x 6,144 152 (6), 2,048 x 2,048 100 (5).
     ``pieces``: rows of w begin on 16 bytes (else they are copied for tiles, and few rows go through registers); ``a_pieces``: rows of a too."""
     q, mb = k / 1024, n * k * 4e-6
 
@@ -772,7 +773,7 @@ def f32_plan(m: int, n: int, k: int, pieces: bool = True, a_pieces: bool = True)
             times[0] = 4 + rounds(16, 16, 2, 8, 10, 512)
     if m <= 65535 * 32:
         if through_ring:
-            times[4] = max(3 + rounds(32, 32, 1, 5.3, 6.2), 3 + mb / 4.9)
+            times[4] = max(3 + rounds(32, 32, 1, 5.3, 7.1), 3 + mb / 4.9)
         else:
             times[1] = 4 + rounds(32, 32, 2, 16, 18, 512)
     if m > 32 and 0 < k <= 1 << 22:
@@ -783,33 +784,39 @@ def f32_plan(m: int, n: int, k: int, pieces: bool = True, a_pieces: bool = True)
     return min(times, key=times.get)
 
 
-def gemm_f32(a: torch.Tensor, w: torch.Tensor, out=None) -> torch.Tensor:
-    """out = a @ w.T in 32-bit: every float input whole, products but for what is below 2^-26 of them, float sums.  a [M, K], w [N, K], both row-major."""
+def gemm_f32(a: torch.Tensor, w: torch.Tensor, out=None, gate_pairs: "str | tuple | None" = None) -> torch.Tensor:
+    """out = a @ w.T in 32-bit: every float input whole, products but for what is below 2^-26 of them, float sums.  a [M, K], w [N, K], both row-major.
+    ``gate_pairs``: the rows of w alternate gate and up rows, out = act(a.w[2j]) * (a.w[2j+1]) [M, N / 2] (bit for bit what ``gated_mul``
+    makes of the product)."""
     _dev(a, w)
     _f32(a, "a")
     _f32(w, "w")
     m, k = a.shape
     n = w.shape[0]
     _need(w.shape[1] == k, f"inner sizes differ: {k} and {w.shape[1]}")
+    _need(not gate_pairs or n % 2 == 0, "gate and up rows come in pairs")
+    width = n // 2 if gate_pairs else n
     if out is None:
-        out = torch.empty((m, n), dtype=torch.float32, device=a.device)
+        out = torch.empty((m, width), dtype=torch.float32, device=a.device)
     _dev(out)
-    _need(out.shape == (m, n) and out.dtype == torch.float32, "out must be float32 [M, N]")
+    _need(out.shape == (m, width) and out.dtype == torch.float32, "out must be float32 [M, N], of half that width with an activation")
+    act = _gate_act(gate_pairs) if gate_pairs else _NO_ACT
     if not m or not n:
         return out
     pieces = not k & 3 and not w.data_ptr() & 15
     form, lib, terms, kw = f32_plan(m, n, k, pieces, not a.data_ptr() & 15), library.core(), None, k
-    if form >= 5:      # the rows of a, scaled, as sums of three bfloat16 numbers, [M, steps, 3, 32]
-        steps = -(-k // F32_STEP)
-        terms = torch.empty((m, steps, 3, F32_STEP), dtype=torch.bfloat16, device=a.device)
-        _check(lib.jv_split_rows_f32(_ptr(terms), _ptr(a), c_int(m), c_int(k), _stream()), "split_rows_f32")
+    if form >= 5:      # the rows of a, scaled, as sums of three bfloat16 numbers, [M, steps, 3, 32] or whole operands of 32 rows
+        steps, fragments = -(-k // F32_STEP), form < _F32_FRAGMENTS
+        terms = torch.empty((-(-m // 32) * 32 if fragments else m, steps, 3, F32_STEP), dtype=torch.bfloat16, device=a.device)
+        split = lib.jv_split_fragments_f32 if fragments else lib.jv_split_rows_f32
+        _check(split(_ptr(terms), _ptr(a), c_int(m), c_int(k), _stream()), "split_rows_f32")
         if not pieces:
             kw = -(-k // 4) * 4
             copy = torch.empty((n, kw), dtype=torch.float32, device=w.device)
             copy[:, :k], copy[:, k:] = w, 0.0
             w = copy
-    _check(lib.jv_gemm_f32(_ptr(out), _ptr(a), _ptr(w), _ptr(terms), c_int(m), c_int(n), c_int(kw), c_int(k), c_int(form), _stream()),
-           "gemm_f32")
+    _check(lib.jv_gemm_f32(_ptr(out), _ptr(a), _ptr(w), _ptr(terms), c_int(m), c_int(n), c_int(kw), c_int(k), c_int(form), *act,
+                           _stream()), "gemm_f32")
     return out
 
 
@@ -1231,7 +1238,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
     if isinstance(x, UnscaledRows):
         scale, x = x, x.x
     if x.dtype == torch.float32:
-        y = gemm_f32(x, w)
+        y = gemm_f32(x, w, gate_pairs=gate_pairs)
+        gate_pairs = None
     else:
         _need(x.dtype == w.dtype, "x and w must have one type")
         m, (n, k) = x.shape[0], w.shape
