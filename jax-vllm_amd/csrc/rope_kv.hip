@@ -216,17 +216,25 @@ __global__ void __launch_bounds__(256) qk_norm_rope_write_fast_kernel(
 // a lane holds two 16-byte pieces of a head, the same places of its two halves, so both numbers
 // of every rotation pair sit in one lane and a head takes only D/16 lanes (bf16): a wave prepares
 // 64 / (D/16) heads of one token with two 16-byte loads and stores a lane.  q in place, k to its
-// page; the v heads are written by v_pages_write_kernel.
+// page; the first v_blocks blocks write the v heads of 16 tokens each to their pages.
+// Microseconds in a graph, 32 q and 8 kv heads of 128, v heads in a launch of their own and its slots looked up one after another -> now:
+// 256 tokens 7.7 -> 6.2, 1,003 11.2 -> 7.8, 2,048 15.0 -> 12.1, 1,501 beside 24 tokens that decode 15.4 -> 9.9; 16 and 4 heads in float,
+// 1,003 tokens 11.3 -> 7.9.  (Three groups of heads a wave with one look at the angles: 26 at 2,048 tokens.)
 template <typename T, int D>
 __global__ void __launch_bounds__(256) qk_norm_rope_write_wide_kernel(
     T* __restrict__ qkv, const int* __restrict__ slot_mapping, const float* __restrict__ q_w,
     const float* __restrict__ k_w, float eps, const float* __restrict__ cos_sin, T* __restrict__ k_pages,
-    int page_size, int n_tokens, int nq, int nkv) {
+    int page_size, int n_tokens, int nq, int nkv, VPages<T> vp, int v_blocks) {
   constexpr int EP = 16 / (int)sizeof(T), HALF = D / 2, LPH = HALF / EP, HPW = 64 / LPH;
   static_assert(LPH >= 1 && LPH <= 64 && (LPH & (LPH - 1)) == 0, "lanes per head must be a power of two");
+  extern __shared__ __attribute__((aligned(16))) unsigned char v_tile_mem[];
+  if ((int)blockIdx.x < v_blocks) {
+    v_pages_tile<T>(vp, blockIdx.x / nkv, blockIdx.x % nkv, v_tile_mem);
+    return;
+  }
   const int lane = threadIdx.x & 63;
   const int walk = nq + nkv, groups = (walk + HPW - 1) / HPW;
-  const long long item = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const long long item = (long long)(blockIdx.x - v_blocks) * 4 + (threadIdx.x >> 6);
   if (item >= (long long)n_tokens * groups) return;
   const long long t = item / groups;
   const int grp = (int)(item - t * groups);
@@ -285,14 +293,16 @@ __global__ void __launch_bounds__(256) qk_norm_rope_write_wide_kernel(
 
 template <typename T, int D>
 static int launch_rope_wide(void* qkv, const int* slot_mapping, const float* q_w, const float* k_w, float eps,
-                            const float* cos_sin, void* k_pages, int page_size, int n_tokens, int nq, int nkv,
+                            const float* cos_sin, void* k_pages, void* v_pages, int page_size, int n_tokens, int nq, int nkv,
                             void* stream) {
   constexpr int HPW = 64 / (D / 2 / (16 / (int)sizeof(T)));
-  const long long items = (long long)n_tokens * ((nq + nkv + HPW - 1) / HPW);
-  if ((items + 3) / 4 > 0x7fffffffll) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL((qk_norm_rope_write_wide_kernel<T, D>), dim3((unsigned)((items + 3) / 4)), dim3(256), 0,
-                     (hipStream_t)stream, (T*)qkv, slot_mapping, q_w, k_w, eps, cos_sin, (T*)k_pages, page_size,
-                     n_tokens, nq, nkv);
+  const long long items = (long long)n_tokens * ((nq + nkv + HPW - 1) / HPW), v_blocks = (long long)((n_tokens + 15) / 16) * nkv;
+  if ((items + 3) / 4 + v_blocks > 0x7fffffffll) return (int)hipErrorInvalidValue;
+  const VPages<T> vp{(const T*)qkv + (long long)(nq + nkv) * D, (long long)(nq + 2 * nkv) * D, slot_mapping, (T*)v_pages, page_size,
+                     n_tokens, nkv, D, D, 1.f, nullptr, nullptr, 0, 0.f};
+  hipLaunchKernelGGL((qk_norm_rope_write_wide_kernel<T, D>), dim3((unsigned)((items + 3) / 4 + v_blocks)), dim3(256), v_tile_bytes<T>(D),
+                     (hipStream_t)stream, (T*)qkv, slot_mapping, q_w, k_w, eps, cos_sin, (T*)k_pages, page_size, n_tokens, nq, nkv, vp,
+                     (int)v_blocks);
   return JV_LAUNCH_CHECK();
 }
 
@@ -307,6 +317,14 @@ static int launch_rope_wide(void* qkv, const int* slot_mapping, const float* q_w
     if ((n_heads + 3) / 4 > 65535) return (int)hipErrorInvalidValue;                               \
     const int half = rotary_dim / 2;                                                               \
     const bool v_tile = v_written_by_tile<T>(k_pages, n_tokens, page_size, D);                     \
+    if (v_tile && !interleaved && (!cos_sin || rotary_dim == D) && (D == 64 || D == 128 || D == 256)) {  \
+      if (D == 64) return launch_rope_wide<T, 64>(qkv, slot_mapping, q_w, k_w, eps, cos_sin, k_pages,    \
+                                                  v_pages, page_size, n_tokens, nq, nkv, stream);  \
+      if (D == 128) return launch_rope_wide<T, 128>(qkv, slot_mapping, q_w, k_w, eps, cos_sin, k_pages,  \
+                                                    v_pages, page_size, n_tokens, nq, nkv, stream); \
+      return launch_rope_wide<T, 256>(qkv, slot_mapping, q_w, k_w, eps, cos_sin, k_pages, v_pages, page_size, \
+                                      n_tokens, nq, nkv, stream);                                  \
+    }                                                                                              \
     if (v_tile) {                                                                                  \
       const int e = launch_v_pages_write<T>(qkv, (long long)n_heads * D, (long long)(nq + nkv) * D, \
                                             slot_mapping, v_pages, page_size, n_tokens, nkv, D, D, \
@@ -314,14 +332,6 @@ static int launch_rope_wide(void* qkv, const int* slot_mapping, const float* q_w
       if (e) return e;                                                                             \
     }                                                                                              \
     const int walk = v_tile ? nq + nkv : n_heads;                                                  \
-    if (v_tile && !interleaved && (!cos_sin || rotary_dim == D) && (D == 64 || D == 128 || D == 256)) {  \
-      if (D == 64) return launch_rope_wide<T, 64>(qkv, slot_mapping, q_w, k_w, eps, cos_sin, k_pages,    \
-                                                  page_size, n_tokens, nq, nkv, stream);           \
-      if (D == 128) return launch_rope_wide<T, 128>(qkv, slot_mapping, q_w, k_w, eps, cos_sin, k_pages,  \
-                                                    page_size, n_tokens, nq, nkv, stream);         \
-      return launch_rope_wide<T, 256>(qkv, slot_mapping, q_w, k_w, eps, cos_sin, k_pages, page_size, \
-                                      n_tokens, nq, nkv, stream);                                  \
-    }                                                                                              \
     if ((D == 128 || D == 256) && !interleaved && (!cos_sin || (half % 64 == 0 && half > 0))) {    \
       /* many tokens: a wave walks several heads; few tokens: one head per wave for parallelism */ \
       const int hpw = n_tokens >= 256 ? (walk + 3) / 4 : 1;                                        \
