@@ -16,6 +16,7 @@
 // output embedding, which those do not take, run here in many rounds (151,936 x 2,048 104 us, x resident in LDS 154; 151,936 x 4,096 at two
 // rows 205.4, resident 205.0, staying 208).
 #include "common.h"
+#include "row_source.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
@@ -27,14 +28,23 @@ enum { FEW_BF16 = 0, FEW_F32 = 1, FEW_PAIRS = 2 };
 #define FEW_K 64           // columns of a chunk: a row of it is 128 bytes, 8 pieces of 16
 #define FEW_WAVES 8
 
-// CW: the most chunks of a wave.
-template <int MODE, int TW, int CW>
+// CW: the most chunks of a wave.  SRC (row_source.h): the block makes its MR rows of x itself and scales them; K is then KX columns.
+template <int MODE, int TW, int CW, int SRC = ROWS_GIVEN, int MR = 1, int KX = 64>
 __global__ void __launch_bounds__(64 * FEW_WAVES)
-gemm_few_kernel(void* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, int M, int N, int K, long long ldx, JvAct act) {
+gemm_few_kernel(void* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, int M, int N, int K, long long ldx, JvAct act,
+                RowSource src_rows) {
   constexpr int NT = TW / 16, L = TW / 8, CHUNK = TW * FEW_K, S = 64 * 1024 / (FEW_WAVES * CHUNK * 2) < CW ? 64 * 1024 / (FEW_WAVES * CHUNK * 2) : CW;
   static_assert(NT * 1024 <= S * CHUNK * 2, "the parts meet in the ring's place");
   __shared__ __attribute__((aligned(1024))) bf16_t bufs[FEW_WAVES][S * CHUNK];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, lq = lane >> 4;
+  constexpr int XSTRIDE = KX + 8;
+  __shared__ __attribute__((aligned(16))) bf16_t xmade[SRC == ROWS_GIVEN ? 8 : MR * XSTRIDE];
+  __shared__ float made_sq[MR * 8];
+  RowMaker<SRC, MR, KX> maker;
+  if constexpr (SRC != ROWS_GIVEN) {
+    maker.ask(src_rows, 0, K);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   const int n0 = blockIdx.x * TW, all = K / FEW_K;
   const int first = all * wave / FEW_WAVES, chunks = all * (wave + 1) / FEW_WAVES - first;
   // an instruction brings 8 rows, lane l row l / 8, and fills 1 KB in the order of the lanes; piece c of row r lies at slot
@@ -54,14 +64,24 @@ gemm_few_kernel(void* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t
     if (c < chunks) fetch(c, c);
   // rows of x beyond the last are zeros: their lanes load nothing
   bf16x8 xf[CW][2];
-  const bf16_t* xr = x + (long long)min(li, M - 1) * ldx + first * FEW_K + lq * 8;
+  if constexpr (SRC == ROWS_GIVEN) {
+    const bf16_t* xr = x + (long long)min(li, M - 1) * ldx + first * FEW_K + lq * 8;
 #pragma unroll
-  for (int c = 0; c < CW; ++c)
+    for (int c = 0; c < CW; ++c)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      xf[c][h] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-      if (li < M && c < chunks) xf[c][h] = *(const bf16x8*)(xr + c * FEW_K + h * 32);
-    }
+      for (int h = 0; h < 2; ++h) {
+        xf[c][h] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+        if (li < M && c < chunks) xf[c][h] = *(const bf16x8*)(xr + c * FEW_K + h * 32);
+      }
+  } else {
+    maker.give(src_rows, 0, K, blockIdx.x == 0, xmade, XSTRIDE, made_sq);
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < CW; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        xf[c][h] = c < chunks ? *(const bf16x8*)(xmade + min(li, MR - 1) * XSTRIDE + (first + c) * FEW_K + h * 32 + lq * 8) : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
   for (int c = 0; c < CW; ++c)
@@ -101,6 +121,12 @@ gemm_few_kernel(void* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t
   f32x4 sum = red[wave * FEW_WAVES * 64 + lane];
 #pragma unroll
   for (int p = 1; p < FEW_WAVES; ++p) sum += red[(wave * FEW_WAVES + p) * 64 + lane];
+  if (SRC == ROWS_RESIDUAL) {
+    float sq = 0.f;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) sq += made_sq[min(li, MR - 1) * 8 + w];
+    sum *= rsqrtf(sq * src_rows.inv_width + src_rows.eps);
+  }
   const int m = li, n = n0 + wave * 16 + lq * 4;      // a lane holds y[m][n .. n + 3]; N is a multiple of 4
   if (m >= M || n >= N) return;
   if (MODE == FEW_F32) {
@@ -124,7 +150,7 @@ static int few_launch(void* y, const void* x, const void* W, int M, int N, int K
 #define FEW(CW)                                                                                                                        \
   if (cw <= CW) {                                                                                                                      \
     hipLaunchKernelGGL((gemm_few_kernel<MODE, TW, CW>), dim3((N + TW - 1) / TW), dim3(64 * FEW_WAVES), 0, s, y, (const bf16_t*)x,     \
-                       (const bf16_t*)W, M, N, K, ldx, act);                                                                           \
+                       (const bf16_t*)W, M, N, K, ldx, act, RowSource{});                                                                           \
     return JV_LAUNCH_CHECK();                                                                                                          \
   }
   FEW(2) FEW(4) FEW(8)
@@ -143,5 +169,36 @@ extern "C" int jv_gemm_few_bf16(void* y, const void* x, const void* W, int M, in
   if (mode == FEW_BF16) return tw == 16 ? few_launch<FEW_BF16, 16>(y, x, W, M, N, K, ldx, act, s) : few_launch<FEW_BF16, 32>(y, x, W, M, N, K, ldx, act, s);
   if (mode == FEW_F32) return tw == 16 ? few_launch<FEW_F32, 16>(y, x, W, M, N, K, ldx, act, s) : few_launch<FEW_F32, 32>(y, x, W, M, N, K, ldx, act, s);
   if (mode == FEW_PAIRS) return tw == 16 ? few_launch<FEW_PAIRS, 16>(y, x, W, M, N, K, ldx, act, s) : few_launch<FEW_PAIRS, 32>(y, x, W, M, N, K, ldx, act, s);
+  return (int)hipErrorInvalidValue;
+}
+
+// y = (norm of h + parts) W^T for one or two rows that the blocks make themselves: bf16 [M][N], or with gate_act [M][N / 2].  h_out takes h + parts.
+template <int MODE, int TW, int KX>
+static int few_made(void* y, const void* W, int M, int N, JvAct act, const RowSource& src, hipStream_t s) {
+  constexpr int CW = (KX / FEW_K + FEW_WAVES - 1) / FEW_WAVES;
+  if (M == 1)
+    hipLaunchKernelGGL((gemm_few_kernel<MODE, TW, CW, ROWS_RESIDUAL, 1, KX>), dim3((N + TW - 1) / TW), dim3(64 * FEW_WAVES), 0, s, y, (const bf16_t*)W,
+                       (const bf16_t*)W, M, N, KX, (long long)KX, act, src);
+  else
+    hipLaunchKernelGGL((gemm_few_kernel<MODE, TW, CW, ROWS_RESIDUAL, 2, KX>), dim3((N + TW - 1) / TW), dim3(64 * FEW_WAVES), 0, s, y, (const bf16_t*)W,
+                       (const bf16_t*)W, M, N, KX, (long long)KX, act, src);
+  return JV_LAUNCH_CHECK();
+}
+extern "C" int jv_gemm_few_residual_bf16(void* y, const float* h, float* h_out, const float* parts, int n_parts, long long part_stride, const float* weight,
+                                         float eps, const void* W, int M, int N, int K, int gate_act, float act_limit, float act_slope, int tw, void* stream) {
+  if (M < 1 || M > 2 || N <= 0 || N % 4 || n_parts < 0 || n_parts > 4 || (n_parts && !parts) || h == h_out || (gate_act && !jv_act_known(gate_act)) ||
+      (((uintptr_t)W | (uintptr_t)y) & 15))
+    return (int)hipErrorInvalidValue;
+  RowSource src{};
+  src.h = h; src.h_out = h_out; src.parts = parts; src.n_parts = n_parts; src.part_stride = part_stride; src.weight = weight;
+  src.inv_width = 1.f / (float)K; src.eps = eps;
+  const JvAct act{gate_act, act_limit, act_slope};
+  const hipStream_t s = (hipStream_t)stream;
+#define FEW_MADE(KX)                                                                                                                   \
+  if (K == KX)                                                                                                                         \
+    return gate_act ? (tw == 16 ? few_made<FEW_PAIRS, 16, KX>(y, W, M, N, act, src, s) : few_made<FEW_PAIRS, 32, KX>(y, W, M, N, act, src, s)) \
+                    : (tw == 16 ? few_made<FEW_BF16, 16, KX>(y, W, M, N, act, src, s) : few_made<FEW_BF16, 32, KX>(y, W, M, N, act, src, s));
+  FEW_MADE(1024) FEW_MADE(2048) FEW_MADE(4096)
+#undef FEW_MADE
   return (int)hipErrorInvalidValue;
 }

@@ -17,6 +17,7 @@
 // up rows, y[m, j] = act(x.W[2j]) * (x.W[2j+1]) straight from the float accumulators (a lane
 // holds both numbers of a pair), which saves the activation kernel and its round trip.
 #include "common.h"
+#include "row_source.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -356,10 +357,19 @@ struct RowScale {
 // been multiplied, so all slots but one are in flight.  With 4 slots that is three quarters of a tile on its way
 // in half the registers of the two-tile scheme: what two row tiles of x with 16 pieces a wave need to fit (128
 // registers of x, 64 of W).
-template <int NL, int MT, typename OutT, bool PAIRS, bool EDGE, int SLOTS = 0>
+//
+// SRC (row_source.h): the block makes its columns of x itself, MR (1 or 2) rows of them; ROWS_RESIDUAL with the whole inner size in the block
+// also scales them (MT 1, no EDGE, no SLOTS).
+template <int NL, int MT, typename OutT, bool PAIRS, bool EDGE, int SLOTS = 0, int SRC = ROWS_GIVEN, int MR = 1>
 __global__ void __launch_bounds__(512)
 gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t* __restrict__ W,
-                              int M, int N, int K, long long ldx, long long ldy, RowScale rs) {
+                              int M, int N, int K, long long ldx, long long ldy, RowScale rs, RowSource src) {
+  static_assert(SRC == ROWS_GIVEN || (MT == 1 && !EDGE && SLOTS == 0), "");
+  constexpr int KB = NL * 256, XSTRIDE = KB + SK_PAD;
+  __shared__ __attribute__((aligned(16))) bf16_t xmade[SRC == ROWS_GIVEN ? 8 : MR * XSTRIDE];
+  __shared__ float made_sq[MR * 8];
+  RowMaker<SRC, MR, KB> maker;
+  if constexpr (SRC != ROWS_GIVEN) maker.ask(src, blockIdx.y * KB, K);
   y += (long long)blockIdx.y * M * ldy;
   // the 8 waves' partial tiles, in two buffers that take turns: one barrier per tile (the waves that do
   // not add may run ahead into the next tile, whose partials go to the other buffer; nobody can be two
@@ -372,6 +382,7 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
   const int n_tiles = (N + 15) / 16;
   // x: rows mt * 16 + li (zero beyond M), this wave's columns
   bf16x8 b[MT][NL];
+  if constexpr (SRC == ROWS_GIVEN) {
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -380,13 +391,14 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
       const bf16x8 v = *(const bf16x8*)(x + (long long)m * ldx + (EDGE ? min(k, K - 8) : k));
       b[mt][i] = (!EDGE || k < K) ? v : zero;
     }
+  }
   // a tile beyond the last (the prefetch after the last tile) reads the first pieces of W, the same for all lanes
   // the scale of this lane's output row (wave mt adds row tile mt): asked for now, used after the first tile;
   // without a scale the loads read x (no load inside a branch) and get no weight
   // (one 16-byte load a lane: the 4 lanes of a row hold its 16 shares; every block reads these few lines,
   // so every instruction more would queue up at one place in the L2)
-  f32x4 row_sq;
-  {
+  f32x4 row_sq = {0.f, 0.f, 0.f, 0.f};
+  if constexpr (SRC == ROWS_GIVEN) {
     const int m = min((wk < MT ? wk : 0) * 16 + li, M - 1);
     const float* sp = rs.ssq ? rs.ssq + (long long)m * 16 + lc * 4 : (const float*)x;
     row_sq = *(const f32x4*)sp;
@@ -434,6 +446,12 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
         const float inv = rsqrtf(sq * rs.inv_width + rs.eps);
         s[0] *= inv; s[1] *= inv; s[2] *= inv; s[3] *= inv;
       }
+      if (SRC == ROWS_RESIDUAL && gridDim.y == 1) {
+        float sq = 0.f;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) sq += made_sq[min(li, MR - 1) * 8 + w];
+        s *= rsqrtf(sq * src.inv_width + src.eps);
+      }
       if (m < M) {
         if (PAIRS) {
 #pragma unroll
@@ -462,6 +480,19 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
     };
     bf16x8 a0[NL], a1[NL];
     load_tile(tile, a0);
+    if constexpr (SRC != ROWS_GIVEN) {
+      __builtin_amdgcn_sched_barrier(0);
+      maker.give(src, blockIdx.y * KB, K, blockIdx.x == 0, xmade, XSTRIDE, made_sq);
+      __syncthreads();
+      if (SRC == ROWS_RESIDUAL && gridDim.y > 1 && blockIdx.x == 0 && tid < MR) {
+        float sq = 0.f;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) sq += made_sq[tid * 8 + w];
+        src.ssq_out[tid * 16 + blockIdx.y] = sq;
+      }
+#pragma unroll
+      for (int i = 0; i < NL; ++i) b[0][i] = *(const bf16x8*)(xmade + min(li, MR - 1) * XSTRIDE + (wk * NL + i) * 32 + lc * 8);
+    }
     for (;;) {
       int next = tile + gridDim.x;
       __builtin_amdgcn_sched_barrier(0);
@@ -512,10 +543,10 @@ static int launch_persistent(void* y, const void* x, const void* W, int M, int N
   if (blocks > n_tiles) blocks = n_tiles;
   if (K == ksplit * 8 * NL * 32)
     hipLaunchKernelGGL((gemm_skinny_persistent_kernel<NL, MT, OutT, PAIRS, false, SLOTS>), dim3(blocks, ksplit), dim3(512), 0,
-                       stream, (OutT*)y, (const bf16_t*)x, (const bf16_t*)W, M, N, K, ldx, ldy, rs);
+                       stream, (OutT*)y, (const bf16_t*)x, (const bf16_t*)W, M, N, K, ldx, ldy, rs, RowSource{});
   else
     hipLaunchKernelGGL((gemm_skinny_persistent_kernel<NL, MT, OutT, PAIRS, true, SLOTS>), dim3(blocks, ksplit), dim3(512), 0,
-                       stream, (OutT*)y, (const bf16_t*)x, (const bf16_t*)W, M, N, K, ldx, ldy, rs);
+                       stream, (OutT*)y, (const bf16_t*)x, (const bf16_t*)W, M, N, K, ldx, ldy, rs, RowSource{});
   return JV_LAUNCH_CHECK();
 }
 
@@ -651,4 +682,59 @@ extern "C" int jv_gemm_skinny_scaled_bf16(void* y, const void* x, const void* W,
   if (!ssq || width <= 0) return (int)hipErrorInvalidValue;
   return gemm_skinny_entry(y, x, W, M, N, K, ldx, ldy, out_f32, JvAct{gate_act, act_limit, act_slope}, wr, wk, nks, ksplit,
                            RowScale{ssq, shares, 1.f / (float)width, eps, JvAct{}}, stream);
+}
+
+// One or two rows that the blocks make themselves (RowSource): blocks that stay, an inner size of ksplit * 256 * nl columns exactly.
+template <int NL, typename OutT, bool PAIRS, int SRC>
+static int launch_made(void* y, const void* W, int M, int N, int K, long long ldy, int blocks, int ksplit, RowScale rs, const RowSource& src, hipStream_t s) {
+  const int n_tiles = (N + 15) / 16;
+  blocks = (blocks + ksplit - 1) / ksplit;
+  if (blocks > n_tiles) blocks = n_tiles;
+  if (M == 1)
+    hipLaunchKernelGGL((gemm_skinny_persistent_kernel<NL, 1, OutT, PAIRS, false, 0, SRC, 1>), dim3(blocks, ksplit), dim3(512), 0, s, (OutT*)y,
+                       (const bf16_t*)W, (const bf16_t*)W, M, N, K, 0, ldy, rs, src);
+  else
+    hipLaunchKernelGGL((gemm_skinny_persistent_kernel<NL, 1, OutT, PAIRS, false, 0, SRC, 2>), dim3(blocks, ksplit), dim3(512), 0, s, (OutT*)y,
+                       (const bf16_t*)W, (const bf16_t*)W, M, N, K, 0, ldy, rs, src);
+  return JV_LAUNCH_CHECK();
+}
+template <typename OutT, bool PAIRS, int SRC>
+static int dispatch_made(int nl, void* y, const void* W, int M, int N, int K, long long ldy, int blocks, int ksplit, RowScale rs, const RowSource& src,
+                         hipStream_t s) {
+  if (M < 1 || M > 2 || N <= 0 || blocks < 1 || ksplit < 1 || ksplit > 16 || K != ksplit * 256 * nl) return (int)hipErrorInvalidValue;
+  switch (nl) {
+    case 4: return launch_made<4, OutT, PAIRS, SRC>(y, W, M, N, K, ldy, blocks, ksplit, rs, src, s);
+    case 5: return launch_made<5, OutT, PAIRS, SRC>(y, W, M, N, K, ldy, blocks, ksplit, rs, src, s);
+    case 8: return launch_made<8, OutT, PAIRS, SRC>(y, W, M, N, K, ldy, blocks, ksplit, rs, src, s);
+    case 10: return launch_made<10, OutT, PAIRS, SRC>(y, W, M, N, K, ldy, blocks, ksplit, rs, src, s);
+    case 12: return launch_made<12, OutT, PAIRS, SRC>(y, W, M, N, K, ldy, blocks, ksplit, rs, src, s);
+    case 16: return launch_made<16, OutT, PAIRS, SRC>(y, W, M, N, K, ldy, blocks, ksplit, rs, src, s);
+    case 20: return launch_made<20, OutT, PAIRS, SRC>(y, W, M, N, K, ldy, blocks, ksplit, rs, src, s);
+  }
+  return (int)hipErrorInvalidValue;
+}
+// y = (norm of h + parts) W^T: float partial products [ksplit][M][N], not scaled (ksplit > 1; ssq [M][16] takes ksplit shares of the rows' sums of
+// squares), float [M][N], or with gate_act bf16 [M][N / 2], both scaled.  h_out takes h + parts.
+extern "C" int jv_gemm_skinny_residual_bf16(void* y, const float* h, float* h_out, const float* parts, int n_parts, long long part_stride,
+                                            const float* weight, float* ssq, float eps, const void* W, int M, int N, int K, int gate_act,
+                                            float act_limit, float act_slope, int blocks, int nl, int ksplit, void* stream) {
+  if (n_parts < 0 || n_parts > 4 || (n_parts && !parts) || h == h_out || (ksplit > 1 && (!ssq || gate_act)) || (gate_act && (!jv_act_known(gate_act) || N % 2)))
+    return (int)hipErrorInvalidValue;
+  RowSource src{};
+  src.h = h; src.h_out = h_out; src.parts = parts; src.n_parts = n_parts; src.part_stride = part_stride; src.weight = weight; src.ssq_out = ssq;
+  src.inv_width = 1.f / (float)K; src.eps = eps;
+  RowScale rs{};
+  rs.act = JvAct{gate_act, act_limit, act_slope};
+  const hipStream_t s = (hipStream_t)stream;
+  if (gate_act) return dispatch_made<bf16_t, true, ROWS_RESIDUAL>(nl, y, W, M, N, K, N / 2, blocks, ksplit, rs, src, s);
+  return dispatch_made<float, false, ROWS_RESIDUAL>(nl, y, W, M, N, K, N, blocks, ksplit, rs, src, s);
+}
+// y = x W^T with x the heads of a decode attention whose keys were shared out to `splits` blocks (jv_attn_decode's scratch): float [ksplit][M][N].
+extern "C" int jv_gemm_skinny_splits_bf16(float* y, const float* scratch, int splits, int heads, int head_dim, const float* sinks, const void* W, int M,
+                                          int N, int K, int blocks, int nl, int ksplit, void* stream) {
+  if (splits < 1 || heads < 1 || head_dim % 4 || (long long)heads * head_dim != K) return (int)hipErrorInvalidValue;
+  RowSource src{};
+  src.part_acc = scratch; src.part_ml = (const float2*)(scratch + (long long)M * heads * splits * head_dim);
+  src.sinks = sinks; src.splits = splits; src.heads = heads; src.head_dim = head_dim;
+  return dispatch_made<float, false, ROWS_SPLITS>(nl, y, W, M, N, K, N, blocks, ksplit, RowScale{}, src, (hipStream_t)stream);
 }

@@ -115,6 +115,10 @@ struct AttnArgs {
   const int* slot_mapping;    // [tokens] page * page_size + slot of the token's key, or negative: not stored
   bf16_t* k_pages_out;
   bf16_t* v_pages_out;
+  // DEC_PARTS: rows of parts that are still to be multiplied by rsqrt(sum_{j < sq_shares} row_sq[row * 16 + j] * sq_inv_width + sq_eps), or null
+  const float* row_sq;
+  int sq_shares;
+  float sq_inv_width, sq_eps;
 };
 
 // ------------------------------------------------------------------------------------ prefill
@@ -1262,7 +1266,7 @@ __global__ void __launch_bounds__(64 * DEC_WAVES) PREFILL_OCCUPANCY attn_decode_
   const int n_prep = rows + (takes_new ? 2 : 0);
   struct Head { float v[4][E], w[E]; };
   Head pre[INPUT == DEC_READY ? 1 : PRE];
-  float cs[E], sn[E];
+  float cs[E], sn[E], sq_raw = 0.f, row_scale = 1.f;
   int slot_raw = -1;
   const int half = p.rotary_dim / 2, HE = half / 64;       // pair (e, e + HE) for e < HE
   // no load inside a branch: what is not there is read from the block table and not used
@@ -1294,6 +1298,7 @@ __global__ void __launch_bounds__(64 * DEC_WAVES) PREFILL_OCCUPANCY attn_decode_
 #pragma unroll
         for (int q = 1; q < 4; ++q)
           if (q < p.n_parts) v[e] += h.v[q][e];
+        v[e] *= row_scale;
       }
     }
     const int slot = __builtin_amdgcn_readfirstlane(slot_raw);
@@ -1345,6 +1350,7 @@ __global__ void __launch_bounds__(64 * DEC_WAVES) PREFILL_OCCUPANCY attn_decode_
     int lane_zero;
     asm volatile("v_mov_b32 %0, 0" : "=v"(lane_zero));
     slot_raw = p.slot_mapping[tok + lane_zero];
+    if (INPUT == DEC_PARTS) sq_raw = (p.row_sq ? p.row_sq + (long long)tok * 16 : p.parts)[li];
     const float* cp = p.cos_sin ? p.cos_sin + (long long)tok * p.rotary_dim + lane : (const float*)p.q;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -1509,6 +1515,7 @@ __global__ void __launch_bounds__(64 * DEC_WAVES) PREFILL_OCCUPANCY attn_decode_
     load_tile(t, t < t_hi, kf_a, vf_a);
     if constexpr (INPUT != DEC_READY) {
       __builtin_amdgcn_sched_barrier(0);
+      if (INPUT == DEC_PARTS && p.row_sq) row_scale = rsqrtf(wave_sum(lane < p.sq_shares ? sq_raw : 0.f) * p.sq_inv_width + p.sq_eps);
 #pragma unroll
       for (int i = 0; i < PRE; ++i)
         if (wave + i * WAVES < n_prep) prepare(wave + i * WAVES, pre[i]);
@@ -1710,7 +1717,8 @@ extern "C" long long jv_attn_decode_scratch_floats(int n_work, int nq, int num_s
   return num_splits > 1 ? (long long)n_work * nq * num_splits * (D + 2) : 0;
 }
 
-static int launch_decode(AttnArgs& a, int n_work, float scale, float* scratch, int input, hipStream_t stream) {
+// merge false: the splits' results stay in scratch.
+static int launch_decode(AttnArgs& a, int n_work, float scale, float* scratch, int input, bool merge, hipStream_t stream) {
   const int page_size = a.page_size, table_stride = a.table_stride, nq = a.nq, nkv = a.nkv;
   a.scale_log2 = scale * 1.4426950408889634f;
   if (a.num_splits < 1) a.num_splits = 1;
@@ -1749,7 +1757,7 @@ static int launch_decode(AttnArgs& a, int n_work, float scale, float* scratch, i
   hipLaunchKernelGGL(kernel, dim3((unsigned)n_work * (nkv * mt_per_head), a.num_splits), dim3(64 * DEC_WAVES), shmem, stream, a);
   int e = JV_LAUNCH_CHECK();
   if (e) return e;
-  if (a.num_splits > 1) {
+  if (a.num_splits > 1 && merge) {
     hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(n_work, nq), dim3((D + 63) / 64 * 64), 0, stream, a);
     e = JV_LAUNCH_CHECK();
   }
@@ -1773,19 +1781,22 @@ extern "C" int jv_attn_decode(void* out, const void* q, long long q_row_stride, 
   a.page_size = page_size; a.nq = nq; a.nkv = nkv;
   a.window = window;
   a.num_splits = num_splits;
-  return launch_decode(a, n_work, scale, scratch, DEC_READY, (hipStream_t)stream);
+  return launch_decode(a, n_work, scale, scratch, DEC_READY, true, (hipStream_t)stream);
 }
 
 #ifdef JV_DECODE_FUSED
 // The same from the q/k/v product of a step of single tokens, request r's in row r: per-head norm (with weights), rotation (with a
 // table; half-split pairs, rotary_dim a multiple of 128), the new keys and values into their pages, attention, in one launch.
-// `parts` (n_parts 1..4) or, with null, bf16 rows `qkv`.
+// `parts` (n_parts 1..4) or, with null, bf16 rows `qkv`.  row_sq (parts only; [tokens][16], sq_shares of them, or null): the rows' norm over
+// sq_width columns is still to be applied.  merge 0: where num_splits > 1 the splits' results stay in scratch, [request][head][split][D]
+// and behind them (max, sum) each, and `out` is not written.
 extern "C" int jv_attn_decode_token(void* out, const void* qkv, const float* parts, int n_parts, long long part_stride,
-                                    const float* q_weight, const float* k_weight, float eps, const float* cos_sin, int rotary_dim,
-                                    const int* slot_mapping, void* k_pages, void* v_pages, const int* block_tables, int table_stride,
+                                    const float* row_sq, int sq_shares, int sq_width, float sq_eps, const float* q_weight,
+                                    const float* k_weight, float eps, const float* cos_sin, int rotary_dim, const int* slot_mapping, void* k_pages, void* v_pages, const int* block_tables, int table_stride,
                                     const int* context_lens, int n_work, int page_size, int nq, int nkv, float scale, int window,
-                                    int num_splits, float* scratch, const float* sinks, void* stream) {
+                                    int num_splits, float* scratch, const float* sinks, int merge, void* stream) {
   if (n_work <= 0) return 0;
+  if (row_sq && (!parts || sq_shares < 1 || sq_shares > 16 || sq_width <= 0)) return (int)hipErrorInvalidValue;
   if ((parts && (n_parts < 1 || n_parts > 4)) || (!parts && !qkv) || !slot_mapping || (cos_sin && (rotary_dim % 128 || rotary_dim > D || rotary_dim <= 0)))
     return (int)hipErrorInvalidValue;
   AttnArgs a{};
@@ -1801,8 +1812,9 @@ extern "C" int jv_attn_decode_token(void* out, const void* qkv, const float* par
   a.window = window;
   a.num_splits = num_splits;
   a.parts = parts; a.part_stride = part_stride; a.n_parts = n_parts;
+  a.row_sq = row_sq; a.sq_shares = sq_shares; a.sq_inv_width = row_sq ? 1.f / (float)sq_width : 0.f; a.sq_eps = sq_eps;
   a.rotary_dim = cos_sin ? rotary_dim : 0;
   a.q_weight = q_weight; a.k_weight = k_weight; a.norm_eps = eps; a.cos_sin = cos_sin; a.slot_mapping = slot_mapping;
-  return launch_decode(a, n_work, scale, scratch, parts ? DEC_PARTS : DEC_ROWS, (hipStream_t)stream);
+  return launch_decode(a, n_work, scale, scratch, parts ? DEC_PARTS : DEC_ROWS, merge != 0, (hipStream_t)stream);
 }
 #endif

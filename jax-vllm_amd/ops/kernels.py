@@ -185,6 +185,57 @@ def add_parts_unscaled(h: torch.Tensor, parts: torch.Tensor, weight: torch.Tenso
     return UnscaledRows(xg, ssq, hidden, eps)
 
 
+MADE_MAX_ROWS = 2         # rows that the blocks of a product make for themselves (``csrc/row_source.h``)
+MADE_MAX_SPLITS = 16      # of a decode attention that the output product merges
+
+
+class PendingRows:
+    """Rows ``norm(h + parts[0] + parts[1] + ...)`` that ``linear`` makes in the product that reads them: its blocks do the residual step, each
+    for the columns it multiplies, and leave the stream in ``out`` (another tensor than ``h``, which they all read).  Up to
+    ``MADE_MAX_ROWS`` rows; the reader is asked first (``linear_takes_pending_rows``)."""
+
+    dtype = torch.bfloat16
+
+    def __init__(self, h: torch.Tensor, parts: "torch.Tensor | None", weight: torch.Tensor, eps: float, out: torch.Tensor):
+        _dev(h, parts, weight, out)
+        _f32(h, "h")
+        _f32(weight, "weight", h.shape[1])
+        _need(h.dim() == 2 and h.is_contiguous() and out.shape == h.shape and out.dtype == h.dtype and out.is_contiguous()
+              and out.data_ptr() != h.data_ptr(), "the stream moves from one float tensor [rows, width] to another")
+        _need(0 < h.shape[0] <= MADE_MAX_ROWS, f"at most {MADE_MAX_ROWS} rows")
+        _need(parts is None or (parts.dtype == torch.float32 and parts.dim() == 3 and parts.shape[1:] == h.shape and 1 <= parts.shape[0] <= 4
+                                and parts[0].is_contiguous()), "partial products must be float32 [parts <= 4, *h.shape]")
+        self.h, self.parts, self.weight, self.eps, self.out = h, parts, weight, float(eps), out
+
+    shape = property(lambda self: self.h.shape)
+    device = property(lambda self: self.h.device)
+
+    def operands(self) -> tuple:
+        n = 0 if self.parts is None else self.parts.shape[0]
+        return (_ptr(self.h), _ptr(self.out), _ptr(self.parts), c_int(n), c_longlong(self.parts.stride(0) if n else 0), _ptr(self.weight))
+
+
+class UnscaledParts:
+    """Partial products [parts, M, N] of rows whose RMSNorm scale is still to be applied (``ssq`` as in ``UnscaledRows``, one share for every
+    part): what the product of ``PendingRows`` leaves where its inner size is shared out."""
+
+    def __init__(self, parts: torch.Tensor, ssq: torch.Tensor, width: int, eps: float):
+        self.parts, self.ssq, self.width, self.eps = parts, ssq, int(width), float(eps)
+
+
+class SplitHeads:
+    """The heads [rows, heads * head_dim] of a decode attention as its splits left them (``attn_decode_token`` with ``merge`` False);
+    ``linear`` merges them in the product that reads them (ask ``linear_takes_split_heads`` first)."""
+
+    dtype = torch.bfloat16
+
+    def __init__(self, scratch: torch.Tensor, rows: int, splits: int, heads: int, head_dim: int, sinks):
+        self.scratch, self.splits, self.heads, self.head_dim, self.sinks = scratch, int(splits), int(heads), int(head_dim), sinks
+        self.shape = (int(rows), self.heads * self.head_dim)
+
+    device = property(lambda self: self.scratch.device)
+
+
 def cast_rows(x: torch.Tensor, dtype: torch.dtype, rows=None) -> torch.Tensor:
     """Copy (selected) rows of a float matrix into a new matrix of ``dtype``."""
     _dev(x, rows)
@@ -1235,6 +1286,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
     of its own after the library's product).
     """
     scale = None
+    if isinstance(x, (PendingRows, SplitHeads)):
+        return _linear_made(x, w, gate_pairs, partial_ok, partial_max_width)
     if isinstance(x, UnscaledRows):
         scale, x = x, x.x
     if x.dtype == torch.float32:
@@ -1282,6 +1335,69 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
     if out_dtype is not None and y.dtype != out_dtype:
         y = y.to(out_dtype)
     return y
+
+
+def _made_plan(m: int, w: torch.Tensor, gate_pairs: bool, partial_ok: bool, partial_max_width):
+    """How a product makes its one or two rows itself: (blocks, pieces, parts) of blocks that stay, whose columns fill their pieces, or the tile
+    of ``gemm_few``; None where neither takes it."""
+    n, k = w.shape
+    if not 0 < m <= MADE_MAX_ROWS or w.dtype != torch.bfloat16 or n % 4 or w.data_ptr() & 15 or not w.is_contiguous():
+        return None
+    plan = streaming_plan(m, n, k, gate_pairs, partial_ok, w.device, partial_max_width)
+    if plan is not None and plan[0] != TILE64 and plan[0][0] == -2:
+        (_, blocks, pieces), parts = plan
+        return (blocks, pieces, parts) if k == 256 * pieces * parts and pieces in MADE_PIECES and (gate_pairs or parts > 1) else None
+    if plan in (None, STAGED) and k in MADE_FEW_INNER:
+        return few_tile(m, n, k, compute_units(w.device))
+    return None
+
+
+MADE_PIECES = (4, 5, 8, 10, 12, 16, 20)
+MADE_FEW_INNER = (1024, 2048, 4096)
+
+
+def linear_takes_pending_rows(n_rows: int, w: torch.Tensor, gate_pairs: bool = False, partial_ok: bool = False,
+                              partial_max_width: int | None = PARTIAL_SUM_MAX_WIDTH) -> bool:
+    """Whether ``linear`` with these arguments makes ``PendingRows`` itself.  Microseconds of a layer's four products with the two residual
+    steps and norms, launches of their own / made by the products: 4,096 wide (12,288 inside) one row 82.4 / 78.0, two rows 82.5 / 80.1; 2,048
+    wide (3,072 inside) 29.6 / 24.6, 29.3 / 25.7."""
+    return _made_plan(n_rows, w, gate_pairs, partial_ok, partial_max_width) is not None
+
+
+def linear_takes_split_heads(n_rows: int, w: torch.Tensor, splits: int) -> bool:
+    """Whether ``linear(..., partial_ok=True)`` merges ``SplitHeads`` itself."""
+    return 1 < splits <= MADE_MAX_SPLITS and isinstance(_made_plan(n_rows, w, False, True, PARTIAL_SUM_MAX_WIDTH), tuple)
+
+
+def _linear_made(x, w: torch.Tensor, gate_pairs, partial_ok: bool, partial_max_width):
+    _dev(w)
+    m, (n, k) = x.shape[0], w.shape
+    _need(x.shape[1] == k, "inner sizes differ")
+    plan = _made_plan(m, w, bool(gate_pairs), partial_ok, partial_max_width)
+    _need(plan is not None, "no product makes these rows itself (ask linear_takes_pending_rows or linear_takes_split_heads first)")
+    lib, act = library.core(), _gate_act(gate_pairs) if gate_pairs else _NO_ACT
+    if not isinstance(plan, tuple):
+        _need(isinstance(x, PendingRows), "split heads are merged by blocks that stay")
+        y = torch.empty((m, n // 2 if gate_pairs else n), dtype=torch.bfloat16, device=w.device)
+        _check(lib.jv_gemm_few_residual_bf16(_ptr(y), *x.operands(), c_float(x.eps), _ptr(w), c_int(m), c_int(n), c_int(k), *act, c_int(plan),
+                                             _stream()), "gemm_few_residual")
+        return y
+    blocks, pieces, parts = plan
+    shape = (c_int(m), c_int(n), c_int(k))
+    if isinstance(x, SplitHeads):
+        _need(not gate_pairs and parts > 1, "merged heads leave partial products")
+        y = torch.empty((parts, m, n), dtype=torch.float32, device=w.device)
+        _check(lib.jv_gemm_skinny_splits_bf16(_ptr(y), _ptr(x.scratch), c_int(x.splits), c_int(x.heads), c_int(x.head_dim), _ptr(x.sinks), _ptr(w),
+                                              *shape, c_int(blocks), c_int(pieces), c_int(parts), _stream()), "gemm_skinny_splits")
+        return y
+    if gate_pairs:
+        y, ssq = torch.empty((m, n // 2), dtype=torch.bfloat16, device=w.device), None
+    else:
+        y = torch.empty((parts, m, n), dtype=torch.float32, device=w.device)
+        ssq = torch.empty((m, UNSCALED_MAX_SHARES), dtype=torch.float32, device=w.device)      # a share for every part is written
+    _check(lib.jv_gemm_skinny_residual_bf16(_ptr(y), *x.operands(), _ptr(ssq), c_float(x.eps), _ptr(w), *shape, *act, c_int(blocks), c_int(pieces),
+                                            c_int(parts), _stream()), "gemm_skinny_residual")
+    return y if gate_pairs else UnscaledParts(y, ssq, k, x.eps)
 
 
 def linear_takes_unscaled_rows(n_rows: int, w: torch.Tensor, gate_pairs: bool = False, partial_ok: bool = False,
@@ -1471,19 +1587,26 @@ def attn_decode_token_possible(dtype, head_dim: int, page_size: int, interleaved
 
 
 def attn_decode_token(out, qkv, slot_mapping, q_weight, k_weight, eps, cos_sin, rotary_dim, k_pages, v_pages, block_tables,
-                      context_lens, nq, nkv, head_dim, scale, window=0, num_splits=1, scratch=None, sinks=None) -> None:
+                      context_lens, nq, nkv, head_dim, scale, window=0, num_splits=1, scratch=None, sinks=None, merge: bool = True) -> None:
     """``qk_norm_rope_write`` and ``attn_decode_mfma`` of a step of single tokens (request r's in row r) in one launch: ``qkv`` is
     the q/k/v product, bfloat16 rows or float32 parts [1..4, tokens, (nq + 2 nkv) * D]; new keys and values go to their pages
-    where ``slot_mapping`` is not negative."""
+    where ``slot_mapping`` is not negative.  ``UnscaledParts`` are scaled here.  ``merge`` False: with ``num_splits`` > 1 the splits' results
+    stay in ``scratch`` (see ``SplitHeads``) and ``out``, which may be None, is not written."""
+    unscaled = None
+    if isinstance(qkv, UnscaledParts):
+        unscaled, qkv = qkv, qkv.parts
+        _f32(unscaled.ssq, "ssq", qkv.shape[1] * UNSCALED_MAX_SHARES)
+    merge = bool(merge) or num_splits == 1
     _dev(out, qkv, slot_mapping, q_weight, k_weight, cos_sin, k_pages, v_pages, block_tables, context_lens)
     _sinks_ok(sinks, nq)
     page_size = k_pages.shape[2]
     width = (nq + 2 * nkv) * head_dim
-    n = out.shape[0]
+    n = qkv.shape[-2]
     parts = qkv if qkv.dim() == 3 else None
-    _need(attn_decode_token_possible(out.dtype, head_dim, page_size, False, rotary_dim, cos_sin is not None),
+    _need(attn_decode_token_possible(k_pages.dtype, head_dim, page_size, False, rotary_dim, cos_sin is not None),
           "one launch takes bfloat16, head size 128, half-split pairs, a full rotation or none")
-    _need(out.shape == (n, nq * head_dim) and out.is_contiguous(), "out must be [tokens, nq * D]")
+    _need(not merge or (out is not None and out.shape == (n, nq * head_dim) and out.is_contiguous() and out.dtype == k_pages.dtype),
+          "out must be [tokens, nq * D]")
     _need(qkv.shape[-2:] == (n, width) and qkv.stride(-1) == 1 and qkv.stride(-2) == width,
           "qkv must be [tokens, (nq + 2 nkv) * D], or parts of that")
     _need(qkv.dtype == torch.bfloat16 if parts is None else qkv.dtype == torch.float32 and 1 <= qkv.shape[0] <= 4,
@@ -1494,7 +1617,7 @@ def attn_decode_token(out, qkv, slot_mapping, q_weight, k_weight, eps, cos_sin, 
     if cos_sin is not None:
         _f32(cos_sin, "cos_sin", n * rotary_dim)
     _i32(slot_mapping, "slot_mapping", n)
-    _check_pages(k_pages, v_pages, out.dtype, nkv, page_size, head_dim)
+    _check_pages(k_pages, v_pages, k_pages.dtype, nkv, page_size, head_dim)
     _i32(block_tables, "block_tables")
     _i32(context_lens, "context_lens", n)
     _need(block_tables.dim() == 2 and block_tables.shape[0] == n, "a block table row for every request")
@@ -1507,11 +1630,12 @@ def attn_decode_token(out, qkv, slot_mapping, q_weight, k_weight, eps, cos_sin, 
     lib = _attention_library(head_dim)
     _check(
         lib.jv_attn_decode_token(
-            _ptr(out), _ptr(qkv if parts is None else None), _ptr(parts), c_int(0 if parts is None else parts.shape[0]),
-            c_longlong(0 if parts is None else parts.stride(0)), _ptr(q_weight), _ptr(k_weight), c_float(eps), _ptr(cos_sin),
+            _ptr(out if merge else None), _ptr(qkv if parts is None else None), _ptr(parts), c_int(0 if parts is None else parts.shape[0]),
+            c_longlong(0 if parts is None else parts.stride(0)), _ptr(unscaled.ssq if unscaled else None),
+            c_int(qkv.shape[0] if unscaled else 0), c_int(unscaled.width if unscaled else 0), c_float(unscaled.eps if unscaled else 0.0), _ptr(q_weight), _ptr(k_weight), c_float(eps), _ptr(cos_sin),
             c_int(rotary_dim if cos_sin is not None else 0), _ptr(slot_mapping), _ptr(k_pages), _ptr(v_pages), _ptr(block_tables),
             c_int(block_tables.shape[1]), _ptr(context_lens), c_int(n), c_int(page_size), c_int(nq), c_int(nkv), c_float(scale),
-            c_int(window or 0), c_int(num_splits), _ptr(scratch if num_splits > 1 else None), _ptr(sinks), _stream()),
+            c_int(window or 0), c_int(num_splits), _ptr(scratch if num_splits > 1 else None), _ptr(sinks), c_int(merge), _stream()),
         "attn_decode_token",
     )
 

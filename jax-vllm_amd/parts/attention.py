@@ -219,6 +219,15 @@ class GroupedQueryAttention:
         """x goes into the qkv product and nowhere else: the norm before may leave its scale to that product."""
         return K.linear_takes_unscaled_rows(n_rows, self.w_qkv, partial_ok=self._qkv_parts_ok(), partial_max_width=None)
 
+    def takes_pending_rows(self, n_rows: int, ctx: StepContext, mem: LayerMemory) -> bool:
+        """Whether the qkv product may make its rows itself (``K.PendingRows``): only the launch behind it that goes from the product to the
+        attention applies the norm's scale to its parts."""
+        from . import attention_backend
+
+        rotary_dim, interleaved = self.rotation if self.rotation is not None else (0, False)
+        return (not self.wide and self.b_qkv is None and attention_backend.token_possible(self, ctx, mem, interleaved, rotary_dim)
+                and K.linear_takes_pending_rows(n_rows, self.w_qkv, partial_ok=self._qkv_parts_ok(), partial_max_width=None))
+
     # ---- one product with what else reads the same input (``parts/recurrent.py: ParallelMixer``)
     def input_weight(self):
         """The matrix of the one product this mixer begins with, or None where it has to make that product itself."""
@@ -250,10 +259,9 @@ class GroupedQueryAttention:
             K.add_bias(qkv, self.b_qkv)
         from . import attention_backend
 
-        out = torch.empty((n, self.nq * self.d), dtype=x.dtype, device=x.device)
         if attention_backend.token_possible(self, ctx, mem, interleaved, rotary_dim):
-            attention_backend.run_token(self, out, qkv, cos_sin, rotary_dim, ctx, mem)
-            return self._project(out)
+            return self._project(attention_backend.run_token(self, qkv, cos_sin, rotary_dim, ctx, mem))
+        out = torch.empty((n, self.nq * self.d), dtype=x.dtype, device=x.device)
         parts = None
         if qkv.dim() == 3:
             parts, qkv = qkv, torch.empty(qkv.shape[1:], dtype=x.dtype, device=x.device)

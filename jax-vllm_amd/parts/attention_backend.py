@@ -242,13 +242,18 @@ def _mfma_plan(att, ctx, window: int, keep: int, device) -> MfmaPlan:
     return plan
 
 
-def run_token(att, out, qkv, cos_sin, rotary_dim: int, ctx, mem) -> None:
-    """Head norms, rotation, page writes and attention of a step of single tokens; ``qkv``: the q/k/v product or its parts."""
+def run_token(att, qkv, cos_sin, rotary_dim: int, ctx, mem):
+    """Head norms, rotation, page writes and attention of a step of single tokens; ``qkv``: the q/k/v product or its parts.  Returns the
+    heads [tokens, nq * D], or ``K.SplitHeads`` where the output product merges them."""
     window = K.key_window(att.window, att.chunk)
-    plan = _mfma_plan(att, ctx, window, 0, out.device)
+    n, device = ctx.num_tokens, att.w_o.device
+    plan = _mfma_plan(att, ctx, window, 0, device)
+    merge = plan.num_splits == 1 or not K.linear_takes_split_heads(n, att.w_o, plan.num_splits)
+    out = torch.empty((n, att.nq * att.d), dtype=att.dtype, device=device) if merge else None
     K.attn_decode_token(out, qkv, ctx.slot_mappings[mem.group], att.q_norm, att.k_norm, att.qk_norm_eps or 0.0, cos_sin, rotary_dim,
                         mem.pages["k"], mem.pages["v"], ctx.block_tables[mem.group], ctx.context_lens, att.nq, att.nkv, att.d,
-                        att.scale, window, plan.num_splits, plan.scratch, sinks=att.sinks)
+                        att.scale, window, plan.num_splits, plan.scratch, sinks=att.sinks, merge=merge)
+    return out if merge else K.SplitHeads(plan.scratch, n, plan.num_splits, att.nq, att.d, att.sinks)
 
 
 def run(att, out, qkv, ctx, mem) -> None:

@@ -55,14 +55,37 @@ class PreNormBlock:
             return K.pending_scale(out, self.residual_scale)
         return out.settled() if isinstance(out, K.BiasedOutput) else out
 
+    def _made_by_readers(self, h, delta, mixer, feed_forward, ctx, mem) -> bool:
+        """Whether the products behind both norms make their rows themselves (one or two rows of a decode step)."""
+        n = h.shape[0]
+        if n > K.MADE_MAX_ROWS or not self.has_feed_forward or self.residual_scale != 1.0 or not all(hasattr(p, "pending") for p in self.norms):
+            return False
+        if delta is not None and not _float_parts(delta):
+            return False
+        ask = [getattr(p, "takes_pending_rows", None) for p in (mixer, feed_forward)]
+        return all(a is not None for a in ask) and ask[0](n, ctx, mem) and ask[1](n)
+
     def forward(self, h, delta, mixer, feed_forward, ctx, mem):
         n = h.shape[0]
+        if self._made_by_readers(h, delta, mixer, feed_forward, ctx, mem):
+            between = torch.empty_like(h)                              # the stream between the two sublayers: a product's blocks all read the old one
+            a = self._share(mixer.forward(self.mixer_norm.pending(h, delta, between), ctx, mem))
+            if _float_parts(a):
+                return self._share(feed_forward.forward(self.feed_forward_norm.pending(between, a, h), ctx))
+            y = _add_norm(self.feed_forward_norm, between, a, feed_forward, n)
+            h.copy_(between)
+            return self._share(feed_forward.forward(y, ctx))
         x = _add_norm(self.mixer_norm, h, delta, mixer, n)
         a = self._share(mixer.forward(x, ctx, mem))
         if not self.has_feed_forward:
             return a
         y = _add_norm(self.feed_forward_norm, h, a, feed_forward, n)
         return self._share(feed_forward.forward(y, ctx))
+
+
+def _float_parts(delta) -> bool:
+    """Whether a sublayer's output is a stack of at most four float partial products."""
+    return isinstance(delta, torch.Tensor) and delta.dim() == 3 and delta.dtype == torch.float32 and delta.shape[0] <= 4
 
 
 def _add_norm(norm, h, delta, reader, n_rows: int):

@@ -41,6 +41,10 @@ class GatedMLP:
         """x goes into the gate/up product and nowhere else: the norm before may leave its scale to that product."""
         return K.linear_takes_unscaled_rows(n_rows, self.w_gate_up, gate_pairs=True)
 
+    def takes_pending_rows(self, n_rows: int) -> bool:
+        """Whether the gate/up product may make its rows itself (``K.PendingRows``)."""
+        return K.linear_takes_pending_rows(n_rows, self.w_gate_up, gate_pairs=True)
+
     def forward(self, x, ctx=None) -> torch.Tensor:
         z = K.linear(x, self.w_gate_up, gate_pairs=self.activation)    # gate and up rows alternate in the fused weight
         return K.linear(z, self.w_down, partial_ok=self.partial_out)   # the next norm adds the partial products

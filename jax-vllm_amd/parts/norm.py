@@ -38,6 +38,10 @@ class RMSNorm:
         """Norm over the last axis of an activation tensor (any leading shape)."""
         return K.rmsnorm(x, self.weight, self.eps)
 
+    def pending(self, h: torch.Tensor, delta, out: torch.Tensor):
+        """``norm(h + delta)`` as rows that the product which reads them makes itself, the stream then in ``out``."""
+        return K.PendingRows(h, delta, self.weight, self.eps, out)
+
     def add_norm(self, h: torch.Tensor, delta, rows=None, unscaled_ok: bool = False):
         """The residual step fused with the norm: ``h += delta`` in the float residual stream,
         returns ``norm(h)`` in the activation type.  ``delta`` may be a ``K.PendingNorm``: then what is
