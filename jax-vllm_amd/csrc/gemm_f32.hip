@@ -113,6 +113,19 @@ __device__ __forceinline__ unsigned lds_address(const void* p) {
   return (unsigned)(unsigned long long)(const __attribute__((address_space(3))) void*)p;
 }
 
+// Waits for the oldest of a wave's rounds of L loads on their way: `left` rounds to go, this one among them, at most S of them asked for.
+template <int S, int L>
+__device__ __forceinline__ void wait_oldest(int left) {
+  if constexpr (S > 1) {
+    if (left >= S) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * L) : "memory");
+      return;
+    }
+    if constexpr (S > 2) return wait_oldest<S - 1, L>(left);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 // ---------------------------------------------------------------------------- few rows
 // A block takes TW rows of W by XR rows of A; its 8 waves share out the steps (waves 0 to 3 every fourth of the first half, 4 to
 // 7 of the second), each through a ring of its own in LDS, straight from memory, S steps on their way, no wave waiting for
@@ -173,8 +186,9 @@ gemm_f32_few_kernel(float* __restrict__ C, const float* __restrict__ A, const fl
       }
     }
   };
+  const int mine = (steps - turn + 3) / 4;      // this wave's steps
   if constexpr (DMA)
-    for (int v = 0; v < S; ++v) dma(v, v);
+    for (int v = 0; v < S; ++v) v < mine ? dma(v, v) : (void)0;
   else load_round(0);
   f32x4 sum = {0.f, 0.f, 0.f, 0.f};
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
@@ -194,7 +208,8 @@ gemm_f32_few_kernel(float* __restrict__ C, const float* __restrict__ A, const fl
       f32x4 raw[NT + MT][2];
       if constexpr (DMA) {
         const int i = s0 / 4 + r;
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * L) : "memory");
+        if (i >= mine) break;
+        wait_oldest<S, L>(mine - i);
         const float* b = ring + slot * BUF;
 #pragma unroll
         for (int t = 0; t < NT + MT; ++t) {
@@ -202,7 +217,7 @@ gemm_f32_few_kernel(float* __restrict__ C, const float* __restrict__ A, const fl
           raw[t][0] = *(const f32x4*)(at + p0), raw[t][1] = *(const f32x4*)(at + p1);
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // read before the slot is filled again
-        dma(i + S, slot);
+        if (i + S < mine) dma(i + S, slot);
         slot = slot + 1 == S ? 0 : slot + 1;
         const int k0 = (first + turn + 4 * i) * G32_STEP;
         if (k0 + G32_STEP > K) {      // zeros of A beyond K: what W repeats there does not count
@@ -235,12 +250,14 @@ gemm_f32_few_kernel(float* __restrict__ C, const float* __restrict__ A, const fl
     __builtin_amdgcn_s_barrier();      // (the buffer of the round before the last was read before the last round's barrier)
     asm volatile("" ::: "memory");
     if (turn < TILES) {
+      f32x4 part[4 * R];      // (behind the last step: what the buffer held, not added)
+#pragma unroll
+      for (int s = 0; s < 4 * R; ++s) part[s] = met[round][half][s][turn][lane];
 #pragma unroll
       for (int s = 0; s < 4 * R; ++s)
-        if (s0 + s < steps) sum += met[round][half][s][turn][lane];
+        if (s0 + s < steps) sum += part[s];
     }
   }
-  if constexpr (DMA) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // nothing on its way to this LDS when the block ends
   __syncthreads();
   if (half && turn < TILES) met[0][1][0][turn][lane] = sum;
   __syncthreads();
@@ -253,6 +270,118 @@ gemm_f32_few_kernel(float* __restrict__ C, const float* __restrict__ A, const fl
   for (int e = 0; e < 4; ++e)
     if (n + e < N) r[e] = settle(sum[e], A + (long long)m * K, W + (long long)(n + e) * K, K);
   leave(C, m, n, N, r, act);
+}
+
+// ---------------------------------------------------------------------------- up to 8 rows
+// A block takes 8 G rows of W by 8 rows of A.  Steps go in pairs: lanes 0 to 7 of an operand hold the rows of one step, lanes 8 to 15 those of
+// the next, and of the product the two quarters that belong together count.  So nothing is split or multiplied twice, as it would be for half
+// a tile of 16.  The 8 waves share out the pairs (waves 0 to 3 every fourth of the first half of the steps, 4 to 7 of the second), each through
+// a ring of its own, S pairs on their way; every step leaves its sums in LDS, and after C pairs of each wave they are added in their order.
+// What bounds few rows is a wave's chain from wait to sum (0.8 us a step of each wave with 16 x 16 tiles, which meet every two steps), not the
+// stream of W: hence smaller tiles on twice the units and one meeting for up to 64 pairs.  Straight into registers instead of the ring, a lane a
+// row (32 lines an instruction): 9.0 for 8.4.  Microseconds in graphs with cold weights, 16 x 16 or 32 x 16 tiles / these (rows of W): 8 rows
+// against 2,048 x 2,048 9.7 / 8.4 (8), 2,048 x 3,072 12.5 / 9.7 (8), 512 x 8,192 25.5 / 17.5 (8), 3,072 x 2,048 9.9 / 9.2 (16), 1,024 x 1,024 6.3 /
+// 5.5 (8), 6,144 x 2,048 14.5 / 14.0 (24), 6,144 x 8,192 51 / 45 (24), 32,000 x 2,048 54.6 / 55.2 (16): wide ones stay with 32 x 16.
+template <int G, int S, int C>
+__global__ void __launch_bounds__(512)
+gemm_f32_pairs_kernel(float* __restrict__ out, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K, JvAct act) {
+  constexpr int L = 2 * (G + 1), BUF = L * 256;      // loads of a pair, each 8 rows of a step, 1 KB
+  static_assert(G <= 4 && L * (S - 1) <= 63, "a wave adds what a block leaves; what s_waitcnt counts to");
+  __shared__ __attribute__((aligned(1024))) float bufs[8 * S * BUF];
+  __shared__ f32x4 met[2][8 * C][16 * G];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wave >> 2, turn = wave & 3;
+  const int li = lane & 15, lq = lane >> 4, odd = li >> 3, n0 = blockIdx.x * 8 * G;
+  const int total = (K + G32_STEP - 1) / G32_STEP, first = half ? (total + 1) / 2 : 0, steps = half ? total / 2 : (total + 1) / 2;
+  const int longest = ((total + 1) / 2 + 7) / 8;      // pairs of the wave that has the most
+  const int mine = ((steps + 1) / 2 - turn + 3) / 4;
+  // piece c of row r lies at slot c ^ r; a row's last step may have fewer pieces than 8: the last one again for those
+  const int piece = ((lane & 7) ^ (lane >> 3)) * 16, beyond = max(piece + 16 - (K * 4 - (total - 1) * G32_STEP * 4), 0);
+  unsigned off[G + 1];
+#pragma unroll
+  for (int t = 0; t <= G; ++t) {      // rows behind the last one repeat it
+    const int r = lane >> 3, at = t < G ? min(n0 + t * 8 + r, N - 1) - n0 : min(r, M - 1);
+    off[t] = (unsigned)at * (unsigned)(K * 4) + piece;
+  }
+  const float* ws = W + (long long)n0 * K;
+  float* ring = bufs + wave * S * BUF;
+  const unsigned lds0 = lds_address(ring);
+  auto dma = [&](int i, int slot) {      // the wave's pair i; behind the last step that one again
+#pragma unroll
+    for (int o = 0; o < 2; ++o) {
+      const int s = min(first + 2 * (turn + 4 * i) + o, total - 1), less = s == total - 1 ? beyond : 0;
+#pragma unroll
+      for (int t = 0; t <= G; ++t) lds_load(off[t] - less, (t < G ? ws : A) + s * G32_STEP, lds0 + slot * (BUF * 4) + (2 * t + o) * 1024);
+    }
+  };
+  const int at0 = odd * 256 + (li & 7) * G32_STEP, p0 = at0 + ((2 * lq) ^ (li & 7)) * 4, p1 = at0 + ((2 * lq + 1) ^ (li & 7)) * 4;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int v = 0; v < S; ++v)
+    if (v < mine) dma(v, v);
+  f32x4 sum = zero;
+  int slot = 0;
+  for (int c0 = 0; c0 < longest; c0 += C) {
+    const int stop = min(c0 + C, longest);
+    for (int i = c0; i < stop; ++i) {
+      if (i >= mine) break;
+      wait_oldest<S, L>(mine - i);
+      const float* b = ring + slot * BUF;
+      f32x4 raw[G + 1][2];
+#pragma unroll
+      for (int t = 0; t <= G; ++t) raw[t][0] = *(const f32x4*)(b + t * 512 + p0), raw[t][1] = *(const f32x4*)(b + t * 512 + p1);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // read before the slot is filled again
+      if (i + S < mine) dma(i + S, slot);
+      slot = slot + 1 == S ? 0 : slot + 1;
+      const int s = 2 * (turn + 4 * i);
+      if ((first + s + 2) * G32_STEP > K) {      // zeros of A beyond K: what W repeats there does not count
+        const int k = (first + s + odd) * G32_STEP + lq * 8;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          if (k + h * 4 >= K) raw[G][h] = zero;
+      }
+      u32x4 wt[G][3], xt[3];
+      split8(raw[G], xt);
+#pragma unroll
+      for (int g = 0; g < G; ++g) split8(raw[g], wt[g]);
+      f32x4 t[G];
+#pragma unroll
+      for (int e = 0; e < G32_PRODUCTS; ++e)
+#pragma unroll
+        for (int g = 0; g < G; ++g) t[g] = mfma(wt[g][G32_W[e]], xt[G32_X[e]], e ? t[g] : zero);
+      f32x4* to = &met[half][(i - c0) * 8 + 2 * turn + odd][(li & 7) * 2 + (lq & 1)];
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        if ((lq >> 1) == odd) to[g * 16] = t[g];
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (turn == 0 && lane < 16 * G) {
+      const int count = min(8 * C, steps - 8 * c0);
+      for (int s = 0; s < count; s += 8) {
+        f32x4 part[8];      // (behind the last step: what the buffer held, not added)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) part[u] = met[half][s + u][lane];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (s + u < count) sum += part[u];
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();      // read before the next sums are left there
+    asm volatile("" ::: "memory");
+  }
+  if (half && turn == 0 && lane < 16 * G) met[1][0][lane] = sum;
+  __syncthreads();
+  if (wave || lane >= 16 * G) return;
+  sum += met[1][0][lane];
+  const int m = lane % 16 / 2, n = n0 + lane / 16 * 8 + lane % 2 * 4;      // a lane holds C[m][n .. n + 3]
+  if (m >= M) return;
+  float r[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (n + e < N) r[e] = settle(sum[e], A + (long long)m * K, W + (long long)(n + e) * K, K);
+  leave(out, m, n, N, r, act);
 }
 
 // ---------------------------------------------------------------------------- many rows
@@ -587,11 +716,17 @@ gemm_f32_rows_kernel(float* __restrict__ C, const unsigned* __restrict__ X, cons
 }
 
 // How C is made (jv_gemm_f32): 0, 1: few rows, 16 x 16 or 32 x 32, through registers; 2 to 4: few rows through the ring, 16 x 16, 32 x 16, 32 x 32
-// (rows of W x rows of A); 5 to 7 tiles of 128 rows of A by 128, 96, 64 of W, 8 to 10 of 64 rows by 96, 64, 32.
+// (rows of W x rows of A), for up to 8 rows of A in pairs of steps with form 2 (8 rows of W while their blocks go to 256 units at once, else 16)
+// and form 4 (24); 5 to 7 tiles of 128 rows of A by 128, 96, 64 of W, 8 to 10 of 64 rows by 96, 64, 32.
 template <int TW, int XR, int S, int R, bool DMA>
 static int few_launch(float* C, const float* A, const float* W, int M, int N, int K, JvAct act, hipStream_t s) {
   if ((M + XR - 1) / XR > 65535) return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL((gemm_f32_few_kernel<TW, XR, S, R, DMA>), dim3((N + TW - 1) / TW, (M + XR - 1) / XR), dim3(512), 0, s, C, A, W, M, N, K, act);
+  return JV_LAUNCH_CHECK();
+}
+template <int G, int S, int C>
+static int pairs_launch(float* out, const float* A, const float* W, int M, int N, int K, JvAct act, hipStream_t s) {
+  hipLaunchKernelGGL((gemm_f32_pairs_kernel<G, S, C>), dim3((N + 8 * G - 1) / (8 * G)), dim3(512), 0, s, out, A, W, M, N, K, act);
   return JV_LAUNCH_CHECK();
 }
 template <int TM, int TW>
@@ -660,9 +795,11 @@ extern "C" int jv_gemm_f32(float* C, const float* A, const float* W, const void*
   switch (form) {
     case 0: return few_launch<16, 16, 1, 2, false>(C, A, W, M, N, K, act, s);
     case 1: return few_launch<32, 32, 1, 1, false>(C, A, W, M, N, K, act, s);
-    case 2: return few_launch<16, 16, 2, 2, true>(C, A, W, M, N, K, act, s);
+    case 2:
+      if (M > 8) return few_launch<16, 16, 2, 2, true>(C, A, W, M, N, K, act, s);
+      return N <= 8 * 256 ? pairs_launch<1, 2, 8>(C, A, W, M, N, K, act, s) : pairs_launch<2, 1, 4>(C, A, W, M, N, K, act, s);
     case 3: return few_launch<32, 16, 1, 1, true>(C, A, W, M, N, K, act, s);
-    case 4: return few_launch<32, 32, 1, 1, true>(C, A, W, M, N, K, act, s);
+    case 4: return M > 8 ? few_launch<32, 32, 1, 1, true>(C, A, W, M, N, K, act, s) : pairs_launch<3, 1, 2>(C, A, W, M, N, K, act, s);
     case 5: return rows_launch<128>(C, X, A, W, M, N, K, KA, act, s);
     case 6: return rows_launch<96>(C, X, A, W, M, N, K, KA, act, s);
     case 7: return rows_launch<64>(C, X, A, W, M, N, K, KA, act, s);

@@ -796,6 +796,10 @@ F32_STEP = 32         # columns of a step of the 32-bit product
 # tiles of the 32-bit product: form, rows of a, rows of w, microseconds of a round per 1,024 columns on one unit and on all
 _F32_TILES = ((5, 128, 128, 23.5, 38.3), (6, 128, 96, 19.6, 30.8), (7, 128, 64, 11.6, 23.2), (8, 64, 96, 16.7, 22.2), (9, 64, 64, 11.2, 16.3),
               (10, 64, 32, 4.0, 10.0))
+# Up to 8 rows: form, rows of w a block, blocks at once, and what a round and the stream of w take, fitted to 297 sizes (1, 4 and 8 rows, n 512 to
+# 65,536, k 512 to 12,288): on the average 2 % from the best (25 % at 1 x 12,288 x 8,192), 0.69 to 1.04 of the time of 16 x 16 and 32 x 16 tiles by the count for more rows.
+_F32_PAIRS = ((2, 8, 256, 2.3, 1.3, 1.7, 2.05, 4.0, 7.2), (2, 16, 512, 2.75, 0.6, 1.95, 5.0, 4.1, 5.05), (3, 32, 512, 0.8, 2.6, 4.15, 7.8, 3.6, 5.2),
+              (4, 24, 256, 1.7, 1.75, 2.8, 4.2, 4.0, 5.1))
 _F32_FRAGMENTS = 8    # forms below take the terms of a in the order of the matrix unit's operands
 
 
@@ -803,7 +807,7 @@ _F32_FRAGMENTS = 8    # forms below take the terms of a in the order of the matr
 def f32_plan(m: int, n: int, k: int, pieces: bool = True, a_pieces: bool = True) -> int:
     """Form of the 32-bit product (``jv_gemm_f32``).  All give the same bits, so it is the one that takes the least time by a count of
     rounds over 256 units, fitted to 199 sizes (17 to 2,048 rows, n 1,024 to 32,000, k 512 to 12,288, in graphs with cold weights): within 2 %
-    of the best form at all of them but 33 to 64 rows of 8,192 x 1,024 (20 %); for example k = 2,048: 5 x 2,048 9.6 us (form 2), 16 x 32,000 57 (3),
+    of the best form at all of them but 33 to 64 rows of 8,192 x 1,024 (20 %); for example k = 2,048: 5 x 2,048 8.4 us (form 2), 16 x 32,000 57 (3),
     37 x 3,072 17.1 (4), 100 x 6,144 39.6 (9; 4 takes 48), 250 x 6,144 48 (7), 1,003 x 6,144 152 (6), 2,048 x 2,048 100 (5).
     ``pieces``: rows of w begin on 16 bytes (else they are copied for tiles, and few rows go through registers); ``a_pieces``: rows of a too."""
     q, mb = k / 1024, n * k * 4e-6
@@ -816,6 +820,11 @@ def f32_plan(m: int, n: int, k: int, pieces: bool = True, a_pieces: bool = True)
         return -(-b // slots) * (fixed + (one + (full - one) * min(1.0, b / slots)) * q)
 
     times, through_ring = {}, pieces and a_pieces and 0 < k <= 1 << 24
+    if m <= 8 and through_ring:
+        for form, tw, slots, start, fixed, one, full, first, rate in _F32_PAIRS:
+            if form != 2 or (n <= 2048) == (tw == 8):
+                times[form] = max(start + rounds(8, tw, fixed, one, full, slots), first + mb / rate)
+        return min(times, key=times.get)
     if m <= 65535 * 16:                                           # the grid's rows
         if through_ring:
             times[2] = max(3 + rounds(16, 16, 1.3, 2.3, 3.2), 5 + mb / 4.2)
