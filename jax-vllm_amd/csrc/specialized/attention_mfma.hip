@@ -1228,7 +1228,7 @@ __global__ void __launch_bounds__(64 * DEC_WAVES) PREFILL_OCCUPANCY attn_decode_
   // pieces of 16 bytes instead of 8, microseconds (before): 64 requests of 512 to 1,536 keys 57.6 (58.5), one of 1,030 keys in 8 splits
   // with its merge 9.9 (10.4), 16 of 400 to 1,200 over 4 kv heads in 4 splits 12.6 (13.3), head size 256, 8 over one 15.5 (16.6).
   const int heads = p.nkv * mt_per_head, w = blockIdx.x / heads, at = blockIdx.x - w * heads;
-  // Without a work list the requests are 0, 1, ... and request r's token is row r (a step of
+  // Without cu_seqlens request r's token is row r, without a work list the requests are 0, 1, ... (a step of
   // decoded tokens only): nothing has to be looked up before the loads below can start.  The
   // kernel's time at small batches is its chain of dependent memory round trips (~1.5 us each
   // for data the previous kernel wrote), so the request's page table row is copied to LDS at
@@ -1787,13 +1787,13 @@ extern "C" int jv_attn_decode(void* out, const void* q, long long q_row_stride, 
 #ifdef JV_DECODE_FUSED
 // The same from the q/k/v product of a step of single tokens, request r's in row r: per-head norm (with weights), rotation (with a
 // table; half-split pairs, rotary_dim a multiple of 128), the new keys and values into their pages, attention, in one launch.
-// `parts` (n_parts 1..4) or, with null, bf16 rows `qkv`.  row_sq (parts only; [tokens][16], sq_shares of them, or null): the rows' norm over
+// `work`: the requests in the order of their blocks, or null.  `parts` (n_parts 1..4) or, with null, bf16 rows `qkv`.  row_sq (parts only; [tokens][16], sq_shares of them, or null): the rows' norm over
 // sq_width columns is still to be applied.  merge 0: where num_splits > 1 the splits' results stay in scratch, [request][head][split][D]
 // and behind them (max, sum) each, and `out` is not written.
 extern "C" int jv_attn_decode_token(void* out, const void* qkv, const float* parts, int n_parts, long long part_stride,
                                     const float* row_sq, int sq_shares, int sq_width, float sq_eps, const float* q_weight,
                                     const float* k_weight, float eps, const float* cos_sin, int rotary_dim, const int* slot_mapping, void* k_pages, void* v_pages, const int* block_tables, int table_stride,
-                                    const int* context_lens, int n_work, int page_size, int nq, int nkv, float scale, int window,
+                                    const int* context_lens, const int* work, int n_work, int page_size, int nq, int nkv, float scale, int window,
                                     int num_splits, float* scratch, const float* sinks, int merge, void* stream) {
   if (n_work <= 0) return 0;
   if (row_sq && (!parts || sq_shares < 1 || sq_shares > 16 || sq_width <= 0)) return (int)hipErrorInvalidValue;
@@ -1807,7 +1807,7 @@ extern "C" int jv_attn_decode_token(void* out, const void* qkv, const float* par
   a.k_pages = (const bf16_t*)k_pages; a.v_pages = (const bf16_t*)v_pages;
   a.k_pages_out = (bf16_t*)k_pages; a.v_pages_out = (bf16_t*)v_pages;
   a.block_tables = block_tables; a.table_stride = table_stride;
-  a.context_lens = context_lens;
+  a.context_lens = context_lens; a.work = work;
   a.page_size = page_size; a.nq = nq; a.nkv = nkv;
   a.window = window;
   a.num_splits = num_splits;

@@ -1589,6 +1589,21 @@ def attn_decode_mfma(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_se
     )
 
 
+DECODE_ORDER_MAX = 1024
+
+
+def decode_order(context_lens: torch.Tensor, at_once: int, window: int = 0) -> torch.Tensor:
+    """int32 [n]: the requests of a step of single tokens in the order in which the blocks of ``attn_decode_mfma`` or ``attn_decode_token``
+    (their ``work``) best take them, ``at_once`` requests' blocks going to the compute units at once."""
+    _dev(context_lens)
+    n = context_lens.numel()
+    _i32(context_lens, "context_lens", n)
+    _need(n <= DECODE_ORDER_MAX and at_once >= 1, f"up to {DECODE_ORDER_MAX} requests, at least one at once")
+    order = torch.empty(n, dtype=torch.int32, device=context_lens.device)
+    _check(library.core().jv_decode_order(_ptr(order), _ptr(context_lens), c_int(n), c_int(at_once), c_int(window or 0), _stream()), "decode_order")
+    return order
+
+
 def attn_decode_token_possible(dtype, head_dim: int, page_size: int, interleaved: bool, rotary_dim: int, rotated: bool) -> bool:
     """Whether ``attn_decode_token`` takes a step of single tokens of these heads."""
     return (mfma_attention_supported(dtype, head_dim, page_size) and head_dim == 128
@@ -1596,11 +1611,13 @@ def attn_decode_token_possible(dtype, head_dim: int, page_size: int, interleaved
 
 
 def attn_decode_token(out, qkv, slot_mapping, q_weight, k_weight, eps, cos_sin, rotary_dim, k_pages, v_pages, block_tables,
-                      context_lens, nq, nkv, head_dim, scale, window=0, num_splits=1, scratch=None, sinks=None, merge: bool = True) -> None:
+                      context_lens, nq, nkv, head_dim, scale, window=0, num_splits=1, scratch=None, sinks=None, merge: bool = True,
+                      work=None) -> None:
     """``qk_norm_rope_write`` and ``attn_decode_mfma`` of a step of single tokens (request r's in row r) in one launch: ``qkv`` is
     the q/k/v product, bfloat16 rows or float32 parts [1..4, tokens, (nq + 2 nkv) * D]; new keys and values go to their pages
     where ``slot_mapping`` is not negative.  ``UnscaledParts`` are scaled here.  ``merge`` False: with ``num_splits`` > 1 the splits' results
-    stay in ``scratch`` (see ``SplitHeads``) and ``out``, which may be None, is not written."""
+    stay in ``scratch`` (see ``SplitHeads``) and ``out``, which may be None, is not written.  ``work``: int32 [tokens], every request
+    once: the order of their blocks (``decode_order``)."""
     unscaled = None
     if isinstance(qkv, UnscaledParts):
         unscaled, qkv = qkv, qkv.parts
@@ -1630,6 +1647,9 @@ def attn_decode_token(out, qkv, slot_mapping, q_weight, k_weight, eps, cos_sin, 
     _i32(block_tables, "block_tables")
     _i32(context_lens, "context_lens", n)
     _need(block_tables.dim() == 2 and block_tables.shape[0] == n, "a block table row for every request")
+    if work is not None:
+        _dev(work)
+        _i32(work, "work", n)
     least = attn_decode_min_splits(block_tables.shape[1], page_size)
     _need(num_splits >= least, f"block tables of {block_tables.shape[1]} pages need at least {least} splits")
     if num_splits > 1:
@@ -1643,7 +1663,7 @@ def attn_decode_token(out, qkv, slot_mapping, q_weight, k_weight, eps, cos_sin, 
             c_longlong(0 if parts is None else parts.stride(0)), _ptr(unscaled.ssq if unscaled else None),
             c_int(qkv.shape[0] if unscaled else 0), c_int(unscaled.width if unscaled else 0), c_float(unscaled.eps if unscaled else 0.0), _ptr(q_weight), _ptr(k_weight), c_float(eps), _ptr(cos_sin),
             c_int(rotary_dim if cos_sin is not None else 0), _ptr(slot_mapping), _ptr(k_pages), _ptr(v_pages), _ptr(block_tables),
-            c_int(block_tables.shape[1]), _ptr(context_lens), c_int(n), c_int(page_size), c_int(nq), c_int(nkv), c_float(scale),
+            c_int(block_tables.shape[1]), _ptr(context_lens), _ptr(work), c_int(n), c_int(page_size), c_int(nq), c_int(nkv), c_float(scale),
             c_int(window or 0), c_int(num_splits), _ptr(scratch if num_splits > 1 else None), _ptr(sinks), c_int(merge), _stream()),
         "attn_decode_token",
     )

@@ -242,6 +242,20 @@ def _mfma_plan(att, ctx, window: int, keep: int, device) -> MfmaPlan:
     return plan
 
 
+def _decode_work(ctx, plan, att, window: int):
+    """The order of a step's decoding requests: the plan's list, or by their lengths where a step of single tokens gives units blocks of more than
+    one request and 512 keys or more (shorter ones differ by less than the look-up takes)."""
+    heads = att.nkv * (-(-(att.nq // att.nkv) // 16))
+    at_once = TARGET_BLOCKS // heads
+    if (not ctx.decode_only or plan.num_splits > 1 or not 0 < at_once < plan.n_decode <= K.DECODE_ORDER_MAX
+            or keys_seen(ctx.max_kv_len, window) < 512):
+        return plan.decode_work
+    key = ("decode_order", at_once, window)      # a result of the device: made anew in every step, also a replayed one
+    if key not in ctx.extras:
+        ctx.extras[key] = K.decode_order(ctx.context_lens, at_once, window)
+    return ctx.extras[key]
+
+
 def run_token(att, qkv, cos_sin, rotary_dim: int, ctx, mem):
     """Head norms, rotation, page writes and attention of a step of single tokens; ``qkv``: the q/k/v product or its parts.  Returns the
     heads [tokens, nq * D], or ``K.SplitHeads`` where the output product merges them."""
@@ -252,7 +266,7 @@ def run_token(att, qkv, cos_sin, rotary_dim: int, ctx, mem):
     out = torch.empty((n, att.nq * att.d), dtype=att.dtype, device=device) if merge else None
     K.attn_decode_token(out, qkv, ctx.slot_mappings[mem.group], att.q_norm, att.k_norm, att.qk_norm_eps or 0.0, cos_sin, rotary_dim,
                         mem.pages["k"], mem.pages["v"], ctx.block_tables[mem.group], ctx.context_lens, att.nq, att.nkv, att.d,
-                        att.scale, window, plan.num_splits, plan.scratch, sinks=att.sinks, merge=merge)
+                        att.scale, window, plan.num_splits, plan.scratch, sinks=att.sinks, merge=merge, work=_decode_work(ctx, plan, att, window))
     return out if merge else K.SplitHeads(plan.scratch, n, plan.num_splits, att.nq, att.d, att.sinks)
 
 
@@ -286,5 +300,5 @@ def run(att, out, qkv, ctx, mem) -> None:
                             window, sinks=sinks, cap=cap, keep=keep, one_group=plan.one_group)
     if plan.n_decode:
         K.attn_decode_mfma(out, qkv, q_row_stride, mem.pages["k"], mem.pages["v"], tables, ctx.cu_seqlens,
-                           ctx.context_lens, plan.decode_work, plan.n_decode, att.nq, att.nkv, att.d, att.scale,
+                           ctx.context_lens, _decode_work(ctx, plan, att, window), plan.n_decode, att.nq, att.nkv, att.d, att.scale,
                            window, plan.num_splits, plan.scratch, sinks=sinks, cap=cap, keep=keep)
