@@ -11,6 +11,11 @@
 // tiles are not full.  2,048 tokens, gate/up + down, microseconds (before: one buffer through registers, 64 rows of W):
 //   32 experts x 512, 4 chosen, width 2,048:    85 + 50   (96 + 76)
 //   64 experts x 1,024, 8 chosen, width 4,096: 478 + 296  (570 + 439)
+// What a block begins and ends with weighs as much as a third of its chunks (17 us at one chunk of 64, 0.95 us for each further): the weights of its
+// rows are not waited for at the start, and its results leave through LDS in whole lines.  Before / so, tiles of 192 rows, 2,048 tokens:
+// 32 x 512, 4 chosen, width 2,048 62.0 + 56.1 / 59.7 + 48.5; 64 x 1,024, 8 chosen, 4,096 tokens, width 4,096 660 + 413 / 634 + 399; tiles of 128, 32 x 768
+// 98.4 + 67.3 / 91.7 + 65.6; of 64, 1,003 tokens 48.5 + 31.7 / 47.9 + 31.7.  Not better: the ring by 4 waves of 96 x 128 (0.81 us a
+// chunk, but 24 us at one: 65.6 + 51.2; 398 + 256 for 432 + 251 at 64 x 1,024 and 2,048 tokens only).
 // Not better: 128 rows of W and two blocks a unit 83 + 50, 495 + 300; a wave for 64 x 128 (one a SIMD: nothing overlaps its own
 // reads) 134 + 71, 626 + 358; a register copy of row tiles to skip empty ones 87 + 56.
 //   MM_GATED:  z[pos] = act(w g) * (w u), g = Wg[e] x[token], u = Wu[e] x[token]    (bf16)
@@ -60,12 +65,13 @@ moe_mfma_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, const
   const int rows = min(TM, offsets[e + 1] - row0);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n0 = (pair - tile * per_tile) * NB;
+  float mine = 1.f;
   if (tid < TM) {                           // rows beyond the tile repeat its last row
     const int s = order[row0 + min(tid, rows - 1)];
     const int token = s / top;
     from[tid] = BY_TOKEN ? token : row0 + min(tid, rows - 1);
     to[tid] = (MODE == MM_DOWN ? (long long)(s - token * top) * n_tokens + token : (long long)(row0 + tid)) * N;
-    wts[tid] = use_weight ? weights[s] : 1.f;
+    if (use_weight) mine = weights[s];      // not waited for until the sums are there
   }
   __syncthreads();
 
@@ -199,27 +205,51 @@ moe_mfma_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, const
     }
   }
   }
-  // a lane holds column l32 of both tiles of W, rows 8 q + 4 half + i of each tile of x
+  // The sums go through LDS, 32 rows of both halves of x at a time, so that a thread leaves 4 neighbouring columns: the activation's code is
+  // there once instead of once for every number a lane holds, and a row is written in whole lines.
+  constexpr int ROW = TW + 4, THREADS = 2 * TW;      // floats of a row there: 4 rows further on lie half the banks further on
+  static_assert(64 * ROW * 4 <= (RING ? SLOTS * HALF : BUFS * BUF) * 2, "");
+  float* const stage = (float*)bufs;
+  const bool fours = N % 4 == 0 && ((unsigned long long)out & 15) == 0;
+  if (tid < TM) wts[tid] = mine;
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+  for (int mt = 0; mt < MT; ++mt) {
+    __syncthreads();
+    // a lane holds column l32 of both tiles of W, rows 8 q + 4 half + i of a tile of x
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int m = wm * (TM / 2) + mt * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
-      if (m >= rows) continue;
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        stage[(wm * 32 + (i >> 2) * 8 + half * 4 + (i & 3)) * ROW + wn * 64 + a * 32 + l32] = acc[a][mt][i];
+    __syncthreads();
+#pragma unroll 1
+    for (int q = tid; q < 64 * NB / 4; q += THREADS) {
+      const int r = q / (NB / 4), o = (q - r * (NB / 4)) * 4, m = (r >> 5) * (TM / 2) + mt * 32 + (r & 31), n = n0 + o;
+      if (m >= rows || n >= N) continue;
       const float w = wts[m];
-      if (GATED) {
-        const int n = n0 + wn * 32 + l32;
-        if (n < N) ((bf16_t*)out)[to[m] + n] = from_f32<bf16_t>(jv_gated(act, acc[0][mt][i] * w, acc[1][mt][i] * w));
+      const long long at = to[m] + n;
+      const f32x4 v = *(const f32x4*)(stage + r * ROW + (GATED ? (o >> 5) * 64 + (o & 31) : o)) * w;
+      if constexpr (MODE == MM_DOWN) {
+        if (fours) *(f32x4*)((float*)out + at) = v;
+        else
+          for (int k = 0; k < 4 && n + k < N; ++k) ((float*)out)[at + k] = v[k];
       } else {
+        typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+        bf16x4 y;
+        if constexpr (GATED) {
+          const f32x4 u = *(const f32x4*)(stage + r * ROW + (o >> 5) * 64 + 32 + (o & 31)) * w;
 #pragma unroll
-        for (int a = 0; a < 2; ++a) {
-          const int n = n0 + wn * 64 + a * 32 + l32;
-          if (n >= N) continue;
-          if (MODE == MM_PLAIN) ((bf16_t*)out)[to[m] + n] = from_f32<bf16_t>(jv_act(act.id, acc[a][mt][i] * w));
-          else ((float*)out)[to[m] + n] = acc[a][mt][i] * w;
+          for (int k = 0; k < 4; ++k) y[k] = from_f32<bf16_t>(jv_gated(act, v[k], u[k]));
+        } else {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) y[k] = from_f32<bf16_t>(jv_act(act.id, v[k]));
         }
+        if (fours) *(bf16x4*)((bf16_t*)out + at) = y;
+        else
+          for (int k = 0; k < 4 && n + k < N; ++k) ((bf16_t*)out)[at + k] = y[k];
       }
     }
+  }
 }
 
 template <int MODE, int TM, int TW, int BUFS>
