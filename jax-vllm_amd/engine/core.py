@@ -285,18 +285,17 @@ class EngineCore:
             # first use: run the launches eagerly (this is the step's result), then record them
             ctx = g.context(ps, self.page_size * max(widths, default=1))
             logits = self.model.forward(g.dev_segment("tokens"), ctx, self.memories, g.dev_segment("rows"))
-            g.logits = torch.empty_like(logits)
-            g.logits.copy_(logits)
             torch.cuda.synchronize()
             graph = torch.cuda.CUDAGraph()
             ctx.extras = {}   # per-step kernel results are recomputed inside the graph; plans stay
             with torch.cuda.graph(graph):
-                out = self.model.forward(g.dev_segment("tokens"), ctx, self.memories, g.dev_segment("rows"))
-                g.logits.copy_(out)
+                # held here, so nothing else the graph makes takes its place: every replay leaves its logits in it (a copy
+                # beside it cost 14 us at 64 rows of 151,936 columns)
+                g.logits = self.model.forward(g.dev_segment("tokens"), ctx, self.memories, g.dev_segment("rows"))
             g.graph, g.ctx = graph, ctx
-        else:
-            g.graph.replay()
-            self.graph_replays += 1
+            return logits[:r]
+        g.graph.replay()
+        self.graph_replays += 1
         return g.logits[:r]
 
     def _state_rows(self, slots) -> list:
