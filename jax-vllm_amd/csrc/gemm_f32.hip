@@ -15,11 +15,9 @@
 // one among them, are then whole.  A sum that is not finite may come from the split (2^80 of the true sum, a value near the
 // largest float, infinity less itself): it is made again from the numbers themselves.
 //
-// Microseconds, before with the 32-bit instruction, both before the scaling: 5 rows against 2,048 x 2,048 10.9 -> 8.8, 6,144 x 2,048 16.4 ->
-// 13.3 (50 MB: the stream of W); 16 rows 13.5 -> 9.1, 18.5 -> 13.4; 300 x 6,144 x 2,048 121 -> 75; 1,003 x 6,144 x 2,048 226 -> 150 with the 5 that
-// the terms of A take; 2,048 x 24,576 x 4,096 3,430 -> 2,222.  The scaling takes 1 to 5 % (24 sizes in graphs with cold weights, in turn,
-// without / with: the same sizes 9.2 / 9.6, 14.6 / 15.0; 9.5 / 9.9, 15.0 / 15.6; 78 / 81; 166 / 172; 2,308 / 2,340 = 176 TFLOP/s of 32-bit
-// products, 1.06 PFLOP/s of the matrix unit's).
+// Microseconds in graphs with cold weights, as first built (tiles of 16, 32 and 64 rows) / now: 5 rows against 2,048 x 2,048 9.6 / 8.4, 6,144 x 2,048 15.0 /
+// 13.9 (50 MB: the stream of W); 300 x 6,144 x 2,048 74 / 64; 1,003 x 6,144 x 2,048 156 / 152 with what the terms of A take; 2,048 x 24,576 x 4,096
+// 2,385 / 2,070 = 199 TFLOP/s of 32-bit products, 1.2 PFLOP/s of the matrix unit's.  The scaling takes 1 to 5 % of it (24 sizes).
 #include "common.h"
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));

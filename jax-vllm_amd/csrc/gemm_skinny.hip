@@ -384,13 +384,13 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
   bf16x8 b[MT][NL];
   if constexpr (SRC == ROWS_GIVEN) {
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int i = 0; i < NL; ++i) {
-      const int k = k0 + i * 32, m = min(mt * 16 + li, M - 1);
-      const bf16x8 v = *(const bf16x8*)(x + (long long)m * ldx + (EDGE ? min(k, K - 8) : k));
-      b[mt][i] = (!EDGE || k < K) ? v : zero;
-    }
+      for (int i = 0; i < NL; ++i) {
+        const int k = k0 + i * 32, m = min(mt * 16 + li, M - 1);
+        const bf16x8 v = *(const bf16x8*)(x + (long long)m * ldx + (EDGE ? min(k, K - 8) : k));
+        b[mt][i] = (!EDGE || k < K) ? v : zero;
+      }
   }
   // a tile beyond the last (the prefetch after the last tile) reads the first pieces of W, the same for all lanes
   // the scale of this lane's output row (wave mt adds row tile mt): asked for now, used after the first tile;
