@@ -1789,7 +1789,7 @@ extern "C" int jv_attn_decode(void* out, const void* q, long long q_row_stride, 
 // table; half-split pairs, rotary_dim a multiple of 128), the new keys and values into their pages, attention, in one launch.
 // `work`: the requests in the order of their blocks, or null.  `parts` (n_parts 1..4) or, with null, bf16 rows `qkv`.  row_sq (parts only; [tokens][16], sq_shares of them, or null): the rows' norm over
 // sq_width columns is still to be applied.  merge 0: where num_splits > 1 the splits' results stay in scratch, [request][head][split][D]
-// and behind them (max, sum) each, and `out` is not written.
+// and behind them (max, sum) each, and `out` is not written; not with `work`, in whose order they would lie there.
 extern "C" int jv_attn_decode_token(void* out, const void* qkv, const float* parts, int n_parts, long long part_stride,
                                     const float* row_sq, int sq_shares, int sq_width, float sq_eps, const float* q_weight,
                                     const float* k_weight, float eps, const float* cos_sin, int rotary_dim, const int* slot_mapping, void* k_pages, void* v_pages, const int* block_tables, int table_stride,
@@ -1797,6 +1797,7 @@ extern "C" int jv_attn_decode_token(void* out, const void* qkv, const float* par
                                     int num_splits, float* scratch, const float* sinks, int merge, void* stream) {
   if (n_work <= 0) return 0;
   if (row_sq && (!parts || sq_shares < 1 || sq_shares > 16 || sq_width <= 0)) return (int)hipErrorInvalidValue;
+  if (work && !merge && num_splits > 1) return (int)hipErrorInvalidValue;
   if ((parts && (n_parts < 1 || n_parts > 4)) || (!parts && !qkv) || !slot_mapping || (cos_sin && (rotary_dim % 128 || rotary_dim > D || rotary_dim <= 0)))
     return (int)hipErrorInvalidValue;
   AttnArgs a{};

@@ -1617,7 +1617,7 @@ def attn_decode_token(out, qkv, slot_mapping, q_weight, k_weight, eps, cos_sin, 
     the q/k/v product, bfloat16 rows or float32 parts [1..4, tokens, (nq + 2 nkv) * D]; new keys and values go to their pages
     where ``slot_mapping`` is not negative.  ``UnscaledParts`` are scaled here.  ``merge`` False: with ``num_splits`` > 1 the splits' results
     stay in ``scratch`` (see ``SplitHeads``) and ``out``, which may be None, is not written.  ``work``: int32 [tokens], every request
-    once: the order of their blocks (``decode_order``)."""
+    once: the order of their blocks (``decode_order``); not with results that stay in ``scratch``, which lie there in the order of the blocks."""
     unscaled = None
     if isinstance(qkv, UnscaledParts):
         unscaled, qkv = qkv, qkv.parts
@@ -1650,6 +1650,7 @@ def attn_decode_token(out, qkv, slot_mapping, q_weight, k_weight, eps, cos_sin, 
     if work is not None:
         _dev(work)
         _i32(work, "work", n)
+        _need(merge, "splits that are left to a reader lie by request: no order of the blocks beside them")
     least = attn_decode_min_splits(block_tables.shape[1], page_size)
     _need(num_splits >= least, f"block tables of {block_tables.shape[1]} pages need at least {least} splits")
     if num_splits > 1:

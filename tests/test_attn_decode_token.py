@@ -133,3 +133,35 @@ def test_token_attention_refuses_what_it_does_not_take():
         K.attn_decode_token(*args(torch.zeros(1, 5 * D, **bf)))
     with pytest.raises(K.KernelArgumentError, match="scratch"):
         K.attn_decode_token(*args(torch.zeros(1, 6 * D, **bf)), num_splits=2)
+
+
+@pytest.mark.gpu
+def test_unmerged_splits_lie_by_request():
+    """The splits' results that a product merges: those of row r belong to request r, so no order of the blocks goes with them."""
+    from jax_vllm_amd.ops import kernels as K
+
+    n, nq, nkv, ps, splits = 3, 4, 1, 16, 2
+    g = torch.Generator().manual_seed(5)
+    qkv = torch.randn(n, (nq + 2 * nkv) * D, generator=g).to(torch.bfloat16).cuda()
+    kp, vp = (torch.randn(1 + 4 * n, nkv, *s, generator=g).to(torch.bfloat16).cuda() for s in ((ps, D), (D, ps)))
+    tables = (1 + torch.arange(4 * n, dtype=torch.int32)).view(n, 4).cuda()
+    pos = torch.tensor([60, 3, 41], dtype=torch.int32).cuda()
+    slots = (tables[torch.arange(n), (pos // ps).long()] * ps + pos % ps).to(torch.int32)
+    work = torch.tensor([2, 0, 1], dtype=torch.int32).cuda()
+
+    def attend(merge, order):
+        scratch = torch.full((K.attn_decode_scratch_floats(n, nq, splits, D),), float("nan")).cuda()
+        out = torch.full((n, nq * D), float("nan"), dtype=torch.bfloat16).cuda()
+        K.attn_decode_token(out if merge else None, qkv, slots, None, None, 0.0, None, 0, kp, vp, tables, pos, nq, nkv, D, 1.0, 0, splits, scratch,
+                            merge=merge, work=order)
+        return out, scratch
+
+    out, scratch = attend(True, None)
+    assert torch.equal(attend(True, work)[0], out)                 # merged, any order
+    kept = attend(False, None)[1]
+    acc, ml = kept[:n * nq * splits * D].view(n, nq, splits, D), kept[n * nq * splits * D:].view(n, nq, splits, 2)
+    f = torch.exp2(ml[..., 0] - ml[..., 0].amax(-1, keepdim=True))
+    merged = (torch.where(f[..., None] > 0, acc, 0.0) * f[..., None]).sum(-2) / (ml[..., 1] * f).sum(-1, keepdim=True)
+    torch.testing.assert_close(merged.view(n, -1), out.float(), rtol=2 ** -7, atol=1e-6)      # row r of scratch is request r; results are bfloat16
+    with pytest.raises(K.KernelArgumentError, match="by request"):
+        attend(False, work)
