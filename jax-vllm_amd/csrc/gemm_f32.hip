@@ -737,28 +737,32 @@ static int tile_launch(float* C, const void* X, const float* A, const float* W, 
 // The same in the order in which gemm_f32_rows_kernel multiplies: [M / 32][steps][term][16 columns][8 columns][32 rows][8].
 __global__ void __launch_bounds__(256)
 split_fragments_kernel(unsigned* __restrict__ y, const float* __restrict__ A, int M, int K, int steps) {
-  const int row = threadIdx.x >> 3, m = blockIdx.x * 32 + row, k = (blockIdx.y * 8 + (threadIdx.x & 7)) * 8;
-  if (m >= M || k >= steps * G32_STEP) return;
-  const float* a = A + (long long)m * K + k;
-  f32x4 v[2];
-  if (k + 8 <= K && ((uintptr_t)a & 15) == 0) {
-    v[0] = *(const f32x4*)a, v[1] = *(const f32x4*)(a + 4);
-  } else {
+  const int row = threadIdx.x >> 3, m = blockIdx.x * 32 + row;
+  if (m >= M) return;
+  // 64 columns a block; a grid has no more than 65,535 blocks of columns, the longest rows have 65,536
+  for (int at = blockIdx.y; at < (steps + 1) / 2; at += gridDim.y) {
+    const int k = (at * 8 + (threadIdx.x & 7)) * 8;
+    if (k >= steps * G32_STEP) return;
+    const float* a = A + (long long)m * K + k;
+    f32x4 v[2];
+    if (k + 8 <= K && ((uintptr_t)a & 15) == 0) {
+      v[0] = *(const f32x4*)a, v[1] = *(const f32x4*)(a + 4);
+    } else {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e / 4][e % 4] = k + e < K ? a[e] : 0.f;
+      for (int e = 0; e < 8; ++e) v[e / 4][e % 4] = k + e < K ? a[e] : 0.f;
+    }
+    u32x4 t[3];
+    split8(v, t);
+    u32x4* out = (u32x4*)y + ((long long)blockIdx.x * steps + k / G32_STEP) * 384 + k % G32_STEP / 16 * 64 + k % 16 / 8 * 32 + row;
+#pragma unroll
+    for (int e = 0; e < 3; ++e) out[e * 128] = t[e];
   }
-  u32x4 t[3];
-  split8(v, t);
-  u32x4* out = (u32x4*)y + ((long long)blockIdx.x * steps + k / G32_STEP) * 384 + k % G32_STEP / 16 * 64 + k % 16 / 8 * 32 + row;
-#pragma unroll
-  for (int e = 0; e < 3; ++e) out[e * 128] = t[e];
 }
 extern "C" int jv_split_fragments_f32(void* X, const float* A, int M, int KA, void* stream) {
   if (M <= 0 || KA <= 0) return 0;
   if ((uintptr_t)X & 15) return (int)hipErrorInvalidValue;
   const int steps = (KA + G32_STEP - 1) / G32_STEP;
-  if ((steps + 1) / 2 > 65535) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL(split_fragments_kernel, dim3((M + 31) / 32, (steps + 1) / 2), dim3(256), 0, (hipStream_t)stream, (unsigned*)X, A, M, KA, steps);
+  hipLaunchKernelGGL(split_fragments_kernel, dim3((M + 31) / 32, (steps + 1) / 2 < 65535 ? (steps + 1) / 2 : 65535), dim3(256), 0, (hipStream_t)stream, (unsigned*)X, A, M, KA, steps);
   return JV_LAUNCH_CHECK();
 }
 template <int TW>

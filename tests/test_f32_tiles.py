@@ -40,3 +40,15 @@ def test_activation_as_an_epilogue(m, n, k, activation):
     assert k_.linear(a, w, gate_pairs=activation).shape == out.shape and k_.gemm_f32(a, w, out, activation) is out
     with pytest.raises(k_.KernelArgumentError, match="pairs"):
         k_.gemm_f32(a, w[:n - 1], gate_pairs=activation)
+
+
+@pytest.mark.gpu
+def test_the_longest_rows():
+    """Every inner size that a plan gives to the tiles: 65,536 blocks of columns split a row of 2^22."""
+    k = 1 << 22
+    assert K().f32_plan(500, 4096, k) == 7 and K().f32_plan(1024, 4096, k) == 5
+    a, w = randn(33, k, seed=1), randn(2, k, seed=2)
+    few = product(10, a, w)
+    assert ((few.double() - a.double() @ w.double().T).abs() <= bound(a, w)).all()
+    for form in (5, 6, 7):
+        assert torch.equal(product(form, a, w), few), form
