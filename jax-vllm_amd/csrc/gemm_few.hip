@@ -37,9 +37,13 @@ gemm_few_kernel(void* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t
   static_assert(NT * 1024 <= S * CHUNK * 2, "the parts meet in the ring's place");
   __shared__ __attribute__((aligned(1024))) bf16_t bufs[FEW_WAVES][S * CHUNK];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, lq = lane >> 4;
-  constexpr int XSTRIDE = KX + 8;
+  // Two blocks a unit: two made rows of 4,096 columns fill what the ring leaves of half its LDS to the byte, so they have no gap between them
+  // and their sums of squares wait in registers for the ring's place.  With 96 bytes more, one block a unit, 12,288 x 4,096 at two rows took 28.3 us
+  // (rows given, and made by a launch before: 25.7).
+  constexpr int XSTRIDE = MR * KX > 4096 ? KX : KX + 8;
   __shared__ __attribute__((aligned(16))) bf16_t xmade[SRC == ROWS_GIVEN ? 8 : MR * XSTRIDE];
-  __shared__ float made_sq[MR * 8];
+  static_assert(sizeof(bufs) + (SRC == ROWS_GIVEN ? 0 : sizeof(xmade)) <= 80 * 1024, "");
+  float made_sq[MR];
   RowMaker<SRC, MR, KX> maker;
   if constexpr (SRC != ROWS_GIVEN) {
     maker.ask(src_rows, 0, K);
@@ -116,6 +120,13 @@ gemm_few_kernel(void* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t
   f32x4* red = (f32x4*)bufs;
 #pragma unroll
   for (int t = 0; t < NT; ++t) red[(t * FEW_WAVES + wave) * 64 + lane] = acc[t];
+  float* const row_sq = (float*)(red + NT * FEW_WAVES * 64);      // [MR][FEW_WAVES]
+  if constexpr (SRC != ROWS_GIVEN) {
+    static_assert(NT * FEW_WAVES * 1024 + MR * FEW_WAVES * 4 <= sizeof(bufs), "");
+#pragma unroll
+    for (int m = 0; m < MR; ++m)
+      if (lane == 0) row_sq[m * FEW_WAVES + wave] = made_sq[m];
+  }
   __syncthreads();
   if (wave >= NT) return;
   f32x4 sum = red[wave * FEW_WAVES * 64 + lane];
@@ -124,7 +135,7 @@ gemm_few_kernel(void* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t
   if (SRC == ROWS_RESIDUAL) {
     float sq = 0.f;
 #pragma unroll
-    for (int w = 0; w < 8; ++w) sq += made_sq[min(li, MR - 1) * 8 + w];
+    for (int w = 0; w < FEW_WAVES; ++w) sq += row_sq[min(li, MR - 1) * FEW_WAVES + w];
     sum *= rsqrtf(sq * src_rows.inv_width + src_rows.eps);
   }
   const int m = li, n = n0 + wave * 16 + lq * 4;      // a lane holds y[m][n .. n + 3]; N is a multiple of 4

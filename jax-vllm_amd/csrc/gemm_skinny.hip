@@ -482,7 +482,12 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
     load_tile(tile, a0);
     if constexpr (SRC != ROWS_GIVEN) {
       __builtin_amdgcn_sched_barrier(0);
-      maker.give(src, blockIdx.y * KB, K, blockIdx.x == 0, xmade, XSTRIDE, made_sq);
+      float sums[MR];
+      maker.give(src, blockIdx.y * KB, K, blockIdx.x == 0, xmade, XSTRIDE, sums);
+      if (SRC == ROWS_RESIDUAL && lane == 0) {
+#pragma unroll
+        for (int m = 0; m < MR; ++m) made_sq[m * 8 + wk] = sums[m];
+      }
       __syncthreads();
       if (SRC == ROWS_RESIDUAL && gridDim.y > 1 && blockIdx.x == 0 && tid < MR) {
         float sq = 0.f;

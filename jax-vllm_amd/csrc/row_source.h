@@ -30,7 +30,7 @@ typedef __bf16 row_bf16x4 __attribute__((ext_vector_type(4)));
 typedef float row_f32x4 __attribute__((ext_vector_type(4)));
 
 // KB columns from k0 on of MR rows (MR = 1 or 2, no more than there are), by the 512 threads of a block in pieces of 4 columns.  ask() only
-// loads; give() leaves the rows in xs (row_stride elements apart) and, for ROWS_RESIDUAL, each wave's sums of squares in sq[row * 8 + wave].
+// loads; give() leaves the rows in xs (row_stride elements apart) and, for ROWS_RESIDUAL, the wave's sums of squares in sq[row], in every lane.
 template <int SRC, int MR, int KB> struct RowMaker {
   static constexpr int IT = (KB + 2047) / 2048;
   row_f32x4 v[MR][IT], e[MR][IT][4], w[IT];
@@ -54,7 +54,7 @@ template <int SRC, int MR, int KB> struct RowMaker {
       }
     }
   }
-  __device__ __forceinline__ void give(const RowSource& s, int k0, int K, bool leave, bf16_t* xs, int row_stride, float* sq) {
+  __device__ __forceinline__ void give(const RowSource& s, int k0, int K, bool leave, bf16_t* xs, int row_stride, float (&sq)[MR]) {
     if constexpr (SRC == ROWS_RESIDUAL) {
 #pragma unroll
       for (int m = 0; m < MR; ++m) {
@@ -79,8 +79,7 @@ template <int SRC, int MR, int KB> struct RowMaker {
             if (leave) *(row_f32x4*)(s.h_out + (long long)m * K + k0 + c) = x;
           }
         }
-        sum = wave_sum(sum);
-        if ((threadIdx.x & 63) == 0) sq[m * 8 + (threadIdx.x >> 6)] = sum;
+        sq[m] = wave_sum(sum);
       }
     } else if constexpr (SRC == ROWS_SPLITS) {
 #pragma unroll
