@@ -381,7 +381,11 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
   const int k0 = (blockIdx.y * 8 + wk) * NL * 32 + lc * 8;     // this lane's first column
   const int n_tiles = (N + 15) / 16;
   // x: rows mt * 16 + li (zero beyond M), this wave's columns
-  bf16x8 b[MT][NL];
+  // 20 pieces of x beside two tiles of W fill the registers, and with what makes the rows 12 to 16 of them spilled: 24,576 x 5,120 at one row 63.0 us
+  // (rows made by a launch before and given: 50.3).  Made rows lie in LDS anyway and are read there for every tile: 48.1.
+  constexpr bool X_STAYS = SRC != ROWS_GIVEN && NL > 16;
+  bf16x8 b[MT][X_STAYS ? 1 : NL];
+  const bf16_t* const x_lane = xmade + min(li, MR - 1) * XSTRIDE + wk * NL * 32 + lc * 8;
   if constexpr (SRC == ROWS_GIVEN) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
@@ -419,8 +423,10 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int i = 0; i < CNT; ++i)
-        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[mt][first + i], acc[mt], 0, 0, 0);
+      for (int i = 0; i < CNT; ++i) {
+        if constexpr (X_STAYS) acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], *(const bf16x8*)(x_lane + (first + i) * 32), acc[mt], 0, 0, 0);
+        else acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[mt][first + i], acc[mt], 0, 0, 0);
+      }
   };
   // the 8 waves' sums of a tile, added in fixed order and stored
   auto reduce_store = [&](int tile, const f32x4 (&acc)[MT], int buf) {
@@ -495,8 +501,10 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
         for (int w = 0; w < 8; ++w) sq += made_sq[tid * 8 + w];
         src.ssq_out[tid * 16 + blockIdx.y] = sq;
       }
+      if constexpr (!X_STAYS) {
 #pragma unroll
-      for (int i = 0; i < NL; ++i) b[0][i] = *(const bf16x8*)(xmade + min(li, MR - 1) * XSTRIDE + (wk * NL + i) * 32 + lc * 8);
+        for (int i = 0; i < NL; ++i) b[0][i] = *(const bf16x8*)(x_lane + i * 32);
+      }
     }
     for (;;) {
       int next = tile + gridDim.x;
