@@ -358,8 +358,8 @@ struct RowScale {
 // in half the registers of the two-tile scheme: what two row tiles of x with 16 pieces a wave need to fit (128
 // registers of x, 64 of W).
 //
-// SRC (row_source.h): the block makes its columns of x itself, MR (1 or 2) rows of them; ROWS_RESIDUAL with the whole inner size in the block
-// also scales them (MT 1, no EDGE, no SLOTS).
+// SRC (row_source.h): the block makes its columns of x itself, MR (1 or 2) rows of them; ROWS_RESIDUAL with PAIRS has the whole inner size in
+// the block and also scales them, else it leaves the rows' sums of squares (MT 1, no EDGE, no SLOTS).
 template <int NL, int MT, typename OutT, bool PAIRS, bool EDGE, int SLOTS = 0, int SRC = ROWS_GIVEN, int MR = 1>
 __global__ void __launch_bounds__(512)
 gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t* __restrict__ W,
@@ -452,7 +452,7 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
         const float inv = rsqrtf(sq * rs.inv_width + rs.eps);
         s[0] *= inv; s[1] *= inv; s[2] *= inv; s[3] *= inv;
       }
-      if (SRC == ROWS_RESIDUAL && gridDim.y == 1) {
+      if (SRC == ROWS_RESIDUAL && PAIRS) {
         float sq = 0.f;
 #pragma unroll
         for (int w = 0; w < 8; ++w) sq += made_sq[min(li, MR - 1) * 8 + w];
@@ -495,7 +495,7 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
         for (int m = 0; m < MR; ++m) made_sq[m * 8 + wk] = sums[m];
       }
       __syncthreads();
-      if (SRC == ROWS_RESIDUAL && gridDim.y > 1 && blockIdx.x == 0 && tid < MR) {
+      if (SRC == ROWS_RESIDUAL && !PAIRS && blockIdx.x == 0 && tid < MR) {
         float sq = 0.f;
 #pragma unroll
         for (int w = 0; w < 8; ++w) sq += made_sq[tid * 8 + w];
@@ -727,11 +727,11 @@ static int dispatch_made(int nl, void* y, const void* W, int M, int N, int K, lo
   return (int)hipErrorInvalidValue;
 }
 // y = (norm of h + parts) W^T: float partial products [ksplit][M][N], not scaled (ksplit > 1; ssq [M][16] takes ksplit shares of the rows' sums of
-// squares), float [M][N], or with gate_act bf16 [M][N / 2], both scaled.  h_out takes h + parts.
+// squares), or with gate_act and ksplit 1 bf16 [M][N / 2], scaled.  h_out takes h + parts.
 extern "C" int jv_gemm_skinny_residual_bf16(void* y, const float* h, float* h_out, const float* parts, int n_parts, long long part_stride,
                                             const float* weight, float* ssq, float eps, const void* W, int M, int N, int K, int gate_act,
                                             float act_limit, float act_slope, int blocks, int nl, int ksplit, void* stream) {
-  if (n_parts < 0 || n_parts > 4 || (n_parts && !parts) || h == h_out || (ksplit > 1 && (!ssq || gate_act)) || (gate_act && (!jv_act_known(gate_act) || N % 2)))
+  if (n_parts < 0 || n_parts > 4 || (n_parts && !parts) || h == h_out || (gate_act ? ksplit != 1 || !jv_act_known(gate_act) || N % 2 : ksplit < 2 || !ssq))
     return (int)hipErrorInvalidValue;
   RowSource src{};
   src.h = h; src.h_out = h_out; src.parts = parts; src.n_parts = n_parts; src.part_stride = part_stride; src.weight = weight; src.ssq_out = ssq;
