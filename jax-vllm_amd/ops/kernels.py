@@ -1378,6 +1378,22 @@ def linear_takes_split_heads(n_rows: int, w: torch.Tensor, splits: int) -> bool:
     return 1 < splits <= MADE_MAX_SPLITS and isinstance(_made_plan(n_rows, w, False, True, PARTIAL_SUM_MAX_WIDTH), tuple)
 
 
+def split_heads_pay(n_rows: int, w: torch.Tensor, splits: int) -> bool:
+    """Whether the output product had better merge the splits itself than read what the merge's launch leaves.  Every block reads ``splits`` times
+    its columns in float, so it depends on how many blocks there are and how long their columns keep them.  Microseconds that merging there spares, over
+    792 products of 2,048 to 12,288 columns, behind an attention of 600 keys: one row, up to 8 splits 0.1 to 2.2 everywhere; 9 to 16 splits 0.5 to 1.9 where no unit gets two
+    blocks and a wave's share is up to 8 pieces, else from 0.5 spared to 1.3 lost (4,096 x 4,096, 512 blocks, 16 splits -0.3; 8,192 x 10,240, 10 pieces -1.3);
+    two rows, 2 to 8 splits 0.2 to 1.1 where every block has one tile of rows and no unit two blocks, up to 8 pieces, else from 0.2 spared (0.6 at one) to 2.5 lost
+    (4,096 x 4,096 -1.1)."""
+    if not linear_takes_split_heads(n_rows, w, splits):
+        return False
+    blocks, pieces, parts = _made_plan(n_rows, w, False, True, PARTIAL_SUM_MAX_WIDTH)
+    tiles, units = -(-w.shape[0] // 16), compute_units(w.device)
+    if n_rows == 1 and splits <= 8:
+        return pieces <= 12
+    return pieces <= 8 and parts * (tiles if n_rows > 1 else min(tiles, -(-blocks // parts))) <= units and n_rows * splits <= 16
+
+
 def _linear_made(x, w: torch.Tensor, gate_pairs, partial_ok: bool, partial_max_width):
     _dev(w)
     m, (n, k) = x.shape[0], w.shape

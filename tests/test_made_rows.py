@@ -138,3 +138,17 @@ def test_a_model_of_few_requests_like_one_of_three(graphs):
             made.clear()
     finally:
         kernels_._linear_made = linear_made
+
+
+def test_when_the_output_product_merges(monkeypatch):
+    """One row up to 8 splits always; more splits, or two rows, while no unit gets a second block (or tile) to read them for."""
+    from jax_vllm_amd.ops import kernels
+
+    monkeypatch.setattr(kernels, "compute_units", lambda device: 256)
+    pays = lambda m, n, k, splits: kernels.split_heads_pay(m, torch.empty(n, k, dtype=BF), splits)
+    shapes = [(2048, 2048), (4096, 4096), (5120, 5120), (2560, 4096), (6144, 2048), (8192, 8192)]
+    assert all(pays(1, n, k, splits) for n, k in shapes for splits in (2, 8)) and not any(pays(1, n, k, 1) for n, k in shapes)
+    assert [pays(1, n, k, 16) for n, k in shapes] == [True, False, True, False, False, True]
+    assert [pays(2, n, k, 8) for n, k in shapes] == [True, False, False, False, False, False]
+    assert not any(pays(2, n, k, 16) or pays(1, n, k, 17) or pays(3, n, k, 4) for n, k in shapes)
+    assert not pays(1, 8192, 10240, 16) and pays(1, 8192, 10240, 8) and pays(2, 1024, 4096, 4) and not pays(2, 1040, 4096, 4)
