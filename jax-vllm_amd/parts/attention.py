@@ -259,7 +259,9 @@ class GroupedQueryAttention:
             K.add_bias(qkv, self.b_qkv)
         from . import attention_backend
 
-        if attention_backend.token_possible(self, ctx, mem, interleaved, rotary_dim):
+        # rows that the products make spare two launches of their own, whatever this one takes
+        if attention_backend.token_possible(self, ctx, mem, interleaved, rotary_dim) and (
+                isinstance(x, K.PendingRows) or attention_backend.token_pays(self, ctx)):
             return self._project(attention_backend.run_token(self, qkv, cos_sin, rotary_dim, ctx, mem))
         out = torch.empty((n, self.nq * self.d), dtype=x.dtype, device=x.device)
         parts = None

@@ -234,6 +234,19 @@ def token_possible(att, ctx, mem, interleaved: bool, rotary_dim: int) -> bool:
             and K.attn_decode_token_possible(att.dtype, att.d, ctx.page_size, interleaved, rotary_dim, att.rotation is not None))
 
 
+TOKEN_GROUP = 6              # q heads of a kv head that a block prepares with its new key and value in one round of loads (4 waves, 2 heads each)
+TOKEN_BLOCKS = 2048          # (request, kv head) pairs from which on a block's start has to be short beside its keys
+
+
+def token_pays(att, ctx) -> bool:
+    """Whether that launch had better stand for the two it replaces, which prepare a head once and not in every block that reads it.  Up to 6 q heads of a kv
+    head: two launches' time over one's, 396 steps of 1 to 256 requests of 30 to 3,000 keys, 1 to 32 kv heads, 0.99 to 1.24, 1.09 on average.  More heads a
+    group come in further rounds of loads (8: 0.92 to 1.16, from 64 requests on 0.94 and more; 16: 0.75 to 1.35, 0.95 on average), and 2,048 pairs or more of
+    a request and a kv head with few keys queue up behind that start (256 requests over 8 kv heads 30 keys 0.88, 200 keys 0.98, 400 1.02; 128 over 32 0.89 to 0.99)."""
+    return att.nq // att.nkv <= TOKEN_GROUP and (
+        ctx.num_tokens * att.nkv < TOKEN_BLOCKS or keys_seen(ctx.max_kv_len, K.key_window(att.window, att.chunk)) >= 1024)
+
+
 def _mfma_plan(att, ctx, window: int, keep: int, device) -> MfmaPlan:
     key = ("mfma_attention_plan", att.nq, att.nkv, att.d, window, keep)
     plan = ctx.plans.get(key)

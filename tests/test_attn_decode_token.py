@@ -165,3 +165,17 @@ def test_unmerged_splits_lie_by_request():
     torch.testing.assert_close(merged.view(n, -1), out.float(), rtol=2 ** -7, atol=1e-6)      # row r of scratch is request r; results are bfloat16
     with pytest.raises(K.KernelArgumentError, match="by request"):
         attend(False, work)
+
+
+def test_where_one_launch_stands_for_two():
+    from types import SimpleNamespace
+
+    from jax_vllm_amd.parts.attention_backend import token_pays
+
+    def pays(nq, nkv, n, keys, window=None, chunk=None):
+        return token_pays(SimpleNamespace(nq=nq, nkv=nkv, window=window, chunk=chunk), SimpleNamespace(num_tokens=n, max_kv_len=keys))
+
+    assert all(pays(g * kv, kv, n, keys) for g in (1, 4, 6) for kv in (1, 8) for n in (1, 64, 255) for keys in (16, 4096))
+    assert not any(pays(g, 1, n, keys) for g in (7, 8, 16, 64) for n in (1, 64, 512) for keys in (16, 4096))
+    # many blocks of few keys, also where a window keeps them few
+    assert not pays(32, 8, 256, 512) and pays(32, 8, 256, 1024) and not pays(32, 8, 256, 4096, window=512) and not pays(32, 32, 64, 4096, chunk=256)
