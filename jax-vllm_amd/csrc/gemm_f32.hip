@@ -74,9 +74,11 @@ __device__ __forceinline__ float settle(float sum, const float* a, const float* 
   }
   return sum;
 }
-// Numbers n .. n + 3 of row m of C, settled; with an activation the rows of W alternate gate and up rows and C is [M, N / 2].
+// Numbers n .. n + 3 of row m of C, settled; with an activation (ACT) the rows of W alternate gate and up rows and C is [M, N / 2].  Kernels without one
+// do not hold its code: beside it the smallest products took 0.1 to 0.2 us more.
+template <bool ACT>
 __device__ __forceinline__ void leave(float* C, int m, int n, int N, const float (&v)[4], JvAct act) {
-  if (act.id) {
+  if constexpr (ACT) {
 #pragma unroll
     for (int e = 0; e < 4; e += 2)
       if (n + e < N) C[(long long)m * (N / 2) + (n + e) / 2] = jv_gated(act, v[e], v[e + 1]);
@@ -87,20 +89,20 @@ __device__ __forceinline__ void leave(float* C, int m, int n, int N, const float
   }
 }
 // The same from sums of scaled products.  `pieces`: N a multiple of 4, C begins on 16 bytes.
+template <bool ACT>
 __device__ __forceinline__ void leave_sums(float* C, int m, int n, int M, int N, const f32x4& v, bool pieces, JvAct act, const float* A, const float* W, int K, int KA) {
   bool ok = pieces && n + 4 <= N;
 #pragma unroll
   for (int e = 0; e < 4; ++e) ok = ok && __builtin_fabsf(v[e]) <= 3.402823466e38f;
-  if (ok && act.id) {
+  if (ok) {
     const f32x4 r = v * G32_UNSCALE;
-    *(f32x2*)(C + (long long)m * (N / 2) + n / 2) = f32x2{jv_gated(act, r[0], r[1]), jv_gated(act, r[2], r[3])};
-  } else if (ok) {
-    *(f32x4*)(C + (long long)m * N + n) = v * G32_UNSCALE;
+    if constexpr (ACT) *(f32x2*)(C + (long long)m * (N / 2) + n / 2) = f32x2{jv_gated(act, r[0], r[1]), jv_gated(act, r[2], r[3])};
+    else *(f32x4*)(C + (long long)m * N + n) = r;
   } else {
     float r[4];
     for (int e = 0; e < 4; ++e)
       if (n + e < N) r[e] = settle(v[e], A + (long long)m * KA, W + (long long)(n + e) * K, KA);
-    leave(C, m, n, N, r, act);
+    leave<ACT>(C, m, n, N, r, act);
   }
 }
 // 16 bytes a lane from base + off straight into LDS, 1 KB in the order of the lanes from `at` on.
@@ -129,7 +131,7 @@ __device__ __forceinline__ void wait_oldest(int left) {
 // 7 of the second), each through a ring of its own in LDS, straight from memory, S steps on their way, no wave waiting for
 // another but once in R steps of each, when the steps' sums meet in LDS and are added in their order.
 // DMA false: operands through registers, a round ahead, for rows that do not begin on 16 bytes.
-template <int TW, int XR, int S, int R, bool DMA>
+template <int TW, int XR, int S, int R, bool DMA, bool ACT>
 __global__ void __launch_bounds__(512)
 gemm_f32_few_kernel(float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K, JvAct act) {
   constexpr int ROWS = TW + XR, L = ROWS / 8, BUF = ROWS * G32_STEP, NT = TW / 16, MT = XR / 16, TILES = NT * MT;
@@ -267,7 +269,7 @@ gemm_f32_few_kernel(float* __restrict__ C, const float* __restrict__ A, const fl
 #pragma unroll
   for (int e = 0; e < 4; ++e)
     if (n + e < N) r[e] = settle(sum[e], A + (long long)m * K, W + (long long)(n + e) * K, K);
-  leave(C, m, n, N, r, act);
+  leave<ACT>(C, m, n, N, r, act);
 }
 
 // ---------------------------------------------------------------------------- up to 8 rows
@@ -280,7 +282,7 @@ gemm_f32_few_kernel(float* __restrict__ C, const float* __restrict__ A, const fl
 // row (32 lines an instruction): 9.0 for 8.4.  Microseconds in graphs with cold weights, 16 x 16 or 32 x 16 tiles / these (rows of W): 8 rows
 // against 2,048 x 2,048 9.7 / 8.4 (8), 2,048 x 3,072 12.5 / 9.7 (8), 512 x 8,192 25.5 / 17.5 (8), 3,072 x 2,048 9.9 / 9.2 (16), 1,024 x 1,024 6.3 /
 // 5.5 (8), 6,144 x 2,048 14.5 / 14.0 (24), 6,144 x 8,192 51 / 45 (24), 32,000 x 2,048 54.6 / 55.2 (16): wide ones stay with 32 x 16.
-template <int G, int S, int C>
+template <int G, int S, int C, bool ACT>
 __global__ void __launch_bounds__(512)
 gemm_f32_pairs_kernel(float* __restrict__ out, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K, JvAct act) {
   constexpr int L = 2 * (G + 1), BUF = L * 256;      // loads of a pair, each 8 rows of a step, 1 KB
@@ -379,7 +381,7 @@ gemm_f32_pairs_kernel(float* __restrict__ out, const float* __restrict__ A, cons
 #pragma unroll
   for (int e = 0; e < 4; ++e)
     if (n + e < N) r[e] = settle(sum[e], A + (long long)m * K, W + (long long)(n + e) * K, K);
-  leave(out, m, n, N, r, act);
+  leave<ACT>(out, m, n, N, r, act);
 }
 
 // ---------------------------------------------------------------------------- many rows
@@ -406,7 +408,7 @@ split_rows_kernel(unsigned* __restrict__ y, const float* __restrict__ A, int K, 
 // Tiles of TM (64) rows of A (as terms) by TW rows of W (as floats); two groups of 2 x 2 waves take a half of the steps each, through
 // rings of S steps in LDS.  Bound by what a SIMD issues: a product of 16 cycles takes 8 of them, a vector instruction 2 to 4
 // (measured), so a wave splits the next 16 rows of W (52 instructions) while it multiplies these with all its rows of A.
-template <int TM, int TW>
+template <int TM, int TW, bool ACT>
 __global__ void __launch_bounds__(512, 2)
 gemm_f32_tile_kernel(float* __restrict__ C, const unsigned* __restrict__ X, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K, int KA, JvAct act) {
   constexpr int MT = TM / 32, NT = TW / 32, XL = TM * 3 / 64, WL = TW / 32, L = XL + WL;      // L: loads of a wave for a step
@@ -548,7 +550,7 @@ gemm_f32_tile_kernel(float* __restrict__ C, const unsigned* __restrict__ X, cons
 #pragma unroll
     for (int a = 0; a < NT; ++a) {
       const int n = n0 + (wn * NT + a) * 16 + lq * 4;
-      leave_sums(C, m, n, M, N, tot[a][b] + meet[((a * MT + b) * 4 + wave) * 64 + lane], pieces, act, A, W, K, KA);
+      leave_sums<ACT>(C, m, n, M, N, tot[a][b] + meet[((a * MT + b) * 4 + wave) * 64 + lane], pieces, act, A, W, K, KA);
     }
   }
 }
@@ -562,7 +564,7 @@ gemm_f32_tile_kernel(float* __restrict__ C, const unsigned* __restrict__ X, cons
 // Against tiles of 128 rows by the 16x16x32 instruction, in which every wave split its W and which were bound by what a SIMD issues,
 // microseconds with the split of A, before -> now: 1,003 x 6,144 x 2,048 160 -> 149, x 2,048 61 -> 56, 384 x 4,096 x 4,096 111 -> 88, 2,048 x 24,576 x
 // 4,096 2,385 -> 2,070 (1.2 PFLOP/s of the matrix unit's, where its power ends it); over 199 sizes 0.94 of the time with what f32_plan takes.
-template <int TW>
+template <int TW, bool ACT>
 __global__ void __launch_bounds__(512, 2)
 gemm_f32_rows_kernel(float* __restrict__ C, const unsigned* __restrict__ X, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K, int KA, JvAct act) {
   constexpr int TM = 128, NT = TW / 32, TERMS = 3 * TW * 64, RING = 3;
@@ -709,7 +711,7 @@ gemm_f32_rows_kernel(float* __restrict__ C, const unsigned* __restrict__ X, cons
     for (int q = 0; q < 4; ++q) {
       const int n = n0 + a * 32 + q * 8 + lh * 4;
       const f32x4 v = f32x4{tot[a][q * 4], tot[a][q * 4 + 1], tot[a][q * 4 + 2], tot[a][q * 4 + 3]} + meet[((a * 4 + q) * 4 + wave) * 64 + lane];
-      leave_sums(C, m, n, M, N, v, pieces, act, A, W, K, KA);
+      leave_sums<ACT>(C, m, n, M, N, v, pieces, act, A, W, K, KA);
     }
 }
 
@@ -719,19 +721,22 @@ gemm_f32_rows_kernel(float* __restrict__ C, const unsigned* __restrict__ X, cons
 template <int TW, int XR, int S, int R, bool DMA>
 static int few_launch(float* C, const float* A, const float* W, int M, int N, int K, JvAct act, hipStream_t s) {
   if ((M + XR - 1) / XR > 65535) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL((gemm_f32_few_kernel<TW, XR, S, R, DMA>), dim3((N + TW - 1) / TW, (M + XR - 1) / XR), dim3(512), 0, s, C, A, W, M, N, K, act);
+  const auto kernel = act.id ? gemm_f32_few_kernel<TW, XR, S, R, DMA, true> : gemm_f32_few_kernel<TW, XR, S, R, DMA, false>;
+  hipLaunchKernelGGL(kernel, dim3((N + TW - 1) / TW, (M + XR - 1) / XR), dim3(512), 0, s, C, A, W, M, N, K, act);
   return JV_LAUNCH_CHECK();
 }
 template <int G, int S, int C>
 static int pairs_launch(float* out, const float* A, const float* W, int M, int N, int K, JvAct act, hipStream_t s) {
-  hipLaunchKernelGGL((gemm_f32_pairs_kernel<G, S, C>), dim3((N + 8 * G - 1) / (8 * G)), dim3(512), 0, s, out, A, W, M, N, K, act);
+  const auto kernel = act.id ? gemm_f32_pairs_kernel<G, S, C, true> : gemm_f32_pairs_kernel<G, S, C, false>;
+  hipLaunchKernelGGL(kernel, dim3((N + 8 * G - 1) / (8 * G)), dim3(512), 0, s, out, A, W, M, N, K, act);
   return JV_LAUNCH_CHECK();
 }
 template <int TM, int TW>
 static int tile_launch(float* C, const void* X, const float* A, const float* W, int M, int N, int K, int KA, JvAct act, hipStream_t s) {
   const long long live = ((long long)M + TM - 1) / TM * (((long long)N + TW - 1) / TW);
   if (live > 1 << 24) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL((gemm_f32_tile_kernel<TM, TW>), dim3((unsigned)((live + 7) / 8 * 8)), dim3(512), 0, s, C, (const unsigned*)X, A, W, M, N, K, KA, act);
+  const auto kernel = act.id ? gemm_f32_tile_kernel<TM, TW, true> : gemm_f32_tile_kernel<TM, TW, false>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((live + 7) / 8 * 8)), dim3(512), 0, s, C, (const unsigned*)X, A, W, M, N, K, KA, act);
   return JV_LAUNCH_CHECK();
 }
 // The same in the order in which gemm_f32_rows_kernel multiplies: [M / 32][steps][term][16 columns][8 columns][32 rows][8].
@@ -769,7 +774,8 @@ template <int TW>
 static int rows_launch(float* C, const void* X, const float* A, const float* W, int M, int N, int K, int KA, JvAct act, hipStream_t s) {
   const long long live = ((long long)M + 127) / 128 * (((long long)N + TW - 1) / TW);
   if (live > 1 << 24) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL((gemm_f32_rows_kernel<TW>), dim3((unsigned)((live + 7) / 8 * 8)), dim3(512), 0, s, C, (const unsigned*)X, A, W, M, N, K, KA, act);
+  const auto kernel = act.id ? gemm_f32_rows_kernel<TW, true> : gemm_f32_rows_kernel<TW, false>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((live + 7) / 8 * 8)), dim3(512), 0, s, C, (const unsigned*)X, A, W, M, N, K, KA, act);
   return JV_LAUNCH_CHECK();
 }
 // Rows of A [M][KA] as terms (of 2^24 times A), [M][steps][3][32] bf16 with zeros behind KA; steps = ceil(KA / 32).
