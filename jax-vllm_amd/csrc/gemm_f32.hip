@@ -15,9 +15,9 @@
 // one among them, are then whole.  A sum that is not finite may come from the split (2^80 of the true sum, a value near the
 // largest float, infinity less itself): it is made again from the numbers themselves.
 //
-// Microseconds in graphs with cold weights, as first built (tiles of 16, 32 and 64 rows) / now: 5 rows against 2,048 x 2,048 9.6 / 8.4, 6,144 x 2,048 15.0 /
-// 13.9 (50 MB: the stream of W); 300 x 6,144 x 2,048 74 / 64; 1,003 x 6,144 x 2,048 156 / 152 with what the terms of A take; 2,048 x 24,576 x 4,096
-// 2,385 / 2,070 = 199 TFLOP/s of 32-bit products, 1.2 PFLOP/s of the matrix unit's.  The scaling takes 1 to 5 % of it (24 sizes).
+// Microseconds in graphs with cold weights, as first built (tiles of 16, 32 and 64 rows) / now: 5 rows against 2,048 x 2,048 10.1 / 8.2, 6,144 x 2,048 14.7 /
+// 13.9 (50 MB: the stream of W); 300 x 6,144 x 2,048 75 / 65; 1,003 x 6,144 x 2,048 153 / 144 with what the terms of A take; 2,048 x 24,576 x 4,096
+// 2,250 / 1,954 = 211 TFLOP/s of 32-bit products, 1.27 PFLOP/s of the matrix unit's.  The scaling takes 1 to 5 % of it (24 sizes).
 #include "common.h"
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -569,14 +569,17 @@ gemm_f32_tile_kernel(float* __restrict__ C, const unsigned* __restrict__ X, cons
 // terms come straight into registers, one or two steps ahead, in pieces of 1 KB in the order of the lanes (split_fragments_kernel; 16 bytes from
 // each of 64 rows an instruction cost a fifth more).  W is split once a group: a thread takes 4 numbers a row two or three steps
 // ahead, splits them beside the products of a step and leaves the terms in a ring of 3 steps in LDS.
+// Both groups' sums go through LDS to rows of C in whole lines: from the lanes that hold them 32 bytes of a row left at once, and one group's waves added and
+// stored everything, 6 us a block longer (2,048 x 24,576 x 512 with those 381 us, 2,048 x 8,192 x 256 85).
 // Against tiles of 128 rows by the 16x16x32 instruction, in which every wave split its W and which were bound by what a SIMD issues,
-// microseconds with the split of A, before -> now: 1,003 x 6,144 x 2,048 160 -> 149, x 2,048 61 -> 56, 384 x 4,096 x 4,096 111 -> 88, 2,048 x 24,576 x
-// 4,096 2,385 -> 2,070 (1.2 PFLOP/s of the matrix unit's, where its power ends it); over 199 sizes 0.94 of the time with what f32_plan takes.
+// microseconds with the split of A, before -> now: 1,003 x 6,144 x 2,048 153 -> 144, x 2,048 61 -> 57, 384 x 4,096 x 4,096 110 -> 86, 2,048 x 24,576 x
+// 4,096 2,250 -> 1,954, x 512 345 -> 310, 2,048 x 8,192 x 256 74 -> 65; 128 rows of W 1.14 to 1.30 times as fast on average by inner size, 96 1.06 to
+// 1.23, 64 1.08 to 1.26.  Behind only where few rows meet many short ones: 65 to 200 x 24,576 x 256 and 512 by 4 to 7 %.
 template <int TW, bool ACT>
 __global__ void __launch_bounds__(512, 2)
 gemm_f32_rows_kernel(float* __restrict__ C, const unsigned* __restrict__ X, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K, int KA, JvAct act) {
   constexpr int TM = 128, NT = TW / 32, TERMS = 3 * TW * 64, RING = 3;
-  static_assert(2 * RING * TERMS <= 160 * 1024 && TM * TW * 4 <= 2 * RING * TERMS, "");
+  static_assert(2 * RING * TERMS <= 160 * 1024 && 2 * TM * (TW + 4) * 4 <= 2 * RING * TERMS, "");
   __shared__ __attribute__((aligned(1024))) char bufs[2 * RING * TERMS];
   const int lane = threadIdx.x & 63, all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), group = all >> 2, wave = all & 3;
   const int mtiles = (M + TM - 1) / TM, live = mtiles * ((N + TW - 1) / TW), per = (live + 7) / 8;
@@ -701,26 +704,23 @@ gemm_f32_rows_kernel(float* __restrict__ C, const unsigned* __restrict__ X, cons
   if constexpr (NT % 2 == 0) tot[NT - 1] += t[1];
   else tot[NT - 1] += steps & 1 ? t[0] : t[1];
   __syncthreads();
-  f32x4* meet = (f32x4*)bufs;
-  if (group) {
-#pragma unroll
-    for (int a = 0; a < NT; ++a)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) meet[((a * 4 + q) * 4 + wave) * 64 + lane] = f32x4{tot[a][q * 4], tot[a][q * 4 + 1], tot[a][q * 4 + 2], tot[a][q * 4 + 3]};
-  }
-  __syncthreads();
-  if (group) return;
-  const bool pieces = !(N & 3) && !((uintptr_t)C & 15);
-  const int m = m0 + wave * 32 + li;
-  if (m >= M) return;
+  // both groups' sums meet in LDS and leave it in whole lines of a row
+  constexpr int ROW = TW + 4, SIDE = TM * ROW;
+  float* const meet = (float*)bufs;
 #pragma unroll
   for (int a = 0; a < NT; ++a)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int n = n0 + a * 32 + q * 8 + lh * 4;
-      const f32x4 v = f32x4{tot[a][q * 4], tot[a][q * 4 + 1], tot[a][q * 4 + 2], tot[a][q * 4 + 3]} + meet[((a * 4 + q) * 4 + wave) * 64 + lane];
-      leave_sums<ACT>(C, m, n, M, N, v, pieces, act, A, W, K, KA);
-    }
+    for (int q = 0; q < 4; ++q)
+      *(f32x4*)(meet + group * SIDE + (wave * 32 + li) * ROW + a * 32 + q * 8 + lh * 4) = f32x4{tot[a][q * 4], tot[a][q * 4 + 1], tot[a][q * 4 + 2], tot[a][q * 4 + 3]};
+  __syncthreads();
+  const bool pieces = !(N & 3) && !((uintptr_t)C & 15);
+#pragma unroll 4
+  for (int i = threadIdx.x; i < TM * TW / 4; i += 512) {
+    const int r = i / (TW / 4), c = (i - r * (TW / 4)) * 4;
+    if (m0 + r >= M || n0 + c >= N) continue;
+    const float* at = meet + r * ROW + c;
+    leave_sums<ACT>(C, m0 + r, n0 + c, M, N, *(const f32x4*)at + *(const f32x4*)(at + SIDE), pieces, act, A, W, K, KA);
+  }
 }
 
 // How C is made (jv_gemm_f32): 0, 1: few rows, 16 x 16 or 32 x 32, through registers; 2 to 4: few rows through the ring, 16 x 16, 32 x 16, 32 x 32
