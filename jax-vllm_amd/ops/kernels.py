@@ -793,9 +793,9 @@ def attn_f32(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_seqlens, c
 
 # --------------------------------------------------------------------------- matrix products
 F32_STEP = 32         # columns of a step of the 32-bit product
-# tiles of the 32-bit product: form, rows of a, rows of w, microseconds of a round per 1,024 columns on one unit and on all
-_F32_TILES = ((5, 128, 128, 23.5, 38.3), (6, 128, 96, 19.6, 30.8), (7, 128, 64, 11.6, 23.2), (8, 64, 96, 16.7, 22.2), (9, 64, 64, 11.2, 16.3),
-              (10, 64, 32, 4.0, 10.0))
+# tiles of the 32-bit product: form, rows of a, rows of w, microseconds that a round takes whatever the columns, and per 1,024 of them on one unit and on all
+_F32_TILES = ((5, 128, 128, 3.0, 30.7, 36.6), (6, 128, 96, 3.1, 22.3, 29.5), (7, 128, 64, 2.25, 16.6, 22.2), (8, 64, 96, 2.45, 20.4, 24.5),
+              (9, 64, 64, 1.6, 16.0, 16.0), (10, 64, 32, 1.5, 9.5, 9.5))
 # Up to 8 rows: form, rows of w a block, blocks at once, and what a round and the stream of w take, fitted to 297 sizes (1, 4 and 8 rows, n 512 to
 # 65,536, k 512 to 12,288): on the average 2 % from the best (25 % at 1 x 12,288 x 8,192), 0.69 to 1.04 of the time of 16 x 16 and 32 x 16 tiles by the count for more rows.
 _F32_PAIRS = ((2, 8, 256, 2.3, 1.3, 1.7, 2.05, 4.0, 7.2), (2, 16, 512, 2.75, 0.6, 1.95, 5.0, 4.1, 5.05), (3, 32, 512, 0.8, 2.6, 4.15, 7.8, 3.6, 5.2),
@@ -806,9 +806,9 @@ _F32_FRAGMENTS = 8    # forms below take the terms of a in the order of the matr
 @functools.lru_cache(maxsize=4096)
 def f32_plan(m: int, n: int, k: int, pieces: bool = True, a_pieces: bool = True) -> int:
     """Form of the 32-bit product (``jv_gemm_f32``).  All give the same bits, so it is the one that takes the least time by a count of
-    rounds over 256 units, fitted to 199 sizes (17 to 2,048 rows, n 1,024 to 32,000, k 512 to 12,288, in graphs with cold weights): within 2 %
-    of the best form at all of them but 33 to 64 rows of 8,192 x 1,024 (20 %); for example k = 2,048: 5 x 2,048 8.4 us (form 2), 16 x 32,000 57 (3),
-    37 x 3,072 17.1 (4), 100 x 6,144 39.6 (9; 4 takes 48), 250 x 6,144 48 (7), 1,003 x 6,144 152 (6), 2,048 x 2,048 100 (5).
+    rounds over 256 units, fitted to 1,777 sizes of 9 to 2,048 rows (n 512 to 32,000, k 256 to 8,192, in graphs with cold weights): 0.2 % from the best form
+    on average, 10 % at most; at 923 other sizes 0.1 % and 10 %; for example k = 2,048: 5 x 2,048 8.2 us (form 2), 16 x 32,000 57 (3), 48 x 3,072 17.1
+    (4; 3 takes 18.7), 100 x 6,144 41 (9; 4 takes 48), 250 x 6,144 50 (7), 1,003 x 6,144 144 (6), 2,048 x 2,048 97 (5).
     ``pieces``: rows of w begin on 16 bytes (else they are copied for tiles, and few rows go through registers); ``a_pieces``: rows of a too."""
     q, mb = k / 1024, n * k * 4e-6
 
@@ -819,6 +819,11 @@ def f32_plan(m: int, n: int, k: int, pieces: bool = True, a_pieces: bool = True)
         b = blocks(tm, tw)
         return -(-b // slots) * (fixed + (one + (full - one) * min(1.0, b / slots)) * q)
 
+    def rounds_of_two(b, fixed, one, all_one, some_two, full):      # 512 blocks at once: from 257 on some unit has two of them
+        last = b % 512
+        part = one + (all_one - one) * last / 256 if last <= 256 else some_two + (full - some_two) * (last - 256) / 256
+        return b // 512 * (fixed + full * q) + (fixed + part * q if last else 0.0)
+
     times, through_ring = {}, pieces and a_pieces and 0 < k <= 1 << 24
     if m <= 8 and through_ring:
         for form, tw, slots, start, fixed, one, full, first, rate in _F32_PAIRS:
@@ -827,19 +832,19 @@ def f32_plan(m: int, n: int, k: int, pieces: bool = True, a_pieces: bool = True)
         return min(times, key=times.get)
     if m <= 65535 * 16:                                           # the grid's rows
         if through_ring:
-            times[2] = max(3 + rounds(16, 16, 1.3, 2.3, 3.2), 5 + mb / 4.2)
-            times[3] = max(3 + rounds(16, 32, 2, 3.3, 7.5, 512), 3 + mb / 5.1)      # two of these to a unit
+            times[2] = max(2.3 + rounds(16, 16, 1.15, 2.6, 3.35), 3.1 + mb / 4.9)
+            times[3] = max(3.1 + rounds_of_two(blocks(16, 32), 0.85, 3.0, 4.7, 7.6, 8.4), 3.2 + mb / 5.6)
         else:
             times[0] = 4 + rounds(16, 16, 2, 8, 10, 512)
     if m <= 65535 * 32:
         if through_ring:
-            times[4] = max(3 + rounds(32, 32, 1, 5.3, 7.1), 3 + mb / 4.9)
+            times[4] = max(1.95 + rounds(32, 32, 2.0, 6.2, 6.2), 3.4 + mb / 4.65)
         else:
             times[1] = 4 + rounds(32, 32, 2, 16, 18, 512)
     if m > 32 and 0 < k <= 1 << 22:
-        for form, tm, tw, one, full in _F32_TILES:
+        for form, tm, tw, fixed, one, full in _F32_TILES:
             if blocks(tm, tw) <= 1 << 24:
-                times[form] = 10 + (0 if pieces else 10 + mb / 2) + m * k * 2e-6 + rounds(tm, tw, 1, one, full)
+                times[form] = (6.0 if through_ring else 10.0) + (0 if pieces else 10 + mb / 2) + m * k * 2e-6 + rounds(tm, tw, fixed, one, full)
     _need(bool(times), f"no 32-bit product for {m} x {n} x {k}")
     return min(times, key=times.get)
 
