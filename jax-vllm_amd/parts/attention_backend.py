@@ -64,7 +64,11 @@ def splits_by_length(tiles: int) -> int:
     for a tile a wave), so tiles are shared out thinly; the merge takes partial results in batches of 8.  Head size 128, one request
     over 8 kv heads, microseconds with its merge: 150 keys 8.4 by one block, 8.9 by four; 300 keys 9.8 by one, 9.25 by eight; 520 keys
     12.1, by four 10.2, by eight 9.3; 1,024 keys 15.2, 10.2 by eight, 10.7 by sixteen; 2,500 keys 13.7 by eight, 12.2 by sixteen, 12.9 by nineteen;
-    7,900 keys 17.3 by sixteen, 16.6 by 24, 17.2 by 32; one over 4 kv heads 15.0 by 32, 17.7 by 61."""
+    7,900 keys 17.3 by sixteen, 16.6 by 24, 17.2 by 32; one over 4 kv heads 15.0 by 32, 17.7 by 61.
+    A recorded step is planned for the most keys its block tables hold, a power of two of pages: the plan of 256 keys serves 129 on, that of 2,048 keys
+    1,025 on.  What that costs there, attention and output product (2,048 rows), 8 kv heads of 4 q heads: 130 to 250 keys by eight or one block, one request
+    14.1 to 15.0 and 13.9 to 14.3, two 14.8 to 15.7 and 14.2 to 14.4, four 15.2 to 16.1 and 14.5 to 14.7; 1,030 to 2,000 keys by sixteen or eight
+    15.4 to 16.2 and 15.4 to 16.2, two requests 15.7 to 16.5 and 16.0 to 16.9."""
     return 1 if tiles < 8 else 8 if tiles <= 48 else max(16, tiles // 8)
 
 
