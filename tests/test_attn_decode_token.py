@@ -30,6 +30,11 @@ CASES = [
     (4, 1, 32, [40, 2000], 50, 4, True, False, 4),
     (16, 4, 16, [300, 18], -64, 0, True, True, 1),
     (16, 4, 16, [300, 18, 63], None, 0, False, False, 3),
+    (16, 4, 16, [64, 128, 0, 63], -64, 2, True, True, 1),      # the first position of a block of positions: its own key alone, no page is read
+    (16, 4, 16, [64, 130, 7], -64, 0, True, True, 3),
+    (8, 2, 16, [40, 64, 0, 31], 1, 4, True, True, 1),          # a window of the own key alone
+    (8, 2, 16, [40, 64, 33], 1, 0, False, True, 4),
+    (4, 1, 8, [32900, 5], None, 2, True, True, 3),             # a table row of more entries than a block keeps: only its own split's are copied
 ]
 
 
@@ -179,3 +184,47 @@ def test_where_one_launch_stands_for_two():
     assert not any(pays(g, 1, n, keys) for g in (7, 8, 16, 64) for n in (1, 64, 512) for keys in (16, 4096))
     # many blocks of few keys, also where a window keeps them few
     assert not pays(32, 8, 256, 512) and pays(32, 8, 256, 1024) and not pays(32, 8, 256, 4096, window=512) and not pays(32, 32, 64, 4096, chunk=256)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_parts,splits", [(1, 1), (2, 8), (4, 1), (4, 3)])
+def test_rows_whose_scale_is_still_to_be_applied(n_parts, splits):
+    """Parts of rows before their RMSNorm's scale (``UnscaledParts``, a share of the sum of squares for every part) as parts of rows behind it, and
+    against the formulas: without head norms, so that the scale is in every score and every value."""
+    from jax_vllm_amd.ops import kernels as K
+
+    n, nq, nkv, ps, width, eps = 3, 12, 4, 16, 1000, 1e-5
+    g = torch.Generator().manual_seed(n_parts + splits)
+    contexts = [70, 1, 200]
+    parts = torch.randn(n_parts, n, (nq + 2 * nkv) * D, generator=g)
+    ssq = torch.rand(n, 16, generator=g) * width                    # shares behind the parts' number are not read into the scale
+    ssq[:, n_parts:] = float("nan")
+    scale = torch.rsqrt(ssq[:, :n_parts].double().sum(-1, keepdim=True) / width + eps)
+    kp, vp = (torch.randn(1 + 13 * n, nkv, *s, generator=g).to(torch.bfloat16) for s in ((ps, D), (D, ps)))
+    tables = (1 + torch.arange(13 * n, dtype=torch.int32)).view(n, 13)
+    slots = torch.tensor([int(tables[i, c // ps]) * ps + c % ps for i, c in enumerate(contexts)], dtype=torch.int32).cuda()
+    pos = torch.tensor(contexts, dtype=torch.int32).cuda()
+    scratch = torch.empty(max(1, K.attn_decode_scratch_floats(n, nq, splits, D))).cuda()
+
+    def attend(qkv):
+        k, v, out = kp.cuda(), vp.cuda(), torch.full((n, nq * D), float("nan"), dtype=torch.bfloat16).cuda()
+        K.attn_decode_token(out, qkv, slots, None, None, 0.0, None, 0, k, v, tables.cuda(), pos, nq, nkv, D, 1 / math.sqrt(D), 0, splits, scratch)
+        return out.float().cpu(), k.cpu(), v.cpu()
+
+    out, k_out, v_out = attend(K.UnscaledParts(parts.cuda(), ssq.cuda(), width, eps))
+    x = (parts.double().sum(0) * scale).view(n, nq + 2 * nkv, D)
+    q, k, v = (part.to(torch.bfloat16).double() for part in x.split([nq, nkv, nkv], 1))
+    want = torch.zeros(n, nq, D, dtype=torch.float64)
+    for i, c in enumerate(contexts):
+        at = [(int(tables[i, j // ps]), j % ps) for j in range(c)]
+        for h in range(nq):
+            m = h // (nq // nkv)
+            keys = torch.stack([kp[p, m, s].double() for p, s in at] + [k[i, m]])
+            vals = torch.stack([vp[p, m, :, s].double() for p, s in at] + [v[i, m]])
+            want[i, h] = torch.softmax(keys @ q[i, h] / math.sqrt(D), 0) @ vals
+    torch.testing.assert_close(out.double(), want.view(n, -1), rtol=2e-2, atol=2e-2)      # as in the test above
+    for i, c in enumerate(contexts):      # heads are bfloat16 once they are scaled
+        torch.testing.assert_close(k_out[tables[i, c // ps], :, c % ps].double(), k[i], rtol=2 ** -7, atol=1e-6)
+        torch.testing.assert_close(v_out[tables[i, c // ps], :, :, c % ps].double(), v[i], rtol=2 ** -7, atol=1e-6)
+    # the scale in float before or behind the sum: a unit of a rounding of prepared heads, weights and results
+    torch.testing.assert_close(out, attend((parts * scale.float()).cuda())[0], rtol=2e-2, atol=2e-2)

@@ -152,3 +152,53 @@ def test_when_the_output_product_merges(monkeypatch):
     assert [pays(2, n, k, 8) for n, k in shapes] == [True, False, False, False, False, False]
     assert not any(pays(2, n, k, 16) or pays(1, n, k, 17) or pays(3, n, k, 4) for n, k in shapes)
     assert not pays(1, 8192, 10240, 16) and pays(1, 8192, 10240, 8) and pays(2, 1024, 4096, 4) and not pays(2, 1040, 4096, 4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("graphs", [True, False])
+def test_a_mixer_that_leaves_no_parts(graphs):
+    """An output product whose inner size (512) is not shared out leaves bfloat16 rows: the stream goes through the second norm's launch and back
+    into its own buffer.  One and two requests as three, whose rows are made by launches of their own."""
+    from jax_vllm_amd import LLM
+    from jax_vllm_amd.config.registry import resolve
+    from jax_vllm_amd.engine.entries import StepEntry
+    from jax_vllm_amd.ops import kernels as kernels_
+    from jax_vllm_amd.parts.model import DecoderModel
+
+    cfg = dict(architectures=["Qwen3ForCausalLM"], head_dim=128, rope_theta=1e6, rms_norm_eps=1e-6, tie_word_embeddings=False, max_position_embeddings=4096,
+               num_hidden_layers=3, hidden_size=2048, num_attention_heads=4, num_key_value_heads=2, intermediate_size=1024, vocab_size=512)
+    arch, typed, _ = resolve(cfg)
+    model = DecoderModel(arch.build_spec(typed))
+    g = torch.Generator().manual_seed(4)
+    tensors = {name: ((1 + 0.05 * torch.randn(t.shape, generator=g)) if len(t.shape) == 1 else torch.randn(t.shape, generator=g) * t.shape[-1] ** -0.5)
+               for name, t in model.tensor_specs().items()}
+    model.bind({n: t.cuda().to(BF if model.tensor_specs()[n].role == "matrix" else torch.float32) for n, t in tensors.items()}, BF)
+    made = []
+    linear_made = kernels_._linear_made
+    kernels_._linear_made = lambda x, *a: made.append(type(x).__name__) or linear_made(x, *a)
+    try:
+        def decode(groups):
+            llm = LLM(model, dtype="bf16", block_size=16, num_blocks=200, max_num_seqs=4, max_model_len=400, max_num_batched_tokens=2048,
+                      use_hip_graphs=graphs, enable_prefix_cache=False)
+            prompts = [torch.randint(0, 512, (n,), generator=torch.Generator().manual_seed(n)).tolist() for n in (40, 17, 99)]
+            out = [[] for _ in prompts]
+            for group in groups:
+                for i in group:
+                    llm.core.start_request(i)
+                llm.core.run([StepEntry(i, prompts[i], []) for i in group])
+                for step in range(4):
+                    for i, row in zip(group, llm.core.run([StepEntry(i, [5 + 7 * step + i], [0]) for i in group])):
+                        out[i].append(row.clone())
+            return torch.stack([torch.stack(o) for o in out])
+
+        want = decode([(0, 1, 2)])
+        assert not made
+        for groups in ([(0,), (1,), (2,)], [(0, 2), (1,)]):
+            got = decode(groups)
+            # one product a layer makes its rows (the other reads what the norm's launch leaves), as often as the launches run on the host
+            assert set(made) == {"PendingRows"} and len(made) % 3 == 0
+            assert len(made) <= 3 * 4 * len(groups) if not graphs else made
+            assert ((got - want).norm() / want.norm()).item() < 1.2e-2      # bfloat16 layers, as above
+            made.clear()
+    finally:
+        kernels_._linear_made = linear_made
