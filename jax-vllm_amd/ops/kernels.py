@@ -1366,6 +1366,8 @@ def _made_plan(m: int, w: torch.Tensor, gate_pairs: bool, partial_ok: bool, part
     return None
 
 
+# The row makers that are built: a block of columns is an array of its threads, so its size is fixed in the code.  256 x pieces x parts columns by blocks that
+# stay (of the pieces they take, 17 is missing), and 1,024, 2,048 or 4,096 by blocks of few rows; at other inner sizes rows come from launches of their own.
 MADE_PIECES = (4, 5, 8, 10, 12, 16, 20)
 MADE_FEW_INNER = (1024, 2048, 4096)
 

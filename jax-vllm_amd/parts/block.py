@@ -56,7 +56,8 @@ class PreNormBlock:
         return out.settled() if isinstance(out, K.BiasedOutput) else out
 
     def _made_by_readers(self, h, delta, mixer, feed_forward, ctx, mem) -> bool:
-        """Whether the products behind both norms make their rows themselves (one or two rows of a decode step)."""
+        """Whether the products behind both norms make their rows themselves (one or two rows of a decode step): both or neither, as the stream
+        goes to a second buffer and back."""
         n = h.shape[0]
         if n > K.MADE_MAX_ROWS or not self.has_feed_forward or self.residual_scale != 1.0 or not all(hasattr(p, "pending") for p in self.norms):
             return False
