@@ -21,6 +21,8 @@ from __future__ import annotations
 from dataclasses import dataclass, field
 from typing import Optional, Sequence
 
+import numpy as np
+
 from .page_pool import NULL_PAGE, OutOfPages, PagePool, chain_hash
 from .state_slots import StateSlotPool
 
@@ -199,7 +201,7 @@ class CacheManager:
         """The step has stored keys and values of these tokens: advance the context, hash the
         pages that became full, give back window pages that no later token will read."""
         rc = self.requests[request_id]
-        rc.tokens.extend(int(t) for t in token_ids)
+        rc.tokens.extend(token_ids.tolist() if isinstance(token_ids, np.ndarray) else map(int, token_ids))
         ps, ctx = self.page_size, rc.context_len
         if self.prefix_cache:
             pool, table = self.groups[0].pool, rc.tables[0]

@@ -20,6 +20,7 @@ import numpy as np
 import torch
 
 from ..cache.manager import CacheManager
+from ..cache.page_pool import NULL_PAGE
 from ..cache.storage import allocate_memories, cache_bytes_per_token, group_keys_of, has_state
 from ..config.engine import EngineConfig
 from .entries import StepEntry
@@ -148,13 +149,7 @@ class EngineCore:
         entries = [e for e in entries if len(e.tokens) > 0]
         if not entries:
             return torch.empty((0, self.vocab_size), dtype=torch.float32, device=self.device)
-        for e in entries:
-            for t in e.tokens:
-                if not 0 <= int(t) < self.vocab_size:
-                    raise ValueError(f"request {e.request_id!r}: token id {t} outside the vocabulary [0, {self.vocab_size})")
-            for w in e.want:
-                if not 0 <= int(w) < len(e.tokens):
-                    raise ValueError(f"request {e.request_id!r}: wanted place {w} outside its {len(e.tokens)} tokens")
+        ids = self._checked_tokens(entries)
         self._reserve_all([(e.request_id, len(e.tokens)) for e in entries])
         self._zero_new_state()
         if self._graphable(entries):
@@ -162,11 +157,35 @@ class EngineCore:
             if not borrow:
                 logits = logits.clone()
         else:
-            token_ids, ctx, logit_rows = self._build(entries)
+            token_ids, ctx, logit_rows = self._build(entries, ids)
             logits = self.model.forward(token_ids, ctx, self.memories, logit_rows)
+        at = 0
         for e in entries:
-            self.cache.commit(e.request_id, e.tokens)
+            self.cache.commit(e.request_id, ids[at:at + len(e.tokens)])
+            at += len(e.tokens)
         return logits
+
+    def _checked_tokens(self, entries) -> np.ndarray:
+        """The entries' token ids one after another; raises for an id outside the vocabulary or a wanted place outside its tokens."""
+        flat = []
+        for e in entries:
+            flat.extend(e.tokens)
+        try:
+            ids = np.asarray(flat)
+            good = ids.dtype.kind in "iu" and ids.ndim == 1 and ids.min() >= 0 and ids.max() < self.vocab_size \
+                and all(0 <= int(w) < len(e.tokens) for e in entries for w in e.want)
+        except (TypeError, ValueError, OverflowError):
+            good = False
+        if good:
+            return ids
+        for e in entries:      # numbers of other types, and what is wrong with the first bad one
+            for t in e.tokens:
+                if not 0 <= int(t) < self.vocab_size:
+                    raise ValueError(f"request {e.request_id!r}: token id {t} outside the vocabulary [0, {self.vocab_size})")
+            for w in e.want:
+                if not 0 <= int(w) < len(e.tokens):
+                    raise ValueError(f"request {e.request_id!r}: wanted place {w} outside its {len(e.tokens)} tokens")
+        return np.asarray([int(t) for t in flat], dtype=np.int64)
 
     def _reserve_all(self, needs) -> None:
         """Pages for every (request, new tokens) of a step, or ``OutOfPages`` with no table changed:
@@ -307,9 +326,9 @@ class EngineCore:
         if rows:
             torch._foreach_zero_(rows)      # few launches for all of a model's state tensors
 
-    def _build(self, entries):
+    def _build(self, entries, ids: np.ndarray):
         """All per-token and per-request integers of the step, packed on the host into one
-        pinned buffer and copied to the device at once."""
+        pinned buffer and copied to the device at once.  ``ids``: the entries' tokens one after another."""
         cache, ps = self.cache, self.page_size
         n_groups = len(self.group_keys)
         q_lens = [len(e.tokens) for e in entries]
@@ -318,11 +337,12 @@ class EngineCore:
         n, r = sum(q_lens), len(entries)
         tables = [[cache.block_table(e.request_id, g) for e in entries] for g in range(n_groups)]
         widths = [max(1, max(len(t) for t in tables[g])) for g in range(n_groups)]
-        m = sum(len(e.want) for e in entries)
+        starts = np.concatenate([[0], np.cumsum(q_lens)])
+        wanted = [at + int(w) for at, e in zip(starts.tolist(), entries) for w in e.want]
 
-        sizes = [n, n, n, r + 1, r, r, m] + [n] * n_groups + [r * w for w in widths] + [n]
-        offsets = np.concatenate([[0], np.cumsum(sizes)])
-        buf = torch.empty(int(offsets[-1]), dtype=torch.int32, pin_memory=True)
+        sizes = [n, n, n, r + 1, r, r, len(wanted)] + [n] * n_groups + [r * w for w in widths] + [n]
+        offsets = np.concatenate([[0], np.cumsum(sizes)]).tolist()
+        buf = torch.empty(offsets[-1], dtype=torch.int32, pin_memory=True)
         host = buf.numpy()
 
         def seg(i):
@@ -330,37 +350,26 @@ class EngineCore:
 
         tok, pos, treq, cu, ctxl, slot_ids, rows = (seg(i) for i in range(7))
         prev = seg(7 + 2 * n_groups)     # the token before each token in its request: a portion's first one comes from the cache manager
-        cu[0] = 0
-        at, row_at = 0, 0
-        for i, e in enumerate(entries):
-            ql = q_lens[i]
-            tok[at:at + ql] = np.asarray(e.tokens, dtype=np.int32)
-            prev[at] = cache.last_token(e.request_id)
-            prev[at + 1:at + ql] = tok[at:at + ql - 1]
-            pos[at:at + ql] = np.arange(ctx_lens[i], ctx_lens[i] + ql, dtype=np.int32)
-            treq[at:at + ql] = i
-            for w in e.want:
-                rows[row_at] = at + int(w)
-                row_at += 1
-            at += ql
-            cu[i + 1] = at
-        ctxl[:] = ctx_lens
-        slot_ids[:] = slots
+        cu[:], ctxl[:], slot_ids[:], rows[:], tok[:] = starts, ctx_lens, slots, wanted, ids
+        treq[:] = np.repeat(np.arange(r, dtype=np.int32), q_lens)
+        pos[:] = np.arange(n, dtype=np.int32) + (ctxl - cu[:r])[treq]
+        prev[1:] = tok[:-1]
+        prev[cu[:r]] = [cache.last_token(e.request_id) for e in entries]
         for g in range(n_groups):
-            sm = seg(7 + g)
-            at = 0
-            for i, e in enumerate(entries):
-                sm[at:at + q_lens[i]] = cache.slot_mapping(e.request_id, g, q_lens[i])
-                at += q_lens[i]
             bt = seg(7 + n_groups + g).reshape(r, widths[g])
             bt[:] = 0
             for i, t in enumerate(tables[g]):
                 bt[i, :len(t)] = t
+            pages = bt[treq, pos // ps]
+            if (pages == NULL_PAGE).any():
+                for e, ql in zip(entries, q_lens):
+                    cache.slot_mapping(e.request_id, g, ql)      # says which position has none
+            np.add(pages * ps, pos % ps, out=seg(7 + g))
 
         dev = buf.to(self.device, non_blocking=True)
 
         def dseg(i):
-            return dev[int(offsets[i]):int(offsets[i + 1])]
+            return dev[offsets[i]:offsets[i + 1]]
 
         ctx = StepContext(
             num_tokens=n, num_requests=r, positions=dseg(1), token_req=dseg(2), cu_seqlens=dseg(3),

@@ -394,8 +394,9 @@ def gate_activation_known(activation) -> bool:
 
 def _gate_act(activation) -> tuple:
     """(id, limit, slope) of a gated feed-forward's activation as the entry points take it."""
-    _need(gate_activation_known(activation), f"no kernel for the gate activation {activation!r}: there are {sorted(GATE_ACTIVATIONS)}, "
-          "the clamped one as (\"clamped\", limit, slope)")
+    if not gate_activation_known(activation):
+        raise KernelArgumentError(f"no kernel for the gate activation {activation!r}: there are {sorted(GATE_ACTIVATIONS)}, "
+                                  "the clamped one as (\"clamped\", limit, slope)")
     name, limit, slope = activation if isinstance(activation, tuple) else (activation, 0.0, 0.0)
     return c_int(GATE_ACTIVATIONS[name]), c_float(limit), c_float(slope)
 
@@ -1225,6 +1226,7 @@ SHARES_MAX_ROWS = 1024
 _SHARES_TILES = {(128, 128): 0.6, (256, 128): 0.9, (256, 256): 1.6}      # rows of x, rows of w: microseconds a chunk of 64 columns
 
 
+@functools.lru_cache(maxsize=4096)
 def shares_plan(m: int, n: int, k: int, cus: int = 256):
     """How ``linear`` runs a bfloat16 product of 129 to 1,024 rows whose reader adds partial products through
     ``gemm_shares``: (rows of x, rows of w of a tile, parts of the inner size), or None where the library is better.
@@ -1252,6 +1254,7 @@ def shares_plan(m: int, n: int, k: int, cus: int = 256):
     return best[1] if best is not None and best[0] < 3.0 + k * (0.0036 + 1.32e-9 * m * n) else None
 
 
+@functools.lru_cache(maxsize=4096)
 def tall_shares_plan(m: int, n: int, k: int, cus: int = 256):
     """The same for 1,025 to 1,792 rows against a long inner size: halves of it by tiles of 192 x 256, or of 256 x 256 where those would
     be more blocks than compute units, if they are one round that leaves at most a quarter of the units idle.  The library, whose tiles leave
@@ -2496,6 +2499,7 @@ def moe_tile_rows_for(dtype, hidden: int, ff: int, entries: int, experts: int) -
     return moe_tile_rows()
 
 
+@functools.lru_cache(maxsize=4096)
 def moe_one_launch(n: int, experts: int, top: int, always: int = 0) -> bool:
     """Whether choice and grouping of n tokens run as one block."""
     return bool(library.core().jv_moe_route_group_fits(c_int(n), c_int(experts), c_int(top), c_int(always)))
@@ -2524,6 +2528,7 @@ def _router_logits_plan(x, w_router, one_launch: bool):
 ROUTER_FUSED_MAX_ROWS = 64      # 17..64 rows: logits and choice in one launch
 
 
+@functools.lru_cache(maxsize=4096)
 def rows_by_tiles(m: int, n: int, k: int, cus: int = 256) -> bool:
     """Whether ``gemm_rows_f32out`` runs as tiles of 128 x 128 (``gemm_shares``, the inner size in one piece) instead of blocks of 16
     rows that share the inner size out to their waves: those are one round trip to memory while each compute unit has one of
@@ -2602,7 +2607,8 @@ def moe_route(logits: "torch.Tensor | None", top: int, x=None, w_router=None, lo
         if logits is not None and logits_out is not None:
             whole = logits.sum(0) if logits.dim() == 3 else logits
             logits_out.copy_(whole if bias is None else whole + bias)
-    _need(score in ROUTER_SCORES, f"no router score {score!r}: there are {sorted(ROUTER_SCORES)}")
+    if score not in ROUTER_SCORES:
+        raise KernelArgumentError(f"no router score {score!r}: there are {sorted(ROUTER_SCORES)}")
     if logits is not None:
         _dev(logits)
         _f32(logits, "logits")
@@ -2621,8 +2627,8 @@ def moe_route(logits: "torch.Tensor | None", top: int, x=None, w_router=None, lo
     if bias is not None:
         _dev(bias)
         _f32(bias, "bias", experts)
-    _need(score in CORRECTED_SCORES or (correction is None and weight_scale == 1.0),
-          f"a correction of the choice and a constant on the weights belong to the scores {CORRECTED_SCORES}")
+    if score not in CORRECTED_SCORES and (correction is not None or weight_scale != 1.0):
+        raise KernelArgumentError(f"a correction of the choice and a constant on the weights belong to the scores {CORRECTED_SCORES}")
     if correction is not None:
         _dev(correction)
         _f32(correction, "correction", experts)

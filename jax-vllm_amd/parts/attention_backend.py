@@ -17,6 +17,7 @@ from __future__ import annotations
 from dataclasses import dataclass
 from typing import Optional
 
+import numpy as np
 import torch
 
 from ..ops import kernels as K
@@ -25,6 +26,13 @@ TARGET_BLOCKS = 256          # blocks of the decode kernel that fill the chip: o
                              # 1,060 keys over 8 kv heads take 13.7 us with 4 splits, 15.5 with 8)
 DECODE_TILE = K.ATTN_DECODE_TILE_KEYS      # keys of a tile of the decode kernel; a block has 4 waves with a tile each
 RESIDENT_BLOCKS = 2          # blocks of the prefill kernel that a compute unit holds at once
+
+
+def upload_i32(values, device) -> torch.Tensor:
+    """int32 on the device from host integers, through pinned memory."""
+    staged = torch.empty(len(values), dtype=torch.int32, pin_memory=True)
+    staged.numpy()[:] = values
+    return staged.to(device, non_blocking=True)
 
 
 @dataclass
@@ -88,7 +96,13 @@ def prefill_work_items(q_lens, context_lens, g: int, window: int, group_rows: in
         if ql <= 1:
             continue
         groups = []
-        for m0 in range(0, ql * g, group_rows):
+        if ql * g > 16 * group_rows:       # all groups at once: 512 of them 90 us instead of 350, a few are quicker one by one
+            m0 = np.arange(0, ql * g, group_rows)
+            end, first = cl + (np.minimum(ql * g, m0 + group_rows) - 1) // g + 1, cl + m0 // g
+            begin = np.maximum(0, first - window + 1) if window > 0 else first - first % -window if window else 0 * first
+            tiles = -(-end // KEY_TILE) - begin // KEY_TILE + np.minimum(begin // KEY_TILE, -(-keep // KEY_TILE))
+            groups = list(zip(tiles.tolist(), m0.tolist()))
+        for m0 in range(0, ql * g if not groups else 0, group_rows):
             last_row = min(ql * g, m0 + group_rows) - 1
             end = cl + last_row // g + 1
             first = cl + m0 // g
@@ -183,7 +197,7 @@ def plan_mfma(ctx, nq: int, nkv: int, head_dim: int, window: int, device, keep: 
         splits = max(splits, K.attn_decode_min_splits(widest, ctx.page_size, keep))
     decode_only = len(decode) == len(ctx.q_lens_host)       # requests 0, 1, ...: the kernel needs no list
     flat = [x for item in prefill for x in item] + ([] if decode_only else decode)
-    dev = torch.tensor(flat, dtype=torch.int32).pin_memory().to(device, non_blocking=True) if flat else None
+    dev = upload_i32(flat, device) if flat else None
     n_pre = len(prefill)
     scratch = None
     if decode and splits > 1:
@@ -228,8 +242,7 @@ def plan_f32(ctx, nq: int, nkv: int, head_dim: int, window: int, device, keep: i
     parts = None
     if splits > 1:
         parts = torch.empty(K.attn_f32_part_floats(len(items), nkv, ranges, head_dim), dtype=torch.float32, device=device)
-    flat = torch.tensor([x for item in items for x in item], dtype=torch.int32)
-    return F32Plan(flat.pin_memory().to(device, non_blocking=True), len(items), splits, parts)
+    return F32Plan(upload_i32([x for item in items for x in item], device), len(items), splits, parts)
 
 
 def token_possible(att, ctx, mem, interleaved: bool, rotary_dim: int) -> bool:
