@@ -339,10 +339,12 @@ static int dispatch_nks(int nks, void* y, const void* x, const void* W, int M, i
 // which write float partial products to y + group * M * ldy (added by the reader, in order).
 // Rows of x that come un-normalised from add_parts_unscaled_kernel: output row m is multiplied by
 // rsqrt(sum_j ssq[m][j] / width + eps), j < shares, ssq rows of 16 floats (the norm's scale commutes with the
-// product; with the inner size shared out every partial product is scaled).  ssq == nullptr: no scale.
+// product; with the inner size shared out every partial product is scaled).  ssq == nullptr: no scale.  Rows that gemm_thin.hip left have up to 256
+// shares, in rows of as many floats: every wave adds an eighth of them.
 struct RowScale {
   const float* ssq;
-  int shares;       // at most 16
+  int shares;       // at most 16, or with rows of 256 floats 256, a multiple of 4
+  int stride;       // floats of a row of ssq: 16 or 256
   float inv_width, eps;
   JvAct act;        // PAIRS: the gate's activation
 };
@@ -401,12 +403,17 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
   // without a scale the loads read x (no load inside a branch) and get no weight
   // (one 16-byte load a lane: the 4 lanes of a row hold its 16 shares; every block reads these few lines,
   // so every instruction more would queue up at one place in the L2)
-  f32x4 row_sq = {0.f, 0.f, 0.f, 0.f};
+  f32x4 row_sq[2];
+  __shared__ float sq_part[8][16];
+  const bool many = rs.stride > 16;
   if constexpr (SRC == ROWS_GIVEN) {
-    const int m = min((wk < MT ? wk : 0) * 16 + li, M - 1);
-    const float* sp = rs.ssq ? rs.ssq + (long long)m * 16 + lc * 4 : (const float*)x;
-    row_sq = *(const f32x4*)sp;
+    const int m = min((wk < MT ? wk : 0) * 16 + li, M - 1), at = many ? wk * 32 + lc * 8 : lc * 4;
+    const float* sp = rs.ssq ? rs.ssq + (long long)m * rs.stride : (const float*)x;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) row_sq[i] = *(const f32x4*)(sp + (!rs.ssq ? 0 : many ? min(at + i * 4, rs.shares - 4) : at));
   }
+  bool first_tile = true;
+  float inv = 1.f;
   // pieces first .. first + CNT - 1 of a tile
   auto load_pieces = [&](int tile, int first, auto& a) {
     constexpr int CNT = sizeof(a) / sizeof(a[0]);
@@ -432,6 +439,14 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
   auto reduce_store = [&](int tile, const f32x4 (&acc)[MT], int buf) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) *(f32x4*)(red[buf] + ((wk * MT + mt) * 256 + lane * 4)) = acc[mt];
+    if (MT == 1 && SRC == ROWS_GIVEN && many && first_tile) {
+      float sq = 0.f;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) sq += wk * 32 + lc * 8 + i * 4 < rs.shares ? (row_sq[i][0] + row_sq[i][1]) + (row_sq[i][2] + row_sq[i][3]) : 0.f;
+      sq += __shfl_xor(sq, 16, 64);
+      sq += __shfl_xor(sq, 32, 64);
+      if (lc == 0) sq_part[wk][li] = sq;
+    }
     __syncthreads();
     if (wk < MT) {                                 // wave mt adds row tile mt, in fixed order: wave 0, 1, ..., 7
       const int mt = wk;
@@ -443,13 +458,20 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
       }
       const int nb = tile * 16 + lc * 4;           // the accumulator holds y^T[n = lc*4+e][m = mt*16 + li]
       const int m = mt * 16 + li;
-      if (rs.ssq) {                                // a fixed order of adding: the same scale in every tile and block
-        float sq = 0.f;
+      if (SRC == ROWS_GIVEN && rs.ssq) {           // a fixed order of adding: the same scale in every tile and block
+        if (first_tile) {
+          float sq = 0.f;
+          if (MT == 1 && many) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sq += lc * 4 + j < rs.shares ? row_sq[j] : 0.f;
-        sq += __shfl_xor(sq, 16, 64);
-        sq += __shfl_xor(sq, 32, 64);
-        const float inv = rsqrtf(sq * rs.inv_width + rs.eps);
+            for (int w = 0; w < 8; ++w) sq += sq_part[w][li];
+          } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sq += lc * 4 + j < rs.shares ? row_sq[0][j] : 0.f;
+            sq += __shfl_xor(sq, 16, 64);
+            sq += __shfl_xor(sq, 32, 64);
+          }
+          inv = rsqrtf(sq * rs.inv_width + rs.eps);
+        }
         s[0] *= inv; s[1] *= inv; s[2] *= inv; s[3] *= inv;
       }
       if (SRC == ROWS_RESIDUAL && PAIRS) {
@@ -471,6 +493,7 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
         }
       }
     }
+    first_tile = false;
   };
   // The next tile's weights are asked for before this tile is multiplied, without a condition (beyond the
   // last tile the last one is read again): after a conditional prefetch the compiler must assume that
@@ -640,7 +663,9 @@ static int gemm_skinny_entry(void* y, const void* x, const void* W, int M, int N
                              int out_f32, JvAct gate_act, int wr, int wk, int nks, int ksplit, RowScale rs,
                              void* stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (rs.ssq && (wr != -2 || rs.shares < 1 || rs.shares > 16)) return (int)hipErrorInvalidValue;   // only the staying blocks scale rows
+  // only the staying blocks scale rows
+  if (rs.ssq && (wr != -2 || rs.shares < 1 || rs.shares > rs.stride || (rs.stride != 16 && (rs.stride != 256 || M > 16 || rs.shares % 4))))
+    return (int)hipErrorInvalidValue;
   if (M > 64 || K <= 0 || K % 8 != 0 || ldx % 8 != 0) return (int)hipErrorInvalidValue;
   if (gate_act.id && (!jv_act_known(gate_act.id) || out_f32 || N % 2 != 0 || wr == -1)) return (int)hipErrorInvalidValue;
   rs.act = gate_act;
@@ -686,15 +711,15 @@ extern "C" int jv_gemm_skinny_bf16(void* y, const void* x, const void* W, int M,
 }
 
 // The same for rows of x that add_parts_unscaled left un-normalised (blocks that stay only, wr == -2):
-// output row m is multiplied by rsqrt(sum_{j < shares} ssq[m * 16 + j] / width + eps).
+// output row m is multiplied by rsqrt(sum_{j < shares} ssq[m * stride + j] / width + eps).
 extern "C" int jv_gemm_skinny_scaled_bf16(void* y, const void* x, const void* W, int M, int N, int K,
                                           long long ldx, long long ldy, int out_f32, int gate_act, float act_limit,
                                    float act_slope, int wr,
-                                          int wk, int nks, int ksplit, const float* ssq, int shares, int width,
-                                          float eps, void* stream) {
-  if (!ssq || width <= 0) return (int)hipErrorInvalidValue;
+                                          int wk, int nks, int ksplit, const float* ssq, int shares, int ssq_stride,
+                                          int width, float eps, void* stream) {
+  if (!ssq || width <= 0 || ((uintptr_t)ssq & 15)) return (int)hipErrorInvalidValue;
   return gemm_skinny_entry(y, x, W, M, N, K, ldx, ldy, out_f32, JvAct{gate_act, act_limit, act_slope}, wr, wk, nks, ksplit,
-                           RowScale{ssq, shares, 1.f / (float)width, eps, JvAct{}}, stream);
+                           RowScale{ssq, shares, ssq_stride, 1.f / (float)width, eps, JvAct{}}, stream);
 }
 
 // One or two rows that the blocks make themselves (RowSource): blocks that stay, an inner size of ksplit * 256 * nl columns exactly.

@@ -358,7 +358,7 @@ static int launch_rope_wide(void* qkv, const int* slot_mapping, const float* q_w
 DEFINE_ROPE(bf16, bf16_t)
 DEFINE_ROPE(f32, float)
 
-// The same with the projection given as n_parts (2..4) float partial products
+// The same with the projection given as n_parts (1..4) float partial products
 // [n_parts][tokens][heads * D]; q is written to `qkv` (the q heads of each row), k and v to their
 // pages.  Only what the fast path takes: head size 128 or 256, half-split pairing, fully rotated
 // or not rotated; anything else is refused (the caller then asks for a whole product).
@@ -382,15 +382,15 @@ extern "C" int jv_qk_norm_rope_write_parts_bf16(
     int page_size, int n_tokens, int nq, int nkv, int D, void* stream) {
   if (n_tokens <= 0) return 0;
   const int half = rotary_dim / 2;
-  if ((D != 128 && D != 256) || n_parts < 2 || n_parts > 4 || (rotary_dim & 1) || rotary_dim > D ||
+  if ((D != 128 && D != 256) || n_parts < 1 || n_parts > 4 || (rotary_dim & 1) || rotary_dim > D ||
       (cos_sin && (half % 64 != 0 || half <= 0)))
     return (int)hipErrorInvalidValue;
 #define ROPE_PARTS_CASE(E, NP)                                                                             \
   if (D == 64 * E && n_parts == NP)                                                                        \
     return launch_rope_parts<bf16_t, E, NP>(qkv, parts, part_stride, slot_mapping, q_w, k_w, eps, cos_sin, \
                                             rotary_dim, k_pages, v_pages, page_size, n_tokens, nq, nkv, stream);
-  ROPE_PARTS_CASE(2, 2) ROPE_PARTS_CASE(2, 3) ROPE_PARTS_CASE(2, 4)
-  ROPE_PARTS_CASE(4, 2) ROPE_PARTS_CASE(4, 3) ROPE_PARTS_CASE(4, 4)
+  ROPE_PARTS_CASE(2, 1) ROPE_PARTS_CASE(2, 2) ROPE_PARTS_CASE(2, 3) ROPE_PARTS_CASE(2, 4)
+  ROPE_PARTS_CASE(4, 1) ROPE_PARTS_CASE(4, 2) ROPE_PARTS_CASE(4, 3) ROPE_PARTS_CASE(4, 4)
 #undef ROPE_PARTS_CASE
   return (int)hipErrorInvalidValue;
 }

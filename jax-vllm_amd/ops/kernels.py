@@ -151,13 +151,33 @@ class UnscaledRows:
     product with them gives has to be multiplied by ``rsqrt(sum(ssq[m]) / width + eps)`` (the scale of
     a row commutes with the product).  ``linear`` does that in the epilogue of its streaming kernels."""
 
+    share, max_shares = UNSCALED_SHARE, UNSCALED_MAX_SHARES
+
     def __init__(self, x: torch.Tensor, ssq: torch.Tensor, width: int, eps: float):
         self.x, self.ssq, self.width, self.eps = x, ssq, int(width), float(eps)   # ssq [rows, 16], width / 512 of them used
-        self.shares = self.width // UNSCALED_SHARE
+        self.shares = self.width // self.share
 
     shape = property(lambda self: self.x.shape)
     dtype = property(lambda self: self.x.dtype)
     device = property(lambda self: self.x.device)
+
+
+class StreamRows(UnscaledRows):
+    """The same as ``gemm_into_stream`` leaves them, with a share of a row's sum of squares for every 16 columns (ssq [rows, 256]); the
+    reader is asked with ``linear_takes_stream_rows``."""
+
+    share, max_shares = 16, 256
+
+
+class PendingProduct:
+    """A sublayer's last product, still to be made: x @ w.T joins the residual stream.  ``gemm_into_stream`` does both in one launch,
+    ``linear`` gives the product as its readers take it."""
+
+    def __init__(self, x: torch.Tensor, w: torch.Tensor):
+        self.x, self.w = x, w
+
+    def linear(self):
+        return linear(self.x, self.w, partial_ok=True)
 
 
 def unscaled_rows_possible(dtype, n_rows: int, hidden: int) -> bool:
@@ -456,7 +476,7 @@ def qk_norm_rope_write(qkv, slot_mapping, q_weight, k_weight, eps, cos_sin, rota
                        k_pages, v_pages, page_size, nq, nkv, head_dim, parts=None) -> None:
     """Per-head q/k RMSNorm (if weights given), rotation (if a ``rope_table`` is given), q in
     place, k and v into their pages (if pages given): K [pages, nkv, page_size, D], V transposed
-    [pages, nkv, D, page_size].  With ``parts`` (float32 [2..4, tokens, (nq + 2 nkv) * D], see
+    [pages, nkv, D, page_size].  With ``parts`` (float32 [1..4, tokens, (nq + 2 nkv) * D], see
     ``linear(..., partial_ok=True)``) the input is the sum of the parts, added in order, and
     ``qkv`` only receives the q heads."""
     _dev(qkv, slot_mapping, q_weight, k_weight, cos_sin, k_pages, v_pages, parts)
@@ -476,8 +496,8 @@ def qk_norm_rope_write(qkv, slot_mapping, q_weight, k_weight, eps, cos_sin, rota
     if parts is not None:
         _need(rope_takes_parts(qkv.dtype, head_dim, interleaved, rotary_dim, cos_sin is not None),
               "partial products are taken for bfloat16, head size 128 or 256, half-split pairing, full rotation")
-        _need(parts.dtype == torch.float32 and parts.dim() == 3 and 2 <= parts.shape[0] <= 4
-              and parts.shape[1:] == qkv.shape, "parts must be float32 [2..4, tokens, (nq + 2 nkv) * D]")
+        _need(parts.dtype == torch.float32 and parts.dim() == 3 and 1 <= parts.shape[0] <= 4
+              and parts.shape[1:] == qkv.shape, "parts must be float32 [1..4, tokens, (nq + 2 nkv) * D]")
         _check(
             library.core().jv_qk_norm_rope_write_parts_bf16(
                 _ptr(qkv), _ptr(parts), c_int(parts.shape[0]), c_longlong(parts.stride(0)),
@@ -937,9 +957,9 @@ def gemm_skinny(x: torch.Tensor, w: torch.Tensor, out_dtype=torch.bfloat16, gate
     if row_scale is not None:
         _need(block_shape[0] == -2, "only the blocks that stay scale their output rows")
         _need(row_scale.x is x and row_scale.ssq.is_cuda and row_scale.ssq.dtype == torch.float32
-              and row_scale.ssq.is_contiguous() and tuple(row_scale.ssq.shape) == (m, UNSCALED_MAX_SHARES)
-              and 1 <= row_scale.shares <= UNSCALED_MAX_SHARES, "row_scale does not belong to x")
-        _check(library.core().jv_gemm_skinny_scaled_bf16(*common, _ptr(row_scale.ssq), c_int(row_scale.shares),
+              and row_scale.ssq.is_contiguous() and tuple(row_scale.ssq.shape) == (m, row_scale.max_shares)
+              and 1 <= row_scale.shares <= row_scale.max_shares, "row_scale does not belong to x")
+        _check(library.core().jv_gemm_skinny_scaled_bf16(*common, _ptr(row_scale.ssq), c_int(row_scale.shares), c_int(row_scale.ssq.shape[1]),
                                                          c_int(row_scale.width), c_float(row_scale.eps), _stream()),
                "gemm_skinny")
         return out
@@ -1205,6 +1225,98 @@ def few_tile(m: int, n: int, k: int, cus: int = 256) -> "int | None":
     return 32 if cus < tiles <= 1.5 * cus or (m > 8 and tiles > 3 * cus and k >= 1536) else 16
 
 
+def thin_slots(m: int, n: int, k: int) -> "int | None":
+    """Slots of the rings of ``csrc/gemm_thin.hip`` where it takes a product of up to 16 rows (any inner size that is a multiple of 64), or None
+    where blocks of eight waves with x in registers (``csrc/gemm_few.hip``) are better: rows of W that give most units one block of 16 and some two, at
+    9 rows or more (us there / here at 16 rows: 5,120 x 1,024 5.1 / 5.5, 5,120 x 3,072 10.4 / 11.4, 6,144 x 3,072 11.2 / 11.7; at 8 rows 4.75 / 4.6, 9.4 / 9.1, 10.2 /
+    9.6), and many of them against short inner sizes (12,288 x 512 at 8 rows 4.7 / 5.0, x 1,024 6.8 / 7.2).  Elsewhere, 54 sizes of 512 to 8,192 rows of W
+    and 512 to 4,096 columns at 1, 4, 8 and 16 rows: 0.82 to 1.01 of the time there."""
+    if 4096 < n <= 6144 and m > 8 and k > 512 or n > 8192 and k <= 1024:
+        return None
+    return 4 if n <= 4096 and k > 512 or n > 16384 else 2
+
+
+_NO_SCALE = (c_void_p(None), c_int(0), c_int(0), c_float(0.0))
+
+
+def gemm_thin_scaled(rows: "StreamRows", w: torch.Tensor, gate_pairs: "str | tuple | None" = None) -> torch.Tensor:
+    """float32 [M, N] of ``StreamRows`` against bfloat16 w [N, K], their norm's scale applied, or with ``gate_pairs`` the activation, bfloat16 [M, N / 2]."""
+    x, ssq = rows.x, rows.ssq
+    _dev(x, w, ssq)
+    _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "gemm_thin takes bfloat16")
+    m, k = x.shape
+    n = w.shape[0]
+    _need(w.shape[1] == k and 0 < m <= SKINNY_AUTO_ROWS and k % 64 == 0 and n % 4 == 0, "inner sizes differ, or more than 16 rows")
+    _need(ssq.dtype == torch.float32 and tuple(ssq.shape) == (m, rows.max_shares) and rows.width == k and k <= 16 * rows.max_shares, "the scale does not belong to x")
+    y = torch.empty((m, n // 2 if gate_pairs else n), dtype=torch.bfloat16 if gate_pairs else torch.float32, device=x.device)
+    _check(library.core().jv_gemm_thin_bf16(
+        _ptr(y), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), c_longlong(k), c_int(FEW_MODES["pairs" if gate_pairs else "float"]),
+        *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), c_int(thin_slots(1, n, k) or 2), _ptr(ssq), c_int(rows.shares), c_int(rows.width),
+        c_float(rows.eps), _stream()), "gemm_thin")
+    return y
+
+
+STREAM_PRODUCT_MAX_WIDTH = 4096      # 256 blocks of 16 columns: one round, and as many shares of a row's sum of squares
+
+
+def stream_product_possible(n_rows: int, w: torch.Tensor) -> bool:
+    """Whether ``gemm_into_stream`` takes a product of so many bfloat16 rows with w."""
+    n, k = w.shape
+    return (w.dtype == torch.bfloat16 and 0 < n_rows <= SKINNY_AUTO_ROWS and k % 64 == 0 and k > 0 and n % 64 == 0 and n <= STREAM_PRODUCT_MAX_WIDTH
+            and w.is_contiguous() and w.data_ptr() % 16 == 0)
+
+
+def gemm_into_stream(h: torch.Tensor, x: torch.Tensor, w: torch.Tensor, weight=None, eps: float = 0.0) -> "StreamRows | None":
+    """h += x @ w.T in the float residual stream, in one launch; with the next norm's ``weight`` returns the rows h * weight with the shares of
+    their sums of squares.  See ``csrc/gemm_thin.hip``; ask ``stream_product_possible`` first."""
+    _dev(h, x, w, weight)
+    _f32(h, "h")
+    m, k = x.shape
+    n = w.shape[0]
+    _need(x.dtype == torch.bfloat16 and w.shape[1] == k and tuple(h.shape) == (m, n) and stream_product_possible(m, w) and x.data_ptr() % 16 == 0,
+          "up to 16 bfloat16 rows against a matrix of up to 4,096 rows of whole chunks of 64 columns, on 16 bytes")
+    rows = ssq = None
+    if weight is not None:
+        _f32(weight, "weight", n)
+        rows = torch.empty((m, n), dtype=torch.bfloat16, device=h.device)
+        ssq = torch.empty((m, StreamRows.max_shares), dtype=torch.float32, device=h.device)      # n / 16 of a row's 256 are written
+    _check(library.core().jv_gemm_thin_stream_bf16(_ptr(h), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), c_longlong(k), c_int(4), _ptr(weight),
+                                                   _ptr(rows), _ptr(ssq), _stream()), "gemm_into_stream")
+    return None if weight is None else StreamRows(rows, ssq, n, eps)
+
+
+def _stream_rows_plan(m: int, w: torch.Tensor, gate_pairs: bool, partial_ok: bool, partial_max_width):
+    """How a product reads ``StreamRows``: the plan of blocks that stay, "thin", or None where neither takes them.  Every block reads the shares of
+    the rows' sums of squares, so many small blocks pay for them (24,576 x 4,096 with its activation at 8 rows 38.5 by them, 37.1 without a scale)."""
+    n, k = w.shape
+    if (w.dtype != torch.bfloat16 or not 0 < m <= SKINNY_AUTO_ROWS or k % 64 or not 0 < k <= STREAM_PRODUCT_MAX_WIDTH or n % 4 or not w.is_contiguous()
+            or w.data_ptr() % 16 or not (gate_pairs or partial_ok)):
+        return None
+    if n > 4096:
+        plan = streaming_plan(m, n, k, gate_pairs, partial_ok, w.device, partial_max_width)
+        if plan is not None and plan[0] != TILE64 and plan[0][0] == -2:
+            return plan
+    return "thin" if n <= 8192 else None
+
+
+def linear_takes_stream_rows(n_rows: int, w: torch.Tensor, gate_pairs: bool = False, partial_ok: bool = False,
+                             partial_max_width: int | None = PARTIAL_SUM_MAX_WIDTH) -> bool:
+    """Whether ``linear`` with these arguments multiplies ``StreamRows``."""
+    return _stream_rows_plan(n_rows, w, gate_pairs, partial_ok, partial_max_width) is not None
+
+
+def _linear_stream_rows(rows: "StreamRows", w: torch.Tensor, gate_pairs, partial_ok: bool, partial_max_width):
+    plan = _stream_rows_plan(rows.shape[0], w, bool(gate_pairs), partial_ok, partial_max_width)
+    _need(plan is not None, "no product applies these rows' scale (ask linear_takes_stream_rows first)")
+    if plan == "thin":
+        y = gemm_thin_scaled(rows, w, gate_pairs)
+        return y if gate_pairs else y.view(1, *y.shape)
+    shape, parts = plan
+    if parts > 1:
+        return gemm_skinny(rows.x, w, torch.float32, block_shape=shape, ksplit=parts, row_scale=rows)
+    return gemm_skinny(rows.x, w, torch.bfloat16 if gate_pairs else torch.float32, gate_pairs=gate_pairs, block_shape=shape, row_scale=rows)
+
+
 def gemm_few(x: torch.Tensor, w: torch.Tensor, tile: int, gate_pairs: "str | tuple | None" = None, out_dtype=torch.bfloat16) -> torch.Tensor:
     """x @ w.T for up to 16 rows of bfloat16 x against bfloat16 w [N, K], K a multiple of 64 up to 4,096, ``tile`` (16 or 32) rows of w a
     block: see ``csrc/gemm_few.hip``.  bfloat16 or float32 [M, N], or with ``gate_pairs`` the activation, bfloat16 [M, N / 2]."""
@@ -1216,6 +1328,12 @@ def gemm_few(x: torch.Tensor, w: torch.Tensor, tile: int, gate_pairs: "str | tup
     _need(out_dtype in (torch.bfloat16, torch.float32) and not (gate_pairs and out_dtype == torch.float32), "the activation's result is bfloat16")
     y = torch.empty((m, n // 2 if gate_pairs else n), dtype=out_dtype, device=x.device)
     mode = "pairs" if gate_pairs else "float" if out_dtype == torch.float32 else "rows"
+    slots = thin_slots(m, n, k)
+    if slots is not None:
+        _check(library.core().jv_gemm_thin_bf16(
+            _ptr(y), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), c_longlong(k), c_int(FEW_MODES[mode]),
+            *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), c_int(slots), *_NO_SCALE, _stream()), "gemm_few")
+        return y
     _check(library.core().jv_gemm_few_bf16(
         _ptr(y), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), c_longlong(k), c_int(FEW_MODES[mode]),
         *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), c_int(tile), _stream()), "gemm_few")
@@ -1305,6 +1423,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
     scale = None
     if isinstance(x, (PendingRows, SplitHeads)):
         return _linear_made(x, w, gate_pairs, partial_ok, partial_max_width)
+    if isinstance(x, StreamRows):
+        return _linear_stream_rows(x, w, gate_pairs, partial_ok, partial_max_width)
     if isinstance(x, UnscaledRows):
         scale, x = x, x.x
     if x.dtype == torch.float32:

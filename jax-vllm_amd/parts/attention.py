@@ -219,6 +219,15 @@ class GroupedQueryAttention:
         """x goes into the qkv product and nowhere else: the norm before may leave its scale to that product."""
         return K.linear_takes_unscaled_rows(n_rows, self.w_qkv, partial_ok=self._qkv_parts_ok(), partial_max_width=None)
 
+    def takes_stream_rows(self, n_rows: int) -> bool:
+        """Whether the qkv product reads ``K.StreamRows`` (its float result goes to a kernel that adds parts)."""
+        return (not self.wide and not self.filtered and self.b_qkv is None and self._qkv_parts_ok()
+                and K.linear_takes_stream_rows(n_rows, self.w_qkv, partial_ok=True, partial_max_width=None))
+
+    def leaves_product(self, n_rows: int) -> bool:
+        """Whether ``forward`` takes ``leave_product`` for so many rows: the output product is then left to the block."""
+        return not self.wide and not self.filtered and self.b_o is None and K.stream_product_possible(n_rows, self.w_o)
+
     def takes_pending_rows(self, n_rows: int, ctx: StepContext, mem: LayerMemory) -> bool:
         """Whether the qkv product may make its rows itself (``K.PendingRows``): only the launch behind it that goes from the product to the
         attention applies the norm's scale to its parts."""
@@ -244,7 +253,7 @@ class GroupedQueryAttention:
         return self._forward_wide(proj, ctx, mem)
 
     # ---- one step
-    def forward(self, x, ctx: StepContext, mem: LayerMemory) -> torch.Tensor:
+    def forward(self, x, ctx: StepContext, mem: LayerMemory, leave_product: bool = False):
         n = x.shape[0]
         if self.wide and not self.filtered:
             return self._forward_wide(K.linear(x, self.w_qkv), ctx, mem)
@@ -262,7 +271,8 @@ class GroupedQueryAttention:
         # rows that the products make spare two launches of their own, whatever this one takes
         if attention_backend.token_possible(self, ctx, mem, interleaved, rotary_dim) and (
                 isinstance(x, K.PendingRows) or attention_backend.token_pays(self, ctx)):
-            return self._project(attention_backend.run_token(self, qkv, cos_sin, rotary_dim, ctx, mem))
+            heads = attention_backend.run_token(self, qkv, cos_sin, rotary_dim, ctx, mem, whole=leave_product)
+            return K.PendingProduct(heads, self.w_o) if leave_product else self._project(heads)
         out = torch.empty((n, self.nq * self.d), dtype=x.dtype, device=x.device)
         parts = None
         if qkv.dim() == 3:
@@ -275,7 +285,7 @@ class GroupedQueryAttention:
             self.nq, self.nkv, self.d, parts=parts,
         )
         attention_backend.run(self, out, qkv, ctx, mem)
-        return self._project(out)
+        return K.PendingProduct(out, self.w_o) if leave_product else self._project(out)
 
     def _project(self, out):
         y = K.linear(out, self.w_o, partial_ok=True)      # the next norm adds the partial products

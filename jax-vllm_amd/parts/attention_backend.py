@@ -286,13 +286,13 @@ def _decode_work(ctx, plan, att, window: int):
     return ctx.extras[key]
 
 
-def run_token(att, qkv, cos_sin, rotary_dim: int, ctx, mem):
+def run_token(att, qkv, cos_sin, rotary_dim: int, ctx, mem, whole: bool = False):
     """Head norms, rotation, page writes and attention of a step of single tokens; ``qkv``: the q/k/v product or its parts.  Returns the
-    heads [tokens, nq * D], or ``K.SplitHeads`` where the output product merges them."""
+    heads [tokens, nq * D], or ``K.SplitHeads`` where the output product merges them (``whole``: never)."""
     window = K.key_window(att.window, att.chunk)
     n, device = ctx.num_tokens, att.w_o.device
     plan = _mfma_plan(att, ctx, window, 0, device)
-    merge = plan.num_splits == 1 or not K.split_heads_pay(n, att.w_o, plan.num_splits)
+    merge = whole or plan.num_splits == 1 or not K.split_heads_pay(n, att.w_o, plan.num_splits)
     out = torch.empty((n, att.nq * att.d), dtype=att.dtype, device=device) if merge else None
     K.attn_decode_token(out, qkv, ctx.slot_mappings[mem.group], att.q_norm, att.k_norm, att.qk_norm_eps or 0.0, cos_sin, rotary_dim,
                         mem.pages["k"], mem.pages["v"], ctx.block_tables[mem.group], ctx.context_lens, att.nq, att.nkv, att.d,

@@ -45,8 +45,18 @@ class GatedMLP:
         """Whether the gate/up product may make its rows itself (``K.PendingRows``)."""
         return K.linear_takes_pending_rows(n_rows, self.w_gate_up, gate_pairs=True)
 
-    def forward(self, x, ctx=None) -> torch.Tensor:
+    def takes_stream_rows(self, n_rows: int) -> bool:
+        """Whether the gate/up product reads ``K.StreamRows``."""
+        return K.linear_takes_stream_rows(n_rows, self.w_gate_up, gate_pairs=True)
+
+    def leaves_product(self, n_rows: int) -> bool:
+        """Whether ``forward`` takes ``leave_product`` for so many rows: the last product is then left to the block."""
+        return self.partial_out and K.stream_product_possible(n_rows, self.w_down)
+
+    def forward(self, x, ctx=None, leave_product: bool = False):
         z = K.linear(x, self.w_gate_up, gate_pairs=self.activation)    # gate and up rows alternate in the fused weight
+        if leave_product:
+            return K.PendingProduct(z, self.w_down)
         return K.linear(z, self.w_down, partial_ok=self.partial_out)   # the next norm adds the partial products
 
 

@@ -12,6 +12,7 @@ from typing import Optional
 
 import torch
 
+from ..ops import kernels as K
 from .spec import (BLOCK_STATE, PagedCacheSpec, LayerMemory, LayerSpec, ModelSpec, StateSpec, StepContext, TensorSpec,
                    build_part, is_replayable, state_specs_of)
 
@@ -138,8 +139,12 @@ class DecoderModel:
         delta = None
         for run, mem in zip(self.spec.schedule, memories):
             layer = self.layers[run.layer]
+            if isinstance(delta, K.PendingProduct) and not getattr(layer.block, "takes_products", False):
+                delta = delta.linear()
             delta = layer.block.forward(h, delta, layer.mixer, layer.feed_forward, ctx, mem)
         if logit_rows.numel() == 0:
             return torch.empty((0, self.spec.vocab_size), dtype=torch.float32, device=h.device)
+        if isinstance(delta, K.PendingProduct) and not hasattr(self.final_norm, "into_stream"):
+            delta = delta.linear()
         x = self.final_norm.add_norm(h, delta, rows=logit_rows)
         return self.head.forward(x)

@@ -42,10 +42,14 @@ class RMSNorm:
         """``norm(h + delta)`` as rows that the product which reads them makes itself, the stream then in ``out``."""
         return K.PendingRows(h, delta, self.weight, self.eps, out)
 
+    def into_stream(self, h: torch.Tensor, product):
+        """``h`` += what a ``K.PendingProduct`` makes, in that product's launch; returns ``K.StreamRows``."""
+        return K.gemm_into_stream(h, product.x, product.w, self.weight, self.eps)
+
     def add_norm(self, h: torch.Tensor, delta, rows=None, unscaled_ok: bool = False):
         """The residual step fused with the norm: ``h += delta`` in the float residual stream,
         returns ``norm(h)`` in the activation type.  ``delta`` may be a ``K.PendingNorm``: then what is
-        added is its own norm of the sublayer's output.  With ``rows`` only those rows are normed
+        added is its own norm of the sublayer's output; or a ``K.PendingProduct``, which joins ``h`` in its own launch.  With ``rows`` only those rows are normed
         and ``h`` is left alone.  With ``unscaled_ok`` the reader multiplies the rows by a matrix
         through ``K.linear`` and nothing else: for the few rows of a decode step whose ``delta``
         comes as partial products the result may then be ``K.UnscaledRows`` (``h * weight`` with
@@ -58,6 +62,9 @@ class RMSNorm:
             K.postnorm_add_rmsnorm(h, delta.y, delta.parts, delta.weight, delta.eps, self.weight, out, rows, out_eps=self.eps,
                                    bias=delta.bias, plain_scale=delta.scale)
             return out
+        if isinstance(delta, K.PendingProduct):
+            K.gemm_into_stream(h, delta.x, delta.w)
+            delta = None
         if (unscaled_ok and rows is None and delta is not None and delta.dim() == 3
                 and K.unscaled_rows_possible(self.dtype, h.shape[0], self.size)):
             return K.add_parts_unscaled(h, delta, self.weight, self.eps)
