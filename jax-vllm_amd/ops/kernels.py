@@ -1317,6 +1317,13 @@ def _linear_stream_rows(rows: "StreamRows", w: torch.Tensor, gate_pairs, partial
     return gemm_skinny(rows.x, w, torch.bfloat16 if gate_pairs else torch.float32, gate_pairs=gate_pairs, block_shape=shape, row_scale=rows)
 
 
+def thin_whole_pays(m: int, n: int, k: int) -> bool:
+    """Whether a narrow product whose reader adds partial products had better leave one of them, by ``csrc/gemm_thin.hip`` with the inner size whole, than
+    2 or 4 by blocks that stay.  Microseconds, whole / parts, at 1 and 8 rows: 2,048 x 3,072 5.0 / 5.6, 5.7 / 6.0, 4,096 x 3,072 6.8 / 9.0, 6.8 / 9.6, 3,072 x 2,048
+    4.5 / 5.6, 4.8 / 6.1, 4,096 x 4,096 7.6 / 8.6, 8.0 / 8.9; but 2,048 x 2,048 4.2 / 4.0, 4.6 / 4.2, 1,024 x 4,096 5.3 / 4.1; at 16 rows 2,048 x 4,096 7.5 / 6.7."""
+    return m <= 8 and 2048 <= n <= 4096 and 2048 <= k <= 4096 and (n > 2048 or 2048 < k < 4096)
+
+
 def gemm_few(x: torch.Tensor, w: torch.Tensor, tile: int, gate_pairs: "str | tuple | None" = None, out_dtype=torch.bfloat16) -> torch.Tensor:
     """x @ w.T for up to 16 rows of bfloat16 x against bfloat16 w [N, K], K a multiple of 64 up to 4,096, ``tile`` (16 or 32) rows of w a
     block: see ``csrc/gemm_few.hip``.  bfloat16 or float32 [M, N], or with ``gate_pairs`` the activation, bfloat16 [M, N / 2]."""
@@ -1458,6 +1465,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
                 return gemm_few(x, w, tile, gate_pairs, out_dtype or torch.bfloat16)
         _need(scale is None or (plan is not None and plan[0][0] == -2),
               "un-normalised rows need a product by the blocks that stay (ask linear_takes_unscaled_rows first)")
+        if (plan is not None and plan[1] > 1 and scale is None and thin_whole_pays(m, n, k) and x.is_contiguous() and w.is_contiguous()
+                and not (x.data_ptr() | w.data_ptr()) & 15):
+            return gemm_few(x, w, 16, out_dtype=torch.float32).view(1, m, n)
         if plan is not None:
             shape, parts = plan
             if shape == TILE64:
