@@ -586,8 +586,9 @@ constexpr int PCS = BN * CPK / 256;        // 16-byte pieces of a K tile (and of
 constexpr bool KB_ADDS = (32 * CPK / 16) % 16 == 0;   // the second key block's chunks are the first's plus a constant
 __device__ __forceinline__ int swizzle(int q) { return q ^ ((q >> 4) & 15); }   // chunk index -> chunk position
 
+#define PREFILL32_OCCUPANCY __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1, D <= 128 ? 2 : 1)))
 template <int PAGES, bool MORE>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1, D <= 128 ? 2 : 1))) attn_prefill32_kernel(AttnArgs p) {
+__device__ __forceinline__ void attn_prefill32_block(const AttnArgs& p, int block) {
   __shared__ __attribute__((aligned(16))) bf16_t Ks[2][BN * D];
   __shared__ __attribute__((aligned(16))) bf16_t Vs[2][D * BN];
   // FAST: pages of 16 keys and a head size that is a power of two.  Every load instruction of a wave
@@ -599,7 +600,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 1
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // a scalar: branches on it are uniform
   const int l32 = lane & 31, h = lane >> 5;
-  const int g = blockIdx.x % p.nkv, item = blockIdx.x / p.nkv;
+  const int g = block % p.nkv, item = block / p.nkv;
   const int r = p.work[3 * item];
   const int G = p.nq / p.nkv, P = FAST ? 16 : p.page_size;
   const PageSplit ps{P, PAGES == 0 ? -1 : (FAST ? 4 : p.page_shift)};
@@ -1174,6 +1175,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 1
       }
   }
 }
+template <int PAGES, bool MORE>
+__global__ void __launch_bounds__(256) PREFILL32_OCCUPANCY attn_prefill32_kernel(AttnArgs p) {
+  attn_prefill32_block<PAGES, MORE>(p, blockIdx.x);
+}
 #endif
 
 // the host's plan: rows per group, and groups a work item may name
@@ -1215,7 +1220,7 @@ constexpr int QN_STRIDE = D + 8;           // bf16 elements of a prepared head i
 constexpr int DEC_NEW_BYTES = 16 * QN_STRIDE * 2 + D * 2 + D * 4 + 16 * 4;      // prepared q heads, the new key, value and scores
 
 template <bool MORE, int INPUT>
-__global__ void __launch_bounds__(64 * DEC_WAVES) PREFILL_OCCUPANCY attn_decode_kernel(AttnArgs p) {
+__device__ __forceinline__ void attn_decode_block(const AttnArgs& p, int block, int split) {
   extern __shared__ __attribute__((aligned(16))) float smem[];  // per wave: m[16], l[16], acc[rows][DEC_STRIDE]
   constexpr int WAVES = DEC_WAVES, THREADS = 64 * WAVES;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1227,7 +1232,7 @@ __global__ void __launch_bounds__(64 * DEC_WAVES) PREFILL_OCCUPANCY attn_decode_
   // uneven these are (requests fastest put all of a request's heads on one die).  With V in
   // pieces of 16 bytes instead of 8, microseconds (before): 64 requests of 512 to 1,536 keys 57.6 (58.5), one of 1,030 keys in 8 splits
   // with its merge 9.9 (10.4), 16 of 400 to 1,200 over 4 kv heads in 4 splits 12.6 (13.3), head size 256, 8 over one 15.5 (16.6).
-  const int heads = p.nkv * mt_per_head, w = blockIdx.x / heads, at = blockIdx.x - w * heads;
+  const int heads = p.nkv * mt_per_head, w = block / heads, at = block - w * heads;
   // Without cu_seqlens request r's token is row r, without a work list the requests are 0, 1, ... (a step of
   // decoded tokens only): nothing has to be looked up before the loads below can start.  The
   // kernel's time at small batches is its chain of dependent memory round trips (~1.5 us each
@@ -1236,7 +1241,6 @@ __global__ void __launch_bounds__(64 * DEC_WAVES) PREFILL_OCCUPANCY attn_decode_
   // after it.
   const int r = p.work ? p.work[w] : w;
   const int g = at / mt_per_head, mt = at - g * mt_per_head;
-  const int split = blockIdx.y;
   const int rows = G - mt * 16 < 16 ? G - mt * 16 : 16;
   const int* gtable = p.block_tables + (long long)r * p.table_stride;
   // A table row beyond DEC_TBL_MAX entries does not fit: the block then copies only the entries of its own
@@ -1606,6 +1610,24 @@ __global__ void __launch_bounds__(64 * DEC_WAVES) PREFILL_OCCUPANCY attn_decode_
   }
 }
 
+template <bool MORE, int INPUT>
+__global__ void __launch_bounds__(64 * DEC_WAVES) PREFILL_OCCUPANCY attn_decode_kernel(AttnArgs p) {
+  attn_decode_block<MORE, INPUT>(p, blockIdx.x, blockIdx.y);
+}
+
+#if defined(JV_PREFILL32) && (JV_HEAD_DIM == 64 || JV_HEAD_DIM == 128)
+#define JV_ATTN_MIXED 1
+// A step's decoded tokens and its prompts in one launch: the decode blocks wait for memory while the prompts' blocks multiply, and both kernels
+// take half a unit's registers, so a unit has one of each where two launches kept it with either.  Decode blocks first: they begin with a chain
+// of look-ups, and the heaviest prompt items follow.  24 requests of 450 to 1,350 keys beside 3 prompts of 1,501 tokens (8 kv heads of 4 q heads of 128)
+// 51.5 us in two launches, 38.2 in one, 42.1 with the prompts' blocks first.
+__global__ void __launch_bounds__(256) PREFILL32_OCCUPANCY attn_mixed_kernel(AttnArgs prompts, AttnArgs decodes, int decode_blocks) {
+  const int all = decode_blocks * decodes.num_splits, block = blockIdx.x;
+  if (block < all) attn_decode_block<false, DEC_READY>(decodes, block % decode_blocks, block / decode_blocks);
+  else attn_prefill32_block<16, false>(prompts, block - all);
+}
+#endif
+
 // merges the splits of one (request, head): grid (n_work, nq), D threads (rounded up to 64)
 __global__ void attn_decode_merge_kernel(AttnArgs p) {
   // All loads of a batch of 8 splits are issued before anything is computed from them: this
@@ -1782,6 +1804,60 @@ extern "C" int jv_attn_decode(void* out, const void* q, long long q_row_stride, 
   a.window = window;
   a.num_splits = num_splits;
   return launch_decode(a, n_work, scale, scratch, DEC_READY, true, (hipStream_t)stream);
+}
+
+// Prompts and decoded tokens of a step in one launch (jv_attn_prefill and jv_attn_decode without cap and keep; pages of 16 keys); jv_attn_mixed_fits: whether
+// it is built, and a block's LDS leaves room for two on a compute unit.
+static size_t mixed_shmem(int table_stride, int G) {
+  return (size_t)DEC_WAVES * (32 + (G < 16 ? G : 16) * DEC_STRIDE) * sizeof(float) + (size_t)((table_stride + 3) / 4 * 4) * sizeof(int);
+}
+extern "C" int jv_attn_mixed_fits(int page_size, int table_stride, int nq, int nkv) {
+#ifdef JV_ATTN_MIXED
+  return page_size == 16 && nkv > 0 && nq % nkv == 0 && table_stride <= DEC_TBL_MAX && 2 * BN * D * 4 + mixed_shmem(table_stride, nq / nkv) <= 80 * 1024;
+#else
+  return 0;
+#endif
+}
+extern "C" int jv_attn_mixed(void* out, const void* q, long long q_row_stride, const void* k_pages, const void* v_pages, const int* block_tables,
+                             int table_stride, const int* cu_seqlens, const int* context_lens, const int* prefill_work, int n_prefill,
+                             const int* decode_work, int n_decode, int page_size, int nq, int nkv, float scale, int window, int num_splits,
+                             float* scratch, const float* sinks, void* stream) {
+#ifdef JV_ATTN_MIXED
+  if (n_prefill <= 0 || n_decode <= 0 || num_splits < 1 || (num_splits > 1 && !scratch) || !jv_attn_mixed_fits(page_size, table_stride, nq, nkv))
+    return (int)hipErrorInvalidValue;
+  AttnArgs a{};
+  a.sinks = sinks;
+  a.out = (bf16_t*)out; a.q = (const bf16_t*)q; a.q_row_stride = q_row_stride;
+  a.k_pages = (const bf16_t*)k_pages; a.v_pages = (const bf16_t*)v_pages;
+  a.block_tables = block_tables; a.table_stride = table_stride;
+  a.cu_seqlens = cu_seqlens; a.context_lens = context_lens;
+  a.page_size = page_size; a.nq = nq; a.nkv = nkv;
+  a.scale_log2 = scale * 1.4426950408889634f; a.window = window; a.num_splits = 1;
+  if (int e = check_common(a)) return e;
+  AttnArgs d = a;
+  a.work = prefill_work;
+  d.work = decode_work;
+  d.num_splits = num_splits;
+  if (num_splits > 1) {
+    d.part_acc = scratch;
+    d.part_ml = scratch + (long long)n_decode * nq * num_splits * D;
+  }
+  const long long blocks = (long long)n_decode * nkv * ((nq / nkv + 15) / 16), grid = blocks * num_splits + (long long)n_prefill * nkv;
+  if ((long long)nkv * page_size * D >= (1ll << 31) || grid >= (1ll << 31)) return (int)hipErrorInvalidValue;
+  const size_t shmem = mixed_shmem(table_stride, nq / nkv);
+  static bool raised = false;
+  if (!raised) {
+    const hipError_t e = hipFuncSetAttribute((const void*)attn_mixed_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 2 * BN * D * 4);
+    if (e != hipSuccess) return (int)e;
+    raised = true;
+  }
+  hipLaunchKernelGGL(attn_mixed_kernel, dim3((unsigned)grid), dim3(256), shmem, (hipStream_t)stream, a, d, (int)blocks);
+  if (num_splits > 1)
+    hipLaunchKernelGGL(attn_decode_merge_kernel, dim3(n_decode, nq), dim3((D + 63) / 64 * 64), 0, (hipStream_t)stream, d);
+  return JV_LAUNCH_CHECK();
+#else
+  return (int)hipErrorInvalidValue;
+#endif
 }
 
 #ifdef JV_DECODE_FUSED

@@ -1745,6 +1745,30 @@ def attn_decode_mfma(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_se
     )
 
 
+@functools.lru_cache(maxsize=4096)
+def attn_mixed_possible(head_dim: int, page_size: int, table_width: int, nq: int, nkv: int) -> bool:
+    """Whether ``attn_mixed`` takes these sizes."""
+    return head_dim in (64, 128) and bool(_attention_library(head_dim).jv_attn_mixed_fits(c_int(page_size), c_int(table_width), c_int(nq), c_int(nkv)))
+
+
+def attn_mixed(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_seqlens, context_lens, prefill_work, n_prefill, decode_work, n_decode,
+               nq, nkv, head_dim, scale, window=0, num_splits=1, scratch=None, sinks=None) -> None:
+    """``attn_prefill_mfma`` and ``attn_decode_mfma`` of a step that has both prompts and decoded tokens, in one launch (ask
+    ``attn_mixed_possible`` first): the same results, to the bit."""
+    _sinks_ok(sinks, nq)
+    page_size = _attn_common(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_seqlens, context_lens, prefill_work, nq, nkv, head_dim)
+    _need(decode_work is not None and decode_work.is_cuda and decode_work.is_contiguous(), "decoded tokens beside prompts need their list")
+    _i32(decode_work, "decode_work")
+    _need(n_prefill > 0 and n_decode > 0 and prefill_work.numel() >= 3 * n_prefill and decode_work.numel() >= n_decode, "work lists shorter than their counts")
+    _need(attn_mixed_possible(head_dim, page_size, block_tables.shape[1], nq, nkv), "these sizes take two launches")
+    _need(num_splits == 1 or (scratch is not None and scratch.is_cuda and scratch.dtype == torch.float32
+                              and scratch.numel() >= attn_decode_scratch_floats(n_decode, nq, num_splits, head_dim)), "scratch too small for the splits")
+    _check(_attention_library(head_dim).jv_attn_mixed(
+        _ptr(out), _ptr(q), c_longlong(q_row_stride), _ptr(k_pages), _ptr(v_pages), _ptr(block_tables), c_int(block_tables.shape[1]), _ptr(cu_seqlens),
+        _ptr(context_lens), _ptr(prefill_work), c_int(n_prefill), _ptr(decode_work), c_int(n_decode), c_int(page_size), c_int(nq), c_int(nkv),
+        c_float(scale), c_int(window or 0), c_int(num_splits), _ptr(scratch if num_splits > 1 else None), _ptr(sinks), _stream()), "attn_mixed")
+
+
 DECODE_ORDER_MAX = 1024
 
 

@@ -324,6 +324,12 @@ def run(att, out, qkv, ctx, mem) -> None:
         return
     plan = _mfma_plan(att, ctx, window, keep, qkv.device)
     tables = ctx.block_tables[mem.group]
+    if (plan.n_prefill and plan.n_decode and not cap and not keep and not plan.one_group
+            and K.attn_mixed_possible(att.d, ctx.page_size, tables.shape[1], att.nq, att.nkv)):
+        K.attn_mixed(out, qkv, q_row_stride, mem.pages["k"], mem.pages["v"], tables, ctx.cu_seqlens, ctx.context_lens, plan.prefill_work,
+                     plan.n_prefill, _decode_work(ctx, plan, att, window), plan.n_decode, att.nq, att.nkv, att.d, att.scale, window,
+                     plan.num_splits, plan.scratch, sinks=sinks)
+        return
     if plan.n_prefill:
         K.attn_prefill_mfma(out, qkv, q_row_stride, mem.pages["k"], mem.pages["v"], tables, ctx.cu_seqlens,
                             ctx.context_lens, plan.prefill_work, plan.n_prefill, att.nq, att.nkv, att.d, att.scale,
