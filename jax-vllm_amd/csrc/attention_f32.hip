@@ -20,6 +20,7 @@
 // by the matrix unit (a 16 x 16 x 4 product keeps it for 32 cycles) and the exponentials, few tokens by what a compute unit
 // pulls from memory.
 #include "common.h"
+#include "f32_terms.h"
 
 typedef float af_f4 __attribute__((ext_vector_type(4)));
 typedef float af_f4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -43,6 +44,8 @@ struct AttnF32Args {
   int keep;
   float* parts;               // [n_work * nkv][part_ranges][AF_WAVES][16][D + 4]: sums, then (maximum, sum of weights)
   int part_ranges;
+  unsigned* terms;            // null, or out's rows as terms too (f32_terms.h); one block an item only
+  int fragments;
 };
 
 __device__ __forceinline__ int af_first_key(int pos, int window) {
@@ -274,8 +277,7 @@ __global__ void __launch_bounds__(64 * AF_WAVES) __attribute__((amdgpu_waves_per
     ml[(wave * AF_ROWS + li) * 2 + 1] = l_all;
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < walk.rows * (D / 4); i += 64 * AF_WAVES) {
-    const int rr = i / (D / 4), d = (i - rr * (D / 4)) * 4;
+  auto result = [&](int rr, int d, int h) {
     float top[AF_WAVES], den[AF_WAVES];
     af_f4 sum[AF_WAVES];
 #pragma unroll
@@ -283,8 +285,24 @@ __global__ void __launch_bounds__(64 * AF_WAVES) __attribute__((amdgpu_waves_per
       top[w] = ml[(w * AF_ROWS + rr) * 2], den[w] = ml[(w * AF_ROWS + rr) * 2 + 1];
       sum[w] = *(const af_f4*)(af_lds + (w * AF_ROWS + rr) * LROW + d);
     }
+    return af_meet(top, den, sum, p.sinks ? p.sinks + h : nullptr);
+  };
+  if (p.terms) {      // 8 elements a thread
+    for (int i = threadIdx.x; i < walk.rows * (D / 8); i += 64 * AF_WAVES) {
+      const int rr = i / (D / 8), d = (i - rr * (D / 8)) * 8;
+      const int qi = (m0 + rr) / G, h = kvh * G + (m0 + rr) - qi * G;
+      const long long token = q_start + qi;
+      const af_f4 v[2] = {result(rr, d, h), result(rr, d + 4, h)};
+      af_f4* out = (af_f4*)(p.out + token * p.nq * D + (long long)h * D + d);
+      out[0] = v[0], out[1] = v[1];
+      f32_terms::leave_terms(p.terms, p.fragments != 0, p.nq * D / G32_STEP, token, (h * D + d) / 8, v);
+    }
+    return;
+  }
+  for (int i = threadIdx.x; i < walk.rows * (D / 4); i += 64 * AF_WAVES) {
+    const int rr = i / (D / 4), d = (i - rr * (D / 4)) * 4;
     const int qi = (m0 + rr) / G, h = kvh * G + (m0 + rr) - qi * G;
-    const af_f4 v = af_meet(top, den, sum, p.sinks ? p.sinks + h : nullptr);
+    const af_f4 v = result(rr, d, h);
     float* out = p.out + (long long)(q_start + qi) * p.nq * D + (long long)h * D + d;
 #pragma unroll
     for (int e = 0; e < 4; ++e) out[e] = v[e];
@@ -367,13 +385,14 @@ extern "C" long long jv_attn_f32_part_floats(int n_work, int nkv, int ranges, in
 extern "C" int jv_attn_f32(float* out, const float* q, long long q_row_stride, const float* k_pages, const float* v_pages,
                            const int* block_tables, int table_stride, const int* cu_seqlens, const int* context_lens,
                            const int* work, int n_work, int splits, float* parts, int part_ranges, int page_size, int nq, int nkv, int D,
-                           float scale, int window, const float* sinks, float cap, int keep, void* stream) {
+                           float scale, int window, const float* sinks, float cap, int keep, void* terms, int fragments, void* stream) {
   if (n_work <= 0) return 0;
+  if (terms && (splits > 1 || (nq * D) % G32_STEP || (((uintptr_t)terms | (uintptr_t)out) & 15))) return (int)hipErrorInvalidValue;
   if (nkv <= 0 || nq % nkv != 0 || page_size <= 0 || page_size % 4 != 0 || keep < 0 || (long long)n_work * nkv > 0x7fffffffll ||
       splits < 1 || splits > 65535 || (splits > 1 && (!parts || part_ranges < 1)))
     return (int)hipErrorInvalidValue;
   const AttnF32Args a = {out, q, q_row_stride, k_pages, v_pages, block_tables, table_stride, cu_seqlens, context_lens, work,
-                         page_size, nq, nkv, scale, window, sinks, cap, keep, parts, part_ranges};
+                         page_size, nq, nkv, scale, window, sinks, cap, keep, parts, part_ranges, (unsigned*)terms, fragments};
   const hipStream_t st = (hipStream_t)stream;
   switch (D) {
     case 32: return attn_f32_launch<2>(a, n_work, splits, st);

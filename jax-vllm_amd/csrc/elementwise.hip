@@ -2,6 +2,7 @@
 // The residual stream is float in every mode; normalised outputs are in the
 // activation type T.  All reductions are float.
 #include "common.h"
+#include "f32_terms.h"
 
 // ---------------------------------------------------------------- embedding gather
 // h[t, :] = float(table[ids[t], :]).  One block per token.  An id outside [0, rows) reads nothing:
@@ -119,6 +120,9 @@ __device__ __forceinline__ void load8<float>(const float* p, float (&v)[8]) {
 // piece beyond the row reads the row's last piece again and only its stores and its share of the sum are
 // left out (a load inside a branch makes the compiler wait for all loads in flight where the branch
 // ends: 1.1 us of a 4.4 us kernel).  A short row's time is the sum of its dependent memory round trips.
+__device__ __forceinline__ float add_squares(float ss, float4 v) {      // spelled out: kernels that stand for one another round alike
+  return ss + fmaf(v.w, v.w, fmaf(v.z, v.z, fmaf(v.y, v.y, v.x * v.x)));
+}
 template <typename T, int V>
 __global__ void __launch_bounds__(256)
 add_rmsnorm_vec_kernel(float* __restrict__ h, const T* __restrict__ delta,
@@ -147,7 +151,7 @@ add_rmsnorm_vec_kernel(float* __restrict__ h, const T* __restrict__ delta,
     if (delta) { v.x += d[k].x; v.y += d[k].y; v.z += d[k].z; v.w += d[k].w; }
     if (c < nvec) {
       if (delta && !rows) *(float4*)(hr + 4 * c) = v;
-      ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+      ss = add_squares(ss, v);
     }
     x[k] = v;
   }
@@ -159,6 +163,59 @@ add_rmsnorm_vec_kernel(float* __restrict__ h, const T* __restrict__ delta,
     const float4 v = x[k];
     if (c < nvec)
       store4<T>(o + 4 * c, float4{v.x * inv * ww[k].x, v.y * inv * ww[k].y, v.z * inv * ww[k].z, v.w * inv * ww[k].w});
+  }
+}
+
+// The same for float rows of every column of V pieces a thread (V even) that a product takes as its terms too (f32_terms.h): neighbouring threads swap
+// pieces, so that each has 8 columns of half of theirs.  Blocks b, b + 8, ... run on one XCD and take 32 rows next to one another: a line of the terms in
+// the order of the operands holds 8 rows, which would else be put together from several L2s.  1,003 rows of 2,048 12.3 us where the norm alone takes 7.8 and
+// a launch for the terms 7.0; 8 rows a block, the terms through LDS in whole lines, 13.5.
+template <int V>
+__global__ void __launch_bounds__(256)
+add_rmsnorm_terms_kernel(float* __restrict__ h, const float* __restrict__ delta, const float* __restrict__ w, float* __restrict__ out,
+                         unsigned* __restrict__ terms, int fragments, int n_rows, int hidden, float eps) {
+  typedef f32_terms::f32x4 f4;
+  __shared__ float red[32];
+  const long long r = (blockIdx.x & ~255) + (blockIdx.x & 7) * 32 + ((blockIdx.x & 255) >> 3);
+  if (r >= n_rows) return;
+  float* hr = h + r * hidden;
+  const float* dr = delta ? delta + r * hidden : w;
+  float4 x[V], ww[V], d[V];
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    const int c = threadIdx.x + k * blockDim.x;
+    ww[k] = *(const float4*)(w + 4 * c);
+    x[k] = *(const float4*)(hr + 4 * c);
+    d[k] = *(const float4*)(dr + (delta ? 4 * c : 0));
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    float4 v = x[k];
+    if (delta) {
+      v.x += d[k].x; v.y += d[k].y; v.z += d[k].z; v.w += d[k].w;
+      *(float4*)(hr + 4 * (threadIdx.x + k * blockDim.x)) = v;
+    }
+    ss = add_squares(ss, v);
+    x[k] = v;
+  }
+  ss = block_sum(ss, red);
+  const float inv = rsqrtf(ss / (float)hidden + eps);
+  f4 o[V];
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    o[k] = f4{x[k].x * inv * ww[k].x, x[k].y * inv * ww[k].y, x[k].z * inv * ww[k].z, x[k].w * inv * ww[k].w};
+    *(f4*)(out + r * hidden + 4 * (threadIdx.x + k * blockDim.x)) = o[k];
+  }
+  const bool odd = threadIdx.x & 1;
+#pragma unroll
+  for (int k = 0; k < V; k += 2) {      // the even thread takes piece k of both, the odd one piece k + 1
+    const f4 mine = odd ? o[k + 1] : o[k], give = odd ? o[k] : o[k + 1];
+    f4 got;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) got[e] = __shfl_xor(give[e], 1, 64);
+    const f4 v[2] = {odd ? got : mine, odd ? mine : got};
+    f32_terms::leave_terms(terms, fragments != 0, hidden / G32_STEP, r, (int)(threadIdx.x + (k + odd) * blockDim.x) >> 1, v);
   }
 }
 
@@ -284,6 +341,26 @@ static void launch_arn_parts(int v, int n_out, int threads, hipStream_t st, floa
     default: ARN_GO(8); break;
   }
 #undef ARN_GO
+}
+
+// Whether jv_add_rmsnorm_terms_f32 takes rows of this width.
+extern "C" int jv_add_rmsnorm_terms_fits(int hidden) {
+  if (hidden <= 0 || hidden % 32 || hidden > 4 * ARN_MAX_V * 256) return 0;
+  int threads, v;
+  arn_shape(hidden / 4, &threads, &v);
+  return hidden / 4 == threads * v && v % 2 == 0;
+}
+// jv_add_rmsnorm_f32 of every row of h, and out as terms in the layout of jv_split_fragments_f32 (fragments) or jv_split_rows_f32.
+extern "C" int jv_add_rmsnorm_terms_f32(float* h, const float* delta, const float* w, float* out, void* terms, int fragments, int n_rows, int hidden,
+                                        float eps, void* stream) {
+  if (n_rows <= 0) return 0;
+  if (!jv_add_rmsnorm_terms_fits(hidden) || !terms || ((uintptr_t)terms & 15)) return (int)hipErrorInvalidValue;
+  int threads, v;
+  arn_shape(hidden / 4, &threads, &v);
+  const auto kernel = v == 2 ? add_rmsnorm_terms_kernel<2> : v == 4 ? add_rmsnorm_terms_kernel<4> : add_rmsnorm_terms_kernel<8>;
+  hipLaunchKernelGGL(kernel, dim3((n_rows + 255) / 256 * 256), dim3(threads), 0, (hipStream_t)stream, h, delta, w, out, (unsigned*)terms, fragments,
+                     n_rows, hidden, eps);
+  return JV_LAUNCH_CHECK();
 }
 
 // ---------------------------------------------------------------- plain RMSNorm over the last axis

@@ -19,37 +19,14 @@
 // 13.9 (50 MB: the stream of W); 300 x 6,144 x 2,048 75 / 65; 1,003 x 6,144 x 2,048 153 / 144 with what the terms of A take; 2,048 x 24,576 x 4,096
 // 2,250 / 1,954 = 211 TFLOP/s of 32-bit products, 1.27 PFLOP/s of the matrix unit's.  The scaling takes 1 to 5 % of it (24 sizes).
 #include "common.h"
+#include "f32_terms.h"
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+using namespace f32_terms;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));      // 16 bytes from any address of a float
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-#define G32_STEP 32            // columns of a step and of v_mfma_f32_16x16x32_bf16
-
-#define G32_SCALE 0x1p24f
-#define G32_UNSCALE 0x1p-48f
-
-// Pair i of a lane's 8 numbers: its part of the three terms of 2^24 times these.
-__device__ __forceinline__ void split_pair(float a, float b, int i, u32x4 (&t)[3]) {
-  a *= G32_SCALE, b *= G32_SCALE;
-#pragma unroll
-  for (int e = 0; e < 3; ++e) {
-    t[e][i] = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){a, b}, bf16x2));
-    if (e < 2) {
-      a -= __uint_as_float(t[e][i] << 16);
-      b -= __uint_as_float(t[e][i] & 0xffff0000u);
-    }
-  }
-}
-__device__ __forceinline__ void split8(const f32x4 (&v)[2], u32x4 (&t)[3]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) split_pair(v[i / 2][i % 2 * 2], v[i / 2][i % 2 * 2 + 1], i, t);
-}
 // The products of a step, (term of w, term of x), from the smallest on.
 #define G32_PRODUCTS 6
 __device__ constexpr int G32_W[G32_PRODUCTS] = {0, 1, 2, 0, 1, 0}, G32_X[G32_PRODUCTS] = {2, 1, 0, 1, 0, 0};
@@ -88,21 +65,27 @@ __device__ __forceinline__ void leave(float* C, int m, int n, int N, const float
       if (n + e < N) C[(long long)m * N + n + e] = v[e];
   }
 }
-// The same from sums of scaled products.  `pieces`: N a multiple of 4, C begins on 16 bytes.
+// The same from sums of scaled products.  `pieces`: N a multiple of 4, C begins on 16 bytes.  `keep` takes the activation's two results too.
 template <bool ACT>
-__device__ __forceinline__ void leave_sums(float* C, int m, int n, int M, int N, const f32x4& v, bool pieces, JvAct act, const float* A, const float* W, int K, int KA) {
+__device__ __forceinline__ void leave_sums(float* C, int m, int n, int M, int N, const f32x4& v, bool pieces, JvAct act, const float* A, const float* W, int K, int KA,
+                                           float* keep = nullptr) {
   bool ok = pieces && n + 4 <= N;
 #pragma unroll
   for (int e = 0; e < 4; ++e) ok = ok && __builtin_fabsf(v[e]) <= 3.402823466e38f;
   if (ok) {
     const f32x4 r = v * G32_UNSCALE;
-    if constexpr (ACT) *(f32x2*)(C + (long long)m * (N / 2) + n / 2) = f32x2{jv_gated(act, r[0], r[1]), jv_gated(act, r[2], r[3])};
-    else *(f32x4*)(C + (long long)m * N + n) = r;
+    if constexpr (ACT) {
+      const f32x2 z = {jv_gated(act, r[0], r[1]), jv_gated(act, r[2], r[3])};
+      *(f32x2*)(C + (long long)m * (N / 2) + n / 2) = z;
+      if (keep) *(f32x2*)keep = z;
+    } else
+      *(f32x4*)(C + (long long)m * N + n) = r;
   } else {
     float r[4];
     for (int e = 0; e < 4; ++e)
       if (n + e < N) r[e] = settle(v[e], A + (long long)m * KA, W + (long long)(n + e) * K, KA);
     leave<ACT>(C, m, n, N, r, act);
+    if (ACT && keep) keep[0] = jv_gated(act, r[0], r[1]), keep[1] = jv_gated(act, r[2], r[3]);
   }
 }
 // 16 bytes a lane from base + off straight into LDS, 1 KB in the order of the lanes from `at` on.
@@ -577,7 +560,8 @@ gemm_f32_tile_kernel(float* __restrict__ C, const unsigned* __restrict__ X, cons
 // 1.23, 64 1.08 to 1.26.  Behind only where few rows meet many short ones: 65 to 200 x 24,576 x 256 and 512 by 4 to 7 %.
 template <int TW, bool ACT>
 __global__ void __launch_bounds__(512, 2)
-gemm_f32_rows_kernel(float* __restrict__ C, const unsigned* __restrict__ X, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K, int KA, JvAct act) {
+gemm_f32_rows_kernel(float* __restrict__ C, const unsigned* __restrict__ X, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K, int KA, JvAct act,
+                     unsigned* __restrict__ terms, bool fragments) {
   constexpr int TM = 128, NT = TW / 32, TERMS = 3 * TW * 64, RING = 3;
   static_assert(2 * RING * TERMS <= 160 * 1024 && 2 * TM * (TW + 4) * 4 <= 2 * RING * TERMS, "");
   __shared__ __attribute__((aligned(1024))) char bufs[2 * RING * TERMS];
@@ -718,8 +702,24 @@ gemm_f32_rows_kernel(float* __restrict__ C, const unsigned* __restrict__ X, cons
   for (int i = threadIdx.x; i < TM * TW / 4; i += 512) {
     const int r = i / (TW / 4), c = (i - r * (TW / 4)) * 4;
     if (m0 + r >= M || n0 + c >= N) continue;
-    const float* at = meet + r * ROW + c;
-    leave_sums<ACT>(C, m0 + r, n0 + c, M, N, *(const f32x4*)at + *(const f32x4*)(at + SIDE), pieces, act, A, W, K, KA);
+    float* at = meet + r * ROW + c;
+    leave_sums<ACT>(C, m0 + r, n0 + c, M, N, *(const f32x4*)at + *(const f32x4*)(at + SIDE), pieces, act, A, W, K, KA, ACT && terms ? at : nullptr);
+  }
+  if constexpr (ACT) {
+    if (!terms) return;
+    __syncthreads();
+    // the results again, 8 a thread, as the terms of the next product's rows; lanes along the rows
+    for (int i = threadIdx.x; i < TM * TW / 16; i += 512) {
+      const int r = i % TM, c = i / TM * 16;
+      if (m0 + r >= M || n0 + c >= N) continue;      // N is a multiple of 64
+      f32x4 v[2];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x2 z = *(const f32x2*)(meet + r * ROW + c + j * 4);
+        v[j / 2][j % 2 * 2] = z[0], v[j / 2][j % 2 * 2 + 1] = z[1];
+      }
+      leave_terms(terms, fragments, N / 64, m0 + r, (n0 + c) / 16, v);
+    }
   }
 }
 
@@ -779,11 +779,11 @@ extern "C" int jv_split_fragments_f32(void* X, const float* A, int M, int KA, vo
   return JV_LAUNCH_CHECK();
 }
 template <int TW>
-static int rows_launch(float* C, const void* X, const float* A, const float* W, int M, int N, int K, int KA, JvAct act, hipStream_t s) {
+static int rows_launch(float* C, const void* X, const float* A, const float* W, int M, int N, int K, int KA, JvAct act, void* terms, bool fragments, hipStream_t s) {
   const long long live = ((long long)M + 127) / 128 * (((long long)N + TW - 1) / TW);
   if (live > 1 << 24) return (int)hipErrorInvalidValue;
   const auto kernel = act.id ? gemm_f32_rows_kernel<TW, true> : gemm_f32_rows_kernel<TW, false>;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)((live + 7) / 8 * 8)), dim3(512), 0, s, C, (const unsigned*)X, A, W, M, N, K, KA, act);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((live + 7) / 8 * 8)), dim3(512), 0, s, C, (const unsigned*)X, A, W, M, N, K, KA, act, (unsigned*)terms, fragments);
   return JV_LAUNCH_CHECK();
 }
 // Rows of A [M][KA] as terms (of 2^24 times A), [M][steps][3][32] bf16 with zeros behind KA; steps = ceil(KA / 32).
@@ -797,13 +797,15 @@ extern "C" int jv_split_rows_f32(void* X, const float* A, int M, int KA, void* s
 }
 // A [M][KA], W [N][K], C [M][N].  K = KA but for tiles, where W may have columns behind KA (finite; as many steps of 32 as KA has).
 // X, for tiles: the rows of A by jv_split_fragments_f32 (forms 5 to 7) or jv_split_rows_f32 (from 8 on).
-// gate_act (JV_ACT_*, not 0): the rows of W alternate gate and up rows and C is [M][N / 2], act(gate) * up.
+// gate_act (JV_ACT_*, not 0): the rows of W alternate gate and up rows and C is [M][N / 2], act(gate) * up; forms 5 to 7 then also leave it as terms
+// (`terms` not null, N a multiple of 64), by rows or with `fragments` as jv_split_fragments_f32 would.
 extern "C" int jv_gemm_f32(float* C, const float* A, const float* W, const void* X, int M, int N, int K, int KA, int form, int gate_act, float act_limit,
-                           float act_slope, void* stream) {
+                           float act_slope, void* terms, int fragments, void* stream) {
   if (M <= 0 || N <= 0) return 0;
   const bool pieces = !(K & 3) && !((uintptr_t)W & 15) && K > 0;
   if (K < 0 || KA > K || (KA + 31) / 32 != (K + 31) / 32) return (int)hipErrorInvalidValue;
   if (gate_act && (!jv_act_known(gate_act) || N % 2)) return (int)hipErrorInvalidValue;
+  if (terms && (!gate_act || N % 64 || form < 5 || form > 7 || (((uintptr_t)terms | (uintptr_t)C) & 15))) return (int)hipErrorInvalidValue;
   if (form >= 5 ? !pieces || !X || ((uintptr_t)X & 15) || K > 1 << 22 : KA != K || (form >= 2 && (!pieces || ((uintptr_t)A & 15) || K > 1 << 24)))
     return (int)hipErrorInvalidValue;
   const JvAct act{gate_act, act_limit, act_slope};
@@ -816,9 +818,9 @@ extern "C" int jv_gemm_f32(float* C, const float* A, const float* W, const void*
       return N <= 8 * 256 ? pairs_launch<1, 2, 8>(C, A, W, M, N, K, act, s) : pairs_launch<2, 1, 4>(C, A, W, M, N, K, act, s);
     case 3: return few_launch<32, 16, 1, 1, true>(C, A, W, M, N, K, act, s);
     case 4: return M > 8 ? few_launch<32, 32, 1, 1, true>(C, A, W, M, N, K, act, s) : pairs_launch<3, 1, 2>(C, A, W, M, N, K, act, s);
-    case 5: return rows_launch<128>(C, X, A, W, M, N, K, KA, act, s);
-    case 6: return rows_launch<96>(C, X, A, W, M, N, K, KA, act, s);
-    case 7: return rows_launch<64>(C, X, A, W, M, N, K, KA, act, s);
+    case 5: return rows_launch<128>(C, X, A, W, M, N, K, KA, act, terms, fragments != 0, s);
+    case 6: return rows_launch<96>(C, X, A, W, M, N, K, KA, act, terms, fragments != 0, s);
+    case 7: return rows_launch<64>(C, X, A, W, M, N, K, KA, act, terms, fragments != 0, s);
     case 8: return tile_launch<64, 96>(C, X, A, W, M, N, K, KA, act, s);
     case 9: return tile_launch<64, 64>(C, X, A, W, M, N, K, KA, act, s);
     case 10: return tile_launch<64, 32>(C, X, A, W, M, N, K, KA, act, s);

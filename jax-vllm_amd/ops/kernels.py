@@ -773,13 +773,14 @@ def attn_f32_part_floats(n_work: int, nkv: int, ranges: int, head_dim: int) -> i
 
 
 def attn_f32(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_seqlens, context_lens, work, n_work,
-             nq, nkv, head_dim, scale, window=0, splits=1, parts=None, sinks=None, cap: float = 0.0, keep: int = 0) -> None:
+             nq, nkv, head_dim, scale, window=0, splits=1, parts=None, sinks=None, cap: float = 0.0, keep: int = 0, terms=None) -> None:
     """Causal attention of every token over its request's pages in true 32-bit on the matrix cores.  ``work`` is int32
     [n_work, 2]: (request index, first row of ``attn_f32_rows`` (query, head-in-group) rows); every row of every request
     must be in exactly one item.  With ``splits`` > 1 that many blocks share out an item's ranges of ``attn_f32_range_keys`` keys
     and ``parts`` (float32, ``attn_f32_part_floats`` entries for at least ``splits`` ranges) holds the ranges' sums; an item
     of more ranges than ``parts`` has room for is one block's all the same.  A row's bits depend neither on that nor on the
-    other rows.  The other arguments: as for ``paged_attention_generic``."""
+    other rows.  ``terms`` (from ``f32_terms``; with ``splits`` 1): takes out's rows as terms too.  The other arguments: as for
+    ``paged_attention_generic``."""
     _dev(out, q, k_pages, v_pages, block_tables, cu_seqlens, context_lens, work, sinks)
     if sinks is not None:
         _f32(sinks, "sinks", nq)
@@ -807,7 +808,8 @@ def attn_f32(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_seqlens, c
                                    c_int(block_tables.shape[1]), _ptr(cu_seqlens), _ptr(context_lens), _ptr(work),
                                    c_int(n_work), c_int(splits), _ptr(parts if splits > 1 else None), c_int(room),
                                    c_int(page_size), c_int(nq), c_int(nkv), c_int(head_dim), c_float(scale), c_int(window or 0), _ptr(sinks),
-                                   c_float(cap), c_int(keep if window else 0), _stream()),
+                                   c_float(cap), c_int(keep if window else 0), _ptr(terms[0] if terms else None), c_int(1 if terms and terms[1] else 0),
+                                   _stream()),
         "attn_f32",
     )
 
@@ -870,10 +872,61 @@ def f32_plan(m: int, n: int, k: int, pieces: bool = True, a_pieces: bool = True)
     return min(times, key=times.get)
 
 
-def gemm_f32(a: torch.Tensor, w: torch.Tensor, out=None, gate_pairs: "str | tuple | None" = None) -> torch.Tensor:
+class TermRows:
+    """Float rows ``x`` that a 32-bit product of many rows reads next, with their terms as that product takes them (``f32_terms``): the kernel that
+    makes the rows leaves both, where the product would make the terms in a launch of its own."""
+
+    dtype = torch.float32
+
+    def __init__(self, x: torch.Tensor, terms: torch.Tensor, fragments: bool):
+        self.x, self.terms, self.fragments = x, terms, bool(fragments)
+
+    shape = property(lambda self: self.x.shape)
+    device = property(lambda self: self.x.device)
+
+
+def f32_terms_layout(m: int, w: torch.Tensor) -> "bool | None":
+    """How ``gemm_f32`` of m rows against w takes the terms of its rows: in the order of the operands (True), by rows (False), or not at all (None)."""
+    n, k = w.shape
+    if w.dtype != torch.float32 or m <= 32 or k % F32_STEP or w.data_ptr() & 15:
+        return None
+    form = f32_plan(m, n, k, True, True)
+    return form < _F32_FRAGMENTS if form >= 5 else None
+
+
+def f32_terms(m: int, k: int, fragments: bool, device) -> torch.Tensor:
+    """Room for the terms of m rows of k (a multiple of 32) columns."""
+    return torch.empty((-(-m // 32) * 32 if fragments else m, k // F32_STEP, 3, F32_STEP), dtype=torch.bfloat16, device=device)
+
+
+@functools.lru_cache(maxsize=4096)
+def add_rmsnorm_terms_possible(hidden: int) -> bool:
+    """Whether ``add_rmsnorm_terms`` takes rows of this width."""
+    return bool(library.core().jv_add_rmsnorm_terms_fits(c_int(hidden)))
+
+
+def add_rmsnorm_terms(h, delta, weight, eps: float, fragments: bool) -> "TermRows":
+    """``add_rmsnorm`` of every float row (``delta`` rows or None), the result with its terms."""
+    _dev(h, delta, weight)
+    _f32(h, "h")
+    n, hidden = h.shape
+    _f32(weight, "weight", hidden)
+    _need(add_rmsnorm_terms_possible(hidden), "rows of this width have no form with terms")
+    _need(delta is None or (delta.shape == h.shape and delta.dtype == torch.float32), "delta must match h")
+    out, terms = torch.empty_like(h), f32_terms(n, hidden, fragments, h.device)
+    _check(library.core().jv_add_rmsnorm_terms_f32(_ptr(h), _ptr(delta), _ptr(weight), _ptr(out), _ptr(terms), c_int(1 if fragments else 0), c_int(n),
+                                                   c_int(hidden), c_float(eps), _stream()), "add_rmsnorm_terms")
+    return TermRows(out, terms, fragments)
+
+
+def gemm_f32(a: "torch.Tensor | TermRows", w: torch.Tensor, out=None, gate_pairs: "str | tuple | None" = None, leave_terms: "bool | None" = None):
     """out = a @ w.T in 32-bit: every float input whole, products but for what is below 2^-26 of them, float sums.  a [M, K], w [N, K], both row-major.
     ``gate_pairs``: the rows of w alternate gate and up rows, out = act(a.w[2j]) * (a.w[2j+1]) [M, N / 2] (bit for bit what ``gated_mul``
-    makes of the product)."""
+    makes of the product).  ``leave_terms`` (``f32_terms_layout`` of the product that reads the activation's result): the result is ``TermRows`` where a
+    tile of 128 rows leaves them."""
+    given = None
+    if isinstance(a, TermRows):
+        given, a = a, a.x
     _dev(a, w)
     _f32(a, "a")
     _f32(w, "w")
@@ -891,19 +944,24 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, out=None, gate_pairs: "str | tupl
         return out
     pieces = not k & 3 and not w.data_ptr() & 15
     form, lib, terms, kw = f32_plan(m, n, k, pieces, not a.data_ptr() & 15), library.core(), None, k
-    if form >= 5:      # the rows of a, scaled, as sums of three bfloat16 numbers, [M, steps, 3, 32] or whole operands of 32 rows
+    if form >= 5 and given is not None and given.fragments == (form < _F32_FRAGMENTS) and k % F32_STEP == 0:
+        terms = given.terms
+        _need(terms.shape[0] >= m and terms.shape[1] * F32_STEP == k, "the terms belong to other rows")
+    elif form >= 5:      # the rows of a, scaled, as sums of three bfloat16 numbers, [M, steps, 3, 32] or whole operands of 32 rows
         steps, fragments = -(-k // F32_STEP), form < _F32_FRAGMENTS
         terms = torch.empty((-(-m // 32) * 32 if fragments else m, steps, 3, F32_STEP), dtype=torch.bfloat16, device=a.device)
         split = lib.jv_split_fragments_f32 if fragments else lib.jv_split_rows_f32
         _check(split(_ptr(terms), _ptr(a), c_int(m), c_int(k), _stream()), "split_rows_f32")
+    if form >= 5:
         if not pieces:
             kw = -(-k // 4) * 4
             copy = torch.empty((n, kw), dtype=torch.float32, device=w.device)
             copy[:, :k], copy[:, k:] = w, 0.0
             w = copy
+    left = f32_terms(m, width, leave_terms, a.device) if leave_terms is not None and gate_pairs and 5 <= form < _F32_FRAGMENTS and n % 64 == 0 else None
     _check(lib.jv_gemm_f32(_ptr(out), _ptr(a), _ptr(w), _ptr(terms), c_int(m), c_int(n), c_int(kw), c_int(k), c_int(form), *act,
-                           _stream()), "gemm_f32")
-    return out
+                           _ptr(left), c_int(1 if leave_terms else 0), _stream()), "gemm_f32")
+    return out if left is None else TermRows(out, left, leave_terms)
 
 
 SKINNY_MAX_ROWS = 64
@@ -1412,7 +1470,7 @@ def gemm_shares(x: torch.Tensor, w: torch.Tensor, form) -> torch.Tensor:
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = False, gate_pairs: "str | tuple | None" = None,
-           partial_max_width: int | None = PARTIAL_SUM_MAX_WIDTH):
+           partial_max_width: int | None = PARTIAL_SUM_MAX_WIDTH, leave_terms: "bool | None" = None):
     """x @ w.T for w stored [out, in].
 
     float32: the library's own kernel on whole float inputs (``gemm_f32``).
@@ -1435,7 +1493,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
     if isinstance(x, UnscaledRows):
         scale, x = x, x.x
     if x.dtype == torch.float32:
-        y = gemm_f32(x, w, gate_pairs=gate_pairs)
+        y = gemm_f32(x, w, gate_pairs=gate_pairs, leave_terms=leave_terms)
+        if isinstance(y, TermRows):
+            return y
         gate_pairs = None
     else:
         _need(x.dtype == w.dtype, "x and w must have one type")

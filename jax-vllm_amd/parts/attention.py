@@ -224,6 +224,10 @@ class GroupedQueryAttention:
         return (not self.wide and not self.filtered and self.b_qkv is None and self._qkv_parts_ok()
                 and K.linear_takes_stream_rows(n_rows, self.w_qkv, partial_ok=True, partial_max_width=None))
 
+    def takes_terms(self, n_rows: int) -> "bool | None":
+        """How the qkv product of so many float rows takes their terms (``K.f32_terms_layout``)."""
+        return None if self.wide or self.filtered else K.f32_terms_layout(n_rows, self.w_qkv)
+
     def leaves_product(self, n_rows: int) -> bool:
         """Whether ``forward`` takes ``leave_product`` for so many rows: the output product is then left to the block."""
         return not self.wide and not self.filtered and self.b_o is None and K.stream_product_possible(n_rows, self.w_o)
@@ -284,7 +288,7 @@ class GroupedQueryAttention:
             mem.pages["k"] if writes else None, mem.pages["v"] if writes else None, ctx.page_size,
             self.nq, self.nkv, self.d, parts=parts,
         )
-        attention_backend.run(self, out, qkv, ctx, mem)
+        out = attention_backend.run(self, out, qkv, ctx, mem, terms=K.f32_terms_layout(n, self.w_o) if out.dtype == torch.float32 else None)
         return K.PendingProduct(out, self.w_o) if leave_product else self._project(out)
 
     def _project(self, out):

@@ -300,7 +300,9 @@ def run_token(att, qkv, cos_sin, rotary_dim: int, ctx, mem, whole: bool = False)
     return out if merge else K.SplitHeads(plan.scratch, n, plan.num_splits, att.nq, att.d, att.sinks)
 
 
-def run(att, out, qkv, ctx, mem) -> None:
+def run(att, out, qkv, ctx, mem, terms: "bool | None" = None):
+    """Attention of the step's tokens into ``out``; returns it, or ``K.TermRows`` where ``terms`` (``K.f32_terms_layout`` of the product that reads it)
+    asks for them and one block makes a row."""
     # q heads of a row sit at the front of the fused q/k/v projection, unless the mixer says where else
     q_row_stride = getattr(att, "q_row_stride", None) or (att.nq + 2 * att.nkv) * att.d
     window = K.key_window(att.window, getattr(att, "chunk", None))
@@ -312,16 +314,17 @@ def run(att, out, qkv, ctx, mem) -> None:
         plan = ctx.plans.get(key)
         if plan is None:
             plan = ctx.plans[key] = plan_f32(ctx, att.nq, att.nkv, att.d, window, qkv.device, keep)
+        left = K.f32_terms(out.shape[0], out.shape[1], terms, out.device) if terms is not None and plan.splits == 1 else None
         K.attn_f32(out, qkv, q_row_stride, mem.pages["k"], mem.pages["v"], ctx.block_tables[mem.group], ctx.cu_seqlens,
                    ctx.context_lens, plan.work, plan.n_work, att.nq, att.nkv, att.d, att.scale, window, plan.splits,
-                   plan.parts, sinks=sinks, cap=cap, keep=keep)
-        return
+                   plan.parts, sinks=sinks, cap=cap, keep=keep, terms=None if left is None else (left, terms))
+        return out if left is None else K.TermRows(out, left, terms)
     if not K.mfma_attention_supported(qkv.dtype, att.d, ctx.page_size):
         K.paged_attention_generic(
             out, qkv, q_row_stride, mem.pages["k"], mem.pages["v"], ctx.block_tables[mem.group], ctx.token_req,
             ctx.positions, att.nq, att.nkv, att.d, att.scale, window, sinks=sinks, cap=cap, keep=keep,
         )
-        return
+        return out
     plan = _mfma_plan(att, ctx, window, keep, qkv.device)
     tables = ctx.block_tables[mem.group]
     if (plan.n_prefill and plan.n_decode and not cap and not keep and not plan.one_group
@@ -329,7 +332,7 @@ def run(att, out, qkv, ctx, mem) -> None:
         K.attn_mixed(out, qkv, q_row_stride, mem.pages["k"], mem.pages["v"], tables, ctx.cu_seqlens, ctx.context_lens, plan.prefill_work,
                      plan.n_prefill, _decode_work(ctx, plan, att, window), plan.n_decode, att.nq, att.nkv, att.d, att.scale, window,
                      plan.num_splits, plan.scratch, sinks=sinks)
-        return
+        return out
     if plan.n_prefill:
         K.attn_prefill_mfma(out, qkv, q_row_stride, mem.pages["k"], mem.pages["v"], tables, ctx.cu_seqlens,
                             ctx.context_lens, plan.prefill_work, plan.n_prefill, att.nq, att.nkv, att.d, att.scale,
@@ -338,3 +341,4 @@ def run(att, out, qkv, ctx, mem) -> None:
         K.attn_decode_mfma(out, qkv, q_row_stride, mem.pages["k"], mem.pages["v"], tables, ctx.cu_seqlens,
                            ctx.context_lens, _decode_work(ctx, plan, att, window), plan.n_decode, att.nq, att.nkv, att.d, att.scale,
                            window, plan.num_splits, plan.scratch, sinks=sinks, cap=cap, keep=keep)
+    return out

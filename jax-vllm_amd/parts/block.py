@@ -76,20 +76,20 @@ class PreNormBlock:
     def _through_stream(self, n: int, mixer, feed_forward) -> bool:
         """Whether both sublayers' last products join the stream in their own launch (few rows of a step): their first products read
         ``K.StreamRows``."""
-        return (self.has_feed_forward and self.residual_scale == 1.0 and n <= K.SKINNY_AUTO_ROWS and all(hasattr(p, "into_stream") for p in self.norms)
+        return (self.has_feed_forward and self.residual_scale == 1.0 and all(hasattr(p, "into_stream") for p in self.norms)
                 and all(hasattr(p, "leaves_product") and p.leaves_product(n) and p.takes_stream_rows(n) for p in (mixer, feed_forward)))
 
     def forward(self, h, delta, mixer, feed_forward, ctx, mem):
         n = h.shape[0]
         # one or two rows of narrow models are made by the products that read them, which then merge the attention's splits too
-        narrow = h.shape[1] <= MADE_WIDTH and not isinstance(delta, K.PendingProduct) and self._made_by_readers(h, delta, mixer, feed_forward, ctx, mem)
-        if not narrow and self._through_stream(n, mixer, feed_forward):
+        narrow = n <= K.MADE_MAX_ROWS and h.shape[1] <= MADE_WIDTH and not isinstance(delta, K.PendingProduct) and self._made_by_readers(h, delta, mixer, feed_forward, ctx, mem)
+        if n <= K.SKINNY_AUTO_ROWS and not narrow and self._through_stream(n, mixer, feed_forward):
             x = self.mixer_norm.into_stream(h, delta) if isinstance(delta, K.PendingProduct) else _add_norm(self.mixer_norm, h, delta, mixer, n)
             y = self.feed_forward_norm.into_stream(h, mixer.forward(x, ctx, mem, leave_product=True))
             return feed_forward.forward(y, ctx, leave_product=True)
         if isinstance(delta, K.PendingProduct):
             delta = delta.linear()
-        if narrow or self._made_by_readers(h, delta, mixer, feed_forward, ctx, mem):
+        if narrow or n <= K.MADE_MAX_ROWS and self._made_by_readers(h, delta, mixer, feed_forward, ctx, mem):
             between = torch.empty_like(h)                              # the stream between the two sublayers: a product's blocks all read the old one
             a = self._share(mixer.forward(self.mixer_norm.pending(h, delta, between), ctx, mem))
             if _float_parts(a):
@@ -119,6 +119,11 @@ def _add_norm(norm, h, delta, reader, n_rows: int):
     if (getattr(norm, "may_leave_scale", False) and ask is not None and not isinstance(delta, K.PendingNorm)
             and ask(n_rows)):
         return norm.add_norm(h, delta, unscaled_ok=True)
+    if n_rows > 32 and getattr(norm, "dtype", None) == torch.float32 and getattr(norm, "may_leave_terms", False) and not isinstance(delta, K.PendingNorm):
+        ask = getattr(reader, "takes_terms", None)
+        layout = ask(n_rows) if ask is not None else None
+        if layout is not None:
+            return norm.add_norm(h, delta, terms=layout)
     return norm.add_norm(h, delta)
 
 

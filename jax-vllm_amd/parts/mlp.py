@@ -49,12 +49,17 @@ class GatedMLP:
         """Whether the gate/up product reads ``K.StreamRows``."""
         return K.linear_takes_stream_rows(n_rows, self.w_gate_up, gate_pairs=True)
 
+    def takes_terms(self, n_rows: int) -> "bool | None":
+        """How the gate/up product of so many float rows takes their terms (``K.f32_terms_layout``)."""
+        return K.f32_terms_layout(n_rows, self.w_gate_up)
+
     def leaves_product(self, n_rows: int) -> bool:
         """Whether ``forward`` takes ``leave_product`` for so many rows: the last product is then left to the block."""
         return self.partial_out and K.stream_product_possible(n_rows, self.w_down)
 
     def forward(self, x, ctx=None, leave_product: bool = False):
-        z = K.linear(x, self.w_gate_up, gate_pairs=self.activation)    # gate and up rows alternate in the fused weight
+        terms = K.f32_terms_layout(x.shape[0], self.w_down) if x.dtype == torch.float32 else None
+        z = K.linear(x, self.w_gate_up, gate_pairs=self.activation, leave_terms=terms)    # gate and up rows alternate in the fused weight
         if leave_product:
             return K.PendingProduct(z, self.w_down)
         return K.linear(z, self.w_down, partial_ok=self.partial_out)   # the next norm adds the partial products

@@ -42,13 +42,16 @@ class RMSNorm:
         """``norm(h + delta)`` as rows that the product which reads them makes itself, the stream then in ``out``."""
         return K.PendingRows(h, delta, self.weight, self.eps, out)
 
+    may_leave_terms = True     # ``add_norm`` takes ``terms``
+
     def into_stream(self, h: torch.Tensor, product):
         """``h`` += what a ``K.PendingProduct`` makes, in that product's launch; returns ``K.StreamRows``."""
         return K.gemm_into_stream(h, product.x, product.w, self.weight, self.eps)
 
-    def add_norm(self, h: torch.Tensor, delta, rows=None, unscaled_ok: bool = False):
+    def add_norm(self, h: torch.Tensor, delta, rows=None, unscaled_ok: bool = False, terms: "bool | None" = None):
         """The residual step fused with the norm: ``h += delta`` in the float residual stream,
-        returns ``norm(h)`` in the activation type.  ``delta`` may be a ``K.PendingNorm``: then what is
+        returns ``norm(h)`` in the activation type (``terms``, for float rows whose reader is a 32-bit product: its
+        ``K.f32_terms_layout``, the result may then be ``K.TermRows``).  ``delta`` may be a ``K.PendingNorm``: then what is
         added is its own norm of the sublayer's output; or a ``K.PendingProduct``, which joins ``h`` in its own launch.  With ``rows`` only those rows are normed
         and ``h`` is left alone.  With ``unscaled_ok`` the reader multiplies the rows by a matrix
         through ``K.linear`` and nothing else: for the few rows of a decode step whose ``delta``
@@ -68,6 +71,9 @@ class RMSNorm:
         if (unscaled_ok and rows is None and delta is not None and delta.dim() == 3
                 and K.unscaled_rows_possible(self.dtype, h.shape[0], self.size)):
             return K.add_parts_unscaled(h, delta, self.weight, self.eps)
+        if (terms is not None and rows is None and self.dtype == torch.float32 and (delta is None or delta.dim() == 2)
+                and K.add_rmsnorm_terms_possible(self.size)):
+            return K.add_rmsnorm_terms(h, delta, self.weight, self.eps, terms)
         n_out = h.shape[0] if rows is None else rows.numel()
         out = torch.empty((n_out, self.size), dtype=self.dtype, device=h.device)
         K.add_rmsnorm(h, delta, self.weight, out, self.eps, rows)
