@@ -30,16 +30,24 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // act(gate) * up in bf16 [M][N / 2]
 enum { ST_PARTS = 0, ST_BF16 = 1, ST_PAIRS = 2 };
 
+// Rows of x whose norm's scale is still to be applied (add_parts_unscaled_kernel): row m of the result is multiplied by
+// rsqrt(sum_j ssq[m * 16 + j] inv_width + eps), j < shares.
+struct StScale {
+  const float* ssq;
+  int shares;
+  float inv_width, eps;
+};
+
 constexpr int st_loads(int total, int waves) {      // loads of a wave: the fewest that share `total` out to whole waves
   int n = (total + waves - 1) / waves;
   while (total % n) ++n;
   return n;
 }
 
-template <int MODE, int TM, int TW>
+template <int MODE, int TM, int TW, bool SCALED>
 __global__ void __launch_bounds__(64 * (TM / 32) * (TW / 32))
 gemm_stream_kernel(void* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, int M, int N, int K,
-                   long long ldx, JvAct act) {
+                   long long ldx, JvAct act, StScale scale) {
   constexpr int WN = TW / 32, WAVES = TM / 32 * WN, ROWS = TM + TW;
   constexpr int LPW = st_loads(ROWS / 8, WAVES), LOADERS = ROWS / 8 / LPW;
   constexpr int FIT = ST_LDS / (ROWS * ST_K * 2), BUFS = FIT < 9 ? FIT : 9;
@@ -72,6 +80,12 @@ gemm_stream_kernel(void* __restrict__ y, const bf16_t* __restrict__ x, const bf1
 #pragma unroll
   for (int i = 0; i < 16; ++i) acc[i] = 0.f;
   const int wm = wave / WN, wn = wave - wm * WN, l32 = lane & 31, half = lane >> 5, swz = (l32 >> 1) & 7;
+  // a lane's row of the result: its shares, eight in either half of the wave, asked for before everything else
+  f32x4 sq[SCALED ? 2 : 1];
+  if constexpr (SCALED) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) sq[i] = *(const f32x4*)(scale.ssq + (long long)min(wm * 32 + l32, M - 1) * 16 + half * 8 + i * 4);
+  }
   for (int c = 0; c < BUFS - 1 && c < chunks; ++c) fetch(c, c);
   for (int c = 0, buf = 0; c < chunks; ++c, buf = buf + 1 == BUFS ? 0 : buf + 1) {
     // this wave's part of chunk c is there (loads arrive in order; those of the next BUFS - 2 chunks may be on their way)
@@ -89,6 +103,15 @@ gemm_stream_kernel(void* __restrict__ y, const bf16_t* __restrict__ x, const bf1
   }
   // a lane holds row l32 of the wave's rows of x, columns 8 q + 4 half + e of its rows of W
   const int m = wm * 32 + l32;
+  if constexpr (SCALED) {
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) t += half * 8 + i * 4 + e < scale.shares ? sq[i][e] : 0.f;
+    t += __shfl_xor(t, 32, 64);
+    acc *= rsqrtf(t * scale.inv_width + scale.eps);
+  }
   if (m >= M) return;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -113,44 +136,48 @@ gemm_stream_kernel(void* __restrict__ y, const bf16_t* __restrict__ x, const bf1
 }
 
 template <int MODE, int TM, int TW>
-static int st_launch(void* y, const void* x, const void* W, int M, int N, int K, long long ldx, int ksplit, JvAct act, hipStream_t s) {
-  hipLaunchKernelGGL((gemm_stream_kernel<MODE, TM, TW>), dim3((N + TW - 1) / TW, ksplit), dim3(2 * TM / 32 * TW), 0, s, y,
-                     (const bf16_t*)x, (const bf16_t*)W, M, N, K, ldx, act);
+static int st_launch(void* y, const void* x, const void* W, int M, int N, int K, long long ldx, int ksplit, JvAct act, StScale scale, hipStream_t s) {
+  const auto kernel = scale.ssq ? gemm_stream_kernel<MODE, TM, TW, true> : gemm_stream_kernel<MODE, TM, TW, false>;
+  hipLaunchKernelGGL(kernel, dim3((N + TW - 1) / TW, ksplit), dim3(2 * TM / 32 * TW), 0, s, y, (const bf16_t*)x, (const bf16_t*)W, M, N, K, ldx, act, scale);
   return JV_LAUNCH_CHECK();
 }
 template <int MODE, int TM>
-static int st_tw(int tw, void* y, const void* x, const void* W, int M, int N, int K, long long ldx, int ksplit, JvAct act, hipStream_t s) {
+static int st_tw(int tw, void* y, const void* x, const void* W, int M, int N, int K, long long ldx, int ksplit, JvAct act, StScale scale, hipStream_t s) {
   switch (tw) {
-    case 32: return st_launch<MODE, TM, 32>(y, x, W, M, N, K, ldx, ksplit, act, s);
-    case 64: return st_launch<MODE, TM, 64>(y, x, W, M, N, K, ldx, ksplit, act, s);
-    case 96: return st_launch<MODE, TM, 96>(y, x, W, M, N, K, ldx, ksplit, act, s);
-    case 128: return st_launch<MODE, TM, 128>(y, x, W, M, N, K, ldx, ksplit, act, s);
+    case 32: return st_launch<MODE, TM, 32>(y, x, W, M, N, K, ldx, ksplit, act, scale, s);
+    case 64: return st_launch<MODE, TM, 64>(y, x, W, M, N, K, ldx, ksplit, act, scale, s);
+    case 96: return st_launch<MODE, TM, 96>(y, x, W, M, N, K, ldx, ksplit, act, scale, s);
+    case 128: return st_launch<MODE, TM, 128>(y, x, W, M, N, K, ldx, ksplit, act, scale, s);
   }
   return (int)hipErrorInvalidValue;
 }
 template <int MODE>
-static int st_tm(int tm, int tw, void* y, const void* x, const void* W, int M, int N, int K, long long ldx, int ksplit, JvAct act, hipStream_t s) {
+static int st_tm(int tm, int tw, void* y, const void* x, const void* W, int M, int N, int K, long long ldx, int ksplit, JvAct act, StScale scale, hipStream_t s) {
   switch (tm) {
-    case 32: return st_tw<MODE, 32>(tw, y, x, W, M, N, K, ldx, ksplit, act, s);
-    case 64: return st_tw<MODE, 64>(tw, y, x, W, M, N, K, ldx, ksplit, act, s);
-    case 128: return st_tw<MODE, 128>(tw, y, x, W, M, N, K, ldx, ksplit, act, s);
+    case 32: return st_tw<MODE, 32>(tw, y, x, W, M, N, K, ldx, ksplit, act, scale, s);
+    case 64: return st_tw<MODE, 64>(tw, y, x, W, M, N, K, ldx, ksplit, act, scale, s);
+    case 128: return st_tw<MODE, 128>(tw, y, x, W, M, N, K, ldx, ksplit, act, scale, s);
   }
   return (int)hipErrorInvalidValue;
 }
+// ssq (rows of 16 floats, `shares` of them) or null: the scale of the norm over `width` columns is applied to the rows.
 // mode: ST_*; tm (32, 64, 128; at least M) and tw (32, 64, 96, 128): rows of x and of W of a block; ksplit > 1: ST_PARTS only.
 extern "C" int jv_gemm_stream_bf16(void* y, const void* x, const void* W, int M, int N, int K, long long ldx, int mode, int gate_act,
-                                   float act_limit, float act_slope, int tm, int tw, int ksplit, void* stream) {
+                                   float act_limit, float act_slope, int tm, int tw, int ksplit, const float* ssq, int shares, int width,
+                                   float eps, void* stream) {
   if (M <= 0 || N <= 0) return 0;
+  if (ssq && (shares < 1 || shares > 16 || width <= 0 || ((uintptr_t)ssq & 15))) return (int)hipErrorInvalidValue;
   if (M > tm || K < ST_K || K % ST_K || N % 4 || ldx % 8 || ksplit < 1 || ksplit > K / ST_K || (ksplit > 1 && mode != ST_PARTS) ||
       (((uintptr_t)x | (uintptr_t)W | (uintptr_t)y) & 15))
     return (int)hipErrorInvalidValue;
   if (mode == ST_PAIRS && !jv_act_known(gate_act)) return (int)hipErrorInvalidValue;
   const JvAct act{gate_act, act_limit, act_slope};
+  const StScale scale{ssq, shares, ssq ? 1.f / (float)width : 0.f, eps};
   const hipStream_t s = (hipStream_t)stream;
   switch (mode) {
-    case ST_PARTS: return st_tm<ST_PARTS>(tm, tw, y, x, W, M, N, K, ldx, ksplit, act, s);
-    case ST_BF16: return st_tm<ST_BF16>(tm, tw, y, x, W, M, N, K, ldx, ksplit, act, s);
-    case ST_PAIRS: return st_tm<ST_PAIRS>(tm, tw, y, x, W, M, N, K, ldx, ksplit, act, s);
+    case ST_PARTS: return st_tm<ST_PARTS>(tm, tw, y, x, W, M, N, K, ldx, ksplit, act, scale, s);
+    case ST_BF16: return st_tm<ST_BF16>(tm, tw, y, x, W, M, N, K, ldx, ksplit, act, scale, s);
+    case ST_PAIRS: return st_tm<ST_PAIRS>(tm, tw, y, x, W, M, N, K, ldx, ksplit, act, scale, s);
   }
   return (int)hipErrorInvalidValue;
 }

@@ -181,7 +181,7 @@ class PendingProduct:
 
 
 def unscaled_rows_possible(dtype, n_rows: int, hidden: int) -> bool:
-    return (dtype == torch.bfloat16 and 0 < n_rows <= SKINNY_AUTO_ROWS and hidden % UNSCALED_SHARE == 0
+    return (dtype == torch.bfloat16 and 0 < n_rows <= STREAM_MAX_ROWS and hidden % UNSCALED_SHARE == 0
             and hidden // UNSCALED_SHARE <= UNSCALED_MAX_SHARES)
 
 
@@ -196,7 +196,7 @@ def add_parts_unscaled(h: torch.Tensor, parts: torch.Tensor, weight: torch.Tenso
     _f32(weight, "weight", hidden)
     _need(parts.dtype == torch.float32 and parts.dim() == 3 and parts.shape[1:] == h.shape and 1 <= parts.shape[0] <= 4,
           "partial products must be float32 [parts <= 4, *h.shape]")
-    _need(unscaled_rows_possible(torch.bfloat16, n, hidden), "at most 16 rows of a width that is a multiple of 512, at most 8192")
+    _need(unscaled_rows_possible(torch.bfloat16, n, hidden), "at most 128 rows of a width that is a multiple of 512, at most 8192")
     xg = torch.empty((n, hidden), dtype=torch.bfloat16, device=h.device)
     ssq = torch.empty((n, UNSCALED_MAX_SHARES), dtype=torch.float32, device=h.device)    # hidden / 512 of a row's 16 are written
     _check(library.core().jv_add_parts_unscaled_bf16(_ptr(h), _ptr(parts), c_int(parts.shape[0]), c_longlong(parts.stride(0)),
@@ -1176,6 +1176,7 @@ def streaming_plan(m: int, n: int, k: int, gate_pairs: bool = False, partial_ok:
 
 STREAM_MAX_ROWS = 128
 STREAM_MODES = {"parts": 0, "rows": 1, "pairs": 2}
+_NO_SCALE = (c_void_p(None), c_int(0), c_int(0), c_float(0.0))
 
 
 def _ring_time(m: int, n: int, k: int, tm: int, tw: int, parts: int, cus: int) -> float:
@@ -1239,7 +1240,7 @@ def ring_plan(m: int, n: int, k: int, mode: str, cus: int = 256):
 
 
 def gemm_stream(x: torch.Tensor, w: torch.Tensor, form, mode: str = "rows", gate_pairs: "str | tuple | None" = None,
-                out_dtype=torch.bfloat16) -> torch.Tensor:
+                out_dtype=torch.bfloat16, row_scale: "UnscaledRows | None" = None) -> torch.Tensor:
     """x @ w.T for 17 to 128 rows of bfloat16 x (any up to 128 are taken) against bfloat16 w [N, K], K a multiple of 64: chunks
     of both through a ring in LDS.  ``form``: (rows of x, rows of w, parts of the inner size) of a block, see
     ``ring_plan``; ``mode``: "parts": float32 [parts, M, N], to be added in order; "rows": bfloat16 [M, N] (or float32, with
@@ -1253,11 +1254,17 @@ def gemm_stream(x: torch.Tensor, w: torch.Tensor, form, mode: str = "rows", gate
     _need(mode in STREAM_MODES and (parts == 1 or mode == "parts") and (mode == "pairs") == bool(gate_pairs), "only partial products have parts")
     as_float = mode == "parts" or out_dtype == torch.float32
     _need(not (as_float and gate_pairs), "the activation's result is bfloat16")
+    ssq = None
+    if row_scale is not None:      # x is row_scale.x: rows of the result, of every partial product, are multiplied by their norm's scale
+        ssq = row_scale.ssq
+        _need(row_scale.x is x and ssq.is_cuda and ssq.dtype == torch.float32 and ssq.is_contiguous() and tuple(ssq.shape) == (m, UNSCALED_MAX_SHARES)
+              and 1 <= row_scale.shares <= UNSCALED_MAX_SHARES, "row_scale does not belong to x")
     shape = (parts, m, n) if mode == "parts" else (m, n // 2) if gate_pairs else (m, n)
     y = torch.empty(shape, dtype=torch.float32 if as_float else torch.bfloat16, device=x.device)
     _check(library.core().jv_gemm_stream_bf16(
         _ptr(y), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), c_longlong(k), c_int(STREAM_MODES["parts" if as_float else mode]),
-        *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), c_int(tm), c_int(tw), c_int(parts), _stream()), "gemm_stream")
+        *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), c_int(tm), c_int(tw), c_int(parts),
+        *(_NO_SCALE if ssq is None else (_ptr(ssq), c_int(row_scale.shares), c_int(row_scale.width), c_float(row_scale.eps))), _stream()), "gemm_stream")
     return y
 
 
@@ -1293,8 +1300,6 @@ def thin_slots(m: int, n: int, k: int) -> "int | None":
         return None
     return 4 if n <= 4096 and k > 512 or n > 16384 else 2
 
-
-_NO_SCALE = (c_void_p(None), c_int(0), c_int(0), c_float(0.0))
 
 
 def gemm_thin_scaled(rows: "StreamRows", w: torch.Tensor, gate_pairs: "str | tuple | None" = None) -> torch.Tensor:
@@ -1501,14 +1506,14 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
         _need(x.dtype == w.dtype, "x and w must have one type")
         m, (n, k) = x.shape[0], w.shape
         # (chunks of 64 columns; tensors of other inner sizes are never asked for their device's compute units)
-        if k % 64 == 0 and SKINNY_AUTO_ROWS < m <= STREAM_MAX_ROWS and scale is None and w.dtype == torch.bfloat16:
+        if k % 64 == 0 and SKINNY_AUTO_ROWS < m <= STREAM_MAX_ROWS and w.dtype == torch.bfloat16:
             parts_ok = partial_ok and not gate_pairs and out_dtype in (None, torch.bfloat16) and (
                 partial_max_width is None or n <= partial_max_width)
             mode = "pairs" if gate_pairs else "parts" if parts_ok and k >= 128 else "rows"
             form = ring_plan(m, n, k, mode, compute_units(x.device))
             if form is not None and out_dtype in (None, torch.bfloat16, torch.float32) and x.is_contiguous() and w.is_contiguous() \
                     and not (x.data_ptr() | w.data_ptr()) & 15 and not (gate_pairs and out_dtype == torch.float32):
-                return gemm_stream(x, w, form, mode, gate_pairs, out_dtype or torch.bfloat16)
+                return gemm_stream(x, w, form, mode, gate_pairs, out_dtype or torch.bfloat16, scale)
         elif k % 64 == 0 and m > STREAM_MAX_ROWS and partial_ok and not gate_pairs and scale is None and w.dtype == torch.bfloat16 \
                 and out_dtype in (None, torch.bfloat16) and partial_max_width is not None and n <= partial_max_width:
             cus = compute_units(x.device)
@@ -1627,9 +1632,16 @@ def _linear_made(x, w: torch.Tensor, gate_pairs, partial_ok: bool, partial_max_w
 
 def linear_takes_unscaled_rows(n_rows: int, w: torch.Tensor, gate_pairs: bool = False, partial_ok: bool = False,
                                partial_max_width: int | None = PARTIAL_SUM_MAX_WIDTH) -> bool:
-    """Whether ``linear`` with these arguments multiplies ``UnscaledRows`` (its plan is the blocks that stay)."""
+    """Whether ``linear`` with these arguments multiplies ``UnscaledRows`` (its plan is the blocks that stay, or the ring of 17 to 128 rows)."""
     if w.dtype != torch.bfloat16 or not unscaled_rows_possible(torch.bfloat16, n_rows, w.shape[1]):
         return False
+    if n_rows > SKINNY_AUTO_ROWS:
+        n, k = w.shape
+        if k % 64:
+            return False
+        parts_ok = partial_ok and not gate_pairs and (partial_max_width is None or n <= partial_max_width)
+        if ring_plan(n_rows, n, k, "pairs" if gate_pairs else "parts" if parts_ok else "rows", compute_units(w.device)) is not None:
+            return w.is_contiguous() and not w.data_ptr() & 15
     plan = streaming_plan(n_rows, w.shape[0], w.shape[1], bool(gate_pairs), partial_ok, w.device, partial_max_width)
     return plan is not None and plan[0] != TILE64 and plan[0][0] == -2
 
