@@ -1179,6 +1179,321 @@ template <int PAGES, bool MORE>
 __global__ void __launch_bounds__(256) PREFILL32_OCCUPANCY attn_prefill32_kernel(AttnArgs p) {
   attn_prefill32_block<PAGES, MORE>(p, blockIdx.x);
 }
+
+#if JV_HEAD_DIM == 256
+#define JV_PREFILL_HALVES 1
+// Head size 256 at pages of 16 keys.  32 rows' results and queries alone are 192 registers a lane: a wave that has a SIMD and all
+// of them to itself carried them between its register files and spilled (353 of them with the overlap below).  Here two waves share 32 rows: each
+// scores one of a tile's two 32-key blocks, the pair's maxima and probabilities meet in LDS, and each multiplies them into half of the head's
+// elements.  Half the registers, two waves a SIMD, and every fragment of K and V^T is still read once for 32 rows.  Two barriers a tile: A hands
+// over the maxima and this tile's V^T, B the probabilities and the K of the tile after next; between them the next tile's scores are multiplied
+// under this one's exponentials, behind B the next maxima are found under the products with V^T.  K and V^T are asked for a whole tile's time ahead.
+// Bounds: the matrix unit, 33 of 75 cycles in the long run (LDS about 25), and a start and an end of 15 us in which 64 KB of queries a
+// block come and as much of results go with nothing beside them.  2,048 tokens, 16 heads over one: window 1,024 68.5 -> 51.4 us, 128 39 -> 23; 8,192
+// tokens without one 677 -> 622 (0.88 PFLOP/s); 4,096 tokens, window 1,024, capped scores 140 -> 108.
+template <bool MORE>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) attn_prefill_halves_kernel(AttnArgs p) {
+  constexpr int PC = BN * CPK / 512, HDB = NDB / 2;      // 16-byte pieces of a K (and of a V^T) tile a thread; 32-row blocks of O^T a wave
+  __shared__ __attribute__((aligned(16))) bf16_t Ks[2][BN * D];
+  __shared__ __attribute__((aligned(16))) bf16_t Vs[2][D * BN];
+  __shared__ __attribute__((aligned(16))) bf16_t Ps[4][32 * BN];      // of 32 rows: [row][8 pieces of 8 keys], piece c at c ^ (row % 8)
+  __shared__ float meet[8][32];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), rt = wave >> 1, hf = wave & 1;
+  const int l32 = lane & 31, h = lane >> 5;
+  const int g = blockIdx.x % p.nkv, item = blockIdx.x / p.nkv;
+  const int r = p.work[3 * item], G = p.nq / p.nkv;
+  const int q_start = p.cu_seqlens[r], q_len = p.cu_seqlens[r + 1] - q_start, ctx = p.context_lens[r], M = q_len * G;
+  const int* gtable = p.block_tables + (long long)r * p.table_stride;
+  int blk_begin[2], blk_end[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int m0 = p.work[3 * item + 1 + t];
+    blk_begin[t] = blk_end[t] = 0;
+    if (m0 >= 0 && m0 < M) {
+      const int last_row = (M < m0 + 64 ? M : m0 + 64) - 1;
+      blk_end[t] = ctx + last_row / G + 1;
+      blk_begin[t] = first_key(ctx + m0 / G, p.window);
+    }
+  }
+  const int m0 = p.work[3 * item + 1 + (rt >> 1)], wave_first = m0 + (rt & 1) * 32;
+  const bool wave_live = m0 >= 0 && wave_first < M;      // the same in both waves of a pair
+  const int wave_last = (M < wave_first + 32 ? M : wave_first + 32) - 1;
+  const int wave_min_pos = ctx + wave_first / G, wave_full_begin = wave_live ? first_key(ctx + wave_last / G, p.window) : 0;
+  const int row = wave_first + l32;
+  const bool row_ok = wave_live && row < M;
+  const int qi = row_ok ? row / G : 0, hg = row_ok ? row - qi * G : 0;
+  const int pos = ctx + qi, row_first = first_key(pos, p.window);
+  bf16x8 qf[NQS];
+  {
+    const bf16_t* qrow = p.q + (long long)(q_start + qi) * p.q_row_stride + (long long)(g * G + hg) * D + h * 8;
+    const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int ks = 0; ks < NQS; ++ks) qf[ks] = row_ok ? *(const bf16x8*)(qrow + ks * 16) : zero8;
+  }
+  // the tiles the block walks: as in attn_prefill32_block
+  int j_first, kv_end, gap_from = NO_GAP, gap_to = NO_GAP;
+  {
+    int b0 = blk_begin[0] / BN * BN, e0 = blk_end[0];
+    int b1 = blk_begin[1] / BN * BN, e1 = blk_end[1];
+    if (e1 <= b1) { b1 = b0; e1 = e0; }
+    if (e0 <= b0) { b0 = b1; e0 = e1; }
+    if (b1 < b0) { int x = b0; b0 = b1; b1 = x; x = e0; e0 = e1; e1 = x; }
+    j_first = b0;
+    kv_end = e0 > e1 ? e0 : e1;
+    const int e0_up = (e0 + BN - 1) / BN * BN;
+    if (b1 > e0_up) { gap_from = e0_up; gap_to = b1; }
+  }
+  int keep_from = NO_GAP, keep_to = NO_GAP;
+  if (MORE && p.keep > 0 && kv_end > j_first) {
+    const int keep_up = (p.keep + BN - 1) / BN * BN;
+    if (keep_up < j_first) { keep_from = keep_up; keep_to = j_first; }
+    if (keep_up > gap_from) gap_from = keep_up < gap_to ? keep_up : NO_GAP;
+    j_first = 0;
+  }
+  auto next_tile = [&](int j0) {
+    if (MORE && j0 + BN == keep_from) return keep_to;
+    return j0 + BN == gap_from ? gap_to : j0 + BN;
+  };
+  if (kv_end <= j_first) return;                    // nothing to do (the same in every thread)
+  const int last_page = (kv_end - 1) >> 4;
+
+  // instruction i of a wave brings its 1 KB of page i of the tile: two keys of K, 32 elements' rows of V^T
+  const unsigned page_stride = (unsigned)p.nkv * 16u * (unsigned)D;
+  auto k_swizzle = [&](unsigned q) { return q ^ ((q / CPK) & 15); };
+  auto v_swizzle = [&](unsigned q) { return q ^ ((q >> 4) & 1); };
+  const unsigned q0 = k_swizzle(wave * 64 + lane), qv0 = v_swizzle(wave * 64 + lane);
+  const unsigned k_off = (g * 16 + q0 / CPK) * D + q0 % CPK * 8, v_off = (g * D + (qv0 >> 1)) * 16 + (qv0 & 1) * 8;
+  auto dma16 = [&](const bf16_t* src, const bf16_t* lds) {
+    const unsigned at = (unsigned)(unsigned long long)(const __attribute__((address_space(3))) void*)lds;
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(at) : "memory", "m0");
+  };
+  typedef const __attribute__((address_space(4))) int* ctable_t;
+  const ctable_t ctable = (ctable_t)(unsigned long long)gtable;
+  auto pages_of = [&](int j0, unsigned (&pg)[PC]) {      // behind the last page that one again: its keys are masked, its values cleared
+#pragma unroll
+    for (int i = 0; i < PC; ++i) pg[i] = (unsigned)ctable[(j0 >> 4) + i < last_page ? (j0 >> 4) + i : last_page];
+  };
+  auto fetch_k = [&](int b, const unsigned (&pg)[PC]) {
+#pragma unroll
+    for (int i = 0; i < PC; ++i) dma16(p.k_pages + (unsigned long long)pg[i] * page_stride + k_off, &Ks[b][(8 * i + wave) * 64 * 8]);
+  };
+  auto fetch_v = [&](int b, const unsigned (&pg)[PC]) {
+#pragma unroll
+    for (int i = 0; i < PC; ++i) dma16(p.v_pages + (unsigned long long)pg[i] * page_stride + v_off, &Vs[b][(8 * i + wave) * 64 * 8]);
+  };
+  auto fix_tail = [&](int j0, int b) {      // values at or behind kv_end become zeros: a thread cleans what it asked for
+#pragma unroll
+    for (int i = 0; i < PC; ++i) {
+      const int key = j0 + i * 16 + (int)(qv0 & 1) * 8;
+      if (key + 8 > kv_end) {
+        bf16x8* at = (bf16x8*)&Vs[b][((8 * i + wave) * 64 + lane) * 8];
+        bf16x8 v = *at;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (key + e >= kv_end) v[e] = (bf16_t)0.f;
+        *at = v;
+      }
+    }
+  };
+  auto barrier = [&]() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+  // LDS read addresses (elements): K of this wave's 32 keys, V^T of its half of the elements, its pair's probabilities
+  const int krow = ((l32 >> 4) << 4) | (((l32 >> 2) & 1) << 3) | (((l32 >> 3) & 1) << 2) | (l32 & 3);
+  unsigned kr = (hf * 32 + krow) * CPK + h;
+  const unsigned vr0 = v_swizzle((hf * HDB * 32 + l32) * 2 + h) * 8;
+  bf16_t* const prow = Ps[rt] + l32 * BN;
+  auto piece = [&](int c) { return (c ^ (l32 & 7)) * 8; };
+  auto acc_key = [&](int e) { return hf * 32 + 16 * (e >> 3) + 8 * h + 4 * ((e >> 2) & 1) + (e & 3); };      // of the tile
+
+  float m_run = -INFINITY, m_ref = -INFINITY, l_lane = 0.f, alpha = 1.f, m_use = 0.f, tmax = -INFINITY;
+  f32x16 acc[HDB], sc, sn;
+#pragma unroll
+  for (int db = 0; db < HDB; ++db)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[db][e] = 0.f;
+  constexpr int GS = NQS / 4;      // score steps of a group
+  bf16x8 kf[2][GS];
+  auto read_k = [&](const bf16_t* Kb, int grp, bf16x8 (&f)[GS]) {
+#pragma unroll
+    for (int i = 0; i < GS; ++i) {
+      f[i] = *(const bf16x8*)(Kb + k_swizzle(kr + 2 * (grp * GS + i)) * 8);
+    }
+  };
+  auto score = [&](f32x16& s, int grp, const bf16x8 (&f)[GS]) {
+#pragma unroll
+    for (int i = 0; i < GS; ++i) s = mfma32(f[i], qf[grp * GS + i], s);
+  };
+  auto clear = [](f32x16& s) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) s[e] = 0.f;
+  };
+  auto mask_and_max = [&](f32x16& s, int j0) {
+    tmax = -INFINITY;
+    if (MORE && p.cap > 0.f) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s[e] = capped_score(s[e], p.cap_in, p.cap);
+    }
+    if (!(j0 + BN - 1 <= wave_min_pos && (j0 >= wave_full_begin || (MORE && j0 + BN <= p.keep)))) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int j = j0 + acc_key(e);
+        s[e] = row_ok && j <= pos && (j >= row_first || (MORE && j < p.keep)) ? s[e] : -INFINITY;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) tmax = fmaxf(tmax, s[e]);
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    if (h == 0) meet[wave][l32] = tmax;
+  };
+  // the pair's maximum; most tiles leave the reference of the exponents and with it sums and outputs as they are
+  auto follow = [&](float other) {
+    const float m_new = fmaxf(m_run, fmaxf(tmax, other));
+    m_run = m_new;
+    const bool grown = (m_new - m_ref) * p.scale_log2 > RESCALE_STEP;
+    alpha = grown ? fast_exp2((m_ref - m_new) * p.scale_log2) : 1.f;
+    if (grown) m_ref = m_new;
+    if (__builtin_amdgcn_ballot_w64(grown) != 0) {
+      l_lane *= alpha;
+#pragma unroll
+      for (int db = 0; db < HDB; ++db)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[db][e] *= alpha;
+    }
+    m_use = m_ref == -INFINITY ? 0.f : m_ref * p.scale_log2;
+  };
+  auto probabilities = [&](int half8) {      // of 8 of the lane's keys, to the pair's piece
+    bf16x8 pb;
+    float psum = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float pv = fast_exp2(fmaf(sc[8 * half8 + e], p.scale_log2, -m_use));
+      psum += pv;
+      pb[e] = (bf16_t)pv;
+    }
+    l_lane += psum;
+    *(bf16x8*)(prow + piece(hf * 4 + half8 * 2 + h)) = pb;
+  };
+
+  int j0 = j_first, j1 = next_tile(j0), j2 = j1 < kv_end ? next_tile(j1) : j1;
+  unsigned pg1[PC], pg2[PC];      // of tiles t + 1 and t + 2
+  pages_of(j0, pg2);
+  fetch_k(0, pg2);
+  fetch_v(0, pg2);
+  if (j1 < kv_end) {
+    pages_of(j1, pg1);
+    fetch_k(1, pg1);
+    if (j2 < kv_end) pages_of(j2, pg2);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PC) : "memory");
+  } else {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PC) : "memory");
+  }
+  barrier();
+  clear(sc);
+#pragma unroll
+  for (int grp = 0; grp < 4; ++grp) {
+    read_k(Ks[0], grp, kf[0]);
+    score(sc, grp, kf[0]);
+  }
+  mask_and_max(sc, j0);
+  // K(0) has been read: K(2) goes there; K(1) is needed from the loop's first barrier on
+  if (j1 < kv_end) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  barrier();
+  if (j1 < kv_end && j2 < kv_end) fetch_k(0, pg2);
+  for (int b = 0;; b ^= 1) {
+    asm volatile("" : "+v"(kr));      // addresses are made anew for each tile: kept, they would be spilled
+    const bool has1 = j1 < kv_end, has2 = has1 && j2 < kv_end;
+    const int j3 = has2 ? next_tile(j2) : j2;
+    const bool has3 = has2 && j3 < kv_end;
+    // behind the last tile the scores of an old one are multiplied once more, for nothing: a branch would cost every tile more
+    const bf16_t* Kb = Ks[b ^ 1];
+    read_k(Kb, 0, kf[0]);
+    // V(t) is there: behind it only K(t + 2) was asked for
+    if (has2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PC) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (j0 + BN > kv_end) fix_tail(j0, b);
+    barrier();                                                               // A: the maxima and V(t); everybody has read V(t - 1)
+    if (has1) fetch_v(b ^ 1, pg1);
+#pragma unroll
+    for (int i = 0; i < PC; ++i) pg1[i] = pg2[i];
+    if (has3) pages_of(j3, pg2);
+    const float other = meet[wave ^ 1][l32];
+    clear(sn);
+    read_k(Kb, 1, kf[1]);
+    __builtin_amdgcn_sched_barrier(0);
+    JV_PRIO(1);
+    score(sn, 0, kf[0]);
+    follow(other);
+    __builtin_amdgcn_sched_barrier(0);
+    read_k(Kb, 2, kf[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    score(sn, 1, kf[1]);
+    probabilities(0);
+    __builtin_amdgcn_sched_barrier(0);
+    read_k(Kb, 3, kf[1]);
+    __builtin_amdgcn_sched_barrier(0);
+    score(sn, 2, kf[0]);
+    probabilities(1);
+    const bf16_t* Vb = Vs[b];
+    bf16x8 vf[2][HDB], pf[2];
+    auto read_v = [&](int t, int set) {
+#pragma unroll
+      for (int db = 0; db < HDB; ++db) vf[set][db] = *(const bf16x8*)(Vb + vr0 + t * (2 * D * 8) + db * (32 * 2 * 8));
+    };
+    auto read_p = [&](int t, int set) { pf[set] = *(const bf16x8*)(prow + piece(2 * t + h)); };
+    __builtin_amdgcn_sched_barrier(0);
+    read_v(0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    score(sn, 3, kf[1]);
+    JV_PRIO(0);
+    // K(t + 2) is there: behind it only V(t + 1) was asked for
+    if (has2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PC) : "memory");
+    barrier();                                                               // B: the probabilities and K(t + 2); everybody has read K(t + 1)
+    if (has3) fetch_k(b ^ 1, pg2);
+    read_p(0, 0);
+    JV_PRIO(1);
+#pragma unroll
+    for (int t = 0; t < BN / 16; ++t) {
+      if (t + 1 < BN / 16) {
+        read_p(t + 1, (t + 1) & 1);
+        read_v(t + 1, (t + 1) & 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int db = 0; db < HDB; ++db) acc[db] = mfma32(vf[t & 1][db], pf[t & 1], acc[db]);
+      if (t == 1) mask_and_max(sn, j1);      // of the next tile, under the products
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    JV_PRIO(0);
+    if (!has1) break;
+    sc = sn;
+    j0 = j1; j1 = j2; j2 = j3;
+  }
+
+  float l = l_lane + __shfl_xor(l_lane, 32, 64);
+  if (h == 0) meet[wave][l32] = l;      // the maxima were read before the last barrier
+  barrier();
+  l = hf ? meet[wave ^ 1][l32] + l : l + meet[wave ^ 1][l32];
+  if (row_ok) {
+    if (p.sinks) l += fast_exp2(p.sinks[g * G + hg] * 1.4426950408889634f - m_ref * p.scale_log2);
+    const float inv = 1.f / l;
+    bf16_t* o = p.out + (long long)(q_start + qi) * p.nq * D + (long long)(g * G + hg) * D + hf * HDB * 32 + h * 4;
+#pragma unroll
+    for (int db = 0; db < HDB; ++db)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        bf16x4 v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = (bf16_t)(acc[db][4 * i + j] * inv);
+        *(bf16x4*)(o + db * 32 + i * 8) = v;
+      }
+  }
+}
+#endif
 #endif
 
 // the host's plan: rows per group, and groups a work item may name
@@ -1724,11 +2039,17 @@ extern "C" int jv_attn_prefill(void* out, const void* q, long long q_row_stride,
       return mode == 1 ? attn_prefill_kernel<1, M> : (mode == 2 ? attn_prefill_kernel<2, M> : attn_prefill_kernel<0, M>);
 #endif
 #ifdef JV_PREFILL32
-    return (page_size == 16 && pow2) ? attn_prefill32_kernel<pow2 ? 16 : 1, M>
+    return (page_size == 16 && pow2 && D < 256) ? attn_prefill32_kernel<pow2 && D < 256 ? 16 : 1, M>
            : mode == 1 ? attn_prefill32_kernel<1, M>
            : mode == 2 ? attn_prefill32_kernel<2, M> : attn_prefill32_kernel<0, M>;
 #endif
   };
+#ifdef JV_PREFILL_HALVES
+  if (page_size == 16 && !one_group) {
+    hipLaunchKernelGGL((more ? attn_prefill_halves_kernel<true> : attn_prefill_halves_kernel<false>), dim3(n_work * nkv), dim3(512), 0, (hipStream_t)stream, a);
+    return JV_LAUNCH_CHECK();
+  }
+#endif
   void (*kernel)(AttnArgs) = more ? pick(std::true_type{}) : pick(std::false_type{});
   hipLaunchKernelGGL(kernel, dim3(n_work * nkv), dim3(256), 0, (hipStream_t)stream, a);
   return JV_LAUNCH_CHECK();

@@ -160,15 +160,26 @@ def prefill_item_shape(rows: int, nkv: int, group_rows: int, kernel_groups: int,
 
 def few_rows_of_256(rows: int, keys: int, group_rows: int, compute_units: int, page_size: int = 16) -> bool:
     """Whether a step's prompt portions at head size 256 take items of one group (16 rows a wave) instead of two (32): while
-    those give no more than a quarter of the compute units a second block, unless pages of 16 and 2,048 keys make up for the start
-    (only there does the larger form overlap its own work); with pages of 16 also where nobody sees more than 256 keys, for an item
-    of two groups is slow to start.  Microseconds, two groups / one, 1,064 steps measured: 300 tokens of 16 heads over one 26 / 20, 2,048
-    over 2 90 / 95, 2,048 over one with a window of 1,024 73 / 107, of 256 44 / 43, of 128 39 / 34, 4,000 over 8 kv heads with 128
-    51 / 35; 512 after 4,000 181 / 194, with pages of 32 203 / 192, of 24 259 / 209; 2,048 over 8 kv heads with pages of 32 98 / 93."""
+    those give no more than a quarter of the compute units a second block, with pages of 16 and 2,048 keys no longer; with pages of 16 also where
+    nobody sees more than 256 keys, for an item of two groups is slow to start.  (At pages of 16 ``halves_items`` has the last word.)  Microseconds,
+    two groups / one: 512 tokens after 4,000, 16 heads over one, with pages of 32 203 / 192, of 24 259 / 209; 2,048 over 8 kv heads with pages of 32 98 / 93."""
     few = 4 * -(-rows // group_rows) <= 5 * compute_units
     if page_size != 16:
         return few
     return keys <= 256 or (few and keys < 2048)
+
+
+def halves_items(one_group: bool, groups: int, keys: int, window: int, compute_units: int):
+    """(Whether 16 rows a wave take them, groups per item) at head size 256 and pages of 16 keys, where two waves share 32 rows of the
+    other form.  Items of two neighbouring groups once they give half of the compute units a block or walk far (no slower then, and half the
+    reads), else of one group.  The 16 rows a wave remain for up to 256 keys without a sliding window, and with one while the items are few.  Microseconds, 16 rows a wave / items
+    of one group / of two, 16 heads over one: 64 tokens 10.1 / 10.7 / 13.9, 300 20.3 / 19.5 / 21.4, 512 28.6 / 26.3 / 27.3, 1,000 50.5 / 45.4 /
+    43.4, 2,048 with a window of 1,024 104 / 91 / 51, of 256 44 / 43 / 27, of 128 33 / 33 / 23; 512 after 4,000 193 / 154 / 155; blocks
+    of 256 keys, 1,400 tokens 23.1 / 24.8 / 22.1; of 128, 4,000 over 8 kv heads 48.5 / 50.8 / 51.7."""
+    pairs = 2 * groups > compute_units or keys >= 2048
+    if one_group and keys <= 256 and (window <= 0 or not pairs):
+        return True, 1
+    return False, 2 if pairs else 1
 
 
 def plan_mfma(ctx, nq: int, nkv: int, head_dim: int, window: int, device, keep: int = 0) -> MfmaPlan:
@@ -178,11 +189,14 @@ def plan_mfma(ctx, nq: int, nkv: int, head_dim: int, window: int, device, keep: 
     groups_per_item, balance = prefill_item_shape(rows, nkv, group_rows, kernel_groups, K.compute_units(device),
                                                   K.attn_prefill_waves_split(head_dim))
     cus = K.compute_units(device)
-    one_group = head_dim == 256 and few_rows_of_256(
-        rows * nkv, max([keys_seen(cl + ql, window, keep) for ql, cl in zip(ctx.q_lens_host, ctx.context_lens_host) if ql > 1],
-                        default=0), group_rows, cus, ctx.page_size)
-    if one_group:
-        groups_per_item, balance = 1, False
+    one_group = False
+    if head_dim == 256:
+        keys = max([keys_seen(cl + ql, window, keep) for ql, cl in zip(ctx.q_lens_host, ctx.context_lens_host) if ql > 1], default=0)
+        one_group = few_rows_of_256(rows * nkv, keys, group_rows, cus, ctx.page_size)
+        if ctx.page_size == 16:
+            one_group, groups_per_item, balance = *halves_items(one_group, -(-rows // group_rows) * nkv, keys, window, cus), False
+        elif one_group:
+            groups_per_item, balance = 1, False
     prefill = prefill_work_items(ctx.q_lens_host, ctx.context_lens_host, g, window, group_rows, groups_per_item,
                                  balance=balance, keep=keep)
     # head size 256: items of two groups have a unit each, and items of one group were not helped (168 steps of 257 to 512 items, all
