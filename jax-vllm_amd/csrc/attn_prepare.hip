@@ -14,6 +14,7 @@
 // pad of the pages is never written and stays the zero the storage starts with.  Sums, norms and angles
 // are float.  The first kernel: one block a token; its row is kept in LDS between the passes.
 #include "common.h"
+#include "recurrence_token.h"
 #include "v_pages_write.h"
 
 template <typename T>
@@ -89,36 +90,51 @@ attn_prepare_wide_kernel(T* __restrict__ q_out, const T* __restrict__ qkv, long 
 // the v heads (left out with v_elsewhere: the tile writer of many tokens takes them).  The head is kept in LDS
 // between its norm and its rotation (dk floats a wave).
 template <typename T>
-__global__ void __launch_bounds__(256)
-attn_prepare_heads_kernel(T* __restrict__ q_out, const T* __restrict__ qkv, long long ld,
-                          const float* __restrict__ bias, const float* __restrict__ q_w,
-                          const float* __restrict__ k_w, float eps, const float* __restrict__ cos_sin,
-                          int rot_dims, const int* __restrict__ slot_mapping, T* __restrict__ k_pages,
-                          T* __restrict__ v_pages, int page_size, int nq, int nkv, int dk, int dv, int dp,
-                          float v_scale, int v_elsewhere, long long v_off, const int* __restrict__ positions,
-                          float qt_coef, int qt_every, const T* __restrict__ v_first, long long first_stride,
-                          float mix) {
-  extern __shared__ float heads_lds[];     // [4 waves][dk]
+struct HeadsArgs {
+  T* q_out;
+  const T* qkv;
+  long long ld;
+  const float *bias, *q_w, *k_w;
+  float eps;
+  const float* cos_sin;
+  int rot_dims;
+  const int* slot_mapping;
+  T *k_pages, *v_pages;
+  int page_size, nq, nkv, dk, dv, dp;
+  float v_scale;
+  int v_elsewhere;
+  long long v_off;
+  const int* positions;
+  float qt_coef;
+  int qt_every;
+  const T* v_first;
+  long long first_stride;
+  float mix;
+};
+template <typename T>
+__device__ __forceinline__ void attn_prepare_heads_block(const HeadsArgs<T>& p, long long t, int first_head, float* heads_lds) {
+  const float *bias = p.bias, *q_w = p.q_w, *k_w = p.k_w, *cos_sin = p.cos_sin;
+  const int rot_dims = p.rot_dims, page_size = p.page_size, nq = p.nq, nkv = p.nkv, dk = p.dk, dv = p.dv, dp = p.dp;
+  T *k_pages = p.k_pages, *v_pages = p.v_pages;
   const int lane = threadIdx.x & (JV_WAVE - 1), wid = threadIdx.x / JV_WAVE;
   float* buf = heads_lds + wid * dk;
-  const long long t = blockIdx.x;
-  const int head = blockIdx.y * 4 + wid;
+  const int head = first_head + wid;
   const int n_heads = nq + 2 * nkv;
   const bool live = head < n_heads;
   const bool is_q = live && head < nq, is_v = live && head >= nq + nkv, is_k = live && !is_q && !is_v;
-  const int sm = slot_mapping ? slot_mapping[t] : -1;
+  const int sm = p.slot_mapping ? p.slot_mapping[t] : -1;
   const bool store = sm >= 0 && k_pages != nullptr;
   const long long page = store ? sm / page_size : 0;
   const int slot = store ? sm % page_size : 0;
-  const T* x = qkv + t * ld;
-  if (is_v && store && !v_elsewhere) {
+  const T* x = p.qkv + t * p.ld;
+  if (is_v && store && !p.v_elsewhere) {
     const int kvh = head - nq - nkv;
-    const long long c0 = v_off + (long long)kvh * dv;
+    const long long c0 = p.v_off + (long long)kvh * dv;
     T* dst = v_pages + (page * nkv + kvh) * (long long)dp * page_size + slot;
     for (int i = lane; i < dv; i += JV_WAVE) {
       float v = to_f32(x[c0 + i]) + (bias ? bias[c0 + i] : 0.f);
-      if (v_first) v = (1.f - mix) * v + mix * to_f32(v_first[t * first_stride + (long long)kvh * dv + i]);
-      dst[(long long)i * page_size] = from_f32<T>(v * v_scale);
+      if (p.v_first) v = (1.f - p.mix) * v + p.mix * to_f32(p.v_first[t * p.first_stride + (long long)kvh * dv + i]);
+      dst[(long long)i * page_size] = from_f32<T>(v * p.v_scale);
     }
   }
   const bool work = is_q || (is_k && store);      // a k head that nobody will read is skipped
@@ -132,13 +148,13 @@ attn_prepare_heads_kernel(T* __restrict__ q_out, const T* __restrict__ qkv, long
       buf[i] = a;
       ss = fmaf(a, a, ss);
     }
-    if (w) inv = rsqrtf(wave_sum(ss) / (float)dk + eps);
+    if (w) inv = rsqrtf(wave_sum(ss) / (float)dk + p.eps);
   }
   __syncthreads();      // every wave arrives once: the head in LDS is readable by the wave's other lanes
   if (!work) return;
-  const float temp = (is_q && positions) ? 1.f + qt_coef * logf((float)((positions[t] + 1) / qt_every) + 1.f) : 1.f;
+  const float temp = (is_q && p.positions) ? 1.f + p.qt_coef * logf((float)((p.positions[t] + 1) / p.qt_every) + 1.f) : 1.f;
   const int half = rot_dims / 2;
-  T* dst = is_q ? q_out + (t * nq + head) * dp : k_pages + ((page * nkv + (head - nq)) * page_size + slot) * (long long)dp;
+  T* dst = is_q ? p.q_out + (t * nq + head) * dp : k_pages + ((page * nkv + (head - nq)) * page_size + slot) * (long long)dp;
   for (int i = lane; i < (is_q ? dp : dk); i += JV_WAVE) {
     float val = 0.f;
     if (i < dk) {
@@ -153,6 +169,25 @@ attn_prepare_heads_kernel(T* __restrict__ q_out, const T* __restrict__ qkv, long
     }
     dst[i] = from_f32<T>(val * temp);
   }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256)
+attn_prepare_heads_kernel(HeadsArgs<T> p) {
+  extern __shared__ float heads_lds[];     // [4 waves][dk]
+  attn_prepare_heads_block<T>(p, blockIdx.x, blockIdx.y * 4, heads_lds);
+}
+
+// The same beside the recurrent mixer that reads the other columns of the same rows (recurrence_token.h): its blocks move states and keep
+// memory busy, these are a chain of round trips and had a launch
+// of their own (5.4 us as profiled beside 9.9 and 11.8).  16 requests through 8 layers, 6 of them with both, 1,013 -> 981 us.
+template <typename T, bool DELTA>
+__global__ void __launch_bounds__(TK_THREADS)
+attn_prepare_beside_token_kernel(HeadsArgs<T> p, int n, TokenArgs a, int n_requests) {
+  extern __shared__ float heads_lds[];     // [8 waves][dk]
+  const int tokens = n_requests * a.heads, block = blockIdx.x;
+  if (block < tokens) recurrence_token_block<T, DELTA>(a, block % n_requests, block / n_requests);
+  else attn_prepare_heads_block<T>(p, (block - tokens) % n, (block - tokens) / n * (TK_THREADS / 64), heads_lds);
 }
 
 // The q and k heads of many tokens, 16 bytes a lane: a head of dk elements takes dk / EP lanes (a power of two), a
@@ -239,8 +274,9 @@ attn_prepare_heads_vec_kernel(T* __restrict__ q_out, const T* __restrict__ qkv, 
                                             int nkv, int dk, int dv, int dp, float v_scale, int per_head,       \
                                             long long v_off, const int* positions, float qt_coef, int qt_every, \
                                             const void* v_first, long long first_stride, float mix,             \
-                                            void* stream) {                                                     \
+                                            void* stream, const TokenLaunch* beside) {                          \
     if (n <= 0) return 0;                                                                                       \
+    if (beside && (beside->bytes != (int)sizeof(T) || (q_w && !per_head))) return (int)hipErrorInvalidValue;    \
     if (v_first && q_w && !per_head) return (int)hipErrorInvalidValue;                                          \
     if (v_off < 0 || (positions && (qt_every <= 0 || (q_w && !per_head)))) return (int)hipErrorInvalidValue;    \
     if (q_w && !per_head && v_off != (long long)(nq + nkv) * dk) return (int)hipErrorInvalidValue;              \
@@ -252,6 +288,10 @@ attn_prepare_heads_vec_kernel(T* __restrict__ q_out, const T* __restrict__ qkv, 
       constexpr int EP = 16 / (int)sizeof(T);                                                                   \
       const bool v_tile = slot_mapping && v_written_by_tile<T>(k_pages, n, page_size, dv) &&                    \
                           ld % EP == 0 && v_off % EP == 0 && ((uintptr_t)qkv % 16) == 0;                        \
+      if (beside && (v_tile || (size_t)(TK_THREADS / 64) * dk * sizeof(float) > 24 * 1024)) {                   \
+        if (const int e = jv_token_launch(beside, stream)) return e;                                            \
+        beside = nullptr;                                                                                       \
+      }                                                                                                         \
       if (v_tile) {                                                                                             \
         const int e = launch_v_pages_write<T>(qkv, ld, v_off, slot_mapping, v_pages, page_size, n, nkv, dv,     \
                                               dp, v_scale, stream, bias ? bias + v_off : nullptr, v_first,      \
@@ -272,11 +312,20 @@ attn_prepare_heads_vec_kernel(T* __restrict__ q_out, const T* __restrict__ qkv, 
       }                                                                                                         \
       const int walk = (v_tile || !slot_mapping) ? nq + nkv : nq + 2 * nkv;                                     \
       if ((walk + 3) / 4 > 65535 || (size_t)4 * dk * sizeof(float) > 64 * 1024) return (int)hipErrorInvalidValue; \
+      const HeadsArgs<T> args = {(T*)q_out, (const T*)qkv, ld, bias, q_w, k_w, eps, cos_sin, rot_dims, slot_mapping,  \
+                                 (T*)k_pages, (T*)v_pages, page_size, nq, nkv, dk, dv, dp, v_scale, v_tile ? 1 : 0,  \
+                                 v_off, positions, qt_coef, qt_every, (const T*)v_first, first_stride, mix};    \
+      if (beside) {                                                                                             \
+        const long long blocks = (long long)beside->n_requests * beside->args.heads + (long long)n * ((walk + 7) / 8);  \
+        if (blocks > 0x7fffffffll) return (int)hipErrorInvalidValue;                                            \
+        void (*kernel)(HeadsArgs<T>, int, TokenArgs, int) =                                                     \
+            beside->delta ? attn_prepare_beside_token_kernel<T, true> : attn_prepare_beside_token_kernel<T, false>;  \
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(TK_THREADS), (size_t)(TK_THREADS / 64) * dk * sizeof(float),  \
+                           (hipStream_t)stream, args, n, beside->args, beside->n_requests);                     \
+        return JV_LAUNCH_CHECK();                                                                               \
+      }                                                                                                         \
       hipLaunchKernelGGL(attn_prepare_heads_kernel<T>, dim3(n, (walk + 3) / 4), dim3(256),                      \
-                         (size_t)4 * dk * sizeof(float), (hipStream_t)stream, (T*)q_out, (const T*)qkv, ld,     \
-                         bias, q_w, k_w, eps, cos_sin, rot_dims, slot_mapping, (T*)k_pages, (T*)v_pages,        \
-                         page_size, nq, nkv, dk, dv, dp, v_scale, v_tile ? 1 : 0, v_off, positions, qt_coef,   \
-                         qt_every, (const T*)v_first, first_stride, mix);                                       \
+                         (size_t)4 * dk * sizeof(float), (hipStream_t)stream, args);                            \
       return JV_LAUNCH_CHECK();                                                                                 \
     }                                                                                                           \
     const size_t shmem = (size_t)(nq + nkv) * dk * sizeof(float);                                               \

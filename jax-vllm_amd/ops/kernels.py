@@ -526,7 +526,7 @@ def padded_head_dim(dk: int, dv: int) -> int:
 def attn_prepare_wide(qkv, bias, q_weight, k_weight, eps: float, cos_sin, rot_dims: int, slot_mapping, k_pages, v_pages,
                       page_size: int, nq: int, nkv: int, dk: int, dv: int, dp: int, v_scale: float = 1.0,
                       norm_per_head: bool = False, values_are_keys: bool = False, positions=None,
-                      q_temperature: "tuple | None" = None, v_first=None, v_mix: float = 0.0) -> torch.Tensor:
+                      q_temperature: "tuple | None" = None, v_first=None, v_mix: float = 0.0, beside: "HeldToken | None" = None) -> torch.Tensor:
     """Attention input whose key and value sizes differ, whose q/k norm spans the whole projection, or whose rows
     carry more than q, k and v.  ``qkv`` rows
     begin with [q: nq * dk | k: nkv * dk | v: nkv * dv] (further columns are left alone); ``bias`` (float32, that width) is added first; with
@@ -537,7 +537,8 @@ def attn_prepare_wide(qkv, bias, q_weight, k_weight, eps: float, cos_sin, rot_di
     bias-free norm and rotation; needs dv == dk and no whole-projection norm).  ``q_temperature`` (coef, every) with
     ``positions`` (int32 [n]): q at position p is multiplied by 1 + coef * ln(floor((p + 1) / every) + 1).  ``v_first`` (a
     [n, nkv * dv] view of qkv's type with unit column stride): v becomes (1 - v_mix) v + v_mix v_first before it is stored
-    (not beside a norm over the whole projection).  Returns q as [n, nq * dp] with every head padded with zeros to ``dp``; keys go to
+    (not beside a norm over the whole projection).  ``beside``: a recurrent mixer's token of the same step, launched here, with few tokens in
+    the same launch (not beside that norm either).  Returns q as [n, nq * dp] with every head padded with zeros to ``dp``; keys go to
     [pages, nkv, page_size, dp], values to [pages, nkv, dp, page_size] (their pad is never written)."""
     _dev(qkv, bias, q_weight, k_weight, cos_sin, slot_mapping, k_pages, v_pages)
     n, ld = qkv.shape
@@ -570,6 +571,7 @@ def attn_prepare_wide(qkv, bias, q_weight, k_weight, eps: float, cos_sin, rot_di
         _need(v_first.is_cuda and v_first.dtype == qkv.dtype and v_first.shape == (n, nkv * dv) and (n == 0 or v_first.stride(1) == 1),
               "v_first must be a [n, nkv * dv] view of qkv's type with unit column stride")
         _need(q_weight is None or norm_per_head, "values are blended beside a per-head norm or none")
+    _need(beside is None or q_weight is None or norm_per_head, "no launch beside a norm over the whole projection")
     q = torch.empty((n, nq * dp), dtype=qkv.dtype, device=qkv.device)
     fn = getattr(library.core(), f"jv_attn_prepare_wide_{_suffix(qkv.dtype)}")
     _check(fn(_ptr(q), _ptr(qkv), c_longlong(ld), _ptr(bias), _ptr(q_weight), _ptr(k_weight), c_float(eps),
@@ -577,7 +579,8 @@ def attn_prepare_wide(qkv, bias, q_weight, k_weight, eps: float, cos_sin, rot_di
               _ptr(k_pages), _ptr(v_pages), c_int(page_size), c_int(n), c_int(nq), c_int(nkv), c_int(dk), c_int(dv),
               c_int(dp), c_float(v_scale), c_int(1 if norm_per_head else 0), c_longlong(v_off),
               _ptr(positions if q_temperature is not None else None), c_float(coef), c_int(every), _ptr(v_first),
-              c_longlong(0 if v_first is None else v_first.stride(0)), c_float(v_mix), _stream()), "attn_prepare_wide")
+              c_longlong(0 if v_first is None else v_first.stride(0)), c_float(v_mix), _stream(), beside and beside.args),
+           "attn_prepare_wide")
     return q
 
 
@@ -2605,11 +2608,20 @@ def _token_operands(proj, cols, norm_weight, state, slot_ids, cu_seqlens, heads:
     return torch.empty((n, heads * vdim), dtype=proj.dtype, device=proj.device)
 
 
+class HeldToken:
+    """A launch of ``delta_token`` or ``gated_linear_token`` that another kernel's launch of the same step takes along (``attn_prepare_wide``'s
+    ``beside``); its result is ``out``.  Holds addresses: for a launch right behind, while its caller holds the tensors."""
+
+    def __init__(self):
+        self.args = ctypes.create_string_buffer(library.core().jv_token_launch_bytes())
+        self.out = None
+
+
 def delta_token(proj, at: int, conv_weight, conv_state, dt_bias, a_log, unit_eps: float, q_scale: float, norm_weight, eps: float,
-                out_scale: float, state, slot_ids, cu_seqlens, heads: int, dim: int, vdim: int) -> torch.Tensor:
+                out_scale: float, state, slot_ids, cu_seqlens, heads: int, dim: int, vdim: int, hold: "HeldToken | None" = None) -> torch.Tensor:
     """A decode step (one token a request at most) of the gated delta rule behind its input product, in one launch: ``short_conv``,
     ``recurrence_gates``, ``head_unit_norm``, ``recurrence_steps`` and ``group_gated_norm`` over the columns [q | k | v | gate | decay |
-    write strength] of ``proj`` from ``at``, a q/k head per head.  Returns [n, heads * vdim] of ``proj``'s type."""
+    write strength] of ``proj`` from ``at``, a q/k head per head.  Returns [n, heads * vdim] of ``proj``'s type.  ``hold``: takes the launch."""
     channels = heads * (2 * dim + vdim)
     gate_at = at + channels
     out = _token_operands(proj, ((at, channels + heads * (vdim + 2)),), norm_weight, state, slot_ids, cu_seqlens, heads, dim, vdim)
@@ -2626,7 +2638,9 @@ def delta_token(proj, at: int, conv_weight, conv_state, dt_bias, a_log, unit_eps
     _check(fn(_ptr(out), _ptr(proj), c_longlong(proj.shape[1]), c_int(at), c_int(gate_at), c_int(gate_at + heads * vdim),
               c_int(gate_at + heads * vdim + heads), c_int(taps), _ptr(conv_weight), _ptr(conv_state), _ptr(dt_bias), _ptr(a_log),
               c_float(unit_eps), c_float(q_scale), _ptr(norm_weight), c_float(eps), c_float(out_scale), _ptr(state), _ptr(slot_ids),
-              _ptr(cu_seqlens), c_int(slot_ids.numel()), c_int(heads), c_int(dim), c_int(vdim), _stream()), "delta_token")
+              _ptr(cu_seqlens), c_int(slot_ids.numel()), c_int(heads), c_int(dim), c_int(vdim), _stream(), hold and hold.args), "delta_token")
+    if hold:
+        hold.out = out
     return out
 
 
@@ -2636,10 +2650,10 @@ def gated_linear_token_possible(dim: int, vdim: int, rank: int, state: torch.Ten
 
 
 def gated_linear_token(proj, at: int, decay_up, decay_bias, tau: float, q_scale: float, norm_weight, eps: float, state, slot_ids,
-                       cu_seqlens, heads: int, dim: int, vdim: int) -> torch.Tensor:
+                       cu_seqlens, heads: int, dim: int, vdim: int, hold: "HeldToken | None" = None) -> torch.Tensor:
     """A decode step (one token a request at most) of gated linear attention behind its input product, in one launch:
     ``low_rank_decay``, ``wkv_steps`` read after the update and ``group_gated_norm`` over the columns [q | k | v | gate | the decay's
-    inner size] of ``proj`` from ``at``.  Returns [n, heads * vdim] of ``proj``'s type."""
+    inner size] of ``proj`` from ``at``.  Returns [n, heads * vdim] of ``proj``'s type.  ``hold``: takes the launch."""
     gate_at = at + heads * (2 * dim + vdim)
     rank = decay_up.shape[1]
     out = _token_operands(proj, ((at, heads * (2 * dim + 2 * vdim) + rank),), norm_weight, state, slot_ids, cu_seqlens, heads, dim, vdim)
@@ -2649,8 +2663,10 @@ def gated_linear_token(proj, at: int, decay_up, decay_bias, tau: float, q_scale:
     fn = getattr(library.core(), f"jv_gated_linear_token_{_suffix(proj.dtype)}")
     _check(fn(_ptr(out), _ptr(proj), c_longlong(proj.shape[1]), c_int(at), c_int(gate_at), c_int(gate_at + heads * vdim), c_int(rank),
               _ptr(decay_up), _ptr(decay_bias), c_float(tau), c_float(q_scale), _ptr(norm_weight), c_float(eps), _ptr(state),
-              _ptr(slot_ids), _ptr(cu_seqlens), c_int(slot_ids.numel()), c_int(heads), c_int(dim), c_int(vdim), _stream()),
+              _ptr(slot_ids), _ptr(cu_seqlens), c_int(slot_ids.numel()), c_int(heads), c_int(dim), c_int(vdim), _stream(), hold and hold.args),
            "gated_linear_token")
+    if hold:
+        hold.out = out
     return out
 
 

@@ -249,12 +249,17 @@ class GroupedQueryAttention:
     def share_input(self, weight: torch.Tensor) -> None:
         self.w_qkv = weight
 
-    def forward_projected(self, proj, at: int, ctx: StepContext, mem: LayerMemory) -> torch.Tensor:
+    @property
+    def takes_beside(self) -> bool:
+        """Whether ``forward_projected`` takes a ``K.HeldToken`` along."""
+        return self.wide and not self.filtered and (self.q_norm is None or self.qk_norm == "head")
+
+    def forward_projected(self, proj, at: int, ctx: StepContext, mem: LayerMemory, beside=None) -> torch.Tensor:
         """The rest of the mixer behind its input product, whose columns begin at ``at`` (0: the heads are read from the
         rows' beginning)."""
         if at:
             raise ValueError("the attention's heads begin its rows")
-        return self._forward_wide(proj, ctx, mem)
+        return self._forward_wide(proj, ctx, mem, beside)
 
     # ---- one step
     def forward(self, x, ctx: StepContext, mem: LayerMemory, leave_product: bool = False):
@@ -317,7 +322,7 @@ class GroupedQueryAttention:
             K.add_bias(y, self.b_o)
         return y
 
-    def _forward_wide(self, qkv, ctx: StepContext, mem: LayerMemory):
+    def _forward_wide(self, qkv, ctx: StepContext, mem: LayerMemory, beside=None):
         rotary_dim, interleaved = self.rotation if self.rotation is not None else (0, False)
         cos_sin = self.position.rotation_table(ctx) if self.rotation is not None else None
         if interleaved:
@@ -339,7 +344,7 @@ class GroupedQueryAttention:
             mem.pages["v"] if writes else None, ctx.page_size, self.nq, self.nkv, self.dk, self.dv, self.d, self.v_scale,
             norm_per_head=self.qk_norm == "head", values_are_keys=self.values_are_keys,
             positions=ctx.positions if self.q_temperature is not None else None, q_temperature=self.q_temperature,
-            v_first=values, v_mix=self.blend)
+            v_first=values, v_mix=self.blend, beside=beside)
         out = torch.empty((qkv.shape[0], self.nq * self.d), dtype=qkv.dtype, device=qkv.device)
         from . import attention_backend
 

@@ -195,13 +195,28 @@ class GatedDeltaMixer:
     def forward(self, x, ctx: StepContext, mem: LayerMemory):
         return self.forward_projected(K.linear(x, self.w_in), 0, ctx, mem)
 
+    # ---- a token of a step, also beside another kernel's blocks (``ParallelMixer``)
+    def token_possible(self, ctx: StepContext, mem: LayerMemory) -> bool:
+        return ctx.decode_only and self.qk_heads == self.heads and K.recurrence_token_possible(self.dim, self.vdim, mem.states["S"])
+
+    def _token(self, proj, at: int, ctx: StepContext, mem: LayerMemory, hold=None):
+        return K.delta_token(proj, at, self.conv_w, mem.states["conv"], self.dt_bias, self.a_log, self.unit_eps, self.dim ** -0.5,
+                             self.norm_weight, self.eps, self.out_scale, mem.states["S"], ctx.slot_ids, ctx.cu_seqlens, self.heads,
+                             self.dim, self.vdim, hold=hold)
+
+    def hold_token(self, proj, at: int, ctx: StepContext, mem: LayerMemory):
+        held = K.HeldToken()
+        self._token(proj, at, ctx, mem, hold=held)
+        return held
+
+    def finish_token(self, held):
+        return K.linear(held.out, self.w_o, partial_ok=True)
+
     def forward_projected(self, proj, at: int, ctx: StepContext, mem: LayerMemory):
         """The mixer behind its input product, whose columns begin at ``at``."""
         H, d, dv, qk, inner = self.heads, self.dim, self.vdim, self.qk, self.inner
-        if ctx.decode_only and self.qk_heads == H and K.recurrence_token_possible(d, dv, mem.states["S"]):
-            y = K.delta_token(proj, at, self.conv_w, mem.states["conv"], self.dt_bias, self.a_log, self.unit_eps, d ** -0.5,
-                              self.norm_weight, self.eps, self.out_scale, mem.states["S"], ctx.slot_ids, ctx.cu_seqlens, H, d, dv)
-            return K.linear(y, self.w_o, partial_ok=True)
+        if self.token_possible(ctx, mem):
+            return K.linear(self._token(proj, at, ctx, mem), self.w_o, partial_ok=True)
         qkv = K.short_conv(proj, at, self.channels, self.conv_w, None, mem.states["conv"], ctx.slot_ids, ctx.cu_seqlens,
                            ctx.max_q_len)
         gate_at = at + self.channels
@@ -348,16 +363,30 @@ class GatedLinearAttention:
     def forward(self, x, ctx: StepContext, mem: LayerMemory):
         return self.forward_projected(K.linear(x, self.w_in), 0, ctx, mem)
 
+    # ---- a token of a step, also beside another kernel's blocks (``ParallelMixer``)
+    def token_possible(self, ctx: StepContext, mem: LayerMemory) -> bool:
+        return ctx.decode_only and K.gated_linear_token_possible(self.dim, self.vdim, self.rank, mem.states["S"])
+
+    def _token(self, proj, at: int, ctx: StepContext, mem: LayerMemory, hold=None):
+        return K.gated_linear_token(proj, at, self.w_decay_up, self.b_decay, self.tau, self.dim ** -0.5, self.norm_weight, self.eps,
+                                    mem.states["S"], ctx.slot_ids, ctx.cu_seqlens, self.heads, self.dim, self.vdim, hold=hold)
+
+    def hold_token(self, proj, at: int, ctx: StepContext, mem: LayerMemory):
+        held = K.HeldToken()
+        self._token(proj, at, ctx, mem, hold=held)
+        return held
+
+    def finish_token(self, held):
+        return K.linear(held.out, self.w_o, partial_ok=True)
+
     def forward_projected(self, proj, at: int, ctx: StepContext, mem: LayerMemory):
         """The mixer behind its input product, whose columns begin at ``at``."""
         H, d, dv = self.heads, self.dim, self.vdim
         k_at, v_at = at + H * d, at + 2 * H * d
         gate_at = v_at + H * dv
         low_at = gate_at + H * dv
-        if ctx.decode_only and K.gated_linear_token_possible(d, dv, self.rank, mem.states["S"]):
-            y = K.gated_linear_token(proj, at, self.w_decay_up, self.b_decay, self.tau, d ** -0.5, self.norm_weight, self.eps,
-                                     mem.states["S"], ctx.slot_ids, ctx.cu_seqlens, H, d, dv)
-            return K.linear(y, self.w_o, partial_ok=True)
+        if self.token_possible(ctx, mem):
+            return K.linear(self._token(proj, at, ctx, mem), self.w_o, partial_ok=True)
         log_decay = K.low_rank_decay(proj[:, low_at:low_at + self.rank], self.w_decay_up, self.b_decay, self.tau)
         o = K.wkv_steps(proj[:, at:k_at], proj[:, k_at:v_at], proj[:, v_at:gate_at], log_decay, None, None, mem.states["S"],
                         ctx.slot_ids, ctx.cu_seqlens, H, d, dv, chunk_plan=K.wkv_chunk_plan(ctx, d), after=True,
@@ -438,8 +467,14 @@ class ParallelMixer:
     def forward(self, x, ctx: StepContext, mem: LayerMemory):
         if self.w_in is not None and x.shape[0] <= K.SKINNY_MAX_ROWS:
             proj = K.linear(x, self.w_in)
-            results = [part.forward_projected(proj, at, ctx, mem.below(prefix))
-                       for (prefix, part, _), at in zip(self.sides, (0, self.right_at))]
+            (left_name, left, _), (right_name, right, _) = self.sides
+            right_mem = mem.below(right_name)
+            if getattr(left, "takes_beside", False) and hasattr(right, "hold_token") and right.token_possible(ctx, right_mem):
+                held = right.hold_token(proj, self.right_at, ctx, right_mem)
+                results = [left.forward_projected(proj, 0, ctx, mem.below(left_name), beside=held), right.finish_token(held)]
+            else:
+                results = [part.forward_projected(proj, at, ctx, mem.below(prefix))
+                           for (prefix, part, _), at in zip(self.sides, (0, self.right_at))]
         else:
             results = [part.forward(x, ctx, mem.below(prefix)) for prefix, part, _ in self.sides]
         if self.out_norm_eps is not None:
