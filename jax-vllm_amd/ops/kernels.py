@@ -31,7 +31,8 @@ def _suffix(dtype: torch.dtype) -> str:
 
 
 # An eager step is launched call by call, and a short prompt's kernels are shorter than what a careless wrapper costs (37 tokens
-# through 36 layers: 330 launches, 4.6 ms of kernels): these four run several times per launch.  A torch without a GPU build, which can
+# through 36 layers: 330 launches, 4.6 ms of kernels): these few run several times per launch (and the sizes that a tensor's shape
+# gives go to the entry points as they are, for ctypes takes a plain int as a C int).  A torch without a GPU build, which can
 # plan but not launch, has neither name.
 _raw_stream, _device_index = (getattr(torch._C, name, None) for name in ("_cuda_getCurrentRawStream", "_cuda_getDevice"))
 
@@ -45,6 +46,22 @@ def _stream() -> c_void_p:
 
 def _ptr(t) -> c_void_p:
     return c_void_p(None if t is None else t.data_ptr())
+
+
+_KINDS = {"p": c_void_p, "i": c_int, "l": c_longlong, "f": c_float}
+
+
+@functools.lru_cache(maxsize=None)
+def _entry(name: str, kinds: str, head_dim: "int | None" = None):
+    """Entry point ``name`` of the core library, or of a head size's attention library, with its arguments' types: it takes plain numbers and addresses, where
+    an object of ctypes for each argument would cost a third of a short prompt's wrappers (294 launches of 37 tokens through 36 layers)."""
+    fn = getattr(library.core() if head_dim is None else _attention_library(head_dim), name)
+    fn.argtypes = [_KINDS[kind] for kind in kinds]
+    return fn
+
+
+def _address(t) -> "int | None":
+    return None if t is None else t.data_ptr()
 
 
 def _need(cond: bool, msg: str) -> None:
@@ -65,16 +82,19 @@ def _check(code: int, name: str) -> None:
         raise RuntimeError(f"{name}: HIP error {code}")
 
 
+def _typed(t, dtype, kind: str, name: str, n: int | None) -> None:
+    if t.dtype != dtype:
+        raise KernelArgumentError(f"{name} must be {kind}")
+    if n is not None and t.numel() != n:
+        raise KernelArgumentError(f"{name} must have {n} entries, has {t.numel()}")
+
+
 def _i32(t, name: str, n: int | None = None) -> None:
-    _need(t.dtype == torch.int32, f"{name} must be int32")
-    if n is not None:
-        _need(t.numel() == n, f"{name} must have {n} entries, has {t.numel()}")
+    _typed(t, torch.int32, "int32", name, n)
 
 
 def _f32(t, name: str, n: int | None = None) -> None:
-    _need(t.dtype == torch.float32, f"{name} must be float32")
-    if n is not None:
-        _need(t.numel() == n, f"{name} must have {n} entries, has {t.numel()}")
+    _typed(t, torch.float32, "float32", name, n)
 
 
 # --------------------------------------------------------------------------- embedding
@@ -199,9 +219,9 @@ def add_parts_unscaled(h: torch.Tensor, parts: torch.Tensor, weight: torch.Tenso
     _need(unscaled_rows_possible(torch.bfloat16, n, hidden), "at most 128 rows of a width that is a multiple of 512, at most 8192")
     xg = torch.empty((n, hidden), dtype=torch.bfloat16, device=h.device)
     ssq = torch.empty((n, UNSCALED_MAX_SHARES), dtype=torch.float32, device=h.device)    # hidden / 512 of a row's 16 are written
-    _check(library.core().jv_add_parts_unscaled_bf16(_ptr(h), _ptr(parts), c_int(parts.shape[0]), c_longlong(parts.stride(0)),
-                                                     _ptr(weight), _ptr(xg), _ptr(ssq), c_int(n), c_int(hidden), _stream()),
-           "add_parts_unscaled")
+    _check(_entry("jv_add_parts_unscaled_bf16", "ppilpppiip")(
+        h.data_ptr(), parts.data_ptr(), parts.shape[0], parts.stride(0), weight.data_ptr(), xg.data_ptr(), ssq.data_ptr(), n, hidden, _stream()),
+        "add_parts_unscaled")
     return UnscaledRows(xg, ssq, hidden, eps)
 
 
@@ -499,11 +519,10 @@ def qk_norm_rope_write(qkv, slot_mapping, q_weight, k_weight, eps, cos_sin, rota
         _need(parts.dtype == torch.float32 and parts.dim() == 3 and 1 <= parts.shape[0] <= 4
               and parts.shape[1:] == qkv.shape, "parts must be float32 [1..4, tokens, (nq + 2 nkv) * D]")
         _check(
-            library.core().jv_qk_norm_rope_write_parts_bf16(
-                _ptr(qkv), _ptr(parts), c_int(parts.shape[0]), c_longlong(parts.stride(0)),
-                _ptr(slot_mapping if k_pages is not None else None), _ptr(q_weight), _ptr(k_weight), c_float(eps),
-                _ptr(cos_sin), c_int(rotary_dim if cos_sin is not None else 0), _ptr(k_pages), _ptr(v_pages),
-                c_int(page_size), c_int(n), c_int(nq), c_int(nkv), c_int(head_dim), _stream()),
+            _entry("jv_qk_norm_rope_write_parts_bf16", "ppilpppfpippiiiiip")(
+                qkv.data_ptr(), parts.data_ptr(), parts.shape[0], parts.stride(0), _address(slot_mapping if k_pages is not None else None),
+                _address(q_weight), _address(k_weight), eps, _address(cos_sin), rotary_dim if cos_sin is not None else 0, _address(k_pages),
+                _address(v_pages), page_size, n, nq, nkv, head_dim, _stream()),
             "qk_norm_rope_write",
         )
         return
@@ -1260,14 +1279,14 @@ def gemm_stream(x: torch.Tensor, w: torch.Tensor, form, mode: str = "rows", gate
     ssq = None
     if row_scale is not None:      # x is row_scale.x: rows of the result, of every partial product, are multiplied by their norm's scale
         ssq = row_scale.ssq
-        _need(row_scale.x is x and ssq.is_cuda and ssq.dtype == torch.float32 and ssq.is_contiguous() and tuple(ssq.shape) == (m, UNSCALED_MAX_SHARES)
+        _need(row_scale.x is x and ssq.is_cuda and ssq.dtype == torch.float32 and ssq.is_contiguous() and ssq.shape == (m, UNSCALED_MAX_SHARES)
               and 1 <= row_scale.shares <= UNSCALED_MAX_SHARES, "row_scale does not belong to x")
     shape = (parts, m, n) if mode == "parts" else (m, n // 2) if gate_pairs else (m, n)
     y = torch.empty(shape, dtype=torch.float32 if as_float else torch.bfloat16, device=x.device)
-    _check(library.core().jv_gemm_stream_bf16(
-        _ptr(y), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), c_longlong(k), c_int(STREAM_MODES["parts" if as_float else mode]),
-        *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), c_int(tm), c_int(tw), c_int(parts),
-        *(_NO_SCALE if ssq is None else (_ptr(ssq), c_int(row_scale.shares), c_int(row_scale.width), c_float(row_scale.eps))), _stream()), "gemm_stream")
+    _check(_entry("jv_gemm_stream_bf16", "pppiiiliiffiiipiifp")(
+        y.data_ptr(), x.data_ptr(), w.data_ptr(), m, n, k, k, STREAM_MODES["parts" if as_float else mode],
+        *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), tm, tw, parts,
+        *(_NO_SCALE if ssq is None else (ssq.data_ptr(), row_scale.shares, row_scale.width, row_scale.eps)), _stream()), "gemm_stream")
     return y
 
 
@@ -1633,17 +1652,22 @@ def _linear_made(x, w: torch.Tensor, gate_pairs, partial_ok: bool, partial_max_w
     return y if gate_pairs else UnscaledParts(y, ssq, k, x.eps)
 
 
+@functools.lru_cache(maxsize=4096)
+def _ring_takes_unscaled(m: int, n: int, k: int, gate_pairs: bool, partial_ok: bool, partial_max_width, cus: int) -> bool:
+    parts_ok = partial_ok and not gate_pairs and (partial_max_width is None or n <= partial_max_width)
+    return ring_plan(m, n, k, "pairs" if gate_pairs else "parts" if parts_ok else "rows", cus) is not None
+
+
 def linear_takes_unscaled_rows(n_rows: int, w: torch.Tensor, gate_pairs: bool = False, partial_ok: bool = False,
                                partial_max_width: int | None = PARTIAL_SUM_MAX_WIDTH) -> bool:
     """Whether ``linear`` with these arguments multiplies ``UnscaledRows`` (its plan is the blocks that stay, or the ring of 17 to 128 rows)."""
-    if w.dtype != torch.bfloat16 or not unscaled_rows_possible(torch.bfloat16, n_rows, w.shape[1]):
+    n, k = w.shape
+    if w.dtype != torch.bfloat16 or not unscaled_rows_possible(torch.bfloat16, n_rows, k):
         return False
     if n_rows > SKINNY_AUTO_ROWS:
-        n, k = w.shape
         if k % 64:
             return False
-        parts_ok = partial_ok and not gate_pairs and (partial_max_width is None or n <= partial_max_width)
-        if ring_plan(n_rows, n, k, "pairs" if gate_pairs else "parts" if parts_ok else "rows", compute_units(w.device)) is not None:
+        if _ring_takes_unscaled(n_rows, n, k, bool(gate_pairs), bool(partial_ok), partial_max_width, compute_units(w.device)):
             return w.is_contiguous() and not w.data_ptr() & 15
     plan = streaming_plan(n_rows, w.shape[0], w.shape[1], bool(gate_pairs), partial_ok, w.device, partial_max_width)
     return plan is not None and plan[0] != TILE64 and plan[0][0] == -2
@@ -1754,12 +1778,11 @@ def attn_prefill_mfma(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_s
     page_size = _attn_common(out, q, q_row_stride, k_pages, v_pages, block_tables, cu_seqlens, context_lens, work,
                              nq, nkv, head_dim)
     _need(work.numel() >= 3 * n_work, "work list shorter than n_work")
-    lib = _attention_library(head_dim)
     _check(
-        lib.jv_attn_prefill(_ptr(out), _ptr(q), c_longlong(q_row_stride), _ptr(k_pages), _ptr(v_pages),
-                            _ptr(block_tables), c_int(block_tables.shape[1]), _ptr(cu_seqlens), _ptr(context_lens),
-                            _ptr(work), c_int(n_work), c_int(page_size), c_int(nq), c_int(nkv), c_float(scale),
-                            c_int(window or 0), _ptr(sinks), c_float(cap), c_int(keep if window else 0), c_int(one_group), _stream()),
+        _entry("jv_attn_prefill", "pplpppipppiiiifipfiip", head_dim)(
+            out.data_ptr(), q.data_ptr(), q_row_stride, k_pages.data_ptr(), v_pages.data_ptr(), block_tables.data_ptr(), block_tables.shape[1],
+            cu_seqlens.data_ptr(), context_lens.data_ptr(), work.data_ptr(), n_work, page_size, nq, nkv, scale, window or 0, _address(sinks), cap,
+            keep if window else 0, bool(one_group), _stream()),
         "attn_prefill_mfma",
     )
 
