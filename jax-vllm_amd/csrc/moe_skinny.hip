@@ -112,27 +112,28 @@ moe_skinny_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, con
   }
 }
 
-// The same where an expert's rows begin on 16 bytes and the inner size is a multiple of 64 up to 4,096: WK of a block's 8 waves share
+// The same where an expert's rows begin on 16 bytes and the inner size is a multiple of 64 up to 4,096: WK of a block's waves share
 // out the inner size of 16 rows of W, the others take further 16 rows.  A wave asks for its rows of x (into registers, where they
 // stay) and for its first chunks of W (whole lines, straight into a ring of its own in LDS) in one go and waits for no other wave
-// before the parts meet; two blocks of 64 KB share a unit, so one's chain of addresses runs beside the other's stream.
+// before the parts meet; several blocks share a unit, so one's chain of addresses runs beside the others' streams: two of 64 KB, or four and more of
+// half of that or less where their slices stay long enough (microseconds in graphs, cold weights, two of 64 KB / so: 16 tokens, 4 of 32 experts, 768 x 2,048
+// 30.2 + 16.5 / 28.9 + 15.4, 512 x 2,048 27.1 + 13.9 / 25.8 + 12.6; 48 of 64 x 1,024, width 4,096, down 102.7 / 99.0; inner sizes of 4,096 as before: 152 / 152).
 // Both products of a layer in a graph, cold weights, microseconds (the kernel above): 32 experts x 768, 4 chosen, width 2,048: 4
 // tokens 28.2 (29.9), 16 56.3 (59.9), 48 62.7 (69.9); 32 x 512 of width 1,536: 1 token 10.7 (14.2), 8 31.1 (35.0); 64 x 1,024, 8 chosen, width
 // 4,096: 16 tokens 252 (261), 48 288 (318), 5.5 TB/s.  Not better: one wave a row tile at inner sizes up to 512, 4 at 2,048.
 #define MF_K 64            // columns of a chunk: a row of it is 128 bytes, 8 pieces of 16
-#define MF_WAVES 8
 
-// CW: the most chunks of a wave.
-template <int MODE, int WK, int CW>
-__global__ void __launch_bounds__(64 * MF_WAVES)
+// WAVES of a block, the KB of their rings; CW: the most chunks of a wave.
+template <int MODE, int WAVES, int KB, int WK, int CW>
+__global__ void __launch_bounds__(64 * WAVES)
 moe_few_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, const bf16_t* __restrict__ W0,
                const bf16_t* __restrict__ W1, const int* __restrict__ meta, const int* __restrict__ offsets,
                const int* __restrict__ tile_expert, const int* __restrict__ tile_row0, const int* __restrict__ order,
                const float* __restrict__ weights, int top, int n_tokens, int K, int N, JvAct act, int use_weight) {
   constexpr bool GATED = MODE == MS_GATED, BY_TOKEN = MODE != MS_DOWN;
-  constexpr int NT = MF_WAVES / WK, NB = 16 * NT, MATS = GATED ? 2 : 1, L = 2 * MATS, CHUNK = 16 * MATS * MF_K;
-  constexpr int FIT = 64 * 1024 / (MF_WAVES * CHUNK * 2), S = FIT < CW ? FIT : CW;
-  __shared__ __attribute__((aligned(1024))) bf16_t bufs[MF_WAVES][S * CHUNK];
+  constexpr int NT = WAVES / WK, NB = 16 * NT, MATS = GATED ? 2 : 1, L = 2 * MATS, CHUNK = 16 * MATS * MF_K;
+  constexpr int FIT = KB * 1024 / (WAVES * CHUNK * 2), S = FIT < CW ? FIT : CW;
+  __shared__ __attribute__((aligned(1024))) bf16_t bufs[WAVES][S * CHUNK];
   const int per_tile = (N + NB - 1) / NB, tile = blockIdx.x / per_tile;      // (neighbouring blocks: see the kernel above)
   const int tiles = meta[0], e = tile_expert[tile], row0 = tile_row0[tile];
   if (tile >= tiles) return;
@@ -195,15 +196,15 @@ moe_few_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, const 
   static_assert(MATS * 1024 <= S * CHUNK * 2, "the parts meet in the ring's place");
   __syncthreads();
 #pragma unroll
-  for (int t = 0; t < MATS; ++t) red[(t * MF_WAVES + wave) * 64 + lane] = acc[t];
+  for (int t = 0; t < MATS; ++t) red[(t * WAVES + wave) * 64 + lane] = acc[t];
   __syncthreads();
   if (part) return;
   ms_f32x4 sum[MATS];
 #pragma unroll
   for (int t = 0; t < MATS; ++t) {
-    sum[t] = red[(t * MF_WAVES + wave) * 64 + lane];
+    sum[t] = red[(t * WAVES + wave) * 64 + lane];
 #pragma unroll
-    for (int p = 1; p < WK; ++p) sum[t] += red[(t * MF_WAVES + wave + p) * 64 + lane];
+    for (int p = 1; p < WK; ++p) sum[t] += red[(t * WAVES + wave + p) * 64 + lane];
   }
   const int n = n0 + lq * 4;      // a lane holds outputs n .. n + 3 of row li; N is a multiple of 4
   if (li >= rows || n >= N) return;
@@ -220,12 +221,12 @@ moe_few_kernel(void* __restrict__ out, const bf16_t* __restrict__ a_rows, const 
   }
 }
 
-template <int MODE, int WK, int CW, typename... Args>
+template <int MODE, int WAVES, int KB, int WK, int CW, typename... Args>
 static int launch_moe_few(int max_tiles, int N, hipStream_t stream, Args... args) {
-  const int nb = 16 * MF_WAVES / WK;
+  const int nb = 16 * WAVES / WK;
   const long long blocks = (long long)max_tiles * ((N + nb - 1) / nb);
   if (blocks > 0x7fffffffll) return (int)hipErrorInvalidValue;
-  hipLaunchKernelGGL((moe_few_kernel<MODE, WK, CW>), dim3((unsigned)blocks), dim3(64 * MF_WAVES), 0, stream, args...);
+  hipLaunchKernelGGL((moe_few_kernel<MODE, WAVES, KB, WK, CW>), dim3((unsigned)blocks), dim3(64 * WAVES), 0, stream, args...);
   return JV_LAUNCH_CHECK();
 }
 
@@ -234,18 +235,20 @@ static int launch_moe_skinny(void* out, const void* a, const void* W0, const voi
                              const int* tile_expert, const int* tile_row0, const int* order, const float* weights,
                              int max_tiles, int top, int n_tokens, int K, int N, JvAct act, int use_weight, void* stream) {
   if (K < 8 || K % 8) return (int)hipErrorInvalidValue;
-  if (K % MF_K == 0 && K <= 8 * MF_WAVES * MF_K && N % 4 == 0 && (((uintptr_t)out | (uintptr_t)a | (uintptr_t)W0 | (uintptr_t)W1) & 15) == 0) {
-    auto go = [&](auto wk, auto cw) {
-      return launch_moe_few<MODE, decltype(wk)::value, decltype(cw)::value>(
+  if (K % MF_K == 0 && K <= 4096 && N % 4 == 0 && (((uintptr_t)out | (uintptr_t)a | (uintptr_t)W0 | (uintptr_t)W1) & 15) == 0) {
+    auto go = [&](auto waves, auto kb, auto wk, auto cw) {
+      return launch_moe_few<MODE, decltype(waves)::value, decltype(kb)::value, decltype(wk)::value, decltype(cw)::value>(
           max_tiles, N, (hipStream_t)stream, out, (const bf16_t*)a, (const bf16_t*)W0, (const bf16_t*)W1, meta, offsets, tile_expert,
           tile_row0, order, weights, top, n_tokens, K, N, act, use_weight);
     };
-    using std::integral_constant;
-    if (K <= 512) return go(integral_constant<int, 2>{}, integral_constant<int, 4>{});
-    if (K <= 1024 && MODE == MS_GATED) return go(integral_constant<int, 4>{}, integral_constant<int, 4>{});
-    if (K <= 1024) return go(integral_constant<int, 2>{}, integral_constant<int, 8>{});
-    if (K <= 2048) return go(integral_constant<int, 8>{}, integral_constant<int, 4>{});
-    return go(integral_constant<int, 8>{}, integral_constant<int, 8>{});
+#define GO(WAVES, KB, WK, CW) \
+  go(std::integral_constant<int, WAVES>{}, std::integral_constant<int, KB>{}, std::integral_constant<int, WK>{}, std::integral_constant<int, CW>{})
+    if (K <= 512) return GO(4, 24, 2, 4);
+    if (K <= 1024 && MODE == MS_GATED) return GO(8, 64, 4, 4);
+    if (K <= 1024) return GO(4, 24, 2, 8);
+    if (K <= 2048) return GO(8, 32, 8, 4);
+    return GO(8, 64, 8, 8);
+#undef GO
   }
   const int wk = K >= 2048 ? 4 : 2;
   auto kernel = wk == 4 ? moe_skinny_kernel<MODE, 4> : moe_skinny_kernel<MODE, 2>;
