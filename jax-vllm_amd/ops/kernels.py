@@ -1397,16 +1397,21 @@ def gemm_into_stream(h: torch.Tensor, x: torch.Tensor, w: torch.Tensor, weight=N
 
 def _stream_rows_plan(m: int, w: torch.Tensor, gate_pairs: bool, partial_ok: bool, partial_max_width):
     """How a product reads ``StreamRows``: the plan of blocks that stay, "thin", or None where neither takes them.  Every block reads the shares of
-    the rows' sums of squares, so many small blocks pay for them (24,576 x 4,096 with its activation at 8 rows 38.5 by them, 37.1 without a scale)."""
+    the rows' sums of squares, so many small blocks pay for them where W is large (24,576 x 4,096 with its activation at 8 rows 38.5 by them, 37.1 without a
+    scale).  Small blocks ("thin") also leave one sum instead of two or four.  Microseconds in graphs, cold weights, blocks that stay / small ones, at 1, 8
+    and 16 rows: 6,144 x 2,048 9.2 / 7.5, 9.7 / 8.0, 10.6 / 9.1; x 3,072 13.7 / 9.8, 14.9 / 10.8, 16.5 / 12.4; x 4,096 11.7 / 10.9, 12.1 / 11.8, but 13.3 / 14.2;
+    5,120 x 3,584 11.4 / 9.9, 12.1 / 11.2, 12.8 / 13.0; 8,192 x 4,096 14.7 / 14.1, 15.3 / 14.5, 16.4 / 15.1; 12,288 x 2,048 13.7 / 11.7, 14.2 / 12.2, 15.4 /
+    13.2; 16,384 x 2,048 with its activation 16.2 / 14.7, 16.2 / 14.5, 16.9 / 17.1; 10,240 x 4,096 16.8 / 17.4, 17.9 / 18.5, 19.7 / 20.6; 24,576 x 2,048 at 16
+    rows 23.1 / 25.4."""
     n, k = w.shape
     if (w.dtype != torch.bfloat16 or not 0 < m <= SKINNY_AUTO_ROWS or k % 64 or not 0 < k <= STREAM_PRODUCT_MAX_WIDTH or n % 4 or not w.is_contiguous()
             or w.data_ptr() % 16 or not (gate_pairs or partial_ok)):
         return None
-    if n > 4096:
+    if n > 16384 or (k > 2560 if n > 8192 else n > 4096 and n <= 6144 and k > 3072 and m > 8):
         plan = streaming_plan(m, n, k, gate_pairs, partial_ok, w.device, partial_max_width)
         if plan is not None and plan[0] != TILE64 and plan[0][0] == -2:
             return plan
-    return "thin" if n <= 8192 else None
+    return "thin" if n <= 16384 else None
 
 
 def linear_takes_stream_rows(n_rows: int, w: torch.Tensor, gate_pairs: bool = False, partial_ok: bool = False,
