@@ -1460,7 +1460,8 @@ def _linear_stream_rows(rows: "StreamRows", w: torch.Tensor, gate_pairs, partial
     shape, parts = plan
     if parts > 1:
         return gemm_skinny(rows.x, w, torch.float32, block_shape=shape, ksplit=parts, row_scale=rows)
-    return gemm_skinny(rows.x, w, torch.bfloat16 if gate_pairs else torch.float32, gate_pairs=gate_pairs, block_shape=shape, row_scale=rows)
+    y = gemm_skinny(rows.x, w, torch.bfloat16 if gate_pairs else torch.float32, gate_pairs=gate_pairs, block_shape=shape, row_scale=rows)
+    return y if gate_pairs else y.view(1, *y.shape)
 
 
 def thin_whole_pays(m: int, n: int, k: int) -> bool:

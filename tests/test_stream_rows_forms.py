@@ -14,3 +14,12 @@ def test_lines_between_the_forms(m, n, k, pairs, thin):
 
     assert (kernels._stream_rows_plan(m, randn(n, k, seed=1).bfloat16(), pairs, not pairs, None) == "thin") == thin
     product(m, n, k, pairs)
+
+
+@pytest.mark.gpu
+def test_a_whole_inner_size_by_blocks_that_stay_is_one_part():
+    """A reader of partial products gets [1, M, N], also where blocks that stay hold the whole inner size (a q/k/v product of 16,388 columns)."""
+    test_lines_between_the_forms(8, 16388, 512, False, False)
+    w = randn(16388, 512, seed=1).bfloat16()
+    rows = K().StreamRows(randn(8, 512, seed=2).bfloat16(), randn(8, 256, seed=3) ** 2, 512, 1e-6)
+    assert K().linear(rows, w, partial_ok=True, partial_max_width=None).shape == (1, 8, 16388)
