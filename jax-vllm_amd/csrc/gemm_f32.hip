@@ -273,40 +273,15 @@ gemm_f32_few_kernel(float* __restrict__ C, const float* __restrict__ A, const fl
 // row (32 lines an instruction): 9.0 for 8.4.  Microseconds in graphs with cold weights, 16 x 16 or 32 x 16 tiles / these (rows of W): 8 rows
 // against 2,048 x 2,048 9.7 / 8.4 (8), 2,048 x 3,072 12.5 / 9.7 (8), 512 x 8,192 25.5 / 17.5 (8), 3,072 x 2,048 9.9 / 9.2 (16), 1,024 x 1,024 6.3 /
 // 5.5 (8), 6,144 x 2,048 14.5 / 14.0 (24), 6,144 x 8,192 51 / 45 (24), 32,000 x 2,048 54.6 / 55.2 (16): wide ones stay with 32 x 16.
-//
-// PAIRS_STREAM: the product joins the residual stream in place (a block owns its columns of it) and the block leaves the new rows times the next norm's
-// weight and its share of every row's sum of squares; PAIRS_SCALED: the product that reads such rows multiplies its results by the norm's scale, a wave
-// a row of shares, asked for before everything else.  A norm between two products (4.4 us) is no launch then: 8 layers of width 2,048, 5 requests
-// decoding, 613 -> 570 us.
-enum { PAIRS_PLAIN = 0, PAIRS_SCALED = 1, PAIRS_STREAM = 2 };
-#define PAIRS_SHARES 256      // of a row's sum of squares: floats of a row of ssq
-struct PairsNorm {
-  const float* ssq;           // PAIRS_SCALED: result row m times rsqrt(sum_j ssq[m][j] inv_width + eps), j < shares
-  int shares;
-  float inv_width, eps;
-  const float* weight;        // PAIRS_STREAM, beside h in out's place: of the next norm, or null: the stream alone
-  float* rows;
-  float* left;
-};
-template <int G, int S, int C, bool ACT, int MODE>
+template <int G, int S, int C, bool ACT>
 __global__ void __launch_bounds__(512)
-gemm_f32_pairs_kernel(float* __restrict__ out, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K, JvAct act, PairsNorm norm) {
+gemm_f32_pairs_kernel(float* __restrict__ out, const float* __restrict__ A, const float* __restrict__ W, int M, int N, int K, JvAct act) {
   constexpr int L = 2 * (G + 1), BUF = L * 256;      // loads of a pair, each 8 rows of a step, 1 KB
   static_assert(G <= 4 && L * (S - 1) <= 63, "a wave adds what a block leaves; what s_waitcnt counts to");
   __shared__ __attribute__((aligned(1024))) float bufs[8 * S * BUF];
   __shared__ f32x4 met[2][8 * C][16 * G];
-  __shared__ float scales[MODE == PAIRS_SCALED ? 8 : 1];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = wave >> 2, turn = wave & 3;
   const int li = lane & 15, lq = lane >> 4, odd = li >> 3, n0 = blockIdx.x * 8 * G;
-  const int m = lane % 16 / 2, n = n0 + lane / 16 * 8 + lane % 2 * 4;      // at the end lane < 16 G of wave 0 holds C[m][n .. n + 3]
-  f32x4 early = {0.f, 0.f, 0.f, 0.f}, weight = early;      // what the end reads, asked for first
-  if constexpr (MODE == PAIRS_SCALED) early = *(const f32x4*)(norm.ssq + (long long)min(wave, M - 1) * PAIRS_SHARES + lane * 4);
-  if constexpr (MODE == PAIRS_STREAM)
-    if (wave == 0) {
-      const int at = min(n, N - 4);
-      early = *(const f32x4*)(out + (long long)min(m, M - 1) * N + at);
-      if (norm.weight) weight = *(const f32x4*)(norm.weight + at);
-    }
   const int total = (K + G32_STEP - 1) / G32_STEP, first = half ? (total + 1) / 2 : 0, steps = half ? total / 2 : (total + 1) / 2;
   const int longest = ((total + 1) / 2 + 7) / 8;      // pairs of the wave that has the most
   const int mine = ((steps + 1) / 2 - turn + 3) / 4;
@@ -388,39 +363,16 @@ gemm_f32_pairs_kernel(float* __restrict__ out, const float* __restrict__ A, cons
     asm volatile("" ::: "memory");
   }
   if (half && turn == 0 && lane < 16 * G) met[1][0][lane] = sum;
-  if constexpr (MODE == PAIRS_SCALED) {
-    float t = 0.f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) t += lane * 4 + e < norm.shares ? early[e] : 0.f;
-#pragma unroll
-    for (int d = 1; d < 64; d *= 2) t += __shfl_xor(t, d, 64);
-    if (lane == 0) scales[wave] = rsqrtf(t * norm.inv_width + norm.eps);
-  }
   __syncthreads();
   if (wave || lane >= 16 * G) return;
   sum += met[1][0][lane];
+  const int m = lane % 16 / 2, n = n0 + lane / 16 * 8 + lane % 2 * 4;      // a lane holds C[m][n .. n + 3]
   if (m >= M) return;
-  float r[4] = {0.f, 0.f, 0.f, 0.f};
+  float r[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e)
     if (n + e < N) r[e] = settle(sum[e], A + (long long)m * K, W + (long long)(n + e) * K, K);
-  if constexpr (MODE == PAIRS_SCALED) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) r[e] *= scales[m];
-  }
-  if constexpr (MODE == PAIRS_STREAM) {      // N is a multiple of 4: a lane's four are there or none
-    const f32x4 v = early + f32x4{r[0], r[1], r[2], r[3]};
-    float sq = n < N ? (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]) : 0.f;
-    sq += __shfl_xor(sq, 1, 64);      // (the lanes of a row come and go together)
-#pragma unroll
-    for (int g = 1; g < G; g *= 2) sq += __shfl_xor(sq, 16 * g, 64);
-    if (norm.weight && lane < 16 && !(lane & 1)) norm.left[(long long)m * PAIRS_SHARES + blockIdx.x] = sq;
-    if (n >= N) return;
-    *(f32x4*)(out + (long long)m * N + n) = v;
-    if (norm.weight) *(f32x4*)(norm.rows + (long long)m * N + n) = v * weight;
-  } else {
-    leave<ACT>(out, m, n, N, r, act);
-  }
+  leave<ACT>(out, m, n, N, r, act);
 }
 
 // ---------------------------------------------------------------------------- many rows
@@ -781,11 +733,10 @@ static int few_launch(float* C, const float* A, const float* W, int M, int N, in
   hipLaunchKernelGGL(kernel, dim3((N + TW - 1) / TW, (M + XR - 1) / XR), dim3(512), 0, s, C, A, W, M, N, K, act);
   return JV_LAUNCH_CHECK();
 }
-template <int G, int S, int C, int MODE = PAIRS_PLAIN>
-static int pairs_launch(float* out, const float* A, const float* W, int M, int N, int K, JvAct act, hipStream_t s, PairsNorm norm = {}) {
-  static_assert(MODE != PAIRS_STREAM || (G & (G - 1)) == 0, "the shares meet by halves");
-  const auto kernel = act.id && MODE != PAIRS_STREAM ? gemm_f32_pairs_kernel<G, S, C, MODE != PAIRS_STREAM, MODE> : gemm_f32_pairs_kernel<G, S, C, false, MODE>;
-  hipLaunchKernelGGL(kernel, dim3((N + 8 * G - 1) / (8 * G)), dim3(512), 0, s, out, A, W, M, N, K, act, norm);
+template <int G, int S, int C>
+static int pairs_launch(float* out, const float* A, const float* W, int M, int N, int K, JvAct act, hipStream_t s) {
+  const auto kernel = act.id ? gemm_f32_pairs_kernel<G, S, C, true> : gemm_f32_pairs_kernel<G, S, C, false>;
+  hipLaunchKernelGGL(kernel, dim3((N + 8 * G - 1) / (8 * G)), dim3(512), 0, s, out, A, W, M, N, K, act);
   return JV_LAUNCH_CHECK();
 }
 template <int TM, int TW>
@@ -875,35 +826,4 @@ extern "C" int jv_gemm_f32(float* C, const float* A, const float* W, const void*
     case 10: return tile_launch<64, 32>(C, X, A, W, M, N, K, KA, act, s);
   }
   return (int)hipErrorInvalidValue;
-}
-
-static bool pairs_sizes(const float* C, const float* A, const float* W, int M, int N, int K) {
-  return M <= 8 && K > 0 && K <= 1 << 24 && K % 4 == 0 && !(((uintptr_t)C | (uintptr_t)A | (uintptr_t)W) & 15);
-}
-// The product of up to 8 rows that jv_gemm_f32_stream left, their norm's scale applied; form 2 or 4; ssq: rows of 256 floats, `shares` of them.
-extern "C" int jv_gemm_f32_scaled(float* C, const float* A, const float* W, int M, int N, int K, int form, int gate_act, float act_limit, float act_slope,
-                                  const float* ssq, int shares, int width, float eps, void* stream) {
-  if (M <= 0 || N <= 0) return 0;
-  if (!pairs_sizes(C, A, W, M, N, K) || (gate_act && (!jv_act_known(gate_act) || N % 2)) || !ssq || ((uintptr_t)ssq & 15) || shares < 1 ||
-      shares > PAIRS_SHARES || width <= 0 || (form != 2 && form != 4))
-    return (int)hipErrorInvalidValue;
-  const JvAct act{gate_act, act_limit, act_slope};
-  const PairsNorm norm{ssq, shares, 1.f / (float)width, eps, nullptr, nullptr, nullptr};
-  const hipStream_t s = (hipStream_t)stream;
-  if (form == 4) return pairs_launch<3, 1, 2, PAIRS_SCALED>(C, A, W, M, N, K, act, s, norm);
-  return N <= 8 * 256 ? pairs_launch<1, 2, 8, PAIRS_SCALED>(C, A, W, M, N, K, act, s, norm) : pairs_launch<2, 1, 4, PAIRS_SCALED>(C, A, W, M, N, K, act, s, norm);
-}
-// Columns of a share of jv_gemm_f32_stream's sums of squares, the columns of a block.
-extern "C" int jv_gemm_f32_stream_share(int N) { return N <= 8 * 256 ? 8 : 16; }
-// h += A W^T in place for up to 8 rows and 4,096 columns; with a weight rows = h * weight and ssq[row * 256 + block] the blocks' shares of the rows' sums
-// of squares.
-extern "C" int jv_gemm_f32_stream(float* h, const float* A, const float* W, int M, int N, int K, const float* weight, float* rows, float* ssq, void* stream) {
-  if (M <= 0 || N <= 0) return 0;
-  if (!pairs_sizes(h, A, W, M, N, K) || N % 4 || N > 16 * PAIRS_SHARES ||
-      (weight && (!rows || !ssq || (((uintptr_t)weight | (uintptr_t)rows | (uintptr_t)ssq) & 15))))
-    return (int)hipErrorInvalidValue;
-  const PairsNorm norm{nullptr, 0, 0.f, 0.f, weight, rows, ssq};
-  const hipStream_t s = (hipStream_t)stream;
-  return N <= 8 * 256 ? pairs_launch<1, 2, 8, PAIRS_STREAM>(h, A, W, M, N, K, JvAct{}, s, norm)
-                      : pairs_launch<2, 1, 4, PAIRS_STREAM>(h, A, W, M, N, K, JvAct{}, s, norm);
 }

@@ -183,14 +183,10 @@ class UnscaledRows:
 
 
 class StreamRows(UnscaledRows):
-    """The same as ``gemm_into_stream`` leaves them, with a share of a row's sum of squares for every 16 columns (ssq [rows, 256]; float rows: the
-    columns of a block, and the last share may have fewer); the reader is asked with ``linear_takes_stream_rows``."""
+    """The same as ``gemm_into_stream`` leaves them, with a share of a row's sum of squares for every 16 columns (ssq [rows, 256]); the
+    reader is asked with ``linear_takes_stream_rows``."""
 
     share, max_shares = 16, 256
-
-    def __init__(self, x: torch.Tensor, ssq: torch.Tensor, width: int, eps: float, share: int = 16):
-        super().__init__(x, ssq, width, eps)
-        self.shares = -(-self.width // share)
 
 
 class PendingProduct:
@@ -849,7 +845,6 @@ _F32_TILES = ((5, 128, 128, 3.0, 30.7, 36.6), (6, 128, 96, 3.1, 22.3, 29.5), (7,
 # 65,536, k 512 to 12,288): on the average 2 % from the best (25 % at 1 x 12,288 x 8,192), 0.69 to 1.04 of the time of 16 x 16 and 32 x 16 tiles by the count for more rows.
 _F32_PAIRS = ((2, 8, 256, 2.3, 1.3, 1.7, 2.05, 4.0, 7.2), (2, 16, 512, 2.75, 0.6, 1.95, 5.0, 4.1, 5.05), (3, 32, 512, 0.8, 2.6, 4.15, 7.8, 3.6, 5.2),
               (4, 24, 256, 1.7, 1.75, 2.8, 4.2, 4.0, 5.1))
-F32_PAIRS_MAX_ROWS = 8
 _F32_FRAGMENTS = 8    # forms below take the terms of a in the order of the matrix unit's operands
 
 
@@ -1356,33 +1351,13 @@ def stream_product_possible(n_rows: int, w: torch.Tensor) -> bool:
             and w.is_contiguous() and w.data_ptr() % 16 == 0)
 
 
-def f32_stream_product_possible(n_rows: int, w: torch.Tensor) -> bool:
-    """Whether ``gemm_into_stream`` takes a product of so many float rows with w: up to 8 rows, where the 32-bit products are by blocks that own their
-    columns (``csrc/gemm_f32.hip``)."""
-    n, k = w.shape
-    return (w.dtype == torch.float32 and 0 < n_rows <= F32_PAIRS_MAX_ROWS and 0 < k <= 1 << 24 and k % 4 == 0 and n % 4 == 0 and n <= STREAM_PRODUCT_MAX_WIDTH
-            and w.is_contiguous() and w.data_ptr() % 16 == 0)
-
-
 def gemm_into_stream(h: torch.Tensor, x: torch.Tensor, w: torch.Tensor, weight=None, eps: float = 0.0) -> "StreamRows | None":
     """h += x @ w.T in the float residual stream, in one launch; with the next norm's ``weight`` returns the rows h * weight with the shares of
-    their sums of squares.  See ``csrc/gemm_thin.hip``, for float rows ``csrc/gemm_f32.hip``; ask ``stream_product_possible`` (``f32_stream_product_possible``)
-    first."""
+    their sums of squares.  See ``csrc/gemm_thin.hip``; ask ``stream_product_possible`` first."""
     _dev(h, x, w, weight)
     _f32(h, "h")
     m, k = x.shape
     n = w.shape[0]
-    if x.dtype == torch.float32:
-        _need(w.shape[1] == k and h.shape == (m, n) and f32_stream_product_possible(m, w) and not (x.data_ptr() | h.data_ptr()) & 15,
-              "up to 8 float rows against a matrix of up to 4,096 rows of whole pieces of 4 columns, on 16 bytes")
-        rows = ssq = None
-        if weight is not None:
-            _f32(weight, "weight", n)
-            _need(not weight.data_ptr() & 15, "the weight begins on 16 bytes")
-            rows, ssq = torch.empty_like(h), torch.empty((m, StreamRows.max_shares), dtype=torch.float32, device=h.device)
-        lib = library.core()
-        _check(lib.jv_gemm_f32_stream(_ptr(h), _ptr(x), _ptr(w), m, n, k, _ptr(weight), _ptr(rows), _ptr(ssq), _stream()), "gemm_into_stream")
-        return None if weight is None else StreamRows(rows, ssq, n, eps, lib.jv_gemm_f32_stream_share(n))
     _need(x.dtype == torch.bfloat16 and w.shape[1] == k and tuple(h.shape) == (m, n) and stream_product_possible(m, w) and x.data_ptr() % 16 == 0,
           "up to 16 bfloat16 rows against a matrix of up to 4,096 rows of whole chunks of 64 columns, on 16 bytes")
     rows = ssq = None
@@ -1417,41 +1392,10 @@ def _stream_rows_plan(m: int, w: torch.Tensor, gate_pairs: bool, partial_ok: boo
 def linear_takes_stream_rows(n_rows: int, w: torch.Tensor, gate_pairs: bool = False, partial_ok: bool = False,
                              partial_max_width: int | None = PARTIAL_SUM_MAX_WIDTH) -> bool:
     """Whether ``linear`` with these arguments multiplies ``StreamRows``."""
-    if w.dtype == torch.float32:
-        return _f32_stream_rows_form(n_rows, w, gate_pairs) is not None
     return _stream_rows_plan(n_rows, w, gate_pairs, partial_ok, partial_max_width) is not None
 
 
-def _f32_stream_rows_form(m: int, w: torch.Tensor, gate_pairs) -> "int | None":
-    """Form of the 32-bit product that reads ``StreamRows`` of float, or None where it is not by the blocks of up to 8 rows."""
-    n, k = w.shape
-    if (w.dtype != torch.float32 or not 0 < m <= F32_PAIRS_MAX_ROWS or not 0 < k <= STREAM_PRODUCT_MAX_WIDTH or k % 4 or n == 0 or (gate_pairs and n % 2)
-            or not w.is_contiguous() or w.data_ptr() % 16):
-        return None
-    form = f32_plan(m, n, k)
-    return form if form in (2, 4) else 2 if n <= STREAM_PRODUCT_MAX_WIDTH else None      # (small ones: a launch less is worth more than the form)
-
-
-def gemm_f32_scaled(rows: "StreamRows", w: torch.Tensor, gate_pairs: "str | tuple | None" = None) -> torch.Tensor:
-    """float32 [M, N] of float ``StreamRows`` against float w [N, K], their norm's scale applied, with ``gate_pairs`` then the activation [M, N / 2]."""
-    x, ssq = rows.x, rows.ssq
-    _dev(x, w, ssq)
-    _f32(x, "x")
-    _f32(ssq, "ssq")
-    m, k = x.shape
-    n = w.shape[0]
-    form = _f32_stream_rows_form(m, w, gate_pairs)
-    _need(form is not None and w.shape[1] == k, "no product of these sizes applies the rows' scale (ask linear_takes_stream_rows first)")
-    _need(ssq.shape == (m, rows.max_shares) and rows.width == k and 1 <= rows.shares <= rows.max_shares, "the scale does not belong to x")
-    y = torch.empty((m, n // 2 if gate_pairs else n), dtype=torch.float32, device=x.device)
-    _check(library.core().jv_gemm_f32_scaled(_ptr(y), _ptr(x), _ptr(w), m, n, k, form, *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), _ptr(ssq),
-                                             rows.shares, rows.width, c_float(rows.eps), _stream()), "gemm_f32_scaled")
-    return y
-
-
 def _linear_stream_rows(rows: "StreamRows", w: torch.Tensor, gate_pairs, partial_ok: bool, partial_max_width):
-    if rows.dtype == torch.float32:
-        return gemm_f32_scaled(rows, w, gate_pairs)
     plan = _stream_rows_plan(rows.shape[0], w, bool(gate_pairs), partial_ok, partial_max_width)
     _need(plan is not None, "no product applies these rows' scale (ask linear_takes_stream_rows first)")
     if plan == "thin":

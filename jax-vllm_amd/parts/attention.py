@@ -220,8 +220,8 @@ class GroupedQueryAttention:
         return K.linear_takes_unscaled_rows(n_rows, self.w_qkv, partial_ok=self._qkv_parts_ok(), partial_max_width=None)
 
     def takes_stream_rows(self, n_rows: int) -> bool:
-        """Whether the qkv product reads ``K.StreamRows`` (in bfloat16 its float result goes to a kernel that adds parts)."""
-        return (not self.wide and not self.filtered and self.b_qkv is None and (self.dtype == torch.float32 or self._qkv_parts_ok())
+        """Whether the qkv product reads ``K.StreamRows`` (its float result goes to a kernel that adds parts)."""
+        return (not self.wide and not self.filtered and self.b_qkv is None and self._qkv_parts_ok()
                 and K.linear_takes_stream_rows(n_rows, self.w_qkv, partial_ok=True, partial_max_width=None))
 
     def takes_terms(self, n_rows: int) -> "bool | None":
@@ -230,8 +230,7 @@ class GroupedQueryAttention:
 
     def leaves_product(self, n_rows: int) -> bool:
         """Whether ``forward`` takes ``leave_product`` for so many rows: the output product is then left to the block."""
-        return not self.wide and not self.filtered and self.b_o is None and (
-            K.stream_product_possible(n_rows, self.w_o) or K.f32_stream_product_possible(n_rows, self.w_o))
+        return not self.wide and not self.filtered and self.b_o is None and K.stream_product_possible(n_rows, self.w_o)
 
     def takes_pending_rows(self, n_rows: int, ctx: StepContext, mem: LayerMemory) -> bool:
         """Whether the qkv product may make its rows itself (``K.PendingRows``): only the launch behind it that goes from the product to the
