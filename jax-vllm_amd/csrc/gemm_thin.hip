@@ -8,7 +8,9 @@
 // while every unit has one block at most and beyond 1,024 blocks, 2 between, where more blocks at once count for more (microseconds at 8 rows by 4 / 2
 // slots, before: 4,096 x 4,096 8.0 / 8.4, 9.4; 2,048 x 2,048 4.6 / 4.9, 5.1; 6,144 x 2,048 with its activation 8.0 / 7.2, 8.2; 8,192 x 2,048
 // 8.4 / 8.0, 9.6; 12,288 x 4,096 19.2 / 19.4, 22.7; 8 waves 4,096 x 4,096 8.8, two waves of 8 slots 9.0).  Every wave makes two sums, of an eighth of
-// the inner size each, and the eighths are added in ascending order: the bits of gemm_few.hip, whatever the other rows and the slots.
+// the inner size each, and the eighths are added in ascending order: the bits of gemm_few.hip, whatever the other rows, the slots and the tiles.
+// A chunk of more than 8 rows of x is as large as one of 16 rows of W, so a block then takes 32 of them where that leaves no unit more (16 rows, one tile / two:
+// 6,144 x 4,096 13.4 / 11.7, 8,192 x 2,048 9.5 / 8.6, 24,576 x 4,096 41.4 / 36.5).
 //
 // THIN_STREAM: the product joins the residual stream h in place (a block owns its columns of it), and the block leaves the new rows times the next
 // norm's weight in bf16 and its share of every row's sum of squares; the scale is left to the product that reads them (SCALED: its epilogue, up to
@@ -39,32 +41,33 @@ struct ThinStream {        // THIN_STREAM, beside h in y's place
   float* ssq;
 };
 
-// XL: instructions (of 8 rows) that bring a chunk of x; S: slots of the ring.
-template <int MODE, bool SCALED, int XL, int S>
+// XL: instructions (of 8 rows) that bring a chunk of x; S: slots of the ring; NT: tiles of 16 rows of W a block takes (THIN_STREAM: one).
+template <int MODE, bool SCALED, int XL, int S, int NT>
 __global__ void __launch_bounds__(64 * THIN_WAVES)
 gemm_thin_kernel(void* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, int M, int N, int K, long long ldx, JvAct act,
                  ThinScale scale, ThinStream stream) {
-  constexpr int L = 2 + XL, CHUNK = L * 8 * THIN_K, PER = 16 / THIN_WAVES;
+  constexpr int WL = 2 * NT, L = WL + XL, CHUNK = L * 8 * THIN_K, PER = 16 / THIN_WAVES;
+  static_assert(MODE != THIN_STREAM || NT == 1, "a share of a row is 16 columns");
   __shared__ __attribute__((aligned(1024))) bf16_t bufs[THIN_WAVES][S * CHUNK];
   __shared__ float sq_part[THIN_WAVES][16];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, lq = lane >> 4;
-  const int n0 = blockIdx.x * 16, all = K / THIN_K;
+  const int n0 = blockIdx.x * (16 * NT), all = K / THIN_K;
   const int first = all * wave / THIN_WAVES, chunks = all * (wave + 1) / THIN_WAVES - first, last = max(chunks - 1, 0);
   // an instruction brings 8 rows, lane l row l / 8, and fills 1 KB in the order of the lanes; piece c of row r lies at slot c ^ (r % 8) of
   // its row.  Rows beyond the last repeat it, chunks beyond a wave's last too (into slots that nobody reads).
   const int piece = first * THIN_K + ((lane & 7) ^ (lane >> 3)) * 8;
   const bf16_t* src[L];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) src[j] = W + (long long)min(n0 + j * 8 + (lane >> 3), N - 1) * K + piece;
+  for (int j = 0; j < WL; ++j) src[j] = W + (long long)min(n0 + j * 8 + (lane >> 3), N - 1) * K + piece;
 #pragma unroll
-  for (int j = 0; j < XL; ++j) src[2 + j] = x + (long long)min(j * 8 + (lane >> 3), M - 1) * ldx + piece;
+  for (int j = 0; j < XL; ++j) src[WL + j] = x + (long long)min(j * 8 + (lane >> 3), M - 1) * ldx + piece;
   const unsigned lds0 = (unsigned)(unsigned long long)(const __attribute__((address_space(3))) void*)bufs[wave];
   auto fetch = [&](int c, int slot) {
 #pragma unroll
     for (int j = 0; j < L; ++j)
       asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src[j] + c * THIN_K), "s"(lds0 + slot * (CHUNK * 2) + j * 1024) : "memory", "m0");
   };
-  const int m = li, n = n0 + lq * 4;      // a lane holds y[m][n .. n + 3]; N is a multiple of 4
+  const int m = li, n = n0 + (NT > 1 ? wave * 16 : 0) + lq * 4;      // at the end a lane of wave t < NT holds y[m][n .. n + 3]; N is a multiple of 4
   const int mc = min(m, M - 1), nc = min(n, N - 4);
   // what the epilogue reads is asked for first, so that it costs no round trip of its own at the end
   f32x4 hv = {0.f, 0.f, 0.f, 0.f}, wv = {0.f, 0.f, 0.f, 0.f}, rq[SCALED ? PER : 1];
@@ -80,34 +83,38 @@ gemm_thin_kernel(void* __restrict__ y, const bf16_t* __restrict__ x, const bf16_
 #pragma unroll
   for (int c = 0; c < S; ++c) fetch(min(c, last), c);
   const int second = all * (2 * wave + 1) / (2 * THIN_WAVES) - first;      // the chunk with which the wave's second eighth begins
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acc0 = acc;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 acc[NT], acc0[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = acc0[t] = zero;
+  auto next_eighth = [&]() {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc0[t] = acc[t], acc[t] = zero;
+  };
   for (int c0 = 0; c0 < chunks; c0 += S) {
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       if (c0 + s >= chunks) break;
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * L) : "memory");      // the oldest chunk is there, S - 1 are on their way
       const bf16_t* b = bufs[wave] + s * CHUNK;
-      bf16x8 wf[2], xf[2];
+      bf16x8 wf[NT][2], xf[2];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int at = (((h * 4 + lq) ^ li) & 7) * 8;
-        wf[h] = *(const bf16x8*)(b + li * THIN_K + at);
-        xf[h] = *(const bf16x8*)(b + (16 + (XL == 1 ? li & 7 : li)) * THIN_K + at);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) wf[t][h] = *(const bf16x8*)(b + (t * 16 + li) * THIN_K + at);
+        xf[h] = *(const bf16x8*)(b + (16 * NT + (XL == 1 ? li & 7 : li)) * THIN_K + at);
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // read before the slot is filled again
       fetch(min(c0 + s + S, last), s);
-      if (c0 + s == second) {
-        acc0 = acc;
-        acc = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
+      if (c0 + s == second) next_eighth();
 #pragma unroll
-      for (int h = 0; h < 2; ++h) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h], xf[h], acc, 0, 0, 0);
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[t][h], xf[h], acc[t], 0, 0, 0);
     }
   }
-  if (second >= chunks) {
-    acc0 = acc;
-    acc = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+  if (second >= chunks) next_eighth();
   if constexpr (SCALED) {
     float t = 0.f;
 #pragma unroll
@@ -119,13 +126,16 @@ gemm_thin_kernel(void* __restrict__ y, const bf16_t* __restrict__ x, const bf16_
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // nothing of the ring is still being filled where the sums meet
   __syncthreads();
   f32x4* red = (f32x4*)bufs;
-  red[2 * wave * 64 + lane] = acc0;
-  red[(2 * wave + 1) * 64 + lane] = acc;
-  __syncthreads();
-  if (wave) return;
-  f32x4 sum = red[lane];
 #pragma unroll
-  for (int p = 1; p < 2 * THIN_WAVES; ++p) sum += red[p * 64 + lane];
+  for (int t = 0; t < NT; ++t) {
+    red[(2 * wave * NT + t) * 64 + lane] = acc0[t];
+    red[((2 * wave + 1) * NT + t) * 64 + lane] = acc[t];
+  }
+  __syncthreads();
+  if (wave >= NT) return;
+  f32x4 sum = red[wave * 64 + lane];
+#pragma unroll
+  for (int p = 1; p < 2 * THIN_WAVES; ++p) sum += red[(p * NT + wave) * 64 + lane];
   if constexpr (SCALED) {
     float t = 0.f;
 #pragma unroll
@@ -164,11 +174,11 @@ gemm_thin_kernel(void* __restrict__ y, const bf16_t* __restrict__ x, const bf16_
   }
 }
 
-template <int MODE, bool SCALED>
+template <int MODE, bool SCALED, int NT = 1>
 static int thin_launch(void* y, const void* x, const void* W, int M, int N, int K, long long ldx, int slots, JvAct act, ThinScale scale, ThinStream stream,
                        hipStream_t st) {
 #define THIN(XL, S)                                                                                                                      \
-  hipLaunchKernelGGL((gemm_thin_kernel<MODE, SCALED, XL, S>), dim3((N + 15) / 16), dim3(64 * THIN_WAVES), 0, st, y, (const bf16_t*)x, \
+  hipLaunchKernelGGL((gemm_thin_kernel<MODE, SCALED, XL, S, NT>), dim3((N + 16 * NT - 1) / (16 * NT)), dim3(64 * THIN_WAVES), 0, st, y, (const bf16_t*)x, \
                      (const bf16_t*)W, M, N, K, ldx, act, scale, stream)
   if (slots == 4) {
     if (M <= 8) THIN(1, 4); else THIN(2, 4);
@@ -182,21 +192,24 @@ static int thin_launch(void* y, const void* x, const void* W, int M, int N, int 
 static bool thin_sizes(const void* y, const void* x, const void* W, int M, int N, int K, long long ldx) {
   return M <= 16 && K >= THIN_K && K % THIN_K == 0 && N % 4 == 0 && ldx >= K && ldx % 8 == 0 && !(((uintptr_t)x | (uintptr_t)W | (uintptr_t)y) & 15);
 }
-// mode: THIN_BF16, THIN_F32 or THIN_PAIRS; slots (2, 4) of a wave's ring; ssq (rows of 256 floats, shares of them, a multiple of 4) or null.
+// mode: THIN_BF16, THIN_F32 or THIN_PAIRS; slots (2, 4) of a wave's ring; tiles (1, 2) of 16 rows of W of a block; ssq (rows of 256 floats, shares of them, a multiple of 4) or null.
 extern "C" int jv_gemm_thin_bf16(void* y, const void* x, const void* W, int M, int N, int K, long long ldx, int mode, int gate_act, float act_limit,
-                                 float act_slope, int slots, const float* ssq, int shares, int width, float eps, void* stream) {
+                                 float act_slope, int slots, int tiles, const float* ssq, int shares, int width, float eps, void* stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (!thin_sizes(y, x, W, M, N, K, ldx) || mode < THIN_BF16 || mode > THIN_PAIRS || (mode == THIN_PAIRS && !jv_act_known(gate_act)) ||
+  if (!thin_sizes(y, x, W, M, N, K, ldx) || mode < THIN_BF16 || mode > THIN_PAIRS || (mode == THIN_PAIRS && !jv_act_known(gate_act)) || tiles < 1 || tiles > 2 ||
       (ssq && (shares < 4 || shares > THIN_SHARES || shares % 4 || width <= 0 || ((uintptr_t)ssq & 15))))
     return (int)hipErrorInvalidValue;
   const JvAct act{gate_act, act_limit, act_slope};
   const ThinScale scale{ssq, shares, 1.f / (float)width, eps};
   const hipStream_t st = (hipStream_t)stream;
 #define THIN(MODE)                                                                                                      \
+  if (tiles == 2)                                                                                                       \
+    return ssq ? thin_launch<MODE, true, 2>(y, x, W, M, N, K, ldx, slots, act, scale, ThinStream{}, st)                 \
+               : thin_launch<MODE, false, 2>(y, x, W, M, N, K, ldx, slots, act, scale, ThinStream{}, st);               \
   return ssq ? thin_launch<MODE, true>(y, x, W, M, N, K, ldx, slots, act, scale, ThinStream{}, st)                      \
              : thin_launch<MODE, false>(y, x, W, M, N, K, ldx, slots, act, scale, ThinStream{}, st)
-  if (mode == THIN_F32) THIN(THIN_F32);
-  if (mode == THIN_PAIRS) THIN(THIN_PAIRS);
+  if (mode == THIN_F32) { THIN(THIN_F32); }
+  if (mode == THIN_PAIRS) { THIN(THIN_PAIRS); }
   THIN(THIN_BF16);
 #undef THIN
 }

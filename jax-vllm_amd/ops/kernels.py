@@ -1312,16 +1312,30 @@ def few_tile(m: int, n: int, k: int, cus: int = 256) -> "int | None":
     return 32 if cus < tiles <= 1.5 * cus or (m > 8 and tiles > 3 * cus and k >= 1536) else 16
 
 
+def thin_tiles(m: int, n: int, cus: int = 256) -> int:
+    """Tiles of 16 rows of W that a block of ``csrc/gemm_thin.hip`` takes: two for 9 to 16 rows, whose chunks of x are as large as those of a tile of W,
+    where that leaves no unit more tiles than one each would.  Microseconds at 16 rows, one tile / two: 6,144 x 2,048 8.3 / 7.5, x 4,096 13.4 / 11.7, 8,192 x 2,048
+    9.5 / 8.6, 16,384 x 2,048 15.4 / 14.4, 24,576 x 4,096 41.4 / 36.5; but 11,296 x 2,048 12.3 / 12.8, 12,288 x 4,096 20.9 / 22.3, 4,096 x 2,048 6.2 / 7.7 (more
+    tiles for some unit), and up to 8 rows 8,192 x 2,048 8.6 / 8.9, 6,144 x 4,096 12.2 / 12.0."""
+    return 2 if m > 8 and 2 * -(-(-(-n // 32)) // cus) <= -(-(-(-n // 16)) // cus) else 1
+
+
 def thin_slots(m: int, n: int, k: int) -> "int | None":
     """Slots of the rings of ``csrc/gemm_thin.hip`` where it takes a product of up to 16 rows (any inner size that is a multiple of 64), or None
-    where blocks of eight waves with x in registers (``csrc/gemm_few.hip``) are better: rows of W that give most units one block of 16 and some two, at
-    9 rows or more (us there / here at 16 rows: 5,120 x 1,024 5.1 / 5.5, 5,120 x 3,072 10.4 / 11.4, 6,144 x 3,072 11.2 / 11.7; at 8 rows 4.75 / 4.6, 9.4 / 9.1, 10.2 /
-    9.6), and many of them against short inner sizes (12,288 x 512 at 8 rows 4.7 / 5.0, x 1,024 6.8 / 7.2).  Elsewhere, 54 sizes of 512 to 8,192 rows of W
-    and 512 to 4,096 columns at 1, 4, 8 and 16 rows: 0.82 to 1.01 of the time there."""
-    if 4096 < n <= 6144 and m > 8 and k > 512 or n > 8192 and k <= 1024:
+    where blocks of eight waves with x in registers (``csrc/gemm_few.hip``) are better: short inner sizes of 9 rows or more against rows of W that give most
+    units one block of 16 and some two (us there / here at 9 rows 5,120 x 1,024 4.9 / 5.1), and of many rows of W (12,288 x 512 at 8 rows
+    4.7 / 5.0, x 1,024 6.8 / 7.2).  Elsewhere, 54 sizes of 512 to 8,192 rows of W and 512 to 4,096 columns at 1, 4, 8 and 16 rows: 0.82 to 1.01 of the
+    time there."""
+    if 4096 < n <= 6144 and m > 8 and 512 < k <= 1024 or n > 8192 and k <= 1024:
         return None
-    return 4 if n <= 4096 and k > 512 or n > 16384 else 2
+    return 4 if thin_tiles(m, n) == 1 and (n <= 4096 and k > 512 or n > 16384) else 2
 
+
+def thin_tiles_pay(m: int, n: int, k: int) -> bool:
+    """Whether two tiles a block are better than blocks that stay or have x in registers: 9 to 16 rows, inner sizes beyond 1,024, and of very many rows of W
+    from 4,096 on.  Microseconds at 9 / 16 rows, there and here: 24,576 x 4,096 with its activation 36.5, 34.8 / 38.3, 35.8, 16,384 x 4,096 26.8, 25.3 / 27.7, 24.4,
+    6,144 x 4,096 13.5, 12.2 / 14.2, 11.5, 32,000 x 2,048 27.4, 27.0 / 28.1, 27.1, 151,936 x 4,096 213, 207 / 225, 221, but x 2,048 115, 112 / 121, 123."""
+    return thin_tiles(m, n) == 2 and k > 1024 and (n <= 65536 or k >= 4096)
 
 
 def gemm_thin_scaled(rows: "StreamRows", w: torch.Tensor, gate_pairs: "str | tuple | None" = None) -> torch.Tensor:
@@ -1336,7 +1350,7 @@ def gemm_thin_scaled(rows: "StreamRows", w: torch.Tensor, gate_pairs: "str | tup
     y = torch.empty((m, n // 2 if gate_pairs else n), dtype=torch.bfloat16 if gate_pairs else torch.float32, device=x.device)
     _check(library.core().jv_gemm_thin_bf16(
         _ptr(y), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), c_longlong(k), c_int(FEW_MODES["pairs" if gate_pairs else "float"]),
-        *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), c_int(thin_slots(1, n, k) or 2), _ptr(ssq), c_int(rows.shares), c_int(rows.width),
+        *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), c_int(thin_slots(m, n, k) or 2), c_int(thin_tiles(m, n)), _ptr(ssq), c_int(rows.shares), c_int(rows.width),
         c_float(rows.eps), _stream()), "gemm_thin")
     return y
 
@@ -1374,15 +1388,17 @@ def _stream_rows_plan(m: int, w: torch.Tensor, gate_pairs: bool, partial_ok: boo
     """How a product reads ``StreamRows``: the plan of blocks that stay, "thin", or None where neither takes them.  Every block reads the shares of
     the rows' sums of squares, so many small blocks pay for them where W is large (24,576 x 4,096 with its activation at 8 rows 38.5 by them, 37.1 without a
     scale).  Small blocks ("thin") also leave one sum instead of two or four.  Microseconds in graphs, cold weights, blocks that stay / small ones, at 1, 8
-    and 16 rows: 6,144 x 2,048 9.2 / 7.5, 9.7 / 8.0, 10.6 / 9.1; x 3,072 13.7 / 9.8, 14.9 / 10.8, 16.5 / 12.4; x 4,096 11.7 / 10.9, 12.1 / 11.8, but 13.3 / 14.2;
-    5,120 x 3,584 11.4 / 9.9, 12.1 / 11.2, 12.8 / 13.0; 8,192 x 4,096 14.7 / 14.1, 15.3 / 14.5, 16.4 / 15.1; 12,288 x 2,048 13.7 / 11.7, 14.2 / 12.2, 15.4 /
+    and 16 rows: 6,144 x 2,048 9.2 / 7.5, 9.7 / 8.0, 10.6 / 9.1; x 3,072 13.7 / 9.8, 14.9 / 10.8, 16.5 / 12.4; x 4,096 11.7 / 10.9, 12.1 / 11.8, 13.3 / 12.0;
+    8,192 x 4,096 14.7 / 14.1, 15.3 / 14.5, 16.4 / 15.1; 12,288 x 2,048 13.7 / 11.7, 14.2 / 12.2, 15.4 /
     13.2; 16,384 x 2,048 with its activation 16.2 / 14.7, 16.2 / 14.5, 16.9 / 17.1; 10,240 x 4,096 16.8 / 17.4, 17.9 / 18.5, 19.7 / 20.6; 24,576 x 2,048 at 16
     rows 23.1 / 25.4."""
     n, k = w.shape
     if (w.dtype != torch.bfloat16 or not 0 < m <= SKINNY_AUTO_ROWS or k % 64 or not 0 < k <= STREAM_PRODUCT_MAX_WIDTH or n % 4 or not w.is_contiguous()
             or w.data_ptr() % 16 or not (gate_pairs or partial_ok)):
         return None
-    if n > 16384 or (k > 2560 if n > 8192 else n > 4096 and n <= 6144 and k > 3072 and m > 8):
+    if thin_tiles_pay(m, n, k):
+        return "thin"
+    if n > 16384 or n > 8192 and k > 2560:
         plan = streaming_plan(m, n, k, gate_pairs, partial_ok, w.device, partial_max_width)
         if plan is not None and plan[0] != TILE64 and plan[0][0] == -2:
             return plan
@@ -1430,7 +1446,7 @@ def gemm_few(x: torch.Tensor, w: torch.Tensor, tile: int, gate_pairs: "str | tup
     if slots is not None:
         _check(library.core().jv_gemm_thin_bf16(
             _ptr(y), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), c_longlong(k), c_int(FEW_MODES[mode]),
-            *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), c_int(slots), *_NO_SCALE, _stream()), "gemm_few")
+            *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), c_int(slots), c_int(thin_tiles(m, n)), *_NO_SCALE, _stream()), "gemm_few")
         return y
     _check(library.core().jv_gemm_few_bf16(
         _ptr(y), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), c_longlong(k), c_int(FEW_MODES[mode]),
@@ -1558,9 +1574,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
                 return gemm_few(x, w, tile, gate_pairs, out_dtype or torch.bfloat16)
         _need(scale is None or (plan is not None and plan[0][0] == -2),
               "un-normalised rows need a product by the blocks that stay (ask linear_takes_unscaled_rows first)")
-        if (plan is not None and plan[1] > 1 and scale is None and thin_whole_pays(m, n, k) and x.is_contiguous() and w.is_contiguous()
-                and not (x.data_ptr() | w.data_ptr()) & 15):
-            return gemm_few(x, w, 16, out_dtype=torch.float32).view(1, m, n)
+        if (plan is not None and plan != STAGED and scale is None and m <= SKINNY_AUTO_ROWS and not (k % 64 or n % 4) and k <= FEW_MAX_INNER and w.dtype == torch.bfloat16
+                and (plan[1] > 1 and thin_whole_pays(m, n, k) or thin_tiles_pay(m, n, k)) and out_dtype in (None, torch.bfloat16, torch.float32)
+                and not (gate_pairs and out_dtype == torch.float32) and x.is_contiguous() and w.is_contiguous() and not (x.data_ptr() | w.data_ptr()) & 15):
+            if plan[1] > 1:
+                return gemm_few(x, w, 16, out_dtype=torch.float32).view(1, m, n)
+            return gemm_few(x, w, 16, gate_pairs, out_dtype or torch.bfloat16)
         if plan is not None:
             shape, parts = plan
             if shape == TILE64:

@@ -7,7 +7,7 @@ from .test_thin_products import test_rows_with_many_shares_of_their_scale as pro
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k,pairs,thin", [
-    (8, 6144, 3136, False, True), (9, 6144, 3072, False, True), (9, 6144, 3136, False, False), (9, 6148, 3136, False, True), (16, 8192, 4096, False, True),
+    (8, 6144, 3136, False, True), (9, 6144, 3072, False, True), (9, 6144, 3136, False, True), (9, 16388, 2624, False, False), (9, 24576, 2624, False, True), (16, 8192, 4096, False, True),
     (1, 8196, 2560, False, True), (8, 8200, 2624, False, False), (16, 16384, 64, True, True), (3, 12288, 2624, True, True)])
 def test_lines_between_the_forms(m, n, k, pairs, thin):
     from jax_vllm_amd.ops import kernels

@@ -1,0 +1,42 @@
+"""Products of 9 to 16 rows by blocks of two tiles of W: the bits of one tile a block, and the sizes where the rule changes sides."""
+import pytest
+import torch
+
+from .test_kernels_gpu import K, randn
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [9, 16])
+@pytest.mark.parametrize("n,k", [(4100, 1088), (6144, 4096), (8192, 64), (16388, 1152)])
+@pytest.mark.parametrize("form", ["bf16", "float", "pairs"])
+def test_the_bits_of_one_tile_a_block(monkeypatch, m, n, k, form):
+    x, w = randn(m, k, seed=m).bfloat16(), randn(n, k, seed=n).bfloat16()
+    args = dict(gate_pairs="silu") if form == "pairs" else dict(out_dtype=torch.float32 if form == "float" else torch.bfloat16)
+    monkeypatch.setattr(K(), "thin_slots", lambda *_: 2)
+    monkeypatch.setattr(K(), "thin_tiles", lambda *_: 2)
+    y = K().gemm_few(x, w, 16, **args)
+    monkeypatch.setattr(K(), "thin_tiles", lambda *_: 1)
+    assert torch.equal(y, K().gemm_few(x, w, 16, **args))
+    rows = K().StreamRows(x, torch.rand(m, 256, device="cuda") + 0.1, k, 1e-6)
+    one = K().gemm_thin_scaled(rows, w, args.get("gate_pairs"))
+    monkeypatch.setattr(K(), "thin_tiles", lambda *_: 2)
+    assert torch.equal(one, K().gemm_thin_scaled(rows, w, args.get("gate_pairs")))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,partial", [(9, 6144, 4096, True), (16, 6146, 2048, True), (12, 24576, 2048, False), (16, 32000, 1088, False), (9, 12288, 2048, False)])
+def test_linear_around_the_rule(m, n, k, partial):
+    x, w = randn(m, k, seed=3).bfloat16(), randn(n, k, seed=4).bfloat16()
+    y = K().linear(x, w, partial_ok=partial, partial_max_width=None)
+    y = y.sum(0) if y.dim() == 3 else y
+    z = x.double() @ w.double().T
+    # a sum of k products in float in any order, and a rounding of bfloat16
+    assert ((y.double() - z).abs() <= 2.0 ** -24 * k * (x.double().abs() @ w.double().abs().T) + 2.0 ** -8 * z.abs()).all()
+
+
+def test_where_two_tiles_are_taken():
+    from jax_vllm_amd.ops import kernels
+
+    assert [kernels.thin_tiles(16, n) for n in (4096, 4100, 8192, 8196, 12288, 12292, 16384, 16388, 24576)] == [1, 2, 2, 1, 1, 2, 2, 1, 2]
+    assert kernels.thin_tiles(8, 8192) == 1 and kernels.thin_tiles_pay(9, 8192, 2048) and not kernels.thin_tiles_pay(9, 8192, 1024)
+    assert not kernels.thin_tiles_pay(9, 151936, 2048) and kernels.thin_tiles_pay(9, 151936, 4096)
