@@ -217,8 +217,8 @@ def add_parts_unscaled(h: torch.Tensor, parts: torch.Tensor, weight: torch.Tenso
     _need(parts.dtype == torch.float32 and parts.dim() == 3 and parts.shape[1:] == h.shape and 1 <= parts.shape[0] <= 4,
           "partial products must be float32 [parts <= 4, *h.shape]")
     _need(unscaled_rows_possible(torch.bfloat16, n, hidden), "at most 128 rows of a width that is a multiple of 512, at most 8192")
-    xg = torch.empty((n, hidden), dtype=torch.bfloat16, device=h.device)
-    ssq = torch.empty((n, UNSCALED_MAX_SHARES), dtype=torch.float32, device=h.device)    # hidden / 512 of a row's 16 are written
+    xg = h.new_empty((n, hidden), dtype=torch.bfloat16)
+    ssq = h.new_empty((n, UNSCALED_MAX_SHARES))    # hidden / 512 of a row's 16 are written
     _check(_entry("jv_add_parts_unscaled_bf16", "ppilpppiip")(
         h.data_ptr(), parts.data_ptr(), parts.shape[0], parts.stride(0), weight.data_ptr(), xg.data_ptr(), ssq.data_ptr(), n, hidden, _stream()),
         "add_parts_unscaled")
@@ -1282,7 +1282,7 @@ def gemm_stream(x: torch.Tensor, w: torch.Tensor, form, mode: str = "rows", gate
         _need(row_scale.x is x and ssq.is_cuda and ssq.dtype == torch.float32 and ssq.is_contiguous() and ssq.shape == (m, UNSCALED_MAX_SHARES)
               and 1 <= row_scale.shares <= UNSCALED_MAX_SHARES, "row_scale does not belong to x")
     shape = (parts, m, n) if mode == "parts" else (m, n // 2) if gate_pairs else (m, n)
-    y = torch.empty(shape, dtype=torch.float32 if as_float else torch.bfloat16, device=x.device)
+    y = x.new_empty(shape, dtype=torch.float32) if as_float else x.new_empty(shape)
     _check(_entry("jv_gemm_stream_bf16", "pppiiiliiffiiipiifp")(
         y.data_ptr(), x.data_ptr(), w.data_ptr(), m, n, k, k, STREAM_MODES["parts" if as_float else mode],
         *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), tm, tw, parts,

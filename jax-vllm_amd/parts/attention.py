@@ -282,10 +282,10 @@ class GroupedQueryAttention:
                 isinstance(x, K.PendingRows) or attention_backend.token_pays(self, ctx)):
             heads = attention_backend.run_token(self, qkv, cos_sin, rotary_dim, ctx, mem, whole=leave_product)
             return K.PendingProduct(heads, self.w_o) if leave_product else self._project(heads)
-        out = torch.empty((n, self.nq * self.d), dtype=x.dtype, device=x.device)
         parts = None
         if qkv.dim() == 3:
-            parts, qkv = qkv, torch.empty(qkv.shape[1:], dtype=x.dtype, device=x.device)
+            parts, qkv = qkv, qkv.new_empty(qkv.shape[1:], dtype=x.dtype)
+        out = qkv.new_empty((n, self.nq * self.d))
         writes = mem.writes
         K.qk_norm_rope_write(
             qkv, ctx.slot_mappings[mem.group] if writes else None, self.q_norm, self.k_norm,
