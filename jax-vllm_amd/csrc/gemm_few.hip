@@ -9,12 +9,9 @@
 // what they share is the memory.  TW follows from where more are a further round (few_tile, with the figures).  The parts are added
 // in ascending order, so a row's result does not depend on the others.
 //
-// Microseconds in a graph, cold weights, at 1, 8 and 16 rows (before, x staged chunk by chunk in LDS for all waves of a block):
-// 6,144 x 2,048 with its activation 8.7, 9.1, 9.0 (9.8, 11.2, 11.8), 11,296 x 2,048 12.0, 12.5, 14.0 (17.3, 15.3, 17.3),
-// 2,048 x 2,048 4.0, 4.7, 5.4 (5.5, 6.2, 7.1), 1,536 x 768 2.9, 3.2, 3.4 (4.6, 5.0, 6.2), 3,072 x 4,096 7.9, 8.6, 10.1 (9.4, 10.4, 13.2).
-// Blocks that stay are better from about 16,384 rows of W on (24,576 x 2,048 at 16 rows 22.5, here 26.3); one and two rows against the
-// output embedding, which those do not take, run here in many rounds (151,936 x 2,048 104 us, x resident in LDS 154; 151,936 x 4,096 at two
-// rows 205.4, resident 205.0, staying 208).
+// Microseconds in a graph, cold weights, at 1, 8 and 16 rows (before, x staged chunk by chunk in LDS for all waves of a block): 1,536 x 768 2.9, 3.2, 3.4 (4.6,
+// 5.0, 6.2), 2,048 x 2,048 4.0, 4.7, 5.4 (5.5, 6.2, 7.1).  Given rows of longer inner sizes, and most of shorter ones, go through gemm_thin.hip, to the same bits
+// (thin_slots has the figures of both); given rows are taken up to 2,048 columns here, rows that the blocks make up to 4,096.
 #include "common.h"
 #include "row_source.h"
 
@@ -164,7 +161,7 @@ static int few_launch(void* y, const void* x, const void* W, int M, int N, int K
                        (const bf16_t*)W, M, N, K, ldx, act, RowSource{});                                                                           \
     return JV_LAUNCH_CHECK();                                                                                                          \
   }
-  FEW(2) FEW(4) FEW(8)
+  FEW(2) FEW(4)
 #undef FEW
   return (int)hipErrorInvalidValue;
 }

@@ -1291,7 +1291,7 @@ def gemm_stream(x: torch.Tensor, w: torch.Tensor, form, mode: str = "rows", gate
 
 
 FEW_MODES = {"rows": 0, "float": 1, "pairs": 2}
-FEW_MAX_INNER = 4096      # eight waves of eight chunks of 64 columns, x in registers
+FEW_MAX_INNER = 4096      # columns up to which ``few_tile`` was measured
 
 
 def few_tile(m: int, n: int, k: int, cus: int = 256) -> "int | None":
