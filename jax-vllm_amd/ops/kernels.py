@@ -53,8 +53,9 @@ _KINDS = {"p": c_void_p, "i": c_int, "l": c_longlong, "f": c_float}
 
 @functools.lru_cache(maxsize=None)
 def _entry(name: str, kinds: str, head_dim: "int | None" = None):
-    """Entry point ``name`` of the core library, or of a head size's attention library, with its arguments' types: it takes plain numbers and addresses, where
-    an object of ctypes for each argument would cost a third of a short prompt's wrappers (294 launches of 37 tokens through 36 layers)."""
+    """Entry point ``name`` of the core library, or of a head size's attention library, with its arguments' types: it takes plain numbers and addresses
+    instead of an object of ctypes for each (294 launches of 37 tokens through 36 layers wait for the host: 4,029 us with those, 3,970 with this and checks that build no
+    message, 3,930 with results that are allocated from a tensor at hand)."""
     fn = getattr(library.core() if head_dim is None else _attention_library(head_dim), name)
     fn.argtypes = [_KINDS[kind] for kind in kinds]
     return fn
