@@ -120,8 +120,10 @@ __device__ __forceinline__ void load8<float>(const float* p, float (&v)[8]) {
 // piece beyond the row reads the row's last piece again and only its stores and its share of the sum are
 // left out (a load inside a branch makes the compiler wait for all loads in flight where the branch
 // ends: 1.1 us of a 4.4 us kernel).  A short row's time is the sum of its dependent memory round trips.
-__device__ __forceinline__ float add_squares(float ss, float4 v) {      // spelled out: kernels that stand for one another round alike
-  return ss + fmaf(v.w, v.w, fmaf(v.z, v.z, fmaf(v.y, v.y, v.x * v.x)));
+// Spelled out, in the order that the compiler gives the plain sum of four squares: kernels that stand for one another round alike, and a row has the
+// bits it has always had.
+__device__ __forceinline__ float add_squares(float ss, float4 v) {
+  return ss + fmaf(v.w, v.w, fmaf(v.z, v.z, fmaf(v.x, v.x, v.y * v.y)));
 }
 template <typename T, int V>
 __global__ void __launch_bounds__(256)
