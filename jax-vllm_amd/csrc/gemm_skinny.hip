@@ -340,11 +340,12 @@ static int dispatch_nks(int nks, void* y, const void* x, const void* W, int M, i
 // Rows of x that come un-normalised from add_parts_unscaled_kernel: output row m is multiplied by
 // rsqrt(sum_j ssq[m][j] / width + eps), j < shares, ssq rows of 16 floats (the norm's scale commutes with the
 // product; with the inner size shared out every partial product is scaled).  ssq == nullptr: no scale.  Rows that gemm_thin.hip left have up to 256
-// shares, in rows of as many floats: every wave adds an eighth of them.
+// shares, in rows of as many floats: every wave adds an eighth of them, in a form of its own (MANY), for the second load and the scale
+// that it keeps cost every other product 3 to 13 % (16,384 x 5,120 at one row 29.7 us, with them 33.9; 10,240 x 2,048 11.2, 12.0).
 struct RowScale {
   const float* ssq;
   int shares;       // at most 16, or with rows of 256 floats 256, a multiple of 4
-  int stride;       // floats of a row of ssq: 16 or 256
+  int stride;       // floats of a row of ssq: 16, or 256 (MANY)
   float inv_width, eps;
   JvAct act;        // PAIRS: the gate's activation
 };
@@ -362,11 +363,12 @@ struct RowScale {
 //
 // SRC (row_source.h): the block makes its columns of x itself, MR (1 or 2) rows of them; ROWS_RESIDUAL with PAIRS has the whole inner size in
 // the block and also scales them, else it leaves the rows' sums of squares (MT 1, no EDGE, no SLOTS).
-template <int NL, int MT, typename OutT, bool PAIRS, bool EDGE, int SLOTS = 0, int SRC = ROWS_GIVEN, int MR = 1>
+template <int NL, int MT, typename OutT, bool PAIRS, bool EDGE, int SLOTS = 0, int SRC = ROWS_GIVEN, int MR = 1, bool MANY = false>
 __global__ void __launch_bounds__(512)
 gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t* __restrict__ W,
                               int M, int N, int K, long long ldx, long long ldy, RowScale rs, RowSource src) {
   static_assert(SRC == ROWS_GIVEN || (MT == 1 && !EDGE && SLOTS == 0), "");
+  static_assert(!MANY || (MT == 1 && SLOTS == 0 && SRC == ROWS_GIVEN), "");
   constexpr int KB = NL * 256, XSTRIDE = KB + SK_PAD;
   __shared__ __attribute__((aligned(16))) bf16_t xmade[SRC == ROWS_GIVEN ? 8 : MR * XSTRIDE];
   __shared__ float made_sq[MR * 8];
@@ -403,17 +405,19 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
   // without a scale the loads read x (no load inside a branch) and get no weight
   // (one 16-byte load a lane: the 4 lanes of a row hold its 16 shares; every block reads these few lines,
   // so every instruction more would queue up at one place in the L2)
-  f32x4 row_sq[2];
-  __shared__ float sq_part[8][16];
-  const bool many = rs.stride > 16;
-  if constexpr (SRC == ROWS_GIVEN) {
-    const int m = min((wk < MT ? wk : 0) * 16 + li, M - 1), at = many ? wk * 32 + lc * 8 : lc * 4;
-    const float* sp = rs.ssq ? rs.ssq + (long long)m * rs.stride : (const float*)x;
+  f32x4 row_sq[MANY ? 2 : 1];
+  __shared__ float sq_part[MANY ? 8 : 1][16];
+  [[maybe_unused]] bool first_tile = true;
+  [[maybe_unused]] float many_inv = 1.f;
+  if constexpr (MANY) {
+    const float* sp = rs.ssq + (long long)min(li, M - 1) * rs.stride;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) row_sq[i] = *(const f32x4*)(sp + (!rs.ssq ? 0 : many ? min(at + i * 4, rs.shares - 4) : at));
+    for (int i = 0; i < 2; ++i) row_sq[i] = *(const f32x4*)(sp + min(wk * 32 + lc * 8 + i * 4, rs.shares - 4));
+  } else if constexpr (SRC == ROWS_GIVEN) {
+    const int m = min((wk < MT ? wk : 0) * 16 + li, M - 1);
+    const float* sp = rs.ssq ? rs.ssq + (long long)m * 16 + lc * 4 : (const float*)x;
+    row_sq[0] = *(const f32x4*)sp;
   }
-  bool first_tile = true;
-  float inv = 1.f;
   // pieces first .. first + CNT - 1 of a tile
   auto load_pieces = [&](int tile, int first, auto& a) {
     constexpr int CNT = sizeof(a) / sizeof(a[0]);
@@ -439,13 +443,15 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
   auto reduce_store = [&](int tile, const f32x4 (&acc)[MT], int buf) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) *(f32x4*)(red[buf] + ((wk * MT + mt) * 256 + lane * 4)) = acc[mt];
-    if (MT == 1 && SRC == ROWS_GIVEN && many && first_tile) {
-      float sq = 0.f;
+    if constexpr (MANY) {
+      if (first_tile) {
+        float sq = 0.f;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) sq += wk * 32 + lc * 8 + i * 4 < rs.shares ? (row_sq[i][0] + row_sq[i][1]) + (row_sq[i][2] + row_sq[i][3]) : 0.f;
-      sq += __shfl_xor(sq, 16, 64);
-      sq += __shfl_xor(sq, 32, 64);
-      if (lc == 0) sq_part[wk][li] = sq;
+        for (int i = 0; i < 2; ++i) sq += wk * 32 + lc * 8 + i * 4 < rs.shares ? (row_sq[i][0] + row_sq[i][1]) + (row_sq[i][2] + row_sq[i][3]) : 0.f;
+        sq += __shfl_xor(sq, 16, 64);
+        sq += __shfl_xor(sq, 32, 64);
+        if (lc == 0) sq_part[wk][li] = sq;
+      }
     }
     __syncthreads();
     if (wk < MT) {                                 // wave mt adds row tile mt, in fixed order: wave 0, 1, ..., 7
@@ -458,20 +464,21 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
       }
       const int nb = tile * 16 + lc * 4;           // the accumulator holds y^T[n = lc*4+e][m = mt*16 + li]
       const int m = mt * 16 + li;
-      if (SRC == ROWS_GIVEN && rs.ssq) {           // a fixed order of adding: the same scale in every tile and block
+      if constexpr (MANY) {
         if (first_tile) {
           float sq = 0.f;
-          if (MT == 1 && many) {
 #pragma unroll
-            for (int w = 0; w < 8; ++w) sq += sq_part[w][li];
-          } else {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) sq += lc * 4 + j < rs.shares ? row_sq[0][j] : 0.f;
-            sq += __shfl_xor(sq, 16, 64);
-            sq += __shfl_xor(sq, 32, 64);
-          }
-          inv = rsqrtf(sq * rs.inv_width + rs.eps);
+          for (int w = 0; w < 8; ++w) sq += sq_part[w][li];
+          many_inv = rsqrtf(sq * rs.inv_width + rs.eps);
         }
+        s[0] *= many_inv; s[1] *= many_inv; s[2] *= many_inv; s[3] *= many_inv;
+      } else if (SRC == ROWS_GIVEN && rs.ssq) {    // a fixed order of adding: the same scale in every tile and block
+        float sq = 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sq += lc * 4 + j < rs.shares ? row_sq[0][j] : 0.f;
+        sq += __shfl_xor(sq, 16, 64);
+        sq += __shfl_xor(sq, 32, 64);
+        const float inv = rsqrtf(sq * rs.inv_width + rs.eps);
         s[0] *= inv; s[1] *= inv; s[2] *= inv; s[3] *= inv;
       }
       if (SRC == ROWS_RESIDUAL && PAIRS) {
@@ -493,7 +500,7 @@ gemm_skinny_persistent_kernel(OutT* __restrict__ y, const bf16_t* __restrict__ x
         }
       }
     }
-    first_tile = false;
+    if constexpr (MANY) first_tile = false;
   };
   // The next tile's weights are asked for before this tile is multiplied, without a condition (beyond the
   // last tile the last one is read again): after a conditional prefetch the compiler must assume that
@@ -577,12 +584,16 @@ static int launch_persistent(void* y, const void* x, const void* W, int M, int N
   const int n_tiles = (N + 15) / 16;
   blocks = (blocks + ksplit - 1) / ksplit;           // per group
   if (blocks > n_tiles) blocks = n_tiles;
-  if (K == ksplit * 8 * NL * 32)
-    hipLaunchKernelGGL((gemm_skinny_persistent_kernel<NL, MT, OutT, PAIRS, false, SLOTS>), dim3(blocks, ksplit), dim3(512), 0,
-                       stream, (OutT*)y, (const bf16_t*)x, (const bf16_t*)W, M, N, K, ldx, ldy, rs, RowSource{});
-  else
-    hipLaunchKernelGGL((gemm_skinny_persistent_kernel<NL, MT, OutT, PAIRS, true, SLOTS>), dim3(blocks, ksplit), dim3(512), 0,
-                       stream, (OutT*)y, (const bf16_t*)x, (const bf16_t*)W, M, N, K, ldx, ldy, rs, RowSource{});
+  const bool edge = K != ksplit * 8 * NL * 32;
+  auto* kernel = edge ? gemm_skinny_persistent_kernel<NL, MT, OutT, PAIRS, true, SLOTS> : gemm_skinny_persistent_kernel<NL, MT, OutT, PAIRS, false, SLOTS>;
+  if (rs.ssq && rs.stride > 16) {      // the activation's result or float rows of an inner size of up to 4,096
+    if constexpr (MT == 1 && NL <= 16 && (PAIRS || sizeof(OutT) == 4))
+      kernel = edge ? gemm_skinny_persistent_kernel<NL, MT, OutT, PAIRS, true, 0, ROWS_GIVEN, 1, true>
+                    : gemm_skinny_persistent_kernel<NL, MT, OutT, PAIRS, false, 0, ROWS_GIVEN, 1, true>;
+    else
+      return (int)hipErrorInvalidValue;
+  }
+  hipLaunchKernelGGL(kernel, dim3(blocks, ksplit), dim3(512), 0, stream, (OutT*)y, (const bf16_t*)x, (const bf16_t*)W, M, N, K, ldx, ldy, rs, RowSource{});
   return JV_LAUNCH_CHECK();
 }
 
