@@ -258,14 +258,84 @@ head_linear_mfma_kernel(bf16_t* __restrict__ y, long long ldy, int ys, const bf1
 
 // More rows than a block of those takes: a wave has 16 rows and 64 outputs at a time, so an operand of x serves four products, and the
 // results go through LDS into whole lines of y (2 bytes at a time the stores took longer than the rest).  The sums keep the order
-// of the kernel above.  What it costs is the way to its operands and back, so with an inner size of up to 32 KS a wave keeps its rows of W in registers
-// and walks several tiles of rows, the next tile's rows of x (and this one's gates) on their way meanwhile; a wave of one tile waited for
-// both once for two steps of products.  Microseconds in a recorded step (before, a tile a wave), 2,048 / 600 rows: 16 heads, 64 into 224 10.7 (16.7) / 5.3 (7.5), 224 into 64 with gates 8.6 (9.6) / 6.0 (=); 64 heads, 128 into 32 12.9 (18.9) / 5.9 (8.0); 8 heads, 128 into 512 14.1 (24.7) /
-// 6.8 (10.8): 1.6 to 2.4 TB/s of x and y.
-// From 480,000 results on it was faster than the kernel above at 16 sizes (2 to 64 heads, 32 to 512 outputs, inner sizes 32 to 512, 80 to 2,048 rows).
+// of the kernel above.  From 480,000 results on it was faster than that at 16 sizes (2 to 64 heads, 32 to 512 outputs, inner sizes 32 to 512, 80 to 2,048 rows).
 #define HL_N 64
+__global__ void __launch_bounds__(256)
+head_linear_lines_kernel(bf16_t* __restrict__ y, long long ldy, int ys, const bf16_t* __restrict__ x, long long ldx,
+                         int xs, const bf16_t* __restrict__ W, int M, int N, int K, const bf16_t* __restrict__ g,
+                         long long ldg, int gn, bool y_pieces, bool g_pieces) {
+  __shared__ __attribute__((aligned(16))) float lines[4][16][HL_N + 4];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lc = lane >> 4;
+  const int h = blockIdx.z, n0 = blockIdx.x * HL_N, m0 = (blockIdx.y * 4 + wave) * 16;
+  if (m0 >= M) return;      // (no barrier below: a wave's lines are its own)
+  const bf16_t* wr[HL_N / 16];
+#pragma unroll
+  for (int t = 0; t < HL_N / 16; ++t) wr[t] = W + ((long long)h * N + min(n0 + t * 16 + li, N - 1)) * K;
+  const bf16_t* xr = x + (long long)min(m0 + li, M - 1) * ldx + (long long)h * xs;
+  const hl_bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  hl_f32x4 acc[HL_N / 16] = {};
+  hl_bf16x8 b = *(const hl_bf16x8*)(xr + min(lc * 8, K - 8)), w[HL_N / 16];
+#pragma unroll
+  for (int t = 0; t < HL_N / 16; ++t) w[t] = *(const hl_bf16x8*)(wr[t] + min(lc * 8, K - 8));
+  for (int k0 = 0; k0 < K; k0 += 32) {
+    const int next = min(k0 + 32 + lc * 8, K - 8);      // asked for without a condition, also behind the last step
+    const hl_bf16x8 bn = *(const hl_bf16x8*)(xr + next);
+    hl_bf16x8 wn[HL_N / 16];
+#pragma unroll
+    for (int t = 0; t < HL_N / 16; ++t) wn[t] = *(const hl_bf16x8*)(wr[t] + next);
+    const hl_bf16x8 bk = k0 + lc * 8 < K ? b : zero;
+#pragma unroll
+    for (int t = 0; t < HL_N / 16; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t], bk, acc[t], 0, 0, 0);
+    b = bn;
+#pragma unroll
+    for (int t = 0; t < HL_N / 16; ++t) w[t] = wn[t];
+  }
+#pragma unroll
+  for (int t = 0; t < HL_N / 16; ++t) *(hl_f32x4*)&lines[wave][li][t * 16 + lc * 4] = acc[t];
+  const int c = (lane & 7) * 8, n = n0 + c;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = i * 8 + (lane >> 3), m = m0 + r;
+    if (m >= M || n >= N) continue;
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; e += 4) *(hl_f32x4*)(v + e) = *(const hl_f32x4*)&lines[wave][r][c + e];
+    if (g) {
+      const bf16_t* gr = g + (long long)m * ldg + (long long)h * gn;
+      hl_bf16x8 gv;
+      if (gn == 1) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) gv[e] = gr[0];
+      } else if (g_pieces && n + 8 <= N) {
+        gv = *(const hl_bf16x8*)(gr + n);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) gv[e] = gr[min(n + e, N - 1)];
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] *= 1.f / (1.f + expf(-(float)gv[e]));
+    }
+    bf16_t* out = y + (long long)m * ldy + (long long)h * ys + n;
+    if (y_pieces && n + 8 <= N) {
+      hl_bf16x8 o;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = (bf16_t)v[e];
+      *(hl_bf16x8*)out = o;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (n + e < N) out[e] = (bf16_t)v[e];
+    }
+  }
+}
+
+// The same with an inner size of up to 32 KS whose rows of W a wave keeps in registers: what a tile costs is the way to its operands and back, so a wave
+// walks several tiles of rows, the next tile's rows of x (and this one's gates) on their way meanwhile; a wave of one tile waits for
+// both once for two steps of products.  Microseconds in a recorded step (a tile a wave), 2,048 / 600 rows: 16 heads, 64 into 224 10.4 (16.4) / 5.1 (7.5),
+// with gates 16.5 (19.7) / 8.2 (9.7); 224 into 64 with gates 9.5 (10.3); 64 heads, 128 into 32 12.7 (19.2) / 5.8 (8.1); 8 heads, 128 into 512 13.9 (24.6) /
+// 6.7 (10.8).  Where the walk pays is the caller's to say, with the blocks along the rows: it does not where steps of 32 columns are filled up
+// with zeros, or where the end of a tile (gates, stores) is most of it and four waves a unit do not cover it.
 #define HL_T (HL_N / 16)
-#define HL_BLOCKS 256
 // A wave's results of a tile: from operand order through its lines in LDS, times the gates, into y.
 struct HlOut {
   bf16_t* y;
@@ -318,90 +388,57 @@ struct HlOut {
   }
 };
 
-// KS: steps of 32 columns whose rows of W stay in registers; 0: any inner size, rows of W read for every tile.
+// KS: steps of 32 columns whose rows of W stay in registers.
 template <int KS>
 __global__ void __launch_bounds__(256)
-head_linear_lines_kernel(HlOut o, const bf16_t* __restrict__ x, long long ldx, int xs, const bf16_t* __restrict__ W, int K) {
+head_linear_walk_kernel(HlOut o, const bf16_t* __restrict__ x, long long ldx, int xs, const bf16_t* __restrict__ W, int K) {
   __shared__ __attribute__((aligned(16))) float lines[4][16][HL_N + 4];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lc = lane >> 4;
   const int h = blockIdx.z, n0 = blockIdx.x * HL_N, tiles = (o.M + 15) / 16;
   int tile = blockIdx.y * 4 + wave;
   if (tile >= tiles) return;      // (no barrier below: a wave's lines are its own)
-  const bf16_t* wr[HL_T];
-#pragma unroll
-  for (int t = 0; t < HL_T; ++t) wr[t] = W + ((long long)h * o.N + min(n0 + t * 16 + li, o.N - 1)) * K;
   const hl_bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  auto row_of = [&](int tile) { return x + (long long)min(tile * 16 + li, o.M - 1) * ldx + (long long)h * xs; };
-  hl_bf16x8 gv[2];
-  auto ask_gates = [&](int tile) {
+  hl_bf16x8 w[KS][HL_T], b[KS], next[KS], gv[2];
+  auto ask = [&](int tile, hl_bf16x8 (&to)[KS]) {
+    const bf16_t* row = x + (long long)min(tile * 16 + li, o.M - 1) * ldx + (long long)h * xs;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) to[s] = *(const hl_bf16x8*)(row + min(s * 32 + lc * 8, K - 8));
+  };
+  ask(tile, b);
+#pragma unroll
+  for (int s = 0; s < KS; ++s)
+#pragma unroll
+    for (int t = 0; t < HL_T; ++t)
+      w[s][t] = *(const hl_bf16x8*)(W + ((long long)h * o.N + min(n0 + t * 16 + li, o.N - 1)) * K + min(s * 32 + lc * 8, K - 8));
+#pragma unroll
+  for (int s = 0; s < KS; ++s)
+#pragma unroll
+    for (int t = 0; t < HL_T; ++t) w[s][t] = s * 32 + lc * 8 < K ? w[s][t] : zero;
+  for (; tile < tiles; tile += gridDim.y * 4) {
     if (o.g) {
 #pragma unroll
       for (int i = 0; i < 2; ++i) gv[i] = o.gates(h, tile * 16 + i * 8 + (lane >> 3), n0 + (lane & 7) * 8);
     }
-  };
-  auto finish = [&](const hl_f32x4 (&acc)[HL_T], int tile) {
+    ask(min(tile + (int)gridDim.y * 4, tiles - 1), next);      // asked for without a condition
+    hl_f32x4 acc[HL_T] = {};
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const hl_bf16x8 bk = s * 32 + lc * 8 < K ? b[s] : zero;
+#pragma unroll
+      for (int t = 0; t < HL_T; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[s][t], bk, acc[t], 0, 0, 0);
+    }
 #pragma unroll
     for (int t = 0; t < HL_T; ++t) *(hl_f32x4*)&lines[wave][li][t * 16 + lc * 4] = acc[t];
     o.leave(lines[wave], h, tile * 16, n0, lane, gv);
-  };
-  if constexpr (KS > 0) {
-    hl_bf16x8 w[KS][HL_T], b[KS], next[KS];
-    auto ask = [&](const bf16_t* row, hl_bf16x8 (&to)[KS]) {
 #pragma unroll
-      for (int s = 0; s < KS; ++s) to[s] = *(const hl_bf16x8*)(row + min(s * 32 + lc * 8, K - 8));
-    };
-    ask(row_of(tile), b);
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-#pragma unroll
-      for (int t = 0; t < HL_T; ++t) {
-        w[s][t] = *(const hl_bf16x8*)(wr[t] + min(s * 32 + lc * 8, K - 8));
-      }
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-#pragma unroll
-      for (int t = 0; t < HL_T; ++t) w[s][t] = s * 32 + lc * 8 < K ? w[s][t] : zero;
-    for (; tile < tiles; tile += gridDim.y * 4) {
-      ask_gates(tile);
-      ask(row_of(min(tile + (int)gridDim.y * 4, tiles - 1)), next);      // asked for without a condition
-      hl_f32x4 acc[HL_T] = {};
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const hl_bf16x8 bk = s * 32 + lc * 8 < K ? b[s] : zero;
-#pragma unroll
-        for (int t = 0; t < HL_T; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[s][t], bk, acc[t], 0, 0, 0);
-      }
-      finish(acc, tile);
-#pragma unroll
-      for (int s = 0; s < KS; ++s) b[s] = next[s];
-    }
-  } else {
-    const bf16_t* xr = row_of(tile);
-    ask_gates(tile);
-    hl_f32x4 acc[HL_T] = {};
-    hl_bf16x8 b = *(const hl_bf16x8*)(xr + min(lc * 8, K - 8)), w[HL_T];
-#pragma unroll
-    for (int t = 0; t < HL_T; ++t) w[t] = *(const hl_bf16x8*)(wr[t] + min(lc * 8, K - 8));
-    for (int k0 = 0; k0 < K; k0 += 32) {
-      const int next = min(k0 + 32 + lc * 8, K - 8);      // asked for without a condition, also behind the last step
-      const hl_bf16x8 bn = *(const hl_bf16x8*)(xr + next);
-      hl_bf16x8 wn[HL_T];
-#pragma unroll
-      for (int t = 0; t < HL_T; ++t) wn[t] = *(const hl_bf16x8*)(wr[t] + next);
-      const hl_bf16x8 bk = k0 + lc * 8 < K ? b : zero;
-#pragma unroll
-      for (int t = 0; t < HL_T; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t], bk, acc[t], 0, 0, 0);
-      b = bn;
-#pragma unroll
-      for (int t = 0; t < HL_T; ++t) w[t] = wn[t];
-    }
-    finish(acc, tile);
+    for (int s = 0; s < KS; ++s) b[s] = next[s];
   }
 }
 
+// walk: blocks along the rows whose waves keep their rows of W (inner sizes up to 256; products of many rows), 0: a tile a wave.
 extern "C" int jv_head_linear_mfma_bf16(void* y, long long ldy, int ys, const void* x, long long ldx, int xs,
                                         const void* W, int M, int N, int K, int heads, const void* g, long long ldg,
-                                        int gn, void* stream) {
+                                        int gn, int walk, void* stream) {
   if (M <= 0 || N <= 0 || heads <= 0) return 0;
   if (g && gn != N && gn != 1) return (int)hipErrorInvalidValue;
   const unsigned gy = (M + 63) / 64;
@@ -409,18 +446,16 @@ extern "C" int jv_head_linear_mfma_bf16(void* y, long long ldy, int ys, const vo
   if (M >= 80 && (long long)M * N * heads >= 480000) {      // fewer rows or outputs: more, shorter waves end sooner
     const bool y_pieces = ldy % 8 == 0 && ys % 8 == 0 && (uintptr_t)y % 16 == 0;
     const bool g_pieces = g && ldg % 8 == 0 && gn % 8 == 0 && (uintptr_t)g % 16 == 0;
-    const HlOut o{(bf16_t*)y, ldy, ys, M, N, (const bf16_t*)g, ldg, gn, y_pieces, g_pieces};
     const unsigned gx = (N + HL_N - 1) / HL_N;
-    auto launch = [&](auto* kernel, unsigned rows) {      // rows: blocks along the rows
-      hipLaunchKernelGGL(kernel, dim3(gx, rows, heads), dim3(256), 0, (hipStream_t)stream, o, (const bf16_t*)x, ldx, xs, (const bf16_t*)W, K);
-    };
-    // As many tiles a wave as leave a block to a compute unit: half of them, or two blocks a unit, 0 to 20 % slower or up to 10 % faster (at
-    // 4,096 rows); four up to 40 % slower.  A wave of a single tile had better not wait for 28 pieces of W first (600 rows of 224 into 64: 6.4 us for 6.0).
-    const unsigned side = gx * heads, fit = (HL_BLOCKS + side - 1) / side, rows = gy < fit ? gy : fit;
-    if (K <= 64) launch(head_linear_lines_kernel<2>, rows);
-    else if (K <= 128) launch(head_linear_lines_kernel<4>, rows);
-    else if (K <= 256 && gy > fit) launch(head_linear_lines_kernel<8>, rows);
-    else launch(head_linear_lines_kernel<0>, gy);
+    if (walk < 0 || (unsigned)walk > gy || (walk && K > 256)) return (int)hipErrorInvalidValue;
+    if (walk) {
+      const HlOut o{(bf16_t*)y, ldy, ys, M, N, (const bf16_t*)g, ldg, gn, y_pieces, g_pieces};
+      auto* kernel = K <= 64 ? head_linear_walk_kernel<2> : K <= 128 ? head_linear_walk_kernel<4> : K <= 192 ? head_linear_walk_kernel<6> : head_linear_walk_kernel<8>;
+      hipLaunchKernelGGL(kernel, dim3(gx, walk, heads), dim3(256), 0, (hipStream_t)stream, o, (const bf16_t*)x, ldx, xs, (const bf16_t*)W, K);
+      return JV_LAUNCH_CHECK();
+    }
+    hipLaunchKernelGGL(head_linear_lines_kernel, dim3(gx, gy, heads), dim3(256), 0, (hipStream_t)stream, (bf16_t*)y,
+                       ldy, ys, (const bf16_t*)x, ldx, xs, (const bf16_t*)W, M, N, K, (const bf16_t*)g, ldg, gn, y_pieces, g_pieces);
     return JV_LAUNCH_CHECK();
   }
   hipLaunchKernelGGL(head_linear_mfma_kernel, dim3((N + 15) / 16, gy, heads), dim3(256), 0, (hipStream_t)stream,

@@ -32,3 +32,27 @@ def test_several_tiles_a_wave(n, heads, N, K, gate):
     assert bool(((y.cpu().double().view(n, heads, N) - want).abs() <= bound).all())
     for a in range(0, n, 79):                                      # up to 79 rows: the form of a tile a wave
         assert torch.equal(run(a, min(a + 79, n)), y[a:a + 79])
+
+
+def test_where_a_wave_walks_several_tiles():
+    from jax_vllm_amd.ops.kernels import head_walk
+
+    # a tile a wave: steps filled up with zeros, one step, an inner size that registers do not hold
+    assert [head_walk(4096, 64, K, 64, False) for K in (16, 32, 56, 72, 96, 160, 216, 264, 512)] == [0] * 9
+    assert all(head_walk(4096, 64, K, 64, False) == 4 for K in (64, 128, 192, 224, 232, 256))
+    # one block a unit, rounded down; twice as many with gates, unless these have less than one and a half tiles a wave
+    assert head_walk(600, 192, 256, 16, False) == 5 and head_walk(600, 192, 256, 16, True) == 5 and head_walk(1024, 192, 256, 16, True) == 10
+    assert head_walk(1216, 192, 256, 16, True, cus=304) == 12 and head_walk(2048, 64, 224, 16, True) == 16
+    assert [head_walk(n, 64, 128, 16, False) for n in (1472, 1473, 1536, 1537)] == [0, 16, 16, 16]
+    assert head_walk(80, 64, 64, 64, False) == 2 and head_walk(80, 64, 128, 64, False) == 0
+    assert head_walk(64 * 200, 40, 64, 400, True) == 1 and head_walk(0, 64, 64, 1, False) == 0 and head_walk(5, 64, 64, 0, False) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,heads,N,K", [(1100, 30, 72, 192), (1100, 30, 72, 232), (1600, 40, 40, 64), (2100, 16, 64, 224)])
+@pytest.mark.parametrize("gate", [None, "element", "head"])
+def test_walks_by_the_rule(n, heads, N, K, gate):
+    from jax_vllm_amd.ops.kernels import head_walk
+
+    assert 0 < head_walk(n, N, K, heads, gate is not None) < -(-n // 64)
+    test_several_tiles_a_wave(n, heads, N, K, gate)
