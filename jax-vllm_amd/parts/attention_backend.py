@@ -169,20 +169,35 @@ def few_rows_of_256(rows: int, keys: int, group_rows: int, compute_units: int, p
     return keys <= 256 or (few and keys < 2048)
 
 
-def halves_items(one_group: bool, groups: int, keys: int, window: int, compute_units: int):
+SHORT_WALK = 400             # keys up to which the halves kernel's start weighs as much as its tiles
+
+
+def halves_items(groups: int, pairs: int, keys: int, window: int, capped: bool, compute_units: int):
     """(Whether 16 rows a wave take them, groups per item) at head size 256 and pages of 16 keys, where two waves share 32 rows of the
-    other form.  Items of two neighbouring groups once they give half of the compute units a block or walk far (no slower then, and half the
-    reads), else of one group.  The 16 rows a wave remain for up to 256 keys without a sliding window, and with one while the items are few.  Microseconds, 16 rows a wave / items
-    of one group / of two, 16 heads over one: 64 tokens 10.1 / 10.7 / 13.9, 300 20.3 / 19.5 / 21.4, 512 28.6 / 26.3 / 27.3, 1,000 50.5 / 45.4 /
-    43.4, 2,048 with a window of 1,024 104 / 91 / 51, of 256 44 / 43 / 27, of 128 33 / 33 / 23; 512 after 4,000 193 / 154 / 155; blocks
-    of 256 keys, 1,400 tokens 23.1 / 24.8 / 22.1; of 128, 4,000 over 8 kv heads 48.5 / 50.8 / 51.7."""
-    pairs = 2 * groups > compute_units or keys >= 2048
-    if one_group and keys <= 256 and (window <= 0 or not pairs):
+    other form.  ``groups``, ``pairs``: items of one group and of two (neighbours of one request) that the prompts have over all kv heads; ``keys``: the most that a
+    query sees; ``capped``: scores go through a cap, which is paid once more for every wave that starts.
+
+    Walks of more than 400 keys: the halves, by pairs once groups alone give half of the compute units a block or the walk is far (no slower then, and half
+    the reads).  Shorter ones: the 16 rows a wave, whose start is short, while the groups are a round of blocks (a quarter of the units a second one), but items of one
+    group where 257 keys and more are scored without a cap and no unit has two; beyond a round the pairs, if the prompts have them (a request of one group has
+    none), where a sliding window or 257 keys bound the walk, and up to 64 keys, a tile, only if they save a round.  Microseconds, 16 rows a wave /
+    items of one group / of two: 16 heads over one, 64 tokens 10.1 / 10.7 / 13.9, 300 20.6 / 20.1 / 22.0, with a cap 22.3 / 22.8 / 24.7, 512 28.6 / 26.3 / 27.3, 1,000 50.5 /
+    45.4 / 43.4, with a window of 100 16.6 / - / 20.1, 2,048 with a window of 1,024 104 / 91 / 51, of 256 44 / 43 / 27, of 128 33 / 33 / 23; 512 after
+    4,000 193 / 154 / 155; 30 prompts of 40 tokens, 8 heads over one 10.5 / 11.9 / 15.4, 16 over 8 18.3 / 20.6 / 14.2, 60 of them, 16 over one 29.5 / 33.5 / 31.7.  1,610 steps
+    (five head layouts, 23 sets of prompts, seven windows, with and without a cap): 1.02 of the best form's time on average, and nowhere more than 1.03 of the 16
+    rows a wave."""
+    if keys > SHORT_WALK:
+        return False, 2 if 2 * groups > compute_units or keys >= 2048 else 1
+    if 4 * groups <= 5 * compute_units:
+        return keys <= 256 or capped or groups > compute_units, 1
+    if (keys <= 256 and window <= 0) or 4 * pairs > 3 * groups:
         return True, 1
-    return False, 2 if pairs else 1
+    if keys <= KEY_TILE and -(-pairs // compute_units) >= -(-4 * groups // (5 * compute_units)):
+        return True, 1
+    return False, 2
 
 
-def plan_mfma(ctx, nq: int, nkv: int, head_dim: int, window: int, device, keep: int = 0) -> MfmaPlan:
+def plan_mfma(ctx, nq: int, nkv: int, head_dim: int, window: int, device, keep: int = 0, capped: bool = False) -> MfmaPlan:
     g = nq // nkv
     group_rows, kernel_groups = K.attn_prefill_geometry(head_dim)
     rows = sum(ql * g for ql in ctx.q_lens_host if ql > 1)
@@ -192,11 +207,12 @@ def plan_mfma(ctx, nq: int, nkv: int, head_dim: int, window: int, device, keep: 
     one_group = False
     if head_dim == 256:
         keys = max([keys_seen(cl + ql, window, keep) for ql, cl in zip(ctx.q_lens_host, ctx.context_lens_host) if ql > 1], default=0)
-        one_group = few_rows_of_256(rows * nkv, keys, group_rows, cus, ctx.page_size)
         if ctx.page_size == 16:
-            one_group, groups_per_item, balance = *halves_items(one_group, -(-rows // group_rows) * nkv, keys, window, cus), False
-        elif one_group:
-            groups_per_item, balance = 1, False
+            groups = [-(-ql * g // group_rows) for ql in ctx.q_lens_host if ql > 1]
+            pairs = sum((n + 1) // 2 for n in groups) * nkv
+            one_group, groups_per_item, balance = *halves_items(sum(groups) * nkv, pairs, keys, window, capped, cus), False
+        elif few_rows_of_256(rows * nkv, keys, group_rows, cus, ctx.page_size):
+            one_group, groups_per_item, balance = True, 1, False
     prefill = prefill_work_items(ctx.q_lens_host, ctx.context_lens_host, g, window, group_rows, groups_per_item,
                                  balance=balance, keep=keep)
     # head size 256: items of two groups have a unit each, and items of one group were not helped (168 steps of 257 to 512 items, all
@@ -279,10 +295,11 @@ def token_pays(att, ctx) -> bool:
 
 
 def _mfma_plan(att, ctx, window: int, keep: int, device) -> MfmaPlan:
-    key = ("mfma_attention_plan", att.nq, att.nkv, att.d, window, keep)
+    capped = att.d == 256 and bool(getattr(att, "softcap", None))      # (nothing else of a plan depends on a cap)
+    key = ("mfma_attention_plan", att.nq, att.nkv, att.d, window, keep, capped)
     plan = ctx.plans.get(key)
     if plan is None:
-        plan = ctx.plans[key] = plan_mfma(ctx, att.nq, att.nkv, att.d, window, device, keep)
+        plan = ctx.plans[key] = plan_mfma(ctx, att.nq, att.nkv, att.d, window, device, keep, capped)
     return plan
 
 

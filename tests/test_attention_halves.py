@@ -11,12 +11,45 @@ from .test_kernels_gpu import K, _mfma_inputs, _mfma_reference, _prefill_work
 
 
 def test_the_rule():
-    assert halves_items(True, 16, 64, 0, 256) == (True, 1)              # few, short
-    assert halves_items(True, 350, 256, -256, 256) == (True, 1)         # blocks
-    assert halves_items(True, 350, 256, 256, 256) == (False, 2)         # a sliding window
-    assert halves_items(True, 128, 1000, 0, 256) == (False, 1)
-    assert halves_items(False, 129, 1000, 1024, 256) == (False, 2)
-    assert halves_items(False, 8, 2048, 0, 256) == (False, 2)           # far walks
+    assert halves_items(16, 8, 64, 0, False, 256) == (True, 1)              # few, short
+    assert halves_items(350, 175, 256, -256, False, 256) == (True, 1)       # blocks
+    assert halves_items(350, 175, 256, 256, False, 256) == (False, 2)       # a sliding window
+    assert halves_items(128, 64, 1000, 0, False, 256) == (False, 1)
+    assert halves_items(129, 65, 1000, 1024, False, 256) == (False, 2)
+    assert halves_items(8, 4, 2048, 0, False, 256) == (False, 2)            # far walks
+
+
+def test_short_walks_beside_a_round_of_blocks():
+    for window in (0, 64, 1024, -64):                                       # groups that are one round: their start alone counts
+        assert halves_items(320, 160, 256, window, False, 256) == (True, 1)
+    assert halves_items(321, 161, 256, 1024, False, 256) == (False, 2)
+    assert halves_items(480, 480, 40, 256, False, 256) == (True, 1)         # requests of one group have no pairs
+    assert halves_items(480, 360, 128, 256, False, 256) == (False, 2) and halves_items(480, 361, 128, 256, False, 256) == (True, 1)
+    assert halves_items(600, 300, 40, 1024, False, 256) == (True, 1) and halves_items(641, 321, 40, 1024, False, 256) == (False, 2)      # as many rounds; one saved
+    assert halves_items(80, 40, 257, 0, False, 256) == (False, 1) and halves_items(80, 40, 257, 0, True, 256) == (True, 1)      # a cap
+    assert halves_items(300, 150, 400, 0, False, 256) == (True, 1) and halves_items(300, 150, 401, 0, True, 256) == (False, 2)
+    assert halves_items(330, 165, 300, 0, True, 256) == (False, 2) and halves_items(330, 165, 300, 0, False, 304) == (True, 1)
+
+
+def test_a_plan_counts_its_items(monkeypatch):
+    """Groups and pairs request by request: 30 prompts of 40 tokens with a q head a kv head have no pair, 16 rows a wave take them."""
+    from types import SimpleNamespace
+
+    from jax_vllm_amd.ops import kernels
+    from jax_vllm_amd.parts import attention_backend
+
+    monkeypatch.setattr(kernels, "compute_units", lambda device: 256)
+    monkeypatch.setattr(attention_backend, "upload_i32", lambda values, device: torch.tensor(values, dtype=torch.int32))
+    asked, rule = [], halves_items
+    monkeypatch.setattr(attention_backend, "halves_items", lambda *a: asked.append(a) or rule(*a))
+
+    def plan(lens, nq, nkv, **kw):
+        ctx = SimpleNamespace(q_lens_host=lens, context_lens_host=[0] * len(lens), page_size=16, block_tables=[torch.zeros(len(lens), 64)])
+        return attention_backend.plan_mfma(ctx, nq, nkv, 256, kw.pop("window", 0), "cpu", **kw)
+
+    assert plan([40] * 30, 16, 16, window=1024).one_group and asked[-1] == (480, 480, 40, 1024, False, 256)
+    plan([1, 129, 1, 300], 16, 8, capped=True)
+    assert asked[-1] == (15 * 8, 8 * 8, 300, 0, True, 256)      # single tokens are no prompt's
 
 
 @pytest.mark.gpu
