@@ -1366,6 +1366,19 @@ def stream_product_possible(n_rows: int, w: torch.Tensor) -> bool:
             and w.is_contiguous() and w.data_ptr() % 16 == 0)
 
 
+def stream_product_pays(n_rows: int, n: int, k: int) -> bool:
+    """Whether a layer's last product had better join the stream, by a block for 16 rows of w over the whole inner size, than leave parts that a launch adds.  A few
+    blocks take long over a long inner size, which parts share out: up to 2,048 rows of w 8,192 columns, 14,336 for more than 1,024 of them and up to 8 rows of x;
+    more rows of w 20,480 columns, or any for more than 8 rows of x.  Microseconds at 1, 8 and 16 rows, there and here (with the launch that adds): 2,048 x 8,192 9.9,
+    11.1, 13.4 / 11.3, 11.8, 12.5; 1,536 x 8,960 9.8, 11.9, 14.2 / 10.9, 11.8, 12.5; 512 x 12,288 11.2, 13.8, 17.1 / 8.7, 9.8, 10.5; 1,024 x 10,240 10.9, 13.8, 16.7 / 9.4, 10.2,
+    10.7; 2,048 x 12,288 13.0, 15.6, 18.9 / 13.4, 14.2, 15.1; 4,096 x 32,768 63.0, 62.0, 63.3 / 60.9, 59.7, 71.3.  A refused product costs the layer's other one its 2 us too, so the line lies
+    where a layer gains nothing: in steps of whole layers at 16 rows, width 1,024 with 8,192 columns 43.7 us a layer both ways, 2,048 with 8,192 54.1 / 56.1; at one row 1,536
+    with 8,960 44.2 / 46.9, 2,560 with 24,576 98.3 / 96.4."""
+    if n > 2048:
+        return k <= 20480 or n_rows > 8
+    return k <= (14336 if n > 1024 and n_rows <= 8 else 8192)
+
+
 def gemm_into_stream(h: torch.Tensor, x: torch.Tensor, w: torch.Tensor, weight=None, eps: float = 0.0) -> "StreamRows | None":
     """h += x @ w.T in the float residual stream, in one launch; with the next norm's ``weight`` returns the rows h * weight with the shares of
     their sums of squares.  See ``csrc/gemm_thin.hip``; ask ``stream_product_possible`` first."""

@@ -230,7 +230,7 @@ class GroupedQueryAttention:
 
     def leaves_product(self, n_rows: int) -> bool:
         """Whether ``forward`` takes ``leave_product`` for so many rows: the output product is then left to the block."""
-        return not self.wide and not self.filtered and self.b_o is None and K.stream_product_possible(n_rows, self.w_o)
+        return not self.wide and not self.filtered and self.b_o is None and K.stream_product_possible(n_rows, self.w_o) and K.stream_product_pays(n_rows, *self.w_o.shape)
 
     def takes_pending_rows(self, n_rows: int, ctx: StepContext, mem: LayerMemory) -> bool:
         """Whether the qkv product may make its rows itself (``K.PendingRows``): only the launch behind it that goes from the product to the

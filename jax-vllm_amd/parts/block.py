@@ -19,8 +19,10 @@ from ..ops import kernels as K
 from .spec import BLOCK_STATE, PartSpec, StateSpec, TensorSpec, build_part, is_replayable, register_part
 
 
-# Up to this width one or two rows go from product to product as parts; wider ones, whose splits a launch merges in any case, through the stream: a
-# step of 36 layers at 4,096 with one row 3,294 us by parts, 3,264 through the stream.
+# Up to this width one or two rows go from product to product as parts; wider ones, whose splits a launch merges in any case, through the stream.  Microseconds a
+# layer by parts / through the stream, one row and two: 2,560 with 9,728 columns in the feed-forward 64.1 / 60.3, 64.1 / 61.3, 4,096 with 12,288 88.4 / 87.9, 90.4 / 88.5.  At
+# 2,048 it hangs on the feed-forward: 3,072 33.1 / 32.9, 35.5 / 33.3, 8,192 45.6 / 44.9, 47.7 / 45.5, but 12,288 54.0 / 56.6, 56.3 / 57.3.  (3,072 and 3,584, and
+# widths below 2,048 with these head counts, have no form by parts that both sublayers take.)
 MADE_WIDTH = 2048
 
 

@@ -55,7 +55,7 @@ class GatedMLP:
 
     def leaves_product(self, n_rows: int) -> bool:
         """Whether ``forward`` takes ``leave_product`` for so many rows: the last product is then left to the block."""
-        return self.partial_out and K.stream_product_possible(n_rows, self.w_down)
+        return self.partial_out and K.stream_product_possible(n_rows, self.w_down) and K.stream_product_pays(n_rows, *self.w_down.shape)
 
     def forward(self, x, ctx=None, leave_product: bool = False):
         terms = K.f32_terms_layout(x.shape[0], self.w_down) if x.dtype == torch.float32 else None

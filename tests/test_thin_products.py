@@ -74,6 +74,29 @@ def test_where_the_stream_takes_a_product():
     assert not kernels.stream_product_possible(1, w(64, 65)[:, 1:])      # off 16 bytes, and no whole rows
 
 
+def test_where_a_layer_leaves_its_products_to_the_stream():
+    from types import SimpleNamespace
+
+    from jax_vllm_amd.ops.kernels import stream_product_pays as pays
+    from jax_vllm_amd.parts.attention import GroupedQueryAttention
+    from jax_vllm_amd.parts.mlp import GatedMLP
+
+    assert pays(16, 2048, 8192) and not pays(16, 2048, 8256) and pays(8, 2048, 14336) and not pays(8, 2048, 14400) and not pays(9, 1536, 8960)
+    assert pays(1, 1024, 8192) and not pays(1, 1024, 8256) and not pays(16, 512, 12288)
+    assert pays(1, 4096, 20480) and not pays(8, 2112, 20544) and pays(9, 2112, 20544) and pays(16, 4096, 12288)
+
+    def w(n, k):
+        return torch.empty(n, k, dtype=torch.bfloat16, device="meta")
+
+    class Weight(torch.Tensor):      # (a meta tensor has no address)
+        data_ptr = lambda self: 0
+
+    for k, leaves in ((8192, True), (10240, False)):
+        weight = w(1024, k).as_subclass(Weight)
+        assert GatedMLP.leaves_product(SimpleNamespace(partial_out=True, w_down=weight), 4) == leaves
+        assert GroupedQueryAttention.leaves_product(SimpleNamespace(wide=False, filtered=False, b_o=None, w_o=weight), 4) == leaves
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("running,prompt", [(1, 0), (3, 0), (16, 0), (0, 12), (2, 9)])
 def test_layers_through_the_stream(monkeypatch, running, prompt):
