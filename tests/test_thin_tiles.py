@@ -40,3 +40,13 @@ def test_where_two_tiles_are_taken():
     assert [kernels.thin_tiles(16, n) for n in (4096, 4100, 8192, 8196, 12288, 12292, 16384, 16388, 24576)] == [1, 2, 2, 1, 1, 2, 2, 1, 2]
     assert kernels.thin_tiles(8, 8192) == 1 and kernels.thin_tiles_pay(9, 8192, 2048) and not kernels.thin_tiles_pay(9, 8192, 1024)
     assert not kernels.thin_tiles_pay(9, 151936, 2048) and kernels.thin_tiles_pay(9, 151936, 4096)
+
+
+def test_where_two_tiles_do_not_pay():
+    from jax_vllm_amd.ops.kernels import thin_tiles_pay as pays
+
+    assert [pays(16, 16384, k) for k in (1024, 1088, 2560, 3072, 4096)] == [False, True, True, True, True]
+    for n in (24576, 32000):      # 10 and 12 whole pieces a wave of the blocks that stay
+        assert [pays(9, n, k) for k in (1088, 2048, 2112, 2560, 3072, 3520, 3584, 4096)] == [True, True, False, False, False, False, True, True]
+    assert [pays(16, 49152, k) for k in (1088, 2048, 3072, 3584)] == [False, False, False, True]
+    assert [pays(16, 65536, k) for k in (2048, 3584)] == [False, True] and [pays(16, 151936, k) for k in (3584, 4096)] == [False, True]
