@@ -1333,16 +1333,18 @@ def thin_slots(m: int, n: int, k: int) -> "int | None":
 
 
 def thin_tiles_pay(m: int, n: int, k: int) -> bool:
-    """Whether two tiles a block are better than blocks that stay or have x in registers: 9 to 16 rows, inner sizes beyond 1,024, and from 16,385 rows of W on only
-    where blocks that stay have pieces of W to spare (1,088 to 2,048 columns up to 32,768 rows, and from 3,584 on); 10 and 12 whole pieces a wave are better.
-    Microseconds at 9 / 16 rows, there and here: 6,144 x 4,096 13.5, 12.2 / 14.2, 11.5, 24,576 x 4,096 with its activation 36.5, 34.8 / 38.3, 35.8, 16,384 x 4,096 26.8, 25.3 /
-    27.7, 24.4, x 3,072 1.01 of the time, 32,000 x 2,048 27.4, 27.0 / 28.1, 27.1; but 24,576 x 2,560 24.2, 25.2 / 25.3, 26.3, 32,000 x 2,560 31.0, 32.0 / 32.0, 34.4, x 3,072 36.3,
-    37.4 / 37.4, 39.9, 49,152 x 2,048 1.02 of the time, x 1,536 1.03, 151,936 x 2,048 115, 112 / 121, 123, x 4,096 213, 207 / 225, 221."""
+    """Whether two tiles a block are better than blocks that stay or have x in registers: 9 to 16 rows, inner sizes beyond 1,024, and from 16,385 rows of W on not
+    where blocks that stay, two to a unit, hold 7 to 10 or 12 whole pieces of 256 columns, nor beyond 32,768 with fewer than 14.  Microseconds at 9 / 16 rows, there and
+    here: 6,144 x 4,096 13.5, 12.2 / 14.2, 11.5, 24,576 x 4,096 with its activation 36.5, 34.8 / 38.3, 35.8, 16,384 x 4,096 26.8, 25.3 / 27.7, 24.4; but 24,576 x 2,560
+    24.2, 25.2 / 25.3, 26.3, 32,000 x 2,560 31.0, 32.0 / 32.0, 34.4, x 3,072 36.3, 37.4 / 37.4, 39.9, 151,936 x 2,048 115, 112 / 121, 123, x 4,096 213, 207 / 225, 221.  Time here
+    over there: 32,000 x 1,344 0.86, 1,856 1.07, 2,624 1.01, 3,008 1.00, 3,136 0.95, 49,152 x 2,048 1.02, x 1,536 1.03, x 3,584 1.00."""
     if thin_tiles(m, n) != 2 or k <= 1024:
         return False
     if n <= 16384:
         return True
-    return k >= (3584 if n <= 65536 else 4096) or (n <= 32768 and k <= 2048)
+    if n <= 32768:
+        return k <= 1536 or 2560 < k < 3072 or k > 3072
+    return k >= (3584 if n <= 65536 else 4096)
 
 
 def gemm_thin_scaled(rows: "StreamRows", w: torch.Tensor, gate_pairs: "str | tuple | None" = None) -> torch.Tensor:

@@ -46,7 +46,7 @@ def test_where_two_tiles_do_not_pay():
     from jax_vllm_amd.ops.kernels import thin_tiles_pay as pays
 
     assert [pays(16, 16384, k) for k in (1024, 1088, 2560, 3072, 4096)] == [False, True, True, True, True]
-    for n in (24576, 32000):      # 10 and 12 whole pieces a wave of the blocks that stay
-        assert [pays(9, n, k) for k in (1088, 2048, 2112, 2560, 3072, 3520, 3584, 4096)] == [True, True, False, False, False, False, True, True]
+    for n in (24576, 32000):      # 7 to 10 pieces a wave of the blocks that stay, and 12 whole ones
+        assert [pays(9, n, k) for k in (1088, 1536, 1600, 2048, 2560, 2624, 3008, 3072, 3136, 4096)] == [True, True, False, False, False, True, True, False, True, True]
     assert [pays(16, 49152, k) for k in (1088, 2048, 3072, 3584)] == [False, False, False, True]
     assert [pays(16, 65536, k) for k in (2048, 3584)] == [False, True] and [pays(16, 151936, k) for k in (3584, 4096)] == [False, True]
