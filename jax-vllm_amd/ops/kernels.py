@@ -1448,9 +1448,11 @@ def _linear_stream_rows(rows: "StreamRows", w: torch.Tensor, gate_pairs, partial
 
 def thin_whole_pays(m: int, n: int, k: int) -> bool:
     """Whether a narrow product whose reader adds partial products had better leave one of them, by ``csrc/gemm_thin.hip`` with the inner size whole, than
-    2 or 4 by blocks that stay.  Microseconds, whole / parts, at 1 and 8 rows: 2,048 x 3,072 5.0 / 5.6, 5.7 / 6.0, 4,096 x 3,072 6.8 / 9.0, 6.8 / 9.6, 3,072 x 2,048
-    4.5 / 5.6, 4.8 / 6.1, 4,096 x 4,096 7.6 / 8.6, 8.0 / 8.9; but 2,048 x 2,048 4.2 / 4.0, 4.6 / 4.2, 1,024 x 4,096 5.3 / 4.1; at 16 rows 2,048 x 4,096 7.5 / 6.7."""
-    return m <= 8 and 2048 <= n <= 4096 and 2048 <= k <= 4096 and (n > 2048 or 2048 < k < 4096)
+    2 or 4 by blocks that stay: up to 8 rows, 2,048 to 4,096 columns, and more than 2,048 rows of W, for up to 2,048 two parts are one round of blocks.  There only longer
+    inner sizes gain, whose parts do not hold x in few registers.  Microseconds, whole / parts, at 1 and 8 rows, in brackets with the launch that adds: 2,112 x 2,048
+    4.4 / 6.0, 4.8 / 6.3 (8.2 / 9.7), x 4,096 5.8 / 7.6, 6.4 / 8.1 (9.9 / 12.0), 4,096 x 3,072 6.8 / 9.0, 6.8 / 9.6, 2,048 x 3,072 5.2 / 5.7, 5.9 / 6.3 (9.1 / 9.8), x 3,584 5.6 / 6.1, 6.3
+    / 6.3; but 2,048 x 2,560 4.9 / 4.9, 5.5 / 5.0 (8.8 / 8.4), x 2,048 4.4 / 4.5, 4.8 / 4.6, 1,024 x 4,096 5.3 / 4.1; at 16 rows 2,048 x 4,096 7.5 / 6.7."""
+    return m <= 8 and 2048 <= n <= 4096 and 2048 <= k <= 4096 and (n > 2048 or 2560 < k < 4096)
 
 
 def gemm_few(x: torch.Tensor, w: torch.Tensor, tile: int, gate_pairs: "str | tuple | None" = None, out_dtype=torch.bfloat16) -> torch.Tensor:

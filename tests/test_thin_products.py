@@ -132,3 +132,35 @@ def test_layers_through_the_stream(monkeypatch, running, prompt):
     assert used
     # two roundings of bfloat16 a layer and product that differ by the order of sums
     assert ((a - b).norm() / b.norm()).item() < 6 * 2.0 ** -8
+
+
+def test_where_one_whole_product_stands_for_parts():
+    from jax_vllm_amd.ops.kernels import thin_whole_pays as pays
+
+    assert pays(8, 2052, 2048) and not pays(9, 2052, 2048) and not pays(8, 2052, 1984) and not pays(8, 2052, 4160)
+    assert pays(1, 4096, 4096) and not pays(1, 4100, 4096) and not pays(1, 2044, 3072)
+    assert [pays(8, 2048, k) for k in (2048, 2560, 2624, 3072, 4032, 4096)] == [False, False, True, True, True, False]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,whole", [(8, 4096, 3072, True), (1, 2052, 2048, True), (8, 2048, 2624, True), (8, 2048, 2560, False), (9, 4096, 3072, False), (8, 4100, 2048, False)])
+def test_one_whole_product_and_its_readers(m, n, k, whole):
+    """What ``linear`` leaves around the rule, and the launches that add partial products behind it."""
+    x, w, h = randn(m, k, seed=m).bfloat16(), randn(n, k, seed=n + k).bfloat16(), randn(m, n, seed=7)
+    weight = 1 + 0.1 * randn(n, seed=8)
+    parts = K().linear(x, w, partial_ok=True)
+    assert (parts.dim() == 3 and parts.shape[0] == 1) == whole
+    z = x.double() @ w.double().T
+    sums = parts.sum(0) if parts.dim() == 3 else parts
+    assert ((sums.double() - z).abs() <= 2.0 ** -24 * k * (x.double().abs() @ w.double().abs().T)).all()      # a sum of k products in float in any order
+    if not whole:
+        return
+    stream, out = h.clone(), torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+    K().add_rmsnorm(stream, parts, weight, out, 1e-6)
+    assert torch.equal(stream, h + parts[0])
+    want = stream.double() * torch.rsqrt(stream.double().square().mean(1, keepdim=True) + 1e-6) * weight.double()
+    torch.testing.assert_close(out.double(), want, rtol=2.0 ** -8, atol=1e-6)
+    if n % 512 == 0:
+        again = h.clone()
+        rows = K().add_parts_unscaled(again, parts, weight, 1e-6)
+        assert torch.equal(again, stream) and torch.equal(rows.x, (stream * weight).bfloat16())
