@@ -1323,13 +1323,14 @@ def thin_tiles(m: int, n: int, cus: int = 256) -> int:
 
 def thin_slots(m: int, n: int, k: int) -> "int | None":
     """Slots of the rings of ``csrc/gemm_thin.hip`` where it takes a product of up to 16 rows (any inner size that is a multiple of 64), or None
-    where blocks of eight waves with x in registers (``csrc/gemm_few.hip``) are better: short inner sizes of 9 rows or more against rows of W that give most
-    units one block of 16 and some two (us there / here at 9 rows 5,120 x 1,024 4.9 / 5.1), and of many rows of W (12,288 x 512 at 8 rows
-    4.7 / 5.0, x 1,024 6.8 / 7.2).  Elsewhere, 54 sizes of 512 to 8,192 rows of W and 512 to 4,096 columns at 1, 4, 8 and 16 rows: 0.82 to 1.01 of the
-    time there."""
-    if 4096 < n <= 6144 and m > 8 and 512 < k <= 1024 or n > 8192 and k <= 1024:
+    where blocks of eight waves with x in registers (``csrc/gemm_few.hip``) are better, all of them of inner sizes up to 1,024: 9 rows or more against rows of W that give
+    most units one block of 16 and some two (us there / here at 9 rows 5,120 x 1,024 4.9 / 5.1); many rows of W (12,288 x 512 at 8 rows 4.7 / 5.0, x 1,024 6.8 /
+    7.2); up to 4 rows beyond 4,096 rows of W (one row, with the activation, 5,120 x 768 4.4 / 4.6, 6,144 x 256 3.2 / 3.4); one and two rows against 257 to 1,024 beyond
+    512 columns (1,024 x 768 at one row 1.03 to 1.04 of the time).  Up to 256 rows of W two slots begin sooner (256 x 1,024 at one row 2.34 by two, 2.53 by four, there 2.33).
+    Elsewhere, 110 sizes of 128 to 8,192 rows of W and 256 to 4,096 columns at 1 to 16 rows: 0.82 to 1.04 of the time there."""
+    if k <= 1024 and (n > 8192 or n > 4096 and (m <= 4 or 512 < k and 8 < m and n <= 6144) or m <= 2 and 256 < n <= 1024 and k > 512):
         return None
-    return 4 if thin_tiles(m, n) == 1 and (n <= 4096 and k > 512 or n > 16384) else 2
+    return 4 if thin_tiles(m, n) == 1 and (256 < n <= 4096 and k > 512 or n > 16384) else 2
 
 
 def thin_tiles_pay(m: int, n: int, k: int) -> bool:

@@ -50,3 +50,14 @@ def test_where_two_tiles_do_not_pay():
         assert [pays(9, n, k) for k in (1088, 1536, 1600, 2048, 2560, 2624, 3008, 3072, 3136, 4096)] == [True, True, False, False, False, True, True, False, True, True]
     assert [pays(16, 49152, k) for k in (1088, 2048, 3072, 3584)] == [False, False, False, True]
     assert [pays(16, 65536, k) for k in (2048, 3584)] == [False, True] and [pays(16, 151936, k) for k in (3584, 4096)] == [False, True]
+
+
+def test_where_blocks_with_x_in_registers_stay_better():
+    from jax_vllm_amd.ops.kernels import thin_slots as slots
+
+    assert [slots(1, 256, k) for k in (512, 576, 1024, 1088)] == [2] * 4 and [slots(1, n, 1024) for n in (260, 1024, 1028)] == [None, None, 4]
+    assert slots(2, 512, 512) == 2 and slots(2, 512, 576) is None and slots(3, 512, 576) == 4
+    assert [slots(4, n, 1024) for n in (4096, 4100, 8192, 8196)] == [4, None, None, None] and slots(4, 4100, 1088) == 2
+    assert [slots(5, n, 512) for n in (4100, 8192, 8196)] == [2, 2, None]
+    assert [slots(9, n, 1024) for n in (4096, 4100, 6144, 6148)] == [4, None, None, 2] and slots(9, 5120, 512) == 2
+    assert slots(1, 32000, 2048) == 4 and slots(16, 24576, 4096) == 2
