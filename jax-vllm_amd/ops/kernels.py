@@ -1095,6 +1095,11 @@ def compute_units(device) -> int:
     return n
 
 
+def _units_of(t: torch.Tensor) -> int:
+    """Compute units of a tensor's device; a tensor elsewhere can be planned for, but not launched with."""
+    return compute_units(t.device) if t.is_cuda else 256
+
+
 STAY_PIECES = (4, 5, 8, 10, 12, 16, 17, 20)
 STAY_PIECES_32_ROWS = (4, 5, 8, 12, 16)      # of these, the ones built for 17..32 rows (two row tiles of x in registers)
 
@@ -1321,7 +1326,12 @@ def thin_tiles(m: int, n: int, cus: int = 256) -> int:
     return 2 if m > 8 and 2 * -(-(-(-n // 32)) // cus) <= -(-(-(-n // 16)) // cus) else 1
 
 
-def thin_slots(m: int, n: int, k: int) -> "int | None":
+def thin_ring(m: int, n: int, k: int, cus: int = 256) -> int:
+    """Slots of a wave's ring in ``csrc/gemm_thin.hip`` (2 or 4; the figures are there)."""
+    return 4 if thin_tiles(m, n, cus) == 1 and (256 < n <= 4096 and k > 512 or n > 16384) else 2
+
+
+def thin_slots(m: int, n: int, k: int, cus: int = 256) -> "int | None":
     """Slots of the rings of ``csrc/gemm_thin.hip`` where it takes a product of up to 16 rows (any inner size that is a multiple of 64), or None
     where blocks of eight waves with x in registers (``csrc/gemm_few.hip``) are better, all of them of inner sizes up to 1,024: 9 rows or more against rows of W that give
     most units one block of 16 and some two (us there / here at 9 rows 5,120 x 1,024 4.9 / 5.1); many rows of W (12,288 x 512 at 8 rows 4.7 / 5.0, x 1,024 6.8 /
@@ -1330,16 +1340,16 @@ def thin_slots(m: int, n: int, k: int) -> "int | None":
     Elsewhere, 110 sizes of 128 to 8,192 rows of W and 256 to 4,096 columns at 1 to 16 rows: 0.82 to 1.04 of the time there."""
     if k <= 1024 and (n > 8192 or n > 4096 and (m <= 4 or 512 < k and 8 < m and n <= 6144) or m <= 2 and 256 < n <= 1024 and k > 512):
         return None
-    return 4 if thin_tiles(m, n) == 1 and (256 < n <= 4096 and k > 512 or n > 16384) else 2
+    return thin_ring(m, n, k, cus)
 
 
-def thin_tiles_pay(m: int, n: int, k: int) -> bool:
+def thin_tiles_pay(m: int, n: int, k: int, cus: int = 256) -> bool:
     """Whether two tiles a block are better than blocks that stay or have x in registers: 9 to 16 rows, inner sizes beyond 1,024, and from 16,385 rows of W on not
     where blocks that stay, two to a unit, hold 7 to 10 or 12 whole pieces of 256 columns, nor beyond 32,768 with fewer than 14.  Microseconds at 9 / 16 rows, there and
     here: 6,144 x 4,096 13.5, 12.2 / 14.2, 11.5, 24,576 x 4,096 with its activation 36.5, 34.8 / 38.3, 35.8, 16,384 x 4,096 26.8, 25.3 / 27.7, 24.4; but 24,576 x 2,560
     24.2, 25.2 / 25.3, 26.3, 32,000 x 2,560 31.0, 32.0 / 32.0, 34.4, x 3,072 36.3, 37.4 / 37.4, 39.9, 151,936 x 2,048 115, 112 / 121, 123, x 4,096 213, 207 / 225, 221.  Time here
     over there: 32,000 x 1,344 0.86, 1,856 1.07, 2,624 1.01, 3,008 1.00, 3,136 0.95, 49,152 x 2,048 1.02, x 1,536 1.03, x 3,584 1.00."""
-    if thin_tiles(m, n) != 2 or k <= 1024:
+    if thin_tiles(m, n, cus) != 2 or k <= 1024:
         return False
     if n <= 16384:
         return True
@@ -1357,10 +1367,10 @@ def gemm_thin_scaled(rows: "StreamRows", w: torch.Tensor, gate_pairs: "str | tup
     n = w.shape[0]
     _need(w.shape[1] == k and 0 < m <= SKINNY_AUTO_ROWS and k % 64 == 0 and n % 4 == 0, "inner sizes differ, or more than 16 rows")
     _need(ssq.dtype == torch.float32 and tuple(ssq.shape) == (m, rows.max_shares) and rows.width == k and k <= 16 * rows.max_shares, "the scale does not belong to x")
-    y = torch.empty((m, n // 2 if gate_pairs else n), dtype=torch.bfloat16 if gate_pairs else torch.float32, device=x.device)
+    y, cus = torch.empty((m, n // 2 if gate_pairs else n), dtype=torch.bfloat16 if gate_pairs else torch.float32, device=x.device), compute_units(x.device)
     _check(library.core().jv_gemm_thin_bf16(
         _ptr(y), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), c_longlong(k), c_int(FEW_MODES["pairs" if gate_pairs else "float"]),
-        *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), c_int(thin_slots(m, n, k) or 2), c_int(thin_tiles(m, n)), _ptr(ssq), c_int(rows.shares), c_int(rows.width),
+        *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), c_int(thin_ring(m, n, k, cus)), c_int(thin_tiles(m, n, cus)), _ptr(ssq), c_int(rows.shares), c_int(rows.width),
         c_float(rows.eps), _stream()), "gemm_thin")
     return y
 
@@ -1419,7 +1429,7 @@ def _stream_rows_plan(m: int, w: torch.Tensor, gate_pairs: bool, partial_ok: boo
     if (w.dtype != torch.bfloat16 or not 0 < m <= SKINNY_AUTO_ROWS or k % 64 or not 0 < k <= STREAM_PRODUCT_MAX_WIDTH or n % 4 or not w.is_contiguous()
             or w.data_ptr() % 16 or not (gate_pairs or partial_ok)):
         return None
-    if thin_tiles_pay(m, n, k):
+    if thin_tiles_pay(m, n, k, _units_of(w)):
         return "thin"
     if n > 16384 or n > 8192 and k > 2560:
         plan = streaming_plan(m, n, k, gate_pairs, partial_ok, w.device, partial_max_width)
@@ -1467,11 +1477,12 @@ def gemm_few(x: torch.Tensor, w: torch.Tensor, tile: int, gate_pairs: "str | tup
     _need(out_dtype in (torch.bfloat16, torch.float32) and not (gate_pairs and out_dtype == torch.float32), "the activation's result is bfloat16")
     y = torch.empty((m, n // 2 if gate_pairs else n), dtype=out_dtype, device=x.device)
     mode = "pairs" if gate_pairs else "float" if out_dtype == torch.float32 else "rows"
-    slots = thin_slots(m, n, k)
+    cus = compute_units(x.device)
+    slots = thin_slots(m, n, k, cus)
     if slots is not None:
         _check(library.core().jv_gemm_thin_bf16(
             _ptr(y), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), c_longlong(k), c_int(FEW_MODES[mode]),
-            *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), c_int(slots), c_int(thin_tiles(m, n)), *_NO_SCALE, _stream()), "gemm_few")
+            *(_gate_act(gate_pairs) if gate_pairs else _NO_ACT), c_int(slots), c_int(thin_tiles(m, n, cus)), *_NO_SCALE, _stream()), "gemm_few")
         return y
     _check(library.core().jv_gemm_few_bf16(
         _ptr(y), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), c_longlong(k), c_int(FEW_MODES[mode]),
@@ -1600,7 +1611,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype=None, partial_ok: bool = 
         _need(scale is None or (plan is not None and plan[0][0] == -2),
               "un-normalised rows need a product by the blocks that stay (ask linear_takes_unscaled_rows first)")
         if (plan is not None and plan != STAGED and scale is None and m <= SKINNY_AUTO_ROWS and not (k % 64 or n % 4) and k <= FEW_MAX_INNER and w.dtype == torch.bfloat16
-                and (plan[1] > 1 and thin_whole_pays(m, n, k) or thin_tiles_pay(m, n, k)) and out_dtype in (None, torch.bfloat16, torch.float32)
+                and (plan[1] > 1 and thin_whole_pays(m, n, k) or thin_tiles_pay(m, n, k, compute_units(x.device))) and out_dtype in (None, torch.bfloat16, torch.float32)
                 and not (gate_pairs and out_dtype == torch.float32) and x.is_contiguous() and w.is_contiguous() and not (x.data_ptr() | w.data_ptr()) & 15):
             if plan[1] > 1:
                 return gemm_few(x, w, 16, out_dtype=torch.float32).view(1, m, n)

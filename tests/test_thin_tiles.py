@@ -61,3 +61,26 @@ def test_where_blocks_with_x_in_registers_stay_better():
     assert [slots(5, n, 512) for n in (4100, 8192, 8196)] == [2, 2, None]
     assert [slots(9, n, 1024) for n in (4096, 4100, 6144, 6148)] == [4, None, None, 2] and slots(9, 5120, 512) == 2
     assert slots(1, 32000, 2048) == 4 and slots(16, 24576, 4096) == 2
+
+
+def test_tiles_are_counted_against_the_device_s_units():
+    from jax_vllm_amd.ops import kernels
+
+    # 384 tiles: one round of 384 units and no need for two a block, two rounds of 192
+    assert [kernels.thin_tiles(16, 6144, cus) for cus in (192, 256, 384)] == [2, 2, 1]
+    assert [kernels.thin_tiles_pay(16, 6144, 4096, cus) for cus in (192, 256, 384)] == [True, True, False]
+    assert [kernels.thin_slots(16, 24576, 2048, cus) for cus in (256, 1536)] == [2, 4]
+    assert kernels._stream_rows_plan(16, torch.empty(6144, 4096, dtype=torch.bfloat16), True, False, None) == "thin"      # planned for, on the CPU
+
+
+@pytest.mark.gpu
+def test_products_ask_for_the_device_s_units(monkeypatch):
+    x, w = randn(16, 2048, seed=1).bfloat16(), randn(6144, 2048, seed=2).bfloat16()
+    rows = K().StreamRows(x, torch.rand(16, 256, device="cuda") + 0.1, 2048, 1e-6)
+    asked, tiles = [], K().thin_tiles
+    monkeypatch.setattr(K(), "compute_units", lambda device: 384)
+    monkeypatch.setattr(K(), "thin_tiles", lambda m, n, cus=256: asked.append(cus) or tiles(m, n, cus))
+    for product in (lambda: K().linear(x, w), lambda: K().gemm_few(x, w, 16), lambda: K().linear(rows, w, gate_pairs="silu")):
+        asked.clear()
+        product()
+        assert asked and set(asked) == {384}
