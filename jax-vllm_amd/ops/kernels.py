@@ -592,6 +592,7 @@ def attn_prepare_wide(qkv, bias, q_weight, k_weight, eps: float, cos_sin, rot_di
               "v_first must be a [n, nkv * dv] view of qkv's type with unit column stride")
         _need(q_weight is None or norm_per_head, "values are blended beside a per-head norm or none")
     _need(beside is None or q_weight is None or norm_per_head, "no launch beside a norm over the whole projection")
+    _need(beside is None or not beside.taken, "a held launch was taken along before")
     q = torch.empty((n, nq * dp), dtype=qkv.dtype, device=qkv.device)
     fn = getattr(library.core(), f"jv_attn_prepare_wide_{_suffix(qkv.dtype)}")
     _check(fn(_ptr(q), _ptr(qkv), c_longlong(ld), _ptr(bias), _ptr(q_weight), _ptr(k_weight), c_float(eps),
@@ -601,6 +602,8 @@ def attn_prepare_wide(qkv, bias, q_weight, k_weight, eps: float, cos_sin, rot_di
               _ptr(positions if q_temperature is not None else None), c_float(coef), c_int(every), _ptr(v_first),
               c_longlong(0 if v_first is None else v_first.stride(0)), c_float(v_mix), _stream(), beside and beside.args),
            "attn_prepare_wide")
+    if beside is not None:
+        beside.taken = True
     return q
 
 
@@ -2713,11 +2716,16 @@ def _token_operands(proj, cols, norm_weight, state, slot_ids, cu_seqlens, heads:
 
 class HeldToken:
     """A launch of ``delta_token`` or ``gated_linear_token`` that another kernel's launch of the same step takes along (``attn_prepare_wide``'s
-    ``beside``); its result is ``out``.  Holds addresses: for a launch right behind, while its caller holds the tensors."""
+    ``beside``); its result is ``out``.  Holds addresses: for a launch right behind, while its caller holds the tensors.  Nobody takes it twice,
+    and ``result`` refuses rows that nobody made."""
 
     def __init__(self):
         self.args = ctypes.create_string_buffer(library.core().jv_token_launch_bytes())
-        self.out = None
+        self.out, self.taken = None, False
+
+    def result(self) -> torch.Tensor:
+        _need(self.taken, "a held launch was not taken along")
+        return self.out
 
 
 def delta_token(proj, at: int, conv_weight, conv_state, dt_bias, a_log, unit_eps: float, q_scale: float, norm_weight, eps: float,

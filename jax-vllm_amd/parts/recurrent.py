@@ -210,7 +210,7 @@ class GatedDeltaMixer:
         return held
 
     def finish_token(self, held):
-        return K.linear(held.out, self.w_o, partial_ok=True)
+        return K.linear(held.result(), self.w_o, partial_ok=True)
 
     def forward_projected(self, proj, at: int, ctx: StepContext, mem: LayerMemory):
         """The mixer behind its input product, whose columns begin at ``at``."""
@@ -377,7 +377,7 @@ class GatedLinearAttention:
         return held
 
     def finish_token(self, held):
-        return K.linear(held.out, self.w_o, partial_ok=True)
+        return K.linear(held.result(), self.w_o, partial_ok=True)
 
     def forward_projected(self, proj, at: int, ctx: StepContext, mem: LayerMemory):
         """The mixer behind its input product, whose columns begin at ``at``."""

@@ -42,3 +42,38 @@ def test_the_bits_of_two_launches(n, nq, nkv, dk, heads, dim, empty, kind, dtype
 
     for a, b in zip(run(False), run(True)):
         assert torch.equal(a, b)
+
+
+def test_a_launch_that_nobody_took_is_no_result():
+    from types import SimpleNamespace
+
+    from jax_vllm_amd.ops import kernels as K
+    from jax_vllm_amd.parts.recurrent import GatedDeltaMixer, GatedLinearAttention
+
+    held = object.__new__(K.HeldToken)
+    held.out, held.taken = torch.zeros(1, 4), False
+    for mixer in (GatedDeltaMixer, GatedLinearAttention):
+        with pytest.raises(K.KernelArgumentError, match="not taken"):
+            mixer.finish_token(SimpleNamespace(w_o=torch.zeros(4, 4)), held)
+    held.taken = True
+    assert held.result() is held.out
+
+
+@pytest.mark.gpu
+def test_a_launch_is_taken_once():
+    from jax_vllm_amd.ops import kernels as K
+
+    heads, dim = 2, 64
+    proj = torch.randn(2, 3 * 64 + heads * 4 * dim + 8, device="cuda")
+    cu, slots = torch.arange(3, dtype=torch.int32, device="cuda"), torch.arange(2, dtype=torch.int32, device="cuda")
+    state = torch.zeros(2, heads, dim, dim, device="cuda")
+    up, held = torch.zeros(heads * dim, 8, device="cuda"), K.HeldToken()
+    K.gated_linear_token(proj, 3 * 64, up, torch.zeros(heads * dim, device="cuda"), 16.0, 1.0, torch.ones(dim, device="cuda"), 1e-5, state, slots, cu, heads, dim,
+                         dim, hold=held)
+    with pytest.raises(K.KernelArgumentError, match="not taken"):
+        held.result()
+    prepare = lambda: K.attn_prepare_wide(proj, None, None, None, 0.0, None, 0, None, None, None, 16, 1, 1, 64, 64, 64, beside=held)
+    prepare()
+    assert held.result() is held.out and held.out.isfinite().all()
+    with pytest.raises(K.KernelArgumentError, match="before"):
+        prepare()
