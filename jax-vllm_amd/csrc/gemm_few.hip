@@ -10,8 +10,8 @@
 // in ascending order, so a row's result does not depend on the others.
 //
 // Microseconds in a graph, cold weights, at 1, 8 and 16 rows (before, x staged chunk by chunk in LDS for all waves of a block): 1,536 x 768 2.9, 3.2, 3.4 (4.6,
-// 5.0, 6.2), 2,048 x 2,048 4.0, 4.7, 5.4 (5.5, 6.2, 7.1).  Given rows of longer inner sizes, and most of shorter ones, go through gemm_thin.hip, to the same bits
-// (thin_slots has the figures of both); given rows are taken up to 2,048 columns here, rows that the blocks make up to 4,096.
+// 5.0, 6.2).  Given rows of longer inner sizes, and many of shorter ones, go through gemm_thin.hip, to the same bits (thin_slots has the figures of both): given
+// rows are taken up to 1,024 columns here, two chunks a wave, rows that the blocks make up to 4,096.
 #include "common.h"
 #include "row_source.h"
 
@@ -154,22 +154,15 @@ gemm_few_kernel(void* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t
 
 template <int MODE, int TW>
 static int few_launch(void* y, const void* x, const void* W, int M, int N, int K, long long ldx, JvAct act, hipStream_t s) {
-  const int cw = (K / FEW_K + FEW_WAVES - 1) / FEW_WAVES;
-#define FEW(CW)                                                                                                                        \
-  if (cw <= CW) {                                                                                                                      \
-    hipLaunchKernelGGL((gemm_few_kernel<MODE, TW, CW>), dim3((N + TW - 1) / TW), dim3(64 * FEW_WAVES), 0, s, y, (const bf16_t*)x,     \
-                       (const bf16_t*)W, M, N, K, ldx, act, RowSource{});                                                                           \
-    return JV_LAUNCH_CHECK();                                                                                                          \
-  }
-  FEW(2) FEW(4)
-#undef FEW
-  return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL((gemm_few_kernel<MODE, TW, 2>), dim3((N + TW - 1) / TW), dim3(64 * FEW_WAVES), 0, s, y, (const bf16_t*)x, (const bf16_t*)W, M, N, K, ldx, act,
+                     RowSource{});
+  return JV_LAUNCH_CHECK();
 }
 // mode: FEW_*; tw (16, 32): rows of W of a block.
 extern "C" int jv_gemm_few_bf16(void* y, const void* x, const void* W, int M, int N, int K, long long ldx, int mode, int gate_act,
                                 float act_limit, float act_slope, int tw, void* stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > 16 || K < FEW_K || K % FEW_K || N % 4 || ldx % 8 || (((uintptr_t)x | (uintptr_t)W | (uintptr_t)y) & 15))
+  if (M > 16 || K < FEW_K || K > 2 * FEW_WAVES * FEW_K || K % FEW_K || N % 4 || ldx % 8 || (((uintptr_t)x | (uintptr_t)W | (uintptr_t)y) & 15))
     return (int)hipErrorInvalidValue;
   if (mode == FEW_PAIRS && !jv_act_known(gate_act)) return (int)hipErrorInvalidValue;
   const JvAct act{gate_act, act_limit, act_slope};

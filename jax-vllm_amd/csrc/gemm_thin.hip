@@ -180,9 +180,13 @@ static int thin_launch(void* y, const void* x, const void* W, int M, int N, int 
 #define THIN(XL, S)                                                                                                                      \
   hipLaunchKernelGGL((gemm_thin_kernel<MODE, SCALED, XL, S, NT>), dim3((N + 16 * NT - 1) / (16 * NT)), dim3(64 * THIN_WAVES), 0, st, y, (const bf16_t*)x, \
                      (const bf16_t*)W, M, N, K, ldx, act, scale, stream)
-  if (slots == 4) {
+  if constexpr (NT == 2) {                     // two tiles: more than 8 rows, rings of two slots
+    if (slots != 2 || M <= 8) return (int)hipErrorInvalidValue;
+    THIN(2, 2);
+  } else if (slots == 4) {
     if (M <= 8) THIN(1, 4); else THIN(2, 4);
-  } else if (slots == 2) {
+  } else if constexpr (MODE != THIN_STREAM) {
+    if (slots != 2) return (int)hipErrorInvalidValue;
     if (M <= 8) THIN(1, 2); else THIN(2, 2);
   } else
     return (int)hipErrorInvalidValue;
@@ -192,33 +196,37 @@ static int thin_launch(void* y, const void* x, const void* W, int M, int N, int 
 static bool thin_sizes(const void* y, const void* x, const void* W, int M, int N, int K, long long ldx) {
   return M <= 16 && K >= THIN_K && K % THIN_K == 0 && N % 4 == 0 && ldx >= K && ldx % 8 == 0 && !(((uintptr_t)x | (uintptr_t)W | (uintptr_t)y) & 15);
 }
-// mode: THIN_BF16, THIN_F32 or THIN_PAIRS; slots (2, 4) of a wave's ring; tiles (1, 2) of 16 rows of W of a block; ssq (rows of 256 floats, shares of them, a multiple of 4) or null.
+// mode: THIN_BF16, THIN_F32 or THIN_PAIRS; slots (2, 4) of a wave's ring; tiles (1, 2; two for 9 rows and more, with two slots) of 16 rows of W of a block; ssq (rows of
+// 256 floats, shares of them, a multiple of 4; float sums and activations only) or null.
 extern "C" int jv_gemm_thin_bf16(void* y, const void* x, const void* W, int M, int N, int K, long long ldx, int mode, int gate_act, float act_limit,
                                  float act_slope, int slots, int tiles, const float* ssq, int shares, int width, float eps, void* stream) {
   if (M <= 0 || N <= 0) return 0;
   if (!thin_sizes(y, x, W, M, N, K, ldx) || mode < THIN_BF16 || mode > THIN_PAIRS || (mode == THIN_PAIRS && !jv_act_known(gate_act)) || tiles < 1 || tiles > 2 ||
-      (ssq && (shares < 4 || shares > THIN_SHARES || shares % 4 || width <= 0 || ((uintptr_t)ssq & 15))))
+      (ssq && (mode == THIN_BF16 || shares < 4 || shares > THIN_SHARES || shares % 4 || width <= 0 || ((uintptr_t)ssq & 15))))
     return (int)hipErrorInvalidValue;
   const JvAct act{gate_act, act_limit, act_slope};
   const ThinScale scale{ssq, shares, 1.f / (float)width, eps};
   const hipStream_t st = (hipStream_t)stream;
-#define THIN(MODE)                                                                                                      \
-  if (tiles == 2)                                                                                                       \
-    return ssq ? thin_launch<MODE, true, 2>(y, x, W, M, N, K, ldx, slots, act, scale, ThinStream{}, st)                 \
-               : thin_launch<MODE, false, 2>(y, x, W, M, N, K, ldx, slots, act, scale, ThinStream{}, st);               \
-  return ssq ? thin_launch<MODE, true>(y, x, W, M, N, K, ldx, slots, act, scale, ThinStream{}, st)                      \
-             : thin_launch<MODE, false>(y, x, W, M, N, K, ldx, slots, act, scale, ThinStream{}, st)
-  if (mode == THIN_F32) { THIN(THIN_F32); }
-  if (mode == THIN_PAIRS) { THIN(THIN_PAIRS); }
-  THIN(THIN_BF16);
+#define THIN(MODE, SCALED)                                                                                              \
+  return tiles == 2 ? thin_launch<MODE, SCALED, 2>(y, x, W, M, N, K, ldx, slots, act, scale, ThinStream{}, st)          \
+                    : thin_launch<MODE, SCALED>(y, x, W, M, N, K, ldx, slots, act, scale, ThinStream{}, st)
+  if (mode == THIN_F32) {
+    if (ssq) { THIN(THIN_F32, true); }
+    THIN(THIN_F32, false);
+  }
+  if (mode == THIN_PAIRS) {
+    if (ssq) { THIN(THIN_PAIRS, true); }
+    THIN(THIN_PAIRS, false);
+  }
+  THIN(THIN_BF16, false);
 #undef THIN
 }
 // h += x W^T in place; with a weight rows = bf16(h * weight) and ssq[row * 256 + block] the blocks' shares of the rows' sums of squares.
-extern "C" int jv_gemm_thin_stream_bf16(float* h, const void* x, const void* W, int M, int N, int K, long long ldx, int slots, const float* weight,
-                                        void* rows, float* ssq, void* stream) {
+extern "C" int jv_gemm_thin_stream_bf16(float* h, const void* x, const void* W, int M, int N, int K, long long ldx, const float* weight, void* rows,
+                                        float* ssq, void* stream) {
   if (M <= 0 || N <= 0) return 0;
   if (!thin_sizes(h, x, W, M, N, K, ldx) ||
       (weight && ((N + 15) / 16 > THIN_SHARES || !rows || !ssq || (((uintptr_t)weight | (uintptr_t)rows) & 15))))
     return (int)hipErrorInvalidValue;
-  return thin_launch<THIN_STREAM, false>(h, x, W, M, N, K, ldx, slots, JvAct{}, ThinScale{}, ThinStream{weight, (bf16_t*)rows, ssq}, (hipStream_t)stream);
+  return thin_launch<THIN_STREAM, false>(h, x, W, M, N, K, ldx, 4, JvAct{}, ThinScale{}, ThinStream{weight, (bf16_t*)rows, ssq}, (hipStream_t)stream);
 }

@@ -1305,11 +1305,8 @@ FEW_MAX_INNER = 4096      # columns up to which ``few_tile`` was measured
 
 def few_tile(m: int, n: int, k: int, cus: int = 256) -> "int | None":
     """Rows of w of a block of ``gemm_few`` (16 or 32) where it takes the product, else None: 32 where 16 would give a unit more than
-    one block and most units only one (4,608 x 3,072 9.3 us against 10.5, 6,144 x 2,048 at 8 rows 9.1 / 9.4, at one row 8.7 / 8.4; 4,096 x
-    2,048 6.8 / 5.9, 8,192 x 2,048 10.0 / 9.1, 11,296 x 2,048 12.6 / 12.0); 9 to 16 rows also where 16 would give units a fourth block
-    (us here by 32 / by 16 / the library at 16 rows: 12,288 x 4,096 26.4 / 25.5 / 26.2, 12,800 26.6 / 30.0 / 26.8, 15,360 28.3 / 31.7 / 28.5, 16,000 30.1 / 32.1 /
-    30.1, 14,336 x 3,072 21.3 / 24.5 / 21.3, 16,000 x 2,688 19.3 / 22.8 / 28.5; fewer rows gain less: 9 rows x 15,360 26.3 / 27.3 / 28.3, 1 row 25.5 / 24.5;
-    inner sizes up to 1,024 do not: 12,304 x 1,024 at 9 rows 7.7 / 7.4).
+    one block and most units only one (6,144 x 2,048 at one row 8.7 / 8.4; 4,096 x 2,048 6.8 / 5.9, 8,192 x 2,048 10.0 / 9.1, 11,296 x 2,048 12.6 / 12.0; 12,304 x 1,024 at 9
+    rows 7.7 / 7.4).  Where ``thin_slots`` gives a product to smaller blocks, only whether it is taken counts.
     One row against the output embedding stays with x resident in LDS where its 4,096 columns are nearly filled: us here / resident, 151,936
     rows of W: k = 4,096 204.6 / 200.4, 3,840 191.4 / 190.4, 3,584 180.3 / 178.5, 3,328 167.5 / 174.4, 2,048 104 / 154; two rows 205.4 / 205.0,
     193.5 / 203.8, 183.2 / 193.4; 65,536 x 4,096 91.2 / 88.0, two rows 92.3 / 93.9; 16,000 x 4,096 25.3 / 25.0."""
@@ -1318,7 +1315,7 @@ def few_tile(m: int, n: int, k: int, cus: int = 256) -> "int | None":
     if m == 1 and n >= 65536 and k >= 3584:
         return None
     tiles = -(-n // 16)
-    return 32 if cus < tiles <= 1.5 * cus or (m > 8 and tiles > 3 * cus and k >= 1536) else 16
+    return 32 if cus < tiles <= 1.5 * cus else 16
 
 
 def thin_tiles(m: int, n: int, cus: int = 256) -> int:
@@ -1415,7 +1412,7 @@ def gemm_into_stream(h: torch.Tensor, x: torch.Tensor, w: torch.Tensor, weight=N
         _f32(weight, "weight", n)
         rows = torch.empty((m, n), dtype=torch.bfloat16, device=h.device)
         ssq = torch.empty((m, StreamRows.max_shares), dtype=torch.float32, device=h.device)      # n / 16 of a row's 256 are written
-    _check(library.core().jv_gemm_thin_stream_bf16(_ptr(h), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), c_longlong(k), c_int(4), _ptr(weight),
+    _check(library.core().jv_gemm_thin_stream_bf16(_ptr(h), _ptr(x), _ptr(w), c_int(m), c_int(n), c_int(k), c_longlong(k), _ptr(weight),
                                                    _ptr(rows), _ptr(ssq), _stream()), "gemm_into_stream")
     return None if weight is None else StreamRows(rows, ssq, n, eps)
 
@@ -1470,8 +1467,9 @@ def thin_whole_pays(m: int, n: int, k: int) -> bool:
 
 
 def gemm_few(x: torch.Tensor, w: torch.Tensor, tile: int, gate_pairs: "str | tuple | None" = None, out_dtype=torch.bfloat16) -> torch.Tensor:
-    """x @ w.T for up to 16 rows of bfloat16 x against bfloat16 w [N, K], K a multiple of 64 up to 4,096, ``tile`` (16 or 32) rows of w a
-    block: see ``csrc/gemm_few.hip``.  bfloat16 or float32 [M, N], or with ``gate_pairs`` the activation, bfloat16 [M, N / 2]."""
+    """x @ w.T for up to 16 rows of bfloat16 x against bfloat16 w [N, K], K a multiple of 64 up to 4,096: by small blocks (``csrc/gemm_thin.hip``) where
+    ``thin_slots`` says so, else by blocks of ``tile`` (16 or 32) rows of w with x in registers (``csrc/gemm_few.hip``), to the same bits.  bfloat16 or float32
+    [M, N], or with ``gate_pairs`` the activation, bfloat16 [M, N / 2]."""
     _dev(x, w)
     _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "gemm_few takes bfloat16")
     m, k = x.shape

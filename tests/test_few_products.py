@@ -25,6 +25,23 @@ def test_few_rows(m, n, k, tile):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(1, 5120, 1024), (4, 4100, 64), (3, 8192, 448), (9, 5120, 1024), (16, 6144, 576), (8, 8196, 1024), (16, 12288, 512), (1, 512, 768),
+                                   (2, 1024, 1024)])
+@pytest.mark.parametrize("tile", [16, 32])
+def test_what_blocks_with_x_in_registers_take(m, n, k, tile):
+    """The sizes that the rule leaves to them, and the bits of small blocks."""
+    assert K().thin_slots(m, n, k) is None and K().few_tile(m, n, k) is not None
+    test_few_rows(m, n, k, tile)
+
+
+@pytest.mark.gpu
+def test_given_rows_of_more_columns_are_refused(monkeypatch):
+    monkeypatch.setattr(K(), "thin_slots", lambda *_: None)
+    with pytest.raises(K().KernelArgumentError):
+        K().gemm_few(randn(2, 1088, seed=1).bfloat16(), randn(64, 1088, seed=2).bfloat16(), 16)
+
+
+@pytest.mark.gpu
 def test_rows_that_are_not_finite_stay_alone():
     x, w = randn(9, 512, seed=1).bfloat16(), randn(64, 512, seed=2).bfloat16()
     clean = K().gemm_few(x, w, 16)
@@ -91,7 +108,9 @@ def test_one_row_against_the_output_embedding_stays_with_x_resident():
 
 
 def test_rows_of_w_of_a_block_where_the_library_was():
-    from jax_vllm_amd.ops.kernels import few_tile, streaming_plan
+    from jax_vllm_amd.ops.kernels import few_tile, streaming_plan, thin_slots, thin_tiles
 
     sizes = ((16, 15360, 4096), (9, 12304, 1536), (16, 12288, 4096), (8, 15360, 4096), (16, 15360, 1024))
-    assert streaming_plan(16, 15360, 4096) is None and [few_tile(*s) for s in sizes] == [32, 32, 16, 16, 16]
+    assert streaming_plan(16, 15360, 4096) is None and [few_tile(*s) for s in sizes] == [16] * 5
+    # the tiles of a block are those of the small blocks here
+    assert [thin_slots(*s) and thin_tiles(*s[:2]) for s in sizes] == [2, 2, 1, 1, None]
