@@ -158,15 +158,12 @@ def prefill_item_shape(rows: int, nkv: int, group_rows: int, kernel_groups: int,
     return kernel_groups, blocks <= RESIDENT_BLOCKS * compute_units
 
 
-def few_rows_of_256(rows: int, keys: int, group_rows: int, compute_units: int, page_size: int = 16) -> bool:
-    """Whether a step's prompt portions at head size 256 take items of one group (16 rows a wave) instead of two (32): while
-    those give no more than a quarter of the compute units a second block, with pages of 16 and 2,048 keys no longer; with pages of 16 also where
-    nobody sees more than 256 keys, for an item of two groups is slow to start.  (At pages of 16 ``halves_items`` has the last word.)  Microseconds,
-    two groups / one: 512 tokens after 4,000, 16 heads over one, with pages of 32 203 / 192, of 24 259 / 209; 2,048 over 8 kv heads with pages of 32 98 / 93."""
-    few = 4 * -(-rows // group_rows) <= 5 * compute_units
-    if page_size != 16:
-        return few
-    return keys <= 256 or (few and keys < 2048)
+def few_rows_of_256(rows: int, group_rows: int, compute_units: int) -> bool:
+    """Whether a step's prompt portions at head size 256 and pages of other than 16 keys take items of one group (16 rows a wave) instead of two (32): while those
+    give no more than a quarter of the compute units a second block, whatever the keys, for the larger form has no work of its own to overlap there.  Microseconds, two groups /
+    one: 512 tokens after 4,000, 16 heads over one, with pages of 32 203 / 192, of 24 259 / 209; 2,048 over 8 kv heads with pages of 32 98 / 93.  (Pages of 16:
+    ``halves_items``.)"""
+    return 4 * -(-rows // group_rows) <= 5 * compute_units
 
 
 SHORT_WALK = 400             # keys up to which the halves kernel's start weighs as much as its tiles
@@ -206,12 +203,12 @@ def plan_mfma(ctx, nq: int, nkv: int, head_dim: int, window: int, device, keep: 
     cus = K.compute_units(device)
     one_group = False
     if head_dim == 256:
-        keys = max([keys_seen(cl + ql, window, keep) for ql, cl in zip(ctx.q_lens_host, ctx.context_lens_host) if ql > 1], default=0)
         if ctx.page_size == 16:
+            keys = max([keys_seen(cl + ql, window, keep) for ql, cl in zip(ctx.q_lens_host, ctx.context_lens_host) if ql > 1], default=0)
             groups = [-(-ql * g // group_rows) for ql in ctx.q_lens_host if ql > 1]
             pairs = sum((n + 1) // 2 for n in groups) * nkv
             one_group, groups_per_item, balance = *halves_items(sum(groups) * nkv, pairs, keys, window, capped, cus), False
-        elif few_rows_of_256(rows * nkv, keys, group_rows, cus, ctx.page_size):
+        elif few_rows_of_256(rows * nkv, group_rows, cus):
             one_group, groups_per_item, balance = True, 1, False
     prefill = prefill_work_items(ctx.q_lens_host, ctx.context_lens_host, g, window, group_rows, groups_per_item,
                                  balance=balance, keep=keep)

@@ -10,17 +10,28 @@ from .test_f32_path import reference, run_step
 from .test_kernels_gpu import K, _mfma_inputs, _mfma_reference, _prefill_work, build_paged
 
 
-def test_the_rule():
-    assert few_rows_of_256(300 * 16, 300, 64, 256) and few_rows_of_256(320 * 64, 2047, 64, 256)
-    assert not few_rows_of_256(320 * 64 + 1, 300, 64, 256) and not few_rows_of_256(64, 2048, 64, 256)
+def test_the_rule_of_pages_other_than_16():
+    assert few_rows_of_256(300 * 16, 64, 256) and few_rows_of_256(320 * 64, 64, 256) and not few_rows_of_256(320 * 64 + 1, 64, 256)
+    assert few_rows_of_256(320 * 64 + 1, 64, 304)
 
 
-def test_the_rule_looks_at_pages_and_short_windows():
-    assert few_rows_of_256(64 * 5000, 128, 64, 256) and few_rows_of_256(64 * 5000, 256, 64, 256)      # short walks
-    assert not few_rows_of_256(64 * 5000, 257, 64, 256)
-    for page_size in (8, 24, 32, 64):                     # no work of its own to overlap: rows alone count
-        assert few_rows_of_256(64 * 320, 100000, 64, 256, page_size)
-        assert not few_rows_of_256(64 * 320 + 1, 128, 64, 256, page_size)
+def test_which_rule_a_plan_asks(monkeypatch):
+    """Pages of 16 keys: the rule of the halves, which knows the walk; others count rows alone."""
+    from types import SimpleNamespace
+
+    from jax_vllm_amd.ops import kernels
+    from jax_vllm_amd.parts import attention_backend
+
+    monkeypatch.setattr(kernels, "compute_units", lambda device: 256)
+    monkeypatch.setattr(attention_backend, "upload_i32", lambda values, device: torch.tensor(values, dtype=torch.int32))
+
+    def one_group(page_size, tokens, context, window=0):
+        ctx = SimpleNamespace(q_lens_host=[tokens], context_lens_host=[context], page_size=page_size, block_tables=[torch.zeros(1, 64)])
+        return attention_backend.plan_mfma(ctx, 16, 1, 256, window, "cpu").one_group
+
+    assert one_group(16, 300, 0) is False and one_group(16, 250, 0) and one_group(16, 300, 100000) is False
+    for page_size in (8, 24, 32, 64):
+        assert one_group(page_size, 300, 0) and one_group(page_size, 1280, 100000) and not one_group(page_size, 1281, 0, 128)
 
 
 @pytest.mark.gpu
