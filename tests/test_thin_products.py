@@ -108,11 +108,20 @@ def test_layers_through_the_stream(monkeypatch, running, prompt):
 
     config = dict(architectures=["Qwen3ForCausalLM"], num_hidden_layers=3, hidden_size=512, num_attention_heads=4, num_key_value_heads=2, head_dim=128,
                   intermediate_size=768, vocab_size=512, rope_theta=1e4, rms_norm_eps=1e-6, tie_word_embeddings=False, max_position_embeddings=4096)
-    used = []
-    through = PreNormBlock._through_stream
+    through, layers = PreNormBlock._through_stream, config["num_hidden_layers"]
+    calls = {"into": 0, "scaled": 0, "through": 0}
+    for name, counted in (("gemm_into_stream", "into"), ("gemm_thin_scaled", "scaled")):
+        launch = getattr(K(), name)
+        monkeypatch.setattr(K(), name, lambda *a, launch=launch, counted=counted: calls.update({counted: calls[counted] + 1}) or launch(*a))
+
+    def asked(self, n, *a):
+        ok = through(self, n, *a)
+        calls["through"] += ok
+        return ok
 
     def logits_of(folder, on):
-        monkeypatch.setattr(PreNormBlock, "_through_stream", lambda self, n, *a: on and (used.append(n) or through(self, n, *a)))
+        monkeypatch.setattr(PreNormBlock, "_through_stream", asked if on else lambda self, n, *a: False)
+        calls.update(into=0, scaled=0, through=0)
         llm = LLM(folder, dtype="bf16", block_size=16, num_blocks=200, max_num_seqs=20, max_model_len=256, max_num_batched_tokens=512, enable_prefix_cache=False)
         for i in range(running):
             llm.core.start_request(i)
@@ -128,8 +137,12 @@ def test_layers_through_the_stream(monkeypatch, running, prompt):
 
     with tempfile.TemporaryDirectory() as tmp:
         folder = write_random_model(tmp, config, seed=1, std=0.04, norm_std=0.1)
-        a, b = logits_of(folder, True), logits_of(folder, False)
-    assert used
+        a = logits_of(folder, True)
+        steps, left = divmod(calls["through"], layers)      # steps that were launched, not replayed
+        # every product of a layer joins the stream, all products behind the first norm read it
+        assert steps and not left and calls["into"] == steps * 2 * layers and calls["scaled"] == steps * (2 * layers - 1)
+        b = logits_of(folder, False)
+        assert not any(calls.values())
     # two roundings of bfloat16 a layer and product that differ by the order of sums
     assert ((a - b).norm() / b.norm()).item() < 6 * 2.0 ** -8
 
