@@ -262,6 +262,7 @@ def measure_prefill(llm, rng, vocab, repeats=3):
 KERNEL_GROUPS = (          # substring of a kernel's name -> what it is counted as
     ("gemm_skinny", "products_own"), ("gemm_tile64", "products_own"), ("gemm_rows", "products_own"),
     ("gemm_f32", "products_own"), ("gemm_stream", "products_own"), ("gemm_shares", "products_own"),
+    ("gemm_thin", "products_own"), ("gemm_few", "products_own"),
     ("Cijk", "products_library"), ("rocblas", "products_library"), ("hipblaslt", "products_library"),
     ("attn_", "attention"), ("paged_attention", "attention"),
     ("add_rmsnorm", "norm_residual"), ("add_parts", "norm_residual"), ("rmsnorm", "norm_residual"),

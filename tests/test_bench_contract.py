@@ -54,3 +54,16 @@ def test_the_line_of_a_short_run_has_every_key():
         assert abs(sum(shares.values()) - 1.0) < 0.01 and shares.get("attention", 0) > 0
         assert shares.get("products_own", 0) + shares.get("products_library", 0) > 0.4
     assert abs(line["value"] - 8 / (line["ms_per_step"] * 1e-3)) < 0.01 * line["value"]
+
+
+def test_every_product_of_the_library_is_counted_as_one():
+    """The shares of a step's kernel time: each matrix product that the kernel sources define belongs to the own products."""
+    import re
+    from pathlib import Path
+
+    import bench
+    from jax_vllm_amd.ops import library
+
+    names = {m for f in Path(library.CSRC).rglob("*.hip") for m in re.findall(r"\b(gemm_\w+_kernel)\(", f.read_text())}
+    assert {"gemm_thin_kernel", "gemm_few_kernel", "gemm_skinny_persistent_kernel"} <= names
+    assert {n: next((g for key, g in bench.KERNEL_GROUPS if key in n), "other") for n in names} == dict.fromkeys(names, "products_own")
