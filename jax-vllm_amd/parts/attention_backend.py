@@ -169,7 +169,7 @@ def few_rows_of_256(rows: int, group_rows: int, compute_units: int) -> bool:
 SHORT_WALK = 400             # keys up to which the halves kernel's start weighs as much as its tiles
 
 
-def halves_items(groups: int, pairs: int, keys: int, window: int, capped: bool, compute_units: int):
+def halves_items(groups: int, pairs: int, keys: int, window: int, capped: bool, kv_heads: int, compute_units: int):
     """(Whether 16 rows a wave take them, groups per item) at head size 256 and pages of 16 keys, where two waves share 32 rows of the
     other form.  ``groups``, ``pairs``: items of one group and of two (neighbours of one request) that the prompts have over all kv heads; ``keys``: the most that a
     query sees; ``capped``: scores go through a cap, which is paid once more for every wave that starts.
@@ -177,19 +177,20 @@ def halves_items(groups: int, pairs: int, keys: int, window: int, capped: bool, 
     Walks of more than 400 keys: the halves, by pairs once groups alone give half of the compute units a block or the walk is far (no slower then, and half
     the reads).  Shorter ones: the 16 rows a wave, whose start is short, while the groups are a round of blocks (a quarter of the units a second one), but items of one
     group where 257 keys and more are scored without a cap and no unit has two; beyond a round the pairs, if the prompts have them (a request of one group has
-    none), where a sliding window or 257 keys bound the walk, and up to 64 keys, a tile, only if they save a round.  Microseconds, 16 rows a wave /
+    none), where a sliding window or 257 keys bound the walk, and up to 64 keys, a tile, only if they are one round.  Four kv heads, two dies to a head: not up to 192
+    keys, where the halves take some 14 us more than with other counts (8 heads over 4, whatever the strides and the order of pages; why is not known).  Microseconds, 16 rows a wave /
     items of one group / of two: 16 heads over one, 64 tokens 10.1 / 10.7 / 13.9, 300 20.6 / 20.1 / 22.0, with a cap 22.3 / 22.8 / 24.7, 512 28.6 / 26.3 / 27.3, 1,000 50.5 /
     45.4 / 43.4, with a window of 100 16.6 / - / 20.1, 2,048 with a window of 1,024 104 / 91 / 51, of 256 44 / 43 / 27, of 128 33 / 33 / 23; 512 after
-    4,000 193 / 154 / 155; 30 prompts of 40 tokens, 8 heads over one 10.5 / 11.9 / 15.4, 16 over 8 18.3 / 20.6 / 14.2, 60 of them, 16 over one 29.5 / 33.5 / 31.7.  1,610 steps
-    (five head layouts, 23 sets of prompts, seven windows, with and without a cap): 1.02 of the best form's time on average, and nowhere more than 1.03 of the 16
-    rows a wave."""
+    4,000 193 / 154 / 155; 30 prompts of 40 tokens, 8 heads over one 10.5 / 11.9 / 15.4, 16 over 8 18.3 / 20.6 / 14.2, 60 of them, 16 over one 29.5 / 33.5 / 31.7; 4,096
+    tokens of 8 heads over 4 with a window of 128 33.8 / 34.0 / 38.6, of 32 25.2 / 43.5 / 38.2, of 256 44 / 45 / 41, 2,048 of 16 over 8 with 128 33.1 / 33.3 / 25.4.  Of 2,300
+    steps that the 16 rows a wave took before (16 head layouts, 27 sets of prompts, windows of 32 to 1,024, blocks, with and without a cap) none takes more than 1.02 of their time."""
     if keys > SHORT_WALK:
         return False, 2 if 2 * groups > compute_units or keys >= 2048 else 1
     if 4 * groups <= 5 * compute_units:
         return keys <= 256 or capped or groups > compute_units, 1
     if (keys <= 256 and window <= 0) or 4 * pairs > 3 * groups:
         return True, 1
-    if keys <= KEY_TILE and -(-pairs // compute_units) >= -(-4 * groups // (5 * compute_units)):
+    if keys <= KEY_TILE and pairs > compute_units or keys <= 3 * KEY_TILE and kv_heads == 4:
         return True, 1
     return False, 2
 
@@ -207,7 +208,7 @@ def plan_mfma(ctx, nq: int, nkv: int, head_dim: int, window: int, device, keep: 
             keys = max([keys_seen(cl + ql, window, keep) for ql, cl in zip(ctx.q_lens_host, ctx.context_lens_host) if ql > 1], default=0)
             groups = [-(-ql * g // group_rows) for ql in ctx.q_lens_host if ql > 1]
             pairs = sum((n + 1) // 2 for n in groups) * nkv
-            one_group, groups_per_item, balance = *halves_items(sum(groups) * nkv, pairs, keys, window, capped, cus), False
+            one_group, groups_per_item, balance = *halves_items(sum(groups) * nkv, pairs, keys, window, capped, nkv, cus), False
         elif few_rows_of_256(rows * nkv, group_rows, cus):
             one_group, groups_per_item, balance = True, 1, False
     prefill = prefill_work_items(ctx.q_lens_host, ctx.context_lens_host, g, window, group_rows, groups_per_item,

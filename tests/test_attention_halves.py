@@ -11,24 +11,26 @@ from .test_kernels_gpu import K, _mfma_inputs, _mfma_reference, _prefill_work
 
 
 def test_the_rule():
-    assert halves_items(16, 8, 64, 0, False, 256) == (True, 1)              # few, short
-    assert halves_items(350, 175, 256, -256, False, 256) == (True, 1)       # blocks
-    assert halves_items(350, 175, 256, 256, False, 256) == (False, 2)       # a sliding window
-    assert halves_items(128, 64, 1000, 0, False, 256) == (False, 1)
-    assert halves_items(129, 65, 1000, 1024, False, 256) == (False, 2)
-    assert halves_items(8, 4, 2048, 0, False, 256) == (False, 2)            # far walks
+    assert halves_items(16, 8, 64, 0, False, 8, 256) == (True, 1)              # few, short
+    assert halves_items(350, 175, 256, -256, False, 8, 256) == (True, 1)       # blocks
+    assert halves_items(350, 175, 256, 256, False, 8, 256) == (False, 2)       # a sliding window
+    assert halves_items(128, 64, 1000, 0, False, 8, 256) == (False, 1)
+    assert halves_items(129, 65, 1000, 1024, False, 8, 256) == (False, 2)
+    assert halves_items(8, 4, 2048, 0, False, 8, 256) == (False, 2)            # far walks
 
 
 def test_short_walks_beside_a_round_of_blocks():
     for window in (0, 64, 1024, -64):                                       # groups that are one round: their start alone counts
-        assert halves_items(320, 160, 256, window, False, 256) == (True, 1)
-    assert halves_items(321, 161, 256, 1024, False, 256) == (False, 2)
-    assert halves_items(480, 480, 40, 256, False, 256) == (True, 1)         # requests of one group have no pairs
-    assert halves_items(480, 360, 128, 256, False, 256) == (False, 2) and halves_items(480, 361, 128, 256, False, 256) == (True, 1)
-    assert halves_items(600, 300, 40, 1024, False, 256) == (True, 1) and halves_items(641, 321, 40, 1024, False, 256) == (False, 2)      # as many rounds; one saved
-    assert halves_items(80, 40, 257, 0, False, 256) == (False, 1) and halves_items(80, 40, 257, 0, True, 256) == (True, 1)      # a cap
-    assert halves_items(300, 150, 400, 0, False, 256) == (True, 1) and halves_items(300, 150, 401, 0, True, 256) == (False, 2)
-    assert halves_items(330, 165, 300, 0, True, 256) == (False, 2) and halves_items(330, 165, 300, 0, False, 304) == (True, 1)
+        assert halves_items(320, 160, 256, window, False, 8, 256) == (True, 1)
+    assert halves_items(321, 161, 256, 1024, False, 8, 256) == (False, 2)
+    assert halves_items(480, 480, 40, 256, False, 8, 256) == (True, 1)         # requests of one group have no pairs
+    assert halves_items(480, 360, 128, 256, False, 8, 256) == (False, 2) and halves_items(480, 361, 128, 256, False, 8, 256) == (True, 1)
+    assert halves_items(512, 256, 40, 1024, False, 8, 256) == (False, 2) and halves_items(514, 257, 40, 1024, False, 8, 256) == (True, 1)      # more than a round
+    assert halves_items(514, 257, 65, 1024, False, 8, 256) == (False, 2)
+    assert [halves_items(512, 256, keys, 1024, False, 4, 256)[0] for keys in (64, 65, 192, 193)] == [True, True, True, False]      # four kv heads
+    assert halves_items(80, 40, 257, 0, False, 8, 256) == (False, 1) and halves_items(80, 40, 257, 0, True, 8, 256) == (True, 1)      # a cap
+    assert halves_items(300, 150, 400, 0, False, 8, 256) == (True, 1) and halves_items(300, 150, 401, 0, True, 8, 256) == (False, 2)
+    assert halves_items(330, 165, 300, 0, True, 8, 256) == (False, 2) and halves_items(330, 165, 300, 0, False, 8, 304) == (True, 1)
 
 
 def test_a_plan_counts_its_items(monkeypatch):
@@ -47,9 +49,9 @@ def test_a_plan_counts_its_items(monkeypatch):
         ctx = SimpleNamespace(q_lens_host=lens, context_lens_host=[0] * len(lens), page_size=16, block_tables=[torch.zeros(len(lens), 64)])
         return attention_backend.plan_mfma(ctx, nq, nkv, 256, kw.pop("window", 0), "cpu", **kw)
 
-    assert plan([40] * 30, 16, 16, window=1024).one_group and asked[-1] == (480, 480, 40, 1024, False, 256)
+    assert plan([40] * 30, 16, 16, window=1024).one_group and asked[-1] == (480, 480, 40, 1024, False, 16, 256)
     plan([1, 129, 1, 300], 16, 8, capped=True)
-    assert asked[-1] == (15 * 8, 8 * 8, 300, 0, True, 256)      # single tokens are no prompt's
+    assert asked[-1] == (15 * 8, 8 * 8, 300, 0, True, 8, 256)      # single tokens are no prompt's
 
 
 @pytest.mark.gpu
